@@ -9,7 +9,9 @@ import ctypes
 import os
 import re
 import subprocess
+import tempfile
 import warnings
+from concurrent.futures import ThreadPoolExecutor
 from pathlib import Path
 
 _PKG = Path(__file__).resolve().parent
@@ -17,6 +19,7 @@ _CSRC = _PKG / "csrc"
 _LIBDIR = _PKG / "lib"
 _SO = _LIBDIR / "libconnect6_amd.so"
 _SOURCES = ("c6_forward.hip", "c6_tail.hip", "c6_generic.hip", "c6_env.hip", "c6_api.hip")
+_MODES = ("PrecF32", "PrecBF16", "PrecF16", "PrecBF16F6", "PrecBF16F6W")   # of c6_forward.hip
 _RESOURCES = _LIBDIR / "resource_usage.txt"   # registers, scratch and LDS of every kernel, written by build()
 
 # arithmetic modes (include/connect6_amd.h)
@@ -66,18 +69,33 @@ def build(verbose: bool = False) -> Path:
     """Compile the HIP sources for gfx950 into ``lib/libconnect6_amd.so``."""
     _LIBDIR.mkdir(exist_ok=True)
     hipcc = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
-    cmd = [
-        hipcc, "--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC", "-shared",
+    flags = [
+        hipcc, "--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC",
         # packed-fp32 VALU forms are disabled for every kernel in this library
         "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
         "-Wall", "-Wno-unused-function",
         "-Rpass-analysis=kernel-resource-usage",
-        "-o", str(_SO),
-    ] + [str(_CSRC / s) for s in _SOURCES]
-    proc = subprocess.run(cmd, capture_output=True, text=True)
+    ]
+    # one object file per source and, for the fused kernels, per arithmetic mode
+    units = [(s, ["-DC6_SPLIT"] if s == "c6_forward.hip" else []) for s in _SOURCES]
+    units = [("c6_forward.hip", [f"-DC6_INSTANCE={m}"]) for m in _MODES] + units
+    with tempfile.TemporaryDirectory(dir=_LIBDIR) as tmp:
+        objs = [str(Path(tmp) / f"{i}.o") for i in range(len(units))]
+
+        def compile_unit(i: int) -> subprocess.CompletedProcess:
+            src, defines = units[i]
+            return subprocess.run(flags + defines + ["-c", str(_CSRC / src), "-o", objs[i]],
+                                  capture_output=True, text=True)
+
+        with ThreadPoolExecutor(min(8, os.cpu_count() or 1)) as pool:
+            procs = list(pool.map(compile_unit, range(len(units))))
+        if all(p.returncode == 0 for p in procs):
+            procs.append(subprocess.run([hipcc, "--offload-arch=gfx950", "-fPIC", "-shared", "-o", str(_SO)] + objs,
+                                        capture_output=True, text=True))
+    returncode = next((p.returncode for p in procs if p.returncode != 0), 0)
     remarks, other = [], []
     excerpt = 0   # a resource-usage remark is followed by a source excerpt of two lines: drop those
-    for line in proc.stderr.splitlines():   # (and only those: excerpts of errors and warnings stay)
+    for line in "\n".join(p.stderr for p in procs).splitlines():   # (and only those: excerpts of errors and warnings stay)
         if "-Rpass-analysis=kernel-resource-usage" in line:
             remarks.append(line)
             excerpt = 2
@@ -86,11 +104,11 @@ def build(verbose: bool = False) -> Path:
         else:
             excerpt = 0
             other.append(line)
-    if verbose or proc.returncode != 0:
-        print(proc.stdout)
+    if verbose or returncode != 0:
+        print("\n".join(p.stdout for p in procs))
         print("\n".join(other))
-    if proc.returncode != 0:
-        raise C6Error(f"hipcc failed ({proc.returncode}):\n" + "\n".join(other)[-4000:])
+    if returncode != 0:
+        raise C6Error(f"hipcc failed ({returncode}):\n" + "\n".join(other)[-4000:])
     _RESOURCES.write_text("\n".join(r.split("remark:", 1)[1].rsplit("[", 1)[0].rstrip() for r in remarks) + "\n")
     try:   # the probe is a measurement aid of bench.py, not part of the library
         build_probe()

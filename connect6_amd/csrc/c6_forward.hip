@@ -2143,7 +2143,14 @@ template <class P> __global__ __launch_bounds__(256) void lo_scale_kernel(const 
 // ------------------------------------------------------------------------
 // host side
 // ------------------------------------------------------------------------
-template <class P> static int launch_pack(const PackParams &pp, hipStream_t st) {
+// The library is built with one object file per arithmetic mode (the compiler takes a minute and
+// more for each): C6_INSTANCE names the mode of this object file, C6_SPLIT marks the one that holds
+// the dispatch.  Without either, this file is all of them (what a traced copy is built from).
+template <class P> int launch_pack(const PackParams &pp, hipStream_t st);
+template <class P> int launch_forward(const FwdParams &fp, hipStream_t st);
+
+#ifndef C6_SPLIT
+template <class P> int launch_pack(const PackParams &pp, hipStream_t st) {
   using G = Geo<P>;
   const long long total = (long long)G::TOTAL_FRAGS * 64 + G::TAIL_FLOATS;
   const int threads = 256;
@@ -2159,7 +2166,7 @@ template <class P> static int launch_pack(const PackParams &pp, hipStream_t st) 
   return C6_OK;
 }
 
-template <class P> static int launch_forward(const FwdParams &fp, hipStream_t st) {
+template <class P> int launch_forward(const FwdParams &fp, hipStream_t st) {
   using G = Geo<P>;
   static_assert(G::LDS_BYTES <= 160 * 1024, "activation tile must fit the 160 KiB LDS of a CU");
   int dev = 0;
@@ -2200,6 +2207,13 @@ template <class P> static int launch_forward(const FwdParams &fp, hipStream_t st
   }
   return C6_OK;
 }
+
+#endif  // C6_SPLIT
+
+#ifdef C6_INSTANCE
+template int launch_pack<C6_INSTANCE>(const PackParams &, hipStream_t);
+template int launch_forward<C6_INSTANCE>(const FwdParams &, hipStream_t);
+#else
 
 int dispatch_pack(int prec, const PackParams &pp, hipStream_t st) {
   if (is_cascade(prec)) {  // both sets of the cascade
@@ -2295,5 +2309,7 @@ size_t packed_bytes(int prec) {
   }
   return 0;
 }
+
+#endif  // C6_INSTANCE
 
 }  // namespace c6

@@ -110,11 +110,61 @@ def build(verbose: bool = False) -> Path:
     if returncode != 0:
         raise C6Error(f"hipcc failed ({returncode}):\n" + "\n".join(other)[-4000:])
     _RESOURCES.write_text("\n".join(r.split("remark:", 1)[1].rsplit("[", 1)[0].rstrip() for r in remarks) + "\n")
+    build_host()
     try:   # the probe is a measurement aid of bench.py, not part of the library
         build_probe()
     except C6Error as exc:
         warnings.warn(f"the MFMA probe did not build (bench.py will report it as missing): {exc}")
     return _SO
+
+
+_HOST_SO = _LIBDIR / "_c6_host.so"
+# entry points csrc/c6_host.cpp calls, in the order of its `Abi`
+_HOST_ABI = ("c6_forward", "c6_forward_cascade", "c6_forward_boards", "c6_forward_boards_cascade",
+             "c6_cascade_workspace_bytes", "c6_mask_logits", "c6_softmax_sample", "c6_env_step", "c6_canonical_input")
+
+
+def build_host() -> Path:
+    """Compile ``csrc/c6_host.cpp`` (the host side of a call, a CPython module) with g++."""
+    import sysconfig
+
+    import torch
+    from torch.utils import cpp_extension
+
+    _LIBDIR.mkdir(exist_ok=True)
+    cmd = [os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-fPIC", "-shared", "-Wall",
+           f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", f"-I{sysconfig.get_paths()['include']}"]
+    cmd += [f"-isystem{d}" for d in cpp_extension.include_paths()]
+    cmd += ["-o", str(_HOST_SO), str(_CSRC / "c6_host.cpp")]
+    cmd += [f"-L{d}" for d in cpp_extension.library_paths()] + ["-ltorch_python", "-ltorch_cpu", "-lc10"]
+    proc = subprocess.run(cmd, capture_output=True, text=True)
+    if proc.returncode != 0:
+        raise C6Error(f"g++ failed ({proc.returncode}):\n{proc.stderr[-4000:]}")
+    return _HOST_SO
+
+
+_host = None
+
+
+def host():
+    """The native host side, bound to the entry points of the loaded library."""
+    return _host if _host is not None and _lib is not None else _bind_host(load())
+
+
+def _bind_host(lib: ctypes.CDLL):
+    global _host
+    if not _HOST_SO.exists():
+        raise C6Error(f"{_HOST_SO} is missing: build it with connect6_amd.build(); there is no fallback path")
+    import importlib.util
+
+    import torch  # noqa: F401  (its libraries have to be loaded first)
+
+    spec = importlib.util.spec_from_file_location("_c6_host", _HOST_SO)
+    module = importlib.util.module_from_spec(spec)
+    spec.loader.exec_module(module)
+    module.bind(*[ctypes.cast(getattr(lib, name), ctypes.c_void_p).value for name in _HOST_ABI])
+    _host = module
+    return module
 
 
 _PROBE_SO = _LIBDIR / "libc6_probe.so"
@@ -235,6 +285,7 @@ def load() -> ctypes.CDLL:
     lib.c6_env_step.argtypes = [vp, vp, vp, vp, vp, vp, i32, i64, i32, i32, vp, vp, vp, vp, vp, vp]
     lib.c6_canonical_input.restype = i32
     lib.c6_canonical_input.argtypes = [vp, vp, vp, i64, i32, vp, vp]
+    _bind_host(lib)
     _lib = lib
     return lib
 
@@ -276,6 +327,8 @@ def torch_dtype_code(dtype) -> int:
 
 
 def stream_ptr(device) -> int:
+    """Handle of the current stream on ``device`` (an indexed device of a tensor, or any torch.device)."""
     import torch
 
-    return int(torch.cuda.current_stream(device).cuda_stream)
+    index = device.index
+    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device() if index is None else index)

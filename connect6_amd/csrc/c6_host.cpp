@@ -1,0 +1,365 @@
+// The host side of a call, natively: argument checks, output tensors, the launch.
+//
+// A call on few boards is bound by what the host does between two launches, and most of that was
+// Python around the C ABI: walking the module's parameters to see whether the packed weights are
+// still current (20 tensors), three to six torch.empty calls, a device context, 20-odd ctypes
+// conversions.  Measured per call of the B = 1 forward plus mask_logits: 68 us in Python, of which
+// two thirds are gone here.  The kernels are reached through the C ABI's own entry points, whose
+// addresses connect6_amd/_lib.py hands over (`bind`), so this module links against no GPU library.
+#define PY_SSIZE_T_CLEAN
+#include <Python.h>
+
+#include <torch/csrc/Exceptions.h>
+#include <torch/csrc/autograd/python_variable.h>
+#include <torch/torch.h>
+
+#include <array>
+#include <cstring>
+#include <string>
+
+#include "../../include/connect6_amd.h"
+
+namespace {
+
+struct Abi {
+  decltype(&c6_forward) forward;
+  decltype(&c6_forward_cascade) forward_cascade;
+  decltype(&c6_forward_boards) forward_boards;
+  decltype(&c6_forward_boards_cascade) forward_boards_cascade;
+  decltype(&c6_cascade_workspace_bytes) cascade_workspace_bytes;
+  decltype(&c6_mask_logits) mask_logits;
+  decltype(&c6_softmax_sample) softmax_sample;
+  decltype(&c6_env_step) env_step;
+  decltype(&c6_canonical_input) canonical_input;
+} abi;
+
+PyObject *fail(PyObject *type, const std::string &what) {
+  PyErr_SetString(type, what.c_str());
+  return nullptr;
+}
+
+// A tensor argument, or null for None.  (Callers pass tensors or None only.)
+const at::Tensor *tensor_or_null(PyObject *o) { return o == Py_None ? nullptr : &THPVariable_Unpack(o); }
+
+std::string shape_text(const at::Tensor &t) {
+  std::string s = "(";
+  for (int64_t i = 0; i < t.dim(); ++i) s += (i ? ", " : "") + std::to_string(t.size(i));
+  return s + (t.dim() == 1 ? ",)" : ")");
+}
+
+int dtype_code(at::ScalarType t) {
+  switch (t) {
+    case at::kFloat: return C6_DT_F32;
+    case at::kBFloat16: return C6_DT_BF16;
+    case at::kHalf: return C6_DT_F16;
+    default: return -1;
+  }
+}
+at::ScalarType type_of_code(int code) {
+  return code == C6_DT_BF16 ? at::kBFloat16 : (code == C6_DT_F16 ? at::kHalf : at::kFloat);
+}
+
+template <class T> T *ptr(const at::Tensor &t) { return t.defined() ? static_cast<T *>(t.data_ptr()) : nullptr; }
+
+at::Tensor fresh(at::IntArrayRef shape, at::ScalarType type, const at::Device &dev) {
+  return at::empty(shape, at::TensorOptions().dtype(type).device(dev));
+}
+
+PyObject *wrap(const at::Tensor &t) {
+  if (!t.defined()) Py_RETURN_NONE;
+  return THPVariable_Wrap(t);
+}
+
+// (rc, tensors ...): the caller turns a nonzero rc into the exception for it
+template <size_t N> PyObject *answer(int rc, const std::array<at::Tensor, N> &ts) {
+  PyObject *out = PyTuple_New(N + 1);
+  if (out == nullptr) return nullptr;
+  PyTuple_SET_ITEM(out, 0, PyLong_FromLong(rc));
+  for (size_t i = 0; i < N; ++i) PyTuple_SET_ITEM(out, i + 1, wrap(ts[i]));
+  return out;
+}
+
+bool is_cascade(int prec) { return prec == C6_PREC_BF16C || prec == C6_PREC_BF16C6; }
+
+at::Tensor cascade_workspace(int64_t boards, const at::Device &dev) {
+  size_t bytes = 0;
+  if (abi.cascade_workspace_bytes(boards, &bytes) != C6_OK) return {};
+  return fresh({(int64_t)(bytes / 4)}, at::kInt, dev);
+}
+
+// Uniform draws as the kernels read them: fp32 on the device, one per board.
+bool take_draws(const at::Tensor *u, int64_t total, const at::Device &dev, at::Tensor &out) {
+  out = u->to(dev, at::kFloat).contiguous();
+  if (out.dim() == 1 && out.size(0) == total) return true;
+  fail(PyExc_ValueError, "u must have shape (" + std::to_string(total) + ",), got " + shape_text(out));
+  return false;
+}
+
+// ---- is the packed copy of a module's parameters still current? --------------------------------
+struct ParamKey {
+  const void *impl, *data;
+  int64_t version;
+  int32_t dtype, pad;
+};
+
+bool walk_parameters(PyObject *module, std::string &key, PyObject *&first) {
+  static PyObject *params_name = PyUnicode_InternFromString("_parameters");
+  static PyObject *modules_name = PyUnicode_InternFromString("_modules");
+  static PyObject *dict_name = PyUnicode_InternFromString("__dict__");
+  PyObject *dict = PyObject_GetAttr(module, dict_name);
+  if (dict == nullptr) return false;
+  bool ok = true;
+  PyObject *k, *v;
+  Py_ssize_t pos = 0;
+  PyObject *params = PyDict_GetItem(dict, params_name);
+  while (params != nullptr && PyDict_Check(params) && PyDict_Next(params, &pos, &k, &v)) {
+    if (!THPVariable_Check(v)) continue;
+    const at::Tensor &t = THPVariable_Unpack(v);
+    if (first == nullptr) first = v;
+    // (inference tensors carry no version counter; load_state_dict and refresh_weights bump the epoch)
+    const ParamKey e{t.unsafeGetTensorImpl(), t.has_storage() ? t.data_ptr() : nullptr,
+                     t.is_inference() ? -1 : (int64_t)t._version(), (int32_t)t.scalar_type(), 0};
+    key.append(reinterpret_cast<const char *>(&e), sizeof(e));
+  }
+  pos = 0;
+  PyObject *children = PyDict_GetItem(dict, modules_name);
+  while (ok && children != nullptr && PyDict_Check(children) && PyDict_Next(children, &pos, &k, &v))
+    if (v != Py_None) ok = walk_parameters(v, key, first);
+  Py_DECREF(dict);
+  return ok;
+}
+
+// parameters(module) -> (key, first parameter or None): the key changes whenever a parameter of the
+// module or of a module in it is replaced, moved, retyped or modified in place
+PyObject *parameters(PyObject *, PyObject *module) {
+  std::string key;
+  key.reserve(24 * sizeof(ParamKey));
+  PyObject *first = nullptr;
+  if (!walk_parameters(module, key, first)) return nullptr;
+  PyObject *bytes = PyBytes_FromStringAndSize(key.data(), (Py_ssize_t)key.size());
+  if (bytes == nullptr) return nullptr;
+  PyObject *out = PyTuple_Pack(2, bytes, first != nullptr ? first : Py_None);
+  Py_DECREF(bytes);
+  return out;
+}
+
+// forward(x, packed, prec, groups, boards_per_group, want_logits, want_value, mask_mode, legal, fill, u,
+//         temperature, want_logprob, threshold, logits dtype code, stream)
+//   -> (rc, logits, value, actions, logprob, cascade: boards evaluated twice as an int32[1])
+PyObject *forward(PyObject *, PyObject *const *a, Py_ssize_t n) {
+  if (n != 16) return fail(PyExc_TypeError, "forward takes 16 arguments");
+  HANDLE_TH_ERRORS
+  const at::Tensor x = THPVariable_Unpack(a[0]).contiguous();
+  const at::Tensor &packed = THPVariable_Unpack(a[1]);
+  const int prec = (int)PyLong_AsLong(a[2]);
+  const int64_t groups = PyLong_AsLongLong(a[3]), per = PyLong_AsLongLong(a[4]), total = groups * per;
+  const bool want_logits = PyObject_IsTrue(a[5]) == 1, want_value = PyObject_IsTrue(a[6]) == 1,
+             want_logprob = PyObject_IsTrue(a[12]) == 1;
+  const int mask_mode = (int)PyLong_AsLong(a[7]);
+  const at::Tensor *legal_in = tensor_or_null(a[8]), *u_in = tensor_or_null(a[10]);
+  const float fill = (float)PyFloat_AsDouble(a[9]), temperature = (float)PyFloat_AsDouble(a[11]);
+  const float threshold = (float)PyFloat_AsDouble(a[13]);
+  const int logits_code = (int)PyLong_AsLong(a[14]);
+  void *stream = PyLong_AsVoidPtr(a[15]);
+  if (PyErr_Occurred()) return nullptr;
+  const at::Device dev = x.device();
+  const int x_code = dtype_code(x.scalar_type());
+  if (x_code < 0)
+    return fail(PyExc_ValueError, std::string("unsupported tensor dtype ") + c10::toString(x.scalar_type()) +
+                                      "; expected float32, bfloat16 or float16");
+  at::Tensor legal, u, logits, value, actions, logprob, ws;
+  if (u_in != nullptr && !take_draws(u_in, total, dev, u)) return nullptr;
+  if (legal_in != nullptr) {
+    if (legal_in->dim() != 2 || legal_in->size(0) != total || legal_in->size(1) != C6_ACTIONS)
+      return fail(PyExc_ValueError, "legal mask must have shape (" + std::to_string(total) + ", 361), got " +
+                                        shape_text(*legal_in));
+    if (legal_in->scalar_type() != at::kBool && legal_in->scalar_type() != at::kByte)
+      return fail(PyExc_ValueError, "legal mask must be a bool or uint8 tensor");
+    legal = legal_in->to(dev).contiguous();
+  }
+  const c10::DeviceGuard guard(dev);
+  if (want_logits) logits = fresh({total, C6_ACTIONS}, type_of_code(logits_code), dev);
+  if (want_value) value = fresh({total}, at::kFloat, dev);
+  if (u_in != nullptr) {
+    actions = fresh({total}, at::kLong, dev);
+    if (want_logprob) logprob = fresh({total}, at::kFloat, dev);
+  }
+  const size_t stride = (size_t)packed.numel() / (size_t)(groups > 1 ? groups : 1);
+  const uint8_t *legal_ptr = static_cast<const uint8_t *>(legal.defined() ? legal.data_ptr() : nullptr);
+  int rc;
+  if (is_cascade(prec)) {
+    ws = cascade_workspace(total, dev);
+    rc = abi.forward_cascade(x.data_ptr(), x_code, groups, per, packed.data_ptr(), stride, prec, ptr<void>(logits),
+                             logits_code, ptr<float>(value), mask_mode, legal_ptr, fill, ptr<float>(u), temperature,
+                             ptr<int64_t>(actions), ptr<float>(logprob), threshold, ptr<void>(ws),
+                             ws.defined() ? ws.nbytes() : 0, stream);
+  } else {
+    rc = abi.forward(x.data_ptr(), x_code, groups, per, packed.data_ptr(), stride, prec, ptr<float>(logits),
+                     ptr<float>(value), mask_mode, legal_ptr, fill, ptr<float>(u), temperature,
+                     ptr<int64_t>(actions), ptr<float>(logprob), stream);
+  }
+  return answer<5>(rc, {logits, value, actions, logprob, ws.defined() ? ws.narrow(0, 0, 1) : ws});
+  END_HANDLE_TH_ERRORS
+}
+
+// forward_boards(boards, player, stones_left, index, view, packed, prec, want_logits, mask_mode, fill, u,
+//                temperature, threshold, stream) -> as forward; the state tensors are checked by the caller
+PyObject *forward_boards(PyObject *, PyObject *const *a, Py_ssize_t n) {
+  if (n != 14) return fail(PyExc_TypeError, "forward_boards takes 14 arguments");
+  HANDLE_TH_ERRORS
+  const at::Tensor &boards_in = THPVariable_Unpack(a[0]);
+  const at::Device dev = boards_in.device();
+  const int64_t states = boards_in.size(0);
+  const at::Tensor boards = boards_in.contiguous();
+  const at::Tensor player = THPVariable_Unpack(a[1]).to(dev).contiguous();
+  const at::Tensor left = THPVariable_Unpack(a[2]).to(dev).contiguous();
+  const at::Tensor *index_in = tensor_or_null(a[3]), *u_in = tensor_or_null(a[10]);
+  const int view = (int)PyLong_AsLong(a[4]);
+  const at::Tensor &packed = THPVariable_Unpack(a[5]);
+  const int prec = (int)PyLong_AsLong(a[6]);
+  const bool want_logits = PyObject_IsTrue(a[7]) == 1;
+  const int mask_mode = (int)PyLong_AsLong(a[8]);
+  const float fill = (float)PyFloat_AsDouble(a[9]), temperature = (float)PyFloat_AsDouble(a[11]);
+  const float threshold = (float)PyFloat_AsDouble(a[12]);
+  void *stream = PyLong_AsVoidPtr(a[13]);
+  if (PyErr_Occurred()) return nullptr;
+  at::Tensor index, u, logits, actions, logprob, ws;
+  if (index_in != nullptr) index = index_in->to(dev).contiguous();
+  const int64_t total = index.defined() ? index.numel() : states;
+  if (u_in != nullptr && !take_draws(u_in, total, dev, u)) return nullptr;
+  const c10::DeviceGuard guard(dev);
+  if (want_logits) logits = fresh({total, C6_ACTIONS}, at::kFloat, dev);
+  const at::Tensor value = fresh({total}, at::kFloat, dev);
+  if (u_in != nullptr) {
+    actions = fresh({total}, at::kLong, dev);
+    logprob = fresh({total}, at::kFloat, dev);
+  }
+  int rc;
+  if (is_cascade(prec)) {
+    ws = cascade_workspace(total, dev);
+    rc = abi.forward_boards_cascade(ptr<int8_t>(boards), ptr<int8_t>(player), ptr<int8_t>(left), states,
+                                    ptr<int64_t>(index), view, total, packed.data_ptr(), prec, ptr<void>(logits),
+                                    C6_DT_F32, ptr<float>(value), mask_mode, fill, ptr<float>(u), temperature,
+                                    ptr<int64_t>(actions), ptr<float>(logprob), threshold, ptr<void>(ws),
+                                    ws.defined() ? ws.nbytes() : 0, stream);
+  } else {
+    rc = abi.forward_boards(ptr<int8_t>(boards), ptr<int8_t>(player), ptr<int8_t>(left), states, ptr<int64_t>(index),
+                            view, total, packed.data_ptr(), prec, ptr<float>(logits), ptr<float>(value), mask_mode,
+                            fill, ptr<float>(u), temperature, ptr<int64_t>(actions), ptr<float>(logprob), stream);
+  }
+  return answer<5>(rc, {logits, value, actions, logprob, ws.defined() ? ws.narrow(0, 0, 1) : ws});
+  END_HANDLE_TH_ERRORS
+}
+
+// mask_logits(logits, legal, stream) -> (rc, masked); the fill is the lowest finite value of the type
+PyObject *mask_logits(PyObject *, PyObject *const *a, Py_ssize_t n) {
+  if (n != 3) return fail(PyExc_TypeError, "mask_logits takes 3 arguments");
+  HANDLE_TH_ERRORS
+  const at::Tensor src = THPVariable_Unpack(a[0]).contiguous();
+  const at::Tensor &legal_in = THPVariable_Unpack(a[1]);
+  void *stream = PyLong_AsVoidPtr(a[2]);
+  if (PyErr_Occurred()) return nullptr;
+  const at::Device dev = src.device();
+  const int code = dtype_code(src.scalar_type());
+  if (code < 0)
+    return fail(PyExc_ValueError, std::string("unsupported tensor dtype ") + c10::toString(src.scalar_type()) +
+                                      "; expected float32, bfloat16 or float16");
+  const at::Tensor legal = legal_in.to(dev).contiguous();
+  // bit patterns of -(largest finite value): fp32, bf16, fp16
+  const uint32_t fill = code == C6_DT_F32 ? 0xFF7FFFFFu : (code == C6_DT_BF16 ? 0xFF7Fu : 0xFBFFu);
+  const c10::DeviceGuard guard(dev);
+  const at::Tensor out = fresh(src.sizes(), src.scalar_type(), dev);
+  const int rc = abi.mask_logits(src.data_ptr(), static_cast<const uint8_t *>(legal.data_ptr()), code, src.size(0),
+                                 fill, out.data_ptr(), stream);
+  return answer<1>(rc, {out});
+  END_HANDLE_TH_ERRORS
+}
+
+// sample(logits, legal, temperature, u, want_logprob, stream) -> (rc, actions, logprob)
+PyObject *sample(PyObject *, PyObject *const *a, Py_ssize_t n) {
+  if (n != 6) return fail(PyExc_TypeError, "sample takes 6 arguments");
+  HANDLE_TH_ERRORS
+  const at::Tensor src = THPVariable_Unpack(a[0]).to(at::kFloat).contiguous();
+  const at::Tensor *legal_in = tensor_or_null(a[1]);
+  const float temperature = (float)PyFloat_AsDouble(a[2]);
+  const at::Device dev = src.device();
+  const int64_t b = src.size(0);
+  void *stream = PyLong_AsVoidPtr(a[5]);
+  if (PyErr_Occurred()) return nullptr;
+  at::Tensor legal, u, logprob;
+  if (legal_in != nullptr) legal = legal_in->to(dev).contiguous();
+  if (!take_draws(&THPVariable_Unpack(a[3]), b, dev, u)) return nullptr;
+  const c10::DeviceGuard guard(dev);
+  const at::Tensor actions = fresh({b}, at::kLong, dev);
+  if (PyObject_IsTrue(a[4]) == 1) logprob = fresh({b}, at::kFloat, dev);
+  const int rc = abi.softmax_sample(ptr<float>(src), static_cast<const uint8_t *>(ptr<void>(legal)), ptr<float>(u),
+                                    temperature, b, ptr<int64_t>(actions), ptr<float>(logprob), stream);
+  return answer<2>(rc, {actions, logprob});
+  END_HANDLE_TH_ERRORS
+}
+
+// env_step(boards, player, stones_left, empty_count, move_count, actions, view, win_length, stream)
+//   -> (rc, reward, done, winner, sign, lengths)
+PyObject *env_step(PyObject *, PyObject *const *a, Py_ssize_t n) {
+  if (n != 9) return fail(PyExc_TypeError, "env_step takes 9 arguments");
+  HANDLE_TH_ERRORS
+  const at::Tensor &boards = THPVariable_Unpack(a[0]);
+  const at::Device dev = boards.device();
+  const int64_t num = boards.size(0);
+  const at::Tensor &actions = THPVariable_Unpack(a[5]);
+  const int view = (int)PyLong_AsLong(a[6]), win = (int)PyLong_AsLong(a[7]);
+  void *stream = PyLong_AsVoidPtr(a[8]);
+  if (PyErr_Occurred()) return nullptr;
+  const c10::DeviceGuard guard(dev);
+  const at::Tensor reward = fresh({num}, at::kFloat, dev), done = fresh({num}, at::kBool, dev),
+                   winner = fresh({num}, at::kChar, dev), sign = fresh({num}, at::kChar, dev),
+                   lengths = fresh({num}, at::kShort, dev);
+  const int rc = abi.env_step(ptr<int8_t>(boards), ptr<int8_t>(THPVariable_Unpack(a[1])),
+                              ptr<int8_t>(THPVariable_Unpack(a[2])), ptr<int16_t>(THPVariable_Unpack(a[3])),
+                              ptr<int16_t>(THPVariable_Unpack(a[4])), ptr<int64_t>(actions), view, num,
+                              (int)boards.size(1), win, ptr<float>(reward), static_cast<uint8_t *>(done.data_ptr()),
+                              ptr<int8_t>(winner), ptr<int8_t>(sign), ptr<int16_t>(lengths), stream);
+  return answer<5>(rc, {reward, done, winner, sign, lengths});
+  END_HANDLE_TH_ERRORS
+}
+
+// canonical_input(boards, player, stones_left, stream) -> (rc, planes)
+PyObject *canonical_input(PyObject *, PyObject *const *a, Py_ssize_t n) {
+  if (n != 4) return fail(PyExc_TypeError, "canonical_input takes 4 arguments");
+  HANDLE_TH_ERRORS
+  const at::Tensor boards = THPVariable_Unpack(a[0]).contiguous(), player = THPVariable_Unpack(a[1]).contiguous(),
+                   left = THPVariable_Unpack(a[2]).contiguous();
+  void *stream = PyLong_AsVoidPtr(a[3]);
+  if (PyErr_Occurred()) return nullptr;
+  const at::Device dev = boards.device();
+  const int64_t num = boards.size(0), size = boards.size(2);
+  const c10::DeviceGuard guard(dev);
+  const at::Tensor out = fresh({num, 3, size, size}, at::kFloat, dev);
+  const int rc = abi.canonical_input(ptr<int8_t>(boards), ptr<int8_t>(player), ptr<int8_t>(left), num, (int)size,
+                                     ptr<float>(out), stream);
+  return answer<1>(rc, {out});
+  END_HANDLE_TH_ERRORS
+}
+
+// bind(addresses): the C ABI's entry points, in the order of `Abi`
+PyObject *bind(PyObject *, PyObject *const *a, Py_ssize_t n) {
+  constexpr Py_ssize_t kEntries = sizeof(Abi) / sizeof(void *);
+  if (n != kEntries) return fail(PyExc_TypeError, "bind takes one address per entry point");
+  std::array<void *, kEntries> addr;
+  for (Py_ssize_t i = 0; i < kEntries; ++i) addr[i] = PyLong_AsVoidPtr(a[i]);
+  if (PyErr_Occurred()) return nullptr;
+  std::memcpy(&abi, addr.data(), sizeof(abi));
+  Py_RETURN_NONE;
+}
+
+#define C6_FAST(name) {#name, reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)(void)>(name)), METH_FASTCALL, nullptr}
+PyMethodDef methods[] = {C6_FAST(bind),        C6_FAST(forward),        C6_FAST(forward_boards),
+                         C6_FAST(mask_logits), C6_FAST(sample),         C6_FAST(env_step),
+                         C6_FAST(canonical_input),
+                         {"parameters", parameters, METH_O, nullptr},
+                         {nullptr, nullptr, 0, nullptr}};
+PyModuleDef module_def = {PyModuleDef_HEAD_INIT, "_c6_host", nullptr, -1, methods, nullptr, nullptr, nullptr, nullptr};
+
+}  // namespace
+
+PyMODINIT_FUNC PyInit__c6_host(void) { return PyModule_Create(&module_def); }

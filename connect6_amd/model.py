@@ -104,53 +104,16 @@ def run_forward(
     one-element int32 device tensor, the number of boards that were evaluated twice.
     ``logits_dtype`` other than float32 (the cascade mode's entry point only) makes the kernel
     write the logits rounded to that type."""
-    lib = _lib.load()
-    dev = x.device
-    total = groups * boards_per_group
-    x = x.contiguous()
     if logits_dtype != torch.float32 and prec not in _lib.CASCADES:
         raise ValueError("only the cascade mode's entry point writes logits in another type than float32")
-    logits = torch.empty((total, 361), dtype=logits_dtype, device=dev) if want_logits else None
-    value = torch.empty((total,), dtype=torch.float32, device=dev) if want_value else None
-    actions = logprob = None
-    if u is not None:
-        u = u.to(device=dev, dtype=torch.float32).contiguous()
-        if u.shape != (total,):
-            raise ValueError(f"u must have shape ({total},), got {tuple(u.shape)}")
-        actions = torch.empty((total,), dtype=torch.int64, device=dev)
-        if want_logprob:
-            logprob = torch.empty((total,), dtype=torch.float32, device=dev)
-    if legal is not None:
-        if legal.shape != (total, 361):
-            raise ValueError(f"legal mask must have shape ({total}, 361), got {tuple(legal.shape)}")
-        if legal.dtype == torch.bool:
-            legal = legal.contiguous().view(torch.uint8)
-        elif legal.dtype != torch.uint8:
-            raise ValueError("legal mask must be a bool or uint8 tensor")
-        legal = legal.to(dev).contiguous()
-
-    def ptr(t):
-        return t.data_ptr() if t is not None else None
-
-    stride = packed.numel() // groups if groups > 1 else packed.numel()
-    with torch.cuda.device(dev):
-        if prec in _lib.CASCADES:
-            ws = torch.empty(_lib.cascade_workspace_bytes(total) // 4, dtype=torch.int32, device=dev)
-            rc = lib.c6_forward_cascade(
-                x.data_ptr(), _lib.torch_dtype_code(x.dtype), groups, boards_per_group, packed.data_ptr(),
-                stride, prec, ptr(logits), _lib.torch_dtype_code(logits_dtype), ptr(value), mask_mode, ptr(legal), fill,
-                ptr(u), float(temperature), ptr(actions), ptr(logprob),
-                float(_lib.CASCADE_THRESHOLD if threshold is None else threshold),
-                ws.data_ptr(), ws.numel() * 4, _lib.stream_ptr(dev))
-            if stats is not None:
-                stats["second_pass"] = ws[:1]
-            _lib.check(rc, "c6_forward_cascade")
-            return logits, value, actions, logprob
-        rc = lib.c6_forward(x.data_ptr(), _lib.torch_dtype_code(x.dtype), groups, boards_per_group,
-                            packed.data_ptr(), stride, prec, ptr(logits), ptr(value), mask_mode,
-                            ptr(legal), fill, ptr(u), float(temperature), ptr(actions),
-                            ptr(logprob), _lib.stream_ptr(dev))
-    _lib.check(rc, "c6_forward")
+    rc, logits, value, actions, logprob, twice = _lib.host().forward(
+        x, packed, prec, groups, boards_per_group, want_logits, want_value, mask_mode, legal, fill, u, temperature,
+        want_logprob, _lib.CASCADE_THRESHOLD if threshold is None else threshold,
+        _lib.torch_dtype_code(logits_dtype), _lib.stream_ptr(x.device))
+    if twice is not None and stats is not None:
+        stats["second_pass"] = twice
+    if rc != 0:
+        _lib.check(rc, "c6_forward_cascade" if prec in _lib.CASCADES else "c6_forward")
     return logits, value, actions, logprob
 
 
@@ -388,17 +351,14 @@ class PolicyValueNet(nn.Module):
     def packed_weights(self, prec: int) -> torch.Tensor:
         """Kernel-layout copy of the parameters; rebuilt whenever a parameter
         was modified in place, replaced or moved."""
-        params = list(self.parameters())
-        # inference tensors carry no version counter; load_state_dict / refresh_weights bump the epoch
-        key = (self._epoch,) + tuple(
-            (p.data_ptr(), -1 if p.is_inference() else p._version, p.dtype) for p in params
-        )
-        dev = params[0].device
-        stream = torch.cuda.current_stream(dev)
+        key, first = _lib.host().parameters(self)
+        dev = first.device
+        stream_ptr = _lib.stream_ptr(dev)
         hit = self._packed.get(prec)
-        if hit is not None and hit[0] == key:
-            _, buf, packed_on, done = hit
-            if packed_on != stream.cuda_stream:
+        if hit is not None and hit[0] == self._epoch and hit[1] == key:
+            _, _, buf, packed_on, done = hit
+            if packed_on != stream_ptr:
+                stream = torch.cuda.current_stream(dev)
                 stream.wait_event(done)  # the pack kernel ran on another stream
                 # ... whose allocator owns the buffer: a repack drops it, and without this note the
                 # memory could be handed out again while a forward here still reads it
@@ -407,14 +367,15 @@ class PolicyValueNet(nn.Module):
         buf = torch.empty(_lib.packed_bytes(prec), dtype=torch.uint8, device=dev)
         pack_state({k: v for k, v in self.state_dict().items()}, prec, buf)
         done = torch.cuda.Event()
-        done.record(stream)
-        self._packed[prec] = (key, buf, stream.cuda_stream, done)
+        done.record(torch.cuda.current_stream(dev))
+        self._packed[prec] = (self._epoch, key, buf, stream_ptr, done)
         return buf
 
     # -- forward --------------------------------------------------------------
     def _check_input(self, x: torch.Tensor) -> None:
+        shape = x.shape
         expected = (self.input_channels, self.board_size, self.board_size)
-        if x.ndim != 4 or tuple(x.shape[1:]) != expected:
+        if len(shape) != 4 or shape[1:] != expected:
             raise ValueError(
                 f"model input must have shape [B, {expected[0]}, {expected[1]}, {expected[2]}], "
                 f"got {tuple(x.shape)}."
@@ -544,12 +505,11 @@ class PolicyValueNet(nn.Module):
         return actions, logprob, value
 
 
-def _state_tensor(t: torch.Tensor, name: str, shape, dev) -> torch.Tensor:
+def _check_state(t: torch.Tensor, name: str, shape) -> None:
     if t.dtype != torch.int8:
         raise ValueError(f"{name} must be an int8 tensor (as VectorConnect6 holds it), got {t.dtype}")
-    if tuple(t.shape) != tuple(shape):
+    if t.shape != shape:
         raise ValueError(f"{name} must have shape {tuple(shape)}, got {tuple(t.shape)}")
-    return t.to(dev).contiguous()
 
 
 def _forward_boards(
@@ -577,51 +537,23 @@ def _forward_boards(
         raise ValueError(f"boards must have shape [N, 19, 19], got {tuple(boards.shape)}")
     if not 0 <= int(view) <= 7:
         raise ValueError(f"view must be a D4 phase 0..7, got {view}")
-    dev = boards.device
     n = int(boards.shape[0])
-    boards = _state_tensor(boards, "boards", (n, 19, 19), dev)
-    current_player = _state_tensor(current_player, "current_player", (n,), dev)
-    stones_left = _state_tensor(stones_left, "stones_left", (n,), dev)
-    if index is not None:
-        if index.dtype != torch.int64 or index.ndim != 1:
-            raise ValueError("index must be a 1-D int64 tensor of board rows")
-        index = index.to(dev).contiguous()   # entries outside [0, N) are clamped by the kernel
-    b = n if index is None else int(index.numel())
+    _check_state(boards, "boards", (n, 19, 19))
+    _check_state(current_player, "current_player", (n,))
+    _check_state(stones_left, "stones_left", (n,))
+    if index is not None and (index.dtype != torch.int64 or index.ndim != 1):
+        raise ValueError("index must be a 1-D int64 tensor of board rows")
+    # (index entries outside [0, N) are clamped by the kernel)
     prec = model.resolve_precision()
-    packed = model.packed_weights(prec)
-    logits = torch.empty((b, 361), dtype=torch.float32, device=dev) if want_logits else None
-    value = torch.empty((b,), dtype=torch.float32, device=dev)
-    actions = logprob = None
-    if u is not None:
-        u = u.to(device=dev, dtype=torch.float32).contiguous()
-        if u.shape != (b,):
-            raise ValueError(f"u must have shape ({b},), got {tuple(u.shape)}")
-        actions = torch.empty((b,), dtype=torch.int64, device=dev)
-        logprob = torch.empty((b,), dtype=torch.float32, device=dev)
-
-    def ptr(t):
-        return t.data_ptr() if t is not None else None
-
-    with torch.cuda.device(dev):
-        if prec in _lib.CASCADES:
-            ws = torch.empty(_lib.cascade_workspace_bytes(b) // 4, dtype=torch.int32, device=dev)
-            thr = _lib.CASCADE_THRESHOLD if model.cascade_threshold is None else model.cascade_threshold
-            rc = _lib.load().c6_forward_boards_cascade(
-                boards.data_ptr(), current_player.data_ptr(), stones_left.data_ptr(), n, ptr(index),
-                int(view), b, packed.data_ptr(), prec, ptr(logits), _lib.DT_F32, value.data_ptr(),
-                _lib.MASK_INPUT if masked else _lib.MASK_NONE,
-                _FILL_LOWEST if fill is None else float(fill), ptr(u), float(temperature),
-                ptr(actions), ptr(logprob), float(thr), ws.data_ptr(), ws.numel() * 4, _lib.stream_ptr(dev))
-            model.cascade_stats["second_pass"] = ws[:1]
-            _lib.check(rc, "c6_forward_boards_cascade")
-            return logits, value, actions, logprob
-        rc = _lib.load().c6_forward_boards(
-            boards.data_ptr(), current_player.data_ptr(), stones_left.data_ptr(), n, ptr(index),
-            int(view), b, packed.data_ptr(), prec, ptr(logits), value.data_ptr(),
-            _lib.MASK_INPUT if masked else _lib.MASK_NONE,
-            _FILL_LOWEST if fill is None else float(fill), ptr(u), float(temperature),
-            ptr(actions), ptr(logprob), _lib.stream_ptr(dev))
-    _lib.check(rc, "c6_forward_boards")
+    thr = model.cascade_threshold
+    rc, logits, value, actions, logprob, twice = _lib.host().forward_boards(
+        boards, current_player, stones_left, index, int(view), model.packed_weights(prec), prec, want_logits,
+        _lib.MASK_INPUT if masked else _lib.MASK_NONE, _FILL_LOWEST if fill is None else fill, u, temperature,
+        _lib.CASCADE_THRESHOLD if thr is None else thr, _lib.stream_ptr(boards.device))
+    if twice is not None:
+        model.cascade_stats["second_pass"] = twice
+    if rc != 0:
+        _lib.check(rc, "c6_forward_boards_cascade" if prec in _lib.CASCADES else "c6_forward_boards")
     return logits, value, actions, logprob
 
 
@@ -646,18 +578,7 @@ def mask_logits(logits: torch.Tensor, legal_mask: torch.Tensor) -> torch.Tensor:
         )
     if legal_mask.dtype != torch.bool:
         raise ValueError("legal mask must be a bool tensor")
-    lib = _lib.load()
-    src = logits.contiguous()
-    legal = legal_mask.to(logits.device).contiguous().view(torch.uint8)
-    out = torch.empty_like(src)
-    fill = torch.tensor(torch.finfo(src.dtype).min, dtype=src.dtype)
-    if src.dtype == torch.float32:
-        fill_bits = int(fill.view(torch.int32).item()) & 0xFFFFFFFF
-    else:
-        fill_bits = int(fill.view(torch.int16).item()) & 0xFFFF
-    with torch.cuda.device(src.device):
-        rc = lib.c6_mask_logits(src.data_ptr(), legal.data_ptr(), _lib.torch_dtype_code(src.dtype),
-                                int(src.shape[0]), fill_bits, out.data_ptr(),
-                                _lib.stream_ptr(src.device))
-    _lib.check(rc, "c6_mask_logits")
+    rc, out = _lib.host().mask_logits(logits, legal_mask, _lib.stream_ptr(logits.device))
+    if rc != 0:
+        _lib.check(rc, "c6_mask_logits")
     return out

@@ -79,25 +79,12 @@ def sample_actions(
     _require_device_tensor(logits, "logits")
     if logits.ndim != 2 or logits.shape[1] != 361:
         raise ValueError(f"logits must have shape [B, 361], got {tuple(logits.shape)}")
-    lib = _lib.load()
-    dev = logits.device
-    src = logits.float().contiguous()
-    b = int(src.shape[0])
-    if legal is not None:
-        if legal.shape != src.shape or legal.dtype != torch.bool:
-            raise ValueError("legal must be a bool tensor of the logits' shape")
-        legal = legal.to(dev).contiguous().view(torch.uint8)
-    u = u.to(device=dev, dtype=torch.float32).contiguous()
-    if u.shape != (b,):
-        raise ValueError(f"u must have shape ({b},), got {tuple(u.shape)}")
-    actions = torch.empty((b,), dtype=torch.int64, device=dev)
-    logprob = torch.empty((b,), dtype=torch.float32, device=dev) if return_logprob else None
-    with torch.cuda.device(dev):
-        rc = lib.c6_softmax_sample(src.data_ptr(), legal.data_ptr() if legal is not None else None,
-                                   u.data_ptr(), float(temperature), b, actions.data_ptr(),
-                                   logprob.data_ptr() if logprob is not None else None,
-                                   _lib.stream_ptr(dev))
-    _lib.check(rc, "c6_softmax_sample")
+    if legal is not None and (legal.shape != logits.shape or legal.dtype != torch.bool):
+        raise ValueError("legal must be a bool tensor of the logits' shape")
+    rc, actions, logprob = _lib.host().sample(logits, legal, temperature, u, bool(return_logprob),
+                                              _lib.stream_ptr(logits.device))
+    if rc != 0:
+        _lib.check(rc, "c6_softmax_sample")
     return (actions, logprob) if return_logprob else actions
 
 

@@ -47,14 +47,10 @@ def canonical_network_input(
 ) -> torch.Tensor:
     """connect6/vector_env.py:196-218: [N, 3, n, n] float32, planes = own stones, the other
     side's stones, "this decision is the last stone of the turn"."""
-    n_env = _require_state(boards, current_player, stones_left)
-    size = boards.shape[-1]
-    boards, current_player, stones_left = boards.contiguous(), current_player.contiguous(), stones_left.contiguous()
-    out = torch.empty((n_env, 3, size, size), dtype=torch.float32, device=boards.device)
-    with torch.cuda.device(boards.device):
-        rc = _lib.load().c6_canonical_input(boards.data_ptr(), current_player.data_ptr(), stones_left.data_ptr(),
-                                            n_env, size, out.data_ptr(), _lib.stream_ptr(boards.device))
-    _lib.check(rc, "c6_canonical_input")
+    _require_state(boards, current_player, stones_left)
+    rc, out = _lib.host().canonical_input(boards, current_player, stones_left, _lib.stream_ptr(boards.device))
+    if rc != 0:
+        _lib.check(rc, "c6_canonical_input")
     return out
 
 
@@ -152,18 +148,9 @@ class VectorConnect6:
             if bool(occupied.any()):
                 bad = int(torch.nonzero(occupied, as_tuple=False).flatten()[0])
                 raise RuntimeError(f"stone placed on an occupied square in env {bad}")
-        dev = self.device
-        n_env = self.num_envs
-        reward = torch.empty(n_env, dtype=torch.float32, device=dev)
-        done = torch.empty(n_env, dtype=torch.bool, device=dev)
-        winner = torch.empty(n_env, dtype=torch.int8, device=dev)
-        sign = torch.empty(n_env, dtype=torch.int8, device=dev)
-        lengths = torch.empty(n_env, dtype=torch.int16, device=dev)
-        with torch.cuda.device(dev):
-            rc = _lib.load().c6_env_step(
-                self.boards.data_ptr(), self.current_player.data_ptr(), self.stones_left.data_ptr(),
-                self.empty_count.data_ptr(), self.move_count.data_ptr(), actions.data_ptr(), view, n_env,
-                self.board_size, self.win_length, reward.data_ptr(), done.data_ptr(), winner.data_ptr(),
-                sign.data_ptr(), lengths.data_ptr(), _lib.stream_ptr(dev))
-        _lib.check(rc, "c6_env_step")
+        rc, reward, done, winner, sign, lengths = _lib.host().env_step(
+            self.boards, self.current_player, self.stones_left, self.empty_count, self.move_count, actions, view,
+            self.win_length, _lib.stream_ptr(self.boards.device))
+        if rc != 0:
+            _lib.check(rc, "c6_env_step")
         return StepBatch(reward=reward, done=done, winner=winner, transition_sign=sign, game_lengths=lengths)

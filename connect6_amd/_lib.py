@@ -18,7 +18,7 @@ _PKG = Path(__file__).resolve().parent
 _CSRC = _PKG / "csrc"
 _LIBDIR = _PKG / "lib"
 _SO = _LIBDIR / "libconnect6_amd.so"
-_SOURCES = ("c6_forward.hip", "c6_tail.hip", "c6_generic.hip", "c6_env.hip", "c6_api.hip")
+_SOURCES = ("c6_forward.hip", "c6_tail.hip", "c6_generic.hip", "c6_small.hip", "c6_env.hip", "c6_api.hip")
 _MODES = ("PrecF32", "PrecBF16", "PrecF16", "PrecBF16F6", "PrecBF16F6W")   # of c6_forward.hip
 _RESOURCES = _LIBDIR / "resource_usage.txt"   # registers, scratch and LDS of every kernel, written by build()
 
@@ -52,6 +52,9 @@ EXPORTS = (
     "c6_forward_generic",
     "c6_forward_generic_grouped",
     "c6_forward_generic_static",
+    "c6_generic_packed_bytes",
+    "c6_generic_pack",
+    "c6_forward_generic_packed",
     "c6_mask_logits",
     "c6_softmax_sample",
     "c6_d4_expand",
@@ -121,7 +124,8 @@ def build(verbose: bool = False) -> Path:
 _HOST_SO = _LIBDIR / "_c6_host.so"
 # entry points csrc/c6_host.cpp calls, in the order of its `Abi`
 _HOST_ABI = ("c6_forward", "c6_forward_cascade", "c6_forward_boards", "c6_forward_boards_cascade",
-             "c6_cascade_workspace_bytes", "c6_mask_logits", "c6_softmax_sample", "c6_env_step", "c6_canonical_input")
+             "c6_cascade_workspace_bytes", "c6_mask_logits", "c6_softmax_sample", "c6_env_step", "c6_canonical_input",
+             "c6_forward_generic_packed")
 
 
 def build_host() -> Path:
@@ -273,6 +277,14 @@ def load() -> ctypes.CDLL:
     lib.c6_forward_generic_static.argtypes = [vp, i32, i64, i32, i32, ip, ip, ctypes.POINTER(vp),
                                               ctypes.POINTER(vp), vp, vp, vp, vp, i32, vp, vp,
                                               i32, vp, f32, vp]
+    lib.c6_generic_packed_bytes.restype = i32
+    lib.c6_generic_packed_bytes.argtypes = [i32, i32, ip, ip, i32, ctypes.POINTER(ctypes.c_size_t)]
+    lib.c6_generic_pack.restype = i32
+    lib.c6_generic_pack.argtypes = [i64, i32, i32, ip, ip, ctypes.POINTER(vp), ctypes.POINTER(vp), vp, vp, vp, vp,
+                                    i32, vp, ctypes.c_size_t, vp]
+    lib.c6_forward_generic_packed.restype = i32
+    lib.c6_forward_generic_packed.argtypes = [vp, i32, i64, i64, i32, i32, ip, ip, vp, ctypes.c_size_t, i32, vp, vp,
+                                              i32, vp, f32, vp]
     lib.c6_mask_logits.restype = i32
     lib.c6_mask_logits.argtypes = [vp, vp, i32, i64, ctypes.c_uint32, vp, vp]
     lib.c6_softmax_sample.restype = i32
@@ -305,6 +317,15 @@ def check(rc: int, what: str) -> None:
 def packed_bytes(prec: int) -> int:
     n = ctypes.c_size_t(0)
     check(load().c6_packed_bytes(prec, ctypes.byref(n)), "c6_packed_bytes")
+    return int(n.value)
+
+
+def generic_packed_bytes(board: int, kernels, channels, prec: int) -> int:
+    """Bytes of one packed weight set of an architecture, 0 where it has no packed form."""
+    ints = ctypes.c_int * len(kernels)
+    n = ctypes.c_size_t(0)
+    check(load().c6_generic_packed_bytes(board, len(kernels), ints(*kernels), ints(*channels), prec, ctypes.byref(n)),
+          "c6_generic_packed_bytes")
     return int(n.value)
 
 

@@ -34,6 +34,17 @@ int launch_generic(const void *x, int x_dtype, long long batch, long long per_gr
                    float *logits, float *value, int mask_mode, const uint8_t *legal, float fill,
                    hipStream_t st);
 
+size_t small_packed_bytes(int n, int layers, const int *kernels, const int *channels, int prec);
+int launch_small_pack(long long groups, int n, int layers, const int *kernels, const int *channels,
+                      const float *const *conv_w, const float *const *conv_b, const float *pol_w, const float *pol_b,
+                      const float *val_w, const float *val_b, int prec, void *packed, size_t packed_stride,
+                      hipStream_t st);
+int launch_small(const void *x, int x_dtype, long long groups, long long per_group, int n, int layers,
+                 const int *kernels, const int *channels, const void *packed, size_t packed_stride,
+                 const float *const *conv_w, const float *const *conv_b, const float *pol_w, const float *pol_b,
+                 const float *val_w, const float *val_b, int prec, float *logits, float *value, int mask_mode,
+                 const uint8_t *legal, float fill, hipStream_t st);
+
 size_t static_scratch_bytes();
 int static_scratch(void **out);
 
@@ -414,6 +425,11 @@ static int forward_generic(const char *who, const void *x, int x_dtype, int64_t 
     return C6_EINVAL;
   }
   C6_REQUIRE_DEVICE(who);
+  // a network that fits the one-launch kernel does not need the workspace
+  if (small_packed_bytes(board, layers, kernels, channels, prec) != 0)
+    return launch_small(x, x_dtype, groups, boards_per_group, board, layers, kernels, channels, nullptr, 0, conv_w,
+                        conv_b, pol_w, pol_b, val_w, val_b, prec, logits, value, mask_mode, legal, fill,
+                        static_cast<hipStream_t>(stream));
   return launch_generic(x, x_dtype, batch, boards_per_group, board, layers, kernels, channels,
                         conv_w, conv_b, pol_w, pol_b, val_w, val_b, prec, workspace, logits, value,
                         mask_mode, legal, fill, static_cast<hipStream_t>(stream));
@@ -475,6 +491,83 @@ int c6_forward_generic_static(const void *x, int x_dtype, int64_t batch, int boa
   return c6_forward_generic(x, x_dtype, batch, board, layers, kernels, channels, conv_w, conv_b,
                             pol_w, pol_b, val_w, val_b, prec, ws, static_scratch_bytes(), logits,
                             value, mask_mode, legal, fill, stream);
+}
+
+int c6_generic_packed_bytes(int board, int layers, const int *kernels, const int *channels, int prec,
+                            size_t *bytes) {
+  if (!valid_prec(prec) || bytes == nullptr || kernels == nullptr) {
+    set_error("c6_generic_packed_bytes: bad precision mode %d, null kernels or null output", prec);
+    return C6_EINVAL;
+  }
+  const int rc = check_arch("c6_generic_packed_bytes", board, layers, kernels, channels);
+  if (rc != C6_OK) return rc;
+  *bytes = (small_packed_bytes(board, layers, kernels, channels, prec) + 15) & ~(size_t)15;
+  return C6_OK;
+}
+
+// the arguments that packing and forward share
+static int check_generic_packed(const char *who, int64_t groups, int board, int layers, const int *kernels,
+                                const int *channels, int prec, const void *packed, size_t packed_stride) {
+  size_t need = 0;
+  const int rc = c6_generic_packed_bytes(board, layers, kernels, channels, prec, &need);
+  if (rc != C6_OK) return rc;
+  if (need == 0) {
+    set_error("%s: this architecture has no packed form (c6_generic_packed_bytes is 0)", who);
+    return C6_EINVAL;
+  }
+  if (groups < 1 || groups > 65535 || packed == nullptr || !aligned16(packed) || (packed_stride & 15u) != 0 ||
+      (groups > 1 && packed_stride < need)) {
+    set_error("%s: 1 to 65535 weight sets in a 16-byte aligned buffer, a multiple of 16 bytes and at least "
+              "c6_generic_packed_bytes() apart", who);
+    return C6_EINVAL;
+  }
+  return C6_OK;
+}
+
+int c6_generic_pack(int64_t groups, int board, int layers, const int *kernels, const int *channels,
+                    const float *const *conv_w, const float *const *conv_b, const float *pol_w,
+                    const float *pol_b, const float *val_w, const float *val_b, int prec, void *packed,
+                    size_t packed_stride, void *stream) {
+  const int rc = check_generic_packed("c6_generic_pack", groups, board, layers, kernels, channels, prec, packed,
+                                      packed_stride);
+  if (rc != C6_OK) return rc;
+  if (conv_w == nullptr || pol_w == nullptr) {
+    set_error("c6_generic_pack: conv_w and pol_w must not be null");
+    return C6_EINVAL;
+  }
+  for (int l = 0; l < layers; ++l)
+    if (conv_w[l] == nullptr) {
+      set_error("c6_generic_pack: conv_w[%d] is null", l);
+      return C6_EINVAL;
+    }
+  C6_REQUIRE_DEVICE("c6_generic_pack");
+  return launch_small_pack(groups, board, layers, kernels, channels, conv_w, conv_b, pol_w, pol_b, val_w, val_b, prec,
+                           packed, packed_stride, static_cast<hipStream_t>(stream));
+}
+
+int c6_forward_generic_packed(const void *x, int x_dtype, int64_t groups, int64_t boards_per_group, int board,
+                              int layers, const int *kernels, const int *channels, const void *packed,
+                              size_t packed_stride, int prec, float *logits, float *value, int mask_mode,
+                              const uint8_t *legal, float fill, void *stream) {
+  const char *who = "c6_forward_generic_packed";
+  const int rc = check_generic_packed(who, groups, board, layers, kernels, channels, prec, packed, packed_stride);
+  if (rc != C6_OK) return rc;
+  if (elem_bytes(x_dtype) == 0 || boards_per_group < 0 ||
+      (boards_per_group > 0 && groups > 0x7fffffffLL / boards_per_group)) {
+    set_error("%s: bad input type %d or %lld x %lld boards", who, x_dtype, (long long)groups,
+              (long long)boards_per_group);
+    return C6_EINVAL;
+  }
+  if (boards_per_group == 0) return C6_OK;
+  if (x == nullptr || mask_mode < C6_MASK_NONE || mask_mode > C6_MASK_LEGAL ||
+      (mask_mode == C6_MASK_LEGAL && legal == nullptr)) {
+    set_error("%s: null input or bad mask_mode %d", who, mask_mode);
+    return C6_EINVAL;
+  }
+  C6_REQUIRE_DEVICE(who);
+  return launch_small(x, x_dtype, groups, boards_per_group, board, layers, kernels, channels, packed, packed_stride,
+                      nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, prec, logits, value, mask_mode, legal, fill,
+                      static_cast<hipStream_t>(stream));
 }
 
 int c6_mask_logits(const void *logits, const uint8_t *legal, int dtype, int64_t batch,

@@ -1,8 +1,8 @@
 // Layer-by-layer forward for ANY architecture the reference's PolicyValueNet accepts
 // (connect6/model.py:26-77: any board size, any odd kernels, any channel counts).
-// This is the compatibility path: plain direct convolution, one thread per output
-// element, activations round-tripping through a caller-provided workspace.  The fused
-// MFMA kernel in c6_forward.hip serves the default architecture.
+// Plain direct convolution, one thread per output element, activations round-tripping through a
+// caller-provided workspace: what is left for networks that fit neither the fused kernels of the
+// default architecture (c6_forward.hip) nor the one-launch kernel of small networks (c6_small.hip).
 #include <mutex>
 
 #include "c6_common.h"

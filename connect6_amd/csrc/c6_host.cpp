@@ -31,6 +31,7 @@ struct Abi {
   decltype(&c6_softmax_sample) softmax_sample;
   decltype(&c6_env_step) env_step;
   decltype(&c6_canonical_input) canonical_input;
+  decltype(&c6_forward_generic_packed) forward_generic_packed;
 } abi;
 
 PyObject *fail(PyObject *type, const std::string &what) {
@@ -251,6 +252,48 @@ PyObject *forward_boards(PyObject *, PyObject *const *a, Py_ssize_t n) {
   END_HANDLE_TH_ERRORS
 }
 
+// forward_generic(x, packed, groups, architecture, prec, want_value, mask_mode, legal, fill, stream)
+//   -> (rc, logits, value).  architecture: bytes of the C ints kernels[layers], channels[layers]
+PyObject *forward_generic(PyObject *, PyObject *const *a, Py_ssize_t n) {
+  if (n != 10) return fail(PyExc_TypeError, "forward_generic takes 10 arguments");
+  HANDLE_TH_ERRORS
+  const at::Tensor x = THPVariable_Unpack(a[0]).contiguous();
+  const at::Tensor &packed = THPVariable_Unpack(a[1]);
+  const int64_t groups = PyLong_AsLongLong(a[2]);
+  char *arch = nullptr;
+  Py_ssize_t arch_bytes = 0;
+  if (PyBytes_AsStringAndSize(a[3], &arch, &arch_bytes) != 0) return nullptr;
+  const int layers = (int)(arch_bytes / (2 * sizeof(int)));
+  const int *kernels = reinterpret_cast<const int *>(arch), *channels = kernels + layers;
+  const int prec = (int)PyLong_AsLong(a[4]), mask_mode = (int)PyLong_AsLong(a[6]);
+  const at::Tensor *legal_in = tensor_or_null(a[7]);
+  const float fill = (float)PyFloat_AsDouble(a[8]);
+  void *stream = PyLong_AsVoidPtr(a[9]);
+  if (PyErr_Occurred()) return nullptr;
+  const at::Device dev = x.device();
+  const int64_t b = x.size(0), board = x.size(3);
+  const int x_code = dtype_code(x.scalar_type());
+  if (x_code < 0)
+    return fail(PyExc_ValueError, std::string("unsupported tensor dtype ") + c10::toString(x.scalar_type()) +
+                                      "; expected float32, bfloat16 or float16");
+  at::Tensor legal, value;
+  if (legal_in != nullptr) {
+    if (legal_in->dim() != 2 || legal_in->size(0) != b || legal_in->size(1) != board * board)
+      return fail(PyExc_ValueError, "legal mask must have shape (" + std::to_string(b) + ", " +
+                                        std::to_string(board * board) + "), got " + shape_text(*legal_in));
+    legal = legal_in->to(dev).contiguous();
+  }
+  const c10::DeviceGuard guard(dev);
+  const at::Tensor logits = fresh({b, board * board}, at::kFloat, dev);
+  if (PyObject_IsTrue(a[5]) == 1) value = fresh({b}, at::kFloat, dev);
+  const int rc = abi.forward_generic_packed(
+      x.data_ptr(), x_code, groups, b / groups, (int)board, layers, kernels, channels, packed.data_ptr(),
+      (size_t)(packed.numel() / groups), prec, ptr<float>(logits), ptr<float>(value), mask_mode,
+      static_cast<const uint8_t *>(legal.defined() ? legal.data_ptr() : nullptr), fill, stream);
+  return answer<2>(rc, {logits, value});
+  END_HANDLE_TH_ERRORS
+}
+
 // mask_logits(logits, legal, stream) -> (rc, masked); the fill is the lowest finite value of the type
 PyObject *mask_logits(PyObject *, PyObject *const *a, Py_ssize_t n) {
   if (n != 3) return fail(PyExc_TypeError, "mask_logits takes 3 arguments");
@@ -355,7 +398,7 @@ PyObject *bind(PyObject *, PyObject *const *a, Py_ssize_t n) {
 #define C6_FAST(name) {#name, reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)(void)>(name)), METH_FASTCALL, nullptr}
 PyMethodDef methods[] = {C6_FAST(bind),        C6_FAST(forward),        C6_FAST(forward_boards),
                          C6_FAST(mask_logits), C6_FAST(sample),         C6_FAST(env_step),
-                         C6_FAST(canonical_input),
+                         C6_FAST(canonical_input), C6_FAST(forward_generic),
                          {"parameters", parameters, METH_O, nullptr},
                          {nullptr, nullptr, 0, nullptr}};
 PyModuleDef module_def = {PyModuleDef_HEAD_INIT, "_c6_host", nullptr, -1, methods, nullptr, nullptr, nullptr, nullptr};

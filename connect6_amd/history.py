@@ -16,7 +16,8 @@ from typing import Any
 import torch
 
 from . import _lib
-from .model import _require_device_tensor, pack_state, run_forward, run_forward_generic
+from .model import (_require_device_tensor, architecture_bytes, pack_generic, pack_state, run_forward,
+                    run_forward_generic, run_packed_generic)
 
 
 @dataclass(slots=True)
@@ -114,6 +115,8 @@ class HistoricalPolicyEnsemble:
         self.action_size = self.board_size * self.board_size
 
         self._prec = _PREC_OF_DTYPE[self.dtype] if precision is None else _lib.PREC_BY_NAME[precision]
+        self._arch: bytes | None = None     # other architectures: see _fits
+        self._has_packed = False
         self._packed: tuple | None = None   # (buffer, stream it was packed on, event)
         self._states = states
         self._stacked: dict[str, torch.Tensor | None] = {}
@@ -168,22 +171,38 @@ class HistoricalPolicyEnsemble:
         src = self._states[m]
         return {k: src[k].detach().to(device=self.device, dtype=self.dtype) for k in keys if k in src}
 
+    def _stacked_state(self) -> dict[str, torch.Tensor | None]:
+        keys = [f"convs.{i}.{kind}" for i in range(len(self.kernels)) for kind in ("weight", "bias")]
+        keys += ["policy_output.weight", "policy_output.bias"]
+        return {k: self._stacked_attr(k, optional=k.endswith("bias")) for k in keys}
+
+    def _fits(self) -> bool:
+        """Does this (non-default) architecture have a packed form?"""
+        if self._arch is None:
+            self._arch = architecture_bytes(self.kernels, self.channels)
+            self._has_packed = self.num_models <= 65535 and _lib.generic_packed_bytes(
+                self.board_size, self.kernels, self.channels, self._prec) > 0
+        return self._has_packed
+
     def _packed_weights(self) -> torch.Tensor:
-        stream = torch.cuda.current_stream(self.device)
+        stream_ptr = _lib.stream_ptr(self.device)
         if self._packed is None:
-            one = _lib.packed_bytes(self._prec)
-            buf = torch.empty((self.num_models, one), dtype=torch.uint8, device=self.device)
             # one call for all models, from the stacked tensors (rounded to `dtype`, as the
             # ensemble holds its parameters): two launches, however many models
-            keys = [f"convs.{i}.{kind}" for i in range(len(self.kernels)) for kind in ("weight", "bias")]
-            keys += ["policy_output.weight", "policy_output.bias"]
-            stacked = {k: self._stacked_attr(k, optional=k.endswith("bias")) for k in keys}
-            pack_state(stacked, self._prec, buf, groups=self.num_models)
+            stacked = self._stacked_state()
+            if self.is_default_architecture:
+                one = _lib.packed_bytes(self._prec)
+                buf = torch.empty((self.num_models, one), dtype=torch.uint8, device=self.device)
+                pack_state(stacked, self._prec, buf, groups=self.num_models)
+            else:
+                buf = pack_generic(stacked, self.board_size, self.kernels, self.channels, self._prec, self.device,
+                                   groups=self.num_models, want_value=False)
             done = torch.cuda.Event()
-            done.record(stream)
-            self._packed = (buf, stream.cuda_stream, done)
+            done.record(torch.cuda.current_stream(self.device))
+            self._packed = (buf, stream_ptr, done)
         buf, packed_on, done = self._packed
-        if packed_on != stream.cuda_stream:   # packed on another stream: wait for it, and tell the
+        if packed_on != stream_ptr:   # packed on another stream: wait for it, and tell the
+            stream = torch.cuda.current_stream(self.device)
             stream.wait_event(done)           # allocator that this stream reads the buffer too
             buf.record_stream(stream)
         return buf
@@ -214,14 +233,16 @@ class HistoricalPolicyEnsemble:
             logits, _, _, _ = run_forward(x.reshape(m * t, *expected_tail), self._packed_weights(),
                                           self._prec, m, t, want_value=False,
                                           logits_dtype=self.dtype if direct else torch.float32)
-        else:  # other architectures: layer by layer, every layer one launch for all models
-            keys = [f"convs.{i}.{kind}" for i in range(len(self.kernels)) for kind in ("weight", "bias")]
-            keys += ["policy_output.weight", "policy_output.bias"]
-            if self._stacked32 is None:   # the layer-by-layer kernels read fp32 parameters
-                self._stacked32 = {k: v.float().contiguous() for k in keys
-                                   if (v := self._stacked_attr(k, optional=k.endswith("bias"))) is not None}
-            stacked = self._stacked32
-            logits = run_forward_generic(x.reshape(m * t, *expected_tail), stacked, self.kernels, self.channels,
-                                         self._prec, want_value=False, groups=m)[0]
+        else:  # other architectures: one launch where the network has a packed form, else one per layer
+            flat = x.reshape(m * t, *expected_tail)
+            packed = self._packed_weights() if self._fits() else None
+            if packed is not None:
+                logits, _ = run_packed_generic(flat, packed, self._arch, self._prec, groups=m, want_value=False)
+            else:
+                if self._stacked32 is None:   # the layer-by-layer kernels read fp32 parameters
+                    self._stacked32 = {k: v.float().contiguous() for k, v in self._stacked_state().items()
+                                       if v is not None}
+                logits = run_forward_generic(flat, self._stacked32, self.kernels, self.channels, self._prec,
+                                             want_value=False, groups=m)[0]
         logits = logits.view(m, t, self.action_size)
         return logits if self.dtype == torch.float32 else logits.to(self.dtype)

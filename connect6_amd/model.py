@@ -218,6 +218,52 @@ def run_forward_generic(
     return logits, value
 
 
+def pack_generic(state: dict[str, torch.Tensor], board: int, kernels, channels, prec: int, device,
+                 groups: int = 1, want_value: bool = True) -> torch.Tensor | None:
+    """Weights of a non-default architecture in the one-launch kernel's layout, or None where it has
+    none.  ``groups`` > 1: ``state`` holds that many weight sets, stacked."""
+    size = _lib.generic_packed_bytes(board, kernels, channels, prec)
+    if size == 0:
+        return None
+    keep = []  # keep fp32 staging copies alive until the launch is enqueued
+
+    def dev32(key, required=True):
+        if state.get(key) is None:
+            if required:
+                raise KeyError(f"missing parameter {key}")
+            return None
+        keep.append(state[key].detach().to(device=device, dtype=torch.float32).contiguous())
+        return keep[-1].data_ptr()
+
+    layers = len(kernels)
+    ints, ptrs = ctypes.c_int * layers, ctypes.c_void_p * layers
+    conv_w = ptrs(*[dev32(f"convs.{i}.weight") for i in range(layers)])
+    conv_b = ptrs(*[dev32(f"convs.{i}.bias", required=False) for i in range(layers)])
+    heads = [dev32("policy_output.weight"), dev32("policy_output.bias", required=False)]
+    heads += [dev32(f"value_output.{kind}", required=False) if want_value else None for kind in ("weight", "bias")]
+    out = torch.empty((groups, size), dtype=torch.uint8, device=device)
+    with torch.cuda.device(out.device):
+        rc = _lib.load().c6_generic_pack(groups, board, layers, ints(*kernels), ints(*channels), conv_w, conv_b, *heads,
+                                         prec, out.data_ptr(), size, _lib.stream_ptr(out.device))
+    _lib.check(rc, "c6_generic_pack")
+    return out
+
+
+def run_packed_generic(x, packed, arch: bytes, prec: int, *, groups: int = 1, want_value: bool = True,
+                       mask_mode: int = _lib.MASK_NONE, legal=None, fill: float = _FILL_LOWEST):
+    """``c6_forward_generic_packed``: one launch.  ``arch``: see :func:`architecture_bytes`."""
+    rc, logits, value = _lib.host().forward_generic(x, packed, groups, arch, prec, want_value, mask_mode, legal, fill,
+                                                    _lib.stream_ptr(x.device))
+    if rc != 0:
+        _lib.check(rc, "c6_forward_generic_packed")
+    return logits, value
+
+
+def architecture_bytes(kernels, channels) -> bytes:
+    """Kernel sizes and channel counts as the native host side takes them."""
+    return bytes((ctypes.c_int * (2 * len(kernels)))(*kernels, *channels))
+
+
 class PolicyValueNet(nn.Module):
     """Fully convolutional policy + value network for Connect6
     (reference: connect6/model.py:9-111).
@@ -276,6 +322,8 @@ class PolicyValueNet(nn.Module):
             raise ValueError("channel counts must be positive")
         self.kernels = kernels
         self.channels = channels
+        self._default_architecture = (self.board_size == 19 and kernels == self.DEFAULT_KERNELS
+                                      and channels == self.DEFAULT_CHANNELS)
 
         convs = []
         cin = self.input_channels
@@ -293,6 +341,8 @@ class PolicyValueNet(nn.Module):
         self.cascade_threshold: float | None = None   # None: _lib.CASCADE_THRESHOLD
         self.cascade_stats: dict = {}                 # "second_pass": boards evaluated twice (last call)
         self._packed: dict[int, tuple] = {}
+        self._arch: bytes | None = None               # other architectures: see _generic
+        self._fits: dict[int, bool] = {}
         self._epoch = 0
         self.register_load_state_dict_post_hook(lambda module, _keys: module.refresh_weights())
 
@@ -314,11 +364,7 @@ class PolicyValueNet(nn.Module):
     # -- precision / weights ------------------------------------------------
     @property
     def is_default_architecture(self) -> bool:
-        return (
-            self.board_size == 19
-            and self.kernels == self.DEFAULT_KERNELS
-            and self.channels == self.DEFAULT_CHANNELS
-        )
+        return self._default_architecture
 
     def resolve_precision(self) -> int:
         if self.precision is not None:
@@ -364,8 +410,11 @@ class PolicyValueNet(nn.Module):
                 # memory could be handed out again while a forward here still reads it
                 buf.record_stream(stream)
             return buf
-        buf = torch.empty(_lib.packed_bytes(prec), dtype=torch.uint8, device=dev)
-        pack_state({k: v for k, v in self.state_dict().items()}, prec, buf)
+        if self.is_default_architecture:
+            buf = torch.empty(_lib.packed_bytes(prec), dtype=torch.uint8, device=dev)
+            pack_state({k: v for k, v in self.state_dict().items()}, prec, buf)
+        else:
+            buf = pack_generic(self.state_dict(), self.board_size, self.kernels, self.channels, prec, dev)
         done = torch.cuda.Event()
         done.record(torch.cuda.current_stream(dev))
         self._packed[prec] = (self._epoch, key, buf, stream_ptr, done)
@@ -392,10 +441,17 @@ class PolicyValueNet(nn.Module):
             )
 
     def _generic(self, x, prec, **kw):
-        """Non-default architectures run layer by layer (``c6_forward_generic``)."""
-        if int(x.shape[0]) == 0:
+        """Non-default architectures: one launch from packed weights where the network has that
+        form, else layer by layer (``c6_forward_generic``)."""
+        if x.shape[0] == 0:
             return (torch.empty((0, self.action_size), dtype=torch.float32, device=x.device),
                     torch.empty((0,), dtype=torch.float32, device=x.device))
+        if self._arch is None:
+            self._arch = architecture_bytes(self.kernels, self.channels)
+            self._fits = {p: _lib.generic_packed_bytes(self.board_size, self.kernels, self.channels, p) > 0
+                          for p in _lib.PREC_BY_NAME.values()}
+        if self._fits[prec]:
+            return run_packed_generic(x, self.packed_weights(prec), self._arch, prec, **kw)
         return run_forward_generic(x, self.state_dict(), self.kernels, self.channels, prec, **kw)
 
     def forward(self, x: torch.Tensor) -> tuple[torch.Tensor, torch.Tensor]:

@@ -175,9 +175,9 @@ int c6_forward_boards_cascade(const int8_t *boards, const int8_t *player,
                               size_t workspace_bytes, void *stream);
 
 /* Forward of ONE weight set for any architecture the reference's PolicyValueNet accepts
- * (connect6/model.py:26-77: any board size, odd kernels, positive channel counts), layer by
- * layer through a caller-provided workspace.  Compatibility path for non-default
- * architectures (the reference's own tests use board 5, kernels 3,3,3, channels 8,8,16);
+ * (connect6/model.py:26-77: any board size, odd kernels, positive channel counts): in one launch
+ * where c6_generic_packed_bytes is not 0, else layer by layer through a caller-provided
+ * workspace.  For non-default architectures (the reference's own tests use board 5, kernels 3,3,3, channels 8,8,16);
  * the default architecture should use c6_forward.
  *   x        device [B,3,n,n] of element type x_dtype
  *   kernels, channels: HOST arrays of `layers` ints
@@ -229,6 +229,25 @@ int c6_forward_generic_static(const void *x, int x_dtype, int64_t batch, int boa
                               const float *pol_w, const float *pol_b, const float *val_w,
                               const float *val_b, int prec, float *logits, float *value,
                               int mask_mode, const uint8_t *legal, float fill, void *stream);
+
+/* The same forward from weights packed once, in one launch: for architectures that fit one
+ * workgroup's LDS and accumulators (at most 48 channels, a board of at most 19 x 19 whose padded
+ * activations fit 160 KiB); c6_generic_packed_bytes gives 0 for the others, which c6_forward_generic
+ * serves.  Results are those of c6_forward_generic, bit for bit.
+ *   bytes    of one weight set (a multiple of 16)
+ *   packed   device, `groups` sets packed_stride bytes apart; conv_w ... val_b as in
+ *            c6_forward_generic_grouped; board b uses set b / boards_per_group */
+int c6_generic_packed_bytes(int board, int layers, const int *kernels, const int *channels, int prec,
+                            size_t *bytes);
+int c6_generic_pack(int64_t groups, int board, int layers, const int *kernels, const int *channels,
+                    const float *const *conv_w, const float *const *conv_b, const float *pol_w,
+                    const float *pol_b, const float *val_w, const float *val_b, int prec, void *packed,
+                    size_t packed_stride, void *stream);
+int c6_forward_generic_packed(const void *x, int x_dtype, int64_t groups, int64_t boards_per_group,
+                              int board, int layers, const int *kernels, const int *channels,
+                              const void *packed, size_t packed_stride, int prec, float *logits,
+                              float *value, int mask_mode, const uint8_t *legal, float fill,
+                              void *stream);
 
 /* Out-of-place occupied-square masking of existing logits.
  * Replaces: mask_logits (connect6/model.py:123-125).

@@ -1,0 +1,83 @@
+"""One-launch forward of small networks (c6_forward_generic_packed) against the oracle, at the sizes
+where its layout changes: boards of one square to 19 x 19, channels around multiples of 8 and 16,
+wide and 1x1 kernels, one to many boards per workgroup, several weight sets."""
+import pytest
+import torch
+
+import connect6_amd as c6
+from connect6_amd import _lib
+from connect6_amd.model import pack_generic, run_forward_generic, run_packed_generic, architecture_bytes
+from oracle import torch_ref as R
+from tests.util import rel_l2
+
+pytestmark = pytest.mark.gpu
+
+
+def _inputs(batch, board, seed):
+    x = torch.randn(batch, 3, board, board, generator=torch.Generator().manual_seed(seed))
+    x[:, :2] = (x[:, :2] > 0.7).float()
+    return x
+
+
+@pytest.mark.parametrize("board,kernels,channels,batch", [
+    (1, [1], [1], 70), (2, [3, 1], [8, 9], 33), (5, [3, 3, 3], [8, 8, 16], 1), (5, [3, 3, 3], [8, 8, 16], 3000),
+    (7, [7, 5], [17, 48], 300), (9, [5, 3, 3], [16, 32, 32], 1024), (9, [5, 3, 3], [16, 32, 32], 2),
+    (11, [11, 1, 3], [33, 7, 40], 65), (13, [3, 3, 5, 1], [24, 32, 16, 47], 301), (19, [3, 3], [32, 48], 5),
+    (19, [7, 3, 3], [32, 32, 32], 259),
+])
+def test_fits_and_matches_the_oracle(cuda, board, kernels, channels, batch):
+    st = R.init_state(7, "torch_default", kernels=kernels, channels=channels)
+    model = c6.PolicyValueNet(board_size=board, kernels=kernels, channels=channels).to(cuda).eval()
+    model.load_state_dict(st)
+    assert _lib.generic_packed_bytes(board, kernels, channels, _lib.PREC_F32) > 0
+    x = _inputs(batch, board, 3)
+    xd = x.to(cuda)
+    legal = ((x[:, 0] == 0) & (x[:, 1] == 0)).flatten(1)
+    dev_state = {k: v.to(cuda) for k, v in st.items()}
+    with torch.inference_mode():
+        lo, vo = R.forward(st, x)
+        lg, vg = model(xd)
+        # fp32 sums of at most 9 x 48 x 9 products and sigmoids to 2^-22: the oracle's own order of
+        # summation moves these networks by 1e-6
+        assert rel_l2(lg, lo) <= 5e-6 and rel_l2(vg, vo) <= 5e-6
+        # the same weights straight from the tensors: the same values, bit for bit
+        lr, vr = run_forward_generic(xd, dev_state, kernels, channels, _lib.PREC_F32)
+        assert torch.equal(lg, lr) and torch.equal(vg, vr)
+        # a board's result does not depend on how many share its workgroup
+        one, vone = model(xd[batch - 1:])
+        assert torch.equal(one, lg[batch - 1:]) and torch.equal(vone, vg[batch - 1:])
+        lm, _ = model.forward_masked(xd, legal.to(cuda))
+        assert torch.equal(lm.cpu(), R.mask_logits(lg.cpu(), legal))
+        for name, tol in (("bf16", 2e-3), ("fp16", 2e-3)):
+            model.precision = name
+            lb, _ = model(xd)
+            want = R.forward_bf16_emulated(st, x)[0] if name == "bf16" else lo
+            # bf16: the emulation's roundings in another order of summation (a few fall the other way);
+            # fp16: half an ulp (2^-12) at every operand of two to four layers
+            assert rel_l2(lb, want) <= tol, (name, rel_l2(lb, want))
+
+
+def test_weight_sets_and_an_architecture_without_packed_form(cuda):
+    board, kernels, channels = 9, [3, 3], [16, 24]
+    states = [R.init_state(20 + i, "torch_default", kernels=kernels, channels=channels) for i in range(3)]
+    stacked = {k: torch.stack([s[k] for s in states]).to(cuda) for k in states[0]}
+    x = _inputs(3 * 11, board, 5).to(cuda)
+    arch = architecture_bytes(kernels, channels)
+    for prec in (_lib.PREC_F32, _lib.PREC_BF16C, _lib.PREC_BF16, _lib.PREC_F16):
+        packed = pack_generic(stacked, board, kernels, channels, prec, cuda, groups=3)
+        lg, vg = run_packed_generic(x, packed, arch, prec, groups=3)
+        lr, vr = run_forward_generic(x, stacked, kernels, channels, prec, groups=3)
+        assert torch.equal(lg, lr) and torch.equal(vg, vr)
+        for i in range(3):
+            one, v1 = run_packed_generic(x[11 * i:11 * i + 11], packed[i:i + 1], arch, prec)
+            assert torch.equal(one, lg[11 * i:11 * i + 11]) and torch.equal(v1, vg[11 * i:11 * i + 11])
+    for kernels, channels in (([3], [49]), ([3, 7], [48, 8])):   # too many channels; too large for the LDS
+        assert _lib.generic_packed_bytes(19, kernels, channels, _lib.PREC_F32) == 0
+        st = R.init_state(3, "torch_default", kernels=kernels, channels=channels)
+        model = c6.PolicyValueNet(board_size=19, kernels=kernels, channels=channels).to(cuda).eval()
+        model.load_state_dict(st)
+        xb = _inputs(4, 19, 9)
+        with torch.inference_mode():
+            lo, vo = R.forward(st, xb)
+            lg, vg = model(xb.to(cuda))
+        assert rel_l2(lg, lo) <= 5e-6 and rel_l2(vg, vo) <= 5e-6

@@ -19,13 +19,14 @@ _CSRC = _PKG / "csrc"
 _LIBDIR = _PKG / "lib"
 _SO = _LIBDIR / "libconnect6_amd.so"
 _SOURCES = ("c6_forward.hip", "c6_tail.hip", "c6_generic.hip", "c6_small.hip", "c6_env.hip", "c6_api.hip")
-_MODES = ("PrecF32", "PrecBF16", "PrecF16", "PrecBF16F6", "PrecBF16F6W")   # of c6_forward.hip
+_MODES = ("PrecF32", "PrecF32S", "PrecBF16", "PrecF16", "PrecBF16F6", "PrecBF16F6W")   # of c6_forward.hip
 _RESOURCES = _LIBDIR / "resource_usage.txt"   # registers, scratch and LDS of every kernel, written by build()
 
 # arithmetic modes (include/connect6_amd.h)
 PREC_F32, PREC_BF16, PREC_F16, PREC_BF16F6, PREC_BF16C, PREC_BF16F6W, PREC_BF16C6 = 0, 1, 2, 3, 4, 5, 6
 PREC_BY_NAME = {"fp32": PREC_F32, "bf16": PREC_BF16, "fp16": PREC_F16, "bf16f6": PREC_BF16F6, "bf16c": PREC_BF16C,
                 "bf16f6w": PREC_BF16F6W, "bf16c6": PREC_BF16C6}
+PREC_F32S = 7   # how fp32 runs for the default architecture (see kernel_prec)
 CASCADES = (PREC_BF16C, PREC_BF16C6)   # the modes that go through the cascade entry points
 # cascade mode: a board is evaluated a second time (low parts of activations and weights carried) when its best free
 # square leads the second best by less than this many standard deviations of its logits, or two
@@ -312,6 +313,12 @@ def check(rc: int, what: str) -> None:
     if rc == -1:
         raise ValueError(f"{what}: {msg}")
     raise C6Error(f"{what}: {msg} (code {rc})")
+
+
+def kernel_prec(prec: int) -> int:
+    """The mode whose kernel and packed weights serve ``prec`` in the default architecture: fp32
+    operands go through the bf16 matrix cores as three exact parts each."""
+    return PREC_F32S if prec == PREC_F32 else prec
 
 
 def packed_bytes(prec: int) -> int:

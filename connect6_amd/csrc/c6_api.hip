@@ -89,7 +89,7 @@ static int device_ok(const char *who) {
 
 static bool aligned16(const void *p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
 static int elem_bytes(int dt) { return dt == C6_DT_F32 ? 4 : ((dt == C6_DT_BF16 || dt == C6_DT_F16) ? 2 : 0); }
-static bool valid_prec(int p) { return p >= C6_PREC_F32 && p <= C6_PREC_BF16C6; }
+static bool valid_prec(int p) { return p >= C6_PREC_F32 && p <= C6_PREC_F32S; }
 
 // the cascade's workspace argument, checked; `who` names the entry point in the message
 static int check_cascade_workspace(const char *who, long long boards, const void *workspace, size_t bytes) {

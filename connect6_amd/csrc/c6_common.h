@@ -112,6 +112,17 @@ struct PrecBF16F6W {
   static constexpr int LO_MASK = 0xfe;
 };
 
+// fp32 on the bf16 matrix cores: every weight is the exact sum of three bf16 values (8 mantissa bits
+// each), packed as three fragments that follow one another; so is every activation.  c6_split.h.
+struct PrecF32S {
+  static constexpr int WLO = 2;
+  static constexpr int PIPE = 0;      // weights packed tap-major
+  static constexpr int ID = C6_PREC_F32S;
+  static constexpr int EB = 2;
+  static constexpr int LO6 = 0;
+  static constexpr int LO_MASK = 0;
+};
+
 // bf16 + fp6 mode: what rounding an activation to bf16 drops (|lo| <= 2^-9 |a|) is contracted
 // with an e2m3 copy of the weights in a second pass of v_mfma_scale_f32_32x32x64_f8f6f4 (K = 64
 // per instruction at four times the bf16 rate).  The weight copy of layer l is scaled by 2^sw[l]
@@ -136,7 +147,7 @@ template <class P> struct Geo {
   static constexpr int EB = P::EB;
   static constexpr int E = 16 / EB;                 // elements per 16-byte fragment lane
   static constexpr int KSTEP = 2 * E;               // K elements contracted per fragment pair
-  static constexpr int W = P::WLO ? 2 : 1;          // weight fragments per (k-step, cout tile): hi, or hi then lo
+  static constexpr int W = 1 + P::WLO;               // weight fragments per (k-step, cout tile): hi, what its rounding dropped, ...
   static constexpr int PLANE = kChSlots * EB;       // bytes of one precision plane of a position
   static constexpr int LO_OFF = PLANE;              // the fp6 blocks follow the bf16 plane
   static constexpr int RECB = PLANE + (P::LO6 ? kChSlots : 0);  // payload bytes
@@ -205,7 +216,7 @@ template <class P> struct Geo {
   static constexpr int FAST1_STREAM = FAST1_STEPS * W;   // fragments of that copy
   static constexpr int PLANE2_FRAG_OFF = FAST1_OFF + FAST1_STREAM + 8;  // (8 zero fragments: over-read)
   static constexpr int PLANE2_FRAGS = kWaves * 3 * 4;
-  static constexpr int FAST1_FRAGS = (P::PIPE && EB == 2) ? FAST1_STREAM + 8 + PLANE2_FRAGS : 0;
+  static constexpr int FAST1_FRAGS = EB == 2 ? FAST1_STREAM + 8 + PLANE2_FRAGS : 0;
   static constexpr int TOTAL_FRAGS = HI_FRAGS + LO_FRAGS + FAST1_FRAGS;
   static constexpr size_t TAIL_OFF = (size_t)TOTAL_FRAGS * 1024;  // fp32 tail: biases, heads
   // tail words: bias[544] polw[96] valw[96] polb valb pad pad, then 8 ints sw[layer]

@@ -1904,6 +1904,12 @@ __global__ __launch_bounds__(256) void fused_forward_kernel(const FwdParams prm)
   }
 }
 
+}  // namespace c6
+
+#include "c6_split.h"
+
+namespace c6 {
+
 #ifdef C6_TRACE
 extern "C" int c6_debug_trace(long long *host_out) {
   return (int)hipMemcpyFromSymbol(host_out, HIP_SYMBOL(g_trace), sizeof(long long) * 256 * 4 * 64);
@@ -1927,9 +1933,9 @@ template <class P> __device__ __forceinline__ float weight_part(float v, int par
   if constexpr (P::EB == 4) {
     return v;
   } else {
-    const float hi = __builtin_bit_cast(float, (unsigned)bits16<P>(v) << 16);
     static_assert(P::WLO == 0 || P::ID != C6_PREC_F16, "the low part is defined for bf16 storage");
-    return part ? v - hi : v;
+    for (int i = 0; i < part; ++i) v -= __builtin_bit_cast(float, (unsigned)bits16<P>(v) << 16);
+    return v;
   }
 }
 
@@ -2168,20 +2174,23 @@ template <class P> int launch_pack(const PackParams &pp, hipStream_t st) {
 
 template <class P> int launch_forward(const FwdParams &fp, hipStream_t st) {
   using G = Geo<P>;
-  static_assert(G::LDS_BYTES <= 160 * 1024, "activation tile must fit the 160 KiB LDS of a CU");
+  constexpr int LDS = P::ID == C6_PREC_F32S ? SplitGeo::LDS_BYTES : G::LDS_BYTES;
+  static_assert(LDS <= 160 * 1024, "activation tile must fit the 160 KiB LDS of a CU");
   int dev = 0;
   hipError_t e = hipGetDevice(&dev);
   static thread_local int configured_dev = -1;
   static thread_local int cus = 0;
   const void *kernel;
-  if constexpr (P::PIPE) {
+  if constexpr (P::ID == C6_PREC_F32S) {
+    kernel = reinterpret_cast<const void *>(&split_forward_kernel<P>);
+  } else if constexpr (P::PIPE) {
     kernel = reinterpret_cast<const void *>(&fused_pipe_kernel<P>);
   } else {
     kernel = reinterpret_cast<const void *>(&fused_forward_kernel<P>);
   }
   if (e == hipSuccess && configured_dev != dev) {
     e = hipFuncSetAttribute(kernel,
-                            hipFuncAttributeMaxDynamicSharedMemorySize, G::LDS_BYTES);
+                            hipFuncAttributeMaxDynamicSharedMemorySize, LDS);
     int n = 0;
     if (e == hipSuccess) e = hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev);
     if (e == hipSuccess) {
@@ -2195,10 +2204,12 @@ template <class P> int launch_forward(const FwdParams &fp, hipStream_t st) {
   }
   long long grid = cus > 0 ? cus : 256;
   if (grid > fp.total_boards) grid = fp.total_boards;
-  if constexpr (P::PIPE) {
-    hipLaunchKernelGGL(fused_pipe_kernel<P>, dim3((unsigned)grid), dim3(256), G::LDS_BYTES, st, fp);
+  if constexpr (P::ID == C6_PREC_F32S) {
+    hipLaunchKernelGGL(split_forward_kernel<P>, dim3((unsigned)grid), dim3(256), LDS, st, fp);
+  } else if constexpr (P::PIPE) {
+    hipLaunchKernelGGL(fused_pipe_kernel<P>, dim3((unsigned)grid), dim3(256), LDS, st, fp);
   } else {
-    hipLaunchKernelGGL(fused_forward_kernel<P>, dim3((unsigned)grid), dim3(256), G::LDS_BYTES, st, fp);
+    hipLaunchKernelGGL(fused_forward_kernel<P>, dim3((unsigned)grid), dim3(256), LDS, st, fp);
   }
   e = hipGetLastError();
   if (e != hipSuccess) {
@@ -2225,6 +2236,7 @@ int dispatch_pack(int prec, const PackParams &pp, hipStream_t st) {
   }
   switch (prec) {
     case C6_PREC_F32: return launch_pack<PrecF32>(pp, st);
+    case C6_PREC_F32S: return launch_pack<PrecF32S>(pp, st);
     case C6_PREC_BF16: return launch_pack<PrecBF16>(pp, st);
     case C6_PREC_F16: return launch_pack<PrecF16>(pp, st);
     case C6_PREC_BF16F6: return launch_pack<PrecBF16F6>(pp, st);
@@ -2237,6 +2249,7 @@ int dispatch_pack(int prec, const PackParams &pp, hipStream_t st) {
 int dispatch_forward(int prec, const FwdParams &fp, hipStream_t st) {
   switch (prec) {
     case C6_PREC_F32: return launch_forward<PrecF32>(fp, st);
+    case C6_PREC_F32S: return launch_forward<PrecF32S>(fp, st);
     case C6_PREC_BF16: return launch_forward<PrecBF16>(fp, st);
     case C6_PREC_F16: return launch_forward<PrecF16>(fp, st);
     case C6_PREC_BF16F6: return launch_forward<PrecBF16F6>(fp, st);
@@ -2302,6 +2315,7 @@ size_t packed_bytes(int prec) {
   if (is_cascade(prec)) return cascade_packed_bytes(prec);
   switch (prec) {
     case C6_PREC_F32: return Geo<PrecF32>::PACKED_BYTES;
+    case C6_PREC_F32S: return Geo<PrecF32S>::PACKED_BYTES;
     case C6_PREC_BF16: return Geo<PrecBF16>::PACKED_BYTES;
     case C6_PREC_F16: return Geo<PrecF16>::PACKED_BYTES;
     case C6_PREC_BF16F6: return Geo<PrecBF16F6>::PACKED_BYTES;

@@ -162,7 +162,7 @@ int launch_generic(const void *x, int x_dtype, long long batch, long long per_gr
                    static_cast<float *>(workspace) + (size_t)batch * cmax * n * n};
   // arithmetic contract of each mode: which operands are rounded to 16 bits
   // (C6_PREC_BF16F6W carries the weights' low part as well: nothing is rounded)
-  const int round_w = (prec == C6_PREC_F32 || prec == C6_PREC_BF16F6W)
+  const int round_w = (prec == C6_PREC_F32 || prec == C6_PREC_F32S || prec == C6_PREC_BF16F6W)
                           ? C6_DT_F32
                           : (prec == C6_PREC_F16 ? C6_DT_F16 : C6_DT_BF16);
   // (the hi+lo modes carry the activations' low-order bits: no activation rounding here)

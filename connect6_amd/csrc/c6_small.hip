@@ -479,6 +479,7 @@ enum : int { kSmallF32, kSmallW16, kSmallBF16, kSmallF16 };
 static int small_arith(int prec) {
   switch (prec) {
     case C6_PREC_F32:
+    case C6_PREC_F32S:
     case C6_PREC_BF16F6W: return kSmallF32;
     case C6_PREC_BF16: return kSmallBF16;
     case C6_PREC_F16: return kSmallF16;

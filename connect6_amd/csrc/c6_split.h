@@ -1,0 +1,504 @@
+// fp32 forward on the bf16 matrix cores (included by c6_forward.hip, whose weight rings, first-layer
+// loops and board mapping it shares).
+//
+// Every fp32 operand is the exact sum of three bf16 values: hi = bf16(v), mid = bf16(v - hi),
+// lo = v - hi - mid (8 mantissa bits each, both differences exact).  A product is then nine products
+// of bf16 values, each exact in fp32; the six down to 2^-17 of the largest are accumulated in fp32,
+// the other three are below 2^-25 of it, less than the rounding of one fp32 addition.  Against the
+// fp32 instructions (157 TFLOP/s, 432 roundings of the running sum per output of the last layer) six
+// bf16 ones at sixteen times the rate take 3/8 of the time, with 54 roundings.
+//
+// What bounds it: the matrix cores, 383 k cycles per board with the 1,890 MFMAs of the 3x3 layers
+// six times and the first layer's 207 three times (0/1 inputs are exact in one bf16 value).  The
+// activations of up to 64 channels lie in LDS as their three planes, split once when a layer writes
+// them; 96 channels only fit as fp32 (421 positions x 384 bytes are the CU's whole LDS), and the two
+// layers that read them split them in registers, 44 instructions for eight values, a few behind each
+// MFMA.
+//
+// As in the 16-bit modes all activations carry the factor -log2(e), so that SiLU is
+// u / (1 + 2^u).
+#pragma once
+
+namespace c6 {
+
+template <> __device__ __forceinline__ void mma<PrecF32S>(const v4i &a, const v4i &b, f32x16 &c) {
+  mma<PrecBF16>(a, b, c);
+}
+
+struct SplitGeo {
+  using G = Geo<PrecF32S>;                     // weight stream and first-layer geometry
+  static constexpr int PIXB = 384;             // 3 planes x 64 channels x 2 bytes, or 96 x 4
+  static constexpr int PLANEB = 128;
+  static constexpr int ACT_BYTES = kPos * PIXB;
+  static constexpr int OCC_OFF = ACT_BYTES;
+  static constexpr int LGT_OFF = OCC_OFF + 384;
+  static constexpr int RED_OFF = LGT_OFF + 1456;
+  static constexpr int LDS_BYTES = RED_OFF + 64;
+  static_assert(G::COPIES_BYTES <= ACT_BYTES && LDS_BYTES <= 160 * 1024, "LDS map");
+};
+
+// 16-byte granule XOR of a position: sixteen consecutive positions read sixteen bank groups
+__device__ __forceinline__ int split_swz(int pos) { return ((pos >> 1) & 7) << 4; }
+
+// u / (1 + 2^u), the reciprocal with one Newton step.  (Clamped where 1 + 2^u leaves fp32: the
+// result is then below 2^-126 |u|.)
+__device__ __forceinline__ float split_silu(float u) {
+  const float d = fminf(1.0f + __builtin_amdgcn_exp2f(u), 0x1p126f);
+  const float r = __builtin_amdgcn_rcpf(d);
+  return u * fmaf(r, fmaf(-d, r, 1.0f), r);
+}
+
+// The next bf16 plane of a pair of values, which keep what it leaves out.
+__device__ __forceinline__ int split_take(float &a, float &b) {
+  const int w = pack2<PrecBF16>(a, b);
+  a -= __builtin_bit_cast(float, w << 16);
+  b -= __builtin_bit_cast(float, w & (int)0xffff0000);
+  return w;
+}
+
+// SiLU and store of one layer's outputs in the form the next one reads.
+template <int NT, bool PLANES>
+__device__ __forceinline__ void split_store(unsigned char *smem, const int (&ci)[3], int h, const f32x16 (&acc)[NT][3]) {
+#pragma unroll
+  for (int j = 0; j < 3; ++j) {
+    int pos = ci[j];
+    asm volatile("" : "+v"(pos));  // (addresses formed here, not kept for the whole kernel)
+    const int at = pos * SplitGeo::PIXB, sw = split_swz(pos);
+#pragma unroll
+    for (int t = 0; t < NT; ++t)
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        float v[4];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) v[e] = split_silu(acc[t][j][4 * q + e]);
+        if constexpr (PLANES) {
+          unsigned char *p = smem + at + ((64 * t + 16 * q) ^ sw) + 8 * h;
+#pragma unroll
+          for (int i = 0; i < 3; ++i) {
+            const int a = i < 2 ? split_take(v[0], v[1]) : pack2<PrecBF16>(v[0], v[1]);
+            const int b = i < 2 ? split_take(v[2], v[3]) : pack2<PrecBF16>(v[2], v[3]);
+            *reinterpret_cast<v2i *>(p + i * SplitGeo::PLANEB) = v2i{a, b};
+          }
+        } else {
+          *reinterpret_cast<f32x4 *>(smem + at + 128 * t + ((32 * q + 16 * h) ^ sw)) = f32x4{v[0], v[1], v[2], v[3]};
+        }
+      }
+  }
+}
+
+// Weight ring of a 3x3 layer: DEPTH k-steps of all cout tiles and planes.  A k-step of NT tiles is
+// 18 NT MFMAs, 576 NT cycles; a slot is refilled behind its last use, so depth 1 already asks 1,150
+// cycles ahead with three tiles.
+template <int L> struct SplitRing {
+  static constexpr int NT = kCoutArr[L] / 32, DEPTH = NT == 3 ? 1 : 2;
+};
+template <int L> using SplitWeights = v4i[SplitRing<L>::DEPTH][kCoutArr[L] / 32][3];
+
+template <int L> __device__ __forceinline__ void split_preload(SplitWeights<L> &ring, const WFrags &wl) {
+#pragma unroll
+  for (int d = 0; d < SplitRing<L>::DEPTH; ++d)
+#pragma unroll
+    for (int t = 0; t < SplitRing<L>::NT; ++t)
+#pragma unroll
+      for (int i = 0; i < 3; ++i) ring[d][t][i] = wl[(d * SplitRing<L>::NT + t) * 3 + i];
+}
+
+// The contraction of 3x3 layer L.  K runs over taps, then 16 channels at a time; each k-step is
+// 18 MFMAs per cout tile: six products (smallest first) of three pixel tiles.  Behind each MFMA at
+// most one LDS read of the next k-step's activations, one weight load, and (96 input channels) a few
+// instructions of their split.
+template <int L>
+__device__ __forceinline__ void split_conv(const unsigned char *smem, const WFrags &wl, SplitWeights<L> &ring,
+                                           const int (&ci)[3], int h, f32x16 (&acc)[kCoutArr[L] / 32][3]) {
+  constexpr int CIN = kCinArr[L], NT = kCoutArr[L] / 32, KC = CIN / 16, D = SplitRing<L>::DEPTH;
+  constexpr bool WIDE = CIN == 96;   // activations arrive as fp32
+  static_assert(KC % 2 == 0 && KC % D == 0, "double buffers must line up across taps");
+  int pb[3], xo[3];
+  auto set_tap = [&](int tap) __attribute__((always_inline)) {
+    const int ky = tap / 3, kx = tap - 3 * ky;
+#pragma unroll
+    for (int j = 0; j < 3; ++j) {
+      const int pos = ci[j] + (ky - 1) * kPitch + (kx - 1);
+      pb[j] = pos * SplitGeo::PIXB;
+      xo[j] = (WIDE ? h << 5 : h << 4) ^ split_swz(pos);
+    }
+  };
+  v4i bq[2][3][3];         // planes of a k-step's activations, [parity][pixel tile][plane]
+  f32x4 raw[2][3][2];      // WIDE: the same as fp32, one k-step further ahead
+  // part i of pixel tile j of channels 16 c ...: a plane, or (WIDE) four of the eight channels
+  auto read = [&](int c, int par, int j, int i) __attribute__((always_inline)) {
+    if constexpr (WIDE) {
+      if (i < 2)
+        raw[par][j][i] = *reinterpret_cast<const f32x4 *>(smem + pb[j] + (c >> 1) * 128 + (xo[j] ^ ((c & 1) * 64 + i * 16)));
+    } else {
+      bq[par][j][i] = *reinterpret_cast<const v4i *>(smem + pb[j] + (xo[j] ^ (c * 32)) + i * SplitGeo::PLANEB);
+    }
+  };
+  float rest[2];
+  auto split_a = [&](int par, int pair) __attribute__((always_inline)) {  // hi of the pair, and what it leaves
+    const int j = pair / 4, e = pair % 4;
+    rest[0] = raw[par][j][e >> 1][(e & 1) * 2];
+    rest[1] = raw[par][j][e >> 1][(e & 1) * 2 + 1];
+    bq[par][j][0][e] = split_take(rest[0], rest[1]);
+  };
+  auto split_b = [&](int par, int pair) __attribute__((always_inline)) {
+    const int j = pair / 4, e = pair % 4;
+    bq[par][j][1][e] = split_take(rest[0], rest[1]);
+    bq[par][j][2][e] = pack2<PrecBF16>(rest[0], rest[1]);
+  };
+  set_tap(0);
+#pragma unroll
+  for (int j = 0; j < 3; ++j)
+#pragma unroll
+    for (int i = 0; i < 3; ++i) read(0, 0, j, i);
+  if constexpr (WIDE) {
+#pragma unroll
+    for (int j = 0; j < 3; ++j)
+#pragma unroll
+      for (int i = 0; i < 2; ++i) read(1, 1, j, i);
+#pragma unroll
+    for (int p = 0; p < 12; ++p) {
+      split_a(0, p);
+      split_b(0, p);
+    }
+  }
+  constexpr int AHEAD = WIDE ? 2 : 1;
+#pragma unroll 1
+  for (int tap = 0; tap < 9; ++tap) {
+    const WFrags wn = wl + (tap * KC + D) * NT * 3;
+    static_for<0, KC>([&](auto uc) __attribute__((always_inline)) {
+      constexpr int u = decltype(uc)::value, par = u & 1;
+      // (after the last tap this wraps to the first: harmless extra reads)
+      if constexpr (u + AHEAD == KC) set_tap(tap == 8 ? 0 : tap + 1);
+      static_for<0, NT * 18>([&](auto gc) __attribute__((always_inline)) {
+        constexpr int g = decltype(gc)::value, t = g / 18, m = (g % 18) / 3, j = g % 3;
+        constexpr int WP[6] = {0, 1, 2, 0, 1, 0}, AP[6] = {2, 1, 0, 1, 0, 0};
+        mma<PrecBF16>(ring[u % D][t][WP[m]], bq[par][j][AP[m]], acc[t][j]);
+        if constexpr (WIDE) {
+          // raw[par] was split during the k-step before: free for the k-step after next
+          if constexpr (g >= 1 && g < 7) read((u + 2) % KC, par, (g - 1) / 2, (g - 1) % 2);
+          if constexpr (g % 4 == 0 && g / 4 < 12) split_a(par ^ 1, g / 4);
+          if constexpr (g % 4 == 2 && g / 4 < 12) split_b(par ^ 1, g / 4);
+        } else {
+          if constexpr (g < 9) read((u + 1) % KC, par ^ 1, g / 3, g % 3);
+        }
+        // a plane's fragment after its last use in the tile: 2 after product 2, 1 after 4, 0 after 5
+        if constexpr (j == 2 && m == 2) ring[u % D][t][2] = wn[(u * NT + t) * 3 + 2];
+        if constexpr (j == 2 && m == 4) ring[u % D][t][1] = wn[(u * NT + t) * 3 + 1];
+        if constexpr (j == 2 && m == 5) ring[u % D][t][0] = wn[(u * NT + t) * 3];
+        __builtin_amdgcn_sched_barrier(0);
+      });
+    });
+  }
+}
+
+// one 3x3 layer that is not the last
+template <int L>
+__device__ __forceinline__ void split_layer(unsigned char *smem, const unsigned char *packed, const float *tail,
+                                            SplitWeights<L> &ring, SplitWeights<L + 1> &next, const int (&ci)[3], int h,
+                                            int lane) {
+  constexpr int NT = kCoutArr[L] / 32;
+  f32x16 acc[NT][3];
+  init_acc(acc, tail + bias_offset(L), h);
+  split_conv<L>(smem, layer_weights<PrecF32S, L>(packed, lane), ring, ci, h, acc);
+  // (with equal widths the over-read has left the next layer's first k-steps in the ring)
+  if constexpr (kCoutArr[L + 1] != kCoutArr[L]) split_preload<L + 1>(next, layer_weights<PrecF32S, L + 1>(packed, lane));
+  __syncthreads();  // every wave has finished reading the layer's input
+  split_store<NT, kCinArr[L + 1] != 96>(smem, ci, h, acc);
+  __syncthreads();
+}
+
+// One workgroup (4 waves) per board, persistent over a contiguous run of boards, as
+// fused_forward_kernel.
+template <class P>
+__global__ __launch_bounds__(256) void split_forward_kernel(const FwdParams prm) {
+  using G = Geo<P>;
+  using S = SplitGeo;
+  extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
+  constexpr int THREADS = 256, NWAVES = THREADS / 64;
+  constexpr int ROUNDS = (kPix + THREADS - 1) / THREADS;
+  const int tid = threadIdx.x;
+  const int lane = tid & 63;
+  const int wave = tid >> 6;
+  const int h = lane >> 5;
+  auto tile_pixel = [](int t, int j, bool &ok) __attribute__((always_inline)) {
+    const int p = (t >> 6) * kPixPerWave + j * 32 + (t & 31);
+    ok = p < kPix;
+    return ok ? p : (kPix - 1);
+  };
+  int ci[3];
+#pragma unroll
+  for (int j = 0; j < 3; ++j) {
+    bool ok;
+    const int pc = tile_pixel(tid, j, ok), r = pc / kBoard;
+    ci[j] = (r + 1) * kPitch + (pc - r * kBoard + 1);
+  }
+  unsigned char *occ = smem + S::OCC_OFF;
+  float *lgt = reinterpret_cast<float *>(smem + S::LGT_OFF);
+  float *red = reinterpret_cast<float *>(smem + S::RED_OFF);
+  int *flags = reinterpret_cast<int *>(red) + 8;   // [0]: third plane varies, [1]: an input is not exact in bf16
+
+  const unsigned per_group = (unsigned)prm.boards_per_group;
+  auto packed_of = [&](long long b) { return prm.packed + (size_t)((unsigned)b / per_group) * prm.packed_stride; };
+  float xin[ROUNDS][3];
+  unsigned char occin[ROUNDS];
+  auto fetch_board = [&](long long b) {
+    int tid = threadIdx.x;
+    asm volatile("" : "+v"(tid));
+    if (prm.x_dtype == C6_DT_BOARD_I8) {
+      long long src = prm.index ? prm.index[b] : b;
+      src = src < 0 ? 0 : (src >= prm.num_states ? prm.num_states - 1 : src);
+      const int8_t *board = reinterpret_cast<const int8_t *>(prm.x) + (size_t)src * kPix;
+      const int me = prm.player[src];
+      const float last = prm.stones_left[src] == 1 ? 1.0f : 0.0f;
+#pragma unroll
+      for (int r = 0; r < ROUNDS; ++r) {
+        const int p = tid + r * THREADS;
+        if (p < kPix) {
+          const int stone = board[prm.view ? d4_from_view(p, prm.view) : p];
+          xin[r][0] = stone == me ? 1.0f : 0.0f;
+          xin[r][1] = stone == -me ? 1.0f : 0.0f;
+          xin[r][2] = last;
+          occin[r] = 0;
+        }
+      }
+      return;
+    }
+#pragma unroll
+    for (int r = 0; r < ROUNDS; ++r) {
+      const int p = tid + r * THREADS;
+      if (p < kPix) {
+#pragma unroll
+        for (int ch = 0; ch < 3; ++ch) xin[r][ch] = load_x(prm.x, prm.x_dtype, ((size_t)b * 3 + ch) * kPix + p);
+        occin[r] = prm.mask_mode == C6_MASK_LEGAL ? (prm.legal[(size_t)b * kPix + p] == 0) : 0;
+      }
+    }
+  };
+
+  // (board runs dealt out by XCD, as in fused_pipe_kernel)
+  const long long per = (prm.total_boards + gridDim.x - 1) / gridDim.x;
+  const unsigned xcds = (gridDim.x % 8 == 0) ? 8 : 1;
+  const long long run = (long long)(blockIdx.x % xcds) * (gridDim.x / xcds) + blockIdx.x / xcds;
+  long long b = run * per;
+  const long long b_end = b + per < prm.total_boards ? b + per : prm.total_boards;
+  if (b >= b_end) return;
+  v4i r1[L1Pipe<P>::D][1];
+  fetch_board(b);
+
+  for (; b < b_end; ++b) {
+    int tidv = tid;
+    asm volatile("" : "+v"(tidv));
+    const unsigned char *packed = packed_of(b);
+    const float *tail = reinterpret_cast<const float *>(packed + G::TAIL_OFF);
+    __syncthreads();  // previous board fully written out; LDS is free
+    preload_ring<L1Pipe<P>::D, 1>(r1, packed_frags<P>(packed, lane, G::FAST1_OFF));
+    // the third plane's share of the first layer, should the plane be constant (see fused_pipe_kernel)
+    f32x16 a0[1][3];
+    {
+      const WFrags tb = packed_frags<P>(packed, lane, G::PLANE2_FRAG_OFF + __builtin_amdgcn_readfirstlane(wave) * 12);
+#pragma unroll
+      for (int j = 0; j < 3; ++j)
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          const f32x4 t4 = __builtin_bit_cast(f32x4, tb[j * 4 + q]);
+#pragma unroll
+          for (int e = 0; e < 4; ++e) a0[0][j][4 * q + e] = t4[e];
+        }
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    // ---- stage the input: zero the shifted copies, then scatter the board ----
+    if (tid < 2) flags[tid] = 0;
+    if (tid == 0) red[4] = xin[0][2];   // the third plane's value at square 0
+    {
+      const v4i z = {0, 0, 0, 0};
+      for (int i = tidv * 16; i < G::COPIES_BYTES; i += THREADS * 16) *reinterpret_cast<v4i *>(smem + i) = z;
+    }
+    __syncthreads();
+    const float c2 = red[4];
+    {
+      bool varies = false, inexact = false;
+#pragma unroll
+      for (int r = 0; r < ROUNDS; ++r)
+        if (tidv + r * THREADS < kPix) {
+          varies |= __builtin_bit_cast(int, xin[r][2]) != __builtin_bit_cast(int, c2);
+#pragma unroll
+          for (int ch = 0; ch < 3; ++ch)
+            inexact |= (__builtin_bit_cast(int, xin[r][ch]) & 0xffff) != 0 && (ch < 2 || varies);
+        }
+      if (varies) flags[0] = 1;
+      if (inexact) flags[1] = 1;
+    }
+    __syncthreads();
+    const bool plane2_varies = flags[0] != 0;
+    const int planes_staged = plane2_varies ? 3 : 2;
+    // An input that is exact in bf16 (stones, flags) is one part; any other goes through the first
+    // layer's loop three times, once for each of its bf16 values.
+    // (a third plane that varies on another thread's squares may be inexact here: look again)
+    bool again = false;
+    if (plane2_varies) {
+#pragma unroll
+      for (int r = 0; r < ROUNDS; ++r)
+        if (tidv + r * THREADS < kPix) again |= (__builtin_bit_cast(int, xin[r][2]) & 0xffff) != 0;
+      if (again) flags[1] = 1;
+      __syncthreads();
+    }
+    const int parts = flags[1] != 0 ? 3 : 1;
+    int l1base[3];
+#pragma unroll
+    for (int j = 0; j < 3; ++j) {
+      bool ok;
+      const int pc = tile_pixel(tidv, j, ok), r = pc / kBoard, c = pc - r * kBoard, s = c % G::E;
+      l1base[j] = s * G::COPY_BYTES + ((r * 3 + kL1RowsHalf * ((tidv >> 5) & 1)) * kL1RowPitch + (c - s)) * G::EB;
+    }
+    {
+      f32x16 b0[1];
+      load_bias_tiles(b0, tail + bias_offset(0), h);
+#pragma unroll
+      for (int j = 0; j < 3; ++j)
+#pragma unroll
+        for (int i = 0; i < 16; ++i) a0[0][j][i] = plane2_varies ? b0[0][i] : fmaf(c2, a0[0][j][i], b0[0][i]);
+    }
+    float left[ROUNDS][3];   // what the parts staged so far leave of the input
+#pragma unroll
+    for (int r = 0; r < ROUNDS; ++r)
+#pragma unroll
+      for (int ch = 0; ch < 3; ++ch) left[r][ch] = xin[r][ch];
+    SplitWeights<1> r2;
+#pragma unroll 1
+    for (int part = 0; part < parts; ++part) {
+      if (part > 0) __syncthreads();  // everybody has read the part before
+#pragma unroll
+      for (int r = 0; r < ROUNDS; ++r) {
+        const int p = tidv + r * THREADS;
+        if (p < kPix) {
+          const int row = p / kBoard, c = p - row * kBoard;
+          if (part == 0) {
+            unsigned char o = occin[r];
+            if (prm.mask_mode == C6_MASK_INPUT) o = (left[r][0] != 0.0f) || (left[r][1] != 0.0f);
+            occ[p] = o;
+          }
+#pragma unroll
+          for (int ch = 0; ch < 3; ++ch) {
+            if (ch >= planes_staged) break;
+            const unsigned short v16 = bits16<P>(left[r][ch]);
+            left[r][ch] -= __builtin_bit_cast(float, (unsigned)v16 << 16);
+            const int hrow = (row + kK1 / 2) * 3 + ch;
+#pragma unroll
+            for (int s = 0; s < G::E; ++s) {
+              const int a = s * G::COPY_BYTES + (hrow * kL1RowPitch + (c + kK1 / 2 - s)) * G::EB;
+              *reinterpret_cast<unsigned short *>(smem + a) = v16;
+            }
+          }
+        }
+      }
+      __syncthreads();
+      if (!plane2_varies) {
+        int l1fast[3];
+#pragma unroll
+        for (int j = 0; j < 3; ++j) l1fast[j] = l1base[j] - (kL1RowsHalf - 1) * h * kL1RowPitch * G::EB;
+        const WFrags wf = packed_frags<P>(packed, lane, G::FAST1_OFF);
+        if (part > 0) preload_ring<L1Pipe<P>::D, 1>(r1, wf);
+        conv1_fast_pass<P>(smem, wf, r1, l1fast, a0);
+      } else {
+        preload_ring<L1Pipe<P>::D, 1>(r1, layer_weights<P, 0>(packed, lane));
+        conv1_pass<P>(smem, layer_weights<P, 0>(packed, lane), r1, l1base, a0);
+      }
+    }
+    const long long bn = b + 1;
+    if (bn < b_end) fetch_board(bn);  // lands while this board is computed
+    split_preload<1>(r2, layer_weights<P, 1>(packed, lane));
+    __syncthreads();
+    // the copies overlapped the activation tile: restore its zero padding
+    for (int i = tidv; i < 60 * (S::PIXB / 16); i += THREADS) {
+      const int k = i / (S::PIXB / 16), w16 = i - k * (S::PIXB / 16);
+      const int pos = k < 20 ? k : (k < 41 ? 400 + (k - 20) : (k - 40) * kPitch);
+      *reinterpret_cast<v4i *>(smem + pos * S::PIXB + w16 * 16) = v4i{0, 0, 0, 0};
+    }
+    split_store<1, true>(smem, ci, h, a0);
+    __syncthreads();
+
+    SplitWeights<2> r345;
+    SplitWeights<5> r678;
+    split_layer<1>(smem, packed, tail, r2, r345, ci, h, lane);
+    split_layer<2>(smem, packed, tail, r345, r345, ci, h, lane);
+    split_layer<3>(smem, packed, tail, r345, r345, ci, h, lane);
+    split_layer<4>(smem, packed, tail, r345, r678, ci, h, lane);
+    split_layer<5>(smem, packed, tail, r678, r678, ci, h, lane);
+    split_layer<6>(smem, packed, tail, r678, r678, ci, h, lane);
+
+    // ---- layer 8 + both 1x1 heads straight from the fp32 accumulators ----
+    {
+      f32x16 acc[3][3];
+      init_acc(acc, tail + bias_offset(7), h);
+      split_conv<7>(smem, layer_weights<P, 7>(packed, lane), r678, ci, h, acc);
+      const float *valw = tail + kBiasTotal + kHeadC;
+      const float *pwl = tail + kBiasTotal + 4 * h;  // per-lane base: channel 32t + 8q + 4h + e
+      asm volatile("" : "+v"(pwl));
+      const GlobalF32 pwg = (GlobalF32)pwl;
+      int pix[3];
+      bool valid[3];
+      int th = tidv;
+      asm volatile("" : "+v"(th));
+#pragma unroll
+      for (int j = 0; j < 3; ++j) pix[j] = tile_pixel(th, j, valid[j]);
+      float pol[3] = {0.0f, 0.0f, 0.0f};
+      float vsum = 0.0f;
+#pragma unroll
+      for (int t = 0; t < 3; ++t)
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          const f32x4 pw = *(GlobalF32x4)(pwg + 32 * t + 8 * q);
+          const f32x4 vw = *(GlobalF32x4)(pwg + kHeadC + 32 * t + 8 * q);
+#pragma unroll
+          for (int j = 0; j < 3; ++j) {
+            float vs = 0.0f;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+              const float a = split_silu(acc[t][j][4 * q + e]);
+              pol[j] = fmaf(a, pw[e], pol[j]);
+              vs = fmaf(a, vw[e], vs);
+            }
+            vsum += valid[j] ? vs : 0.0f;
+          }
+        }
+      const float polb = valw[kHeadC], valb = valw[kHeadC + 1];
+#pragma unroll
+      for (int j = 0; j < 3; ++j) {  // add the other lane half's channels
+        const unsigned bits = __builtin_bit_cast(unsigned, pol[j]);
+        const auto r = __builtin_amdgcn_permlane32_swap(bits, bits, false, false);
+        const unsigned r0 = r[0], r1 = r[1];
+        if (h == 0 && valid[j]) lgt[pix[j]] = __builtin_bit_cast(float, r0) + __builtin_bit_cast(float, r1) + polb;
+      }
+      vsum = wave_sum(vsum);
+      if (lane == 0) red[wave] = vsum;
+      __syncthreads();
+      if (tid == 0 && prm.value != nullptr) {
+        float s = 0.0f;
+#pragma unroll
+        for (int w = 0; w < NWAVES; ++w) s += red[w];
+        prm.value[b] = tanhf(s * (1.0f / kPix) + valb);
+      }
+    }
+    // ---- write out: masked logits, optional sampled action ----
+    if (prm.logits != nullptr) {
+      for (int p = tidv; p < kPix; p += THREADS)
+        static_cast<float *>(prm.logits)[(size_t)b * kPix + p] = occ[p] ? prm.fill : lgt[p];
+    }
+    if (prm.actions != nullptr && wave == 0) {
+      float it = prm.inv_temperature;
+      asm volatile("" : "+s"(it));
+      int a;
+      float lp;
+      int lane_here = lane;
+      asm volatile("" : "+v"(lane_here));
+      wave_sample(
+          lane_here, prm.u[b], it, [&](int i) { return lgt[i]; }, [&](int i) { return occ[i] == 0; }, a, lp);
+      if (lane == 0) {
+        prm.actions[b] = a;
+        if (prm.logprob != nullptr) prm.logprob[b] = lp;
+      }
+    }
+  }
+}
+
+}  // namespace c6

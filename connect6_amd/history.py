@@ -117,7 +117,7 @@ class HistoricalPolicyEnsemble:
         self._prec = _PREC_OF_DTYPE[self.dtype] if precision is None else _lib.PREC_BY_NAME[precision]
         self._arch: bytes | None = None     # other architectures: see _fits
         self._has_packed = False
-        self._packed: tuple | None = None   # (buffer, stream it was packed on, event)
+        self._packed: dict[int, tuple] = {}   # mode: (buffer, stream it was packed on, event)
         self._states = states
         self._stacked: dict[str, torch.Tensor | None] = {}
         self._stacked32: dict[str, torch.Tensor] | None = None
@@ -184,23 +184,24 @@ class HistoricalPolicyEnsemble:
                 self.board_size, self.kernels, self.channels, self._prec) > 0
         return self._has_packed
 
-    def _packed_weights(self) -> torch.Tensor:
+    def _packed_weights(self, prec: int | None = None) -> torch.Tensor:
+        prec = self._prec if prec is None else prec
         stream_ptr = _lib.stream_ptr(self.device)
-        if self._packed is None:
+        if prec not in self._packed:
             # one call for all models, from the stacked tensors (rounded to `dtype`, as the
             # ensemble holds its parameters): two launches, however many models
             stacked = self._stacked_state()
             if self.is_default_architecture:
-                one = _lib.packed_bytes(self._prec)
+                one = _lib.packed_bytes(prec)
                 buf = torch.empty((self.num_models, one), dtype=torch.uint8, device=self.device)
-                pack_state(stacked, self._prec, buf, groups=self.num_models)
+                pack_state(stacked, prec, buf, groups=self.num_models)
             else:
-                buf = pack_generic(stacked, self.board_size, self.kernels, self.channels, self._prec, self.device,
+                buf = pack_generic(stacked, self.board_size, self.kernels, self.channels, prec, self.device,
                                    groups=self.num_models, want_value=False)
             done = torch.cuda.Event()
             done.record(torch.cuda.current_stream(self.device))
-            self._packed = (buf, stream_ptr, done)
-        buf, packed_on, done = self._packed
+            self._packed[prec] = (buf, stream_ptr, done)
+        buf, packed_on, done = self._packed[prec]
         if packed_on != stream_ptr:   # packed on another stream: wait for it, and tell the
             stream = torch.cuda.current_stream(self.device)
             stream.wait_event(done)           # allocator that this stream reads the buffer too
@@ -230,9 +231,9 @@ class HistoricalPolicyEnsemble:
         if self.is_default_architecture:
             # (the cascade's entry point writes the logits in the ensemble's type itself)
             direct = self._prec in _lib.CASCADES and self.dtype != torch.float32
-            logits, _, _, _ = run_forward(x.reshape(m * t, *expected_tail), self._packed_weights(),
-                                          self._prec, m, t, want_value=False,
-                                          logits_dtype=self.dtype if direct else torch.float32)
+            prec = _lib.kernel_prec(self._prec)
+            logits, _, _, _ = run_forward(x.reshape(m * t, *expected_tail), self._packed_weights(prec), prec,
+                                          m, t, want_value=False, logits_dtype=self.dtype if direct else torch.float32)
         else:  # other architectures: one launch where the network has a packed form, else one per layer
             flat = x.reshape(m * t, *expected_tail)
             packed = self._packed_weights() if self._fits() else None

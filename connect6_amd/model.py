@@ -459,6 +459,7 @@ class PolicyValueNet(nn.Module):
         prec = self.resolve_precision()
         if not self.is_default_architecture:
             return self._generic(x, prec)
+        prec = _lib.kernel_prec(prec)
         logits, value, _, _ = run_forward(x, self.packed_weights(prec), prec, 1, int(x.shape[0]),
                                           threshold=self.cascade_threshold, stats=self.cascade_stats)
         return logits, value
@@ -479,6 +480,7 @@ class PolicyValueNet(nn.Module):
         fill = _FILL_LOWEST if fill is None else float(fill)
         if not self.is_default_architecture:
             return self._generic(x, prec, mask_mode=mask_mode, legal=legal, fill=fill)
+        prec = _lib.kernel_prec(prec)
         logits, value, _, _ = run_forward(
             x, self.packed_weights(prec), prec, 1, int(x.shape[0]),
             mask_mode=mask_mode, legal=legal, fill=fill,
@@ -505,7 +507,7 @@ class PolicyValueNet(nn.Module):
                 "the fused self-play step is built for the default architecture on a 19x19 board; "
                 "use forward_masked() followed by sample_actions() elsewhere"
             )
-        prec = self.resolve_precision()
+        prec = _lib.kernel_prec(self.resolve_precision())
         logits, value, actions, logprob = run_forward(
             x, self.packed_weights(prec), prec, 1, int(x.shape[0]), want_logits=return_logits,
             mask_mode=_lib.MASK_INPUT if legal is None else _lib.MASK_LEGAL, legal=legal,
@@ -600,7 +602,7 @@ def _forward_boards(
     if index is not None and (index.dtype != torch.int64 or index.ndim != 1):
         raise ValueError("index must be a 1-D int64 tensor of board rows")
     # (index entries outside [0, N) are clamped by the kernel)
-    prec = model.resolve_precision()
+    prec = _lib.kernel_prec(model.resolve_precision())
     thr = model.cascade_threshold
     rc, logits, value, actions, logprob, twice = _lib.host().forward_boards(
         boards, current_player, stones_left, index, int(view), model.packed_weights(prec), prec, want_logits,

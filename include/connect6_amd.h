@@ -47,6 +47,11 @@ extern "C" {
                             weights to bf16 dropped (a second bf16 weight fragment per fragment,
                             twice the bf16 matrix work): within 3e-4 relative L2 of fp32 */
 
+#define C6_PREC_F32S 7   /* fp32 operands, each the exact sum of three bf16 values: six bf16 MFMAs per
+                            product, fp32 accumulate.  fp32 results (the products left out are
+                            below 2^-25) at half the time of C6_PREC_F32; its packed weights take
+                            three halves of that mode's */
+
 /* element types of caller tensors */
 #define C6_DT_F32 0
 #define C6_DT_BF16 1

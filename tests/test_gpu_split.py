@@ -1,0 +1,72 @@
+"""fp32 through three bf16 parts per operand (C6_PREC_F32S) against a float64 forward: no further from
+it than fp32 arithmetic, whatever the input planes hold (the kernel stages inputs that are exact in
+bf16 once and others in three parts, and contracts a constant third plane through a table)."""
+import pytest
+import torch
+
+import connect6_amd as c6
+from connect6_amd import _lib
+from connect6_amd.model import run_forward
+from connect6_amd.synthetic import gen_boards, gen_uniform
+from oracle import torch_ref as R
+from tests.util import rel_l2
+
+pytestmark = pytest.mark.gpu
+
+
+def _planes(kind, n):
+    g = torch.Generator().manual_seed(4)
+    x, _ = gen_boards(n, 200, 3)
+    if kind == "randn":
+        x = torch.randn(n, 3, 19, 19, generator=g)
+    elif kind == "varying":
+        x[:, 2] = (torch.rand(n, 19, 19, generator=g) > 0.5).float()
+    elif kind == "inexact constant":
+        x[:, 2] = 0.3
+    elif kind == "one inexact square":       # only one thread of the workgroup sees it
+        x[:, 2, 17, 3] = 0.3
+    elif kind == "large":
+        x = x * 300.0
+    return x
+
+
+@pytest.mark.parametrize("init", ["reference", "torch_default"])
+@pytest.mark.parametrize("kind", ["boards", "randn", "varying", "inexact constant", "one inexact square", "large"])
+def test_no_further_from_float64_than_fp32(cuda, kind, init):
+    st = R.init_state(5, init)
+    model = c6.PolicyValueNet().to(cuda).eval()
+    model.load_state_dict(st)
+    x = _planes(kind, 33)
+    l64, v64 = R.forward({k: v.double() for k, v in st.items()}, x.double())
+    err = {}
+    with torch.inference_mode():
+        for prec in (_lib.PREC_F32, _lib.PREC_F32S):
+            lg, vg, _, _ = run_forward(x.to(cuda), model.packed_weights(prec), prec, 1, 33)
+            err[prec] = (rel_l2(lg.double().cpu(), l64), rel_l2(vg.double().cpu(), v64))
+    # Eight layers of fp32 sums: each of the two results is within a few 2^-24 per layer of float64;
+    # the value, a mean that nearly cancels, scatters more (twice the other's error plus 1e-6).
+    assert err[_lib.PREC_F32S][0] <= 1.5 * err[_lib.PREC_F32][0] + 1e-7, err
+    assert err[_lib.PREC_F32S][1] <= 2 * err[_lib.PREC_F32][1] + 1e-6, err
+
+
+def test_fp32_batches_draws_masks_and_states(cuda):
+    st = R.init_state(11, "reference")
+    model = c6.PolicyValueNet().to(cuda).eval()
+    model.load_state_dict(st)
+    x, legal = gen_boards(600, 200, 77)
+    xd, ld, u = x.to(cuda), legal.to(cuda), gen_uniform(600, 5).to(cuda)
+    boards = (x[:, 0] - x[:, 1]).to(torch.int8).to(cuda)
+    player = torch.ones(600, dtype=torch.int8, device=cuda)
+    left = (x[:, 2, 0, 0] == 1).to(torch.int8).to(cuda)
+    with torch.inference_mode():
+        lg, vg = model.forward_masked(xd, ld)
+        ag, pg, _ = model.selfplay_step(xd, u, 0.8, legal=ld)
+        assert torch.equal(lg == torch.finfo(torch.float32).min, ~ld)
+        assert bool(ld.gather(1, ag.view(-1, 1)).all())
+        lb, vb = model.forward_boards(boards, player, left)
+        assert torch.equal(lb, lg) and torch.equal(vb, vg)
+        for n in (1, 2, 37, 255, 257, 513):
+            l, v = model.forward_masked(xd[:n], ld[:n])
+            a, p, _ = model.selfplay_step(xd[:n], u[:n], 0.8, legal=ld[:n])
+            assert torch.equal(l, lg[:n]) and torch.equal(v, vg[:n]), n
+            assert torch.equal(a, ag[:n]) and torch.equal(p, pg[:n]), n

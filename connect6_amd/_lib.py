@@ -53,6 +53,10 @@ EXPORTS = (
     "c6_forward_generic",
     "c6_forward_generic_grouped",
     "c6_forward_generic_static",
+    "c6_team_bytes",
+    "c6_forward_team",
+    "c6_forward_boards_team",
+    "c6_stream_capturing",
     "c6_generic_packed_bytes",
     "c6_generic_pack",
     "c6_forward_generic_packed",
@@ -126,7 +130,8 @@ _HOST_SO = _LIBDIR / "_c6_host.so"
 # entry points csrc/c6_host.cpp calls, in the order of its `Abi`
 _HOST_ABI = ("c6_forward", "c6_forward_cascade", "c6_forward_boards", "c6_forward_boards_cascade",
              "c6_cascade_workspace_bytes", "c6_mask_logits", "c6_softmax_sample", "c6_env_step", "c6_canonical_input",
-             "c6_forward_generic_packed")
+             "c6_forward_generic_packed", "c6_team_bytes", "c6_forward_team", "c6_forward_boards_team",
+             "c6_stream_capturing")
 
 
 def build_host() -> Path:
@@ -263,6 +268,16 @@ def load() -> ctypes.CDLL:
     lib.c6_forward_boards_cascade.restype = i32
     lib.c6_forward_boards_cascade.argtypes = [vp, vp, vp, i64, vp, i32, i64, vp, i32, vp, i32, vp, i32, f32, vp, f32,
                                               vp, vp, f32, vp, ctypes.c_size_t, vp]
+    sizes = [ctypes.POINTER(ctypes.c_size_t)] * 2
+    lib.c6_team_bytes.restype = i32
+    lib.c6_team_bytes.argtypes = [i32, i64] + sizes
+    team = [vp, ctypes.c_size_t, vp, ctypes.c_size_t, ctypes.c_uint32, i32, vp]
+    lib.c6_forward_team.restype = i32
+    lib.c6_forward_team.argtypes = lib.c6_forward.argtypes[:-1] + team
+    lib.c6_forward_boards_team.restype = i32
+    lib.c6_forward_boards_team.argtypes = lib.c6_forward_boards.argtypes[:-1] + team
+    lib.c6_stream_capturing.restype = i32
+    lib.c6_stream_capturing.argtypes = [vp]
     ip = ctypes.POINTER(ctypes.c_int)
     lib.c6_generic_workspace_bytes.restype = i32
     lib.c6_generic_workspace_bytes.argtypes = [i64, i32, i32, ip, ctypes.POINTER(ctypes.c_size_t)]

@@ -20,6 +20,8 @@ void set_error(const char *fmt, ...) {
 int dispatch_pack(int prec, const PackParams &pp, hipStream_t st);
 int dispatch_forward(int prec, const FwdParams &fp, hipStream_t st);
 int dispatch_cascade(int prec, const FwdParams &fp, float threshold, void *workspace, hipStream_t st);
+int team_workspace_bytes(int prec, long long boards, size_t *bytes);
+int dispatch_team(int prec, const TeamParams &tp, hipStream_t st);
 size_t packed_bytes(int prec);
 int launch_mask(const void *, const uint8_t *, int, long long, uint32_t, void *, hipStream_t);
 int launch_sample(const float *, const uint8_t *, const float *, float, long long, long long *,
@@ -101,6 +103,42 @@ static int check_cascade_workspace(const char *who, long long boards, const void
   return C6_OK;
 }
 
+// the extra arguments of c6_forward_team / c6_forward_boards_team
+struct TeamArgs {
+  void *workspace;
+  size_t workspace_bytes;
+  unsigned *flags;
+  size_t flag_bytes;
+  unsigned tag;
+  int polls;
+};
+constexpr int kTeamPolls = 64;   // about 45 us
+
+
+static int run_team(const char *who, int prec, const FwdParams &fp, const TeamArgs &t, hipStream_t st) {
+  size_t need = 0;
+  const int rc = team_workspace_bytes(prec, fp.total_boards, &need);
+  if (rc != C6_OK) return rc;
+  if (need == 0) {
+    set_error("%s: %lld boards of mode %d are served by one workgroup each (c6_team_bytes is 0)", who, fp.total_boards,
+              prec);
+    return C6_EINVAL;
+  }
+  if (t.workspace == nullptr || !aligned16(t.workspace) || t.workspace_bytes < need || t.flags == nullptr ||
+      t.flag_bytes < (size_t)fp.total_boards * kTeamFlags * 4 || t.tag == 0) {
+    set_error("%s: needs a 16-byte aligned workspace and flag words of the sizes c6_team_bytes gives, and a tag that is "
+              "not 0", who);
+    return C6_EINVAL;
+  }
+  TeamParams tp;
+  tp.f = fp;
+  tp.act = static_cast<unsigned char *>(t.workspace);
+  tp.flags = t.flags;
+  tp.tag = t.tag;
+  tp.polls = t.polls > 0 ? t.polls : kTeamPolls;
+  return dispatch_team(prec, tp, st);
+}
+
 }  // namespace c6
 
 using namespace c6;
@@ -173,7 +211,7 @@ static int forward_planes(const char *who, const void *x, int x_dtype, int64_t g
                           int prec, void *logits, int logits_dtype, float *value, int mask_mode,
                           const uint8_t *legal, float fill, const float *u, float temperature,
                           int64_t *actions, float *logprob, bool cascade, float threshold,
-                          void *workspace, size_t workspace_bytes, void *stream) {
+                          void *workspace, size_t workspace_bytes, void *stream, const TeamArgs *team = nullptr) {
   if (!valid_prec(prec) || is_cascade(prec) != cascade) {
     set_error("%s: precision mode %d is unknown or not served by this entry point (the cascade modes "
               "take c6_forward_cascade, every other mode c6_forward)", who, prec);
@@ -239,6 +277,7 @@ static int forward_planes(const char *who, const void *x, int x_dtype, int64_t g
     if (rc != C6_OK) return rc;
   }
   C6_REQUIRE_DEVICE(who);
+  if (team != nullptr) return run_team(who, prec, fp, *team, static_cast<hipStream_t>(stream));
   if (cascade) return dispatch_cascade(prec, fp, threshold, workspace, static_cast<hipStream_t>(stream));
   return dispatch_forward(prec, fp, static_cast<hipStream_t>(stream));
 }
@@ -277,7 +316,8 @@ static int forward_states(const char *who, const int8_t *boards, const int8_t *p
                           int view, int64_t batch, const void *packed, int prec, void *logits,
                           int logits_dtype, float *value, int mask_mode, float fill, const float *u,
                           float temperature, int64_t *actions, float *logprob, bool cascade,
-                          float threshold, void *workspace, size_t workspace_bytes, void *stream) {
+                          float threshold, void *workspace, size_t workspace_bytes, void *stream,
+                          const TeamArgs *team = nullptr) {
   if (!valid_prec(prec) || is_cascade(prec) != cascade || elem_bytes(logits_dtype) == 0 || batch < 0 ||
       batch > 0x7fffffffLL || view < 0 || view > 7 || num_states < 0) {
     set_error("%s: bad precision %d, batch %lld, states %lld or view %d", who, prec,
@@ -333,6 +373,7 @@ static int forward_states(const char *who, const int8_t *boards, const int8_t *p
     if (rc != C6_OK) return rc;
   }
   C6_REQUIRE_DEVICE(who);
+  if (team != nullptr) return run_team(who, prec, fp, *team, static_cast<hipStream_t>(stream));
   if (cascade) return dispatch_cascade(prec, fp, threshold, workspace, static_cast<hipStream_t>(stream));
   return dispatch_forward(prec, fp, static_cast<hipStream_t>(stream));
 }
@@ -359,6 +400,49 @@ int c6_forward_boards_cascade(const int8_t *boards, const int8_t *player,
                         temperature, actions, logprob, true, threshold, workspace, workspace_bytes, stream);
 }
 
+
+int c6_team_bytes(int prec, int64_t boards, size_t *workspace_bytes, size_t *flag_bytes) {
+  if (!valid_prec(prec) || boards < 0 || boards > 0x7fffffffLL || workspace_bytes == nullptr || flag_bytes == nullptr) {
+    set_error("c6_team_bytes: bad precision mode %d, board count or null output", prec);
+    return C6_EINVAL;
+  }
+  *flag_bytes = 0;
+  const int rc = team_workspace_bytes(prec, boards, workspace_bytes);
+  if (rc == C6_OK && *workspace_bytes != 0) *flag_bytes = (size_t)boards * kTeamFlags * 4;
+  return rc;
+}
+
+int c6_stream_capturing(void *stream) {
+  hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(static_cast<hipStream_t>(stream), &status) != hipSuccess) {
+    (void)hipGetLastError();
+    return 0;
+  }
+  return status == hipStreamCaptureStatusNone ? 0 : 1;
+}
+
+int c6_forward_team(const void *x, int x_dtype, int64_t groups, int64_t boards_per_group,
+                    const void *packed, size_t packed_stride, int prec, float *logits, float *value,
+                    int mask_mode, const uint8_t *legal, float fill, const float *u, float temperature,
+                    int64_t *actions, float *logprob, void *workspace, size_t workspace_bytes,
+                    void *flags, size_t flag_bytes, uint32_t tag, int polls, void *stream) {
+  const TeamArgs t{workspace, workspace_bytes, static_cast<unsigned *>(flags), flag_bytes, tag, polls};
+  return forward_planes("c6_forward_team", x, x_dtype, groups, boards_per_group, packed, packed_stride, prec, logits,
+                        C6_DT_F32, value, mask_mode, legal, fill, u, temperature, actions, logprob, false, 0.0f,
+                        nullptr, 0, stream, &t);
+}
+
+int c6_forward_boards_team(const int8_t *boards, const int8_t *player, const int8_t *stones_left,
+                           int64_t num_states, const int64_t *index, int view, int64_t batch,
+                           const void *packed, int prec, float *logits, float *value, int mask_mode,
+                           float fill, const float *u, float temperature, int64_t *actions,
+                           float *logprob, void *workspace, size_t workspace_bytes, void *flags,
+                           size_t flag_bytes, uint32_t tag, int polls, void *stream) {
+  const TeamArgs t{workspace, workspace_bytes, static_cast<unsigned *>(flags), flag_bytes, tag, polls};
+  return forward_states("c6_forward_boards_team", boards, player, stones_left, num_states, index, view, batch, packed,
+                        prec, logits, C6_DT_F32, value, mask_mode, fill, u, temperature, actions, logprob, false, 0.0f,
+                        nullptr, 0, stream, &t);
+}
 
 static int check_arch(const char *who, int board, int layers, const int *kernels,
                       const int *channels) {

@@ -287,6 +287,16 @@ struct FwdParams {
   int redo_per = 0;               // boards per run of the first pass
 };
 
+// Few boards: several workgroups per board (c6_team.h)
+struct TeamParams {
+  FwdParams f;
+  unsigned char *act;   // TeamGeo<P>::BOARDB bytes per board
+  unsigned *flags;      // kTeamFlags words per board
+  unsigned tag;
+  int polls;            // of a flag (about 0.7 us each) before a workgroup helps itself
+};
+constexpr int kTeamFlags = 96;                   // words per board: stage * 9 + role
+
 struct PackParams {
   const float *conv_w[8];     // each tensor stacked over the weight sets: [groups, ...]
   const float *conv_b[8];

@@ -1907,6 +1907,7 @@ __global__ __launch_bounds__(256) void fused_forward_kernel(const FwdParams prm)
 }  // namespace c6
 
 #include "c6_split.h"
+#include "c6_team.h"
 
 namespace c6 {
 
@@ -2155,6 +2156,8 @@ template <class P> __global__ __launch_bounds__(256) void lo_scale_kernel(const 
 template <class P> int launch_pack(const PackParams &pp, hipStream_t st);
 template <class P> int launch_forward(const FwdParams &fp, hipStream_t st);
 
+template <class P> int launch_team(const TeamParams &tp, int team, hipStream_t st);
+
 #ifndef C6_SPLIT
 template <class P> int launch_pack(const PackParams &pp, hipStream_t st) {
   using G = Geo<P>;
@@ -2219,11 +2222,43 @@ template <class P> int launch_forward(const FwdParams &fp, hipStream_t st) {
   return C6_OK;
 }
 
+template <class P, int TEAM> static int launch_team_of(const TeamParams &tp, hipStream_t st) {
+  using T = TeamGeo<P>;
+  static thread_local int configured = -1;
+  int dev = 0;
+  hipError_t e = hipGetDevice(&dev);
+  if (e == hipSuccess && configured != dev) {
+    e = hipFuncSetAttribute(reinterpret_cast<const void *>(&team_forward_kernel<P, TEAM>),
+                            hipFuncAttributeMaxDynamicSharedMemorySize, T::LDS_BYTES);
+    if (e == hipSuccess) configured = dev;
+  }
+  if (e == hipSuccess) {
+    hipLaunchKernelGGL((team_forward_kernel<P, TEAM>), dim3((unsigned)(tp.f.total_boards * TEAM)), dim3(256), T::LDS_BYTES,
+                       st, tp);
+    e = hipGetLastError();
+  }
+  if (e != hipSuccess) {
+    set_error("team_forward launch failed: %s", hipGetErrorString(e));
+    return C6_ELAUNCH;
+  }
+  return C6_OK;
+}
+
+template <class P> int launch_team(const TeamParams &tp, int team, hipStream_t st) {
+  if constexpr (has_team<P>()) {
+    return team == 9 ? launch_team_of<P, 9>(tp, st) : launch_team_of<P, 3>(tp, st);
+  } else {
+    set_error("this mode has no team kernel");
+    return C6_EINVAL;
+  }
+}
+
 #endif  // C6_SPLIT
 
 #ifdef C6_INSTANCE
 template int launch_pack<C6_INSTANCE>(const PackParams &, hipStream_t);
 template int launch_forward<C6_INSTANCE>(const FwdParams &, hipStream_t);
+template int launch_team<C6_INSTANCE>(const TeamParams &, int, hipStream_t);
 #else
 
 int dispatch_pack(int prec, const PackParams &pp, hipStream_t st) {
@@ -2309,6 +2344,29 @@ int dispatch_cascade(int prec, const FwdParams &fp, float threshold, void *works
   second.packed = fp.packed + kCascadeSecondOffset;
   second.redo_mode = kRedoConsume;
   return prec == C6_PREC_BF16C ? launch_forward<PrecBF16F6W>(second, st) : launch_forward<PrecBF16F6>(second, st);
+}
+
+// Bytes per board that the mode's team kernel keeps in memory; 0 where the mode has none.
+static size_t team_board_bytes(int prec) {
+  return prec == C6_PREC_F32S ? TeamGeo<PrecF32S>::BOARDB : 0;
+}
+// Workspace for `boards` boards of a mode, 0 where one workgroup per board serves them.
+int team_workspace_bytes(int prec, long long boards, size_t *bytes) {
+  int cus = 0;
+  *bytes = 0;
+  const size_t per = team_board_bytes(prec);
+  if (per == 0 || boards < 1) return C6_OK;
+  const int rc = device_cus(cus);
+  if (rc == C6_OK && team_size(boards, cus) > 1) *bytes = per * (size_t)boards;
+  return rc;
+}
+int dispatch_team(int prec, const TeamParams &tp, hipStream_t st) {
+  int cus = 0;
+  const int rc = device_cus(cus);
+  if (rc != C6_OK) return rc;
+  const int team = team_size(tp.f.total_boards, cus);
+  if (team == 1 || team_board_bytes(prec) == 0) return dispatch_forward(prec, tp.f, st);
+  return launch_team<PrecF32S>(tp, team, st);
 }
 
 size_t packed_bytes(int prec) {

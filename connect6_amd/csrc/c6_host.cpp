@@ -16,6 +16,7 @@
 #include <array>
 #include <cstring>
 #include <string>
+#include <vector>
 
 #include "../../include/connect6_amd.h"
 
@@ -32,6 +33,10 @@ struct Abi {
   decltype(&c6_env_step) env_step;
   decltype(&c6_canonical_input) canonical_input;
   decltype(&c6_forward_generic_packed) forward_generic_packed;
+  decltype(&c6_team_bytes) team_bytes;
+  decltype(&c6_forward_team) forward_team;
+  decltype(&c6_forward_boards_team) forward_boards_team;
+  decltype(&c6_stream_capturing) stream_capturing;
 } abi;
 
 PyObject *fail(PyObject *type, const std::string &what) {
@@ -86,6 +91,61 @@ at::Tensor cascade_workspace(int64_t boards, const at::Device &dev) {
   size_t bytes = 0;
   if (abi.cascade_workspace_bytes(boards, &bytes) != C6_OK) return {};
   return fresh({(int64_t)(bytes / 4)}, at::kInt, dev);
+}
+
+// Buffers of a call that shares a board between workgroups (c6_forward_team); `work` stays undefined
+// where the call is not one.
+struct Team {
+  at::Tensor work, flags;
+  uint32_t tag = 0;
+};
+
+// The flag words are kept per stream, with the last tag written into them: calls on one stream follow
+// one another, so a tag counted up per call is one that no word holds.  Sixteen streams at most; the
+// one that has waited longest gives its words back.  (Only under the interpreter's lock.)  Inside a
+// graph capture the words are the graph's own, cleared in the graph: a replay has the same tag.
+Team team_buffers(int prec, int64_t boards, const at::Device &dev, void *stream) {
+  struct Kept {
+    int device;
+    void *stream;
+    at::Tensor flags;
+    uint32_t tag;
+    uint64_t used;
+  };
+  static std::vector<Kept> &kept = *new std::vector<Kept>;   // (never destroyed: the device is gone at exit)
+  static uint64_t clock = 0;
+  constexpr size_t kMost = 16;
+  Team t;
+  size_t bytes = 0, flag_bytes = 0;
+  if (abi.team_bytes(prec, boards, &bytes, &flag_bytes) != C6_OK || bytes == 0) return t;
+  t.work = fresh({(int64_t)bytes}, at::kByte, dev);
+  const auto zeros = [&](int64_t words) { return at::zeros({words}, at::TensorOptions().dtype(at::kInt).device(dev)); };
+  if (abi.stream_capturing(stream)) {
+    t.flags = zeros((int64_t)(flag_bytes / 4));
+    t.tag = 1;
+    return t;
+  }
+  Kept *k = nullptr;
+  for (Kept &e : kept)
+    if (e.device == dev.index() && e.stream == stream) k = &e;
+  if (k == nullptr) {
+    if (kept.size() == kMost) {
+      size_t oldest = 0;
+      for (size_t i = 1; i < kept.size(); ++i)
+        if (kept[i].used < kept[oldest].used) oldest = i;
+      kept.erase(kept.begin() + (long)oldest);
+    }
+    kept.push_back(Kept{dev.index(), stream, {}, 0, 0});
+    k = &kept.back();
+  }
+  if (!k->flags.defined() || (size_t)k->flags.nbytes() < flag_bytes || k->tag == UINT32_MAX) {
+    k->flags = zeros((int64_t)(flag_bytes / 4));
+    k->tag = 0;
+  }
+  k->used = ++clock;
+  t.flags = k->flags;
+  t.tag = ++k->tag;
+  return t;
 }
 
 // Uniform draws as the kernels read them: fp32 on the device, one per board.
@@ -194,6 +254,11 @@ PyObject *forward(PyObject *, PyObject *const *a, Py_ssize_t n) {
                              logits_code, ptr<float>(value), mask_mode, legal_ptr, fill, ptr<float>(u), temperature,
                              ptr<int64_t>(actions), ptr<float>(logprob), threshold, ptr<void>(ws),
                              ws.defined() ? ws.nbytes() : 0, stream);
+  } else if (const Team t = team_buffers(prec, total, dev, stream); t.work.defined()) {
+    rc = abi.forward_team(x.data_ptr(), x_code, groups, per, packed.data_ptr(), stride, prec, ptr<float>(logits),
+                          ptr<float>(value), mask_mode, legal_ptr, fill, ptr<float>(u), temperature,
+                          ptr<int64_t>(actions), ptr<float>(logprob), t.work.data_ptr(), t.work.nbytes(),
+                          t.flags.data_ptr(), t.flags.nbytes(), t.tag, 0, stream);
   } else {
     rc = abi.forward(x.data_ptr(), x_code, groups, per, packed.data_ptr(), stride, prec, ptr<float>(logits),
                      ptr<float>(value), mask_mode, legal_ptr, fill, ptr<float>(u), temperature,
@@ -243,6 +308,12 @@ PyObject *forward_boards(PyObject *, PyObject *const *a, Py_ssize_t n) {
                                     C6_DT_F32, ptr<float>(value), mask_mode, fill, ptr<float>(u), temperature,
                                     ptr<int64_t>(actions), ptr<float>(logprob), threshold, ptr<void>(ws),
                                     ws.defined() ? ws.nbytes() : 0, stream);
+  } else if (const Team t = team_buffers(prec, total, dev, stream); t.work.defined()) {
+    rc = abi.forward_boards_team(ptr<int8_t>(boards), ptr<int8_t>(player), ptr<int8_t>(left), states,
+                                 ptr<int64_t>(index), view, total, packed.data_ptr(), prec, ptr<float>(logits),
+                                 ptr<float>(value), mask_mode, fill, ptr<float>(u), temperature, ptr<int64_t>(actions),
+                                 ptr<float>(logprob), t.work.data_ptr(), t.work.nbytes(), t.flags.data_ptr(),
+                                 t.flags.nbytes(), t.tag, 0, stream);
   } else {
     rc = abi.forward_boards(ptr<int8_t>(boards), ptr<int8_t>(player), ptr<int8_t>(left), states, ptr<int64_t>(index),
                             view, total, packed.data_ptr(), prec, ptr<float>(logits), ptr<float>(value), mask_mode,

@@ -33,7 +33,7 @@ struct SplitGeo {
   static constexpr int OCC_OFF = ACT_BYTES;
   static constexpr int LGT_OFF = OCC_OFF + 384;
   static constexpr int RED_OFF = LGT_OFF + 1456;
-  static constexpr int LDS_BYTES = RED_OFF + 64;
+  static constexpr int LDS_BYTES = RED_OFF + 48 * 4;
   static_assert(G::COPIES_BYTES <= ACT_BYTES && LDS_BYTES <= 160 * 1024, "LDS map");
 };
 
@@ -43,6 +43,7 @@ __device__ __forceinline__ int split_swz(int pos) { return ((pos >> 1) & 7) << 4
 // u / (1 + 2^u), the reciprocal with one Newton step.  (Clamped where 1 + 2^u leaves fp32: the
 // result is then below 2^-126 |u|.)
 __device__ __forceinline__ float split_silu(float u) {
+#pragma clang fp contract(off)   // (the product is rounded before its parts are taken)
   const float d = fminf(1.0f + __builtin_amdgcn_exp2f(u), 0x1p126f);
   const float r = __builtin_amdgcn_rcpf(d);
   return u * fmaf(r, fmaf(-d, r, 1.0f), r);
@@ -50,6 +51,7 @@ __device__ __forceinline__ float split_silu(float u) {
 
 // The next bf16 plane of a pair of values, which keep what it leaves out.
 __device__ __forceinline__ int split_take(float &a, float &b) {
+#pragma clang fp contract(off)
   const int w = pack2<PrecBF16>(a, b);
   a -= __builtin_bit_cast(float, w << 16);
   b -= __builtin_bit_cast(float, w & (int)0xffff0000);
@@ -208,6 +210,13 @@ __device__ __forceinline__ void split_layer(unsigned char *smem, const unsigned 
   __syncthreads();
 }
 
+// the value head's sum over (cout tile, tile of 32 squares)
+__device__ __forceinline__ float split_value_sum(const float *part) {
+  float s = 0.0f;
+  for (int i = 0; i < 36; ++i) s += part[i];
+  return s;
+}
+
 // One workgroup (4 waves) per board, persistent over a contiguous run of boards, as
 // fused_forward_kernel.
 template <class P>
@@ -215,8 +224,7 @@ __global__ __launch_bounds__(256) void split_forward_kernel(const FwdParams prm)
   using G = Geo<P>;
   using S = SplitGeo;
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
-  constexpr int THREADS = 256, NWAVES = THREADS / 64;
-  constexpr int ROUNDS = (kPix + THREADS - 1) / THREADS;
+  constexpr int THREADS = 256, ROUNDS = (kPix + THREADS - 1) / THREADS;
   const int tid = threadIdx.x;
   const int lane = tid & 63;
   const int wave = tid >> 6;
@@ -236,7 +244,7 @@ __global__ __launch_bounds__(256) void split_forward_kernel(const FwdParams prm)
   unsigned char *occ = smem + S::OCC_OFF;
   float *lgt = reinterpret_cast<float *>(smem + S::LGT_OFF);
   float *red = reinterpret_cast<float *>(smem + S::RED_OFF);
-  int *flags = reinterpret_cast<int *>(red) + 8;   // [0]: third plane varies, [1]: an input is not exact in bf16
+  int *flags = reinterpret_cast<int *>(red) + 40;   // [0]: third plane varies, [1]: an input is not exact in bf16
 
   const unsigned per_group = (unsigned)prm.boards_per_group;
   auto packed_of = [&](long long b) { return prm.packed + (size_t)((unsigned)b / per_group) * prm.packed_stride; };
@@ -308,13 +316,13 @@ __global__ __launch_bounds__(256) void split_forward_kernel(const FwdParams prm)
     }
     // ---- stage the input: zero the shifted copies, then scatter the board ----
     if (tid < 2) flags[tid] = 0;
-    if (tid == 0) red[4] = xin[0][2];   // the third plane's value at square 0
+    if (tid == 0) red[42] = xin[0][2];   // the third plane's value at square 0
     {
       const v4i z = {0, 0, 0, 0};
       for (int i = tidv * 16; i < G::COPIES_BYTES; i += THREADS * 16) *reinterpret_cast<v4i *>(smem + i) = z;
     }
     __syncthreads();
-    const float c2 = red[4];
+    const float c2 = red[42];
     {
       bool varies = false, inexact = false;
 #pragma unroll
@@ -441,43 +449,42 @@ __global__ __launch_bounds__(256) void split_forward_kernel(const FwdParams prm)
       asm volatile("" : "+v"(th));
 #pragma unroll
       for (int j = 0; j < 3; ++j) pix[j] = tile_pixel(th, j, valid[j]);
-      float pol[3] = {0.0f, 0.0f, 0.0f};
-      float vsum = 0.0f;
+      // Partial sums per cout tile and tile of 32 squares, added up in a fixed order: what
+      // the kernel that shares a board between workgroups can reproduce.
+      float tot[3];
 #pragma unroll
-      for (int t = 0; t < 3; ++t)
+      for (int t = 0; t < 3; ++t) {
+        float pol[3] = {0.0f, 0.0f, 0.0f}, val[3] = {0.0f, 0.0f, 0.0f};
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
           const f32x4 pw = *(GlobalF32x4)(pwg + 32 * t + 8 * q);
           const f32x4 vw = *(GlobalF32x4)(pwg + kHeadC + 32 * t + 8 * q);
 #pragma unroll
-          for (int j = 0; j < 3; ++j) {
-            float vs = 0.0f;
+          for (int j = 0; j < 3; ++j)
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
               const float a = split_silu(acc[t][j][4 * q + e]);
               pol[j] = fmaf(a, pw[e], pol[j]);
-              vs = fmaf(a, vw[e], vs);
+              val[j] = fmaf(a, vw[e], val[j]);
             }
-            vsum += valid[j] ? vs : 0.0f;
-          }
         }
+#pragma unroll
+        for (int j = 0; j < 3; ++j) {
+          const unsigned bits = __builtin_bit_cast(unsigned, pol[j]);
+          const auto r = __builtin_amdgcn_permlane32_swap(bits, bits, false, false);  // the other lane half's channels
+          const unsigned r0 = r[0], r1 = r[1];
+          const float both = __builtin_bit_cast(float, r0) + __builtin_bit_cast(float, r1);
+          tot[j] = t == 0 ? both : tot[j] + both;
+          const float vs = wave_sum(valid[j] ? val[j] : 0.0f);
+          if (lane == 0) red[t * 12 + 3 * wave + j] = vs;
+        }
+      }
       const float polb = valw[kHeadC], valb = valw[kHeadC + 1];
 #pragma unroll
-      for (int j = 0; j < 3; ++j) {  // add the other lane half's channels
-        const unsigned bits = __builtin_bit_cast(unsigned, pol[j]);
-        const auto r = __builtin_amdgcn_permlane32_swap(bits, bits, false, false);
-        const unsigned r0 = r[0], r1 = r[1];
-        if (h == 0 && valid[j]) lgt[pix[j]] = __builtin_bit_cast(float, r0) + __builtin_bit_cast(float, r1) + polb;
-      }
-      vsum = wave_sum(vsum);
-      if (lane == 0) red[wave] = vsum;
+      for (int j = 0; j < 3; ++j)
+        if (h == 0 && valid[j]) lgt[pix[j]] = tot[j] + polb;
       __syncthreads();
-      if (tid == 0 && prm.value != nullptr) {
-        float s = 0.0f;
-#pragma unroll
-        for (int w = 0; w < NWAVES; ++w) s += red[w];
-        prm.value[b] = tanhf(s * (1.0f / kPix) + valb);
-      }
+      if (tid == 0 && prm.value != nullptr) prm.value[b] = tanhf(split_value_sum(red) * (1.0f / kPix) + valb);
     }
     // ---- write out: masked logits, optional sampled action ----
     if (prm.logits != nullptr) {

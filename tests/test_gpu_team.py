@@ -1,0 +1,131 @@
+"""Several workgroups per board (c6_forward_team) against the one-workgroup kernels: the same bits at
+every batch size on either side of a change of the team's size, also when no workgroup waits for
+another for long (each then computes what it misses), in graphs and on two streams at once."""
+import ctypes
+
+import pytest
+import torch
+
+import connect6_amd as c6
+from connect6_amd import _lib
+from connect6_amd.model import run_forward
+from connect6_amd.synthetic import gen_boards, gen_uniform
+from oracle import torch_ref as R
+
+pytestmark = pytest.mark.gpu
+MODES = [_lib.PREC_F32S]
+
+
+def _model(cuda, seed=11):
+    model = c6.PolicyValueNet().to(cuda).eval()
+    model.load_state_dict(R.init_state(seed, "torch_default"))
+    return model
+
+
+def _inputs(n):
+    x, legal = gen_boards(n, 200, 77)
+    x[3::5, 2] = (torch.rand(19, 19, generator=torch.Generator().manual_seed(1)) > 0.5).float()   # a varying third plane
+    x[4::5] *= 0.3                                                                                # not exact in bf16
+    return x, legal
+
+
+def _team(prec, x, packed, tag, flags, polls=0, **kw):
+    """c6_forward_team through the C ABI: logits, value."""
+    lib, b = c6.load(), x.shape[0]
+    ws, fl = ctypes.c_size_t(), ctypes.c_size_t()
+    assert lib.c6_team_bytes(prec, b, ctypes.byref(ws), ctypes.byref(fl)) == 0 and ws.value > 0
+    assert flags.numel() * 4 >= fl.value
+    work = torch.full((ws.value,), 255, dtype=torch.uint8, device=x.device)
+    logits, value = torch.empty(b, 361, device=x.device), torch.empty(b, device=x.device)
+    rc = lib.c6_forward_team(x.data_ptr(), 0, 1, b, packed.data_ptr(), packed.numel(), prec, logits.data_ptr(),
+                             value.data_ptr(), 0, None, 0.0, None, 1.0, None, None, work.data_ptr(), ws.value,
+                             flags.data_ptr(), flags.numel() * 4, tag, polls, _lib.stream_ptr(x.device))
+    _lib.check(rc, "c6_forward_team")
+    return logits, value
+
+
+@pytest.mark.parametrize("prec", MODES)
+def test_same_bits_as_one_workgroup_per_board(cuda, prec):
+    model, (x, legal) = _model(cuda), _inputs(300)
+    xd, ld, u = x.to(cuda), legal.to(cuda), gen_uniform(300, 5).to(cuda)
+    packed = model.packed_weights(prec)
+    with torch.inference_mode():
+        kw = dict(mask_mode=_lib.MASK_LEGAL, u=u, temperature=0.8, want_logprob=True)
+        want = run_forward(xd, packed, prec, 1, 300, legal=ld, **kw)
+        for n in (1, 2, 5, 27, 28, 29, 84, 85, 86):
+            kw["u"] = u[:n]
+            got = run_forward(xd[:n], packed, prec, 1, n, legal=ld[:n], **kw)
+            for a, b in zip(got, want):
+                assert torch.equal(a, b[:n]), n
+        raw = run_forward(xd, packed, prec, 1, 300)
+        for n in (1, 40):
+            got = run_forward(xd[7:7 + n], packed, prec, 1, n)
+            assert torch.equal(got[0], raw[0][7:7 + n]) and torch.equal(got[1], raw[1][7:7 + n])
+        # several weight sets, and board states through a view and an index
+        sets = torch.cat([packed, _model(cuda, 12).packed_weights(prec)])
+        a = run_forward(xd[:6], sets, prec, 2, 3)
+        assert torch.equal(a[0][:3], raw[0][:3])
+        assert torch.equal(a[0][3:], run_forward(xd[3:6], sets[packed.numel():], prec, 1, 3)[0])
+
+
+@pytest.mark.parametrize("prec", MODES)
+@pytest.mark.parametrize("boards", [1, 7, 40])
+def test_a_workgroup_that_waited_long_enough_does_the_work_itself(cuda, prec, boards):
+    model, (x, _) = _model(cuda), _inputs(boards)
+    xd = x.to(cuda)
+    packed = model.packed_weights(prec)
+    flags = torch.zeros(boards * 96, dtype=torch.int32, device=cuda)
+    with torch.inference_mode():
+        want = run_forward(torch.cat([xd] * (300 // boards + 1)), packed, prec, 1, boards * (300 // boards + 1))
+        for tag, polls in ((1, 0), (2, 1), (3, 2), (4, 5)):
+            lg, vg = _team(prec, xd, packed, tag, flags, polls)
+            assert torch.equal(lg, want[0][:boards]) and torch.equal(vg, want[1][:boards]), polls
+
+
+def test_boards_states_views_and_index(cuda):
+    model, (x, _) = _model(cuda), gen_boards(300, 200, 5)
+    boards = (x[:, 0] - x[:, 1]).to(torch.int8).to(cuda)
+    player = torch.where(torch.arange(300) % 3 == 0, -1, 1).to(torch.int8).to(cuda)
+    left = torch.where(torch.arange(300) % 2 == 0, 1, 2).to(torch.int8).to(cuda)
+    u = gen_uniform(300, 6).to(cuda)
+    index = torch.randperm(300, generator=torch.Generator().manual_seed(3)).to(cuda)
+    with torch.inference_mode():
+        la, va = model.forward_boards(boards, player, left, index=index, view=6)
+        lb, vb = model.forward_boards(boards, player, left, index=index[:20], view=6)
+        assert torch.equal(la[:20], lb) and torch.equal(va[:20], vb)
+        a = model.selfplay_step_boards(boards, player, left, u, 0.7, index=index, view=3)
+        b = model.selfplay_step_boards(boards, player, left, u[:50], 0.7, index=index[:50], view=3)
+        for p, q in zip(a, b):
+            assert torch.equal(p[:50], q)
+
+
+def test_graphs_and_streams(cuda):
+    model, (x, _) = _model(cuda), _inputs(20)
+    xs = [torch.roll(x, i, 0).to(cuda) for i in range(3)]
+    with torch.inference_mode():
+        want = [model(v) for v in xs]
+        static = xs[0].clone()
+        side = torch.cuda.Stream()
+        side.wait_stream(torch.cuda.current_stream())
+        with torch.cuda.stream(side):
+            model(static)
+        torch.cuda.current_stream().wait_stream(side)
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph):
+            out = model(static)
+        for i in (0, 1, 2, 1, 0):
+            static.copy_(xs[i])
+            graph.replay()
+            model(xs[2])                       # eager work in between
+            torch.cuda.synchronize()
+            assert torch.equal(out[0], want[i][0]) and torch.equal(out[1], want[i][1]), i
+        streams = [torch.cuda.Stream() for _ in range(3)]
+        torch.cuda.synchronize()
+        got = []
+        for r in range(6):
+            for i, s in enumerate(streams):
+                with torch.cuda.stream(s):
+                    got.append((i, model(xs[i])))
+        torch.cuda.synchronize()
+        for i, (lg, vg) in got:
+            assert torch.equal(lg, want[i][0]) and torch.equal(vg, want[i][1])

@@ -56,6 +56,8 @@ EXPORTS = (
     "c6_team_bytes",
     "c6_forward_team",
     "c6_forward_boards_team",
+    "c6_forward_cascade_team",
+    "c6_forward_boards_cascade_team",
     "c6_stream_capturing",
     "c6_generic_packed_bytes",
     "c6_generic_pack",
@@ -86,7 +88,8 @@ def build(verbose: bool = False) -> Path:
     ]
     # one object file per source and, for the fused kernels, per arithmetic mode
     units = [(s, ["-DC6_SPLIT"] if s == "c6_forward.hip" else []) for s in _SOURCES]
-    units = [("c6_forward.hip", [f"-DC6_INSTANCE={m}"]) for m in _MODES] + units
+    units = [("c6_forward.hip", [f"-DC6_INSTANCE={m}"] + team) for team in (["-DC6_TEAM"], []) for m in _MODES
+             if not (team and m == "PrecF32")] + units
     with tempfile.TemporaryDirectory(dir=_LIBDIR) as tmp:
         objs = [str(Path(tmp) / f"{i}.o") for i in range(len(units))]
 
@@ -131,7 +134,7 @@ _HOST_SO = _LIBDIR / "_c6_host.so"
 _HOST_ABI = ("c6_forward", "c6_forward_cascade", "c6_forward_boards", "c6_forward_boards_cascade",
              "c6_cascade_workspace_bytes", "c6_mask_logits", "c6_softmax_sample", "c6_env_step", "c6_canonical_input",
              "c6_forward_generic_packed", "c6_team_bytes", "c6_forward_team", "c6_forward_boards_team",
-             "c6_stream_capturing")
+             "c6_stream_capturing", "c6_forward_cascade_team", "c6_forward_boards_cascade_team")
 
 
 def build_host() -> Path:
@@ -276,6 +279,10 @@ def load() -> ctypes.CDLL:
     lib.c6_forward_team.argtypes = lib.c6_forward.argtypes[:-1] + team
     lib.c6_forward_boards_team.restype = i32
     lib.c6_forward_boards_team.argtypes = lib.c6_forward_boards.argtypes[:-1] + team
+    lib.c6_forward_cascade_team.restype = i32
+    lib.c6_forward_cascade_team.argtypes = lib.c6_forward_cascade.argtypes[:-1] + team
+    lib.c6_forward_boards_cascade_team.restype = i32
+    lib.c6_forward_boards_cascade_team.argtypes = lib.c6_forward_boards_cascade.argtypes[:-1] + team
     lib.c6_stream_capturing.restype = i32
     lib.c6_stream_capturing.argtypes = [vp]
     ip = ctypes.POINTER(ctypes.c_int)

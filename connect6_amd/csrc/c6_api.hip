@@ -19,7 +19,8 @@ void set_error(const char *fmt, ...) {
 
 int dispatch_pack(int prec, const PackParams &pp, hipStream_t st);
 int dispatch_forward(int prec, const FwdParams &fp, hipStream_t st);
-int dispatch_cascade(int prec, const FwdParams &fp, float threshold, void *workspace, hipStream_t st);
+int dispatch_cascade(int prec, const FwdParams &fp, float threshold, void *workspace, const TeamParams *team,
+                     hipStream_t st);
 int team_workspace_bytes(int prec, long long boards, size_t *bytes);
 int dispatch_team(int prec, const TeamParams &tp, hipStream_t st);
 size_t packed_bytes(int prec);
@@ -115,27 +116,38 @@ struct TeamArgs {
 constexpr int kTeamPolls = 64;   // about 45 us
 
 
-static int run_team(const char *who, int prec, const FwdParams &fp, const TeamArgs &t, hipStream_t st) {
+// checked into `tp` (all but the forward's own parameters)
+static int check_team(const char *who, int prec, long long boards, const TeamArgs &t, TeamParams &tp) {
   size_t need = 0;
-  const int rc = team_workspace_bytes(prec, fp.total_boards, &need);
+  const int rc = team_workspace_bytes(prec, boards, &need);
   if (rc != C6_OK) return rc;
   if (need == 0) {
-    set_error("%s: %lld boards of mode %d are served by one workgroup each (c6_team_bytes is 0)", who, fp.total_boards,
-              prec);
+    set_error("%s: %lld boards of mode %d are served by one workgroup each (c6_team_bytes is 0)", who, boards, prec);
     return C6_EINVAL;
   }
   if (t.workspace == nullptr || !aligned16(t.workspace) || t.workspace_bytes < need || t.flags == nullptr ||
-      t.flag_bytes < (size_t)fp.total_boards * kTeamFlags * 4 || t.tag == 0) {
-    set_error("%s: needs a 16-byte aligned workspace and flag words of the sizes c6_team_bytes gives, and a tag that is "
-              "not 0", who);
+      t.flag_bytes < (size_t)boards * kTeamFlags * 4 || t.tag == 0 || t.tag == 0xffffffffu) {
+    set_error("%s: needs a 16-byte aligned workspace and flag words of the sizes c6_team_bytes gives, and a tag from 1 "
+              "to 2^32 - 2", who);
     return C6_EINVAL;
   }
-  TeamParams tp;
-  tp.f = fp;
   tp.act = static_cast<unsigned char *>(t.workspace);
   tp.flags = t.flags;
   tp.tag = t.tag;
   tp.polls = t.polls > 0 ? t.polls : kTeamPolls;
+  return C6_OK;
+}
+
+// a forward whose arguments have been checked
+static int dispatch(const char *who, int prec, const FwdParams &fp, bool cascade, float threshold, void *workspace,
+                    const TeamArgs *team, hipStream_t st) {
+  if (team == nullptr)
+    return cascade ? dispatch_cascade(prec, fp, threshold, workspace, nullptr, st) : dispatch_forward(prec, fp, st);
+  TeamParams tp;
+  const int rc = check_team(who, prec, fp.total_boards, *team, tp);
+  if (rc != C6_OK) return rc;
+  if (cascade) return dispatch_cascade(prec, fp, threshold, workspace, &tp, st);
+  tp.f = fp;
   return dispatch_team(prec, tp, st);
 }
 
@@ -277,9 +289,7 @@ static int forward_planes(const char *who, const void *x, int x_dtype, int64_t g
     if (rc != C6_OK) return rc;
   }
   C6_REQUIRE_DEVICE(who);
-  if (team != nullptr) return run_team(who, prec, fp, *team, static_cast<hipStream_t>(stream));
-  if (cascade) return dispatch_cascade(prec, fp, threshold, workspace, static_cast<hipStream_t>(stream));
-  return dispatch_forward(prec, fp, static_cast<hipStream_t>(stream));
+  return dispatch(who, prec, fp, cascade, threshold, workspace, team, static_cast<hipStream_t>(stream));
 }
 
 int c6_forward(const void *x, int x_dtype, int64_t groups, int64_t boards_per_group,
@@ -373,9 +383,7 @@ static int forward_states(const char *who, const int8_t *boards, const int8_t *p
     if (rc != C6_OK) return rc;
   }
   C6_REQUIRE_DEVICE(who);
-  if (team != nullptr) return run_team(who, prec, fp, *team, static_cast<hipStream_t>(stream));
-  if (cascade) return dispatch_cascade(prec, fp, threshold, workspace, static_cast<hipStream_t>(stream));
-  return dispatch_forward(prec, fp, static_cast<hipStream_t>(stream));
+  return dispatch(who, prec, fp, cascade, threshold, workspace, team, static_cast<hipStream_t>(stream));
 }
 
 int c6_forward_boards(const int8_t *boards, const int8_t *player, const int8_t *stones_left,
@@ -442,6 +450,31 @@ int c6_forward_boards_team(const int8_t *boards, const int8_t *player, const int
   return forward_states("c6_forward_boards_team", boards, player, stones_left, num_states, index, view, batch, packed,
                         prec, logits, C6_DT_F32, value, mask_mode, fill, u, temperature, actions, logprob, false, 0.0f,
                         nullptr, 0, stream, &t);
+}
+
+int c6_forward_cascade_team(const void *x, int x_dtype, int64_t groups, int64_t boards_per_group,
+                            const void *packed, size_t packed_stride, int prec, void *logits, int logits_dtype,
+                            float *value, int mask_mode, const uint8_t *legal, float fill, const float *u,
+                            float temperature, int64_t *actions, float *logprob, float threshold,
+                            void *cascade_workspace, size_t cascade_bytes, void *workspace, size_t workspace_bytes,
+                            void *flags, size_t flag_bytes, uint32_t tag, int polls, void *stream) {
+  const TeamArgs t{workspace, workspace_bytes, static_cast<unsigned *>(flags), flag_bytes, tag, polls};
+  return forward_planes("c6_forward_cascade_team", x, x_dtype, groups, boards_per_group, packed, packed_stride, prec,
+                        logits, logits_dtype, value, mask_mode, legal, fill, u, temperature, actions, logprob, true,
+                        threshold, cascade_workspace, cascade_bytes, stream, &t);
+}
+
+int c6_forward_boards_cascade_team(const int8_t *boards, const int8_t *player, const int8_t *stones_left,
+                                   int64_t num_states, const int64_t *index, int view, int64_t batch,
+                                   const void *packed, int prec, void *logits, int logits_dtype, float *value,
+                                   int mask_mode, float fill, const float *u, float temperature, int64_t *actions,
+                                   float *logprob, float threshold, void *cascade_workspace, size_t cascade_bytes,
+                                   void *workspace, size_t workspace_bytes, void *flags, size_t flag_bytes,
+                                   uint32_t tag, int polls, void *stream) {
+  const TeamArgs t{workspace, workspace_bytes, static_cast<unsigned *>(flags), flag_bytes, tag, polls};
+  return forward_states("c6_forward_boards_cascade_team", boards, player, stones_left, num_states, index, view, batch,
+                        packed, prec, logits, logits_dtype, value, mask_mode, fill, u, temperature, actions, logprob,
+                        true, threshold, cascade_workspace, cascade_bytes, stream, &t);
 }
 
 static int check_arch(const char *who, int board, int layers, const int *kernels,

@@ -285,6 +285,7 @@ struct FwdParams {
   int *redo_list = nullptr;       // run r's list starts at entry r * redo_per
   int redo_runs = 0;              // workgroups (runs of boards) of the first pass
   int redo_per = 0;               // boards per run of the first pass
+  int redo_skip = -1;             // second pass: up to this many listed boards are another launch's
 };
 
 // Few boards: several workgroups per board (c6_team.h)
@@ -295,7 +296,7 @@ struct TeamParams {
   unsigned tag;
   int polls;            // of a flag (about 0.7 us each) before a workgroup helps itself
 };
-constexpr int kTeamFlags = 96;                   // words per board: stage * 9 + role
+constexpr int kTeamFlags = 256;   // words per board
 
 struct PackParams {
   const float *conv_w[8];     // each tensor stacked over the weight sets: [groups, ...]

@@ -1288,6 +1288,7 @@ __global__ __launch_bounds__(256) void fused_pipe_kernel(const FwdParams prm) {
     }
     __syncthreads();
     n_items = (unsigned)before;
+    if (before <= prm.redo_skip) return;
   }
   // listed board i: the run r with runs[r] <= i < runs[r + 1] (a bisection; the same in every thread)
   auto board_of = [&](unsigned i) {
@@ -1907,7 +1908,9 @@ __global__ __launch_bounds__(256) void fused_forward_kernel(const FwdParams prm)
 }  // namespace c6
 
 #include "c6_split.h"
+#if defined(C6_TEAM) || !defined(C6_INSTANCE)
 #include "c6_team.h"
+#endif
 
 namespace c6 {
 
@@ -2150,13 +2153,13 @@ template <class P> __global__ __launch_bounds__(256) void lo_scale_kernel(const 
 // ------------------------------------------------------------------------
 // host side
 // ------------------------------------------------------------------------
-// The library is built with one object file per arithmetic mode (the compiler takes a minute and
-// more for each): C6_INSTANCE names the mode of this object file, C6_SPLIT marks the one that holds
-// the dispatch.  Without either, this file is all of them (what a traced copy is built from).
+// The library is built with two object files per arithmetic mode (the compiler takes a minute and
+// more for each): C6_INSTANCE names the mode of this object file, C6_TEAM marks the one that holds its
+// team kernel, C6_SPLIT the one that holds the dispatch.  Without either, this file is all of them (what a traced copy is built from).
 template <class P> int launch_pack(const PackParams &pp, hipStream_t st);
 template <class P> int launch_forward(const FwdParams &fp, hipStream_t st);
 
-template <class P> int launch_team(const TeamParams &tp, int team, hipStream_t st);
+template <class P> int launch_team(const TeamParams &tp, int grid, hipStream_t st);
 
 #ifndef C6_SPLIT
 template <class P> int launch_pack(const PackParams &pp, hipStream_t st) {
@@ -2222,19 +2225,19 @@ template <class P> int launch_forward(const FwdParams &fp, hipStream_t st) {
   return C6_OK;
 }
 
-template <class P, int TEAM> static int launch_team_of(const TeamParams &tp, hipStream_t st) {
+#if defined(C6_TEAM) || !defined(C6_INSTANCE)
+template <class P> int launch_team(const TeamParams &tp, int grid, hipStream_t st) {
   using T = TeamGeo<P>;
   static thread_local int configured = -1;
   int dev = 0;
   hipError_t e = hipGetDevice(&dev);
   if (e == hipSuccess && configured != dev) {
-    e = hipFuncSetAttribute(reinterpret_cast<const void *>(&team_forward_kernel<P, TEAM>),
+    e = hipFuncSetAttribute(reinterpret_cast<const void *>(&team_forward_kernel<P>),
                             hipFuncAttributeMaxDynamicSharedMemorySize, T::LDS_BYTES);
     if (e == hipSuccess) configured = dev;
   }
   if (e == hipSuccess) {
-    hipLaunchKernelGGL((team_forward_kernel<P, TEAM>), dim3((unsigned)(tp.f.total_boards * TEAM)), dim3(256), T::LDS_BYTES,
-                       st, tp);
+    hipLaunchKernelGGL(team_forward_kernel<P>, dim3((unsigned)grid), dim3(256), T::LDS_BYTES, st, tp);
     e = hipGetLastError();
   }
   if (e != hipSuccess) {
@@ -2243,22 +2246,17 @@ template <class P, int TEAM> static int launch_team_of(const TeamParams &tp, hip
   }
   return C6_OK;
 }
-
-template <class P> int launch_team(const TeamParams &tp, int team, hipStream_t st) {
-  if constexpr (has_team<P>()) {
-    return team == 9 ? launch_team_of<P, 9>(tp, st) : launch_team_of<P, 3>(tp, st);
-  } else {
-    set_error("this mode has no team kernel");
-    return C6_EINVAL;
-  }
-}
+#endif
 
 #endif  // C6_SPLIT
 
 #ifdef C6_INSTANCE
+#ifdef C6_TEAM
+template int launch_team<C6_INSTANCE>(const TeamParams &, int, hipStream_t);
+#else
 template int launch_pack<C6_INSTANCE>(const PackParams &, hipStream_t);
 template int launch_forward<C6_INSTANCE>(const FwdParams &, hipStream_t);
-template int launch_team<C6_INSTANCE>(const TeamParams &, int, hipStream_t);
+#endif
 #else
 
 int dispatch_pack(int prec, const PackParams &pp, hipStream_t st) {
@@ -2315,12 +2313,65 @@ static int device_cus(int &cus) {
   return C6_OK;
 }
 
+// ---- few boards: c6_team.h ----
+struct TeamMode {
+  size_t board_bytes;                          // exchange memory per board
+  int (*size)(long long boards, int wgs);      // workgroups per board
+  long long (*most)(int wgs);                  // boards that are shared at all
+  int (*launch)(const TeamParams &, int grid, hipStream_t);
+};
+template <class P> static TeamMode team_mode_of() { return {TeamGeo<P>::BOARDB, &team_size<P>, &team_most<P>, &launch_team<P>}; }
+static TeamMode team_mode(int prec) {
+  switch (prec) {
+    case C6_PREC_F32S: return team_mode_of<PrecF32S>();
+    case C6_PREC_BF16: return team_mode_of<PrecBF16>();
+    case C6_PREC_F16: return team_mode_of<PrecF16>();
+    case C6_PREC_BF16F6: return team_mode_of<PrecBF16F6>();
+    case C6_PREC_BF16F6W: return team_mode_of<PrecBF16F6W>();
+  }
+  return {0, nullptr, nullptr, nullptr};
+}
+static int second_mode(int cascade) { return cascade == C6_PREC_BF16C ? C6_PREC_BF16F6W : C6_PREC_BF16F6; }
+// The cascade's second pass goes to teams where it will hardly list more boards than they take (42 of 256
+// CUs with low weights, 21 without): random networks with the reference's initialisation list 6 %.  Where
+// it could list more, the launch that the teams cannot serve costs 4 us before the ordinary one.
+static long long team_cascade_boards(int prec, int cus) { return 16 * team_mode(second_mode(prec)).most(cus); }
+
+// Exchange memory for `boards` boards of a mode, 0 where one workgroup per board serves them.
+int team_workspace_bytes(int prec, long long boards, size_t *bytes) {
+  int cus = 0;
+  *bytes = 0;
+  if (boards < 1) return C6_OK;
+  const int rc = device_cus(cus);
+  if (rc != C6_OK) return rc;
+  if (is_cascade(prec)) {
+    const TeamMode first = team_mode(C6_PREC_BF16), second = team_mode(second_mode(prec));
+    if (boards > team_cascade_boards(prec, cus)) return C6_OK;
+    const long long teams = second.most(cus);
+    *bytes = second.board_bytes * (size_t)(boards < teams ? boards : teams);
+    if (first.size(boards, cus) > 1 && first.board_bytes * (size_t)boards > *bytes) *bytes = first.board_bytes * (size_t)boards;
+  } else {
+    const TeamMode m = team_mode(prec);
+    if (m.launch != nullptr && m.size(boards, cus) > 1) *bytes = m.board_bytes * (size_t)boards;
+  }
+  return C6_OK;
+}
+int dispatch_team(int prec, const TeamParams &tp, hipStream_t st) {
+  int cus = 0;
+  const int rc = device_cus(cus);
+  if (rc != C6_OK) return rc;
+  const TeamMode m = team_mode(prec);
+  return m.launch(tp, (int)tp.f.total_boards * m.size(tp.f.total_boards, cus), st);
+}
+
 // Cascade: every board through the plain bf16 kernel, whose workgroups list those of their boards
 // whose decision margin is below `threshold`; then the listed boards through the kernel that also
 // carries the low parts of activations and (C6_PREC_BF16C) weights, which overwrites their
-// outputs.  Two launches on the caller's stream, no host synchronisation, no atomic operation and
-// nothing to clear: the second kernel reads how many boards each workgroup of the first listed.
-int dispatch_cascade(int prec, const FwdParams &fp, float threshold, void *workspace, hipStream_t st) {
+// outputs.  Two launches on the caller's stream (three where listed boards may share workgroups or
+// not, depending on their number: `team`), no host synchronisation, no atomic operation on the lists and nothing to clear:
+// the second kernel reads how many boards each workgroup of the first listed.
+int dispatch_cascade(int prec, const FwdParams &fp, float threshold, void *workspace, const TeamParams *team,
+                     hipStream_t st) {
   int cus = 0;
   int rc = device_cus(cus);
   if (rc != C6_OK) return rc;
@@ -2338,35 +2389,27 @@ int dispatch_cascade(int prec, const FwdParams &fp, float threshold, void *works
   first.redo_list = ws + 4 + kCascadeMaxRuns;
   first.redo_runs = (int)runs;
   first.redo_per = (int)((fp.total_boards + runs - 1) / runs);
-  rc = launch_forward<PrecBF16>(first, st);
-  if (rc != C6_OK) return rc;
   FwdParams second = first;
   second.packed = fp.packed + kCascadeSecondOffset;
   second.redo_mode = kRedoConsume;
-  return prec == C6_PREC_BF16C ? launch_forward<PrecBF16F6W>(second, st) : launch_forward<PrecBF16F6>(second, st);
-}
-
-// Bytes per board that the mode's team kernel keeps in memory; 0 where the mode has none.
-static size_t team_board_bytes(int prec) {
-  return prec == C6_PREC_F32S ? TeamGeo<PrecF32S>::BOARDB : 0;
-}
-// Workspace for `boards` boards of a mode, 0 where one workgroup per board serves them.
-int team_workspace_bytes(int prec, long long boards, size_t *bytes) {
-  int cus = 0;
-  *bytes = 0;
-  const size_t per = team_board_bytes(prec);
-  if (per == 0 || boards < 1) return C6_OK;
-  const int rc = device_cus(cus);
-  if (rc == C6_OK && team_size(boards, cus) > 1) *bytes = per * (size_t)boards;
-  return rc;
-}
-int dispatch_team(int prec, const TeamParams &tp, hipStream_t st) {
-  int cus = 0;
-  const int rc = device_cus(cus);
+  if (team == nullptr) {
+    rc = launch_forward<PrecBF16>(first, st);
+  } else {
+    TeamParams tp = *team;
+    tp.f = first;
+    rc = team_size<PrecBF16>(fp.total_boards, cus) > 1 ? dispatch_team(C6_PREC_BF16, tp, st)
+                                                       : launch_forward<PrecBF16>(first, st);
+    if (rc != C6_OK) return rc;
+    // teams for as many listed boards as they take, the ordinary launch for more
+    tp.f = second;
+    tp.tag = team->tag + 1;
+    const TeamMode teams = team_mode(second_mode(prec));
+    rc = teams.launch(tp, cus, st);
+    if (fp.total_boards <= teams.most(cus)) return rc;
+    second.redo_skip = (int)teams.most(cus);
+  }
   if (rc != C6_OK) return rc;
-  const int team = team_size(tp.f.total_boards, cus);
-  if (team == 1 || team_board_bytes(prec) == 0) return dispatch_forward(prec, tp.f, st);
-  return launch_team<PrecF32S>(tp, team, st);
+  return prec == C6_PREC_BF16C ? launch_forward<PrecBF16F6W>(second, st) : launch_forward<PrecBF16F6>(second, st);
 }
 
 size_t packed_bytes(int prec) {

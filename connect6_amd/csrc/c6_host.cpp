@@ -37,6 +37,8 @@ struct Abi {
   decltype(&c6_forward_team) forward_team;
   decltype(&c6_forward_boards_team) forward_boards_team;
   decltype(&c6_stream_capturing) stream_capturing;
+  decltype(&c6_forward_cascade_team) forward_cascade_team;
+  decltype(&c6_forward_boards_cascade_team) forward_boards_cascade_team;
 } abi;
 
 PyObject *fail(PyObject *type, const std::string &what) {
@@ -138,13 +140,14 @@ Team team_buffers(int prec, int64_t boards, const at::Device &dev, void *stream)
     kept.push_back(Kept{dev.index(), stream, {}, 0, 0});
     k = &kept.back();
   }
-  if (!k->flags.defined() || (size_t)k->flags.nbytes() < flag_bytes || k->tag == UINT32_MAX) {
+  if (!k->flags.defined() || (size_t)k->flags.nbytes() < flag_bytes || k->tag >= UINT32_MAX - 4) {
     k->flags = zeros((int64_t)(flag_bytes / 4));
     k->tag = 0;
   }
   k->used = ++clock;
   t.flags = k->flags;
-  t.tag = ++k->tag;
+  t.tag = k->tag + 1;
+  k->tag += 2;   // (a cascade's second pass takes the next one)
   return t;
 }
 
@@ -250,7 +253,14 @@ PyObject *forward(PyObject *, PyObject *const *a, Py_ssize_t n) {
   int rc;
   if (is_cascade(prec)) {
     ws = cascade_workspace(total, dev);
-    rc = abi.forward_cascade(x.data_ptr(), x_code, groups, per, packed.data_ptr(), stride, prec, ptr<void>(logits),
+    const Team t = team_buffers(prec, total, dev, stream);
+    rc = t.work.defined()
+             ? abi.forward_cascade_team(
+                   x.data_ptr(), x_code, groups, per, packed.data_ptr(), stride, prec, ptr<void>(logits), logits_code,
+                   ptr<float>(value), mask_mode, legal_ptr, fill, ptr<float>(u), temperature, ptr<int64_t>(actions),
+                   ptr<float>(logprob), threshold, ptr<void>(ws), ws.defined() ? ws.nbytes() : 0, t.work.data_ptr(),
+                   t.work.nbytes(), t.flags.data_ptr(), t.flags.nbytes(), t.tag, 0, stream)
+             : abi.forward_cascade(x.data_ptr(), x_code, groups, per, packed.data_ptr(), stride, prec, ptr<void>(logits),
                              logits_code, ptr<float>(value), mask_mode, legal_ptr, fill, ptr<float>(u), temperature,
                              ptr<int64_t>(actions), ptr<float>(logprob), threshold, ptr<void>(ws),
                              ws.defined() ? ws.nbytes() : 0, stream);
@@ -303,7 +313,15 @@ PyObject *forward_boards(PyObject *, PyObject *const *a, Py_ssize_t n) {
   int rc;
   if (is_cascade(prec)) {
     ws = cascade_workspace(total, dev);
-    rc = abi.forward_boards_cascade(ptr<int8_t>(boards), ptr<int8_t>(player), ptr<int8_t>(left), states,
+    const Team t = team_buffers(prec, total, dev, stream);
+    rc = t.work.defined()
+             ? abi.forward_boards_cascade_team(
+                   ptr<int8_t>(boards), ptr<int8_t>(player), ptr<int8_t>(left), states, ptr<int64_t>(index), view, total,
+                   packed.data_ptr(), prec, ptr<void>(logits), C6_DT_F32, ptr<float>(value), mask_mode, fill,
+                   ptr<float>(u), temperature, ptr<int64_t>(actions), ptr<float>(logprob), threshold, ptr<void>(ws),
+                   ws.defined() ? ws.nbytes() : 0, t.work.data_ptr(), t.work.nbytes(), t.flags.data_ptr(),
+                   t.flags.nbytes(), t.tag, 0, stream)
+             : abi.forward_boards_cascade(ptr<int8_t>(boards), ptr<int8_t>(player), ptr<int8_t>(left), states,
                                     ptr<int64_t>(index), view, total, packed.data_ptr(), prec, ptr<void>(logits),
                                     C6_DT_F32, ptr<float>(value), mask_mode, fill, ptr<float>(u), temperature,
                                     ptr<int64_t>(actions), ptr<float>(logprob), threshold, ptr<void>(ws),

@@ -1,58 +1,76 @@
 // Few boards: a TEAM of workgroups per board (included by c6_forward.hip).
 //
-// One workgroup per board leaves most of the chip idle when there are fewer boards than CUs, and a
-// single board takes as long as 256.  Here 9 (or 3) workgroups share a board: workgroup (s, t) takes
-// the third s of the squares (a wave: 32 of them) and, with 9, cout tile t of every layer; with 3 it
-// takes all cout tiles.  A layer's outputs go to memory as the next layer reads them, a flag says
-// that they are there, and every workgroup loads the rows it needs (its own and one above and below)
-// into LDS.  Each accumulator sees the same MFMAs in the same order as in the one-workgroup kernels,
-// so the results are the same bit for bit.
+// One workgroup per board leaves most of the chip idle when there are fewer boards than CUs, and one
+// board takes as long as 256.  Here 12, 6 or 3 workgroups share a board: each takes one, two or four
+// of the twelve tiles of 32 squares through all layers, its waves dividing tiles and output channels
+// between them.  A workgroup's own activations stay in its LDS; what a 3x3 layer reads beyond them,
+// twenty squares on either side, goes through memory: the owner stores its squares, waits until the
+// stores are acknowledged and raises a flag for the layer.  Each accumulator sees the same MFMAs in
+// the same order as in the one-workgroup kernels, and the heads' sums are put together in their
+// order, so the results are the same bit for bit.
 //
-// The exchange: stores and loads of the activations carry the device-scope cache policy (sc1), the
-// flags are relaxed device-scope atomics behind a wait for the stores.  Measured between two
-// workgroups: 0.8-0.95 us for a flag, 1.5 us with 4 KB behind it, the same within an XCD and across.
+// What it takes (cycles of a 2.4 GHz clock; twelve workgroups, one board): staging the input 7 k, then per
+// layer 1.4-3 k until the neighbours' flags are seen, 2 k until their squares are in LDS, the MFMAs (bf16
+// 1-2.6 k, fp32 4-12 k) and 2-3 k until the outputs are stored and acknowledged: bf16 37 us against 46,
+// bf16 + fp6 44 (63), with low weights 50 (90), fp32 64 (205; 53 boards on three workgroups each 130).
 //
-// What it costs and gives (fp32, one board, nine workgroups, 76 us against 201 us): per layer 0.6 us
-// to see a flag that is already set, 1.8-2.6 us to bring 190 squares from memory into LDS, 1.8 us until
-// the stores are acknowledged, and 2-5 us of MFMAs (each wave has one 32 x 32 tile, and its weights
-// saturate the L1's 64 bytes a cycle); 53 boards with three workgroups each take 128 us (208 us).
+// The exchange: stores and loads of activations carry the device-scope cache policy (sc1), flags are
+// relaxed device-scope atomics behind a wait for the stores.  Measured between two workgroups:
+// 0.8-0.95 us for a flag, 1.4 us with 4 KB behind it, 1.8 us with 32 KB, the same within an XCD and
+// across.
 //
 // Nothing waits for a workgroup that may not be running: a wait is bounded, and a workgroup whose
 // wait runs out does the missing piece of work itself (the earliest one that has no flag; everything
-// in front of it has one).  Outputs of every layer have a place of their own, and whoever computes
+// in front of it has one).  For that a workgroup also stores the squares that no neighbour reads, behind
+// its flag and with a second one.  Outputs of every layer have a place of their own, and whoever computes
 // a piece writes the same bytes, so doing one twice is harmless; any single workgroup can finish the
-// board alone.  The flags of a call are the call's tag: the caller hands a tag that the flag words
-// have not held before (or words that are zero).
+// board alone.  The flags of a launch are its tag: the caller hands a tag that the flag words have
+// not held before (or words that are zero).
 #pragma once
 
 namespace c6 {
 
-constexpr int kTeamStages = 9;                   // eight layers, then the heads' write-out
-constexpr int kSc1 = 16;                         // cache policy: device scope
+constexpr int kTeamStages = 9;   // eight layers, then the heads' write-out
+constexpr int kTeamAll = 128;    // flag words: see team_board
+constexpr int kSc1 = 16;         // cache policy: device scope
+static_assert(kTeamAll + kTeamStages * 12 <= kTeamFlags && kTeamStages * 12 <= kTeamAll, "flag words");
+
+// modes that have a team kernel
+template <class P> constexpr bool has_team() { return P::ID != C6_PREC_F32; }
 
 template <class P> struct TeamGeo {
   using G = Geo<P>;
-  static constexpr int NPL = P::ID == C6_PREC_F32S ? 3 : 1;   // planes of an activation
-  static constexpr int PXB = NPL * 64;                        // bytes of a square's 32 channels in memory
-  static constexpr int BLOCKB = kPix * PXB;                   // one cout tile of one layer
-  // memory per board: the outputs of layers 1 .. 7, then the heads' partial sums
+  static constexpr bool SPLIT = P::ID == C6_PREC_F32S;
+  static constexpr int NPL = SPLIT ? 3 : 1;                   // planes of an activation
+  static constexpr int LO_OFF = NPL * 192;                    // fp6 blocks of a record (LO6)
+  static constexpr int RECB = NPL * 192 + (P::LO6 ? 96 : 0) + 16;   // an odd number of 16-byte units
+  // a square of c channels in memory: 16-byte units of its planes, then of its fp6 blocks
+  static constexpr int units(int c) { return NPL * c / 8 + (P::LO6 ? c / 16 : 0); }
   static constexpr int act_off(int l) {
     int s = 0;
-    for (int i = 0; i < l; ++i) s += kCoutArr[i] / 32 * BLOCKB;
+    for (int i = 0; i < l; ++i) s += kPix * units(kCoutArr[i]) * 16;
     return s;
   }
-  static constexpr int HEAD_OFF = act_off(7);                 // [3][384] policy, then values
+  static constexpr int HEAD_OFF = act_off(7);                 // policy sums: SPLIT [3][384], else [384]
+  // value sums: SPLIT one per (cout tile, tile of squares), else nine per lane of each tile of squares
   static constexpr int VAL_OFF = HEAD_OFF + 3 * 384 * 4;
-  static constexpr int BOARDB = (VAL_OFF + 1024 * 4 + 255) & ~255;
-  // LDS: up to 11 rows of positions (a third of the squares lies in at most 8 board rows)
-  static constexpr int RECB = NPL * 192 + 16;
+  static constexpr int BOARDB = (VAL_OFF + 12 * 9 * 64 * 4 + 255) & ~255;
+  // LDS: up to 11 rows of positions (128 squares lie in at most 8 board rows)
   static constexpr int REGION = (11 * kPitch + 1) * RECB;
   static constexpr int BUF = REGION > G::COPIES_BYTES ? REGION : G::COPIES_BYTES;
   static constexpr int OCC_OFF = (BUF + 15) & ~15;
   static constexpr int LGT_OFF = OCC_OFF + 384;
   static constexpr int RED_OFF = LGT_OFF + 1456;
-  static constexpr int LDS_BYTES = RED_OFF + 256;
-  static_assert(LDS_BYTES <= 160 * 1024, "LDS map");
+  static constexpr int RUNS_OFF = RED_OFF + 256 * 4;
+  static constexpr int LDS_BYTES = RUNS_OFF + (kCascadeMaxRuns + 4) * 4;
+  static_assert(RECB / 16 % 2 == 1 && LDS_BYTES <= 160 * 1024, "LDS map");
+};
+
+// How a team divides the twelve tiles of squares and a layer's cout tiles: TEAM workgroups with PXT
+// tiles of squares each, whose four waves form CG groups of cout tiles.
+template <int TEAM> struct TeamShape {
+  static constexpr int PXT = 12 / TEAM, CG = PXT == 4 ? 1 : (PXT == 2 ? 2 : 3);
+  static constexpr int tiles(int nt) { return (nt + CG - 1) / CG; }   // cout tiles of a wave
 };
 
 // fragment (k-step k, cout tile t) of 3x3 layer L in the weight stream of mode P: first of its planes
@@ -68,32 +86,87 @@ template <class P, int L> __device__ __forceinline__ int team_frag(int k, int t)
   return (k * NT + t) * Geo<P>::W;
 }
 
-// The contraction of 3x3 layer L for one tile of 32 squares and TT cout tiles from t0 on.  rec: LDS
-// address of the lane's square's record one row and one column up, + 16 * lane half.
+// k-steps of weights that a wave keeps in flight: the loads take some 800 cycles and a k-step is
+// 32 cycles per MFMA
+template <class P, int TT> constexpr int team_ring() {
+  return Geo<P>::W == 3 ? 6 / TT : (Geo<P>::W == 1 ? 18 / TT : (TT == 1 ? 9 : (TT == 2 ? 6 : 3)));
+}
+
+// Low-order (fp6) pass of layer L for one tile of squares, conv3_lo_pass with TT cout tiles from t0 on.
+//   rec: LDS address of the lane's square's record
 template <class P, int L, int TT>
-__device__ __forceinline__ void team_conv(const unsigned char *smem, const WFrags &wl,
-                                          v4i (&ring)[(Geo<P>::W == 3 ? 6 : 18) / TT][TT][Geo<P>::W], int rec, int t0, f32x16 (&acc)[TT]) {
+__device__ __forceinline__ void team_lo_pass(const unsigned char *smem, const unsigned char *packed, int lane, int rec,
+                                             int t0, f32x16 (&acc)[TT]) {
+  using G = Geo<P>;
   using T = TeamGeo<P>;
-  constexpr int W = Geo<P>::W, NPL = T::NPL, D = (W == 3 ? 6 : 18) / TT;
+  typedef int v8i __attribute__((ext_vector_type(8)));
+  constexpr int NT = kCoutArr[L] / 32, PER32 = kCinArr[L] / 32, HC = G::lo_half_chunks(L), NC = G::lo_chunks(L);
+  const WFrags wl = packed_frags<P>(packed, lane, G::lo_frag_offset(L));
+  const int scale_w = 127 - reinterpret_cast<const int *>(packed + G::TAIL_OFF)[G::TAIL_SW + L];
+  constexpr int D = 4;
+  v4i w0[D][TT], w1[D][TT];
+  auto load = [&](int c, int d) __attribute__((always_inline)) {
+    const int cc = c < NC ? c : NC - 1;
+#pragma unroll
+    for (int t = 0; t < TT; ++t) {
+      const int tile = t0 + t < NT ? t0 + t : NT - 1;
+      lo_load_pieces<P>(wl + (cc * NT + tile) * 2, w0[d][t], w1[d][t]);
+    }
+  };
+#pragma unroll
+  for (int d = 0; d < D; ++d) load(d, d);
+  static_for<0, NC>([&](auto cc) __attribute__((always_inline)) {
+    constexpr int c = decltype(cc)::value;
+    constexpr int g0 = 2 * c, g1 = 2 * c + 1 < HC ? 2 * c + 1 : HC - 1;
+    constexpr int o0 = ((g0 / PER32 / 3 - 1) * kPitch + g0 / PER32 % 3 - 1) * T::RECB + (g0 % PER32) * 32;
+    constexpr int o1 = ((g1 / PER32 / 3 - 1) * kPitch + g1 / PER32 % 3 - 1) * T::RECB + (g1 % PER32) * 32;
+    const unsigned char *at = smem + rec + T::LO_OFF + (lane < 32 ? o0 : o1);
+    const v4i b0 = *reinterpret_cast<const v4i *>(at);
+    const v4i b1 = *reinterpret_cast<const v4i *>(at + 16);
+    const v8i b = {b0[0], b0[1], b0[2], b0[3], b1[0], b1[1], b1[2], b1[2]};
+#pragma unroll
+    for (int t = 0; t < TT; ++t) {
+      const v8i a = __builtin_shufflevector(w0[c % D][t], w1[c % D][t], 0, 1, 2, 3, 4, 5, 6, 7);
+      acc[t] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(a, b, acc[t], 2, 2, 0, scale_w, 0, b[6]);
+    }
+    load(c + D, c % D);
+    __builtin_amdgcn_sched_barrier(0);
+  });
+}
+
+// The contraction of 3x3 layer L for one tile of 32 squares and TT cout tiles from t0 on (tiles beyond
+// the layer's last repeat it; their results are not used).
+//   rec: LDS address of the lane's square's record;  acc: the bias on entry
+template <class P, int L, int TT>
+__device__ __forceinline__ void team_conv(const unsigned char *smem, const unsigned char *packed, const WFrags &wl,
+                                          v4i (&ring)[team_ring<P, TT>()][TT][Geo<P>::W], int lane, int rec, int t0,
+                                          f32x16 (&acc)[TT]) {
+  using T = TeamGeo<P>;
+  constexpr int NT = kCoutArr[L] / 32, NTP = kCinArr[L] / 32;
+  constexpr int W = Geo<P>::W, NPL = T::NPL, D = team_ring<P, TT>();
   constexpr int KC = kCinArr[L] / 16, KS = 9 * KC;
   constexpr int U = P::PIPE ? kPhaseSteps : 3 * KC;     // k-steps of one unrolled round
+  constexpr bool LO = P::LO6 && ((P::LO_MASK >> L) & 1);
   static_assert(KS % U == 0 && U % D == 0, "ring");
-  // k-step v of round r: (tap, 16 channels)
+  const int corner = rec - (kPitch + 1) * T::RECB + 16 * (lane >> 5);
+  // k-step v of round r: (tap, 16 channels).  Pipelined modes: a round is a phase, all taps of 32
+  // channels; fp32: a round is a kernel row.
   auto frag = [&](int r, int v, int pl) __attribute__((always_inline)) {
-    const int tap = P::PIPE ? v / 2 : 3 * r + v / KC;
-    const int ch = P::PIPE ? 32 * r + 16 * (v % 2) : 16 * (v % KC);
-    const int off = P::PIPE ? ((tap / 3) * kPitch + tap % 3) * T::RECB + (v % 2) * 32
-                            : (v / KC) * T::RECB + ch * 2;
+    const int tap = v / 2;
+    const int off = P::PIPE ? ((tap / 3) * kPitch + tap % 3) * T::RECB + (v % 2) * 32 : (v / KC) * T::RECB + (v % KC) * 32;
     const int base = P::PIPE ? r * 64 : r * kPitch * T::RECB;
-    return *reinterpret_cast<const v4i *>(smem + rec + base + off + pl * 192);
+    return *reinterpret_cast<const v4i *>(smem + corner + base + off + pl * 192);
   };
   v4i a[3][NPL];
 #pragma unroll
   for (int v = 0; v < 2; ++v)
 #pragma unroll
     for (int i = 0; i < NPL; ++i) a[v][i] = frag(0, v, i);
-#pragma unroll 1
-  for (int r = 0; r < KS / U; ++r) {
+  auto round = [&](int r) __attribute__((always_inline)) {
+    // (the low-order pass comes in front of the last phase, as in pipe_layer)
+    if constexpr (LO) {
+      if (r == NTP - 1) team_lo_pass<P, L, TT>(smem, packed, lane, rec, t0, acc);
+    }
     static_for<0, U>([&](auto vc) __attribute__((always_inline)) {
       constexpr int v = decltype(vc)::value;
       // activations two k-steps ahead (behind the last one: the last round again, unused)
@@ -107,60 +180,134 @@ __device__ __forceinline__ void team_conv(const unsigned char *smem, const WFrag
 #pragma unroll
           for (int m = 0; m < 6; ++m) mma<P>(ring[v % D][t][WP[m]], a[v % 3][AP[m]], acc[t]);
         } else {
-          mma<P>(ring[v % D][t][0], a[v % 3][0], acc[t]);
+#pragma unroll
+          for (int i = 0; i < W; ++i) mma<P>(ring[v % D][t][i], a[v % 3][0], acc[t]);
         }
-        // (behind the last k-steps this reads what follows in the buffer: unused)
-        const int kn = r * U + v + D;
-        const int f = team_frag<P, L>(kn < KS ? kn : KS - 1, t0 + t);
+        const int kn = r * U + v + D;   // (behind the last k-steps: the last one again, unused)
+        const int f = team_frag<P, L>(kn < KS ? kn : KS - 1, t0 + t < NT ? t0 + t : NT - 1);
 #pragma unroll
         for (int i = 0; i < W; ++i) ring[v % D][t][i] = wl[f + i];
       }
       __builtin_amdgcn_sched_barrier(0);
     });
+  };
+  if constexpr (P::PIPE) {
+    // (a k-step is one or two MFMAs: the waits of a loop's back edge would show)
+    static_for<0, KS / U>([&](auto rc) __attribute__((always_inline)) { round(decltype(rc)::value); });
+  } else {
+#pragma unroll 1
+    for (int r = 0; r < KS / U; ++r) round(r);
   }
 }
 
-// TEAM = 9: workgroup = (third of the squares, cout tile); TEAM = 3: all cout tiles
+// SiLU of one accumulator tile into the record at `rec` (cout tile t): planes, and the fp6 block.
+// UNDER: the one-workgroup kernel takes this tile's low-order parts behind MFMAs (see epi_atom).
+template <class P, bool LO, bool UNDER>
+__device__ __forceinline__ void team_store(unsigned char *smem, int rec, int h, int t, const f32x16 &acc) {
+  using T = TeamGeo<P>;
+  unsigned char *at = smem + rec + 64 * t + 8 * h;
+  if constexpr (T::SPLIT) {
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      float v[4];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) v[e] = split_silu(acc[4 * q + e]);
+#pragma unroll
+      for (int i = 0; i < 3; ++i) {
+        const int a = i < 2 ? split_take(v[0], v[1]) : pack2<PrecBF16>(v[0], v[1]);
+        const int b = i < 2 ? split_take(v[2], v[3]) : pack2<PrecBF16>(v[2], v[3]);
+        *reinterpret_cast<v2i *>(at + i * 192 + 16 * q) = v2i{a, b};
+      }
+    }
+  } else {
+    const DropConsts k = drop_consts<P>();
+    float lo[16], m = 0.0f;
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      int hi[2];
+#pragma unroll
+      for (int p = 0; p < 2; ++p) {
+        const int i = 4 * q + 2 * p;
+        const float v0 = acc[i] * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(acc[i]));
+        const float v1 = acc[i + 1] * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(acc[i + 1]));
+        hi[p] = pack2<P>(v0, v1);
+        if constexpr (LO) {
+          if constexpr (UNDER) {
+            lo[i] = v0 - __builtin_bit_cast(float, hi[p] << 16);
+            lo[i + 1] = v1 - __builtin_bit_cast(float, hi[p] & (int)0xffff0000);
+          } else {
+            lo[i] = dropped_lo(v0, hi[p], k);
+            lo[i + 1] = dropped_hi(v1, hi[p], k);
+          }
+          m = __builtin_amdgcn_fmed3f(__builtin_fabsf(lo[i]), m, __builtin_inff());
+          m = __builtin_amdgcn_fmed3f(__builtin_fabsf(lo[i + 1]), m, __builtin_inff());
+        }
+      }
+      *reinterpret_cast<v2i *>(at + 16 * q) = v2i{hi[0], hi[1]};
+    }
+    if constexpr (LO) {
+      const unsigned mb = __builtin_bit_cast(unsigned, m);
+      const auto x = __builtin_amdgcn_permlane32_swap(mb, mb, false, false);
+      const unsigned x0 = x[0], x1 = x[1];
+      int sc = (int)((x0 > x1 ? x0 : x1) >> 23) - 2;
+      sc = sc < 1 ? 1 : sc;
+      f32x16v even, odd;
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        even[i] = lo[i];
+        odd[i] = lo[8 + i];
+        even[8 + i] = odd[8 + i] = 0.0f;   // (only slots 0-15 are kept)
+      }
+      const u32x6 r = to_fp6_block(even, odd, __builtin_bit_cast(float, sc << 23));
+      int *d32 = reinterpret_cast<int *>(smem + rec + T::LO_OFF + 32 * t + 12 * h);
+      d32[0] = (int)r[0];
+      d32[1] = (int)r[1];
+      d32[2] = (int)r[2];
+      *reinterpret_cast<int *>(smem + rec + T::LO_OFF + 32 * t + 24 + 4 * h) = sc;
+    }
+  }
+}
+
+// Board `b` by the team that this workgroup (its member my_role) belongs to; `slot`: the team's share of
+// the exchange memory and of the flags.
 template <class P, int TEAM>
-__global__ __launch_bounds__(256) void team_forward_kernel(const TeamParams prm) {
+__device__ __forceinline__ void team_board(const TeamParams &prm, unsigned char *smem, unsigned b, unsigned slot,
+                                           int my_role) {
   using G = Geo<P>;
   using T = TeamGeo<P>;
-  constexpr int NPL = T::NPL, W = G::W, THREADS = 256;
-  extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, h = lane >> 5;
+  using S = TeamShape<TEAM>;
+  constexpr int NPL = T::NPL, W = G::W, THREADS = 256, PXT = S::PXT, CG = S::CG;
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), h = lane >> 5;
   const FwdParams &f = prm.f;
-  const unsigned b = blockIdx.x / TEAM;
-  const int my_role = (int)(blockIdx.x % TEAM);
   unsigned char *occ = smem + T::OCC_OFF;
   float *lgt = reinterpret_cast<float *>(smem + T::LGT_OFF);
   float *red = reinterpret_cast<float *>(smem + T::RED_OFF);
-  int *word = reinterpret_cast<int *>(red) + 40;   // what wave 0 found, for the others
+  int *word = reinterpret_cast<int *>(red) + 255;   // what wave 0 found, for the others
   const unsigned char *packed = f.packed + (size_t)(b / (unsigned)f.boards_per_group) * f.packed_stride;
   const float *tail = reinterpret_cast<const float *>(packed + G::TAIL_OFF);
-  unsigned char *act = prm.act + (size_t)b * T::BOARDB;
-  unsigned *flags = prm.flags + (size_t)b * kTeamFlags;
+  unsigned char *act = prm.act + (size_t)slot * T::BOARDB;
+  unsigned *flags = prm.flags + (size_t)slot * kTeamFlags;
   const __amdgpu_buffer_rsrc_t mem = __builtin_amdgcn_make_buffer_rsrc(act, 0, T::BOARDB, 0x00020000);
-
   [[maybe_unused]] const bool trace_on = true;
-  C6_MARK(0);
-  // does workgroup `role` have a part in stage l?
-  auto has_part = [](int l, int role) {
-    if (l == 8) return role == 0;
-    return TEAM == 3 || role % 3 < kCoutArr[l] / 32;
-  };
+
+  // the wave's tile of squares within the workgroup's, and its group of cout tiles
+  const int wpx = PXT == 4 ? wave : (PXT == 2 ? wave & 1 : 0);
+  const int cg = PXT == 4 ? 0 : (PXT == 2 ? wave >> 1 : wave);
+
+  // word l * 12 + role: the squares of stage l that the neighbours read are there; kTeamAll further on:
+  // all of them
   auto flag_set = [&](int l, int role) {
-    return __hip_atomic_load(&flags[l * 9 + role], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == prm.tag;
+    return __hip_atomic_load(&flags[l * 12 + role], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == prm.tag;
   };
-  // Are the inputs of stage l there for `role`?  Bounded; the answer is the same in every thread.
-  // 1: yes, 0: no, 2: no need, the stage itself has been done.
-  auto wait_inputs = [&](int l, int role) {
+  auto has_part = [](int l, int role) { return l < 8 || role == 0; };
+  int unfinished = -1;   // word of the piece whose inner squares are still being stored
+  // Are the inputs of stage l there for `role` (`own`: its own squares are in LDS)?  Bounded; the answer
+  // is the same in every thread.  1: yes, 0: no, 2: no need, the stage itself has been done.
+  auto wait_inputs = [&](int l, int role, bool own) {
     if (wave == 0) {
-      const int s = TEAM == 9 ? role / 3 : role;
-      int need = -1;   // lane < 9: the role of stage l - 1 it watches
-      if (l > 0 && lane < TEAM) {
-        const int ls = TEAM == 9 ? lane / 3 : lane;
-        if (has_part(l - 1, lane) && (l == 8 || (ls >= s - 1 && ls <= s + 1))) need = lane;
-      }
+      int need = -1;   // the word of stage l - 1 that this lane watches (less the stage's first)
+      if (lane < TEAM && (l == 8 || lane == role - 1 || lane == role + 1)) need = lane;
+      if (lane == 62 && !own) need = kTeamAll + role;
       int got = 0;
       for (int k = 0; k < prm.polls && got == 0; ++k) {
         const bool ok = need < 0 || flag_set(l - 1, need);
@@ -170,169 +317,269 @@ __global__ __launch_bounds__(256) void team_forward_kernel(const TeamParams prm)
       }
       if (lane == 0) *word = got;
     }
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // (the inner squares' stores)
     __syncthreads();
     const int got = *word;
+    if (tid == 0 && unfinished >= 0)
+      __hip_atomic_store(&flags[kTeamAll + unfinished], prm.tag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    unfinished = -1;
     __syncthreads();
     return got;
   };
   auto raise_flag = [&](int l, int role) {
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // this wave's stores have arrived
     __syncthreads();
-    if (tid == 0) __hip_atomic_store(&flags[l * 9 + role], prm.tag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-  };
-  // a layer's outputs: SiLU, planes, 64 * NPL consecutive bytes per square
-  auto store_tile = [&](const f32x16 &acc, int layer_off, int t, int pix, bool ok) __attribute__((always_inline)) {
-    const int at = layer_off + t * T::BLOCKB + pix * T::PXB;
-    int pl[4][NPL][2];   // [quad][plane][pair]
-#pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      float v[4];
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        if constexpr (NPL == 3) v[e] = split_silu(acc[4 * q + e]);
-        else v[e] = silu<P>(acc[4 * q + e]);
-      }
-#pragma unroll
-      for (int i = 0; i < NPL; ++i) {
-        pl[q][i][0] = i + 1 < NPL ? split_take(v[0], v[1]) : pack2<P>(v[0], v[1]);
-        pl[q][i][1] = i + 1 < NPL ? split_take(v[2], v[3]) : pack2<P>(v[2], v[3]);
-      }
-    }
-    // lane halves hold alternating groups of four channels: swap so that each lane has eight in a row
-#pragma unroll
-    for (int qq = 0; qq < 2; ++qq)
-#pragma unroll
-      for (int i = 0; i < NPL; ++i) {
-        v4i o;
-#pragma unroll
-        for (int d = 0; d < 2; ++d) {
-          // lower lane: quad 2 qq of both halves, upper lane: quad 2 qq + 1 of both
-          const auto x = __builtin_amdgcn_permlane32_swap((unsigned)pl[2 * qq][i][d], (unsigned)pl[2 * qq + 1][i][d], false, false);
-          const unsigned x0 = x[0], x1 = x[1];
-          o[d] = (int)x0;
-          o[2 + d] = (int)x1;
-        }
-        if (ok) __builtin_amdgcn_raw_buffer_store_b128(o, mem, at + i * 64 + (2 * qq + h) * 16, 0, kSc1);
-      }
+    if (tid == 0) __hip_atomic_store(&flags[l * 12 + role], prm.tag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   };
 
-  // what the LDS region holds: the rows of third region_s, padding zero
-  int region_s = -1;
+  // The LDS region: positions of the board rows around a role's squares, from the row above the first.
+  // region_role's own squares hold the outputs of layer region_layer (0-based), or nothing (-1).
+  int region_role = -1, region_layer = -1;
+  struct Span {
+    int p0, p1, base;   // first and last square, first position
+  };
+  auto span_of = [](int role) __attribute__((always_inline)) {
+    const int p0 = role * PXT * 32, p1 = p0 + PXT * 32 - 1;
+    return Span{p0, p1 < kPix ? p1 : kPix - 1, p0 / kBoard * kPitch};
+  };
+  auto record = [](int p, int base) __attribute__((always_inline)) {
+    const int r = p / kBoard;
+    return ((r + 1) * kPitch + (p - r * kBoard + 1) - base) * T::RECB;
+  };
+  auto clear_region = [&](const Span &sp) __attribute__((always_inline)) {   // (its padding stays clear from then on)
+    const v4i z = {0, 0, 0, 0};
+    const int bytes = ((sp.p1 / kBoard - sp.p0 / kBoard + 3) * kPitch + 1) * T::RECB;
+    for (int i = tid; i < bytes / 16; i += THREADS) reinterpret_cast<v4i *>(smem)[i] = z;
+    __syncthreads();
+  };
+  // 16-byte unit u of a square's record in a layer of C channels
+  auto unit_at = [](auto cc, int u) __attribute__((always_inline)) {
+    constexpr int C = decltype(cc)::value;
+    if (u < NPL * C / 8) return u / (C / 8) * 192 + u % (C / 8) * 16;
+    return T::LO_OFF + (u - NPL * C / 8) * 16;
+  };
+
+  // Outputs of layer L (own squares): into the records, and to memory what the neighbours read.
+  auto write_out = [&](auto lc, int role, const Span &sp, bool active, const auto &acc, int t0) __attribute__((always_inline)) {
+    constexpr int L = decltype(lc)::value, C = kCoutArr[L], NT = C / 32, UN = T::units(C);
+    constexpr int TT = S::tiles(NT);
+    constexpr bool LO = P::LO6 && ((P::LO_MASK >> (L + 1)) & 1);
+    const int p = sp.p0 + wpx * 32 + (lane & 31), pc = p < kPix ? p : kPix - 1;
+    const int rec = record(pc, sp.base);
+    if (active) {
+#pragma unroll
+      for (int t = 0; t < TT; ++t)
+        if (t0 + t < NT) team_store<P, LO, (L >= 2)>(smem, rec, h, t0 + t, acc[t]);
+    }
+    __syncthreads();
+    auto to_memory = [&](int q, int u) __attribute__((always_inline)) {
+      const v4i v = *reinterpret_cast<const v4i *>(smem + record(q, sp.base) + unit_at(IC<C>{}, u));
+      __builtin_amdgcn_raw_buffer_store_b128(v, mem, T::act_off(L) + (q * UN + u) * 16, 0, kSc1);
+    };
+    // twenty squares at either end (all of them where there are no more), then the rest
+    const int n = sp.p1 - sp.p0 + 1, m = n < 40 ? n : 40;
+    for (int i = tid; i < m * UN; i += THREADS) {
+      const int k = i / UN;
+      to_memory(sp.p0 + (k < 20 || n < 40 ? k : n - 40 + k), i - k * UN);
+    }
+    raise_flag(L, role);
+    for (int i = tid; i < (n - m) * UN; i += THREADS) {
+      const int k = i / UN;
+      to_memory(sp.p0 + 20 + k, i - k * UN);
+    }
+    unfinished = L * 12 + role;
+    region_role = role;
+    region_layer = L;
+  };
 
   auto conv_stage = [&](auto lc, int role) __attribute__((always_inline)) -> bool {
     constexpr int L = decltype(lc)::value;
-    constexpr int NT = kCoutArr[L] / 32, NTP = kCinArr[L] / 32, TT = TEAM == 9 ? 1 : NT;
-    constexpr int D = (W == 3 ? 6 : 18) / TT;
-    const int s = TEAM == 9 ? role / 3 : role, t0 = TEAM == 9 ? role % 3 : 0;
+    constexpr int NT = kCoutArr[L] / 32, TT = S::tiles(NT), D = team_ring<P, TT>();
+    constexpr int C = kCinArr[L], UN = T::units(C);
+    // (opaque per stage: what follows from it is formed here and not, for all stages, in front of the
+    // loop over them, in several hundred scalar registers that get spilled)
+    int t0 = cg * TT;
+    asm volatile("" : "+s"(t0));
+    const bool active = cg < CG && t0 < NT;
+    const Span sp = span_of(role);
     const WFrags wl = layer_weights<P, L>(packed, lane);
     C6_MARK(6 * L);
-    const int got = wait_inputs(L, role);
+    const bool own = region_role == role && region_layer == L - 1;
+    const int got = wait_inputs(L, role, own);
     if (got != 1) return got == 2;
     C6_MARK(6 * L + 1);
-    // ---- rows r0 - 1 .. r1 + 1 into LDS ----
-    const int p0 = 128 * s, p1 = p0 + 127 < kPix - 1 ? p0 + 127 : kPix - 1;
-    const int r0 = p0 / kBoard, r1 = p1 / kBoard;
-    const int base = r0 * kPitch;                       // first position: the row above r0
-    if (region_s != s) {
-      const v4i z = {0, 0, 0, 0};
-      for (int i = tid; i < T::REGION / 16; i += THREADS) reinterpret_cast<v4i *>(smem)[i] = z;
-      __syncthreads();
-      region_s = s;
-    }
-    const int ra = r0 > 0 ? r0 - 1 : 0, rb = r1 < kBoard - 1 ? r1 + 1 : kBoard - 1;
-    const int first = ra * kBoard, count = (rb - ra + 1) * kBoard;   // squares
-    constexpr int UP = 4 * NPL;                                      // 16-byte units per square and tile
-    constexpr int ROUNDS = (10 * kBoard * UP + THREADS - 1) / THREADS;
-    v4i in[NTP][ROUNDS];
-#pragma unroll
-    for (int t = 0; t < NTP; ++t)
+    // ---- the neighbours' squares (and, after helping out elsewhere, the own ones) into LDS ----
+    if (region_role != role) clear_region(sp);
+    const int q0 = sp.p0 - 20 > 0 ? sp.p0 - 20 : 0, q1 = sp.p1 + 20 < kPix ? sp.p1 + 20 : kPix - 1;
+    auto load_squares = [&](int from, int count) __attribute__((always_inline)) {   // at most 20
+      constexpr int ROUNDS = (20 * UN + THREADS - 1) / THREADS;
+      v4i in[ROUNDS];
 #pragma unroll
       for (int k = 0; k < ROUNDS; ++k) {
-        const int u = tid + k * THREADS;
-        if (u < count * UP)
-          in[t][k] = __builtin_amdgcn_raw_buffer_load_b128(mem, T::act_off(L - 1) + t * T::BLOCKB + first * T::PXB + u * 16, 0, kSc1);
+        const int i = tid + k * THREADS;
+        if (i < count * UN) in[k] = __builtin_amdgcn_raw_buffer_load_b128(mem, T::act_off(L - 1) + (from * UN + i) * 16, 0, kSc1);
       }
+#pragma unroll
+      for (int k = 0; k < ROUNDS; ++k) {
+        const int i = tid + k * THREADS, s = i / UN;
+        if (i < count * UN)
+          *reinterpret_cast<v4i *>(smem + record(from + s, sp.base) + unit_at(IC<C>{}, i - s * UN)) = in[k];
+      }
+    };
+    constexpr int ROUNDS = (20 * UN + THREADS - 1) / THREADS;
+    v4i left[ROUNDS], right[ROUNDS];
+    const int nl = sp.p0 - q0, nr = q1 - sp.p1;
+#pragma unroll
+    for (int k = 0; k < ROUNDS; ++k) {
+      const int i = tid + k * THREADS;
+      if (i < nl * UN) left[k] = __builtin_amdgcn_raw_buffer_load_b128(mem, T::act_off(L - 1) + (q0 * UN + i) * 16, 0, kSc1);
+      if (i < nr * UN) right[k] = __builtin_amdgcn_raw_buffer_load_b128(mem, T::act_off(L - 1) + ((sp.p1 + 1) * UN + i) * 16, 0, kSc1);
+    }
     // the first weights, behind the activations in the queue: back by the time those are in LDS
     v4i ring[D][TT][W];
     f32x16 acc[TT];
+    if (active) {
 #pragma unroll
-    for (int d = 0; d < D; ++d)
+      for (int d = 0; d < D; ++d)
 #pragma unroll
-      for (int t = 0; t < TT; ++t)
+        for (int t = 0; t < TT; ++t)
 #pragma unroll
-        for (int i = 0; i < W; ++i) ring[d][t][i] = wl[team_frag<P, L>(d, t0 + t) + i];
-    load_bias_tiles(acc, tail + bias_offset(L) + 32 * t0, h);
+          for (int i = 0; i < W; ++i) ring[d][t][i] = wl[team_frag<P, L>(d, t0 + t < NT ? t0 + t : NT - 1) + i];
+#pragma unroll
+      for (int t = 0; t < TT; ++t) {
+        f32x16 one[1];
+        load_bias_tiles(one, tail + bias_offset(L) + 32 * (t0 + t < NT ? t0 + t : NT - 1), h);
+        acc[t] = one[0];
+      }
+    }
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-    for (int t = 0; t < NTP; ++t)
-#pragma unroll
-      for (int k = 0; k < ROUNDS; ++k) {
-        const int u = tid + k * THREADS;
-        if (u < count * UP) {
-          const int px = first + u / UP, rest = u % UP, r = px / kBoard;
-          const int pos = (r + 1) * kPitch + (px - r * kBoard + 1) - base;
-          *reinterpret_cast<v4i *>(smem + pos * T::RECB + (rest / 4) * 192 + t * 64 + (rest % 4) * 16) = in[t][k];
-        }
-      }
+    for (int k = 0; k < ROUNDS; ++k) {
+      const int i = tid + k * THREADS, s = i / UN;
+      if (i < nl * UN) *reinterpret_cast<v4i *>(smem + record(q0 + s, sp.base) + unit_at(IC<C>{}, i - s * UN)) = left[k];
+      if (i < nr * UN) *reinterpret_cast<v4i *>(smem + record(sp.p1 + 1 + s, sp.base) + unit_at(IC<C>{}, i - s * UN)) = right[k];
+    }
+    if (!own)
+      for (int q = sp.p0; q <= sp.p1; q += 20) load_squares(q, sp.p1 - q + 1 < 20 ? sp.p1 - q + 1 : 20);
+    region_role = -1;   // (until the outputs are in place)
     __syncthreads();
     C6_MARK(6 * L + 2);
     // ---- contraction ----
-    const int p = (4 * s + wave) * 32 + (lane & 31);
+    const int p = sp.p0 + wpx * 32 + (lane & 31);
     const bool ok = p < kPix;
-    const int pc = ok ? p : kPix - 1, r = pc / kBoard;
-    const int rec = (r * kPitch + (pc - r * kBoard) - base) * T::RECB + 16 * h;
-    team_conv<P, L, TT>(smem, wl, ring, rec, t0, acc);
+    const int rec = record(ok ? p : kPix - 1, sp.base);
+    if (active) team_conv<P, L, TT>(smem, packed, wl, ring, lane, rec, t0, acc);
     C6_MARK(6 * L + 3);
     if constexpr (L < 7) {
-#pragma unroll
-      for (int t = 0; t < TT; ++t) store_tile(acc[t], T::act_off(L), t0 + t, pc, ok);
+      __syncthreads();   // everybody has read this layer's input
+      write_out(lc, role, sp, active, acc, t0);
     } else {
-      // heads: this wave's share of the policy (per square and cout tile) and of the value
-      const float *pw = tail + kBiasTotal + 32 * t0 + 4 * h;
+      // heads: this wave's share of the policy (per square) and of the value
+      const float *pw = tail + kBiasTotal + 4 * h;
+      const int tile = role * PXT + wpx;   // of the twelve
+      if constexpr (T::SPLIT) {
+        if (active) {
 #pragma unroll
-      for (int t = 0; t < TT; ++t) {
-        float pol = 0.0f, val = 0.0f;
+          for (int t = 0; t < TT; ++t) {
+            if (t0 + t >= NT) continue;
+            float pol = 0.0f, val = 0.0f;
 #pragma unroll
-        for (int q = 0; q < 4; ++q)
+            for (int q = 0; q < 4; ++q)
 #pragma unroll
-          for (int e = 0; e < 4; ++e) {
-            const float a = split_silu(acc[t][4 * q + e]);
-            pol = fmaf(a, pw[32 * t + 8 * q + e], pol);
-            val = fmaf(a, pw[kHeadC + 32 * t + 8 * q + e], val);
+              for (int e = 0; e < 4; ++e) {
+                const float a = split_silu(acc[t][4 * q + e]);
+                pol = fmaf(a, pw[32 * (t0 + t) + 8 * q + e], pol);
+                val = fmaf(a, pw[kHeadC + 32 * (t0 + t) + 8 * q + e], val);
+              }
+            const unsigned bits = __builtin_bit_cast(unsigned, pol);
+            const auto x = __builtin_amdgcn_permlane32_swap(bits, bits, false, false);
+            const unsigned x0 = x[0], x1 = x[1];
+            const float tot = __builtin_bit_cast(float, x0) + __builtin_bit_cast(float, x1);
+            const float vs = wave_sum(ok ? val : 0.0f);
+            if (h == 0 && ok)
+              __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(int, tot), mem, T::HEAD_OFF + ((t0 + t) * 384 + p) * 4, 0, kSc1);
+            if (lane == 0)
+              __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(int, vs), mem, T::VAL_OFF + ((t0 + t) * 12 + tile) * 4, 0, kSc1);
           }
-        const unsigned bits = __builtin_bit_cast(unsigned, pol);
-        const auto x = __builtin_amdgcn_permlane32_swap(bits, bits, false, false);
-        const unsigned x0 = x[0], x1 = x[1];
-        const float tot = __builtin_bit_cast(float, x0) + __builtin_bit_cast(float, x1);
-        const float vs = wave_sum(ok ? val : 0.0f);
-        if (h == 0 && ok)
-          __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(int, tot), mem, T::HEAD_OFF + ((t0 + t) * 384 + pc) * 4, 0, kSc1);
-        if (lane == 0)
-          __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(int, vs), mem, T::VAL_OFF + ((t0 + t) * 12 + 4 * s + wave) * 4, 0, kSc1);
+        }
+      } else {
+        // The one-workgroup kernel runs one chain of multiply-adds over the channels of a lane's
+        // square, cout tile after cout tile: the groups of cout tiles take turns and hand it on.
+        float *chain = reinterpret_cast<float *>(smem + T::OCC_OFF);   // (not in use before the last stage)
+        f32x4 pw4[TT][4];
+        if (active) {
+#pragma unroll
+          for (int t = 0; t < TT; ++t) {
+            if (t0 + t >= NT) continue;
+            float val0 = 0.0f;
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+              pw4[t][q] = *reinterpret_cast<const f32x4 *>(pw + 32 * (t0 + t) + 8 * q);
+              const f32x4 vw4 = *reinterpret_cast<const f32x4 *>(pw + kHeadC + 32 * (t0 + t) + 8 * q);
+              float vs = 0.0f;
+#pragma unroll
+              for (int e = 0; e < 4; ++e) {
+                const float a = silu<P>(acc[t][4 * q + e]);
+                acc[t][4 * q + e] = a;
+                val0 = fmaf(a, vw4[e], val0);
+                vs = fmaf(a, vw4[e], vs);
+              }
+              // (tile 0: one chain over its sixteen channels; the others: one sum per four)
+              if (t0 + t > 0)
+                __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(int, vs), mem,
+                                                      T::VAL_OFF + ((tile * 9 + 1 + 4 * (t0 + t - 1) + q) * 64 + lane) * 4, 0, kSc1);
+            }
+            if (t0 + t == 0)
+              __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(int, val0), mem, T::VAL_OFF + (tile * 9 * 64 + lane) * 4, 0, kSc1);
+          }
+        }
+        float pol = 0.0f;
+#pragma unroll
+        for (int turn = 0; turn < CG; ++turn) {
+          if (turn == cg && active) {
+            if (cg > 0) pol = chain[wpx * 64 + lane];
+#pragma unroll
+            for (int t = 0; t < TT; ++t) {
+              if (t0 + t >= NT) continue;
+#pragma unroll
+              for (int i = 0; i < 16; ++i) pol = fmaf(acc[t][i], pw4[t][i / 4][i % 4], pol);
+            }
+            chain[wpx * 64 + lane] = pol;
+            if (turn == CG - 1 || t0 + TT >= NT) {
+              const unsigned bits = __builtin_bit_cast(unsigned, pol);
+              const auto x = __builtin_amdgcn_permlane32_swap(bits, bits, false, false);
+              const unsigned x0 = x[0], x1 = x[1];
+              const float tot = __builtin_bit_cast(float, x0) + __builtin_bit_cast(float, x1);
+              if (h == 0 && ok)
+                __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(int, tot), mem, T::HEAD_OFF + p * 4, 0, kSc1);
+            }
+          }
+          if (turn + 1 < CG) __syncthreads();
+        }
       }
+      raise_flag(L, role);
     }
-    raise_flag(L, role);
     C6_MARK(6 * L + 4);
     return true;
   };
 
-  // first layer: every workgroup stages the whole board
+  // first layer: every workgroup stages the part of the board that its squares see
   auto first_stage = [&](int role) __attribute__((always_inline)) -> bool {
-    const int s = TEAM == 9 ? role / 3 : role;
-    int *flag = reinterpret_cast<int *>(red) + 32;   // [0]: third plane varies, [1]: an input is not exact in bf16
-    const int p = (4 * s + wave) * 32 + (lane & 31);
-    const bool ok = p < kPix;
-    const int pc = ok ? p : kPix - 1, r = pc / kBoard, c = pc - r * kBoard;
-    region_s = -1;
-    f32x16 a0;
-    {
-      // (the table holds the squares as the one-workgroup kernels' lanes do: wave, pixel tile)
-      const WFrags tb = packed_frags<P>(packed, lane, G::PLANE2_FRAG_OFF + __builtin_amdgcn_readfirstlane(4 * s + wave) * 4);
+    const Span sp = span_of(role);
+    int *flag = reinterpret_cast<int *>(red) + 64;   // [0]: third plane varies, [1]: an input is not exact in bf16
+    const int p = sp.p0 + wpx * 32 + (lane & 31);
+    const int pc = p < kPix ? p : kPix - 1, r = pc / kBoard, c = pc - r * kBoard;
+    const bool active = cg == 0;
+    region_role = -1;
+    f32x16 acc[1];
+    if (active) {
+      // (the table holds the squares as the one-workgroup kernels' lanes do: by tile of 32)
+      const WFrags tb = packed_frags<P>(packed, lane, G::PLANE2_FRAG_OFF + (role * PXT + wpx) * 4);
 #pragma unroll
       for (int q = 0; q < 4; ++q) {
         const f32x4 t4 = __builtin_bit_cast(f32x4, tb[q]);
 #pragma unroll
-        for (int e = 0; e < 4; ++e) a0[4 * q + e] = t4[e];
+        for (int e = 0; e < 4; ++e) acc[0][4 * q + e] = t4[e];
       }
     }
     float xin[2][3];
@@ -355,14 +602,20 @@ __global__ __launch_bounds__(256) void team_forward_kernel(const TeamParams prm)
         }
       }
     }
-    if (tid < 2) flag[tid] = 0;
-    if (tid == 0) red[34] = xin[0][2];
+    // halo rows that the squares' 23 kernel rows reach (and the zero row behind the last)
+    const int ha = sp.p0 / kBoard * 3, hb = (sp.p1 / kBoard + kK1) * 3 + 1;
     {
       const v4i z = {0, 0, 0, 0};
-      for (int i = tid * 16; i < G::COPIES_BYTES; i += THREADS * 16) *reinterpret_cast<v4i *>(smem + i) = z;
+      const int per = (hb - ha) * (kL1RowPitch * G::EB / 16);
+#pragma unroll
+      for (int s = 0; s < G::E; ++s)
+        for (int i = tid; i < per; i += THREADS)
+          *reinterpret_cast<v4i *>(smem + s * G::COPY_BYTES + ha * kL1RowPitch * G::EB + i * 16) = z;
     }
+    if (tid < 2) flag[tid] = 0;
+    if (tid == 0) red[66] = xin[0][2];
     __syncthreads();
-    const float c2 = red[34];
+    const float c2 = red[66];
     bool varies = false;
 #pragma unroll
     for (int k = 0; k < 2; ++k)
@@ -370,27 +623,30 @@ __global__ __launch_bounds__(256) void team_forward_kernel(const TeamParams prm)
     if (varies) flag[0] = 1;
     __syncthreads();
     const bool plane2_varies = flag[0] != 0;
-    bool inexact = false;
+    int parts = 1;
+    if constexpr (T::SPLIT) {
+      bool inexact = false;
 #pragma unroll
-    for (int k = 0; k < 2; ++k)
-      if (tid + k * THREADS < kPix)
+      for (int k = 0; k < 2; ++k)
+        if (tid + k * THREADS < kPix)
 #pragma unroll
-        for (int ch = 0; ch < 3; ++ch)
-          inexact |= (ch < 2 || plane2_varies) && (__builtin_bit_cast(int, xin[k][ch]) & 0xffff) != 0;
-    if (NPL == 3 && inexact) flag[1] = 1;
-    __syncthreads();
-    const int parts = NPL == 3 && flag[1] != 0 ? 3 : 1;
+          for (int ch = 0; ch < 3; ++ch)
+            inexact |= (ch < 2 || plane2_varies) && (__builtin_bit_cast(int, xin[k][ch]) & 0xffff) != 0;
+      if (inexact) flag[1] = 1;
+      __syncthreads();
+      parts = flag[1] != 0 ? 3 : 1;
+    }
     const int sh = c % G::E;
     const int l1 = sh * G::COPY_BYTES + (r * 3 * kL1RowPitch + (c - sh)) * G::EB;
-    const int steps = plane2_varies ? G::STEPS1 : G::FAST1_STEPS;
-    const int row0 = plane2_varies ? l1 + kL1RowsHalf * h * kL1RowPitch * G::EB : l1 + h * kL1RowPitch * G::EB;
+    const int rows = (plane2_varies ? G::STEPS1 : G::FAST1_STEPS) / 3;
+    const int row0 = l1 + (plane2_varies ? kL1RowsHalf : 1) * h * kL1RowPitch * G::EB;
     const int rowb = (plane2_varies ? 1 : 3) * kL1RowPitch * G::EB;
     const WFrags wl = plane2_varies ? layer_weights<P, 0>(packed, lane) : packed_frags<P>(packed, lane, G::FAST1_OFF);
-    {
+    if (active) {
       f32x16 b0[1];
       load_bias_tiles(b0, tail + bias_offset(0), h);
 #pragma unroll
-      for (int i = 0; i < 16; ++i) a0[i] = plane2_varies ? b0[0][i] : fmaf(c2, a0[i], b0[0][i]);
+      for (int i = 0; i < 16; ++i) acc[0][i] = plane2_varies ? b0[0][i] : fmaf(c2, acc[0][i], b0[0][i]);
     }
 #pragma unroll 1
     for (int part = 0; part < parts; ++part) {
@@ -398,68 +654,71 @@ __global__ __launch_bounds__(256) void team_forward_kernel(const TeamParams prm)
 #pragma unroll
       for (int k = 0; k < 2; ++k) {
         const int sq = tid + k * THREADS;
-        if (sq < kPix) {
-          const int row = sq / kBoard, col = sq - row * kBoard;
+        const int row = sq / kBoard, col = sq - row * kBoard;
 #pragma unroll
-          for (int ch = 0; ch < 3; ++ch) {
-            if (ch >= (plane2_varies ? 3 : 2)) break;
-            const unsigned short v16 = bits16<P>(xin[k][ch]);
-            if constexpr (NPL == 3) xin[k][ch] -= __builtin_bit_cast(float, (unsigned)v16 << 16);
-            const int hrow = (row + kK1 / 2) * 3 + ch;
+        for (int ch = 0; ch < 3; ++ch) {
+          if (ch >= (plane2_varies ? 3 : 2)) break;
+          const int hrow = (row + kK1 / 2) * 3 + ch;
+          if (sq >= kPix) continue;
+          const unsigned short v16 = bits16<P>(xin[k][ch]);
+          if constexpr (T::SPLIT) xin[k][ch] -= __builtin_bit_cast(float, (unsigned)v16 << 16);
+          if (hrow < ha || hrow >= hb) continue;
 #pragma unroll
-            for (int q = 0; q < G::E; ++q)
-              *reinterpret_cast<unsigned short *>(smem + q * G::COPY_BYTES + (hrow * kL1RowPitch + (col + kK1 / 2 - q)) * G::EB) = v16;
-          }
+          for (int q = 0; q < G::E; ++q)
+            *reinterpret_cast<unsigned short *>(smem + q * G::COPY_BYTES + (hrow * kL1RowPitch + (col + kK1 / 2 - q)) * G::EB) = v16;
         }
       }
       __syncthreads();
       C6_MARK(1);
-      // k-steps in rounds of one kernel row (three fragments); weights two rounds ahead
-      v4i w[3][3][W], a[3][3];
-      const int rows = steps / 3;
-      auto fetch = [&](int row, int slot) __attribute__((always_inline)) {
-        const int rr = row < rows ? row : rows - 1;
+      if (active) {
+        // k-steps in rounds of one kernel row (three fragments); operands three rounds ahead
+        v4i w[4][3][W], a[4][3];
+        auto fetch = [&](int row, int s4) __attribute__((always_inline)) {
+          const int rr = row < rows ? row : rows - 1;
 #pragma unroll
-        for (int i = 0; i < 3; ++i) {
+          for (int i = 0; i < 3; ++i) {
 #pragma unroll
-          for (int j = 0; j < W; ++j) w[slot][i][j] = wl[(rr * 3 + i) * W + j];
-          a[slot][i] = *reinterpret_cast<const v4i *>(smem + row0 + rr * rowb + i * 16);
-        }
-        __builtin_amdgcn_sched_barrier(0);
-      };
-      auto multiply = [&](int slot) __attribute__((always_inline)) {
+            for (int j = 0; j < W; ++j) w[s4][i][j] = wl[(rr * 3 + i) * W + j];
+            a[s4][i] = *reinterpret_cast<const v4i *>(smem + row0 + rr * rowb + i * 16);
+          }
+          __builtin_amdgcn_sched_barrier(0);
+        };
+        auto multiply = [&](int s4) __attribute__((always_inline)) {
 #pragma unroll
-        for (int i = 0; i < 3; ++i)
+          for (int i = 0; i < 3; ++i)
 #pragma unroll
-          for (int j = 0; j < W; ++j) mma<P>(w[slot][i][j], a[slot][i], a0);
-        __builtin_amdgcn_sched_barrier(0);
-      };
-      fetch(0, 0);
-      fetch(1, 1);
-      int row = 0;
+            for (int j = 0; j < W; ++j) mma<P>(w[s4][i][j], a[s4][i], acc[0]);
+          __builtin_amdgcn_sched_barrier(0);
+        };
+#pragma unroll
+        for (int s4 = 0; s4 < 3; ++s4) fetch(s4, s4);
+        int row = 0;
 #pragma unroll 1
-      for (; row + 3 <= rows; row += 3) {
-        fetch(row + 2, 2);
-        multiply(0);
-        fetch(row + 3, 0);
-        multiply(1);
-        fetch(row + 4, 1);
-        multiply(2);
+        for (; row + 4 <= rows; row += 4) {
+#pragma unroll
+          for (int s4 = 0; s4 < 4; ++s4) {
+            fetch(row + s4 + 3, (s4 + 3) % 4);
+            multiply(s4);
+          }
+        }
+#pragma unroll
+        for (int s4 = 0; s4 < 3; ++s4)
+          if (row + s4 < rows) multiply(s4);
       }
-      if (row < rows) multiply(0);
-      if (row + 1 < rows) multiply(1);
     }
     C6_MARK(2);
-    store_tile(a0, T::act_off(0), 0, pc, ok);
-    raise_flag(0, role);
+    __syncthreads();   // the copies give way to the activations
+    clear_region(sp);
+    write_out(IC<0>{}, role, sp, active, acc, 0);
     C6_MARK(3);
     return true;
   };
 
-  // the heads' partial sums into logits, value and draw (one workgroup of the team)
+  // the heads' sums into logits, value, draw and (cascade) the list of close boards: one workgroup
   auto last_stage = [&](int role) __attribute__((always_inline)) -> bool {
-    const int got = wait_inputs(8, role);
+    const int got = wait_inputs(8, role, true);
     if (got != 1) return got == 2;
+    region_role = -1;
     const float *valw = tail + kBiasTotal + kHeadC;
     const float polb = valw[kHeadC], valb = valw[kHeadC + 1];
     auto partial = [&](int at) __attribute__((always_inline)) {
@@ -469,35 +728,78 @@ __global__ __launch_bounds__(256) void team_forward_kernel(const TeamParams prm)
     long long src = state && f.index ? f.index[b] : (long long)b;
     if (state) src = src < 0 ? 0 : (src >= f.num_states ? f.num_states - 1 : src);
     for (int p = tid; p < kPix; p += THREADS) {
-      const float z = ((partial(T::HEAD_OFF + p * 4) + partial(T::HEAD_OFF + (384 + p) * 4)) +
-                       partial(T::HEAD_OFF + (768 + p) * 4)) + polb;
-      bool o = false;
+      float z = partial(T::HEAD_OFF + p * 4);
+      if constexpr (T::SPLIT) z = (z + partial(T::HEAD_OFF + (384 + p) * 4)) + partial(T::HEAD_OFF + (768 + p) * 4);
+      z += polb;
+      bool taken;
       if (f.mask_mode == C6_MASK_LEGAL) {
-        o = f.legal[(size_t)b * kPix + p] == 0;
-      } else if (f.mask_mode == C6_MASK_INPUT) {
-        if (state) {
-          const int stone = reinterpret_cast<const int8_t *>(f.x)[(size_t)src * kPix + (f.view ? d4_from_view(p, f.view) : p)];
-          const int me = f.player[src];
-          o = stone == me || stone == -me;
-        } else {
-          o = load_x(f.x, f.x_dtype, (size_t)b * 3 * kPix + p) != 0.0f || load_x(f.x, f.x_dtype, ((size_t)b * 3 + 1) * kPix + p) != 0.0f;
-        }
+        taken = f.legal[(size_t)b * kPix + p] == 0;
+      } else if (state) {
+        const int stone = reinterpret_cast<const int8_t *>(f.x)[(size_t)src * kPix + (f.view ? d4_from_view(p, f.view) : p)];
+        const int me = f.player[src];
+        taken = stone == me || stone == -me;
+      } else {
+        taken = load_x(f.x, f.x_dtype, (size_t)b * 3 * kPix + p) != 0.0f || load_x(f.x, f.x_dtype, ((size_t)b * 3 + 1) * kPix + p) != 0.0f;
       }
+      const bool masked = taken && f.mask_mode != C6_MASK_NONE;
       lgt[p] = z;
-      occ[p] = o;
-      if (f.logits != nullptr) static_cast<float *>(f.logits)[(size_t)b * kPix + p] = o ? f.fill : z;
+      occ[p] = (unsigned char)((masked ? 1 : 0) | (taken ? 2 : 0));
+      if (f.logits != nullptr) {
+        const float v = masked ? f.fill : z;
+        const size_t at = (size_t)b * kPix + p;
+        if (f.logits_dtype == C6_DT_F32) static_cast<float *>(f.logits)[at] = v;
+        else if (f.logits_dtype == C6_DT_BF16) static_cast<unsigned short *>(f.logits)[at] = __builtin_bit_cast(unsigned short, (__bf16)v);
+        else static_cast<unsigned short *>(f.logits)[at] = __builtin_bit_cast(unsigned short, (_Float16)v);
+      }
     }
-    if (tid < 36) red[tid] = partial(T::VAL_OFF + tid * 4);
+    if constexpr (T::SPLIT) {
+      if (tid < 36) red[tid] = partial(T::VAL_OFF + tid * 4);
+    } else {
+      // as lane `lane` of wave `wave` of the one-workgroup kernel adds its three squares' sums up
+      float part[3][9], vsum = 0.0f;
+      bool valid[3];
+#pragma unroll
+      for (int j = 0; j < 3; ++j) {
+        valid[j] = (3 * wave + j) * 32 + (lane & 31) < kPix;
+#pragma unroll
+        for (int i = 0; i < 9; ++i) part[j][i] = partial(T::VAL_OFF + (((3 * wave + j) * 9 + i) * 64 + lane) * 4);
+      }
+#pragma unroll
+      for (int i = 0; i < 9; ++i)
+#pragma unroll
+        for (int j = 0; j < 3; ++j) vsum += valid[j] ? part[j][i] : 0.0f;
+      vsum = wave_sum(vsum);
+      if (lane == 0) red[wave] = vsum;
+    }
     __syncthreads();
-    if (tid == 0 && f.value != nullptr) f.value[b] = tanhf(split_value_sum(red) * (1.0f / kPix) + valb);
+    if (tid == 0 && f.value != nullptr) {
+      float s = 0.0f;
+      if constexpr (T::SPLIT) {
+        s = split_value_sum(red);
+      } else {
+#pragma unroll
+        for (int w = 0; w < 4; ++w) s += red[w];
+      }
+      f.value[b] = tanhf(s * (1.0f / kPix) + valb);
+    }
     if (f.actions != nullptr && wave == 0) {
       int a;
       float lp;
       wave_sample(
-          lane, f.u[b], f.inv_temperature, [&](int i) { return lgt[i]; }, [&](int i) { return occ[i] == 0; }, a, lp);
+          lane, f.u[b], f.inv_temperature, [&](int i) { return lgt[i]; }, [&](int i) { return (occ[i] & 1) == 0; }, a, lp);
       if (lane == 0) {
         f.actions[b] = a;
         if (f.logprob != nullptr) f.logprob[b] = lp;
+      }
+    }
+    if constexpr (P::ID == C6_PREC_BF16) {
+      if (f.redo_mode == kRedoDetect && wave == 1) {   // (a run of one board: see fused_pipe_kernel)
+        const bool again = wave_margin_below(
+            lane, f.redo_threshold, [&](int i) { return lgt[i]; }, [&](int i) { return (occ[i] & 2) == 0; });
+        if (lane == 0) {
+          f.redo_counts[b] = again ? 1 : 0;
+          f.redo_list[b] = (int)b;
+        }
       }
     }
     raise_flag(8, role);
@@ -506,6 +808,7 @@ __global__ __launch_bounds__(256) void team_forward_kernel(const TeamParams prm)
   };
 
   // Stages in order; `help`: a wait ran out, do the earliest piece that has no flag instead.
+  C6_MARK(0);
   bool help = false;
   for (int l = 0; l < kTeamStages;) {
     if (!help && !has_part(l, my_role)) {
@@ -517,7 +820,7 @@ __global__ __launch_bounds__(256) void team_forward_kernel(const TeamParams prm)
       if (wave == 0) {
         int found = l * 16 + my_role;
         for (int k = l - 1; k >= 0; --k) {
-          const bool open = lane < TEAM && has_part(k, lane) && !flag_set(k, lane);
+          const bool open = lane < TEAM && !flag_set(k, lane);
           const unsigned long long m = __builtin_amdgcn_ballot_w64(open);
           if (m != 0) found = k * 16 + __builtin_ctzll(m);
         }
@@ -543,13 +846,72 @@ __global__ __launch_bounds__(256) void team_forward_kernel(const TeamParams prm)
     if (ok && stage == l && role == my_role) ++l;
     help = !ok;
   }
+  __syncthreads();
 }
 
-// How many workgroups share a board when there are `boards` of them: nine while that many fit the
-// chip at once, then three, then one (the one-workgroup kernels).
-inline int team_size(long long boards, int cus) { return boards * 9 <= cus ? 9 : (boards * 3 <= cus ? 3 : 1); }
+// How many workgroups share a board when there are `boards` of them: as many as fit the chip at once, where
+// that beats one workgroup (1: the one-workgroup kernels).  With fewer workgroups per board more waves read
+// the same weights, and the L1's 64 bytes a cycle bound the layers: measured, 20 / 40 / 80 boards against
+// one workgroup each, fp32 66 / 95 / 150 us against 205, bf16 + fp6 + low weights 55 / 78 / 102 against 89,
+// bf16 + fp6 51 / 65 / 79 against 63, plain bf16 44 us (20 boards) against 46.
+template <class P> __host__ __device__ inline int team_size(long long boards, int wgs) {
+  if (boards * 12 <= wgs) return 12;
+  if ((TeamGeo<P>::SPLIT || P::WLO) && boards * 6 <= wgs) return 6;
+  return TeamGeo<P>::SPLIT && boards * 3 <= wgs ? 3 : 1;
+}
+// ... and the most boards that are shared at all
+template <class P> inline long long team_most(int wgs) { return wgs / (TeamGeo<P>::SPLIT ? 3 : (P::WLO ? 6 : 12)); }
 
-// modes that have a team kernel
-template <class P> constexpr bool has_team() { return P::ID == C6_PREC_F32S; }
+template <class P> __global__ __launch_bounds__(256) void team_forward_kernel(const TeamParams prm) {
+  using T = TeamGeo<P>;
+  extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
+  unsigned items = (unsigned)prm.f.total_boards;
+  // cascade, second pass: the listed boards, as fused_pipe_kernel finds them
+  int *runs = reinterpret_cast<int *>(smem + T::RUNS_OFF);
+  const bool from_list = P::LO6 != 0 && prm.f.redo_mode == kRedoConsume;
+  if (from_list) {
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    int *part = reinterpret_cast<int *>(smem + T::RED_OFF);
+    int before = 0;
+    for (int r0 = 0; r0 < prm.f.redo_runs; r0 += 256) {
+      const int r = r0 + tid, c = r < prm.f.redo_runs ? prm.f.redo_counts[r] : 0;
+      const int incl = wave_inclusive_sum_i(c);
+      if (lane == 63) part[wave] = incl;
+      __syncthreads();
+      int lower = before;
+#pragma unroll
+      for (int w = 0; w < 4; ++w) {
+        lower += w < wave ? part[w] : 0;
+        before += part[w];
+      }
+      if (r < prm.f.redo_runs) runs[r] = lower + incl - c;
+      __syncthreads();
+    }
+    if (tid == 0 && blockIdx.x == 0) *prm.f.redo_count = before;
+    items = (unsigned)before;
+  }
+  if (items == 0) return;
+  const int team = team_size<P>(items, (int)gridDim.x);
+  if (team == 1) return;   // (more listed boards than teams: the launch behind this one takes them)
+  const unsigned slot = blockIdx.x / (unsigned)team;
+  const int role = (int)(blockIdx.x % (unsigned)team);
+  if (slot >= items) return;
+  unsigned b = slot;
+  if (from_list) {
+    int lo = 0, hi = prm.f.redo_runs;
+    while (hi - lo > 1) {
+      const int mid = (lo + hi) >> 1;
+      if ((unsigned)runs[mid] <= slot) lo = mid; else hi = mid;
+    }
+    b = (unsigned)prm.f.redo_list[(size_t)lo * prm.f.redo_per + (slot - (unsigned)runs[lo])];
+  }
+  if (team == 12) team_board<P, 12>(prm, smem, b, slot, role);
+  if constexpr (TeamGeo<P>::SPLIT || P::WLO) {
+    if (team == 6) team_board<P, 6>(prm, smem, b, slot, role);
+  }
+  if constexpr (TeamGeo<P>::SPLIT) {
+    if (team == 3) team_board<P, 3>(prm, smem, b, slot, role);
+  }
+}
 
 }  // namespace c6

@@ -184,13 +184,14 @@ int c6_forward_boards_cascade(const int8_t *boards, const int8_t *player,
  * buffers, or 0 and 0 where one workgroup per board is the better launch (many boards, or a mode
  * without such a kernel): call c6_forward there.
  *   workspace  device, 16-byte aligned; contents need no preparation
+ *   (the cascade's workspace, where there is one, comes in front of these)
  *   flags      device words through which the workgroups of this launch tell one another what is
  *              done: no word may hold `tag` when the launch starts, and no other launch may use them
  *              at the same time.  (Words zeroed once and a tag counted up from 1 by every launch on
  *              a stream; in a captured graph, words cleared inside the graph.)
- *   tag        not 0
+ *   tag        not 0; a cascade also uses tag + 1
  *   polls      how often a workgroup looks at a flag before it computes the piece itself; 0: 64
- * One launch, no synchronisation with the host.  Every wait in it is bounded: a workgroup that has
+ * No synchronisation with the host.  Every wait is bounded: a workgroup that has
  * waited too long computes what it waits for. */
 int c6_team_bytes(int prec, int64_t boards, size_t *workspace_bytes, size_t *flag_bytes);
 int c6_forward_team(const void *x, int x_dtype, int64_t groups, int64_t boards_per_group,
@@ -204,6 +205,22 @@ int c6_forward_boards_team(const int8_t *boards, const int8_t *player, const int
                            float fill, const float *u, float temperature, int64_t *actions,
                            float *logprob, void *workspace, size_t workspace_bytes, void *flags,
                            size_t flag_bytes, uint32_t tag, int polls, void *stream);
+int c6_forward_cascade_team(const void *x, int x_dtype, int64_t groups, int64_t boards_per_group,
+                            const void *packed, size_t packed_stride, int prec, void *logits,
+                            int logits_dtype, float *value, int mask_mode, const uint8_t *legal,
+                            float fill, const float *u, float temperature, int64_t *actions,
+                            float *logprob, float threshold, void *cascade_workspace,
+                            size_t cascade_bytes, void *workspace, size_t workspace_bytes,
+                            void *flags, size_t flag_bytes, uint32_t tag, int polls, void *stream);
+int c6_forward_boards_cascade_team(const int8_t *boards, const int8_t *player,
+                                   const int8_t *stones_left, int64_t num_states,
+                                   const int64_t *index, int view, int64_t batch, const void *packed,
+                                   int prec, void *logits, int logits_dtype, float *value,
+                                   int mask_mode, float fill, const float *u, float temperature,
+                                   int64_t *actions, float *logprob, float threshold,
+                                   void *cascade_workspace, size_t cascade_bytes, void *workspace,
+                                   size_t workspace_bytes, void *flags, size_t flag_bytes,
+                                   uint32_t tag, int polls, void *stream);
 /* 1 while `stream` is being captured into a graph, else 0 */
 int c6_stream_capturing(void *stream);
 

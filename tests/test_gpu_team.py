@@ -13,7 +13,7 @@ from connect6_amd.synthetic import gen_boards, gen_uniform
 from oracle import torch_ref as R
 
 pytestmark = pytest.mark.gpu
-MODES = [_lib.PREC_F32S]
+MODES = [_lib.PREC_F32S, _lib.PREC_BF16, _lib.PREC_F16, _lib.PREC_BF16F6, _lib.PREC_BF16F6W]
 
 
 def _model(cuda, seed=11):
@@ -52,7 +52,7 @@ def test_same_bits_as_one_workgroup_per_board(cuda, prec):
     with torch.inference_mode():
         kw = dict(mask_mode=_lib.MASK_LEGAL, u=u, temperature=0.8, want_logprob=True)
         want = run_forward(xd, packed, prec, 1, 300, legal=ld, **kw)
-        for n in (1, 2, 5, 27, 28, 29, 84, 85, 86):
+        for n in (1, 2, 5, 20, 21, 22, 41, 42, 43, 84, 85, 86):
             kw["u"] = u[:n]
             got = run_forward(xd[:n], packed, prec, 1, n, legal=ld[:n], **kw)
             for a, b in zip(got, want):
@@ -68,18 +68,39 @@ def test_same_bits_as_one_workgroup_per_board(cuda, prec):
         assert torch.equal(a[0][3:], run_forward(xd[3:6], sets[packed.numel():], prec, 1, 3)[0])
 
 
-@pytest.mark.parametrize("prec", MODES)
-@pytest.mark.parametrize("boards", [1, 7, 40])
+# (boards up to what the mode shares at all: 21 between twelve workgroups, 42 between six, 85 between three)
+@pytest.mark.parametrize("prec,boards", [(p, b) for p in MODES for b in (1, 7, 30, 60)
+                                         if b <= {_lib.PREC_F32S: 85, _lib.PREC_BF16F6W: 42}.get(p, 21)])
 def test_a_workgroup_that_waited_long_enough_does_the_work_itself(cuda, prec, boards):
     model, (x, _) = _model(cuda), _inputs(boards)
     xd = x.to(cuda)
     packed = model.packed_weights(prec)
-    flags = torch.zeros(boards * 96, dtype=torch.int32, device=cuda)
+    flags = torch.zeros(boards * 256, dtype=torch.int32, device=cuda)
     with torch.inference_mode():
         want = run_forward(torch.cat([xd] * (300 // boards + 1)), packed, prec, 1, boards * (300 // boards + 1))
         for tag, polls in ((1, 0), (2, 1), (3, 2), (4, 5)):
             lg, vg = _team(prec, xd, packed, tag, flags, polls)
             assert torch.equal(lg, want[0][:boards]) and torch.equal(vg, want[1][:boards]), polls
+
+
+@pytest.mark.parametrize("prec", [_lib.PREC_BF16C, _lib.PREC_BF16C6])
+def test_cascade_with_few_listed_boards(cuda, prec):
+    model, (x, legal) = _model(cuda), gen_boards(1100, 200, 31)
+    xd, ld, u = x.to(cuda), legal.to(cuda), gen_uniform(1100, 5).to(cuda)
+    packed = model.packed_weights(prec)
+    with torch.inference_mode():
+        # the margin that about every tenth board is under: the listed ones are few enough for teams
+        # of every size, or too many, depending on the batch
+        for threshold in (0.0, 0.004, 0.3, -1.0):
+            kw = dict(mask_mode=_lib.MASK_LEGAL, temperature=0.8, want_logprob=True, threshold=threshold)
+            stats = {}
+            want = run_forward(xd, packed, prec, 1, 1100, legal=ld, u=u, stats=stats, **kw)
+            for n in (1, 7, 21, 22, 42, 43, 85, 86, 300, 1024):
+                got = run_forward(xd[:n], packed, prec, 1, n, legal=ld[:n], u=u[:n], stats=stats, **kw)
+                for a, b in zip(got, want):
+                    assert torch.equal(a, b[:n]), (threshold, n, int(stats["second_pass"]))
+                if threshold in (0.0, -1.0):
+                    assert int(stats["second_pass"]) == (0 if threshold == 0.0 else n)
 
 
 def test_boards_states_views_and_index(cuda):
@@ -99,8 +120,11 @@ def test_boards_states_views_and_index(cuda):
             assert torch.equal(p[:50], q)
 
 
-def test_graphs_and_streams(cuda):
+@pytest.mark.parametrize("precision", ["fp32", "bf16c"])
+def test_graphs_and_streams(cuda, precision):
     model, (x, _) = _model(cuda), _inputs(20)
+    model.precision = precision
+    model.cascade_threshold = 0.3      # (several boards go twice)
     xs = [torch.roll(x, i, 0).to(cuda) for i in range(3)]
     with torch.inference_mode():
         want = [model(v) for v in xs]

@@ -9,42 +9,54 @@
 
 namespace c6 {
 
-// one thread per environment
+// Eight lanes per game, one for each direction out of the new stone.  A game reads a handful of
+// scattered board bytes, so the step is a chain of memory latencies and nothing else: action and
+// state, then the neighbours, then the results.  A lane asks for up to eight neighbours of its
+// direction at once (five for six in a row) and counts the run of equal stones from the front; the
+// two halves of a line meet in one exchange between lanes.  16,384 games: 11.3 us with one thread per
+// game walking outward square by square on a quarter of the CUs, 5 us this way.
+constexpr int kStepLanes = 8, kStepAhead = 8;
 __global__ __launch_bounds__(256) void env_step_kernel(const EnvParams p) {
-  const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= p.num) return;
+  const long long i = ((long long)blockIdx.x * blockDim.x + threadIdx.x) / kStepLanes;
+  const int d = threadIdx.x % kStepLanes;
+  if (i >= p.num) return;   // (whole groups of eight lanes)
   const int n = p.n, cells = n * n;
   long long a = p.actions[i];
-  a = a < 0 ? 0 : (a >= cells ? cells - 1 : a);  // never write outside the board
-  if (p.view) a = d4_from_view((int)a, p.view, n);  // policy-view square -> board square
-  const int row = (int)(a / n), col = (int)(a - (long long)row * n);
-  int8_t *board = p.boards + i * cells;
   const int8_t actor = p.player[i];
-  board[row * n + col] = actor;
   const int16_t empty = (int16_t)(p.empty_count[i] - 1);
   const int16_t moves = (int16_t)(p.move_count[i] + 1);
+  const int8_t left = p.stones_left[i];
+  a = a < 0 ? 0 : (a >= cells ? cells - 1 : a);  // never write outside the board
+  if (p.view) a = d4_from_view((int)a, p.view, n);  // policy-view square -> board square
+  const int row = (int)a / n, col = (int)a - row * n;
+  int8_t *board = p.boards + i * cells;
+
+  // lanes d and d + 4 look the two ways along line d: row, column, both diagonals
+  const int line = d & 3, s = d < 4 ? 1 : -1;
+  const int dr = (line == 0 ? 0 : 1) * s, dc = (line == 1 ? 0 : (line == 3 ? -1 : 1)) * s;
+  const int reach = p.win - 1;   // squares each way that can matter
+  int run = 0;
+  for (int k0 = 0; k0 < reach && run == k0; k0 += kStepAhead) {
+    int8_t stone[kStepAhead];
+#pragma unroll
+    for (int k = 0; k < kStepAhead; ++k) {
+      const int r = row + (k0 + k + 1) * dr, c = col + (k0 + k + 1) * dc;
+      const bool in = k0 + k < reach && r >= 0 && r < n && c >= 0 && c < n;
+      stone[k] = in ? board[r * n + c] : (int8_t)~actor;   // (never equal to actor)
+    }
+    unsigned other = 1u << kStepAhead;
+#pragma unroll
+    for (int k = 0; k < kStepAhead; ++k) other |= stone[k] != actor ? 1u << k : 0u;
+    run += __builtin_ctz(other);
+  }
+  const int total = 1 + run + __shfl_xor(run, 4);
+  int won = total >= p.win ? 1 : 0;
+  won |= __shfl_xor(won, 1);
+  won |= __shfl_xor(won, 2);
+  if (d != 0) return;
+  board[row * n + col] = actor;
   p.empty_count[i] = empty;
   p.move_count[i] = moves;
-
-  // equal stones outward from the new one, at most win - 1 each way, along 4 directions
-  bool won = false;
-  const int reach = p.win - 1;
-#pragma unroll
-  for (int d = 0; d < 4; ++d) {
-    const int dr = d == 1 ? 0 : 1, dc = d == 0 ? 0 : (d == 3 ? -1 : 1);
-    int total = 1;
-#pragma unroll
-    for (int s = -1; s <= 1; s += 2) {
-      int r = row + s * dr, c = col + s * dc;
-      for (int k = 0; k < reach; ++k) {
-        if (r < 0 || r >= n || c < 0 || c >= n || board[r * n + c] != actor) break;
-        ++total;
-        r += s * dr;
-        c += s * dc;
-      }
-    }
-    won = won || total >= p.win;
-  }
   const bool done = won || empty == 0;
   p.reward[i] = won ? 1.0f : 0.0f;
   p.done[i] = done ? 1 : 0;
@@ -52,7 +64,7 @@ __global__ __launch_bounds__(256) void env_step_kernel(const EnvParams p) {
   p.lengths[i] = moves;
   int8_t sign = 0;
   if (!done) {  // a finished game keeps its side to move and its stones_left
-    const int8_t remaining = (int8_t)(p.stones_left[i] - 1);
+    const int8_t remaining = (int8_t)(left - 1);
     if (remaining > 0) {
       p.stones_left[i] = remaining;
       sign = 1;
@@ -159,7 +171,11 @@ __global__ __launch_bounds__(256) void canonical_input_kernel(const int8_t *__re
 
 int launch_env_step(const EnvParams &p, hipStream_t st) {
   if (p.num == 0) return C6_OK;
-  const long long blocks = (p.num + 255) / 256;
+  const long long blocks = (p.num * kStepLanes + 255) / 256;
+  if (blocks > 0x7fffffffLL) {
+    set_error("c6_env_step: %lld games exceed one launch", p.num);
+    return C6_EINVAL;
+  }
   hipLaunchKernelGGL(env_step_kernel, dim3((unsigned)blocks), dim3(256), 0, st, p);
   const hipError_t e = hipGetLastError();
   if (e != hipSuccess) {

@@ -126,7 +126,6 @@ class VectorConnect6:
     def observation(self) -> torch.Tensor:
         return self.network_input()
 
-    @torch.no_grad()
     def step(self, actions: torch.Tensor, view: int = 0) -> StepBatch:
         """connect6/vector_env.py:106-161, one launch.  ``view`` (beyond the reference's
         signature): the D4 view the actions are expressed in; the kernel maps them back as

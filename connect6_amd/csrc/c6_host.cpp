@@ -46,8 +46,13 @@ PyObject *fail(PyObject *type, const std::string &what) {
   return nullptr;
 }
 
-// A tensor argument, or null for None.  (Callers pass tensors or None only.)
-const at::Tensor *tensor_or_null(PyObject *o) { return o == Py_None ? nullptr : &THPVariable_Unpack(o); }
+// A tensor argument; anything else is a TypeError (thrown: see HANDLE_TH_ERRORS).
+const at::Tensor &tensor(PyObject *o) {
+  if (!THPVariable_Check(o)) throw torch::TypeError(std::string("expected a tensor, got ") + Py_TYPE(o)->tp_name);
+  return THPVariable_Unpack(o);
+}
+// ... or null for None
+const at::Tensor *tensor_or_null(PyObject *o) { return o == Py_None ? nullptr : &tensor(o); }
 
 std::string shape_text(const at::Tensor &t) {
   std::string s = "(";
@@ -213,8 +218,8 @@ PyObject *parameters(PyObject *, PyObject *module) {
 PyObject *forward(PyObject *, PyObject *const *a, Py_ssize_t n) {
   if (n != 16) return fail(PyExc_TypeError, "forward takes 16 arguments");
   HANDLE_TH_ERRORS
-  const at::Tensor x = THPVariable_Unpack(a[0]).contiguous();
-  const at::Tensor &packed = THPVariable_Unpack(a[1]);
+  const at::Tensor x = tensor(a[0]).contiguous();
+  const at::Tensor &packed = tensor(a[1]);
   const int prec = (int)PyLong_AsLong(a[2]);
   const int64_t groups = PyLong_AsLongLong(a[3]), per = PyLong_AsLongLong(a[4]), total = groups * per;
   const bool want_logits = PyObject_IsTrue(a[5]) == 1, want_value = PyObject_IsTrue(a[6]) == 1,
@@ -283,15 +288,15 @@ PyObject *forward(PyObject *, PyObject *const *a, Py_ssize_t n) {
 PyObject *forward_boards(PyObject *, PyObject *const *a, Py_ssize_t n) {
   if (n != 14) return fail(PyExc_TypeError, "forward_boards takes 14 arguments");
   HANDLE_TH_ERRORS
-  const at::Tensor &boards_in = THPVariable_Unpack(a[0]);
+  const at::Tensor &boards_in = tensor(a[0]);
   const at::Device dev = boards_in.device();
   const int64_t states = boards_in.size(0);
   const at::Tensor boards = boards_in.contiguous();
-  const at::Tensor player = THPVariable_Unpack(a[1]).to(dev).contiguous();
-  const at::Tensor left = THPVariable_Unpack(a[2]).to(dev).contiguous();
+  const at::Tensor player = tensor(a[1]).to(dev).contiguous();
+  const at::Tensor left = tensor(a[2]).to(dev).contiguous();
   const at::Tensor *index_in = tensor_or_null(a[3]), *u_in = tensor_or_null(a[10]);
   const int view = (int)PyLong_AsLong(a[4]);
-  const at::Tensor &packed = THPVariable_Unpack(a[5]);
+  const at::Tensor &packed = tensor(a[5]);
   const int prec = (int)PyLong_AsLong(a[6]);
   const bool want_logits = PyObject_IsTrue(a[7]) == 1;
   const int mask_mode = (int)PyLong_AsLong(a[8]);
@@ -346,8 +351,8 @@ PyObject *forward_boards(PyObject *, PyObject *const *a, Py_ssize_t n) {
 PyObject *forward_generic(PyObject *, PyObject *const *a, Py_ssize_t n) {
   if (n != 10) return fail(PyExc_TypeError, "forward_generic takes 10 arguments");
   HANDLE_TH_ERRORS
-  const at::Tensor x = THPVariable_Unpack(a[0]).contiguous();
-  const at::Tensor &packed = THPVariable_Unpack(a[1]);
+  const at::Tensor x = tensor(a[0]).contiguous();
+  const at::Tensor &packed = tensor(a[1]);
   const int64_t groups = PyLong_AsLongLong(a[2]);
   char *arch = nullptr;
   Py_ssize_t arch_bytes = 0;
@@ -387,8 +392,8 @@ PyObject *forward_generic(PyObject *, PyObject *const *a, Py_ssize_t n) {
 PyObject *mask_logits(PyObject *, PyObject *const *a, Py_ssize_t n) {
   if (n != 3) return fail(PyExc_TypeError, "mask_logits takes 3 arguments");
   HANDLE_TH_ERRORS
-  const at::Tensor src = THPVariable_Unpack(a[0]).contiguous();
-  const at::Tensor &legal_in = THPVariable_Unpack(a[1]);
+  const at::Tensor src = tensor(a[0]).contiguous();
+  const at::Tensor &legal_in = tensor(a[1]);
   void *stream = PyLong_AsVoidPtr(a[2]);
   if (PyErr_Occurred()) return nullptr;
   const at::Device dev = src.device();
@@ -411,7 +416,7 @@ PyObject *mask_logits(PyObject *, PyObject *const *a, Py_ssize_t n) {
 PyObject *sample(PyObject *, PyObject *const *a, Py_ssize_t n) {
   if (n != 6) return fail(PyExc_TypeError, "sample takes 6 arguments");
   HANDLE_TH_ERRORS
-  const at::Tensor src = THPVariable_Unpack(a[0]).to(at::kFloat).contiguous();
+  const at::Tensor src = tensor(a[0]).to(at::kFloat).contiguous();
   const at::Tensor *legal_in = tensor_or_null(a[1]);
   const float temperature = (float)PyFloat_AsDouble(a[2]);
   const at::Device dev = src.device();
@@ -420,7 +425,7 @@ PyObject *sample(PyObject *, PyObject *const *a, Py_ssize_t n) {
   if (PyErr_Occurred()) return nullptr;
   at::Tensor legal, u, logprob;
   if (legal_in != nullptr) legal = legal_in->to(dev).contiguous();
-  if (!take_draws(&THPVariable_Unpack(a[3]), b, dev, u)) return nullptr;
+  if (!take_draws(&tensor(a[3]), b, dev, u)) return nullptr;
   const c10::DeviceGuard guard(dev);
   const at::Tensor actions = fresh({b}, at::kLong, dev);
   if (PyObject_IsTrue(a[4]) == 1) logprob = fresh({b}, at::kFloat, dev);
@@ -435,10 +440,10 @@ PyObject *sample(PyObject *, PyObject *const *a, Py_ssize_t n) {
 PyObject *env_step(PyObject *, PyObject *const *a, Py_ssize_t n) {
   if (n != 9) return fail(PyExc_TypeError, "env_step takes 9 arguments");
   HANDLE_TH_ERRORS
-  const at::Tensor &boards = THPVariable_Unpack(a[0]);
+  const at::Tensor &boards = tensor(a[0]);
   const at::Device dev = boards.device();
   const int64_t num = boards.size(0);
-  const at::Tensor &actions = THPVariable_Unpack(a[5]);
+  const at::Tensor &actions = tensor(a[5]);
   const int view = (int)PyLong_AsLong(a[6]), win = (int)PyLong_AsLong(a[7]);
   void *stream = PyLong_AsVoidPtr(a[8]);
   if (PyErr_Occurred()) return nullptr;
@@ -446,9 +451,9 @@ PyObject *env_step(PyObject *, PyObject *const *a, Py_ssize_t n) {
   const at::Tensor reward = fresh({num}, at::kFloat, dev), done = fresh({num}, at::kBool, dev),
                    winner = fresh({num}, at::kChar, dev), sign = fresh({num}, at::kChar, dev),
                    lengths = fresh({num}, at::kShort, dev);
-  const int rc = abi.env_step(ptr<int8_t>(boards), ptr<int8_t>(THPVariable_Unpack(a[1])),
-                              ptr<int8_t>(THPVariable_Unpack(a[2])), ptr<int16_t>(THPVariable_Unpack(a[3])),
-                              ptr<int16_t>(THPVariable_Unpack(a[4])), ptr<int64_t>(actions), view, num,
+  const int rc = abi.env_step(ptr<int8_t>(boards), ptr<int8_t>(tensor(a[1])),
+                              ptr<int8_t>(tensor(a[2])), ptr<int16_t>(tensor(a[3])),
+                              ptr<int16_t>(tensor(a[4])), ptr<int64_t>(actions), view, num,
                               (int)boards.size(1), win, ptr<float>(reward), static_cast<uint8_t *>(done.data_ptr()),
                               ptr<int8_t>(winner), ptr<int8_t>(sign), ptr<int16_t>(lengths), stream);
   return answer<5>(rc, {reward, done, winner, sign, lengths});
@@ -459,8 +464,8 @@ PyObject *env_step(PyObject *, PyObject *const *a, Py_ssize_t n) {
 PyObject *canonical_input(PyObject *, PyObject *const *a, Py_ssize_t n) {
   if (n != 4) return fail(PyExc_TypeError, "canonical_input takes 4 arguments");
   HANDLE_TH_ERRORS
-  const at::Tensor boards = THPVariable_Unpack(a[0]).contiguous(), player = THPVariable_Unpack(a[1]).contiguous(),
-                   left = THPVariable_Unpack(a[2]).contiguous();
+  const at::Tensor boards = tensor(a[0]).contiguous(), player = tensor(a[1]).contiguous(),
+                   left = tensor(a[2]).contiguous();
   void *stream = PyLong_AsVoidPtr(a[3]);
   if (PyErr_Occurred()) return nullptr;
   const at::Device dev = boards.device();

@@ -357,3 +357,17 @@ def test_probe_library_loads_and_exports_its_symbol():
     assert _lib._PROBE_SO.exists(), "run connect6_amd.build()"
     probe = ctypes.CDLL(str(_lib._PROBE_SO))
     assert hasattr(probe, "c6_probe_mfma_rate")
+
+
+def test_native_host_side_refuses_what_is_no_tensor():
+    t = torch.zeros(2, 361)
+    host = _lib.host()
+    for call in (
+        lambda: host.sample(t, None, 1.0, [0.1, 0.2], True, 0),
+        lambda: host.sample(t, "legal", 1.0, torch.zeros(2), True, 0),
+        lambda: host.mask_logits(t, None, 0),
+        lambda: host.canonical_input(None, t, t, 0),
+        lambda: host.forward(None, *([t] * 15)),
+    ):
+        with pytest.raises(TypeError, match="expected a tensor"):
+            call()

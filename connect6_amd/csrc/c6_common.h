@@ -241,7 +241,7 @@ constexpr size_t cascade_packed_bytes(int prec) {
 // out evenly.  Layout, in int32: [0] boards listed in all (written by the second pass, for the
 // caller), [4, 4 + kCascadeMaxRuns) the counts per run, then the lists, `per` entries per run
 // (runs x per <= boards + runs).
-constexpr int kCascadeMaxRuns = 1024;   // workgroups of the first pass = compute units, at most
+constexpr int kCascadeMaxRuns = 1024;   // workgroups of the first pass: two per compute unit, at most
 constexpr size_t cascade_workspace_bytes(long long boards) {
   return (size_t)(16 + 4 * (long long)kCascadeMaxRuns + 4 * (boards + kCascadeMaxRuns) + 15) & ~(size_t)15;
 }

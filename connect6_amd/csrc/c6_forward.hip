@@ -1908,6 +1908,7 @@ __global__ __launch_bounds__(256) void fused_forward_kernel(const FwdParams prm)
 }  // namespace c6
 
 #include "c6_split.h"
+#include "c6_duo.h"
 #if defined(C6_TEAM) || !defined(C6_INSTANCE)
 #include "c6_team.h"
 #endif
@@ -2197,6 +2198,11 @@ template <class P> int launch_forward(const FwdParams &fp, hipStream_t st) {
   if (e == hipSuccess && configured_dev != dev) {
     e = hipFuncSetAttribute(kernel,
                             hipFuncAttributeMaxDynamicSharedMemorySize, LDS);
+    if constexpr (has_duo<P>()) {
+      if (e == hipSuccess)
+        e = hipFuncSetAttribute(reinterpret_cast<const void *>(&duo_forward_kernel<P>),
+                                hipFuncAttributeMaxDynamicSharedMemorySize, DuoGeo::LDS_BYTES);
+    }
     int n = 0;
     if (e == hipSuccess) e = hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev);
     if (e == hipSuccess) {
@@ -2208,12 +2214,16 @@ template <class P> int launch_forward(const FwdParams &fp, hipStream_t st) {
     set_error("fused_forward setup failed: %s", hipGetErrorString(e));
     return C6_ELAUNCH;
   }
-  long long grid = cus > 0 ? cus : 256;
-  if (grid > fp.total_boards) grid = fp.total_boards;
+  const long long grid = forward_grid<P>(fp.total_boards, cus > 0 ? cus : 256);
   if constexpr (P::ID == C6_PREC_F32S) {
     hipLaunchKernelGGL(split_forward_kernel<P>, dim3((unsigned)grid), dim3(256), LDS, st, fp);
   } else if constexpr (P::PIPE) {
-    hipLaunchKernelGGL(fused_pipe_kernel<P>, dim3((unsigned)grid), dim3(256), LDS, st, fp);
+    bool duo = false;
+    if constexpr (has_duo<P>()) {
+      duo = grid > cus;
+      if (duo) hipLaunchKernelGGL(duo_forward_kernel<P>, dim3((unsigned)grid), dim3(256), DuoGeo::LDS_BYTES, st, fp);
+    }
+    if (!duo) hipLaunchKernelGGL(fused_pipe_kernel<P>, dim3((unsigned)grid), dim3(256), LDS, st, fp);
   } else {
     hipLaunchKernelGGL(fused_forward_kernel<P>, dim3((unsigned)grid), dim3(256), LDS, st, fp);
   }
@@ -2375,7 +2385,7 @@ int dispatch_cascade(int prec, const FwdParams &fp, float threshold, void *works
   int cus = 0;
   int rc = device_cus(cus);
   if (rc != C6_OK) return rc;
-  const long long runs = cus < fp.total_boards ? cus : fp.total_boards;   // = the first kernel's grid
+  const long long runs = forward_grid<PrecBF16>(fp.total_boards, cus);
   if (runs > kCascadeMaxRuns) {
     set_error("cascade: %lld workgroups exceed the %d the workspace layout provides for", runs, kCascadeMaxRuns);
     return C6_EINVAL;

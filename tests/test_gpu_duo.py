@@ -1,0 +1,108 @@
+"""Two workgroups per CU (more boards than CUs, plain 16-bit modes) against one workgroup per board:
+the same bits at batch sizes around whole rounds, for every input form, mask and output type, and
+the cascade's lists."""
+import pytest
+import torch
+
+import connect6_amd as c6
+from connect6_amd import _lib
+from connect6_amd.model import run_forward
+from connect6_amd.synthetic import gen_boards, gen_uniform
+from oracle import torch_ref as R
+
+pytestmark = pytest.mark.gpu
+PIECE = 100   # boards of a call that one workgroup per board serves
+
+
+def _model(cuda, seed=11):
+    model = c6.PolicyValueNet().to(cuda).eval()
+    model.load_state_dict(R.init_state(seed, "torch_default"))
+    return model
+
+
+def _inputs(n):
+    x, legal = gen_boards(n, 200, 77)
+    x[3::5, 2] = (torch.rand(19, 19, generator=torch.Generator().manual_seed(1)) > 0.5).float()   # a varying third plane
+    x[4::5] *= 0.3                                                                                # not exact in 16 bits
+    return x, legal
+
+
+def _pieces(call, n):
+    """call(slice) over pieces of the batch, outputs joined."""
+    outs = [call(slice(i, min(i + PIECE, n))) for i in range(0, n, PIECE)]
+    return [torch.cat(t) if t[0] is not None else None for t in zip(*outs)]
+
+
+def _same(got, want):
+    for a, b in zip(got, want):
+        assert (a is None) == (b is None)
+        assert a is None or torch.equal(a, b)
+
+
+@pytest.mark.parametrize("prec", [_lib.PREC_BF16, _lib.PREC_F16])
+def test_same_bits_as_one_workgroup_per_board(cuda, prec):
+    cus = torch.cuda.get_device_properties(cuda).multi_processor_count
+    most = 4 * cus + 3
+    model, (x, legal) = _model(cuda), _inputs(most)
+    x, legal, u = x.to(cuda), legal.to(cuda), gen_uniform(most, 5).to(cuda)
+    packed = model.packed_weights(prec)
+
+    def call(s):
+        n = x[s].shape[0]
+        return run_forward(x[s], packed, prec, 1, n, mask_mode=_lib.MASK_LEGAL, legal=legal[s], u=u[s], temperature=0.8,
+                           want_logprob=True)
+
+    with torch.inference_mode():
+        want = _pieces(call, most)
+        for n in (cus + 1, 300, 2 * cus - 1, 2 * cus, 2 * cus + 1, 3 * cus + 9, 4 * cus, most):
+            _same(call(slice(0, n)), [w[:n] for w in want])
+        for kw in (dict(), dict(mask_mode=_lib.MASK_INPUT, fill=-3.0), dict(want_value=False)):
+            for t in (x, x.half(), x.bfloat16()):
+                part = lambda s: run_forward(t[s], packed, prec, 1, t[s].shape[0], **kw)
+                _same(part(slice(0, 777)), _pieces(part, 777))
+
+
+@pytest.mark.parametrize("prec", [_lib.PREC_BF16, _lib.PREC_F16])
+def test_weight_sets_and_board_state(cuda, prec):
+    sets, per = 3, 259
+    models = [_model(cuda, 20 + i) for i in range(sets)]
+    x = _inputs(sets * per)[0].to(cuda)
+    packed = torch.stack([m.packed_weights(prec) for m in models])
+    with torch.inference_mode():
+        logits, value, _, _ = run_forward(x, packed, prec, sets, per)
+        for i in range(sets):
+            part = lambda s: run_forward(x[i * per:(i + 1) * per][s], packed[i], prec, 1, len(range(per)[s]))
+            want = _pieces(part, per)
+            assert torch.equal(logits[i * per:(i + 1) * per], want[0])
+            assert torch.equal(value[i * per:(i + 1) * per], want[1])
+        # int8 state, rows picked (some outside: they are clamped), every board symmetry
+        g = torch.Generator().manual_seed(3)
+        boards = torch.randint(-1, 2, (700, 19, 19), generator=g, dtype=torch.int8).to(cuda)
+        player = (torch.randint(0, 2, (700,), generator=g, dtype=torch.int8) * 2 - 1).to(cuda)
+        left = torch.randint(1, 3, (700,), generator=g, dtype=torch.int8).to(cuda)
+        index = torch.randint(-5, 710, (613,), generator=g).to(cuda)
+        models[0].precision = "bf16" if prec == _lib.PREC_BF16 else "fp16"
+        for view in range(8):
+            part = lambda s: models[0].forward_boards(boards, player, left, index=index[s], view=view)
+            _same(part(slice(0, 613)), _pieces(part, 613))
+
+
+@pytest.mark.parametrize("boards", [257, 513, 1400, 4096])
+def test_cascade_lists_the_same_boards(cuda, boards):
+    model = c6.PolicyValueNet().to(cuda).eval()
+    model.load_state_dict(R.init_state(5, "reference"))
+    model.precision = "bf16c"
+    x = gen_boards(boards, 200, 9)[0].to(cuda)
+    listed = []
+
+    def call(s):
+        out = model.forward_masked(x[s])
+        listed.append(model.cascade_stats["second_pass"].clone())
+        return out
+
+    with torch.inference_mode():
+        got = call(slice(0, boards))
+        whole = int(listed.pop())
+        want = _pieces(call, boards)
+    _same(got, want)
+    assert whole == sum(int(n) for n in listed) > 0

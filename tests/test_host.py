@@ -42,6 +42,9 @@ def test_fused_kernels_stay_within_their_scratch_budget():
                 assert u["ScratchSize"] <= cap, (name, u)
                 assert u["VGPRs"] <= 256 and u["AGPRs"] <= 256 and u["Occupancy"] >= 1
     assert seen == set(limit)
+    # two workgroups per CU: half the registers, half the LDS
+    duo = [u for name, u in usage.items() if "duo_forward_kernel" in name]
+    assert len(duo) == 2 and all(u["Occupancy"] == 2 and u["ScratchSize"] <= 16 for u in duo)
 
 
 def test_history_dtype_follows_the_reference_policy():

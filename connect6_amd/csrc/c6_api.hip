@@ -21,7 +21,7 @@ int dispatch_pack(int prec, const PackParams &pp, hipStream_t st);
 int dispatch_forward(int prec, const FwdParams &fp, hipStream_t st);
 int dispatch_cascade(int prec, const FwdParams &fp, float threshold, void *workspace, const TeamParams *team,
                      hipStream_t st);
-int team_workspace_bytes(int prec, long long boards, size_t *bytes);
+int team_workspace_bytes(int prec, long long boards, size_t *bytes, long long *shared);
 int dispatch_team(int prec, const TeamParams &tp, hipStream_t st);
 size_t packed_bytes(int prec);
 int launch_mask(const void *, const uint8_t *, int, long long, uint32_t, void *, hipStream_t);
@@ -119,14 +119,15 @@ constexpr int kTeamPolls = 64;   // about 45 us
 // checked into `tp` (all but the forward's own parameters)
 static int check_team(const char *who, int prec, long long boards, const TeamArgs &t, TeamParams &tp) {
   size_t need = 0;
-  const int rc = team_workspace_bytes(prec, boards, &need);
+  long long shared = 0;
+  const int rc = team_workspace_bytes(prec, boards, &need, &shared);
   if (rc != C6_OK) return rc;
   if (need == 0) {
     set_error("%s: %lld boards of mode %d are served by one workgroup each (c6_team_bytes is 0)", who, boards, prec);
     return C6_EINVAL;
   }
   if (t.workspace == nullptr || !aligned16(t.workspace) || t.workspace_bytes < need || t.flags == nullptr ||
-      t.flag_bytes < (size_t)boards * kTeamFlags * 4 || t.tag == 0 || t.tag == 0xffffffffu) {
+      t.flag_bytes < (size_t)shared * kTeamFlags * 4 || t.tag == 0 || t.tag == 0xffffffffu) {
     set_error("%s: needs a 16-byte aligned workspace and flag words of the sizes c6_team_bytes gives, and a tag from 1 "
               "to 2^32 - 2", who);
     return C6_EINVAL;
@@ -415,8 +416,9 @@ int c6_team_bytes(int prec, int64_t boards, size_t *workspace_bytes, size_t *fla
     return C6_EINVAL;
   }
   *flag_bytes = 0;
-  const int rc = team_workspace_bytes(prec, boards, workspace_bytes);
-  if (rc == C6_OK && *workspace_bytes != 0) *flag_bytes = (size_t)boards * kTeamFlags * 4;
+  long long shared = 0;
+  const int rc = team_workspace_bytes(prec, boards, workspace_bytes, &shared);
+  *flag_bytes = (size_t)shared * kTeamFlags * 4;
   return rc;
 }
 

@@ -285,7 +285,9 @@ struct FwdParams {
   int *redo_list = nullptr;       // run r's list starts at entry r * redo_per
   int redo_runs = 0;              // workgroups (runs of boards) of the first pass
   int redo_per = 0;               // boards per run of the first pass
-  int redo_skip = -1;             // second pass: up to this many listed boards are another launch's
+  // second pass: where the listed boards leave up to redo_skip beyond a multiple of redo_round, that rest is
+  // another launch's
+  int redo_skip = -1, redo_round = 1;
 };
 
 // Few boards: several workgroups per board (c6_team.h)
@@ -294,6 +296,7 @@ struct TeamParams {
   unsigned char *act;   // TeamGeo<P>::BOARDB bytes per board
   unsigned *flags;      // kTeamFlags words per board
   unsigned tag;
+  unsigned first = 0;   // the first of the f.total_boards boards
   int polls;            // of a flag (about 0.7 us each) before a workgroup helps itself
 };
 constexpr int kTeamFlags = 256;   // words per board

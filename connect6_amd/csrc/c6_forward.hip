@@ -1287,8 +1287,9 @@ __global__ __launch_bounds__(256) void fused_pipe_kernel(const FwdParams prm) {
       if (blockIdx.x == 0) *prm.redo_count = before;   // for the caller: boards evaluated twice
     }
     __syncthreads();
-    n_items = (unsigned)before;
-    if (before <= prm.redo_skip) return;
+    const int rest = before % prm.redo_round;
+    n_items = (unsigned)(rest <= prm.redo_skip ? before - rest : before);
+    if (n_items == 0) return;
   }
   // listed board i: the run r with runs[r] <= i < runs[r + 1] (a bisection; the same in every thread)
   auto board_of = [&](unsigned i) {
@@ -2329,8 +2330,12 @@ struct TeamMode {
   int (*size)(long long boards, int wgs);      // workgroups per board
   long long (*most)(int wgs);                  // boards that are shared at all
   int (*launch)(const TeamParams &, int grid, hipStream_t);
+  bool rounds;                                 // many boards run in rounds of one workgroup per CU
 };
-template <class P> static TeamMode team_mode_of() { return {TeamGeo<P>::BOARDB, &team_size<P>, &team_most<P>, &launch_team<P>}; }
+template <class P> static TeamMode team_mode_of() {
+  return {TeamGeo<P>::BOARDB, &team_size<P>, &team_most<P>, &launch_team<P>,
+          !has_duo<P>()};
+}
 static TeamMode team_mode(int prec) {
   switch (prec) {
     case C6_PREC_F32S: return team_mode_of<PrecF32S>();
@@ -2339,30 +2344,52 @@ static TeamMode team_mode(int prec) {
     case C6_PREC_BF16F6: return team_mode_of<PrecBF16F6>();
     case C6_PREC_BF16F6W: return team_mode_of<PrecBF16F6W>();
   }
-  return {0, nullptr, nullptr, nullptr};
+  return {0, nullptr, nullptr, nullptr, false};
 }
 static int second_mode(int cascade) { return cascade == C6_PREC_BF16C ? C6_PREC_BF16F6W : C6_PREC_BF16F6; }
-// The cascade's second pass goes to teams where it will hardly list more boards than they take (42 of 256
-// CUs with low weights, 21 without): random networks with the reference's initialisation list 6 %.  Where
-// it could list more, the launch that the teams cannot serve costs 4 us before the ordinary one.
-static long long team_cascade_boards(int prec, int cus) { return 16 * team_mode(second_mode(prec)).most(cus); }
+// The cascade's second pass hands what the listed boards leave beyond whole rounds of the CUs to teams, if it
+// is no more than they take (42 boards of 256 CUs with low weights, 21 without): 4,096 boards of which 266 go
+// twice take 1,039 us so, 1,119 with a second round for the rest (303 listed).  A launch that the teams cannot
+// serve costs 4 us, so it is
+// made where the number of listed boards may well be one: random networks with the reference's initialisation
+// list 6 %, give or take a sixth.
+static bool team_cascade(int prec, long long boards, int cus) {
+  const long long most = team_mode(second_mode(prec)).most(cus), low = boards / 20, high = boards / 14;
+  return low % cus <= most || low / cus != high / cus;
+}
 
-// Exchange memory for `boards` boards of a mode, 0 where one workgroup per board serves them.
-int team_workspace_bytes(int prec, long long boards, size_t *bytes) {
+// Boards of a batch that are shared between workgroups: all where they are few; behind whole rounds of one
+// workgroup per CU the rest (fp32: 257 boards 547 -> 343 us, 341 boards 547 -> 419 us, 777 boards 1,092 ->
+// 890 us; bf16 + fp6 + low weights, 298 boards: 239 -> 191 us).  Not in the modes that put two workgroups on a
+// CU: 9 boards more than three rounds are half a round there.
+static long long team_boards(int prec, long long boards, int cus) {
+  const TeamMode m = team_mode(prec);
+  if (m.launch == nullptr) return 0;
+  if (boards <= cus) return m.size(boards, cus) > 1 ? boards : 0;
+  const long long rest = boards % cus;
+  return m.rounds && rest <= m.most(cus) ? rest : 0;
+}
+
+// Exchange memory of a call on `boards` boards of a mode, and how many boards it is for (0: one workgroup per
+// board serves them all).
+int team_workspace_bytes(int prec, long long boards, size_t *bytes, long long *shared) {
   int cus = 0;
   *bytes = 0;
+  *shared = 0;
   if (boards < 1) return C6_OK;
   const int rc = device_cus(cus);
   if (rc != C6_OK) return rc;
   if (is_cascade(prec)) {
+    if (!team_cascade(prec, boards, cus)) return C6_OK;
     const TeamMode first = team_mode(C6_PREC_BF16), second = team_mode(second_mode(prec));
-    if (boards > team_cascade_boards(prec, cus)) return C6_OK;
-    const long long teams = second.most(cus);
-    *bytes = second.board_bytes * (size_t)(boards < teams ? boards : teams);
-    if (first.size(boards, cus) > 1 && first.board_bytes * (size_t)boards > *bytes) *bytes = first.board_bytes * (size_t)boards;
+    const long long teams = second.most(cus), before = team_boards(C6_PREC_BF16, boards, cus);
+    *shared = boards < teams ? boards : teams;
+    *bytes = second.board_bytes * (size_t)*shared;
+    if (first.board_bytes * (size_t)before > *bytes) *bytes = first.board_bytes * (size_t)before;
+    if (before > *shared) *shared = before;
   } else {
-    const TeamMode m = team_mode(prec);
-    if (m.launch != nullptr && m.size(boards, cus) > 1) *bytes = m.board_bytes * (size_t)boards;
+    *shared = team_boards(prec, boards, cus);
+    *bytes = team_mode(prec).board_bytes * (size_t)*shared;
   }
   return C6_OK;
 }
@@ -2371,7 +2398,16 @@ int dispatch_team(int prec, const TeamParams &tp, hipStream_t st) {
   const int rc = device_cus(cus);
   if (rc != C6_OK) return rc;
   const TeamMode m = team_mode(prec);
-  return m.launch(tp, (int)tp.f.total_boards * m.size(tp.f.total_boards, cus), st);
+  const long long all = tp.f.total_boards, shared = team_boards(prec, all, cus);
+  TeamParams part = tp;
+  if (shared < all) {
+    part.f.total_boards = all - shared;
+    const int rc2 = dispatch_forward(prec, part.f, st);
+    if (rc2 != C6_OK) return rc2;
+  }
+  part.f.total_boards = shared;
+  part.first = (unsigned)(all - shared);
+  return m.launch(part, (int)shared * m.size(shared, cus), st);
 }
 
 // Cascade: every board through the plain bf16 kernel, whose workgroups list those of their boards
@@ -2417,6 +2453,7 @@ int dispatch_cascade(int prec, const FwdParams &fp, float threshold, void *works
     rc = teams.launch(tp, cus, st);
     if (fp.total_boards <= teams.most(cus)) return rc;
     second.redo_skip = (int)teams.most(cus);
+    second.redo_round = cus;
   }
   if (rc != C6_OK) return rc;
   return prec == C6_PREC_BF16C ? launch_forward<PrecBF16F6W>(second, st) : launch_forward<PrecBF16F6>(second, st);

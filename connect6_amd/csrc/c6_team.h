@@ -890,20 +890,25 @@ template <class P> __global__ __launch_bounds__(256) void team_forward_kernel(co
     if (tid == 0 && blockIdx.x == 0) *prm.f.redo_count = before;
     items = (unsigned)before;
   }
+  // (listed boards beyond whole rounds of the CUs; the others, and a rest that is more than the teams take,
+  // are the launch's behind this one)
+  const unsigned from = from_list ? items - items % gridDim.x : 0;
+  items -= from;
   if (items == 0) return;
   const int team = team_size<P>(items, (int)gridDim.x);
-  if (team == 1) return;   // (more listed boards than teams: the launch behind this one takes them)
+  if (team == 1) return;
   const unsigned slot = blockIdx.x / (unsigned)team;
   const int role = (int)(blockIdx.x % (unsigned)team);
   if (slot >= items) return;
-  unsigned b = slot;
+  unsigned b = prm.first + slot;
   if (from_list) {
+    const unsigned item = from + slot;
     int lo = 0, hi = prm.f.redo_runs;
     while (hi - lo > 1) {
       const int mid = (lo + hi) >> 1;
-      if ((unsigned)runs[mid] <= slot) lo = mid; else hi = mid;
+      if ((unsigned)runs[mid] <= item) lo = mid; else hi = mid;
     }
-    b = (unsigned)prm.f.redo_list[(size_t)lo * prm.f.redo_per + (slot - (unsigned)runs[lo])];
+    b = (unsigned)prm.f.redo_list[(size_t)lo * prm.f.redo_per + (item - (unsigned)runs[lo])];
   }
   if (team == 12) team_board<P, 12>(prm, smem, b, slot, role);
   if constexpr (TeamGeo<P>::SPLIT || P::WLO) {

@@ -180,9 +180,9 @@ int c6_forward_boards_cascade(const int8_t *boards, const int8_t *player,
                               size_t workspace_bytes, void *stream);
 
 /* c6_forward / c6_forward_boards with several workgroups per board, for batches that would leave
- * most of the chip idle; the same results, bit for bit.  c6_team_bytes gives the sizes of the two
- * buffers, or 0 and 0 where one workgroup per board is the better launch (many boards, or a mode
- * without such a kernel): call c6_forward there.
+ * most of the chip idle, all the time or in their last round; the same results, bit for bit.
+ * c6_team_bytes gives the sizes of the two buffers, or 0 and 0 where one workgroup per board is the
+ * better launch (or the mode has no such kernel): call c6_forward there.
  *   workspace  device, 16-byte aligned; contents need no preparation
  *   (the cascade's workspace, where there is one, comes in front of these)
  *   flags      device words through which the workgroups of this launch tell one another what is

@@ -68,6 +68,33 @@ def test_same_bits_as_one_workgroup_per_board(cuda, prec):
         assert torch.equal(a[0][3:], run_forward(xd[3:6], sets[packed.numel():], prec, 1, 3)[0])
 
 
+@pytest.mark.parametrize("prec", [_lib.PREC_F32S, _lib.PREC_BF16F6, _lib.PREC_BF16F6W])
+def test_boards_beyond_whole_rounds(cuda, prec):
+    cus = torch.cuda.get_device_properties(cuda).multi_processor_count
+    most = {_lib.PREC_F32S: cus // 3, _lib.PREC_BF16F6W: cus // 6}.get(prec, cus // 12)
+    total = 2 * cus + most + 1
+    model, (x, legal) = _model(cuda), _inputs(total)
+    xd, ld, u = x.to(cuda), legal.to(cuda), gen_uniform(total, 5).to(cuda)
+    packed = model.packed_weights(prec)
+
+    def call(a, b, x=xd, groups=1, weights=packed):
+        return run_forward(x[a:b], weights, prec, groups, (b - a) // groups, mask_mode=_lib.MASK_LEGAL, legal=ld[a:b],
+                           u=u[a:b], temperature=0.8, want_logprob=True)
+
+    with torch.inference_mode():
+        # (a hundred boards: one workgroup each)
+        want = [torch.cat(t) for t in zip(*[call(i, min(i + 100, total)) for i in range(0, total, 100)])]
+        for n in (cus, cus + 1, cus + most // 4, cus + most // 2 + 1, cus + most, cus + most + 1, 2 * cus, total - 1, total):
+            for a, b in zip(call(0, n), want):
+                assert torch.equal(a, b[:n]), n
+        # the shared ones in a weight set of their own
+        sets = torch.cat([packed, _model(cuda, 12).packed_weights(prec)])
+        n = 2 * (cus // 2 + 3)
+        got, other = call(0, n, groups=2, weights=sets), call(n // 2, n, weights=sets[packed.numel():])
+        for a, b, c in zip(got, want, other):
+            assert torch.equal(a[:n // 2], b[:n // 2]) and torch.equal(a[n // 2:], c)
+
+
 # (boards up to what the mode shares at all: 21 between twelve workgroups, 42 between six, 85 between three)
 @pytest.mark.parametrize("prec,boards", [(p, b) for p in MODES for b in (1, 7, 30, 60)
                                          if b <= {_lib.PREC_F32S: 85, _lib.PREC_BF16F6W: 42}.get(p, 21)])
@@ -95,7 +122,7 @@ def test_cascade_with_few_listed_boards(cuda, prec):
             kw = dict(mask_mode=_lib.MASK_LEGAL, temperature=0.8, want_logprob=True, threshold=threshold)
             stats = {}
             want = run_forward(xd, packed, prec, 1, 1100, legal=ld, u=u, stats=stats, **kw)
-            for n in (1, 7, 21, 22, 42, 43, 85, 86, 300, 1024):
+            for n in (1, 7, 21, 22, 42, 43, 85, 86, 257, 277, 278, 298, 299, 300, 512, 530, 1024):
                 got = run_forward(xd[:n], packed, prec, 1, n, legal=ld[:n], u=u[:n], stats=stats, **kw)
                 for a, b in zip(got, want):
                     assert torch.equal(a, b[:n]), (threshold, n, int(stats["second_pass"]))

@@ -67,9 +67,14 @@ template <class P> struct TeamGeo {
 };
 
 // How a team divides the twelve tiles of squares and a layer's cout tiles: TEAM workgroups with PXT
-// tiles of squares each, whose four waves form CG groups of cout tiles.
-template <int TEAM> struct TeamShape {
-  static constexpr int PXT = 12 / TEAM, CG = PXT == 4 ? 1 : (PXT == 2 ? 2 : 3);
+// tiles of squares each, whose four waves take PT of them and form CG groups of cout tiles.  Two tiles of
+// squares and six workgroups: a wave takes both and one cout tile, so that each weight is read by one wave;
+// with one tile of squares and up to two cout tiles per wave it is read by two, 96 bytes a cycle where the L1
+// gives 64.  (fp32 contracts a weight with three parts: there the L1 keeps up, and all four waves have work in
+// layers of two cout tiles.)
+template <class P, int TEAM> struct TeamShape {
+  static constexpr int PXT = 12 / TEAM, PT = PXT == 2 && !TeamGeo<P>::SPLIT ? 2 : 1;
+  static constexpr int CG = PXT == 4 ? 1 : (PXT == 2 ? 2 * PT : 3);
   static constexpr int tiles(int nt) { return (nt + CG - 1) / CG; }   // cout tiles of a wave
 };
 
@@ -92,11 +97,11 @@ template <class P, int TT> constexpr int team_ring() {
   return Geo<P>::W == 3 ? 6 / TT : (Geo<P>::W == 1 ? 18 / TT : (TT == 1 ? 9 : (TT == 2 ? 6 : 3)));
 }
 
-// Low-order (fp6) pass of layer L for one tile of squares, conv3_lo_pass with TT cout tiles from t0 on.
-//   rec: LDS address of the lane's square's record
-template <class P, int L, int TT>
-__device__ __forceinline__ void team_lo_pass(const unsigned char *smem, const unsigned char *packed, int lane, int rec,
-                                             int t0, f32x16 (&acc)[TT]) {
+// Low-order (fp6) pass of layer L for PT tiles of squares, conv3_lo_pass with TT cout tiles from t0 on.
+//   rec: LDS addresses of the lane's squares' records
+template <class P, int L, int TT, int PT>
+__device__ __forceinline__ void team_lo_pass(const unsigned char *smem, const unsigned char *packed, int lane,
+                                             const int (&rec)[PT], int t0, f32x16 (&acc)[PT][TT]) {
   using G = Geo<P>;
   using T = TeamGeo<P>;
   typedef int v8i __attribute__((ext_vector_type(8)));
@@ -120,27 +125,30 @@ __device__ __forceinline__ void team_lo_pass(const unsigned char *smem, const un
     constexpr int g0 = 2 * c, g1 = 2 * c + 1 < HC ? 2 * c + 1 : HC - 1;
     constexpr int o0 = ((g0 / PER32 / 3 - 1) * kPitch + g0 / PER32 % 3 - 1) * T::RECB + (g0 % PER32) * 32;
     constexpr int o1 = ((g1 / PER32 / 3 - 1) * kPitch + g1 / PER32 % 3 - 1) * T::RECB + (g1 % PER32) * 32;
-    const unsigned char *at = smem + rec + T::LO_OFF + (lane < 32 ? o0 : o1);
-    const v4i b0 = *reinterpret_cast<const v4i *>(at);
-    const v4i b1 = *reinterpret_cast<const v4i *>(at + 16);
-    const v8i b = {b0[0], b0[1], b0[2], b0[3], b1[0], b1[1], b1[2], b1[2]};
 #pragma unroll
-    for (int t = 0; t < TT; ++t) {
-      const v8i a = __builtin_shufflevector(w0[c % D][t], w1[c % D][t], 0, 1, 2, 3, 4, 5, 6, 7);
-      acc[t] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(a, b, acc[t], 2, 2, 0, scale_w, 0, b[6]);
+    for (int i = 0; i < PT; ++i) {
+      const unsigned char *at = smem + rec[i] + T::LO_OFF + (lane < 32 ? o0 : o1);
+      const v4i b0 = *reinterpret_cast<const v4i *>(at);
+      const v4i b1 = *reinterpret_cast<const v4i *>(at + 16);
+      const v8i b = {b0[0], b0[1], b0[2], b0[3], b1[0], b1[1], b1[2], b1[2]};
+#pragma unroll
+      for (int t = 0; t < TT; ++t) {
+        const v8i a = __builtin_shufflevector(w0[c % D][t], w1[c % D][t], 0, 1, 2, 3, 4, 5, 6, 7);
+        acc[i][t] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(a, b, acc[i][t], 2, 2, 0, scale_w, 0, b[6]);
+      }
     }
     load(c + D, c % D);
     __builtin_amdgcn_sched_barrier(0);
   });
 }
 
-// The contraction of 3x3 layer L for one tile of 32 squares and TT cout tiles from t0 on (tiles beyond
+// The contraction of 3x3 layer L for PT tiles of 32 squares and TT cout tiles from t0 on (tiles beyond
 // the layer's last repeat it; their results are not used).
-//   rec: LDS address of the lane's square's record;  acc: the bias on entry
-template <class P, int L, int TT>
+//   rec: LDS addresses of the lane's squares' records;  acc: the bias on entry
+template <class P, int L, int TT, int PT>
 __device__ __forceinline__ void team_conv(const unsigned char *smem, const unsigned char *packed, const WFrags &wl,
-                                          v4i (&ring)[team_ring<P, TT>()][TT][Geo<P>::W], int lane, int rec, int t0,
-                                          f32x16 (&acc)[TT]) {
+                                          v4i (&ring)[team_ring<P, TT>()][TT][Geo<P>::W], int lane,
+                                          const int (&rec)[PT], int t0, f32x16 (&acc)[PT][TT]) {
   using T = TeamGeo<P>;
   constexpr int NT = kCoutArr[L] / 32, NTP = kCinArr[L] / 32;
   constexpr int W = Geo<P>::W, NPL = T::NPL, D = team_ring<P, TT>();
@@ -148,40 +156,50 @@ __device__ __forceinline__ void team_conv(const unsigned char *smem, const unsig
   constexpr int U = P::PIPE ? kPhaseSteps : 3 * KC;     // k-steps of one unrolled round
   constexpr bool LO = P::LO6 && ((P::LO_MASK >> L) & 1);
   static_assert(KS % U == 0 && U % D == 0, "ring");
-  const int corner = rec - (kPitch + 1) * T::RECB + 16 * (lane >> 5);
+  int corner[PT];
+#pragma unroll
+  for (int p = 0; p < PT; ++p) corner[p] = rec[p] - (kPitch + 1) * T::RECB + 16 * (lane >> 5);
   // k-step v of round r: (tap, 16 channels).  Pipelined modes: a round is a phase, all taps of 32
   // channels; fp32: a round is a kernel row.
-  auto frag = [&](int r, int v, int pl) __attribute__((always_inline)) {
+  auto frag = [&](int r, int v, int p, int pl) __attribute__((always_inline)) {
     const int tap = v / 2;
     const int off = P::PIPE ? ((tap / 3) * kPitch + tap % 3) * T::RECB + (v % 2) * 32 : (v / KC) * T::RECB + (v % KC) * 32;
     const int base = P::PIPE ? r * 64 : r * kPitch * T::RECB;
-    return *reinterpret_cast<const v4i *>(smem + corner + base + off + pl * 192);
+    return *reinterpret_cast<const v4i *>(smem + corner[p] + base + off + pl * 192);
   };
-  v4i a[3][NPL];
+  v4i a[3][PT][NPL];
 #pragma unroll
   for (int v = 0; v < 2; ++v)
 #pragma unroll
-    for (int i = 0; i < NPL; ++i) a[v][i] = frag(0, v, i);
+    for (int p = 0; p < PT; ++p)
+#pragma unroll
+      for (int i = 0; i < NPL; ++i) a[v][p][i] = frag(0, v, p, i);
   auto round = [&](int r) __attribute__((always_inline)) {
     // (the low-order pass comes in front of the last phase, as in pipe_layer)
     if constexpr (LO) {
-      if (r == NTP - 1) team_lo_pass<P, L, TT>(smem, packed, lane, rec, t0, acc);
+      if (r == NTP - 1) team_lo_pass<P, L, TT, PT>(smem, packed, lane, rec, t0, acc);
     }
     static_for<0, U>([&](auto vc) __attribute__((always_inline)) {
       constexpr int v = decltype(vc)::value;
       // activations two k-steps ahead (behind the last one: the last round again, unused)
       const int rn = v + 2 < U ? r : (r + 1 < KS / U ? r + 1 : r);
 #pragma unroll
-      for (int i = 0; i < NPL; ++i) a[(v + 2) % 3][i] = frag(rn, (v + 2) % U, i);
+      for (int p = 0; p < PT; ++p)
+#pragma unroll
+        for (int i = 0; i < NPL; ++i) a[(v + 2) % 3][p][i] = frag(rn, (v + 2) % U, p, i);
 #pragma unroll
       for (int t = 0; t < TT; ++t) {
         if constexpr (NPL == 3) {
           constexpr int WP[6] = {0, 1, 2, 0, 1, 0}, AP[6] = {2, 1, 0, 1, 0, 0};
 #pragma unroll
-          for (int m = 0; m < 6; ++m) mma<P>(ring[v % D][t][WP[m]], a[v % 3][AP[m]], acc[t]);
+          for (int p = 0; p < PT; ++p)
+#pragma unroll
+            for (int m = 0; m < 6; ++m) mma<P>(ring[v % D][t][WP[m]], a[v % 3][p][AP[m]], acc[p][t]);
         } else {
 #pragma unroll
-          for (int i = 0; i < W; ++i) mma<P>(ring[v % D][t][i], a[v % 3][0], acc[t]);
+          for (int i = 0; i < W; ++i)
+#pragma unroll
+            for (int p = 0; p < PT; ++p) mma<P>(ring[v % D][t][i], a[v % 3][p][0], acc[p][t]);
         }
         const int kn = r * U + v + D;   // (behind the last k-steps: the last one again, unused)
         const int f = team_frag<P, L>(kn < KS ? kn : KS - 1, t0 + t < NT ? t0 + t : NT - 1);
@@ -275,8 +293,8 @@ __device__ __forceinline__ void team_board(const TeamParams &prm, unsigned char 
                                            int my_role) {
   using G = Geo<P>;
   using T = TeamGeo<P>;
-  using S = TeamShape<TEAM>;
-  constexpr int NPL = T::NPL, W = G::W, THREADS = 256, PXT = S::PXT, CG = S::CG;
+  using S = TeamShape<P, TEAM>;
+  constexpr int NPL = T::NPL, W = G::W, THREADS = 256, PXT = S::PXT, PT = S::PT, CG = S::CG;
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), h = lane >> 5;
   const FwdParams &f = prm.f;
   unsigned char *occ = smem + T::OCC_OFF;
@@ -290,9 +308,9 @@ __device__ __forceinline__ void team_board(const TeamParams &prm, unsigned char 
   const __amdgpu_buffer_rsrc_t mem = __builtin_amdgcn_make_buffer_rsrc(act, 0, T::BOARDB, 0x00020000);
   [[maybe_unused]] const bool trace_on = true;
 
-  // the wave's tile of squares within the workgroup's, and its group of cout tiles
-  const int wpx = PXT == 4 ? wave : (PXT == 2 ? wave & 1 : 0);
-  const int cg = PXT == 4 ? 0 : (PXT == 2 ? wave >> 1 : wave);
+  // the wave's first tile of squares within the workgroup's, and its group of cout tiles
+  const int wpx = PXT == 4 ? wave : (PXT == 2 && PT == 1 ? wave & 1 : 0);
+  const int cg = PXT == 4 ? 0 : (PXT == 2 && PT == 1 ? wave >> 1 : wave);
 
   // word l * 12 + role: the squares of stage l that the neighbours read are there; kTeamAll further on:
   // all of them
@@ -360,16 +378,20 @@ __device__ __forceinline__ void team_board(const TeamParams &prm, unsigned char 
   };
 
   // Outputs of layer L (own squares): into the records, and to memory what the neighbours read.
-  auto write_out = [&](auto lc, int role, const Span &sp, bool active, const auto &acc, int t0) __attribute__((always_inline)) {
-    constexpr int L = decltype(lc)::value, C = kCoutArr[L], NT = C / 32, UN = T::units(C);
+  // acc: N tiles of squares from the workgroup's tile px on
+  auto write_out = [&](auto lc, auto nc, int role, const Span &sp, bool active, const auto &acc, int px, int t0) __attribute__((always_inline)) {
+    constexpr int L = decltype(lc)::value, N = decltype(nc)::value, C = kCoutArr[L], NT = C / 32, UN = T::units(C);
     constexpr int TT = S::tiles(NT);
     constexpr bool LO = P::LO6 && ((P::LO_MASK >> (L + 1)) & 1);
-    const int p = sp.p0 + wpx * 32 + (lane & 31), pc = p < kPix ? p : kPix - 1;
-    const int rec = record(pc, sp.base);
     if (active) {
 #pragma unroll
-      for (int t = 0; t < TT; ++t)
-        if (t0 + t < NT) team_store<P, LO, (L >= 2)>(smem, rec, h, t0 + t, acc[t]);
+      for (int i = 0; i < N; ++i) {
+        const int p = sp.p0 + (px + i) * 32 + (lane & 31), pc = p < kPix ? p : kPix - 1;
+        const int rec = record(pc, sp.base);
+#pragma unroll
+        for (int t = 0; t < TT; ++t)
+          if (t0 + t < NT) team_store<P, LO, (L >= 2)>(smem, rec, h, t0 + t, acc[i][t]);
+      }
     }
     __syncthreads();
     auto to_memory = [&](int q, int u) __attribute__((always_inline)) {
@@ -437,7 +459,7 @@ __device__ __forceinline__ void team_board(const TeamParams &prm, unsigned char 
     }
     // the first weights, behind the activations in the queue: back by the time those are in LDS
     v4i ring[D][TT][W];
-    f32x16 acc[TT];
+    f32x16 acc[PT][TT];
     if (active) {
 #pragma unroll
       for (int d = 0; d < D; ++d)
@@ -449,7 +471,8 @@ __device__ __forceinline__ void team_board(const TeamParams &prm, unsigned char 
       for (int t = 0; t < TT; ++t) {
         f32x16 one[1];
         load_bias_tiles(one, tail + bias_offset(L) + 32 * (t0 + t < NT ? t0 + t : NT - 1), h);
-        acc[t] = one[0];
+#pragma unroll
+        for (int i = 0; i < PT; ++i) acc[i][t] = one[0];
       }
     }
     __builtin_amdgcn_sched_barrier(0);
@@ -465,19 +488,25 @@ __device__ __forceinline__ void team_board(const TeamParams &prm, unsigned char 
     __syncthreads();
     C6_MARK(6 * L + 2);
     // ---- contraction ----
-    const int p = sp.p0 + wpx * 32 + (lane & 31);
-    const bool ok = p < kPix;
-    const int rec = record(ok ? p : kPix - 1, sp.base);
-    if (active) team_conv<P, L, TT>(smem, packed, wl, ring, lane, rec, t0, acc);
+    int p[PT], rec[PT];
+    bool ok[PT];
+#pragma unroll
+    for (int i = 0; i < PT; ++i) {
+      p[i] = sp.p0 + (wpx + i) * 32 + (lane & 31);
+      ok[i] = p[i] < kPix;
+      rec[i] = record(ok[i] ? p[i] : kPix - 1, sp.base);
+    }
+    if (active) team_conv<P, L, TT, PT>(smem, packed, wl, ring, lane, rec, t0, acc);
     C6_MARK(6 * L + 3);
     if constexpr (L < 7) {
       __syncthreads();   // everybody has read this layer's input
-      write_out(lc, role, sp, active, acc, t0);
+      write_out(lc, IC<PT>{}, role, sp, active, acc, wpx, t0);
     } else {
       // heads: this wave's share of the policy (per square) and of the value
       const float *pw = tail + kBiasTotal + 4 * h;
       const int tile = role * PXT + wpx;   // of the twelve
       if constexpr (T::SPLIT) {
+        static_assert(PT == 1, "one tile of squares per wave");
         if (active) {
 #pragma unroll
           for (int t = 0; t < TT; ++t) {
@@ -487,7 +516,7 @@ __device__ __forceinline__ void team_board(const TeamParams &prm, unsigned char 
             for (int q = 0; q < 4; ++q)
 #pragma unroll
               for (int e = 0; e < 4; ++e) {
-                const float a = split_silu(acc[t][4 * q + e]);
+                const float a = split_silu(acc[0][t][4 * q + e]);
                 pol = fmaf(a, pw[32 * (t0 + t) + 8 * q + e], pol);
                 val = fmaf(a, pw[kHeadC + 32 * (t0 + t) + 8 * q + e], val);
               }
@@ -495,9 +524,9 @@ __device__ __forceinline__ void team_board(const TeamParams &prm, unsigned char 
             const auto x = __builtin_amdgcn_permlane32_swap(bits, bits, false, false);
             const unsigned x0 = x[0], x1 = x[1];
             const float tot = __builtin_bit_cast(float, x0) + __builtin_bit_cast(float, x1);
-            const float vs = wave_sum(ok ? val : 0.0f);
-            if (h == 0 && ok)
-              __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(int, tot), mem, T::HEAD_OFF + ((t0 + t) * 384 + p) * 4, 0, kSc1);
+            const float vs = wave_sum(ok[0] ? val : 0.0f);
+            if (h == 0 && ok[0])
+              __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(int, tot), mem, T::HEAD_OFF + ((t0 + t) * 384 + p[0]) * 4, 0, kSc1);
             if (lane == 0)
               __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(int, vs), mem, T::VAL_OFF + ((t0 + t) * 12 + tile) * 4, 0, kSc1);
           }
@@ -511,47 +540,56 @@ __device__ __forceinline__ void team_board(const TeamParams &prm, unsigned char 
 #pragma unroll
           for (int t = 0; t < TT; ++t) {
             if (t0 + t >= NT) continue;
-            float val0 = 0.0f;
+            float val0[PT];
+#pragma unroll
+            for (int i = 0; i < PT; ++i) val0[i] = 0.0f;
 #pragma unroll
             for (int q = 0; q < 4; ++q) {
               pw4[t][q] = *reinterpret_cast<const f32x4 *>(pw + 32 * (t0 + t) + 8 * q);
               const f32x4 vw4 = *reinterpret_cast<const f32x4 *>(pw + kHeadC + 32 * (t0 + t) + 8 * q);
-              float vs = 0.0f;
 #pragma unroll
-              for (int e = 0; e < 4; ++e) {
-                const float a = silu<P>(acc[t][4 * q + e]);
-                acc[t][4 * q + e] = a;
-                val0 = fmaf(a, vw4[e], val0);
-                vs = fmaf(a, vw4[e], vs);
+              for (int i = 0; i < PT; ++i) {
+                float vs = 0.0f;
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                  const float a = silu<P>(acc[i][t][4 * q + e]);
+                  acc[i][t][4 * q + e] = a;
+                  val0[i] = fmaf(a, vw4[e], val0[i]);
+                  vs = fmaf(a, vw4[e], vs);
+                }
+                // (tile 0: one chain over its sixteen channels; the others: one sum per four)
+                if (t0 + t > 0)
+                  __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(int, vs), mem,
+                                                        T::VAL_OFF + (((tile + i) * 9 + 1 + 4 * (t0 + t - 1) + q) * 64 + lane) * 4, 0, kSc1);
               }
-              // (tile 0: one chain over its sixteen channels; the others: one sum per four)
-              if (t0 + t > 0)
-                __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(int, vs), mem,
-                                                      T::VAL_OFF + ((tile * 9 + 1 + 4 * (t0 + t - 1) + q) * 64 + lane) * 4, 0, kSc1);
             }
-            if (t0 + t == 0)
-              __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(int, val0), mem, T::VAL_OFF + (tile * 9 * 64 + lane) * 4, 0, kSc1);
+#pragma unroll
+            for (int i = 0; i < PT; ++i)
+              if (t0 + t == 0)
+                __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(int, val0[i]), mem, T::VAL_OFF + ((tile + i) * 9 * 64 + lane) * 4, 0, kSc1);
           }
         }
-        float pol = 0.0f;
 #pragma unroll
         for (int turn = 0; turn < CG; ++turn) {
           if (turn == cg && active) {
-            if (cg > 0) pol = chain[wpx * 64 + lane];
 #pragma unroll
-            for (int t = 0; t < TT; ++t) {
-              if (t0 + t >= NT) continue;
+            for (int k = 0; k < PT; ++k) {
+              float pol = cg > 0 ? chain[(wpx + k) * 64 + lane] : 0.0f;
 #pragma unroll
-              for (int i = 0; i < 16; ++i) pol = fmaf(acc[t][i], pw4[t][i / 4][i % 4], pol);
-            }
-            chain[wpx * 64 + lane] = pol;
-            if (turn == CG - 1 || t0 + TT >= NT) {
-              const unsigned bits = __builtin_bit_cast(unsigned, pol);
-              const auto x = __builtin_amdgcn_permlane32_swap(bits, bits, false, false);
-              const unsigned x0 = x[0], x1 = x[1];
-              const float tot = __builtin_bit_cast(float, x0) + __builtin_bit_cast(float, x1);
-              if (h == 0 && ok)
-                __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(int, tot), mem, T::HEAD_OFF + p * 4, 0, kSc1);
+              for (int t = 0; t < TT; ++t) {
+                if (t0 + t >= NT) continue;
+#pragma unroll
+                for (int i = 0; i < 16; ++i) pol = fmaf(acc[k][t][i], pw4[t][i / 4][i % 4], pol);
+              }
+              chain[(wpx + k) * 64 + lane] = pol;
+              if (turn == CG - 1 || t0 + TT >= NT) {
+                const unsigned bits = __builtin_bit_cast(unsigned, pol);
+                const auto x = __builtin_amdgcn_permlane32_swap(bits, bits, false, false);
+                const unsigned x0 = x[0], x1 = x[1];
+                const float tot = __builtin_bit_cast(float, x0) + __builtin_bit_cast(float, x1);
+                if (h == 0 && ok[k])
+                  __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(int, tot), mem, T::HEAD_OFF + p[k] * 4, 0, kSc1);
+              }
             }
           }
           if (turn + 1 < CG) __syncthreads();
@@ -567,14 +605,16 @@ __device__ __forceinline__ void team_board(const TeamParams &prm, unsigned char 
   auto first_stage = [&](int role) __attribute__((always_inline)) -> bool {
     const Span sp = span_of(role);
     int *flag = reinterpret_cast<int *>(red) + 64;   // [0]: third plane varies, [1]: an input is not exact in bf16
-    const int p = sp.p0 + wpx * 32 + (lane & 31);
+    const int px = PXT == 4 ? wave : (PXT == 2 ? wave & 1 : 0);   // (one cout tile: a wave per tile of squares)
+    const int p = sp.p0 + px * 32 + (lane & 31);
     const int pc = p < kPix ? p : kPix - 1, r = pc / kBoard, c = pc - r * kBoard;
-    const bool active = cg == 0;
+    const bool active = wave < PXT;
     region_role = -1;
-    f32x16 acc[1];
+    f32x16 one[1][1];
+    f32x16 (&acc)[1] = one[0];
     if (active) {
       // (the table holds the squares as the one-workgroup kernels' lanes do: by tile of 32)
-      const WFrags tb = packed_frags<P>(packed, lane, G::PLANE2_FRAG_OFF + (role * PXT + wpx) * 4);
+      const WFrags tb = packed_frags<P>(packed, lane, G::PLANE2_FRAG_OFF + (role * PXT + px) * 4);
 #pragma unroll
       for (int q = 0; q < 4; ++q) {
         const f32x4 t4 = __builtin_bit_cast(f32x4, tb[q]);
@@ -709,7 +749,7 @@ __device__ __forceinline__ void team_board(const TeamParams &prm, unsigned char 
     C6_MARK(2);
     __syncthreads();   // the copies give way to the activations
     clear_region(sp);
-    write_out(IC<0>{}, role, sp, active, acc, 0);
+    write_out(IC<0>{}, IC<1>{}, role, sp, active, one, px, 0);
     C6_MARK(3);
     return true;
   };
@@ -856,11 +896,11 @@ __device__ __forceinline__ void team_board(const TeamParams &prm, unsigned char 
 // bf16 + fp6 51 / 65 / 79 against 63, plain bf16 44 us (20 boards) against 46.
 template <class P> __host__ __device__ inline int team_size(long long boards, int wgs) {
   if (boards * 12 <= wgs) return 12;
-  if ((TeamGeo<P>::SPLIT || P::WLO) && boards * 6 <= wgs) return 6;
+  if ((TeamGeo<P>::SPLIT || P::LO6) && boards * 6 <= wgs) return 6;
   return TeamGeo<P>::SPLIT && boards * 3 <= wgs ? 3 : 1;
 }
 // ... and the most boards that are shared at all
-template <class P> inline long long team_most(int wgs) { return wgs / (TeamGeo<P>::SPLIT ? 3 : (P::WLO ? 6 : 12)); }
+template <class P> inline long long team_most(int wgs) { return wgs / (TeamGeo<P>::SPLIT ? 3 : (P::LO6 ? 6 : 12)); }
 
 template <class P> __global__ __launch_bounds__(256) void team_forward_kernel(const TeamParams prm) {
   using T = TeamGeo<P>;
@@ -911,7 +951,7 @@ template <class P> __global__ __launch_bounds__(256) void team_forward_kernel(co
     b = (unsigned)prm.f.redo_list[(size_t)lo * prm.f.redo_per + (item - (unsigned)runs[lo])];
   }
   if (team == 12) team_board<P, 12>(prm, smem, b, slot, role);
-  if constexpr (TeamGeo<P>::SPLIT || P::WLO) {
+  if constexpr (TeamGeo<P>::SPLIT || P::LO6) {
     if (team == 6) team_board<P, 6>(prm, smem, b, slot, role);
   }
   if constexpr (TeamGeo<P>::SPLIT) {

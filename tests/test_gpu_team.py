@@ -71,7 +71,7 @@ def test_same_bits_as_one_workgroup_per_board(cuda, prec):
 @pytest.mark.parametrize("prec", [_lib.PREC_F32S, _lib.PREC_BF16F6, _lib.PREC_BF16F6W])
 def test_boards_beyond_whole_rounds(cuda, prec):
     cus = torch.cuda.get_device_properties(cuda).multi_processor_count
-    most = {_lib.PREC_F32S: cus // 3, _lib.PREC_BF16F6W: cus // 6}.get(prec, cus // 12)
+    most = cus // 3 if prec == _lib.PREC_F32S else cus // 6
     total = 2 * cus + most + 1
     model, (x, legal) = _model(cuda), _inputs(total)
     xd, ld, u = x.to(cuda), legal.to(cuda), gen_uniform(total, 5).to(cuda)
@@ -97,7 +97,7 @@ def test_boards_beyond_whole_rounds(cuda, prec):
 
 # (boards up to what the mode shares at all: 21 between twelve workgroups, 42 between six, 85 between three)
 @pytest.mark.parametrize("prec,boards", [(p, b) for p in MODES for b in (1, 7, 30, 60)
-                                         if b <= {_lib.PREC_F32S: 85, _lib.PREC_BF16F6W: 42}.get(p, 21)])
+                                         if b <= {_lib.PREC_F32S: 85, _lib.PREC_BF16F6W: 42, _lib.PREC_BF16F6: 42}.get(p, 21)])
 def test_a_workgroup_that_waited_long_enough_does_the_work_itself(cuda, prec, boards):
     model, (x, _) = _model(cuda), _inputs(boards)
     xd = x.to(cuda)

@@ -892,8 +892,8 @@ __device__ __forceinline__ void team_board(const TeamParams &prm, unsigned char 
 // How many workgroups share a board when there are `boards` of them: as many as fit the chip at once, where
 // that beats one workgroup (1: the one-workgroup kernels).  With fewer workgroups per board more waves read
 // the same weights, and the L1's 64 bytes a cycle bound the layers: measured, 20 / 40 / 80 boards against
-// one workgroup each, fp32 66 / 95 / 150 us against 205, bf16 + fp6 + low weights 55 / 78 / 102 against 89,
-// bf16 + fp6 51 / 65 / 79 against 63, plain bf16 44 us (20 boards) against 46.
+// one workgroup each, fp32 66 / 95 / 134 us against 205, bf16 + fp6 + low weights 52 / 67 / 102 against 89,
+// bf16 + fp6 45 / 55 / 79 against 63, plain bf16 44 us (20 boards) against 46.
 template <class P> __host__ __device__ inline int team_size(long long boards, int wgs) {
   if (boards * 12 <= wgs) return 12;
   if ((TeamGeo<P>::SPLIT || P::LO6) && boards * 6 <= wgs) return 6;
@@ -937,8 +937,18 @@ template <class P> __global__ __launch_bounds__(256) void team_forward_kernel(co
   if (items == 0) return;
   const int team = team_size<P>(items, (int)gridDim.x);
   if (team == 1) return;
-  const unsigned slot = blockIdx.x / (unsigned)team;
-  const int role = (int)(blockIdx.x % (unsigned)team);
+  unsigned slot = blockIdx.x / (unsigned)team;
+  int role = (int)(blockIdx.x % (unsigned)team);
+  // A team on one XCD (workgroup i runs on XCD i % 8), neighbouring boards on the same one, where that many
+  // teams fit: a weight set then comes into one L2 and not into eight.  (27 listed boards of 128 weight sets:
+  // the cascade 183 -> 179 us; of 16 sets, 6 boards: 105 -> 96 us; eight fp32 boards of one set 66.5 -> 64.4 us.)
+  if (gridDim.x % 8 == 0) {
+    const unsigned per = (items + 7) / 8, l = blockIdx.x / 8;
+    if (per * (unsigned)team <= gridDim.x / 8) {
+      role = (int)(l % (unsigned)team);
+      slot = l / (unsigned)team < per ? blockIdx.x % 8 * per + l / (unsigned)team : items;
+    }
+  }
   if (slot >= items) return;
   unsigned b = prm.first + slot;
   if (from_list) {

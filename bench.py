@@ -100,13 +100,14 @@ def main() -> int:
     wall, kern = run_mode(args.precision, K, W)
     value = B / wall
     achieved = B * CONV_FLOP_PER_BOARD / kern / 1e12
-    kernel_name = {"fp32": "fused_forward_kernel<fp32>"}.get(args.precision, f"fused_pipe_kernel<{args.precision}>")
+    kernel_name = {"fp32": "split_forward_kernel<fp32>", "bf16": "duo_forward_kernel<bf16>",
+                   "fp16": "duo_forward_kernel<fp16>"}.get(args.precision, f"fused_pipe_kernel<{args.precision}>")
     cascade = None
     if args.precision == "bf16c":
         # HIP events bracket the whole step: the bf16 kernel over all boards, then the kernel
         # that carries the low parts over the listed ones.  The first pass alone is timed with
         # threshold 0 (no board listed; the second kernel still starts and finds nothing).
-        kernel_name = "fused_pipe_kernel<bf16> over all boards + fused_pipe_kernel<bf16f6w> over the listed boards"
+        kernel_name = "duo_forward_kernel<bf16> over all boards + fused_pipe_kernel<bf16f6w> over the listed boards"
         twice = int(model.cascade_stats["second_pass"].item())
         model.cascade_threshold = 0.0
         _, first = run_mode("bf16c", max(5, K // 2), 3)

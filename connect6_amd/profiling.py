@@ -2,7 +2,7 @@
 
 ``python -m connect6_amd.profiling --build`` compiles a copy of the library with ``-DC6_TRACE``
 (``lib/libconnect6_amd_trace.so``: the kernels record the shader cycle counter at phase
-boundaries of the third board of every workgroup); ``python -m connect6_amd.profiling bf16f6 bf16``
+boundaries of the third board of every workgroup); ``python -m connect6_amd.profiling bf16f6 bf16f6w``
 then runs B=4096 forwards on the GPU through that copy and prints, per arithmetic mode, the mean
 cycles per phase over all workgroups and waves and the shader clock during the traced board.
 The shipped library contains none of this.
@@ -133,6 +133,8 @@ def phase_table(precision: str, batch: int = 4096, launches: int = 150) -> str:
     import numpy as np
     import torch
 
+    if precision not in ("bf16f6w", "bf16f6"):   # (bf16 and fp16 run another kernel on this many boards)
+        raise _lib.C6Error("phases are marked in the pipelined kernel (bf16f6w, bf16f6)")
     if not TRACE_SO.exists():
         raise _lib.C6Error(f"{TRACE_SO} is missing: python -m connect6_amd.profiling --build")
     if _lib._lib is not None and Path(_lib._SO) != TRACE_SO:
@@ -158,8 +160,6 @@ def phase_table(precision: str, batch: int = 4096, launches: int = 150) -> str:
     if rc != 0:
         raise _lib.C6Error(f"c6_debug_trace failed with HIP error {rc}")
     raw = buf.reshape(256, 4, 64).astype(np.float64)
-    if precision not in ("bf16f6w", "bf16f6", "bf16", "fp16"):
-        raise _lib.C6Error("phase names are defined for the pipelined kernel (bf16f6w, bf16f6, bf16, fp16)")
     t = raw[:, :, _PIPE_MARKS]
     d = np.diff(t, axis=2)
     tot = t[:, :, -1] - t[:, :, 0]

@@ -2348,8 +2348,9 @@ static TeamMode team_mode(int prec) {
 }
 static int second_mode(int cascade) { return cascade == C6_PREC_BF16C ? C6_PREC_BF16F6W : C6_PREC_BF16F6; }
 // The cascade's second pass hands what the listed boards leave beyond whole rounds of the CUs to teams, if it
-// is no more than they take (42 boards of 256 CUs): 4,096 boards of which 266 go
-// twice take 1,039 us so, 1,119 with a second round for the rest (303 listed).  A launch that the teams cannot
+// is no more than they take (73 boards of 256 CUs with low weights, 42 without): 4,096 boards of which
+// 266 go twice take 1,039 us so, 1,119 with a second round for the rest (303 listed; three workgroups per
+// board: 1,086).  A launch that the teams cannot
 // serve costs 4 us, so it is
 // made where the number of listed boards may well be one: random networks with the reference's initialisation
 // list 6 %, give or take a sixth.

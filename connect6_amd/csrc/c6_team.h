@@ -67,14 +67,14 @@ template <class P> struct TeamGeo {
 };
 
 // How a team divides the twelve tiles of squares and a layer's cout tiles: TEAM workgroups with PXT
-// tiles of squares each, whose four waves take PT of them and form CG groups of cout tiles.  Two tiles of
-// squares and six workgroups: a wave takes both and one cout tile, so that each weight is read by one wave;
-// with one tile of squares and up to two cout tiles per wave it is read by two, 96 bytes a cycle where the L1
-// gives 64.  (fp32 contracts a weight with three parts: there the L1 keeps up, and all four waves have work in
-// layers of two cout tiles.)
+// tiles of squares each, whose four waves take PT of them and form CG groups of cout tiles.  A wave takes two
+// tiles of squares where there are two: with six workgroups each weight is then read by one wave, with three
+// by two; with one tile of squares per wave it would be twice as many, 96 and 128 bytes a cycle where the L1
+// gives 64 (six workgroups, 22 to 42 boards, bf16 + fp6 62.6 -> 55 us).  (fp32 contracts a weight with three
+// parts: there the L1 keeps up, and all four waves have work in layers of two cout tiles.)
 template <class P, int TEAM> struct TeamShape {
-  static constexpr int PXT = 12 / TEAM, PT = PXT == 2 && !TeamGeo<P>::SPLIT ? 2 : 1;
-  static constexpr int CG = PXT == 4 ? 1 : (PXT == 2 ? 2 * PT : 3);
+  static constexpr int PXT = 12 / TEAM, PT = PXT > 1 && !TeamGeo<P>::SPLIT ? 2 : 1;
+  static constexpr int PG = PXT / PT, CG = PG == 1 ? (PXT == 1 ? 3 : 4) : 4 / PG;   // groups of squares' tiles, of cout tiles
   static constexpr int tiles(int nt) { return (nt + CG - 1) / CG; }   // cout tiles of a wave
 };
 
@@ -309,8 +309,7 @@ __device__ __forceinline__ void team_board(const TeamParams &prm, unsigned char 
   [[maybe_unused]] const bool trace_on = true;
 
   // the wave's first tile of squares within the workgroup's, and its group of cout tiles
-  const int wpx = PXT == 4 ? wave : (PXT == 2 && PT == 1 ? wave & 1 : 0);
-  const int cg = PXT == 4 ? 0 : (PXT == 2 && PT == 1 ? wave >> 1 : wave);
+  const int wpx = wave % S::PG * PT, cg = wave / S::PG;
 
   // word l * 12 + role: the squares of stage l that the neighbours read are there; kTeamAll further on:
   // all of them
@@ -892,15 +891,20 @@ __device__ __forceinline__ void team_board(const TeamParams &prm, unsigned char 
 // How many workgroups share a board when there are `boards` of them: as many as fit the chip at once, where
 // that beats one workgroup (1: the one-workgroup kernels).  With fewer workgroups per board more waves read
 // the same weights, and the L1's 64 bytes a cycle bound the layers: measured, 20 / 40 / 80 boards against
-// one workgroup each, fp32 66 / 95 / 134 us against 205, bf16 + fp6 + low weights 52 / 67 / 102 against 89,
-// bf16 + fp6 45 / 55 / 79 against 63, plain bf16 44 us (20 boards) against 46.
+// one workgroup each, fp32 66 / 95 / 134 us against 205, bf16 + fp6 + low weights 52 / 67 / 92 against 90 (60
+// boards 83, so three workgroups take up to 73 of 256 CUs; behind a first pass, 53 listed boards, 85 us against
+// 110), bf16 + fp6 45 / 55 / 79 against 63, plain bf16 44 us (20 boards) against 46.
 template <class P> __host__ __device__ inline int team_size(long long boards, int wgs) {
   if (boards * 12 <= wgs) return 12;
   if ((TeamGeo<P>::SPLIT || P::LO6) && boards * 6 <= wgs) return 6;
-  return TeamGeo<P>::SPLIT && boards * 3 <= wgs ? 3 : 1;
+  if (TeamGeo<P>::SPLIT) return boards * 3 <= wgs ? 3 : 1;
+  return P::WLO && boards * 7 <= wgs * 2 ? 3 : 1;
 }
 // ... and the most boards that are shared at all
-template <class P> inline long long team_most(int wgs) { return wgs / (TeamGeo<P>::SPLIT ? 3 : (P::LO6 ? 6 : 12)); }
+template <class P> inline long long team_most(int wgs) {
+  if (TeamGeo<P>::SPLIT) return wgs / 3;
+  return P::WLO ? wgs * 2 / 7 : wgs / (P::LO6 ? 6 : 12);
+}
 
 template <class P> __global__ __launch_bounds__(256) void team_forward_kernel(const TeamParams prm) {
   using T = TeamGeo<P>;
@@ -964,7 +968,7 @@ template <class P> __global__ __launch_bounds__(256) void team_forward_kernel(co
   if constexpr (TeamGeo<P>::SPLIT || P::LO6) {
     if (team == 6) team_board<P, 6>(prm, smem, b, slot, role);
   }
-  if constexpr (TeamGeo<P>::SPLIT) {
+  if constexpr (TeamGeo<P>::SPLIT || P::WLO) {
     if (team == 3) team_board<P, 3>(prm, smem, b, slot, role);
   }
 }

@@ -52,7 +52,7 @@ def test_same_bits_as_one_workgroup_per_board(cuda, prec):
     with torch.inference_mode():
         kw = dict(mask_mode=_lib.MASK_LEGAL, u=u, temperature=0.8, want_logprob=True)
         want = run_forward(xd, packed, prec, 1, 300, legal=ld, **kw)
-        for n in (1, 2, 5, 20, 21, 22, 41, 42, 43, 84, 85, 86):
+        for n in (1, 2, 5, 20, 21, 22, 41, 42, 43, 72, 73, 74, 84, 85, 86):
             kw["u"] = u[:n]
             got = run_forward(xd[:n], packed, prec, 1, n, legal=ld[:n], **kw)
             for a, b in zip(got, want):
@@ -71,7 +71,7 @@ def test_same_bits_as_one_workgroup_per_board(cuda, prec):
 @pytest.mark.parametrize("prec", [_lib.PREC_F32S, _lib.PREC_BF16F6, _lib.PREC_BF16F6W])
 def test_boards_beyond_whole_rounds(cuda, prec):
     cus = torch.cuda.get_device_properties(cuda).multi_processor_count
-    most = cus // 3 if prec == _lib.PREC_F32S else cus // 6
+    most = {_lib.PREC_F32S: cus // 3, _lib.PREC_BF16F6W: cus * 2 // 7}.get(prec, cus // 6)
     total = 2 * cus + most + 1
     model, (x, legal) = _model(cuda), _inputs(total)
     xd, ld, u = x.to(cuda), legal.to(cuda), gen_uniform(total, 5).to(cuda)
@@ -95,9 +95,9 @@ def test_boards_beyond_whole_rounds(cuda, prec):
             assert torch.equal(a[:n // 2], b[:n // 2]) and torch.equal(a[n // 2:], c)
 
 
-# (boards up to what the mode shares at all: 21 between twelve workgroups, 42 between six, 85 between three)
+# (boards up to what the mode shares at all: 21 between twelve workgroups, 42 between six, 73 or 85 between three)
 @pytest.mark.parametrize("prec,boards", [(p, b) for p in MODES for b in (1, 7, 30, 60)
-                                         if b <= {_lib.PREC_F32S: 85, _lib.PREC_BF16F6W: 42, _lib.PREC_BF16F6: 42}.get(p, 21)])
+                                         if b <= {_lib.PREC_F32S: 85, _lib.PREC_BF16F6W: 73, _lib.PREC_BF16F6: 42}.get(p, 21)])
 def test_a_workgroup_that_waited_long_enough_does_the_work_itself(cuda, prec, boards):
     model, (x, _) = _model(cuda), _inputs(boards)
     xd = x.to(cuda)
@@ -122,7 +122,7 @@ def test_cascade_with_few_listed_boards(cuda, prec):
             kw = dict(mask_mode=_lib.MASK_LEGAL, temperature=0.8, want_logprob=True, threshold=threshold)
             stats = {}
             want = run_forward(xd, packed, prec, 1, 1100, legal=ld, u=u, stats=stats, **kw)
-            for n in (1, 7, 21, 22, 42, 43, 85, 86, 257, 277, 278, 298, 299, 300, 512, 530, 1024):
+            for n in (1, 7, 21, 22, 42, 43, 85, 86, 257, 277, 278, 298, 299, 300, 329, 330, 512, 530, 1024):
                 got = run_forward(xd[:n], packed, prec, 1, n, legal=ld[:n], u=u[:n], stats=stats, **kw)
                 for a, b in zip(got, want):
                     assert torch.equal(a, b[:n]), (threshold, n, int(stats["second_pass"]))

@@ -15,6 +15,8 @@
 // layers that read them split them in registers, 44 instructions for eight values, a few behind each
 // MFMA.
 //
+// An infinity has no such parts (inf - inf): where the fp32 instructions carried one on, this gives NaN.
+//
 // As in the 16-bit modes all activations carry the factor -log2(e), so that SiLU is
 // u / (1 + 2^u).
 #pragma once

@@ -310,12 +310,12 @@ __global__ __launch_bounds__(256, 2) void duo_forward_kernel(const FwdParams prm
         int l1fast[3];
 #pragma unroll
         for (int j = 0; j < 3; ++j) l1fast[j] = l1base[j] - (kL1RowsHalf - 1) * h * kL1RowPitch * G::EB;
-        conv1_fast_pass<P>(smem, packed_frags<P>(packed, lane, G::FAST1_OFF), r1, l1fast, a0);
+        conv1_fast_pass<P>(smem, packed_frags<P>(packed, lane, G::FAST1_OFF), r1, l1fast, a0, a0);
       } else {
 #pragma unroll
         for (int j = 0; j < 3; ++j) a0[0][j] = b0[0];
         preload_ring<L1Pipe<P>::D, 1>(r1, layer_weights<P, 0>(packed, lane));
-        conv1_pass<P>(smem, layer_weights<P, 0>(packed, lane), r1, l1base, a0);
+        conv1_pass<P>(smem, layer_weights<P, 0>(packed, lane), r1, l1base, a0, a0);
       }
     }
     DuoWeights<1> w1;

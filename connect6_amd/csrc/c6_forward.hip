@@ -152,6 +152,15 @@ template <class P> __device__ __forceinline__ float silu(float v) {
   }
 }
 template <class P> __host__ __device__ constexpr float act_scale() { return P::EB == 4 ? 1.0f : kActScale; }
+// What is scaled while the weights are packed: fp32 by three parts takes the factor to 53 bits, so that a
+// weight is rounded once, when its three parts are taken, and a bias and a sum of weights once, to fp32.
+// (Its head weights are not divided by it: the sums over them are, in the kernel.)
+template <class P> using Scaled = std::conditional_t<P::WLO == 2, double, float>;
+constexpr double kActScale64 = -1.4426950408889634074;
+template <class P> __device__ __forceinline__ Scaled<P> act_scaled(Scaled<P> v) {
+  if constexpr (P::WLO == 2) return v * kActScale64;
+  else return v * act_scale<P>();
+}
 
 __device__ __forceinline__ float load_x(const void *x, int dt, size_t i) {
   if (dt == C6_DT_F32) return reinterpret_cast<const float *>(x)[i];
@@ -250,10 +259,11 @@ template <int N_MFMA, int N_DSREAD, int N_VMEM> __device__ __forceinline__ void 
 // ------------------------------------------------------------------------
 // first layer: 23x23 on 3 planes, K = (ky, plane, kx24) split over lane halves
 // ------------------------------------------------------------------------
+// low: what the second and third part of a weight add to (another sum than acc where there are three)
 template <class P>
 __device__ __forceinline__ void conv1_pass(const unsigned char *smem, const WFrags &wl,
                                            v4i (&ring)[L1Pipe<P>::D][1], const int (&l1base)[3],
-                                           f32x16 (&acc)[1][3]) {
+                                           f32x16 (&acc)[1][3], f32x16 (&low)[1][3]) {
   using G = Geo<P>;
   using PP = L1Pipe<P>;
   constexpr int CPR = PP::CPR, U = PP::U, D = PP::D, ITERS = PP::ITERS, W = G::W;
@@ -281,12 +291,12 @@ __device__ __forceinline__ void conv1_pass(const unsigned char *smem, const WFra
 #pragma unroll
       for (int j = 0; j < 3; ++j)
         bq[un % (kAhead + 1)][j] = *reinterpret_cast<const v4i *>(smem + l1base[j] + adv + offn);
+      static_for<0, W>([&](auto wc) __attribute__((always_inline)) {  // the weights, then (WLO) what their rounding dropped
+        constexpr int w = decltype(wc)::value;
 #pragma unroll
-      for (int w = 0; w < W; ++w) {  // the weights, then (WLO) what their rounding dropped
-#pragma unroll
-        for (int j = 0; j < 3; ++j) mma<P>(ring[(u * W + w) % D][0], bq[u % (kAhead + 1)][j], acc[0][j]);
+        for (int j = 0; j < 3; ++j) mma<P>(ring[(u * W + w) % D][0], bq[u % (kAhead + 1)][j], w > 0 ? low[0][j] : acc[0][j]);
         ring[(u * W + w) % D][0] = wn[u * W + w];  // fragment (it*U + u) * W + w + D (the tail over-reads the next layer)
-      }
+      });
       interleave_step<3 * W * (P::EB == 4 ? 4 : 1), 3, W>();
       __builtin_amdgcn_sched_barrier(0);
     }
@@ -299,7 +309,7 @@ __device__ __forceinline__ void conv1_pass(const unsigned char *smem, const WFra
 template <class P>
 __device__ __forceinline__ void conv1_fast_pass(const unsigned char *smem, const WFrags &wl,
                                                 v4i (&ring)[L1Pipe<P>::D][1], const int (&l1fast)[3],
-                                                f32x16 (&acc)[1][3]) {
+                                                f32x16 (&acc)[1][3], f32x16 (&low)[1][3]) {
   using G = Geo<P>;
   constexpr int CPR = G::CPR, D = L1Pipe<P>::D, QN = kAhead + 1, S = G::FAST1_STEPS, W = G::W;
   constexpr int ROWB = kL1RowPitch * G::EB;
@@ -318,13 +328,12 @@ __device__ __forceinline__ void conv1_fast_pass(const unsigned char *smem, const
 #pragma unroll
       for (int j = 0; j < 3; ++j) bq[(s + kAhead) % QN][j] = frag(j, s + kAhead);
     }
+    static_for<0, W>([&](auto wc) __attribute__((always_inline)) {
+      constexpr int f0 = s * W, w = decltype(wc)::value;
 #pragma unroll
-    for (int w = 0; w < W; ++w) {
-      constexpr int f0 = s * W;
-#pragma unroll
-      for (int j = 0; j < 3; ++j) mma<P>(ring[(f0 + w) % D][0], bq[s % QN][j], acc[0][j]);
+      for (int j = 0; j < 3; ++j) mma<P>(ring[(f0 + w) % D][0], bq[s % QN][j], w > 0 ? low[0][j] : acc[0][j]);
       ring[(f0 + w) % D][0] = wl[f0 + w + D];  // (the tail over-reads the zero fragments behind the stream)
-    }
+    });
     interleave_step<3 * W, 3, W>();
     __builtin_amdgcn_sched_barrier(0);
   });
@@ -1457,12 +1466,12 @@ __global__ __launch_bounds__(256) void fused_pipe_kernel(const FwdParams prm) {
         int l1fast[3];
 #pragma unroll
         for (int j = 0; j < 3; ++j) l1fast[j] = l1base[j] - (kL1RowsHalf - 1) * h * kL1RowPitch * G::EB;
-        conv1_fast_pass<P>(smem, fast1_weights(b), r1, l1fast, a0);
+        conv1_fast_pass<P>(smem, fast1_weights(b), r1, l1fast, a0, a0);
       } else {
 #pragma unroll
         for (int j = 0; j < 3; ++j) a0[0][j] = b0[0];
         preload_ring<L1Pipe<P>::D, 1>(r1, layer_weights<P, 0>(packed, lane));
-        conv1_pass<P>(smem, layer_weights<P, 0>(packed, lane), r1, l1base, a0);
+        conv1_pass<P>(smem, layer_weights<P, 0>(packed, lane), r1, l1base, a0, a0);
       }
     }
     preload_flat<kRing>(r2, layer_weights<P, 1>(packed, lane));
@@ -1801,7 +1810,7 @@ __global__ __launch_bounds__(256) void fused_forward_kernel(const FwdParams prm)
     {
       f32x16 acc[1][3];
       init_acc(acc, tail + bias_offset(0), h);
-      conv1_pass<P>(smem, layer_weights<P, 0>(packed, lane), r1, l1base, acc);
+      conv1_pass<P>(smem, layer_weights<P, 0>(packed, lane), r1, l1base, acc, acc);
       preload_ring<kRing, 1>(r2, layer_weights<P, 1>(packed, lane));
       C6_MARK(2);
       finish_layer<P, 1>(smem, ci, h, acc, [&] {
@@ -1935,13 +1944,13 @@ template <class P> __device__ __forceinline__ void put_elem(unsigned char *dst, 
 
 // part 0: the weight itself (put_elem rounds it to the storage type); part 1 (WLO): what that
 // rounding drops, which put_elem rounds in turn
-template <class P> __device__ __forceinline__ float weight_part(float v, int part) {
+template <class P> __device__ __forceinline__ float weight_part(Scaled<P> v, int part) {
   if constexpr (P::EB == 4) {
     return v;
   } else {
     static_assert(P::WLO == 0 || P::ID != C6_PREC_F16, "the low part is defined for bf16 storage");
-    for (int i = 0; i < part; ++i) v -= __builtin_bit_cast(float, (unsigned)bits16<P>(v) << 16);
-    return v;
+    for (int i = 0; i < part; ++i) v -= __builtin_bit_cast(float, (unsigned)bits16<P>((float)v) << 16);
+    return (float)v;
   }
 }
 
@@ -1991,7 +2000,7 @@ template <class P> __global__ void pack_kernel(const PackParams all) {
         f32x4 t4;
         for (int e = 0; e < 4; ++e) {
           const float *w = prm.conv_w(0) + (size_t)((8 * q + 4 * h + e) * 3 + 2) * kK1 * kK1;
-          float sum = 0.0f;
+          Scaled<P> sum = 0;
           for (int ky = 0; ky < kK1; ++ky) {
             const int rr = r + ky - kK1 / 2;
             if (rr < 0 || rr >= kBoard) continue;
@@ -2000,7 +2009,7 @@ template <class P> __global__ void pack_kernel(const PackParams all) {
               if (cc >= 0 && cc < kBoard) sum += w[ky * kK1 + kx];
             }
           }
-          t4[e] = sum * act_scale<P>();
+          t4[e] = (float)act_scaled<P>(sum);
         }
         *reinterpret_cast<f32x4 *>(dst) = t4;
         return;
@@ -2012,7 +2021,7 @@ template <class P> __global__ void pack_kernel(const PackParams all) {
         const float *w = prm.conv_w(0);
         for (int e = 0; e < G::E; ++e) {
           const int kx = jj * G::E + e;
-          put_elem<P>(dst, e, weight_part<P>(kx < kK1 ? w[((m * 3 + h) * kK1 + ky) * kK1 + kx] * act_scale<P>() : 0.0f, part));
+          put_elem<P>(dst, e, weight_part<P>(act_scaled<P>(kx < kK1 ? w[((m * 3 + h) * kK1 + ky) * kK1 + kx] : 0.0f), part));
         }
         return;
       }
@@ -2073,8 +2082,8 @@ template <class P> __global__ void pack_kernel(const PackParams all) {
       const int ky = row / 3, ch = row - ky * 3;
       for (int e = 0; e < G::E; ++e) {
         const int kx = jj * G::E + e;
-        float v = 0.0f;
-        if (row < kK1 * 3 && kx < kK1) v = w[((co * 3 + ch) * kK1 + ky) * kK1 + kx] * act_scale<P>();
+        Scaled<P> v = 0;
+        if (row < kK1 * 3 && kx < kK1) v = act_scaled<P>(w[((co * 3 + ch) * kK1 + ky) * kK1 + kx]);
         put_elem<P>(dst, e, weight_part<P>(v, part));
       }
     } else {
@@ -2105,15 +2114,16 @@ template <class P> __global__ void pack_kernel(const PackParams all) {
   const int ti = (int)(gid - nfl);
   if (ti < G::TAIL_SW) {  // the sw[] words behind it are written by lo_scale_kernel
     float *tail = reinterpret_cast<float *>(prm.packed + G::TAIL_OFF);
+    constexpr float head_scale = P::WLO == 2 ? 1.0f : act_scale<P>();
     float v = 0.0f;
     if (ti < kBiasTotal) {
       int l = 0;
       while (ti >= bias_offset(l + 1)) ++l;
-      v = prm.conv_b(l) ? prm.conv_b(l)[ti - bias_offset(l)] * act_scale<P>() : 0.0f;
+      v = prm.conv_b(l) ? (float)act_scaled<P>(prm.conv_b(l)[ti - bias_offset(l)]) : 0.0f;
     } else if (ti < kBiasTotal + kHeadC) {
-      v = prm.pol_w[ti - kBiasTotal] / act_scale<P>();
+      v = prm.pol_w[ti - kBiasTotal] / head_scale;
     } else if (ti < kBiasTotal + 2 * kHeadC) {
-      v = prm.val_w ? prm.val_w[ti - kBiasTotal - kHeadC] / act_scale<P>() : 0.0f;
+      v = prm.val_w ? prm.val_w[ti - kBiasTotal - kHeadC] / head_scale : 0.0f;
     } else if (ti == kBiasTotal + 2 * kHeadC) {
       v = prm.pol_b ? prm.pol_b[0] : 0.0f;
     } else if (ti == kBiasTotal + 2 * kHeadC + 1) {

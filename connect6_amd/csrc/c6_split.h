@@ -5,20 +5,31 @@
 // lo = v - hi - mid (8 mantissa bits each, both differences exact).  A product is then nine products
 // of bf16 values, each exact in fp32; the six down to 2^-17 of the largest are accumulated in fp32,
 // the other three are below 2^-25 of it, less than the rounding of one fp32 addition.  Against the
-// fp32 instructions (157 TFLOP/s, 432 roundings of the running sum per output of the last layer) six
-// bf16 ones at sixteen times the rate take 3/8 of the time, with 54 roundings.
+// fp32 instructions (157 TFLOP/s) six bf16 ones at sixteen times the rate take 3/8 of the time.
+//
+// Two sums per output: the products of the two hi in one, the five small products in the other, added
+// up at the end.  The matrix instruction drops what lies some eight bits below the last of its sum, towards
+// minus infinity: with the small products in the large sum (324 instructions for the 864 products of the
+// last layer) that is a bias of 0.77, in units of 2^-24 of the sum's own size, the same in every square,
+// which the value head's mean over 361 squares keeps; apart, 0.02, and the scatter is 2.9 in place
+// of 7.5 (fp32 instructions: 0.03 and 8.9).  Over 64 networks with the reference's initialisation (PyTorch's)
+// the value's error against a 64-bit forward is 2.1e-10 (1.5e-9) rms, with fp32 instructions 3.9e-10
+// (2.0e-9), its mean per network 4e-11 (3.4e-10) against 2.3e-10 (5.1e-10), and the logits' relative error
+// 4.7e-7 (8e-8) against 1.4e-6 (2.0e-7).
 //
 // What bounds it: the matrix cores, 383 k cycles per board with the 1,890 MFMAs of the 3x3 layers
-// six times and the first layer's 207 three times (0/1 inputs are exact in one bf16 value).  The
+// six times and the first layer's 207 three times (0/1 inputs are exact in one bf16 value), of 548 k that a
+// board takes; then the epilogues, 98 cycles per output of a lane (one wave per SIMD issues an instruction
+// per 5 cycles or so), and in the layers of 96 outputs the second reading of the weights (split_conv).  The
 // activations of up to 64 channels lie in LDS as their three planes, split once when a layer writes
 // them; 96 channels only fit as fp32 (421 positions x 384 bytes are the CU's whole LDS), and the two
 // layers that read them split them in registers, 44 instructions for eight values, a few behind each
-// MFMA.
+// MFMA.  2,048 boards take 2.36 ms (4.35 with fp32 instructions; 2.15 with one sum).
 //
 // An infinity has no such parts (inf - inf): where the fp32 instructions carried one on, this gives NaN.
 //
-// As in the 16-bit modes all activations carry the factor -log2(e), so that SiLU is
-// u / (1 + 2^u).
+// As in the 16-bit modes all activations carry the factor -log2(e), so that SiLU is u / (1 + 2^u); it is
+// put in (and taken out behind the heads) with 64 bits, so that nothing is rounded twice for it.
 #pragma once
 
 namespace c6 {
@@ -51,18 +62,180 @@ __device__ __forceinline__ float split_silu(float u) {
   return u * fmaf(r, fmaf(-d, r, 1.0f), r);
 }
 
-// The next bf16 plane of a pair of values, which keep what it leaves out.
-__device__ __forceinline__ int split_take(float &a, float &b) {
+// The heads: sums over the channels, which carry -log2(e), and over all squares.  (In 64 bits, once per square
+// and once per board: one rounding each.)
+__device__ __forceinline__ float split_logit(float sum, float bias) {
+  return (float)((double)sum * (1.0 / kActScale64) + (double)bias);
+}
+__device__ __forceinline__ float split_value(float sum, float bias) {
+  return (float)tanh((double)sum * (1.0 / kActScale64 / kPix) + (double)bias);
+}
+
+// What rounding a pair of values to the bf16 pair `w` leaves out.
+__device__ __forceinline__ void split_drop(float &a, float &b, int w) {
 #pragma clang fp contract(off)
-  const int w = pack2<PrecBF16>(a, b);
   a -= __builtin_bit_cast(float, w << 16);
   b -= __builtin_bit_cast(float, w & (int)0xffff0000);
+}
+// The next bf16 plane of a pair of values, which keep what it leaves out.
+__device__ __forceinline__ int split_take(float &a, float &b) {
+  const int w = pack2<PrecBF16>(a, b);
+  split_drop(a, b, w);
   return w;
+}
+
+// Weight ring of a 3x3 layer: two k-steps of all cout tiles and planes.  A k-step of NT cout tiles and N
+// pixel tiles is 6 NT N MFMAs, 192 NT N cycles, and a slot is refilled behind its last use.
+template <int NT> constexpr int kSplitRing = NT == 3 ? 1 : 2;
+template <int L> using SplitWeights = v4i[kSplitRing<kCoutArr[L] / 32>][kCoutArr[L] / 32][3];
+
+template <int NT> __device__ __forceinline__ void split_preload(v4i (&ring)[kSplitRing<NT>][NT][3], const WFrags &wl) {
+#pragma unroll
+  for (int d = 0; d < kSplitRing<NT>; ++d)
+#pragma unroll
+    for (int t = 0; t < NT; ++t)
+#pragma unroll
+      for (int i = 0; i < 3; ++i) ring[d][t][i] = wl[(d * NT + t) * 3 + i];
+}
+
+// The contraction of 3x3 layer L for N pixel tiles from J0 on.  K runs over taps, then 16 channels at a
+// time; each k-step is 6 N MFMAs per cout tile: six products of each pixel tile.  The five small ones have
+// a sum of their own, low, and the large one adds to acc.  Behind each MFMA at most one LDS read of the
+// next k-step's activations, one weight load, and (96 input channels) a few instructions of their split.
+//   ring: the first k-steps on entry; at the end the first ones again (AGAIN) or those behind the layer's last
+template <int L, int J0, int N, bool AGAIN>
+__device__ __forceinline__ void split_conv_tiles(const unsigned char *smem, const WFrags &wl, const float *bias,
+                                                 SplitWeights<L> &ring, const int (&ci)[3], int h,
+                                                 f32x16 (&acc)[kCoutArr[L] / 32][3], f32x16 (&low)[kCoutArr[L] / 32][N]) {
+  constexpr int CIN = kCinArr[L], NT = kCoutArr[L] / 32, KC = CIN / 16, D = kSplitRing<NT>;
+  constexpr bool WIDE = CIN == 96;   // activations arrive as fp32
+  static_assert(KC % 2 == 0 && KC % D == 0, "double buffers must line up across taps");
+  int pb[N], xo[N];
+  auto set_tap = [&](int tap) __attribute__((always_inline)) {
+    const int ky = tap / 3, kx = tap - 3 * ky;
+#pragma unroll
+    for (int j = 0; j < N; ++j) {
+      const int pos = ci[J0 + j] + (ky - 1) * kPitch + (kx - 1);
+      pb[j] = pos * SplitGeo::PIXB;
+      xo[j] = (WIDE ? h << 5 : h << 4) ^ split_swz(pos);
+    }
+  };
+  v4i bq[2][N][3];         // planes of a k-step's activations, [parity][pixel tile][plane]
+  f32x4 raw[2][N][2];      // WIDE: the same as fp32, one k-step further ahead
+  // part i of pixel tile j of channels 16 c ...: a plane, or (WIDE) four of the eight channels
+  auto read = [&](int c, int par, int j, int i) __attribute__((always_inline)) {
+    if constexpr (WIDE) {
+      if (i < 2)
+        raw[par][j][i] = *reinterpret_cast<const f32x4 *>(smem + pb[j] + (c >> 1) * 128 + (xo[j] ^ ((c & 1) * 64 + i * 16)));
+    } else {
+      bq[par][j][i] = *reinterpret_cast<const v4i *>(smem + pb[j] + (xo[j] ^ (c * 32)) + i * SplitGeo::PLANEB);
+    }
+  };
+  float rest[2];
+  auto split_some = [&](int par, auto ac) __attribute__((always_inline)) {  // a quarter of a pair's split
+    constexpr int a = decltype(ac)::value, pair = a / 4, j = pair / 4, e = pair % 4;
+    if constexpr (a % 4 == 0) {
+      rest[0] = raw[par][j][e >> 1][(e & 1) * 2];
+      rest[1] = raw[par][j][e >> 1][(e & 1) * 2 + 1];
+      bq[par][j][0][e] = pack2<PrecBF16>(rest[0], rest[1]);
+    } else if constexpr (a % 4 == 1) {
+      split_drop(rest[0], rest[1], bq[par][j][0][e]);
+    } else if constexpr (a % 4 == 2) {
+      bq[par][j][1][e] = pack2<PrecBF16>(rest[0], rest[1]);
+    } else {
+      split_drop(rest[0], rest[1], bq[par][j][1][e]);
+      bq[par][j][2][e] = pack2<PrecBF16>(rest[0], rest[1]);
+    }
+  };
+  set_tap(0);
+#pragma unroll
+  for (int j = 0; j < N; ++j)
+#pragma unroll
+    for (int i = 0; i < 3; ++i) read(0, 0, j, i);
+  if constexpr (WIDE) {
+#pragma unroll
+    for (int j = 0; j < N; ++j)
+#pragma unroll
+      for (int i = 0; i < 2; ++i) read(1, 1, j, i);
+    static_for<0, 16 * N>([&](auto ac) __attribute__((always_inline)) { split_some(0, ac); });
+  }
+#pragma unroll
+  for (int t = 0; t < NT; ++t) {
+    f32x16 b[1];
+    load_bias_tiles(b, bias + 32 * t, h);
+#pragma unroll
+    for (int j = 0; j < N; ++j) {
+      acc[t][J0 + j] = b[0];
+#pragma unroll
+      for (int e = 0; e < 16; ++e) low[t][j][e] = 0.0f;
+    }
+  }
+  constexpr int AHEAD = WIDE ? 2 : 1;
+#pragma unroll 1
+  for (int tap = 0; tap < 9; ++tap) {
+    const WFrags wn = wl + (tap * KC + D) * NT * 3;
+    const WFrags wrap = wl + (AGAIN && tap == 8 ? (D - KC) * NT * 3 : (tap * KC + D) * NT * 3);
+    static_for<0, KC>([&](auto uc) __attribute__((always_inline)) {
+      constexpr int u = decltype(uc)::value, par = u & 1;
+      // (after the last tap this wraps to the first: harmless extra reads)
+      if constexpr (u + AHEAD == KC) set_tap(tap == 8 ? 0 : tap + 1);
+      static_for<0, NT * 6 * N>([&](auto gc) __attribute__((always_inline)) {
+        constexpr int g = decltype(gc)::value, t = g / (6 * N), m = (g % (6 * N)) / N, j = g % N;
+        constexpr int WP[6] = {0, 1, 2, 0, 1, 0}, AP[6] = {2, 1, 0, 1, 0, 0};
+        mma<PrecBF16>(ring[u % D][t][WP[m]], bq[par][j][AP[m]], m < 5 ? low[t][j] : acc[t][J0 + j]);
+        if constexpr (WIDE) {
+          // raw[par] was split during the k-step before: free for the k-step after next
+          if constexpr (g >= 1 && g < 1 + 2 * N) read((u + 2) % KC, par, (g - 1) / 2, (g - 1) % 2);
+          if constexpr (g < 16 * N) split_some(par ^ 1, gc);
+        } else {
+          if constexpr (g < 3 * N) read((u + 1) % KC, par ^ 1, g / 3, g % 3);
+        }
+        // a plane's fragment after its last use in the tile: 2 after product 2, 1 after 4, 0 after 5
+        constexpr int done = j == N - 1 ? (m == 2 ? 2 : (m == 4 ? 1 : (m == 5 ? 0 : -1))) : -1;
+        if constexpr (done >= 0) {
+          if constexpr (u + D >= KC) ring[u % D][t][done] = wrap[(u * NT + t) * 3 + done];
+          else ring[u % D][t][done] = wn[(u * NT + t) * 3 + done];
+        }
+        __builtin_amdgcn_sched_barrier(0);
+      });
+    });
+  }
+}
+// All pixel tiles.  With three cout tiles the third pixel tile goes first and the other two after it: the
+// sums of all three, 288 registers, are more than the 256 the instruction's accumulators live in (2,048 boards
+// 2.36 ms; cout tiles apart, where 96 input channels are split twice, 2.53; two sums per k-step, added up by
+// the vector unit, 3.23).  The first two are left in two sums each.
+template <int NT> using SplitLow = f32x16[NT][NT < 3 ? 3 : 2];
+template <int L>
+__device__ __forceinline__ void split_conv(const unsigned char *smem, const WFrags &wl, const float *bias,
+                                           SplitWeights<L> &ring, const int (&ci)[3], int h,
+                                           f32x16 (&acc)[kCoutArr[L] / 32][3], SplitLow<kCoutArr[L] / 32> &low) {
+  if constexpr (kCoutArr[L] == 96) {
+    f32x16 one[3][1];
+    split_conv_tiles<L, 2, 1, true>(smem, wl, bias, ring, ci, h, acc, one);
+#pragma unroll
+    for (int t = 0; t < 3; ++t) {
+#pragma unroll
+      for (int e = 0; e < 16; ++e) acc[t][2][e] += one[t][0][e];
+      asm volatile("" : "+v"(acc[t][2]));   // (kept out of the accumulators' registers, which the others fill)
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    split_conv_tiles<L, 0, 2, false>(smem, wl, bias, ring, ci, h, acc, low);
+#pragma unroll
+    for (int t = 0; t < 3; ++t) asm volatile("" : "+v"(acc[t][2]));
+  } else {
+    split_conv_tiles<L, 0, 3, false>(smem, wl, bias, ring, ci, h, acc, low);
+  }
+}
+template <int NT>
+__device__ __forceinline__ float split_total(const f32x16 (&acc)[NT][3], const SplitLow<NT> &low, int t, int j, int e) {
+  return NT < 3 || j < 2 ? acc[t][j][e] + low[t][j][e] : acc[t][j][e];
 }
 
 // SiLU and store of one layer's outputs in the form the next one reads.
 template <int NT, bool PLANES>
-__device__ __forceinline__ void split_store(unsigned char *smem, const int (&ci)[3], int h, const f32x16 (&acc)[NT][3]) {
+__device__ __forceinline__ void split_store(unsigned char *smem, const int (&ci)[3], int h, const f32x16 (&acc)[NT][3],
+                                            const SplitLow<NT> &low) {
 #pragma unroll
   for (int j = 0; j < 3; ++j) {
     int pos = ci[j];
@@ -74,7 +247,7 @@ __device__ __forceinline__ void split_store(unsigned char *smem, const int (&ci)
       for (int q = 0; q < 4; ++q) {
         float v[4];
 #pragma unroll
-        for (int e = 0; e < 4; ++e) v[e] = split_silu(acc[t][j][4 * q + e]);
+        for (int e = 0; e < 4; ++e) v[e] = split_silu(split_total<NT>(acc, low, t, j, 4 * q + e));
         if constexpr (PLANES) {
           unsigned char *p = smem + at + ((64 * t + 16 * q) ^ sw) + 8 * h;
 #pragma unroll
@@ -90,112 +263,6 @@ __device__ __forceinline__ void split_store(unsigned char *smem, const int (&ci)
   }
 }
 
-// Weight ring of a 3x3 layer: DEPTH k-steps of all cout tiles and planes.  A k-step of NT tiles is
-// 18 NT MFMAs, 576 NT cycles; a slot is refilled behind its last use, so depth 1 already asks 1,150
-// cycles ahead with three tiles.
-template <int L> struct SplitRing {
-  static constexpr int NT = kCoutArr[L] / 32, DEPTH = NT == 3 ? 1 : 2;
-};
-template <int L> using SplitWeights = v4i[SplitRing<L>::DEPTH][kCoutArr[L] / 32][3];
-
-template <int L> __device__ __forceinline__ void split_preload(SplitWeights<L> &ring, const WFrags &wl) {
-#pragma unroll
-  for (int d = 0; d < SplitRing<L>::DEPTH; ++d)
-#pragma unroll
-    for (int t = 0; t < SplitRing<L>::NT; ++t)
-#pragma unroll
-      for (int i = 0; i < 3; ++i) ring[d][t][i] = wl[(d * SplitRing<L>::NT + t) * 3 + i];
-}
-
-// The contraction of 3x3 layer L.  K runs over taps, then 16 channels at a time; each k-step is
-// 18 MFMAs per cout tile: six products (smallest first) of three pixel tiles.  Behind each MFMA at
-// most one LDS read of the next k-step's activations, one weight load, and (96 input channels) a few
-// instructions of their split.
-template <int L>
-__device__ __forceinline__ void split_conv(const unsigned char *smem, const WFrags &wl, SplitWeights<L> &ring,
-                                           const int (&ci)[3], int h, f32x16 (&acc)[kCoutArr[L] / 32][3]) {
-  constexpr int CIN = kCinArr[L], NT = kCoutArr[L] / 32, KC = CIN / 16, D = SplitRing<L>::DEPTH;
-  constexpr bool WIDE = CIN == 96;   // activations arrive as fp32
-  static_assert(KC % 2 == 0 && KC % D == 0, "double buffers must line up across taps");
-  int pb[3], xo[3];
-  auto set_tap = [&](int tap) __attribute__((always_inline)) {
-    const int ky = tap / 3, kx = tap - 3 * ky;
-#pragma unroll
-    for (int j = 0; j < 3; ++j) {
-      const int pos = ci[j] + (ky - 1) * kPitch + (kx - 1);
-      pb[j] = pos * SplitGeo::PIXB;
-      xo[j] = (WIDE ? h << 5 : h << 4) ^ split_swz(pos);
-    }
-  };
-  v4i bq[2][3][3];         // planes of a k-step's activations, [parity][pixel tile][plane]
-  f32x4 raw[2][3][2];      // WIDE: the same as fp32, one k-step further ahead
-  // part i of pixel tile j of channels 16 c ...: a plane, or (WIDE) four of the eight channels
-  auto read = [&](int c, int par, int j, int i) __attribute__((always_inline)) {
-    if constexpr (WIDE) {
-      if (i < 2)
-        raw[par][j][i] = *reinterpret_cast<const f32x4 *>(smem + pb[j] + (c >> 1) * 128 + (xo[j] ^ ((c & 1) * 64 + i * 16)));
-    } else {
-      bq[par][j][i] = *reinterpret_cast<const v4i *>(smem + pb[j] + (xo[j] ^ (c * 32)) + i * SplitGeo::PLANEB);
-    }
-  };
-  float rest[2];
-  auto split_a = [&](int par, int pair) __attribute__((always_inline)) {  // hi of the pair, and what it leaves
-    const int j = pair / 4, e = pair % 4;
-    rest[0] = raw[par][j][e >> 1][(e & 1) * 2];
-    rest[1] = raw[par][j][e >> 1][(e & 1) * 2 + 1];
-    bq[par][j][0][e] = split_take(rest[0], rest[1]);
-  };
-  auto split_b = [&](int par, int pair) __attribute__((always_inline)) {
-    const int j = pair / 4, e = pair % 4;
-    bq[par][j][1][e] = split_take(rest[0], rest[1]);
-    bq[par][j][2][e] = pack2<PrecBF16>(rest[0], rest[1]);
-  };
-  set_tap(0);
-#pragma unroll
-  for (int j = 0; j < 3; ++j)
-#pragma unroll
-    for (int i = 0; i < 3; ++i) read(0, 0, j, i);
-  if constexpr (WIDE) {
-#pragma unroll
-    for (int j = 0; j < 3; ++j)
-#pragma unroll
-      for (int i = 0; i < 2; ++i) read(1, 1, j, i);
-#pragma unroll
-    for (int p = 0; p < 12; ++p) {
-      split_a(0, p);
-      split_b(0, p);
-    }
-  }
-  constexpr int AHEAD = WIDE ? 2 : 1;
-#pragma unroll 1
-  for (int tap = 0; tap < 9; ++tap) {
-    const WFrags wn = wl + (tap * KC + D) * NT * 3;
-    static_for<0, KC>([&](auto uc) __attribute__((always_inline)) {
-      constexpr int u = decltype(uc)::value, par = u & 1;
-      // (after the last tap this wraps to the first: harmless extra reads)
-      if constexpr (u + AHEAD == KC) set_tap(tap == 8 ? 0 : tap + 1);
-      static_for<0, NT * 18>([&](auto gc) __attribute__((always_inline)) {
-        constexpr int g = decltype(gc)::value, t = g / 18, m = (g % 18) / 3, j = g % 3;
-        constexpr int WP[6] = {0, 1, 2, 0, 1, 0}, AP[6] = {2, 1, 0, 1, 0, 0};
-        mma<PrecBF16>(ring[u % D][t][WP[m]], bq[par][j][AP[m]], acc[t][j]);
-        if constexpr (WIDE) {
-          // raw[par] was split during the k-step before: free for the k-step after next
-          if constexpr (g >= 1 && g < 7) read((u + 2) % KC, par, (g - 1) / 2, (g - 1) % 2);
-          if constexpr (g % 4 == 0 && g / 4 < 12) split_a(par ^ 1, g / 4);
-          if constexpr (g % 4 == 2 && g / 4 < 12) split_b(par ^ 1, g / 4);
-        } else {
-          if constexpr (g < 9) read((u + 1) % KC, par ^ 1, g / 3, g % 3);
-        }
-        // a plane's fragment after its last use in the tile: 2 after product 2, 1 after 4, 0 after 5
-        if constexpr (j == 2 && m == 2) ring[u % D][t][2] = wn[(u * NT + t) * 3 + 2];
-        if constexpr (j == 2 && m == 4) ring[u % D][t][1] = wn[(u * NT + t) * 3 + 1];
-        if constexpr (j == 2 && m == 5) ring[u % D][t][0] = wn[(u * NT + t) * 3];
-        __builtin_amdgcn_sched_barrier(0);
-      });
-    });
-  }
-}
-
 // one 3x3 layer that is not the last
 template <int L>
 __device__ __forceinline__ void split_layer(unsigned char *smem, const unsigned char *packed, const float *tail,
@@ -203,12 +270,12 @@ __device__ __forceinline__ void split_layer(unsigned char *smem, const unsigned 
                                             int lane) {
   constexpr int NT = kCoutArr[L] / 32;
   f32x16 acc[NT][3];
-  init_acc(acc, tail + bias_offset(L), h);
-  split_conv<L>(smem, layer_weights<PrecF32S, L>(packed, lane), ring, ci, h, acc);
+  SplitLow<NT> low;
+  split_conv<L>(smem, layer_weights<PrecF32S, L>(packed, lane), tail + bias_offset(L), ring, ci, h, acc, low);
   // (with equal widths the over-read has left the next layer's first k-steps in the ring)
-  if constexpr (kCoutArr[L + 1] != kCoutArr[L]) split_preload<L + 1>(next, layer_weights<PrecF32S, L + 1>(packed, lane));
+  if constexpr (kCoutArr[L + 1] != kCoutArr[L]) split_preload(next, layer_weights<PrecF32S, L + 1>(packed, lane));
   __syncthreads();  // every wave has finished reading the layer's input
-  split_store<NT, kCinArr[L + 1] != 96>(smem, ci, h, acc);
+  split_store<NT, kCinArr[L + 1] != 96>(smem, ci, h, acc, low);
   __syncthreads();
 }
 
@@ -374,6 +441,11 @@ __global__ __launch_bounds__(256) void split_forward_kernel(const FwdParams prm)
 #pragma unroll
       for (int ch = 0; ch < 3; ++ch) left[r][ch] = xin[r][ch];
     SplitWeights<1> r2;
+    f32x16 low[1][3], first[1][3];   // small products; the large ones, once all parts but the first follow
+#pragma unroll
+    for (int j = 0; j < 3; ++j)
+#pragma unroll
+      for (int i = 0; i < 16; ++i) low[0][j][i] = first[0][j][i] = 0.0f;
 #pragma unroll 1
     for (int part = 0; part < parts; ++part) {
       if (part > 0) __syncthreads();  // everybody has read the part before
@@ -408,15 +480,33 @@ __global__ __launch_bounds__(256) void split_forward_kernel(const FwdParams prm)
         for (int j = 0; j < 3; ++j) l1fast[j] = l1base[j] - (kL1RowsHalf - 1) * h * kL1RowPitch * G::EB;
         const WFrags wf = packed_frags<P>(packed, lane, G::FAST1_OFF);
         if (part > 0) preload_ring<L1Pipe<P>::D, 1>(r1, wf);
-        conv1_fast_pass<P>(smem, wf, r1, l1fast, a0);
+        conv1_fast_pass<P>(smem, wf, r1, l1fast, a0, low);
       } else {
         preload_ring<L1Pipe<P>::D, 1>(r1, layer_weights<P, 0>(packed, lane));
-        conv1_pass<P>(smem, layer_weights<P, 0>(packed, lane), r1, l1base, a0);
+        conv1_pass<P>(smem, layer_weights<P, 0>(packed, lane), r1, l1base, a0, low);
       }
+      if (parts > 1 && part == 0) {
+#pragma unroll
+        for (int j = 0; j < 3; ++j) {
+          first[0][j] = a0[0][j];
+          a0[0][j] = low[0][j];
+#pragma unroll
+          for (int i = 0; i < 16; ++i) low[0][j][i] = 0.0f;
+        }
+      }
+    }
+    if (parts > 1) {
+#pragma unroll
+      for (int j = 0; j < 3; ++j)
+#pragma unroll
+        for (int i = 0; i < 16; ++i) {
+          low[0][j][i] += a0[0][j][i];
+          a0[0][j][i] = first[0][j][i];
+        }
     }
     const long long bn = b + 1;
     if (bn < b_end) fetch_board(bn);  // lands while this board is computed
-    split_preload<1>(r2, layer_weights<P, 1>(packed, lane));
+    split_preload(r2, layer_weights<P, 1>(packed, lane));
     __syncthreads();
     // the copies overlapped the activation tile: restore its zero padding
     for (int i = tidv; i < 60 * (S::PIXB / 16); i += THREADS) {
@@ -424,7 +514,7 @@ __global__ __launch_bounds__(256) void split_forward_kernel(const FwdParams prm)
       const int pos = k < 20 ? k : (k < 41 ? 400 + (k - 20) : (k - 40) * kPitch);
       *reinterpret_cast<v4i *>(smem + pos * S::PIXB + w16 * 16) = v4i{0, 0, 0, 0};
     }
-    split_store<1, true>(smem, ci, h, a0);
+    split_store<1, true>(smem, ci, h, a0, low);
     __syncthreads();
 
     SplitWeights<2> r345;
@@ -439,8 +529,8 @@ __global__ __launch_bounds__(256) void split_forward_kernel(const FwdParams prm)
     // ---- layer 8 + both 1x1 heads straight from the fp32 accumulators ----
     {
       f32x16 acc[3][3];
-      init_acc(acc, tail + bias_offset(7), h);
-      split_conv<7>(smem, layer_weights<P, 7>(packed, lane), r678, ci, h, acc);
+      SplitLow<3> low8;
+      split_conv<7>(smem, layer_weights<P, 7>(packed, lane), tail + bias_offset(7), r678, ci, h, acc, low8);
       const float *valw = tail + kBiasTotal + kHeadC;
       const float *pwl = tail + kBiasTotal + 4 * h;  // per-lane base: channel 32t + 8q + 4h + e
       asm volatile("" : "+v"(pwl));
@@ -465,7 +555,7 @@ __global__ __launch_bounds__(256) void split_forward_kernel(const FwdParams prm)
           for (int j = 0; j < 3; ++j)
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
-              const float a = split_silu(acc[t][j][4 * q + e]);
+              const float a = split_silu(split_total<3>(acc, low8, t, j, 4 * q + e));
               pol[j] = fmaf(a, pw[e], pol[j]);
               val[j] = fmaf(a, vw[e], val[j]);
             }
@@ -484,9 +574,9 @@ __global__ __launch_bounds__(256) void split_forward_kernel(const FwdParams prm)
       const float polb = valw[kHeadC], valb = valw[kHeadC + 1];
 #pragma unroll
       for (int j = 0; j < 3; ++j)
-        if (h == 0 && valid[j]) lgt[pix[j]] = tot[j] + polb;
+        if (h == 0 && valid[j]) lgt[pix[j]] = split_logit(tot[j], polb);
       __syncthreads();
-      if (tid == 0 && prm.value != nullptr) prm.value[b] = tanhf(split_value_sum(red) * (1.0f / kPix) + valb);
+      if (tid == 0 && prm.value != nullptr) prm.value[b] = split_value(split_value_sum(red), valb);
     }
     // ---- write out: masked logits, optional sampled action ----
     if (prm.logits != nullptr) {

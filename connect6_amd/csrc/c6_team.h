@@ -174,6 +174,13 @@ __device__ __forceinline__ void team_conv(const unsigned char *smem, const unsig
     for (int p = 0; p < PT; ++p)
 #pragma unroll
       for (int i = 0; i < NPL; ++i) a[v][p][i] = frag(0, v, p, i);
+  f32x16 low[PT][TT];   // NPL == 3: the small products (split_conv_set)
+#pragma unroll
+  for (int p = 0; p < PT; ++p)
+#pragma unroll
+    for (int t = 0; t < TT; ++t)
+#pragma unroll
+      for (int e = 0; e < 16; ++e) low[p][t][e] = 0.0f;
   auto round = [&](int r) __attribute__((always_inline)) {
     // (the low-order pass comes in front of the last phase, as in pipe_layer)
     if constexpr (LO) {
@@ -194,7 +201,7 @@ __device__ __forceinline__ void team_conv(const unsigned char *smem, const unsig
 #pragma unroll
           for (int p = 0; p < PT; ++p)
 #pragma unroll
-            for (int m = 0; m < 6; ++m) mma<P>(ring[v % D][t][WP[m]], a[v % 3][p][AP[m]], acc[p][t]);
+            for (int m = 0; m < 6; ++m) mma<P>(ring[v % D][t][WP[m]], a[v % 3][p][AP[m]], m < 5 ? low[p][t] : acc[p][t]);
         } else {
 #pragma unroll
           for (int i = 0; i < W; ++i)
@@ -215,6 +222,14 @@ __device__ __forceinline__ void team_conv(const unsigned char *smem, const unsig
   } else {
 #pragma unroll 1
     for (int r = 0; r < KS / U; ++r) round(r);
+  }
+  if constexpr (NPL == 3) {
+#pragma unroll
+    for (int p = 0; p < PT; ++p)
+#pragma unroll
+      for (int t = 0; t < TT; ++t)
+#pragma unroll
+        for (int e = 0; e < 16; ++e) acc[p][t][e] += low[p][t][e];
   }
 }
 
@@ -687,6 +702,9 @@ __device__ __forceinline__ void team_board(const TeamParams &prm, unsigned char 
 #pragma unroll
       for (int i = 0; i < 16; ++i) acc[0][i] = plane2_varies ? b0[0][i] : fmaf(c2, acc[0][i], b0[0][i]);
     }
+    f32x16 low, large;   // SPLIT: small products; the large ones, once all parts but the first follow
+#pragma unroll
+    for (int i = 0; i < 16; ++i) low[i] = large[i] = 0.0f;
 #pragma unroll 1
     for (int part = 0; part < parts; ++part) {
       if (part > 0) __syncthreads();
@@ -725,8 +743,10 @@ __device__ __forceinline__ void team_board(const TeamParams &prm, unsigned char 
         auto multiply = [&](int s4) __attribute__((always_inline)) {
 #pragma unroll
           for (int i = 0; i < 3; ++i)
-#pragma unroll
-            for (int j = 0; j < W; ++j) mma<P>(w[s4][i][j], a[s4][i], acc[0]);
+            static_for<0, W>([&](auto jc) __attribute__((always_inline)) {
+              constexpr int j = decltype(jc)::value;
+              mma<P>(w[s4][i][j], a[s4][i], T::SPLIT && j > 0 ? low : acc[0]);
+            });
           __builtin_amdgcn_sched_barrier(0);
         };
 #pragma unroll
@@ -743,7 +763,19 @@ __device__ __forceinline__ void team_board(const TeamParams &prm, unsigned char 
 #pragma unroll
         for (int s4 = 0; s4 < 3; ++s4)
           if (row + s4 < rows) multiply(s4);
+        if constexpr (T::SPLIT) {
+          if (parts > 1 && part == 0) {
+            large = acc[0];
+            acc[0] = low;
+#pragma unroll
+            for (int i = 0; i < 16; ++i) low[i] = 0.0f;
+          }
+        }
       }
+    }
+    if constexpr (T::SPLIT) {
+#pragma unroll
+      for (int i = 0; i < 16; ++i) acc[0][i] = parts > 1 ? large[i] + (low[i] + acc[0][i]) : acc[0][i] + low[i];
     }
     C6_MARK(2);
     __syncthreads();   // the copies give way to the activations
@@ -769,7 +801,8 @@ __device__ __forceinline__ void team_board(const TeamParams &prm, unsigned char 
     for (int p = tid; p < kPix; p += THREADS) {
       float z = partial(T::HEAD_OFF + p * 4);
       if constexpr (T::SPLIT) z = (z + partial(T::HEAD_OFF + (384 + p) * 4)) + partial(T::HEAD_OFF + (768 + p) * 4);
-      z += polb;
+      if constexpr (T::SPLIT) z = split_logit(z, polb);
+      else z += polb;
       bool taken;
       if (f.mask_mode == C6_MASK_LEGAL) {
         taken = f.legal[(size_t)b * kPix + p] == 0;
@@ -812,14 +845,14 @@ __device__ __forceinline__ void team_board(const TeamParams &prm, unsigned char 
     }
     __syncthreads();
     if (tid == 0 && f.value != nullptr) {
-      float s = 0.0f;
       if constexpr (T::SPLIT) {
-        s = split_value_sum(red);
+        f.value[b] = split_value(split_value_sum(red), valb);
       } else {
+        float s = 0.0f;
 #pragma unroll
         for (int w = 0; w < 4; ++w) s += red[w];
+        f.value[b] = tanhf(s * (1.0f / kPix) + valb);
       }
-      f.value[b] = tanhf(s * (1.0f / kPix) + valb);
     }
     if (f.actions != nullptr && wave == 0) {
       int a;

@@ -43,10 +43,41 @@ def test_no_further_from_float64_than_fp32(cuda, kind, init):
         for prec in (_lib.PREC_F32, _lib.PREC_F32S):
             lg, vg, _, _ = run_forward(x.to(cuda), model.packed_weights(prec), prec, 1, 33)
             err[prec] = (rel_l2(lg.double().cpu(), l64), rel_l2(vg.double().cpu(), v64))
-    # Eight layers of fp32 sums: each of the two results is within a few 2^-24 per layer of float64;
-    # the value, a mean that nearly cancels, scatters more (twice the other's error plus 1e-6).
-    assert err[_lib.PREC_F32S][0] <= 1.5 * err[_lib.PREC_F32][0] + 1e-7, err
-    assert err[_lib.PREC_F32S][1] <= 2 * err[_lib.PREC_F32][1] + 1e-6, err
+    # Eight layers of fp32 sums: each of the two results is within a few 2^-24 per layer of float64
+    # (logits 0.3 to 0.55 of the other's error); the value, a mean that nearly cancels, scatters over 33
+    # boards of one network (over many networks: the test below).
+    assert err[_lib.PREC_F32S][0] <= err[_lib.PREC_F32][0], err
+    assert err[_lib.PREC_F32S][1] <= err[_lib.PREC_F32][1] + 1e-6, err
+
+
+@pytest.mark.parametrize("init", ["reference", "torch_default"])
+def test_value_and_logits_of_many_networks(cuda, init):
+    """Against a float64 forward no larger an error than the fp32 instructions', neither in size nor in its
+    mean over a network's boards (what rounds the same way in every square stays in the value, a mean over
+    them)."""
+    nets, boards = 64, 12
+    err = {p: {"value": [], "logits": []} for p in (_lib.PREC_F32, _lib.PREC_F32S)}
+    for s in range(nets):
+        st = R.init_state(1000 + s, init)
+        model = c6.PolicyValueNet().to(cuda).eval()
+        model.load_state_dict(st)
+        x, _ = gen_boards(boards, 200, 5000 + s)
+        l64, v64 = R.forward({k: v.double() for k, v in st.items()}, x.double())
+        xd = x.to(cuda)
+        with torch.inference_mode():
+            for prec, e in err.items():
+                lg, vg, _, _ = run_forward(xd, model.packed_weights(prec), prec, 1, boards)
+                e["value"].append(vg.double().cpu() - v64)
+                e["logits"].append((lg.double().cpu() - l64) / l64.pow(2).mean().sqrt())
+            one, v1 = model(xd[s % boards: s % boards + 1])   # (a board on its own: the same bits)
+            assert torch.equal(one[0], lg[s % boards]) and torch.equal(v1[0], vg[s % boards])
+    # Measured, this against the fp32 instructions: value 0.53 (PyTorch's initialisation 0.77) of the error and
+    # 0.2 (0.7) of its mean per network, logits 0.33 (0.40).
+    was, now = [{k: torch.stack(v) for k, v in err[p].items()} for p in (_lib.PREC_F32, _lib.PREC_F32S)]
+    for name, of in (("value", lambda e: e["value"]), ("mean of the value's", lambda e: e["value"].mean(1)),
+                     ("logits", lambda e: e["logits"])):
+        a, b = of(was).pow(2).mean().sqrt(), of(now).pow(2).mean().sqrt()
+        assert b <= a, (name, float(a), float(b))
 
 
 def test_fp32_batches_draws_masks_and_states(cuda):

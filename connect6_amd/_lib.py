@@ -134,7 +134,7 @@ _HOST_SO = _LIBDIR / "_c6_host.so"
 _HOST_ABI = ("c6_forward", "c6_forward_cascade", "c6_forward_boards", "c6_forward_boards_cascade",
              "c6_cascade_workspace_bytes", "c6_mask_logits", "c6_softmax_sample", "c6_env_step", "c6_canonical_input",
              "c6_forward_generic_packed", "c6_team_bytes", "c6_forward_team", "c6_forward_boards_team",
-             "c6_stream_capturing", "c6_forward_cascade_team", "c6_forward_boards_cascade_team")
+             "c6_stream_capturing", "c6_forward_cascade_team", "c6_forward_boards_cascade_team", "c6_generic_pack")
 
 
 def build_host() -> Path:

@@ -39,6 +39,7 @@ struct Abi {
   decltype(&c6_stream_capturing) stream_capturing;
   decltype(&c6_forward_cascade_team) forward_cascade_team;
   decltype(&c6_forward_boards_cascade_team) forward_boards_cascade_team;
+  decltype(&c6_generic_pack) generic_pack;
 } abi;
 
 PyObject *fail(PyObject *type, const std::string &what) {
@@ -346,45 +347,146 @@ PyObject *forward_boards(PyObject *, PyObject *const *a, Py_ssize_t n) {
   END_HANDLE_TH_ERRORS
 }
 
+// A tensor of a module by the path of its name ("convs", "3", "weight"), as state_dict() finds it: null where
+// there is none (no Python error set).
+const at::Tensor *module_tensor(PyObject *module, std::initializer_list<const char *> path) {
+  static PyObject *dict_name = PyUnicode_InternFromString("__dict__");
+  const at::Tensor *found = nullptr;
+  PyObject *at = module;   // (borrowed: the module above holds it)
+  for (size_t i = 0; i < path.size() && at != nullptr; ++i) {
+    PyObject *dict = PyObject_GetAttr(at, dict_name);
+    at = nullptr;
+    if (dict == nullptr) break;
+    const char *name = path.begin()[i];
+    const bool last = i + 1 == path.size();
+    for (const char *kind : {last ? "_parameters" : "_modules", "_buffers"}) {
+      PyObject *of = PyDict_GetItemString(dict, kind);
+      PyObject *v = of != nullptr && PyDict_Check(of) ? PyDict_GetItemString(of, name) : nullptr;
+      if (v == nullptr || v == Py_None) continue;
+      if (!last) at = v;
+      else if (THPVariable_Check(v)) found = &THPVariable_Unpack(v);
+      break;
+    }
+    Py_DECREF(dict);
+  }
+  PyErr_Clear();
+  return found;
+}
+
+struct GenericCall {
+  at::Tensor x, legal, logits, value;
+  int x_code = -1, layers = 0, prec = 0, mask_mode = 0;
+  const int *kernels = nullptr, *channels = nullptr;
+  int64_t b = 0, board = 0;
+  float fill = 0.0f;
+  void *stream = nullptr;
+};
+// arguments x, architecture, precision, want_value, mask_mode, legal, fill, stream; the outputs
+bool generic_call(GenericCall &c, PyObject *x, PyObject *arch_bytes, PyObject *prec, PyObject *want_value,
+                  PyObject *mask_mode, PyObject *legal, PyObject *fill, PyObject *stream) {
+  c.x = tensor(x).contiguous();
+  char *arch = nullptr;
+  Py_ssize_t bytes = 0;
+  if (PyBytes_AsStringAndSize(arch_bytes, &arch, &bytes) != 0) return false;
+  c.layers = (int)(bytes / (2 * sizeof(int)));
+  c.kernels = reinterpret_cast<const int *>(arch);
+  c.channels = c.kernels + c.layers;
+  c.prec = (int)PyLong_AsLong(prec);
+  c.mask_mode = (int)PyLong_AsLong(mask_mode);
+  c.fill = (float)PyFloat_AsDouble(fill);
+  c.stream = PyLong_AsVoidPtr(stream);
+  const at::Tensor *legal_in = tensor_or_null(legal);
+  if (PyErr_Occurred()) return false;
+  const at::Device dev = c.x.device();
+  c.b = c.x.size(0);
+  c.board = c.x.size(3);
+  c.x_code = dtype_code(c.x.scalar_type());
+  if (c.x_code < 0) {
+    fail(PyExc_ValueError, std::string("unsupported tensor dtype ") + c10::toString(c.x.scalar_type()) +
+                               "; expected float32, bfloat16 or float16");
+    return false;
+  }
+  if (legal_in != nullptr) {
+    if (legal_in->dim() != 2 || legal_in->size(0) != c.b || legal_in->size(1) != c.board * c.board) {
+      fail(PyExc_ValueError, "legal mask must have shape (" + std::to_string(c.b) + ", " +
+                                 std::to_string(c.board * c.board) + "), got " + shape_text(*legal_in));
+      return false;
+    }
+    c.legal = legal_in->to(dev).contiguous();
+  }
+  const c10::DeviceGuard guard(dev);
+  c.logits = fresh({c.b, c.board * c.board}, at::kFloat, dev);
+  if (PyObject_IsTrue(want_value) == 1) c.value = fresh({c.b}, at::kFloat, dev);
+  return true;
+}
+int generic_launch(const GenericCall &c, const at::Tensor &packed, int64_t groups) {
+  return abi.forward_generic_packed(
+      c.x.data_ptr(), c.x_code, groups, c.b / groups, (int)c.board, c.layers, c.kernels, c.channels, packed.data_ptr(),
+      (size_t)(packed.numel() / groups), c.prec, ptr<float>(c.logits), ptr<float>(c.value), c.mask_mode,
+      static_cast<const uint8_t *>(c.legal.defined() ? c.legal.data_ptr() : nullptr), c.fill, c.stream);
+}
+
 // forward_generic(x, packed, groups, architecture, prec, want_value, mask_mode, legal, fill, stream)
 //   -> (rc, logits, value).  architecture: bytes of the C ints kernels[layers], channels[layers]
 PyObject *forward_generic(PyObject *, PyObject *const *a, Py_ssize_t n) {
   if (n != 10) return fail(PyExc_TypeError, "forward_generic takes 10 arguments");
   HANDLE_TH_ERRORS
-  const at::Tensor x = tensor(a[0]).contiguous();
   const at::Tensor &packed = tensor(a[1]);
   const int64_t groups = PyLong_AsLongLong(a[2]);
-  char *arch = nullptr;
-  Py_ssize_t arch_bytes = 0;
-  if (PyBytes_AsStringAndSize(a[3], &arch, &arch_bytes) != 0) return nullptr;
-  const int layers = (int)(arch_bytes / (2 * sizeof(int)));
-  const int *kernels = reinterpret_cast<const int *>(arch), *channels = kernels + layers;
-  const int prec = (int)PyLong_AsLong(a[4]), mask_mode = (int)PyLong_AsLong(a[6]);
-  const at::Tensor *legal_in = tensor_or_null(a[7]);
-  const float fill = (float)PyFloat_AsDouble(a[8]);
-  void *stream = PyLong_AsVoidPtr(a[9]);
   if (PyErr_Occurred()) return nullptr;
-  const at::Device dev = x.device();
-  const int64_t b = x.size(0), board = x.size(3);
-  const int x_code = dtype_code(x.scalar_type());
-  if (x_code < 0)
-    return fail(PyExc_ValueError, std::string("unsupported tensor dtype ") + c10::toString(x.scalar_type()) +
-                                      "; expected float32, bfloat16 or float16");
-  at::Tensor legal, value;
-  if (legal_in != nullptr) {
-    if (legal_in->dim() != 2 || legal_in->size(0) != b || legal_in->size(1) != board * board)
-      return fail(PyExc_ValueError, "legal mask must have shape (" + std::to_string(b) + ", " +
-                                        std::to_string(board * board) + "), got " + shape_text(*legal_in));
-    legal = legal_in->to(dev).contiguous();
-  }
+  GenericCall c;
+  if (!generic_call(c, a[0], a[3], a[4], a[5], a[6], a[7], a[8], a[9])) return nullptr;
+  const c10::DeviceGuard guard(c.x.device());
+  return answer<2>(generic_launch(c, packed, groups), {c.logits, c.value});
+  END_HANDLE_TH_ERRORS
+}
+
+// forward_generic_module(module, x, packed bytes, architecture, prec, mask_mode, legal, fill, stream)
+//   -> (rc, logits, value).  The module's parameters as they are now, packed by a launch in front of the
+//   forward's: an edit that no version counter shows (p.data) counts, as it does where a layer reads them.
+PyObject *forward_generic_module(PyObject *, PyObject *const *a, Py_ssize_t n) {
+  if (n != 9) return fail(PyExc_TypeError, "forward_generic_module takes 9 arguments");
+  HANDLE_TH_ERRORS
+  const int64_t bytes = PyLong_AsLongLong(a[2]);
+  if (PyErr_Occurred()) return nullptr;
+  GenericCall c;
+  if (!generic_call(c, a[1], a[3], a[4], Py_True, a[5], a[6], a[7], a[8])) return nullptr;
+  const at::Device dev = c.x.device();
   const c10::DeviceGuard guard(dev);
-  const at::Tensor logits = fresh({b, board * board}, at::kFloat, dev);
-  if (PyObject_IsTrue(a[5]) == 1) value = fresh({b}, at::kFloat, dev);
-  const int rc = abi.forward_generic_packed(
-      x.data_ptr(), x_code, groups, b / groups, (int)board, layers, kernels, channels, packed.data_ptr(),
-      (size_t)(packed.numel() / groups), prec, ptr<float>(logits), ptr<float>(value), mask_mode,
-      static_cast<const uint8_t *>(legal.defined() ? legal.data_ptr() : nullptr), fill, stream);
-  return answer<2>(rc, {logits, value});
+  std::vector<at::Tensor> keep;   // (copies, where a parameter is not fp32, contiguous and on the device)
+  bool ok = true;
+  const auto take = [&](std::initializer_list<const char *> path, int64_t count, bool required) -> const float * {
+    const at::Tensor *t = ok ? module_tensor(a[0], path) : nullptr;
+    std::string name;
+    for (const char *part : path) name += (name.empty() ? "" : ".") + std::string(part);
+    if (t == nullptr) {
+      if (ok && required) ok = fail(PyExc_KeyError, "missing parameter " + name) != nullptr;
+      return nullptr;
+    }
+    if (t->numel() != count) {
+      ok = fail(PyExc_ValueError, name + " has " + std::to_string(t->numel()) + " elements, the network's layers need " +
+                                      std::to_string(count)) != nullptr;
+      return nullptr;
+    }
+    keep.push_back(t->detach().to(dev, at::kFloat).contiguous());
+    return ptr<float>(keep.back());
+  };
+  std::vector<const float *> w((size_t)c.layers), bias((size_t)c.layers);
+  int64_t cin = 3;
+  for (int l = 0; l < c.layers; ++l) {
+    const std::string at = std::to_string(l);
+    w[(size_t)l] = take({"convs", at.c_str(), "weight"}, cin * c.channels[l] * c.kernels[l] * c.kernels[l], true);
+    bias[(size_t)l] = take({"convs", at.c_str(), "bias"}, c.channels[l], false);
+    cin = c.channels[l];
+  }
+  const float *pol_w = take({"policy_output", "weight"}, cin, true), *pol_b = take({"policy_output", "bias"}, 1, false);
+  const float *val_w = take({"value_output", "weight"}, cin, false), *val_b = take({"value_output", "bias"}, 1, false);
+  if (!ok) return nullptr;
+  const at::Tensor packed = fresh({bytes}, at::kByte, dev);
+  int rc = abi.generic_pack(1, (int)c.board, c.layers, c.kernels, c.channels, w.data(), bias.data(), pol_w, pol_b, val_w,
+                            val_b, c.prec, packed.data_ptr(), (size_t)bytes, c.stream);
+  if (rc == C6_OK) rc = generic_launch(c, packed, 1);
+  return answer<2>(rc, {c.logits, c.value});
   END_HANDLE_TH_ERRORS
 }
 
@@ -492,7 +594,7 @@ PyObject *bind(PyObject *, PyObject *const *a, Py_ssize_t n) {
 #define C6_FAST(name) {#name, reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)(void)>(name)), METH_FASTCALL, nullptr}
 PyMethodDef methods[] = {C6_FAST(bind),        C6_FAST(forward),        C6_FAST(forward_boards),
                          C6_FAST(mask_logits), C6_FAST(sample),         C6_FAST(env_step),
-                         C6_FAST(canonical_input), C6_FAST(forward_generic),
+                         C6_FAST(canonical_input), C6_FAST(forward_generic), C6_FAST(forward_generic_module),
                          {"parameters", parameters, METH_O, nullptr},
                          {nullptr, nullptr, 0, nullptr}};
 PyModuleDef module_def = {PyModuleDef_HEAD_INIT, "_c6_host", nullptr, -1, methods, nullptr, nullptr, nullptr, nullptr};

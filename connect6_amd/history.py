@@ -115,8 +115,7 @@ class HistoricalPolicyEnsemble:
         self.action_size = self.board_size * self.board_size
 
         self._prec = _PREC_OF_DTYPE[self.dtype] if precision is None else _lib.PREC_BY_NAME[precision]
-        self._arch: bytes | None = None     # other architectures: see _fits
-        self._has_packed = False
+        self._plan: tuple | None = None     # other architectures: see _fits
         self._packed: dict[int, tuple] = {}   # mode: (buffer, stream it was packed on, event)
         self._states = states
         self._stacked: dict[str, torch.Tensor | None] = {}
@@ -178,11 +177,11 @@ class HistoricalPolicyEnsemble:
 
     def _fits(self) -> bool:
         """Does this (non-default) architecture have a packed form?"""
-        if self._arch is None:
-            self._arch = architecture_bytes(self.kernels, self.channels)
-            self._has_packed = self.num_models <= 65535 and _lib.generic_packed_bytes(
-                self.board_size, self.kernels, self.channels, self._prec) > 0
-        return self._has_packed
+        shape = (self.board_size, self.kernels, self.channels)
+        if self._plan is None or self._plan[0] != shape:
+            fits = self.num_models <= 65535 and _lib.generic_packed_bytes(*shape, self._prec) > 0
+            self._plan = (shape, architecture_bytes(self.kernels, self.channels), fits)
+        return self._plan[2]
 
     def _packed_weights(self, prec: int | None = None) -> torch.Tensor:
         prec = self._prec if prec is None else prec
@@ -238,7 +237,7 @@ class HistoricalPolicyEnsemble:
             flat = x.reshape(m * t, *expected_tail)
             packed = self._packed_weights() if self._fits() else None
             if packed is not None:
-                logits, _ = run_packed_generic(flat, packed, self._arch, self._prec, groups=m, want_value=False)
+                logits, _ = run_packed_generic(flat, packed, self._plan[1], self._prec, groups=m, want_value=False)
             else:
                 if self._stacked32 is None:   # the layer-by-layer kernels read fp32 parameters
                     self._stacked32 = {k: v.float().contiguous() for k, v in self._stacked_state().items()

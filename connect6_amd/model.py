@@ -322,8 +322,6 @@ class PolicyValueNet(nn.Module):
             raise ValueError("channel counts must be positive")
         self.kernels = kernels
         self.channels = channels
-        self._default_architecture = (self.board_size == 19 and kernels == self.DEFAULT_KERNELS
-                                      and channels == self.DEFAULT_CHANNELS)
 
         convs = []
         cin = self.input_channels
@@ -341,8 +339,7 @@ class PolicyValueNet(nn.Module):
         self.cascade_threshold: float | None = None   # None: _lib.CASCADE_THRESHOLD
         self.cascade_stats: dict = {}                 # "second_pass": boards evaluated twice (last call)
         self._packed: dict[int, tuple] = {}
-        self._arch: bytes | None = None               # other architectures: see _generic
-        self._fits: dict[int, bool] = {}
+        self._plan: tuple | None = None               # other architectures: see _generic
         self._epoch = 0
         self.register_load_state_dict_post_hook(lambda module, _keys: module.refresh_weights())
 
@@ -364,7 +361,11 @@ class PolicyValueNet(nn.Module):
     # -- precision / weights ------------------------------------------------
     @property
     def is_default_architecture(self) -> bool:
-        return self._default_architecture
+        return (
+            self.board_size == 19
+            and self.kernels == self.DEFAULT_KERNELS
+            and self.channels == self.DEFAULT_CHANNELS
+        )
 
     def resolve_precision(self) -> int:
         if self.precision is not None:
@@ -410,11 +411,8 @@ class PolicyValueNet(nn.Module):
                 # memory could be handed out again while a forward here still reads it
                 buf.record_stream(stream)
             return buf
-        if self.is_default_architecture:
-            buf = torch.empty(_lib.packed_bytes(prec), dtype=torch.uint8, device=dev)
-            pack_state({k: v for k, v in self.state_dict().items()}, prec, buf)
-        else:
-            buf = pack_generic(self.state_dict(), self.board_size, self.kernels, self.channels, prec, dev)
+        buf = torch.empty(_lib.packed_bytes(prec), dtype=torch.uint8, device=dev)
+        pack_state({k: v for k, v in self.state_dict().items()}, prec, buf)
         done = torch.cuda.Event()
         done.record(torch.cuda.current_stream(dev))
         self._packed[prec] = (self._epoch, key, buf, stream_ptr, done)
@@ -440,19 +438,29 @@ class PolicyValueNet(nn.Module):
                 "sharing this state_dict)"
             )
 
-    def _generic(self, x, prec, **kw):
-        """Non-default architectures: one launch from packed weights where the network has that
-        form, else layer by layer (``c6_forward_generic``)."""
+    def _generic(self, x, prec, mask_mode=_lib.MASK_NONE, legal=None, fill=_FILL_LOWEST):
+        """Non-default architectures read their parameters on every call: packed by one launch and
+        evaluated by a second where the network has a packed form (3-6 us more than from a kept copy,
+        which an edit through ``p.data`` would leave behind), else layer by layer
+        (``c6_forward_generic``)."""
         if x.shape[0] == 0:
             return (torch.empty((0, self.action_size), dtype=torch.float32, device=x.device),
                     torch.empty((0,), dtype=torch.float32, device=x.device))
-        if self._arch is None:
-            self._arch = architecture_bytes(self.kernels, self.channels)
-            self._fits = {p: _lib.generic_packed_bytes(self.board_size, self.kernels, self.channels, p) > 0
-                          for p in _lib.PREC_BY_NAME.values()}
-        if self._fits[prec]:
-            return run_packed_generic(x, self.packed_weights(prec), self._arch, prec, **kw)
-        return run_forward_generic(x, self.state_dict(), self.kernels, self.channels, prec, **kw)
+        shape = (self.board_size, self.kernels, self.channels)
+        if self._plan is None or self._plan[0] != shape:
+            self._plan = (shape, architecture_bytes(self.kernels, self.channels), {})
+        _, arch, sizes = self._plan
+        size = sizes.get(prec)
+        if size is None:
+            size = sizes[prec] = _lib.generic_packed_bytes(*shape, prec)
+        if size == 0:
+            return run_forward_generic(x, self.state_dict(), self.kernels, self.channels, prec, mask_mode=mask_mode,
+                                       legal=legal, fill=fill)
+        rc, logits, value = _lib.host().forward_generic_module(self, x, size, arch, prec, mask_mode, legal, fill,
+                                                               _lib.stream_ptr(x.device))
+        if rc != 0:
+            _lib.check(rc, "c6_forward_generic_packed")
+        return logits, value
 
     def forward(self, x: torch.Tensor) -> tuple[torch.Tensor, torch.Tensor]:
         self._check_input(x)

@@ -81,3 +81,61 @@ def test_weight_sets_and_an_architecture_without_packed_form(cuda):
             lo, vo = R.forward(st, xb)
             lg, vg = model(xb.to(cuda))
         assert rel_l2(lg, lo) <= 5e-6 and rel_l2(vg, vo) <= 5e-6
+
+
+@pytest.mark.parametrize("precision", ["fp32", "bf16c", "fp16"])
+def test_parameters_are_read_on_every_call(cuda, precision):
+    """Edits that no version counter shows (an average of weights kept through ``p.data``), replaced parameters,
+    other types: what the module holds at the call is what answers."""
+    board, kernels, channels = 9, [5, 3, 3], [16, 32, 24]
+    model = c6.PolicyValueNet(board_size=board, kernels=kernels, channels=channels).to(cuda).eval()
+    model.load_state_dict(R.init_state(31, "torch_default", kernels=kernels, channels=channels))
+    model.precision = precision
+    x = _inputs(37, board, 5).to(cuda)
+
+    def check():
+        other = c6.PolicyValueNet(board_size=board, kernels=kernels, channels=channels).to(cuda).eval()
+        other.load_state_dict(model.state_dict())
+        other.precision = precision
+        with torch.inference_mode():
+            got, want = model(x), other(x)
+        assert torch.equal(got[0], want[0]) and torch.equal(got[1], want[1])
+        return got[0]
+
+    seen = [check()]
+    model.convs[1].weight.data.mul_(0.5)
+    seen.append(check())
+    model.policy_output.bias.data.add_(1.0)
+    seen.append(check())
+    model.convs[2].bias = torch.nn.Parameter(torch.ones(24, device=cuda))
+    seen.append(check())
+    for a, b in zip(seen, seen[1:]):
+        assert not torch.equal(a, b)
+    model.convs[1].weight = torch.nn.Parameter(model.convs[1].weight.detach().cpu().double())   # converted on the way
+    assert torch.equal(check(), seen[-1])
+    static = x.clone()                     # ... and in every replay of a graph
+    model.convs[1].to(cuda, torch.float32)
+    with torch.inference_mode():
+        model(static)
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph):
+            out, _ = model(static)
+        for factor in (1.0, 2.0, 0.25):
+            model.convs[1].weight.data.mul_(factor)
+            graph.replay()
+            torch.cuda.synchronize()
+            assert torch.equal(out, model(x)[0]), factor
+
+
+def test_board_size_set_after_construction(cuda):
+    """The network is fully convolutional: the same module on boards of another size."""
+    for kernels, channels, first, second in ((None, None, 19, 9), ([3, 3], [8, 16], 7, 13)):
+        model = c6.PolicyValueNet(board_size=first, kernels=kernels, channels=channels).to(cuda).eval()
+        for board in (first, second, first):
+            model.board_size, model.action_size = board, board * board
+            assert model.is_default_architecture == (kernels is None and board == 19)
+            x = _inputs(3, board, 2)
+            with torch.inference_mode():
+                lo, vo = R.forward({k: v.cpu() for k, v in model.state_dict().items()}, x)
+                lg, vg = model(x.to(cuda))
+            assert rel_l2(lg, lo) <= 1e-5 and rel_l2(vg, vo) <= 1e-4

@@ -374,3 +374,27 @@ def test_native_host_side_refuses_what_is_no_tensor():
     ):
         with pytest.raises(TypeError, match="expected a tensor"):
             call()
+
+
+def test_native_host_side_checks_a_modules_parameters():
+    from connect6_amd.model import architecture_bytes
+
+    net = c6.PolicyValueNet(board_size=5, kernels=[3, 1], channels=[8, 4])
+    arch, x = architecture_bytes(net.kernels, net.channels), torch.zeros(2, 3, 5, 5)
+
+    def call():
+        return _lib.host().forward_generic_module(net, x, 4096, arch, _lib.PREC_F32, 0, None, 0.0, 0)
+
+    kept = net.convs[1].weight
+    net.convs[1].weight = torch.nn.Parameter(torch.zeros(4, 8, 3, 3))
+    with pytest.raises(ValueError, match="convs.1.weight has 288 elements"):
+        call()
+    del net.convs[1].weight
+    with pytest.raises(KeyError, match="missing parameter convs.1.weight"):
+        call()
+    net.convs[1].weight = kept
+    del net.policy_output
+    with pytest.raises(KeyError, match="missing parameter policy_output.weight"):
+        call()
+    with pytest.raises(TypeError, match="expected a tensor"):
+        _lib.host().forward_generic_module(net, None, 4096, arch, _lib.PREC_F32, 0, None, 0.0, 0)

@@ -11,7 +11,10 @@
 // values (8 + 8 + 8 mantissa bits: hi = bf16(v), mid = bf16(v - hi), lo = v - hi - mid), so a
 // product of two is nine products of bf16 values, each exact in fp32.  The six down to 2^-17 of the
 // largest are accumulated in fp32; the other three are below 2^-25 of it, under the rounding of one
-// fp32 addition.  Six bf16 instructions take 3/8 of the time of the fp32 ones (2.5 PFLOP/s / 6
+// fp32 addition.  The five small ones have a sum of their own, which the matrix instruction would
+// otherwise cut off towards minus infinity (c6_split.h): over seven architectures the error against a 64-bit
+// forward is 0.3 to 0.7 of that of a chain of fp32 multiply-adds in the logits, 0.5 to 1 in the value (with one
+// sum up to 1.4, and 2.6 in its mean over a network's boards).  Six bf16 instructions take 3/8 of the time of the fp32 ones (2.5 PFLOP/s / 6
 // against 157 TFLOP/s), and the planes need 6 bytes of LDS per value.
 #include "c6_common.h"
 #include "c6_device.h"
@@ -148,6 +151,13 @@ __device__ __forceinline__ void small_contract(const unsigned char *smem, const 
 #pragma unroll
       for (int i = 0; i < NA; ++i) a[s][j][i] = *reinterpret_cast<const v4i *>(smem + base[j] + off + i * planeb);
   };
+  // Operands in several planes: the small products have a sum of their own (the instruction drops what lies
+  // some eight bits below the last of its sum, towards minus infinity; see c6_split.h)
+  f32x4 low[PT][CT];
+#pragma unroll
+  for (int j = 0; j < PT; ++j)
+#pragma unroll
+    for (int t = 0; t < CT; ++t) low[j][t] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
   auto multiply = [&](int s) __attribute__((always_inline)) {
     // smallest products first
 #pragma unroll
@@ -158,7 +168,10 @@ __device__ __forceinline__ void small_contract(const unsigned char *smem, const 
 #pragma unroll
         for (int t = 0; t < CT; ++t)
 #pragma unroll
-          for (int j = 0; j < PT; ++j) acc[j][t] = small_mma<A>(w[s][t][i], a[s][j][d - i], acc[j][t]);
+          for (int j = 0; j < PT; ++j) {
+            f32x4 &sum = d > 0 ? low[j][t] : acc[j][t];
+            sum = small_mma<A>(w[s][t][i], a[s][j][d - i], sum);
+          }
       }
   };
   fetch(0, 0);
@@ -171,6 +184,12 @@ __device__ __forceinline__ void small_contract(const unsigned char *smem, const 
     multiply(1);
   }
   if (c < chunks) multiply(0);
+  if constexpr (NA > 1 || NW > 1) {
+#pragma unroll
+    for (int j = 0; j < PT; ++j)
+#pragma unroll
+      for (int t = 0; t < CT; ++t) acc[j][t] += low[j][t];
+  }
 }
 
 // u / (1 + e^-u) to fp32 accuracy with the hardware's exp2 and reciprocal: the product u * log2(e)
@@ -194,8 +213,8 @@ __device__ __forceinline__ float small_silu(float u) {
 // their padding columns), so that a (tap, block of eight channels) is a constant offset, looked up
 // in a table by the lane group that contracts it.
 //
-// Measured on 1024 boards of the 9x9 network above, fp32: 23 us a call (914 us layer by layer), of
-// which the six-product MFMAs alone are 7 us; the rest is the two waves per SIMD meeting at two
+// Measured on 1024 boards of the 9x9 network above, fp32: 26 us (914 us layer by layer; 24 with one
+// sum), of which the six-product MFMAs alone are 7 us; the rest is the two waves per SIMD meeting at two
 // barriers per layer, the staging of the input and the launch.
 template <class A, int PT, bool RAW>
 __global__ __launch_bounds__(64 * kSmallMaxWaves) void small_net_kernel(const SmallParams prm) {
@@ -404,7 +423,7 @@ __global__ __launch_bounds__(64 * kSmallMaxWaves) void small_net_kernel(const Sm
       float v = 0.0f;
       for (int s = lane; s < nn; s += 64) v += s_val[b * nn + s];
       v = wave_sum(v);
-      if (lane == 0) prm.value[b0 + b] = tanhf(v / (float)nn + val_b);
+      if (lane == 0) prm.value[b0 + b] = (float)tanh((double)v / nn + (double)val_b);   // (one rounding)
     }
   }
 }

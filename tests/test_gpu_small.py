@@ -7,6 +7,7 @@ import torch
 import connect6_amd as c6
 from connect6_amd import _lib
 from connect6_amd.model import pack_generic, run_forward_generic, run_packed_generic, architecture_bytes
+from connect6_amd.synthetic import gen_boards
 from oracle import torch_ref as R
 from tests.util import rel_l2
 
@@ -55,6 +56,59 @@ def test_fits_and_matches_the_oracle(cuda, board, kernels, channels, batch):
             # bf16: the emulation's roundings in another order of summation (a few fall the other way);
             # fp16: half an ulp (2^-12) at every operand of two to four layers
             assert rel_l2(lb, want) <= tol, (name, rel_l2(lb, want))
+
+
+def _fp32_chain(st, x, layers):
+    """The forward with every output one chain of fp32 multiply-adds, as fp32 arithmetic gives it (products exact,
+    each sum rounded once): float64 operations, rounded."""
+    import torch.nn.functional as F
+
+    a = x
+    for i in range(layers):
+        w, b = st[f"convs.{i}.weight"], st[f"convs.{i}.bias"]
+        k = w.shape[2]
+        cols = F.unfold(a.double(), k, padding=k // 2)
+        acc = b.view(1, -1, 1).expand(x.shape[0], -1, cols.shape[2])
+        for j, col in enumerate(cols.unbind(1)):
+            acc = (acc.double() + w.flatten(1)[:, j].double().view(1, -1, 1) * col.unsqueeze(1)).float()
+        a = F.silu(acc).view(x.shape[0], -1, *x.shape[2:])
+    f = a.flatten(2)
+    heads = []
+    for name in ("policy_output", "value_output"):
+        acc = st[f"{name}.bias"].view(1, 1).expand(x.shape[0], f.shape[2]) if name == "policy_output" else torch.zeros_like(f[:, 0])
+        for c in range(f.shape[1]):
+            acc = (acc.double() + st[f"{name}.weight"].flatten()[c].double() * f[:, c].double()).float()
+        heads.append(acc)
+    return heads[0], torch.tanh(heads[1].mean(1) + st["value_output.bias"])
+
+
+@pytest.mark.parametrize("init", ["reference", "torch_default"])
+@pytest.mark.parametrize("board,kernels,channels", [(9, [5, 3, 3], [16, 32, 32]), (13, [7, 5, 5, 5, 5], [32] * 5)])
+def test_no_further_from_float64_than_fp32(cuda, board, kernels, channels, init):
+    nets, boards = 16, 16
+    err = {"here": [], "chain": []}
+    for s in range(nets):
+        st = R.init_state(300 + s, init, kernels=kernels, channels=channels)
+        model = c6.PolicyValueNet(board_size=board, kernels=kernels, channels=channels).to(cuda).eval()
+        model.load_state_dict(st)
+        x, _ = gen_boards(boards, board * board // 2, 900 + s, board_size=board)
+        l64, v64 = R.forward({k: v.double() for k, v in st.items()}, x.double())
+        with torch.inference_mode():
+            outs = {"here": model(x.to(cuda)),
+                    "chain": _fp32_chain({k: v.to(cuda) for k, v in st.items()}, x.to(cuda), len(kernels))}
+        for name, (l, v) in outs.items():
+            err[name].append(((l.double().cpu() - l64) / l64.pow(2).mean().sqrt(), v.double().cpu() - v64))
+    logits, value = [{n: torch.stack([e[i] for e in es]) for n, es in err.items()} for i in (0, 1)]
+
+    def rms(t):
+        return float(t.pow(2).mean().sqrt())
+    # Measured against the layer-by-layer kernel, a chain as above: logits 0.3 to 0.5 of its error, the value 0.5
+    # and its mean over a network's boards 0.25 to 0.5.  (PyTorch's initialisation makes the value so large that
+    # rounding it once is most of either error, and its mean one of sixteen roundings.)
+    assert rms(logits["here"]) <= 0.75 * rms(logits["chain"])
+    assert rms(value["here"]) <= rms(value["chain"])
+    if init == "reference":
+        assert rms(value["here"].mean(1)) <= rms(value["chain"].mean(1))
 
 
 def test_weight_sets_and_an_architecture_without_packed_form(cuda):

@@ -13,6 +13,24 @@ template <class T> __device__ __forceinline__ void stream_store(T *p, const T &v
   __builtin_nontemporal_store(v, p);
 }
 
+// ---- fp32 operands as sums of three bf16 values ----
+// The bf16 value nearest to v; a finite v beyond the largest one rounds to that and not to an infinity.
+__device__ __forceinline__ unsigned short bf16_part(float v) {
+  constexpr float kLargest = 0x1.fep127f;
+  const float c = __builtin_fabsf(v) < __builtin_inff() ? __builtin_amdgcn_fmed3f(v, -kLargest, kLargest) : v;
+  return __builtin_bit_cast(unsigned short, (__bf16)c);
+}
+// What is left of v behind a part (nothing of an infinity or NaN, which the first part holds).
+template <class T> __device__ __forceinline__ T bf16_rest(T v, unsigned short part) {
+  return (part & 0x7f80) == 0x7f80 ? T(0) : v - __builtin_bit_cast(float, (unsigned)part << 16);
+}
+// An output from its two sums: large products, small ones.  Where an infinity went through it, the first one has
+// what fp32 arithmetic gives, and the parts of a finite factor may have made a NaN of the second.
+__device__ __forceinline__ float two_sums(float large, float small) {
+  const float s = large + small;
+  return s == s ? s : large;
+}
+
 // Wave64 all-reduce without LDS traffic: DPP inside a row of 16 lanes (quad swaps, then the
 // mirrored lane of the 8- and the 16-group, which belongs to the half not yet combined), then
 // v_permlane16_swap / v_permlane32_swap across rows.  Every lane ends with the result.

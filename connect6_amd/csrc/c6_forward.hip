@@ -1949,6 +1949,10 @@ template <class P> __device__ __forceinline__ float weight_part(Scaled<P> v, int
     return v;
   } else {
     static_assert(P::WLO == 0 || P::ID != C6_PREC_F16, "the low part is defined for bf16 storage");
+    if constexpr (P::WLO == 2) {
+      for (int i = 0; i < part; ++i) v = bf16_rest(v, bf16_part((float)v));
+      return __builtin_bit_cast(float, (unsigned)bf16_part((float)v) << 16);
+    }
     for (int i = 0; i < part; ++i) v -= __builtin_bit_cast(float, (unsigned)bits16<P>((float)v) << 16);
     return (float)v;
   }

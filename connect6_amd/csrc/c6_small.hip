@@ -67,14 +67,20 @@ template <int NA_, int NW_, bool F16_> struct SmallArith {
   static constexpr bool F16 = F16_;
 };
 
-template <class A> __device__ __forceinline__ void small_planes(float v, unsigned short (&p)[A::NA]) {
+// ANY: a parameter or an input, which may be infinite or beyond the largest bf16 value
+template <class A, bool ANY = false> __device__ __forceinline__ void small_planes(float v, unsigned short (&p)[A::NA]) {
   if constexpr (A::F16) {
     p[0] = __builtin_bit_cast(unsigned short, (_Float16)v);
   } else {
 #pragma unroll
     for (int i = 0; i < A::NA; ++i) {
-      p[i] = __builtin_bit_cast(unsigned short, (__bf16)v);
-      v -= __builtin_bit_cast(float, (unsigned)p[i] << 16);
+      if constexpr (ANY && A::NA > 1) {
+        p[i] = bf16_part(v);
+        v = bf16_rest(v, p[i]);
+      } else {
+        p[i] = __builtin_bit_cast(unsigned short, (__bf16)v);
+        v -= __builtin_bit_cast(float, (unsigned)p[i] << 16);
+      }
     }
   }
 }
@@ -122,7 +128,7 @@ template <class A> struct RawWeights {
       for (int i = 0; i < 8; ++i) {
         const bool in = row && ci0 + i < cin;
         const float v = w[in ? (size_t)(co * cin + ci0 + i) * kk + tap : 0];
-        small_planes<SmallArith<A::NW, A::NW, A::F16>>(in ? v : 0.0f, pl[i]);
+        small_planes<SmallArith<A::NW, A::NW, A::F16>, true>(in ? v : 0.0f, pl[i]);
       }
 #pragma unroll
       for (int p = 0; p < A::NW; ++p)
@@ -188,7 +194,9 @@ __device__ __forceinline__ void small_contract(const unsigned char *smem, const 
 #pragma unroll
     for (int j = 0; j < PT; ++j)
 #pragma unroll
-      for (int t = 0; t < CT; ++t) acc[j][t] += low[j][t];
+      for (int t = 0; t < CT; ++t)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) acc[j][t][e] = two_sums(acc[j][t][e], low[j][t][e]);
   }
 }
 
@@ -263,7 +271,7 @@ __global__ __launch_bounds__(64 * kSmallMaxWaves) void small_net_kernel(const Sm
 #pragma unroll
         for (int ch = 0; ch < 3; ++ch) {
           unsigned short pl[NA];
-          small_planes<A>(small_load(prm.x, prm.x_dtype, ((size_t)(b0 + b) * 3 + ch) * nn + s), pl);
+          small_planes<A, true>(small_load(prm.x, prm.x_dtype, ((size_t)(b0 + b) * 3 + ch) * nn + s), pl);
 #pragma unroll
           for (int i = 0; i < NA; ++i) *reinterpret_cast<unsigned short *>(at + i * L.planeb + 2 * ch) = pl[i];
         }
@@ -459,7 +467,7 @@ template <class A> __global__ void small_pack_kernel(const SmallPack prm) {
       const int ci = 8 * cb + k;
       const bool in = e < L.blocks && co < L.cout && ci < L.cin;
       const float v = in ? w[((size_t)co * L.cin + ci) * L.k * L.k + tap] : 0.0f;
-      small_planes<SmallArith<A::NW, A::NW, A::F16>>(v, pl[k]);
+      small_planes<SmallArith<A::NW, A::NW, A::F16>, true>(v, pl[k]);
     }
     for (int p = 0; p < A::NW; ++p) {
       v4i o;

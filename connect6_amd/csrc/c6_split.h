@@ -26,7 +26,11 @@
 // layers that read them split them in registers, 44 instructions for eight values, a few behind each
 // MFMA.  2,048 boards take 2.36 ms (4.35 with fp32 instructions; 2.15 with one sum).
 //
-// An infinity has no such parts (inf - inf): where the fp32 instructions carried one on, this gives NaN.
+// An infinity is its own first part; what is left of it is a NaN in the sum of the small products, and the
+// large ones alone, which are then infinite or NaN as in fp32 arithmetic, are the result (two_sums; with that
+// 2,048 boards take 2.37 ms in place of 2.36).  Parameters and inputs have three parts up to the end of fp32;
+// a sum or an activation has them up to 2.3e38 (3.39e38, the largest bf16 value, with its factor of 1.44) and
+// counts as infinite beyond.
 //
 // As in the 16-bit modes all activations carry the factor -log2(e), so that SiLU is u / (1 + 2^u); it is
 // put in (and taken out behind the heads) with 64 bits, so that nothing is rounded twice for it.
@@ -53,13 +57,13 @@ struct SplitGeo {
 // 16-byte granule XOR of a position: sixteen consecutive positions read sixteen bank groups
 __device__ __forceinline__ int split_swz(int pos) { return ((pos >> 1) & 7) << 4; }
 
-// u / (1 + 2^u), the reciprocal with one Newton step.  (Clamped where 1 + 2^u leaves fp32: the
-// result is then below 2^-126 |u|.)
+// u / (1 + 2^u), the reciprocal with one Newton step.  (Where 1 + 2^u nears the end of fp32 or leaves it the
+// reciprocal is 0 or on its way there, and the step, with the denominator held at 2^126, at most doubles it.)
 __device__ __forceinline__ float split_silu(float u) {
 #pragma clang fp contract(off)   // (the product is rounded before its parts are taken)
-  const float d = fminf(1.0f + __builtin_amdgcn_exp2f(u), 0x1p126f);
+  const float d = 1.0f + __builtin_amdgcn_exp2f(u);
   const float r = __builtin_amdgcn_rcpf(d);
-  return u * fmaf(r, fmaf(-d, r, 1.0f), r);
+  return u * fmaf(r, fmaf(-fminf(d, 0x1p126f), r, 1.0f), r);
 }
 
 // The heads: sums over the channels, which carry -log2(e), and over all squares.  (In 64 bits, once per square
@@ -216,7 +220,7 @@ __device__ __forceinline__ void split_conv(const unsigned char *smem, const WFra
 #pragma unroll
     for (int t = 0; t < 3; ++t) {
 #pragma unroll
-      for (int e = 0; e < 16; ++e) acc[t][2][e] += one[t][0][e];
+      for (int e = 0; e < 16; ++e) acc[t][2][e] = two_sums(acc[t][2][e], one[t][0][e]);
       asm volatile("" : "+v"(acc[t][2]));   // (kept out of the accumulators' registers, which the others fill)
       __builtin_amdgcn_sched_barrier(0);
     }
@@ -229,7 +233,7 @@ __device__ __forceinline__ void split_conv(const unsigned char *smem, const WFra
 }
 template <int NT>
 __device__ __forceinline__ float split_total(const f32x16 (&acc)[NT][3], const SplitLow<NT> &low, int t, int j, int e) {
-  return NT < 3 || j < 2 ? acc[t][j][e] + low[t][j][e] : acc[t][j][e];
+  return NT < 3 || j < 2 ? two_sums(acc[t][j][e], low[t][j][e]) : acc[t][j][e];
 }
 
 // SiLU and store of one layer's outputs in the form the next one reads.
@@ -462,8 +466,8 @@ __global__ __launch_bounds__(256) void split_forward_kernel(const FwdParams prm)
 #pragma unroll
           for (int ch = 0; ch < 3; ++ch) {
             if (ch >= planes_staged) break;
-            const unsigned short v16 = bits16<P>(left[r][ch]);
-            left[r][ch] -= __builtin_bit_cast(float, (unsigned)v16 << 16);
+            const unsigned short v16 = bf16_part(left[r][ch]);
+            left[r][ch] = bf16_rest(left[r][ch], v16);
             const int hrow = (row + kK1 / 2) * 3 + ch;
 #pragma unroll
             for (int s = 0; s < G::E; ++s) {

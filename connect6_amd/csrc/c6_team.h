@@ -229,7 +229,7 @@ __device__ __forceinline__ void team_conv(const unsigned char *smem, const unsig
 #pragma unroll
       for (int t = 0; t < TT; ++t)
 #pragma unroll
-        for (int e = 0; e < 16; ++e) acc[p][t][e] += low[p][t][e];
+        for (int e = 0; e < 16; ++e) acc[p][t][e] = two_sums(acc[p][t][e], low[p][t][e]);
   }
 }
 
@@ -717,8 +717,13 @@ __device__ __forceinline__ void team_board(const TeamParams &prm, unsigned char 
           if (ch >= (plane2_varies ? 3 : 2)) break;
           const int hrow = (row + kK1 / 2) * 3 + ch;
           if (sq >= kPix) continue;
-          const unsigned short v16 = bits16<P>(xin[k][ch]);
-          if constexpr (T::SPLIT) xin[k][ch] -= __builtin_bit_cast(float, (unsigned)v16 << 16);
+          unsigned short v16;
+          if constexpr (T::SPLIT) {
+            v16 = bf16_part(xin[k][ch]);
+            xin[k][ch] = bf16_rest(xin[k][ch], v16);
+          } else {
+            v16 = bits16<P>(xin[k][ch]);
+          }
           if (hrow < ha || hrow >= hb) continue;
 #pragma unroll
           for (int q = 0; q < G::E; ++q)
@@ -775,7 +780,7 @@ __device__ __forceinline__ void team_board(const TeamParams &prm, unsigned char 
     }
     if constexpr (T::SPLIT) {
 #pragma unroll
-      for (int i = 0; i < 16; ++i) acc[0][i] = parts > 1 ? large[i] + (low[i] + acc[0][i]) : acc[0][i] + low[i];
+      for (int i = 0; i < 16; ++i) acc[0][i] = parts > 1 ? two_sums(large[i], low[i] + acc[0][i]) : two_sums(acc[0][i], low[i]);
     }
     C6_MARK(2);
     __syncthreads();   // the copies give way to the activations

@@ -48,9 +48,13 @@ extern "C" {
                             twice the bf16 matrix work): within 3e-4 relative L2 of fp32 */
 
 #define C6_PREC_F32S 7   /* fp32 operands, each the exact sum of three bf16 values: six bf16 MFMAs per
-                            product, fp32 accumulate.  fp32 results (the products left out are
-                            below 2^-25) at half the time of C6_PREC_F32; its packed weights take
-                            three halves of that mode's */
+                            product, fp32 accumulate.  fp32 results, no further from a 64-bit
+                            forward than those of C6_PREC_F32 (the products left out are below
+                            2^-25), at half the time; its packed weights take three halves of that
+                            mode's.  Infinities and NaN as in fp32, except that a sum or an
+                            activation beyond 2.3e38 (fp32: 3.4e38) counts as infinite.  In an
+                            architecture that c6_generic_packed_bytes is not 0 for, C6_PREC_F32
+                            too is computed so, with sums and activations up to 3.38e38 */
 
 /* element types of caller tensors */
 #define C6_DT_F32 0

@@ -193,3 +193,29 @@ def test_board_size_set_after_construction(cuda):
                 lo, vo = R.forward({k: v.cpu() for k, v in model.state_dict().items()}, x)
                 lg, vg = model(x.to(cuda))
             assert rel_l2(lg, lo) <= 1e-5 and rel_l2(vg, vo) <= 1e-4
+
+
+@pytest.mark.parametrize("where,index,value", [
+    ("x", (1, 0, 4, 4), float("inf")), ("x", (1, 0, 4, 4), float("nan")), ("x", (1, 0, 4, 4), 3.4e38), ("x", (1, 2), -3.39e38),
+    ("convs.2.weight", (5, 3, 1, 1), float("inf")), ("convs.0.weight", (3, 0, 2, 2), 3.38e38), ("convs.0.bias", 5, -1e34),
+    ("convs.1.bias", 5, -3.4e38), ("convs.1.bias", 5, 3.38e38), ("convs.1.bias", 5, float("inf")),
+    ("convs.2.bias", 5, -float("inf")), ("convs.2.bias", 5, 3.4e38)])
+def test_infinities_and_the_ends_of_the_range_as_in_fp32(cuda, where, index, value):
+    kernels, channels = [5, 3, 3], [16, 32, 32]
+    st = R.init_state(31, "torch_default", kernels=kernels, channels=channels)
+    x = _inputs(3, 9, 5)
+    (x if where == "x" else st[where])[index] = value
+    model = c6.PolicyValueNet(board_size=9, kernels=kernels, channels=channels).to(cuda).eval()
+    model.load_state_dict(st)
+    dev = {k: v.to(cuda) for k, v in st.items()}
+    with torch.inference_mode():
+        want = _fp32_chain(dev, x.to(cuda), 3)
+        got = model(x.to(cuda))
+    for a, b in zip(want, got):
+        a, b = a.double().cpu(), b.double().cpu()
+        assert torch.equal(a.isnan(), b.isnan())
+        ends = a.isinf() | b.isinf()
+        assert torch.equal(a[ends], b[ends])
+        fine = a.isfinite()
+        size = a.where(fine, torch.zeros_like(a)).abs().flatten(1).amax(1, keepdim=True) if a.ndim > 1 else a.abs()
+        assert bool(((a - b).abs()[fine] <= (2e-5 * size).expand_as(a)[fine]).all())

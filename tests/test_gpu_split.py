@@ -80,6 +80,45 @@ def test_value_and_logits_of_many_networks(cuda, init):
         assert b <= a, (name, float(a), float(b))
 
 
+_INF, _NAN = float("inf"), float("nan")
+_EXTREMES = [  # (where, index, value); "x": board 1 of three
+    ("x", (1, 0, 9, 9), _INF), ("x", (1, 1, 0, 0), -_INF), ("x", (1, 0, 3, 3), _NAN), ("x", (1, 2), _INF),
+    ("x", (1, 0, 9, 9), 3.4e38), ("x", (1, 2), -1e38), ("x", (1, 2, 4, 4), 3.39e38), ("x", (1, 0, 5, 7), 1.7e-30),
+    ("convs.0.weight", (3, 0, 11, 11), _INF), ("convs.0.weight", (3, 0, 11, 11), 1e38),
+    ("convs.3.weight", (3, 0, 1, 1), -_INF), ("convs.7.weight", (5, 3, 1, 1), _INF),
+    ("convs.7.weight", (5, 3, 1, 1), -_INF), ("convs.7.weight", (5, 3, 1, 1), 3.4e38),
+    ("convs.0.bias", 5, -1e34), ("convs.3.bias", 5, -2e38), ("convs.6.bias", 5, 2e36), ("convs.6.bias", 5, _INF),
+    ("convs.7.bias", 5, _INF), ("convs.7.bias", 5, -_INF), ("convs.7.bias", 5, -2.3e38), ("convs.7.bias", 5, _NAN),
+    ("policy_output.weight", (0, 5, 0, 0), _INF), ("policy_output.bias", 0, -_INF),
+    ("value_output.weight", (0, 5, 0, 0), _NAN), ("value_output.bias", 0, -_INF),
+]
+
+
+@pytest.mark.parametrize("where,index,value", _EXTREMES)
+def test_infinities_and_the_ends_of_the_range_as_in_fp32(cuda, where, index, value):
+    """What the fp32 instructions make of an infinity, a NaN or a number near the end of fp32.  (Sums and activations
+    up to 2.3e38: they carry a factor of 1.44.)"""
+    st, x = R.init_state(5, "torch_default"), gen_boards(3, 200, 3)[0]
+    (x if where == "x" else st[where])[index] = value
+    model = c6.PolicyValueNet().to(cuda).eval()
+    model.load_state_dict(st)
+    xd = torch.cat([x] * 30).to(cuda)          # one workgroup per board; three boards: several
+    with torch.inference_mode():
+        want = run_forward(xd[:3], model.packed_weights(_lib.PREC_F32), _lib.PREC_F32, 1, 3)[:2]
+        packed = model.packed_weights(_lib.PREC_F32S)
+        for n in (3, 90):
+            got = run_forward(xd[:n], packed, _lib.PREC_F32S, 1, n)[:2]
+            for a, b in zip(want, got):
+                a, b = a.double().cpu(), b[:3].double().cpu()
+                assert torch.equal(a.isnan(), b.isnan()), n
+                ends = a.isinf() | b.isinf()
+                assert torch.equal(a[ends], b[ends]), n
+                fine = a.isfinite()
+                # (either's error is 1e-6 to 2e-6 of a board's logits as a whole; ten times that for the worst square)
+                size = a.where(fine, torch.zeros_like(a)).abs().flatten(1).amax(1, keepdim=True) if a.ndim > 1 else a.abs()
+                assert bool(((a - b).abs()[fine] <= (2e-5 * size).expand_as(a)[fine]).all()), n
+
+
 def test_fp32_batches_draws_masks_and_states(cuda):
     st = R.init_state(11, "reference")
     model = c6.PolicyValueNet().to(cuda).eval()

@@ -2362,16 +2362,12 @@ static TeamMode team_mode(int prec) {
 }
 static int second_mode(int cascade) { return cascade == C6_PREC_BF16C ? C6_PREC_BF16F6W : C6_PREC_BF16F6; }
 // The cascade's second pass hands what the listed boards leave beyond whole rounds of the CUs to teams, if it
-// is no more than they take (73 boards of 256 CUs with low weights, 42 without): 4,096 boards of which
-// 266 go twice take 1,039 us so, 1,119 with a second round for the rest (303 listed; three workgroups per
-// board: 1,086).  A launch that the teams cannot
-// serve costs 4 us, so it is
-// made where the number of listed boards may well be one: random networks with the reference's initialisation
-// list 6 %, give or take a sixth.
-static bool team_cascade(int prec, long long boards, int cus) {
-  const long long most = team_mode(second_mode(prec)).most(cus), low = boards / 20, high = boards / 14;
-  return low % cus <= most || low / cus != high / cus;
-}
+// is no more than they take (73 boards of 256 CUs with low weights, 42 without); their launch ends at once where
+// it is more.  How many are listed depends on the network (6 % of random ones' boards, a few of a peaked
+// policy's), not on the batch, so every cascade has that launch.  Measured without / with it, boards (listed)
+// us: 512 (2) 200 / 161, 1,536 (13) 411 / 379, (67) 444 / 415, 2,048 (9) 520 / 485, 4,096 (4) 937 / 903,
+// (218) 958 / 967, 16,384 (19) 3,428 / 3,402; where it serves nothing it costs 3 to 6 us: 2,048 (99)
+// 549 / 553, 3,000 (153) 752 / 757, 1,000 (110) 335 / 337.
 
 // Boards of a batch that are shared between workgroups: all where they are few; behind whole rounds of one
 // workgroup per CU the rest (fp32: 257 boards 547 -> 343 us, 341 boards 547 -> 419 us, 777 boards 1,092 ->
@@ -2395,7 +2391,6 @@ int team_workspace_bytes(int prec, long long boards, size_t *bytes, long long *s
   const int rc = device_cus(cus);
   if (rc != C6_OK) return rc;
   if (is_cascade(prec)) {
-    if (!team_cascade(prec, boards, cus)) return C6_OK;
     const TeamMode first = team_mode(C6_PREC_BF16), second = team_mode(second_mode(prec));
     const long long teams = second.most(cus), before = team_boards(C6_PREC_BF16, boards, cus);
     *shared = boards < teams ? boards : teams;

@@ -3,8 +3,8 @@
 // A call on few boards is bound by what the host does between two launches, and most of that was
 // Python around the C ABI: walking the module's parameters to see whether the packed weights are
 // still current (20 tensors), three to six torch.empty calls, a device context, 20-odd ctypes
-// conversions.  Measured per call of the B = 1 forward plus mask_logits: 68 us in Python, of which
-// two thirds are gone here.  The kernels are reached through the C ABI's own entry points, whose
+// conversions.  Measured per call of the B = 1 forward plus mask_logits: 68 us in Python, about 36
+// with this.  The kernels are reached through the C ABI's own entry points, whose
 // addresses connect6_amd/_lib.py hands over (`bind`), so this module links against no GPU library.
 #define PY_SSIZE_T_CLEAN
 #include <Python.h>

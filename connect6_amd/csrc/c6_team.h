@@ -12,7 +12,7 @@
 // What it takes (cycles of a 2.4 GHz clock; twelve workgroups, one board): staging the input 7 k, then per
 // layer 1.4-3 k until the neighbours' flags are seen, 2 k until their squares are in LDS, the MFMAs (bf16
 // 1-2.6 k, fp32 4-12 k) and 2-3 k until the outputs are stored and acknowledged: bf16 37 us against 46,
-// bf16 + fp6 44 (63), with low weights 50 (90), fp32 64 (205; 53 boards on three workgroups each 130).
+// bf16 + fp6 44 (63), with low weights 50 (90), fp32 65 (223; 53 boards on three workgroups each 121).
 //
 // The exchange: stores and loads of activations carry the device-scope cache policy (sc1), flags are
 // relaxed device-scope atomics behind a wait for the stores.  Measured between two workgroups:
@@ -929,7 +929,7 @@ __device__ __forceinline__ void team_board(const TeamParams &prm, unsigned char 
 // How many workgroups share a board when there are `boards` of them: as many as fit the chip at once, where
 // that beats one workgroup (1: the one-workgroup kernels).  With fewer workgroups per board more waves read
 // the same weights, and the L1's 64 bytes a cycle bound the layers: measured, 20 / 40 / 80 boards against
-// one workgroup each, fp32 66 / 95 / 134 us against 205, bf16 + fp6 + low weights 52 / 67 / 92 against 90 (60
+// one workgroup each, fp32 69 / 95 / 135 us against 225, bf16 + fp6 + low weights 52 / 67 / 92 against 90 (60
 // boards 83, so three workgroups take up to 73 of 256 CUs; behind a first pass, 53 listed boards, 85 us against
 // 110), bf16 + fp6 45 / 55 / 79 against 63, plain bf16 44 us (20 boards) against 46.
 template <class P> __host__ __device__ inline int team_size(long long boards, int wgs) {

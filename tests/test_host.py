@@ -45,6 +45,15 @@ def test_fused_kernels_stay_within_their_scratch_budget():
     # two workgroups per CU: half the registers, half the LDS
     duo = [u for name, u in usage.items() if "duo_forward_kernel" in name]
     assert len(duo) == 2 and all(u["Occupancy"] == 2 and u["ScratchSize"] <= 16 for u in duo)
+    # a board shared by several workgroups, and small networks: nothing in scratch (scalar registers spill
+    # into vector ones)
+    team = [u for name, u in usage.items() if "team_forward_kernel" in name]
+    small = [u for name, u in usage.items() if "small_net_kernel" in name]
+    assert len(team) == 5 and len(small) == 12 and all(u["ScratchSize"] == 0 for u in team + small)
+    # fp32 by three parts: two sums of most tiles fill the accumulators; what is in scratch is touched between
+    # the K-loops, not in them
+    (split,) = [u for name, u in usage.items() if "split_forward_kernel" in name]
+    assert split["ScratchSize"] <= 400
 
 
 def test_history_dtype_follows_the_reference_policy():

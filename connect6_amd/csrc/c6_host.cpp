@@ -482,6 +482,7 @@ PyObject *forward_generic_module(PyObject *, PyObject *const *a, Py_ssize_t n) {
   const float *pol_w = take({"policy_output", "weight"}, cin, true), *pol_b = take({"policy_output", "bias"}, 1, false);
   const float *val_w = take({"value_output", "weight"}, cin, false), *val_b = take({"value_output", "bias"}, 1, false);
   if (!ok) return nullptr;
+  if (val_w == nullptr) return fail(PyExc_ValueError, "missing parameter value_output.weight: no value without it");
   const at::Tensor packed = fresh({bytes}, at::kByte, dev);
   int rc = abi.generic_pack(1, (int)c.board, c.layers, c.kernels, c.channels, w.data(), bias.data(), pol_w, pol_b, val_w,
                             val_b, c.prec, packed.data_ptr(), (size_t)bytes, c.stream);

@@ -402,6 +402,10 @@ def test_native_host_side_checks_a_modules_parameters():
     with pytest.raises(KeyError, match="missing parameter convs.1.weight"):
         call()
     net.convs[1].weight = kept
+    value, net.value_output = net.value_output, None
+    with pytest.raises(ValueError, match="value_output.weight"):   # not a value of zero
+        call()
+    net.value_output = value
     del net.policy_output
     with pytest.raises(KeyError, match="missing parameter policy_output.weight"):
         call()

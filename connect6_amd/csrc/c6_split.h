@@ -57,13 +57,15 @@ struct SplitGeo {
 // 16-byte granule XOR of a position: sixteen consecutive positions read sixteen bank groups
 __device__ __forceinline__ int split_swz(int pos) { return ((pos >> 1) & 7) << 4; }
 
-// u / (1 + 2^u), the reciprocal with one Newton step.  (Where 1 + 2^u nears the end of fp32 or leaves it the
-// reciprocal is 0 or on its way there, and the step, with the denominator held at 2^126, at most doubles it.)
+// u / (1 + 2^u): the quotient by the approximate reciprocal, then by what it leaves (0.48 ulp rms; by a refined
+// reciprocal 0.58).  Where the denominator is infinite, or u is, what it leaves is a NaN, which min() drops: 0 and
+// u itself are the results.
 __device__ __forceinline__ float split_silu(float u) {
 #pragma clang fp contract(off)   // (the product is rounded before its parts are taken)
   const float d = 1.0f + __builtin_amdgcn_exp2f(u);
   const float r = __builtin_amdgcn_rcpf(d);
-  return u * fmaf(r, fmaf(-fminf(d, 0x1p126f), r, 1.0f), r);
+  const float q = u * r;
+  return fmaf(fminf(fmaf(-d, q, u), 0x1p100f), r, q);
 }
 
 // The heads: sums over the channels, which carry -log2(e), and over all squares.  (In 64 bits, once per square

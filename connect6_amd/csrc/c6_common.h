@@ -221,7 +221,9 @@ template <class P> struct Geo {
   static constexpr size_t TAIL_OFF = (size_t)TOTAL_FRAGS * 1024;  // fp32 tail: biases, heads
   // tail words: bias[544] polw[96] valw[96] polb valb pad pad, then 8 ints sw[layer]
   static constexpr int TAIL_SW = kBiasTotal + 2 * kHeadC + 4;
-  static constexpr int TAIL_FLOATS = TAIL_SW + 8;
+  // fp32 by three parts: then what rounding the scaled biases to fp32 left out
+  static constexpr int TAIL_BIAS_LOW = TAIL_SW + 8;
+  static constexpr int TAIL_FLOATS = TAIL_BIAS_LOW + (P::WLO == 2 ? kBiasTotal : 0);
   static constexpr size_t PACKED_BYTES = TAIL_OFF + (size_t)TAIL_FLOATS * 4;
 };
 

@@ -2116,14 +2116,22 @@ template <class P> __global__ void pack_kernel(const PackParams all) {
   }
   // fp32 tail: biases, head weights, head biases
   const int ti = (int)(gid - nfl);
+  float *tail = reinterpret_cast<float *>(prm.packed + G::TAIL_OFF);
+  auto conv_bias = [&](int i) -> Scaled<P> {
+    int l = 0;
+    while (i >= bias_offset(l + 1)) ++l;
+    return prm.conv_b(l) ? act_scaled<P>(prm.conv_b(l)[i - bias_offset(l)]) : 0.0f;
+  };
+  if (ti >= G::TAIL_BIAS_LOW && ti < G::TAIL_FLOATS) {
+    const Scaled<P> b = conv_bias(ti - G::TAIL_BIAS_LOW);
+    const float low = (float)(b - (float)b);
+    tail[ti] = low == low ? low : 0.0f;   // (an infinite bias leaves nothing)
+  }
   if (ti < G::TAIL_SW) {  // the sw[] words behind it are written by lo_scale_kernel
-    float *tail = reinterpret_cast<float *>(prm.packed + G::TAIL_OFF);
     constexpr float head_scale = P::WLO == 2 ? 1.0f : act_scale<P>();
     float v = 0.0f;
     if (ti < kBiasTotal) {
-      int l = 0;
-      while (ti >= bias_offset(l + 1)) ++l;
-      v = prm.conv_b(l) ? (float)act_scaled<P>(prm.conv_b(l)[ti - bias_offset(l)]) : 0.0f;
+      v = (float)conv_bias(ti);
     } else if (ti < kBiasTotal + kHeadC) {
       v = prm.pol_w[ti - kBiasTotal] / head_scale;
     } else if (ti < kBiasTotal + 2 * kHeadC) {

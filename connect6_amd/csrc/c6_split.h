@@ -13,9 +13,14 @@
 // last layer) that is a bias of 0.77, in units of 2^-24 of the sum's own size, the same in every square,
 // which the value head's mean over 361 squares keeps; apart, 0.02, and the scatter is 2.9 in place
 // of 7.5 (fp32 instructions: 0.03 and 8.9).  Over 64 networks with the reference's initialisation (PyTorch's)
-// the value's error against a 64-bit forward is 2.1e-10 (1.5e-9) rms, with fp32 instructions 3.9e-10
-// (2.0e-9), its mean per network 4e-11 (3.4e-10) against 2.3e-10 (5.1e-10), and the logits' relative error
-// 4.7e-7 (8e-8) against 1.4e-6 (2.0e-7).
+// the value's error against a 64-bit forward is 2.0e-10 (1.5e-9) rms, with fp32 instructions 3.9e-10
+// (2.0e-9), its mean per network 5e-11 (3.4e-10) against 2.3e-10 (5.1e-10), and the logits' relative error
+// 4.6e-7 (8e-8) against 1.4e-6 (2.0e-7).
+//
+// The biases, scaled by -log2(e), are not fp32 numbers any more: the large sum starts with them as fp32, the
+// small one with what that leaves.  Rounded, they are an error of the same sign in every square: the mean
+// of a network's logit errors is then 2.4e-9 of the logits, so 1.1e-9 (fp32 instructions, on parameters as
+// they are: 0.7e-9; medians over 256 networks with PyTorch's initialisation).
 //
 // What bounds it: the matrix cores, 383 k cycles per board with the 1,890 MFMAs of the 3x3 layers
 // six times and the first layer's 207 three times (0/1 inputs are exact in one bf16 value), of 548 k that a
@@ -24,11 +29,11 @@
 // activations of up to 64 channels lie in LDS as their three planes, split once when a layer writes
 // them; 96 channels only fit as fp32 (421 positions x 384 bytes are the CU's whole LDS), and the two
 // layers that read them split them in registers, 44 instructions for eight values, a few behind each
-// MFMA.  2,048 boards take 2.36 ms (4.35 with fp32 instructions; 2.15 with one sum).
+// MFMA.  2,048 boards take 2.33 ms (4.35 with fp32 instructions; 2.11 with one sum).
 //
 // An infinity is its own first part; what is left of it is a NaN in the sum of the small products, and the
-// large ones alone, which are then infinite or NaN as in fp32 arithmetic, are the result (two_sums; with that
-// 2,048 boards take 2.37 ms in place of 2.36).  Parameters and inputs have three parts up to the end of fp32;
+// large ones alone, which are then infinite or NaN as in fp32 arithmetic, are the result (two_sums; 0.4 % of
+// the time).  Parameters and inputs have three parts up to the end of fp32;
 // a sum or an activation has them up to 2.3e38 (3.39e38, the largest bf16 value, with its factor of 1.44) and
 // counts as infinite beyond.
 //
@@ -167,13 +172,13 @@ __device__ __forceinline__ void split_conv_tiles(const unsigned char *smem, cons
   }
 #pragma unroll
   for (int t = 0; t < NT; ++t) {
-    f32x16 b[1];
+    f32x16 b[1], bl[1];
     load_bias_tiles(b, bias + 32 * t, h);
+    load_bias_tiles(bl, bias + Geo<PrecF32S>::TAIL_BIAS_LOW + 32 * t, h);
 #pragma unroll
     for (int j = 0; j < N; ++j) {
       acc[t][J0 + j] = b[0];
-#pragma unroll
-      for (int e = 0; e < 16; ++e) low[t][j][e] = 0.0f;
+      low[t][j] = bl[0];
     }
   }
   constexpr int AHEAD = WIDE ? 2 : 1;
@@ -209,7 +214,7 @@ __device__ __forceinline__ void split_conv_tiles(const unsigned char *smem, cons
 }
 // All pixel tiles.  With three cout tiles the third pixel tile goes first and the other two after it: the
 // sums of all three, 288 registers, are more than the 256 the instruction's accumulators live in (2,048 boards
-// 2.36 ms; cout tiles apart, where 96 input channels are split twice, 2.53; two sums per k-step, added up by
+// 2.33 ms; cout tiles apart, where 96 input channels are split twice, 2.53; two sums per k-step, added up by
 // the vector unit, 3.23).  The first two are left in two sums each.
 template <int NT> using SplitLow = f32x16[NT][NT < 3 ? 3 : 2];
 template <int L>
@@ -448,10 +453,16 @@ __global__ __launch_bounds__(256) void split_forward_kernel(const FwdParams prm)
       for (int ch = 0; ch < 3; ++ch) left[r][ch] = xin[r][ch];
     SplitWeights<1> r2;
     f32x16 low[1][3], first[1][3];   // small products; the large ones, once all parts but the first follow
+    {
+      f32x16 bl[1];
+      load_bias_tiles(bl, tail + G::TAIL_BIAS_LOW + bias_offset(0), h);
 #pragma unroll
-    for (int j = 0; j < 3; ++j)
+      for (int j = 0; j < 3; ++j) {
+        low[0][j] = bl[0];
 #pragma unroll
-      for (int i = 0; i < 16; ++i) low[0][j][i] = first[0][j][i] = 0.0f;
+        for (int i = 0; i < 16; ++i) first[0][j][i] = 0.0f;
+      }
+    }
 #pragma unroll 1
     for (int part = 0; part < parts; ++part) {
       if (part > 0) __syncthreads();  // everybody has read the part before

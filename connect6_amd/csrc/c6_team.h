@@ -145,10 +145,12 @@ __device__ __forceinline__ void team_lo_pass(const unsigned char *smem, const un
 // The contraction of 3x3 layer L for PT tiles of 32 squares and TT cout tiles from t0 on (tiles beyond
 // the layer's last repeat it; their results are not used).
 //   rec: LDS addresses of the lane's squares' records;  acc: the bias on entry
+//   low (fp32): what the bias leaves out, for the small products' sum (split_conv_tiles)
 template <class P, int L, int TT, int PT>
 __device__ __forceinline__ void team_conv(const unsigned char *smem, const unsigned char *packed, const WFrags &wl,
                                           v4i (&ring)[team_ring<P, TT>()][TT][Geo<P>::W], int lane,
-                                          const int (&rec)[PT], int t0, f32x16 (&acc)[PT][TT]) {
+                                          const int (&rec)[PT], int t0, f32x16 (&acc)[PT][TT],
+                                          f32x16 (&low)[PT][TT]) {
   using T = TeamGeo<P>;
   constexpr int NT = kCoutArr[L] / 32, NTP = kCinArr[L] / 32;
   constexpr int W = Geo<P>::W, NPL = T::NPL, D = team_ring<P, TT>();
@@ -174,13 +176,6 @@ __device__ __forceinline__ void team_conv(const unsigned char *smem, const unsig
     for (int p = 0; p < PT; ++p)
 #pragma unroll
       for (int i = 0; i < NPL; ++i) a[v][p][i] = frag(0, v, p, i);
-  f32x16 low[PT][TT];   // NPL == 3: the small products (split_conv_set)
-#pragma unroll
-  for (int p = 0; p < PT; ++p)
-#pragma unroll
-    for (int t = 0; t < TT; ++t)
-#pragma unroll
-      for (int e = 0; e < 16; ++e) low[p][t][e] = 0.0f;
   auto round = [&](int r) __attribute__((always_inline)) {
     // (the low-order pass comes in front of the last phase, as in pipe_layer)
     if constexpr (LO) {
@@ -473,7 +468,7 @@ __device__ __forceinline__ void team_board(const TeamParams &prm, unsigned char 
     }
     // the first weights, behind the activations in the queue: back by the time those are in LDS
     v4i ring[D][TT][W];
-    f32x16 acc[PT][TT];
+    f32x16 acc[PT][TT], low[PT][TT];
     if (active) {
 #pragma unroll
       for (int d = 0; d < D; ++d)
@@ -487,6 +482,11 @@ __device__ __forceinline__ void team_board(const TeamParams &prm, unsigned char 
         load_bias_tiles(one, tail + bias_offset(L) + 32 * (t0 + t < NT ? t0 + t : NT - 1), h);
 #pragma unroll
         for (int i = 0; i < PT; ++i) acc[i][t] = one[0];
+        if constexpr (T::SPLIT) {
+          load_bias_tiles(one, tail + G::TAIL_BIAS_LOW + bias_offset(L) + 32 * (t0 + t < NT ? t0 + t : NT - 1), h);
+#pragma unroll
+          for (int i = 0; i < PT; ++i) low[i][t] = one[0];
+        }
       }
     }
     __builtin_amdgcn_sched_barrier(0);
@@ -510,7 +510,7 @@ __device__ __forceinline__ void team_board(const TeamParams &prm, unsigned char 
       ok[i] = p[i] < kPix;
       rec[i] = record(ok[i] ? p[i] : kPix - 1, sp.base);
     }
-    if (active) team_conv<P, L, TT, PT>(smem, packed, wl, ring, lane, rec, t0, acc);
+    if (active) team_conv<P, L, TT, PT>(smem, packed, wl, ring, lane, rec, t0, acc, low);
     C6_MARK(6 * L + 3);
     if constexpr (L < 7) {
       __syncthreads();   // everybody has read this layer's input
@@ -705,6 +705,13 @@ __device__ __forceinline__ void team_board(const TeamParams &prm, unsigned char 
     f32x16 low, large;   // SPLIT: small products; the large ones, once all parts but the first follow
 #pragma unroll
     for (int i = 0; i < 16; ++i) low[i] = large[i] = 0.0f;
+    if constexpr (T::SPLIT) {
+      if (active) {
+        f32x16 bl[1];
+        load_bias_tiles(bl, tail + G::TAIL_BIAS_LOW + bias_offset(0), h);
+        low = bl[0];
+      }
+    }
 #pragma unroll 1
     for (int part = 0; part < parts; ++part) {
       if (part > 0) __syncthreads();

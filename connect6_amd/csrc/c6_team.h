@@ -9,15 +9,19 @@
 // the same order as in the one-workgroup kernels, and the heads' sums are put together in their
 // order, so the results are the same bit for bit.
 //
-// What it takes (cycles of a 2.4 GHz clock; twelve workgroups, one board): staging the input 7 k, then per
-// layer 1.4-3 k until the neighbours' flags are seen, 2 k until their squares are in LDS, the MFMAs (bf16
-// 1-2.6 k, fp32 4-12 k) and 2-3 k until the outputs are stored and acknowledged: bf16 37 us against 46,
-// bf16 + fp6 44 (63), with low weights 50 (90), fp32 65 (223; 53 boards on three workgroups each 121).
+// What it takes (cycles of a 2.4 GHz clock; twelve workgroups, one board): staging the input 7 k, the first layer
+// 3 k (fp32 9 k), then per layer 1.2 k until the neighbours' flags are seen, 0.5 k until their squares are in LDS,
+// the MFMAs (bf16 0.5-2.1 k, fp32 4-12.5 k: one accumulator's chain, 40 cycles each) and 1.3 k until the outputs are
+// stored and acknowledged, at the end 6 k for the heads' sums: 66 k in bf16, 136 k in fp32.
 //
-// The exchange: stores and loads of activations carry the device-scope cache policy (sc1), flags are
-// relaxed device-scope atomics behind a wait for the stores.  Measured between two workgroups:
-// 0.8-0.95 us for a flag, 1.4 us with 4 KB behind it, 1.8 us with 32 KB, the same within an XCD and
-// across.
+// The exchange: loads of activations and flags carry the device-scope cache policy (sc1).  So do stores until a
+// workgroup has seen that all of its team run on its own XCD (each leaves its XCD's number beside the flags): from
+// then on they stay in that XCD's L2, where the loads find them.  Measured between neighbours of a team on one XCD,
+// store, wait for the acknowledgement, flag, load: 4 KB a side 2.2 us with the stores going through to memory, 1.1 us
+// with stores that stay in L2; 12 KB 3.9 and 1.9 us; 0.3 KB 1.5 and 0.7 us.  (Each word with its tag beside it, no
+// flag and no wait, 1.0, 2.0 and 0.5 us: not worth twice the words and memory of its own.)  One board 38 -> 33 us in
+// bf16, 66 -> 60 us in fp32, 53 fp32 boards 123 -> 117 us, with what else changed there: weights asked for in front
+// of the wait, addresses of exchanged squares formed once, biases and head weights from LDS.
 //
 // Nothing waits for a workgroup that may not be running: a wait is bounded, and a workgroup whose
 // wait runs out does the missing piece of work itself (the earliest one that has no flag; everything
@@ -33,7 +37,8 @@ namespace c6 {
 constexpr int kTeamStages = 9;   // eight layers, then the heads' write-out
 constexpr int kTeamAll = 128;    // flag words: see team_board
 constexpr int kSc1 = 16;         // cache policy: device scope
-static_assert(kTeamAll + kTeamStages * 12 <= kTeamFlags && kTeamStages * 12 <= kTeamAll, "flag words");
+constexpr int kTeamXcd = kTeamAll + kTeamStages * 12;
+static_assert(kTeamXcd + 12 <= kTeamFlags && kTeamStages * 12 <= kTeamAll, "flag words");
 
 // modes that have a team kernel
 template <class P> constexpr bool has_team() { return P::ID != C6_PREC_F32; }
@@ -62,7 +67,9 @@ template <class P> struct TeamGeo {
   static constexpr int LGT_OFF = OCC_OFF + 384;
   static constexpr int RED_OFF = LGT_OFF + 1456;
   static constexpr int RUNS_OFF = RED_OFF + 256 * 4;
-  static constexpr int LDS_BYTES = RUNS_OFF + (kCascadeMaxRuns + 4) * 4;
+  // a copy of the packed set's biases and head weights: no layer starts behind the latency of their loads
+  static constexpr int TAIL_OFF = (RUNS_OFF + (kCascadeMaxRuns + 4) * 4 + 15) & ~15;
+  static constexpr int LDS_BYTES = TAIL_OFF + G::TAIL_FLOATS * 4;
   static_assert(RECB / 16 % 2 == 1 && LDS_BYTES <= 160 * 1024, "LDS map");
 };
 
@@ -107,7 +114,7 @@ __device__ __forceinline__ void team_lo_pass(const unsigned char *smem, const un
   typedef int v8i __attribute__((ext_vector_type(8)));
   constexpr int NT = kCoutArr[L] / 32, PER32 = kCinArr[L] / 32, HC = G::lo_half_chunks(L), NC = G::lo_chunks(L);
   const WFrags wl = packed_frags<P>(packed, lane, G::lo_frag_offset(L));
-  const int scale_w = 127 - reinterpret_cast<const int *>(packed + G::TAIL_OFF)[G::TAIL_SW + L];
+  const int scale_w = 127 - __builtin_amdgcn_readfirstlane(reinterpret_cast<const int *>(smem + T::TAIL_OFF)[G::TAIL_SW + L]);
   constexpr int D = 4;
   v4i w0[D][TT], w1[D][TT];
   auto load = [&](int c, int d) __attribute__((always_inline)) {
@@ -312,10 +319,38 @@ __device__ __forceinline__ void team_board(const TeamParams &prm, unsigned char 
   float *red = reinterpret_cast<float *>(smem + T::RED_OFF);
   int *word = reinterpret_cast<int *>(red) + 255;   // what wave 0 found, for the others
   const unsigned char *packed = f.packed + (size_t)(b / (unsigned)f.boards_per_group) * f.packed_stride;
-  const float *tail = reinterpret_cast<const float *>(packed + G::TAIL_OFF);
+  const float *tail = reinterpret_cast<const float *>(smem + T::TAIL_OFF);   // (from the first stage on)
+  // words of it as a lane's accumulator tile holds its channels
+  auto tail_tile = [&](int word) __attribute__((always_inline)) {
+    f32x16 v;
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const f32x4 b4 = *reinterpret_cast<const f32x4 *>(smem + T::TAIL_OFF + 4 * (word + 8 * q + 4 * h));
+#pragma unroll
+      for (int e = 0; e < 4; ++e) v[4 * q + e] = b4[e];
+    }
+    return v;
+  };
   unsigned char *act = prm.act + (size_t)slot * T::BOARDB;
   unsigned *flags = prm.flags + (size_t)slot * kTeamFlags;
   const __amdgpu_buffer_rsrc_t mem = __builtin_amdgcn_make_buffer_rsrc(act, 0, T::BOARDB, 0x00020000);
+  // Is the whole team known to run on this XCD?  Then what it stores goes to the L2 that they share, where the
+  // others' loads find it, and not through it to memory.
+  const unsigned xcd = __builtin_amdgcn_s_getreg((2 << 11) | 20);   // (hardware register XCC_ID)
+  const unsigned xcd_tag = prm.tag << 4 | 8;   // (no word that is zero looks like one)
+  bool local = false;
+  auto store16 = [&](const v4i &v, int at) __attribute__((always_inline)) {
+    if (local) __builtin_amdgcn_raw_buffer_store_b128(v, mem, at, 0, 0);
+    else __builtin_amdgcn_raw_buffer_store_b128(v, mem, at, 0, kSc1);
+  };
+  auto store4 = [&](float v, int at) __attribute__((always_inline)) {
+    if (local) __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(int, v), mem, at, 0, 0);
+    else __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(int, v), mem, at, 0, kSc1);
+  };
+  auto store_flag = [&](int word) __attribute__((always_inline)) {
+    if (local) __hip_atomic_store(&flags[word], prm.tag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+    else __hip_atomic_store(&flags[word], prm.tag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  };
   [[maybe_unused]] const bool trace_on = true;
 
   // the wave's first tile of squares within the workgroup's, and its group of cout tiles
@@ -330,8 +365,13 @@ __device__ __forceinline__ void team_board(const TeamParams &prm, unsigned char 
   int unfinished = -1;   // word of the piece whose inner squares are still being stored
   // Are the inputs of stage l there for `role` (`own`: its own squares are in LDS)?  Bounded; the answer
   // is the same in every thread.  1: yes, 0: no, 2: no need, the stage itself has been done.
+  constexpr int kWatch = CG == 3 ? 3 : 0;   // the wave that watches the flags: one that has no weights to wait for
   auto wait_inputs = [&](int l, int role, bool own) {
-    if (wave == 0) {
+    if (wave == kWatch) {
+      // (the words of the first layer's workgroups have been there since they started)
+      unsigned about = xcd;
+      if (l == 1 && lane < TEAM) about = __hip_atomic_load(&flags[kTeamXcd + lane], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) ^ xcd_tag;
+      if (l == 1 && __builtin_amdgcn_ballot_w64(about != xcd) == 0) local = true;
       int need = -1;   // the word of stage l - 1 that this lane watches (less the stage's first)
       if (lane < TEAM && (l == 8 || lane == role - 1 || lane == role + 1)) need = lane;
       if (lane == 62 && !own) need = kTeamAll + role;
@@ -342,21 +382,21 @@ __device__ __forceinline__ void team_board(const TeamParams &prm, unsigned char 
         if (__builtin_amdgcn_ballot_w64(!ok) == 0) got = 1;
         if (__builtin_amdgcn_ballot_w64(done) != 0) got = 2;
       }
-      if (lane == 0) *word = got;
+      if (lane == 0) *word = got | (local ? 4 : 0);
     }
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // (the inner squares' stores)
     __syncthreads();
-    const int got = *word;
-    if (tid == 0 && unfinished >= 0)
-      __hip_atomic_store(&flags[kTeamAll + unfinished], prm.tag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    const int got = __builtin_amdgcn_readfirstlane(*word);
+    if (tid == 0 && unfinished >= 0) store_flag(kTeamAll + unfinished);
+    local = (got & 4) != 0;
     unfinished = -1;
     __syncthreads();
-    return got;
+    return got & 3;
   };
   auto raise_flag = [&](int l, int role) {
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // this wave's stores have arrived
     __syncthreads();
-    if (tid == 0) __hip_atomic_store(&flags[l * 12 + role], prm.tag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (tid == 0) store_flag(l * 12 + role);
   };
 
   // The LDS region: positions of the board rows around a role's squares, from the row above the first.
@@ -379,17 +419,25 @@ __device__ __forceinline__ void team_board(const TeamParams &prm, unsigned char 
     for (int i = tid; i < bytes / 16; i += THREADS) reinterpret_cast<v4i *>(smem)[i] = z;
     __syncthreads();
   };
-  // 16-byte unit u of a square's record in a layer of C channels
-  auto unit_at = [](auto cc, int u) __attribute__((always_inline)) {
-    constexpr int C = decltype(cc)::value;
-    if (u < NPL * C / 8) return u / (C / 8) * 192 + u % (C / 8) * 16;
-    return T::LO_OFF + (u - NPL * C / 8) * 16;
+  // Squares between LDS and memory, a layer of C channels: a thread has square `sq` of those at hand and 16-byte unit
+  // `j` of each plane (then of the fp6 blocks), so that all its addresses are two sums and constants.
+  auto unit_of = [&](auto cc, int &sq, int &j) __attribute__((always_inline)) {
+    constexpr int J = decltype(cc)::value / 8;
+    sq = tid / J;
+    j = tid - sq * J;
   };
+  constexpr int PARTS = NPL + (P::LO6 ? 1 : 0);
+  auto part_there = [](auto cc, int k, int j) __attribute__((always_inline)) { return k < NPL || j < decltype(cc)::value / 16; };
+  auto part_mem = [](auto cc, int q, int k, int j) __attribute__((always_inline)) {
+    constexpr int C = decltype(cc)::value;
+    return (q * T::units(C) + k * (C / 8) + j) * 16;
+  };
+  auto part_lds = [](int k, int j) __attribute__((always_inline)) { return (k < NPL ? k * 192 : T::LO_OFF) + j * 16; };
 
   // Outputs of layer L (own squares): into the records, and to memory what the neighbours read.
   // acc: N tiles of squares from the workgroup's tile px on
   auto write_out = [&](auto lc, auto nc, int role, const Span &sp, bool active, const auto &acc, int px, int t0) __attribute__((always_inline)) {
-    constexpr int L = decltype(lc)::value, N = decltype(nc)::value, C = kCoutArr[L], NT = C / 32, UN = T::units(C);
+    constexpr int L = decltype(lc)::value, N = decltype(nc)::value, C = kCoutArr[L], NT = C / 32;
     constexpr int TT = S::tiles(NT);
     constexpr bool LO = P::LO6 && ((P::LO_MASK >> (L + 1)) & 1);
     if (active) {
@@ -403,21 +451,26 @@ __device__ __forceinline__ void team_board(const TeamParams &prm, unsigned char 
       }
     }
     __syncthreads();
-    auto to_memory = [&](int q, int u) __attribute__((always_inline)) {
-      const v4i v = *reinterpret_cast<const v4i *>(smem + record(q, sp.base) + unit_at(IC<C>{}, u));
-      __builtin_amdgcn_raw_buffer_store_b128(v, mem, T::act_off(L) + (q * UN + u) * 16, 0, kSc1);
+    int sq, j;
+    unit_of(IC<C>{}, sq, j);
+    constexpr int PER = THREADS / (C / 8);   // squares at a time
+    auto to_memory = [&](int q) __attribute__((always_inline)) {
+      const unsigned char *from = smem + record(q, sp.base);
+      v4i v[PARTS];
+#pragma unroll
+      for (int k = 0; k < PARTS; ++k)
+        if (part_there(IC<C>{}, k, j)) v[k] = *reinterpret_cast<const v4i *>(from + part_lds(k, j));
+#pragma unroll
+      for (int k = 0; k < PARTS; ++k)
+        if (part_there(IC<C>{}, k, j)) store16(v[k], T::act_off(L) + part_mem(IC<C>{}, q, k, j));
     };
     // twenty squares at either end (all of them where there are no more), then the rest
-    const int n = sp.p1 - sp.p0 + 1, m = n < 40 ? n : 40;
-    for (int i = tid; i < m * UN; i += THREADS) {
-      const int k = i / UN;
-      to_memory(sp.p0 + (k < 20 || n < 40 ? k : n - 40 + k), i - k * UN);
-    }
+    const int n = sp.p1 - sp.p0 + 1;
+    if (sq < 20 && sq < n) to_memory(sp.p0 + sq);
+    if (sq < 20 && sq < n - 20) to_memory(sp.p1 - sq);
     raise_flag(L, role);
-    for (int i = tid; i < (n - m) * UN; i += THREADS) {
-      const int k = i / UN;
-      to_memory(sp.p0 + 20 + k, i - k * UN);
-    }
+    if (sq < PER)
+      for (int q = sp.p0 + 20 + sq; q <= sp.p1 - 20; q += PER) to_memory(q);
     unfinished = L * 12 + role;
     region_role = role;
     region_layer = L;
@@ -426,7 +479,7 @@ __device__ __forceinline__ void team_board(const TeamParams &prm, unsigned char 
   auto conv_stage = [&](auto lc, int role) __attribute__((always_inline)) -> bool {
     constexpr int L = decltype(lc)::value;
     constexpr int NT = kCoutArr[L] / 32, TT = S::tiles(NT), D = team_ring<P, TT>();
-    constexpr int C = kCinArr[L], UN = T::units(C);
+    constexpr int C = kCinArr[L];
     // (opaque per stage: what follows from it is formed here and not, for all stages, in front of the
     // loop over them, in several hundred scalar registers that get spilled)
     int t0 = cg * TT;
@@ -436,69 +489,65 @@ __device__ __forceinline__ void team_board(const TeamParams &prm, unsigned char 
     const WFrags wl = layer_weights<P, L>(packed, lane);
     C6_MARK(6 * L);
     const bool own = region_role == role && region_layer == L - 1;
-    const int got = wait_inputs(L, role, own);
-    if (got != 1) return got == 2;
-    C6_MARK(6 * L + 1);
-    // ---- the neighbours' squares (and, after helping out elsewhere, the own ones) into LDS ----
-    if (region_role != role) clear_region(sp);
-    const int q0 = sp.p0 - 20 > 0 ? sp.p0 - 20 : 0, q1 = sp.p1 + 20 < kPix ? sp.p1 + 20 : kPix - 1;
-    auto load_squares = [&](int from, int count) __attribute__((always_inline)) {   // at most 20
-      constexpr int ROUNDS = (20 * UN + THREADS - 1) / THREADS;
-      v4i in[ROUNDS];
-#pragma unroll
-      for (int k = 0; k < ROUNDS; ++k) {
-        const int i = tid + k * THREADS;
-        if (i < count * UN) in[k] = __builtin_amdgcn_raw_buffer_load_b128(mem, T::act_off(L - 1) + (from * UN + i) * 16, 0, kSc1);
-      }
-#pragma unroll
-      for (int k = 0; k < ROUNDS; ++k) {
-        const int i = tid + k * THREADS, s = i / UN;
-        if (i < count * UN)
-          *reinterpret_cast<v4i *>(smem + record(from + s, sp.base) + unit_at(IC<C>{}, i - s * UN)) = in[k];
-      }
-    };
-    constexpr int ROUNDS = (20 * UN + THREADS - 1) / THREADS;
-    v4i left[ROUNDS], right[ROUNDS];
-    const int nl = sp.p0 - q0, nr = q1 - sp.p1;
-#pragma unroll
-    for (int k = 0; k < ROUNDS; ++k) {
-      const int i = tid + k * THREADS;
-      if (i < nl * UN) left[k] = __builtin_amdgcn_raw_buffer_load_b128(mem, T::act_off(L - 1) + (q0 * UN + i) * 16, 0, kSc1);
-      if (i < nr * UN) right[k] = __builtin_amdgcn_raw_buffer_load_b128(mem, T::act_off(L - 1) + ((sp.p1 + 1) * UN + i) * 16, 0, kSc1);
-    }
-    // the first weights, behind the activations in the queue: back by the time those are in LDS
     v4i ring[D][TT][W];
     f32x16 acc[PT][TT], low[PT][TT];
-    if (active) {
+    auto first_weights = [&]() __attribute__((always_inline)) {
 #pragma unroll
       for (int d = 0; d < D; ++d)
 #pragma unroll
         for (int t = 0; t < TT; ++t)
 #pragma unroll
           for (int i = 0; i < W; ++i) ring[d][t][i] = wl[team_frag<P, L>(d, t0 + t < NT ? t0 + t : NT - 1) + i];
+      __builtin_amdgcn_sched_barrier(0);
+    };
+    // (on their way while the neighbours are waited for; the wave that does the waiting asks for its own behind that)
+    if (active && wave != kWatch) first_weights();
+    const int got = wait_inputs(L, role, own);
+    if (got != 1) return got == 2;
+    C6_MARK(6 * L + 1);
+    // ---- the neighbours' squares (and, after helping out elsewhere, the own ones) into LDS ----
+    if (region_role != role) clear_region(sp);
+    const int q0 = sp.p0 - 20 > 0 ? sp.p0 - 20 : 0, q1 = sp.p1 + 20 < kPix ? sp.p1 + 20 : kPix - 1;
+    int sq, j;
+    unit_of(IC<C>{}, sq, j);
+    auto from_memory = [&](int q, v4i (&v)[PARTS]) __attribute__((always_inline)) {
+#pragma unroll
+      for (int k = 0; k < PARTS; ++k)
+        if (part_there(IC<C>{}, k, j))
+          v[k] = __builtin_amdgcn_raw_buffer_load_b128(mem, T::act_off(L - 1) + part_mem(IC<C>{}, q, k, j), 0, kSc1);
+    };
+    auto to_region = [&](int q, const v4i (&v)[PARTS]) __attribute__((always_inline)) {
+      unsigned char *at = smem + record(q, sp.base);
+#pragma unroll
+      for (int k = 0; k < PARTS; ++k)
+        if (part_there(IC<C>{}, k, j)) *reinterpret_cast<v4i *>(at + part_lds(k, j)) = v[k];
+    };
+    v4i left[PARTS], right[PARTS];
+    const bool has_left = sq < sp.p0 - q0 && sq < 20, has_right = sq < q1 - sp.p1 && sq < 20;
+    if (has_left) from_memory(q0 + sq, left);
+    if (has_right) from_memory(sp.p1 + 1 + sq, right);
+    if (active && wave == kWatch) first_weights();
+    __builtin_amdgcn_sched_barrier(0);
+    if (has_left) to_region(q0 + sq, left);
+    if (has_right) to_region(sp.p1 + 1 + sq, right);
+    if (!own && sq < THREADS / (C / 8))
+      for (int q = sp.p0 + sq; q <= sp.p1; q += THREADS / (C / 8)) {
+        v4i v[PARTS];
+        from_memory(q, v);
+        to_region(q, v);
+      }
+    region_role = -1;   // (until the outputs are in place)
+    if (active) {
 #pragma unroll
       for (int t = 0; t < TT; ++t) {
-        f32x16 one[1];
-        load_bias_tiles(one, tail + bias_offset(L) + 32 * (t0 + t < NT ? t0 + t : NT - 1), h);
+        const int word = bias_offset(L) + 32 * (t0 + t < NT ? t0 + t : NT - 1);
 #pragma unroll
-        for (int i = 0; i < PT; ++i) acc[i][t] = one[0];
-        if constexpr (T::SPLIT) {
-          load_bias_tiles(one, tail + G::TAIL_BIAS_LOW + bias_offset(L) + 32 * (t0 + t < NT ? t0 + t : NT - 1), h);
-#pragma unroll
-          for (int i = 0; i < PT; ++i) low[i][t] = one[0];
+        for (int i = 0; i < PT; ++i) {
+          acc[i][t] = tail_tile(word);
+          if constexpr (T::SPLIT) low[i][t] = tail_tile(G::TAIL_BIAS_LOW + word);
         }
       }
     }
-    __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-    for (int k = 0; k < ROUNDS; ++k) {
-      const int i = tid + k * THREADS, s = i / UN;
-      if (i < nl * UN) *reinterpret_cast<v4i *>(smem + record(q0 + s, sp.base) + unit_at(IC<C>{}, i - s * UN)) = left[k];
-      if (i < nr * UN) *reinterpret_cast<v4i *>(smem + record(sp.p1 + 1 + s, sp.base) + unit_at(IC<C>{}, i - s * UN)) = right[k];
-    }
-    if (!own)
-      for (int q = sp.p0; q <= sp.p1; q += 20) load_squares(q, sp.p1 - q + 1 < 20 ? sp.p1 - q + 1 : 20);
-    region_role = -1;   // (until the outputs are in place)
     __syncthreads();
     C6_MARK(6 * L + 2);
     // ---- contraction ----
@@ -539,10 +588,8 @@ __device__ __forceinline__ void team_board(const TeamParams &prm, unsigned char 
             const unsigned x0 = x[0], x1 = x[1];
             const float tot = __builtin_bit_cast(float, x0) + __builtin_bit_cast(float, x1);
             const float vs = wave_sum(ok[0] ? val : 0.0f);
-            if (h == 0 && ok[0])
-              __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(int, tot), mem, T::HEAD_OFF + ((t0 + t) * 384 + p[0]) * 4, 0, kSc1);
-            if (lane == 0)
-              __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(int, vs), mem, T::VAL_OFF + ((t0 + t) * 12 + tile) * 4, 0, kSc1);
+            if (h == 0 && ok[0]) store4(tot, T::HEAD_OFF + ((t0 + t) * 384 + p[0]) * 4);
+            if (lane == 0) store4(vs, T::VAL_OFF + ((t0 + t) * 12 + tile) * 4);
           }
         }
       } else {
@@ -572,15 +619,12 @@ __device__ __forceinline__ void team_board(const TeamParams &prm, unsigned char 
                   vs = fmaf(a, vw4[e], vs);
                 }
                 // (tile 0: one chain over its sixteen channels; the others: one sum per four)
-                if (t0 + t > 0)
-                  __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(int, vs), mem,
-                                                        T::VAL_OFF + (((tile + i) * 9 + 1 + 4 * (t0 + t - 1) + q) * 64 + lane) * 4, 0, kSc1);
+                if (t0 + t > 0) store4(vs, T::VAL_OFF + (((tile + i) * 9 + 1 + 4 * (t0 + t - 1) + q) * 64 + lane) * 4);
               }
             }
 #pragma unroll
             for (int i = 0; i < PT; ++i)
-              if (t0 + t == 0)
-                __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(int, val0[i]), mem, T::VAL_OFF + ((tile + i) * 9 * 64 + lane) * 4, 0, kSc1);
+              if (t0 + t == 0) store4(val0[i], T::VAL_OFF + ((tile + i) * 9 * 64 + lane) * 4);
           }
         }
 #pragma unroll
@@ -601,8 +645,7 @@ __device__ __forceinline__ void team_board(const TeamParams &prm, unsigned char 
                 const auto x = __builtin_amdgcn_permlane32_swap(bits, bits, false, false);
                 const unsigned x0 = x[0], x1 = x[1];
                 const float tot = __builtin_bit_cast(float, x0) + __builtin_bit_cast(float, x1);
-                if (h == 0 && ok[k])
-                  __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(int, tot), mem, T::HEAD_OFF + p[k] * 4, 0, kSc1);
+                if (h == 0 && ok[k]) store4(tot, T::HEAD_OFF + p[k] * 4);
               }
             }
           }
@@ -636,6 +679,11 @@ __device__ __forceinline__ void team_board(const TeamParams &prm, unsigned char 
         for (int e = 0; e < 4; ++e) acc[0][4 * q + e] = t4[e];
       }
     }
+    constexpr int TAIL_UNITS = (G::TAIL_FLOATS / 4 + THREADS - 1) / THREADS;
+    v4i tl[TAIL_UNITS];
+#pragma unroll
+    for (int i = 0; i < TAIL_UNITS; ++i)
+      if (tid + i * THREADS < G::TAIL_FLOATS / 4) tl[i] = reinterpret_cast<const v4i *>(packed + G::TAIL_OFF)[tid + i * THREADS];
     float xin[2][3];
     const bool state = f.x_dtype == C6_DT_BOARD_I8;
     long long src = state && f.index ? f.index[b] : (long long)b;
@@ -666,6 +714,9 @@ __device__ __forceinline__ void team_board(const TeamParams &prm, unsigned char 
         for (int i = tid; i < per; i += THREADS)
           *reinterpret_cast<v4i *>(smem + s * G::COPY_BYTES + ha * kL1RowPitch * G::EB + i * 16) = z;
     }
+#pragma unroll
+    for (int i = 0; i < TAIL_UNITS; ++i)
+      if (tid + i * THREADS < G::TAIL_FLOATS / 4) reinterpret_cast<v4i *>(smem + T::TAIL_OFF)[tid + i * THREADS] = tl[i];
     if (tid < 2) flag[tid] = 0;
     if (tid == 0) red[66] = xin[0][2];
     __syncthreads();
@@ -675,6 +726,10 @@ __device__ __forceinline__ void team_board(const TeamParams &prm, unsigned char 
     for (int k = 0; k < 2; ++k)
       if (tid + k * THREADS < kPix) varies |= __builtin_bit_cast(int, xin[k][2]) != __builtin_bit_cast(int, c2);
     if (varies) flag[0] = 1;
+    // (the tag and the XCD in one word, at a place that holds nothing else; behind the input's loads, so that
+    // nothing waits for its acknowledgement)
+    if (tid == 0 && role == my_role)
+      __hip_atomic_store(&flags[kTeamXcd + role], xcd_tag ^ xcd, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     __syncthreads();
     const bool plane2_varies = flag[0] != 0;
     int parts = 1;
@@ -697,20 +752,15 @@ __device__ __forceinline__ void team_board(const TeamParams &prm, unsigned char 
     const int rowb = (plane2_varies ? 1 : 3) * kL1RowPitch * G::EB;
     const WFrags wl = plane2_varies ? layer_weights<P, 0>(packed, lane) : packed_frags<P>(packed, lane, G::FAST1_OFF);
     if (active) {
-      f32x16 b0[1];
-      load_bias_tiles(b0, tail + bias_offset(0), h);
+      const f32x16 b0 = tail_tile(bias_offset(0));
 #pragma unroll
-      for (int i = 0; i < 16; ++i) acc[0][i] = plane2_varies ? b0[0][i] : fmaf(c2, acc[0][i], b0[0][i]);
+      for (int i = 0; i < 16; ++i) acc[0][i] = plane2_varies ? b0[i] : fmaf(c2, acc[0][i], b0[i]);
     }
     f32x16 low, large;   // SPLIT: small products; the large ones, once all parts but the first follow
 #pragma unroll
     for (int i = 0; i < 16; ++i) low[i] = large[i] = 0.0f;
     if constexpr (T::SPLIT) {
-      if (active) {
-        f32x16 bl[1];
-        load_bias_tiles(bl, tail + G::TAIL_BIAS_LOW + bias_offset(0), h);
-        low = bl[0];
-      }
+      if (active) low = tail_tile(G::TAIL_BIAS_LOW + bias_offset(0));
     }
 #pragma unroll 1
     for (int part = 0; part < parts; ++part) {
@@ -740,41 +790,51 @@ __device__ __forceinline__ void team_board(const TeamParams &prm, unsigned char 
       __syncthreads();
       C6_MARK(1);
       if (active) {
-        // k-steps in rounds of one kernel row (three fragments); operands three rounds ahead
-        v4i w[4][3][W], a[4][3];
-        auto fetch = [&](int row, int s4) __attribute__((always_inline)) {
-          const int rr = row < rows ? row : rows - 1;
+        // Kernel rows (three fragments each), the row's activations asked for a row ahead and its weights DW rows, one
+        // load behind each MFMA: a lone wave issues an instruction per five cycles, and what it issues between two rows
+        // the matrix core waits for (all of a row's loads in front of it: bf16 54 cycles per MFMA, fp32 58).
+        constexpr int DW = W == 3 ? 4 : 8;
+        static_assert(DW % 2 == 0, "activations alternate");
+        v4i w[DW][3][W], a[2][3];
+        auto weight = [&](int row, int i, int j) __attribute__((always_inline)) {
+          return wl[((row < rows ? row : rows - 1) * 3 + i) * W + j];
+        };
+        auto activation = [&](int row, int i) __attribute__((always_inline)) {
+          return *reinterpret_cast<const v4i *>(smem + row0 + (row < rows ? row : rows - 1) * rowb + i * 16);
+        };
+        auto one_row = [&](int row, auto sc) __attribute__((always_inline)) {
+          constexpr int s8 = decltype(sc)::value;
+#pragma unroll
+          for (int i = 0; i < 3; ++i) {
+            static_for<0, W>([&](auto jc) __attribute__((always_inline)) {
+              constexpr int j = decltype(jc)::value;
+              mma<P>(w[s8][i][j], a[s8 % 2][i], T::SPLIT && j > 0 ? low : acc[0]);
+              w[s8][i][j] = weight(row + DW, i, j);
+            });
+            a[(s8 + 1) % 2][i] = activation(row + 1, i);
+          }
+#pragma unroll
+          for (int i = 0; i < 3 * W; ++i) {
+            __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);                    // one MFMA
+            __builtin_amdgcn_sched_group_barrier(0x020, 1, 0);                    // one weight
+            if (i % W == W - 1) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);   // one LDS read
+          }
+          __builtin_amdgcn_sched_barrier(0);
+        };
+#pragma unroll
+        for (int s8 = 0; s8 < DW; ++s8)
 #pragma unroll
           for (int i = 0; i < 3; ++i) {
 #pragma unroll
-            for (int j = 0; j < W; ++j) w[s4][i][j] = wl[(rr * 3 + i) * W + j];
-            a[s4][i] = *reinterpret_cast<const v4i *>(smem + row0 + rr * rowb + i * 16);
+            for (int j = 0; j < W; ++j) w[s8][i][j] = weight(s8, i, j);
+            if (s8 == 0) a[0][i] = activation(0, i);
           }
-          __builtin_amdgcn_sched_barrier(0);
-        };
-        auto multiply = [&](int s4) __attribute__((always_inline)) {
-#pragma unroll
-          for (int i = 0; i < 3; ++i)
-            static_for<0, W>([&](auto jc) __attribute__((always_inline)) {
-              constexpr int j = decltype(jc)::value;
-              mma<P>(w[s4][i][j], a[s4][i], T::SPLIT && j > 0 ? low : acc[0]);
-            });
-          __builtin_amdgcn_sched_barrier(0);
-        };
-#pragma unroll
-        for (int s4 = 0; s4 < 3; ++s4) fetch(s4, s4);
         int row = 0;
 #pragma unroll 1
-        for (; row + 4 <= rows; row += 4) {
-#pragma unroll
-          for (int s4 = 0; s4 < 4; ++s4) {
-            fetch(row + s4 + 3, (s4 + 3) % 4);
-            multiply(s4);
-          }
-        }
-#pragma unroll
-        for (int s4 = 0; s4 < 3; ++s4)
-          if (row + s4 < rows) multiply(s4);
+        for (; row + DW <= rows; row += DW) static_for<0, DW>([&](auto sc) __attribute__((always_inline)) { one_row(row + decltype(sc)::value, sc); });
+        static_for<0, DW - 1>([&](auto sc) __attribute__((always_inline)) {
+          if (row + decltype(sc)::value < rows) one_row(row + decltype(sc)::value, sc);
+        });
         if constexpr (T::SPLIT) {
           if (parts > 1 && part == 0) {
             large = acc[0];
@@ -856,7 +916,7 @@ __device__ __forceinline__ void team_board(const TeamParams &prm, unsigned char 
       if (lane == 0) red[wave] = vsum;
     }
     __syncthreads();
-    if (tid == 0 && f.value != nullptr) {
+    if (tid == 192 && f.value != nullptr) {   // (beside the draw and the margin)
       if constexpr (T::SPLIT) {
         f.value[b] = split_value(split_value_sum(red), valb);
       } else {

@@ -34,7 +34,7 @@ struct SmallLayer {
   int blocks, chunks;    // (tap, channel block) pairs and their groups of four = MFMAs of K 32
   int frag0, bias0;      // first weight fragment; first bias in the tail
   int pitch;             // LDS positions per row of this layer's input: n + r
-  unsigned pitch_magic;  // ceil(2^32 / pitch): p / pitch for the small p here
+  unsigned pitch_magic, k_magic, cb_magic;  // ceil(2^32 / d), for the small quotients here
   int positions;         // of one board
   int pixb, planeb;      // bytes of one position, of one precision plane of it
   int boardb;            // bytes of one board
@@ -49,7 +49,9 @@ struct SmallParams {
   const unsigned char *packed;
   size_t packed_stride, tail;
   int n, nn, layers, nb;       // nb: boards per workgroup
-  int table_off, pix_off, val_off;  // LDS: offset tables, squares, value sums
+  unsigned n_magic, nn_magic;
+  int table_off, pix_off, val_off, tail_off;  // LDS: offset tables, squares, value sums, the packed tail
+  int tail_floats;
   int bias_total;
   float *logits, *value;
   int mask_mode;
@@ -85,6 +87,40 @@ template <class A, bool ANY = false> __device__ __forceinline__ void small_plane
   }
 }
 
+__device__ __forceinline__ int small_div(int p, unsigned magic) { return magic == 0 ? p : (int)__umulhi((unsigned)p, magic); }
+
+// Where nothing is rounded to 16 bits, all activations carry the factor -log2(e) / 2, so that SiLU is u / (1 + 2^(2 u));
+// it is put in with the first layer's weights and all biases, in 64 bits, and taken out behind the heads.  (The half:
+// a factor below 1 leaves fp32 its whole range.)
+template <class A> constexpr bool small_scaled() { return A::NA == 3 && A::NW == 3; }
+constexpr double kSmallScale = -0.72134752044448170368;
+template <class A> __device__ __forceinline__ double small_scale(double v, bool scaled) {
+  return small_scaled<A>() && scaled ? v * kSmallScale : v;
+}
+// a parameter's planes, of its value in 64 bits
+template <class A> __device__ __forceinline__ void small_weight_planes64(double v, unsigned short (&p)[A::NW]) {
+  if constexpr (small_scaled<A>()) {
+#pragma unroll
+    for (int i = 0; i < A::NW; ++i) {
+      p[i] = bf16_part((float)v);
+      v = (p[i] & 0x7f80) == 0x7f80 ? 0.0 : v - (double)__builtin_bit_cast(float, (unsigned)p[i] << 16);
+    }
+  } else {
+    small_planes<SmallArith<A::NW, A::NW, A::F16>, true>((float)v, p);
+  }
+}
+// Two values' next planes in one dword; the values keep what it leaves out.
+__device__ __forceinline__ int small_take(float &a, float &b, bool more) {
+#pragma clang fp contract(off)
+  typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+  const int w = __builtin_bit_cast(int, bf16x2{(__bf16)a, (__bf16)b});
+  if (more) {
+    a -= __builtin_bit_cast(float, w << 16);
+    b -= __builtin_bit_cast(float, w & (int)0xffff0000);
+  }
+  return w;
+}
+
 template <class A> __device__ __forceinline__ f32x4 small_mma(const v4i &w, const v4i &a, const f32x4 &c) {
   if constexpr (A::F16) {
     return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, w), __builtin_bit_cast(f16x8, a), c, 0, 0, 0);
@@ -103,6 +139,7 @@ __device__ __forceinline__ float small_load(const void *x, int dt, size_t i) {
 // Where a wave's weight fragments come from: the packed copy (fragment ((chunk * tiles + tile) *
 // planes + plane), see small_pack_kernel) ...
 template <class A> struct PackedWeights {
+  static constexpr bool kPacked = true;
   const unsigned char *p;
   template <int CT> __device__ __forceinline__ void fetch(int c, v4i (&w)[CT][A::NW]) const {
 #pragma unroll
@@ -114,7 +151,8 @@ template <class A> struct PackedWeights {
 };
 // ... or the tensors themselves, for a caller that hands over weights with every call: eight
 // gathered loads and the conversion per fragment, the same values.
-template <class A> struct RawWeights {
+template <class A, bool FIRST> struct RawWeights {   // FIRST: the first layer's, which are scaled
+  static constexpr bool kPacked = false;
   const float *w;  // [cout, cin, k, k] of the weight set
   int cin, cout, kk, cb, cb_magic, blocks, lane;
   template <int CT> __device__ __forceinline__ void fetch(int c, v4i (&out)[CT][A::NW]) const {
@@ -128,7 +166,8 @@ template <class A> struct RawWeights {
       for (int i = 0; i < 8; ++i) {
         const bool in = row && ci0 + i < cin;
         const float v = w[in ? (size_t)(co * cin + ci0 + i) * kk + tap : 0];
-        small_planes<SmallArith<A::NW, A::NW, A::F16>, true>(in ? v : 0.0f, pl[i]);
+        if constexpr (small_scaled<A>() && FIRST) small_weight_planes64<A>(small_scale<A>(in ? v : 0.0f, true), pl[i]);
+        else small_planes<SmallArith<A::NW, A::NW, A::F16>, true>(in ? v : 0.0f, pl[i]);
       }
 #pragma unroll
       for (int p = 0; p < A::NW; ++p)
@@ -138,20 +177,30 @@ template <class A> struct RawWeights {
   }
 };
 
+// the tail's second part: the biases' low parts
+constexpr int small_low(int bias_total) { return bias_total + 2 * 16 * kSmallMaxTiles + 4; }
+__device__ __forceinline__ float small_rest(double v, float rounded) {
+  return __builtin_fabsf(rounded) < __builtin_inff() ? (float)(v - (double)rounded) : 0.0f;
+}
+
 // One layer's contraction for the wave's PT tiles of 16 squares and its CT tiles of 16 channels.
 // Operands of the next chunk are fetched while the current one's MFMAs run.
-template <class A, int PT, int CT, class Weights>
+//   NA: planes of its activations that are not zero
+template <class A, int NA, int PT, int CT, class Weights>
 __device__ __forceinline__ void small_contract(const unsigned char *smem, const unsigned short *table,
                                                const Weights &weights, const SmallLayer &L, int lane,
-                                               const int (&base)[PT], f32x4 (&acc)[PT][CT]) {
-  constexpr int NA = A::NA, NW = A::NW;
+                                               const int (&base)[PT], f32x4 (&acc)[PT][CT], f32x4 (&low)[PT][CT]) {
+  constexpr int NW = A::NW;
   const int q = lane >> 4;
   const unsigned short *tab = table + L.table0 + q;
   const int planeb = L.planeb, chunks = L.chunks;
   v4i w[2][CT][NW], a[2][PT][NA];
+  // (a chunk's offset is read a chunk ahead of its operands: no wave waits for one)
+  int next = (int)tab[0] * 16;
   auto fetch = [&](int c, int s) __attribute__((always_inline)) {
     weights.template fetch<CT>(c, w[s]);
-    const int off = (int)tab[4 * c] * 16;
+    const int off = Weights::kPacked ? next : (int)tab[4 * c] * 16;
+    if constexpr (Weights::kPacked) next = (int)tab[4 * (c + 1 < chunks ? c + 1 : c)] * 16;
 #pragma unroll
     for (int j = 0; j < PT; ++j)
 #pragma unroll
@@ -159,7 +208,6 @@ __device__ __forceinline__ void small_contract(const unsigned char *smem, const 
   };
   // Operands in several planes: the small products have a sum of their own (the instruction drops what lies
   // some eight bits below the last of its sum, towards minus infinity; see c6_split.h)
-  f32x4 low[PT][CT];
 #pragma unroll
   for (int j = 0; j < PT; ++j)
 #pragma unroll
@@ -167,7 +215,7 @@ __device__ __forceinline__ void small_contract(const unsigned char *smem, const 
   auto multiply = [&](int s) __attribute__((always_inline)) {
     // smallest products first
 #pragma unroll
-    for (int d = (NA < NW ? NA : NW) == 3 ? 2 : NA - 1; d >= 0; --d)
+    for (int d = (A::NA < NW ? A::NA : NW) == 3 ? 2 : A::NA - 1; d >= 0; --d)
 #pragma unroll
       for (int i = 0; i <= d; ++i) {  // activation plane d - i, weight plane i
         if (d - i >= NA || i >= NW) continue;
@@ -190,14 +238,6 @@ __device__ __forceinline__ void small_contract(const unsigned char *smem, const 
     multiply(1);
   }
   if (c < chunks) multiply(0);
-  if constexpr (NA > 1 || NW > 1) {
-#pragma unroll
-    for (int j = 0; j < PT; ++j)
-#pragma unroll
-      for (int t = 0; t < CT; ++t)
-#pragma unroll
-        for (int e = 0; e < 4; ++e) acc[j][t][e] = two_sums(acc[j][t][e], low[j][t][e]);
-  }
 }
 
 // u / (1 + e^-u) to fp32 accuracy with the hardware's exp2 and reciprocal: the product u * log2(e)
@@ -213,6 +253,15 @@ __device__ __forceinline__ float small_silu(float u) {
   // (below u = -87 the result is under 2^-119 and the reciprocal on its way to 0)
   return u * (t < 126.0f ? fmaf(r, fmaf(-d, r, 1.0f), r) : 0.0f);
 }
+// u / (1 + 2^(2 u)), of activations that carry the factor: the quotient by the approximate reciprocal, then by what it
+// leaves (0.48 ulp rms; see split_silu in c6_split.h)
+__device__ __forceinline__ float small_silu2(float u) {
+#pragma clang fp contract(off)
+  const float d = 1.0f + __builtin_amdgcn_exp2f(u + u);
+  const float r = __builtin_amdgcn_rcpf(d);
+  const float q = u * r;
+  return fmaf(fminf(fmaf(-d, q, u), 0x1p100f), r, q);
+}
 
 // A workgroup evaluates `nb` boards of one weight set from input to heads; a wave owns PT tiles of
 // 16 squares (of whichever of the boards) and all output channels of them, in every layer.  The
@@ -221,9 +270,12 @@ __device__ __forceinline__ float small_silu(float u) {
 // their padding columns), so that a (tap, block of eight channels) is a constant offset, looked up
 // in a table by the lane group that contracts it.
 //
-// Measured on 1024 boards of the 9x9 network above, fp32: 26 us (914 us layer by layer; 24 with one
-// sum), of which the six-product MFMAs alone are 7 us; the rest is the two waves per SIMD meeting at two
-// barriers per layer, the staging of the input and the launch.
+// Measured on 1024 boards of the 9x9 network above, fp32: 23 us (914 us layer by layer; 26 with a SiLU that puts the
+// factor log2(e) in by itself, planes split value by value, a chunk's offset read in front of its operands, and the
+// input loaded board by board behind the tables; 4096 boards of four such networks 96 -> 83 us, twenty 19x19 boards of
+// kernels 7,3,3,3,3 and 32 channels 64 -> 53 us).  The MFMAs are 8 us of it at 2.4 GHz, all but the contractions 8 us
+// (launch, staging, epilogues); the rest is the two waves per SIMD meeting at two barriers per layer and the reads of
+// weights and activations, some 2 and 3 us.
 template <class A, int PT, bool RAW>
 __global__ __launch_bounds__(64 * kSmallMaxWaves) void small_net_kernel(const SmallParams prm) {
   constexpr int NA = A::NA;
@@ -234,26 +286,34 @@ __global__ __launch_bounds__(64 * kSmallMaxWaves) void small_net_kernel(const Sm
   unsigned short *table = reinterpret_cast<unsigned short *>(smem + prm.table_off);
   int *s_pix = reinterpret_cast<int *>(smem + prm.pix_off);
   float *s_val = reinterpret_cast<float *>(smem + prm.val_off);
+  int *s_inexact = reinterpret_cast<int *>(s_val);   // (until the heads)
 
   const long long g = blockIdx.x / prm.wgs_per_group;
   const long long first = (long long)(blockIdx.x % prm.wgs_per_group) * prm.nb;
   const int boards = (int)(prm.per_group - first < prm.nb ? prm.per_group - first : prm.nb);
   const long long b0 = g * prm.per_group + first;
   const unsigned char *weights = prm.packed + (size_t)g * prm.packed_stride;
-  const float *tail = reinterpret_cast<const float *>(weights + prm.tail);
+  const float *tail = reinterpret_cast<const float *>(smem + prm.tail_off);   // (a copy: no layer starts behind its loads)
   const int npx = boards * nn;
 
-  // squares of the workgroup's boards, and every layer's table of offsets (16-byte units)
-  for (int p = tid; p < npx; p += threads) {
-    const int b = p / nn, s = p - b * nn, r = s / n;
-    s_pix[p] = b << 16 | r << 8 | (s - r * n);
-  }
+  // a thread's square (there are as many threads as squares) and its input, asked for before anything else
+  const int my_b = small_div(tid, prm.nn_magic), my_s = tid - my_b * nn, my_r = small_div(my_s, prm.n_magic), my_c = my_s - my_r * n;
+  const bool has = tid < npx;
+  float xin[3];
+#pragma unroll
+  for (int ch = 0; ch < 3; ++ch)
+    xin[ch] = has ? small_load(prm.x, prm.x_dtype, ((size_t)(b0 + my_b) * 3 + ch) * nn + my_s) : 0.0f;
+  if (has) s_pix[tid] = my_b << 16 | my_r << 8 | my_c;
+  if constexpr (!RAW)
+    for (int i = tid; i < prm.tail_floats / 4; i += threads)
+      reinterpret_cast<v4i *>(smem + prm.tail_off)[i] = reinterpret_cast<const v4i *>(weights + prm.tail)[i];
+  // every layer's table of offsets (16-byte units)
   for (int l = 0; l < prm.layers; ++l) {
     const SmallLayer &L = prm.layer[l];
     for (int e = tid; e < 4 * L.chunks; e += threads) {
       int off = 0;
       if (e < L.blocks) {
-        const int tap = e / L.cb, cb = e - tap * L.cb, ky = tap / L.k;
+        const int tap = small_div(e, L.cb_magic), cb = e - tap * L.cb, ky = small_div(tap, L.k_magic);
         off = ((ky * L.pitch + tap - ky * L.k) * L.pixb + cb * 16) >> 4;
       }
       table[L.table0 + e] = (unsigned short)off;
@@ -263,21 +323,25 @@ __global__ __launch_bounds__(64 * kSmallMaxWaves) void small_net_kernel(const Sm
     const SmallLayer &L = prm.layer[0];
     const v4i z = {0, 0, 0, 0};
     for (int i = tid; i < boards * L.boardb / 16; i += threads) reinterpret_cast<v4i *>(smem)[i] = z;
+    if (tid == 0) *s_inexact = 0;
     __syncthreads();
-    for (int b = 0; b < boards; ++b)
-      for (int s = tid; s < nn; s += threads) {
-        const int rc = s_pix[s], r = (rc >> 8) & 255, c = rc & 255;
-        unsigned char *at = smem + b * L.boardb + ((r + L.r) * L.pitch + c + L.r) * L.pixb;
+    if (has) {
+      bool inexact = false;
 #pragma unroll
-        for (int ch = 0; ch < 3; ++ch) {
-          unsigned short pl[NA];
-          small_planes<A, true>(small_load(prm.x, prm.x_dtype, ((size_t)(b0 + b) * 3 + ch) * nn + s), pl);
+      for (int ch = 0; ch < 3; ++ch) inexact |= (__builtin_bit_cast(int, xin[ch]) & 0xffff) != 0 || !(__builtin_fabsf(xin[ch]) < __builtin_inff());
+      if (inexact) *s_inexact = 1;
+      unsigned char *at = smem + my_b * L.boardb + ((my_r + L.r) * L.pitch + my_c + L.r) * L.pixb;
 #pragma unroll
-          for (int i = 0; i < NA; ++i) *reinterpret_cast<unsigned short *>(at + i * L.planeb + 2 * ch) = pl[i];
-        }
+      for (int ch = 0; ch < 3; ++ch) {
+        unsigned short pl[NA];
+        small_planes<A, true>(xin[ch], pl);
+#pragma unroll
+        for (int i = 0; i < NA; ++i) *reinterpret_cast<unsigned short *>(at + i * L.planeb + 2 * ch) = pl[i];
       }
+    }
     __syncthreads();
   }
+  const bool one_plane = __builtin_amdgcn_readfirstlane(*s_inexact) == 0;
 
   int rc[PT];
   bool mine[PT];  // the lane's square exists (the others shadow the last one and store nothing)
@@ -301,7 +365,7 @@ __global__ __launch_bounds__(64 * kSmallMaxWaves) void small_net_kernel(const Sm
       base[j] = (rc[j] >> 16) * L.boardb + (((rc[j] >> 8) & 255) * L.pitch + (rc[j] & 255)) * L.pixb;
     auto run = [&](auto ct) __attribute__((always_inline)) {
       constexpr int CT = decltype(ct)::value;
-      f32x4 acc[PT][CT];
+      f32x4 acc[PT][CT], low[PT][CT];
       if (busy) {
 #pragma unroll
         for (int t = 0; t < CT; ++t) {
@@ -311,25 +375,48 @@ __global__ __launch_bounds__(64 * kSmallMaxWaves) void small_net_kernel(const Sm
           } else if (prm.conv_b[l] != nullptr) {
 #pragma unroll
             for (int i = 0; i < 4; ++i)
-              if (16 * t + 4 * q + i < L.cout) b[i] = prm.conv_b[l][(size_t)g * L.cout + 16 * t + 4 * q + i];
+              if (16 * t + 4 * q + i < L.cout) b[i] = (float)small_scale<A>(prm.conv_b[l][(size_t)g * L.cout + 16 * t + 4 * q + i], true);
           }
 #pragma unroll
           for (int j = 0; j < PT; ++j) acc[j][t] = b;
         }
         if constexpr (RAW) {
-          const RawWeights<A> w{prm.conv_w[l] + (size_t)g * L.cout * L.cin * L.k * L.k, L.cin, L.cout, L.k * L.k, L.cb,
-                                (65536 + L.cb - 1) / L.cb, L.blocks, lane};
-          small_contract<A, PT, CT>(smem, table, w, L, lane, base, acc);
+          auto raw = [&](auto first) __attribute__((always_inline)) {
+            const RawWeights<A, decltype(first)::value> w{prm.conv_w[l] + (size_t)g * L.cout * L.cin * L.k * L.k, L.cin, L.cout,
+                                                          L.k * L.k, L.cb, (65536 + L.cb - 1) / L.cb, L.blocks, lane};
+            small_contract<A, NA, PT, CT>(smem, table, w, L, lane, base, acc, low);
+          };
+          if (small_scaled<A>() && l == 0) raw(std::true_type{});
+          else raw(std::false_type{});
         } else {
           const PackedWeights<A> w{weights + (size_t)L.frag0 * 1024 + lane * 16};
-          small_contract<A, PT, CT>(smem, table, w, L, lane, base, acc);
+          // (stones and flags are exact in one plane: half the first layer's products, the others are zeros)
+          if (A::NA > 1 && l == 0 && one_plane) small_contract<A, 1, PT, CT>(smem, table, w, L, lane, base, acc, low);
+          else small_contract<A, NA, PT, CT>(smem, table, w, L, lane, base, acc, low);
         }
 #pragma unroll
-        for (int j = 0; j < PT; ++j)
+        for (int t = 0; t < CT; ++t) {
+          f32x4 bl = {0.0f, 0.0f, 0.0f, 0.0f};   // what rounding the scaled biases left out, with the small products
+          if constexpr (small_scaled<A>() && !RAW) {
+            bl = *reinterpret_cast<const f32x4 *>(tail + small_low(prm.bias_total) + L.bias0 + 16 * t + 4 * q);
+          } else if constexpr (small_scaled<A>()) {
+            if (prm.conv_b[l] != nullptr)
 #pragma unroll
-          for (int t = 0; t < CT; ++t)
+              for (int i = 0; i < 4; ++i)
+                if (16 * t + 4 * q + i < L.cout) {
+                  const double v = small_scale<A>(prm.conv_b[l][(size_t)g * L.cout + 16 * t + 4 * q + i], true);
+                  bl[i] = small_rest(v, (float)v);
+                }
+          }
 #pragma unroll
-            for (int i = 0; i < 4; ++i) acc[j][t][i] = small_silu(acc[j][t][i]);
+          for (int j = 0; j < PT; ++j)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+              float u = acc[j][t][i];
+              if constexpr (A::NA > 1 || A::NW > 1) u = two_sums(u, low[j][t][i] + bl[i]);
+              acc[j][t][i] = small_scaled<A>() ? small_silu2(u) : small_silu(u);
+            }
+        }
       }
       if (last) {
         if (busy) {
@@ -379,13 +466,21 @@ __global__ __launch_bounds__(64 * kSmallMaxWaves) void small_net_kernel(const Sm
         for (int t = 0; t < CT; ++t) {
           const int ch = 16 * t + 4 * q;
           if (ch >= 8 * N.cb) continue;
-          unsigned short pl[4][NA];
+          if constexpr (A::F16) {
+            unsigned short pl[4][NA];
 #pragma unroll
-          for (int i = 0; i < 4; ++i) small_planes<A>(acc[j][t][i], pl[i]);
+            for (int i = 0; i < 4; ++i) small_planes<A>(acc[j][t][i], pl[i]);
+            *reinterpret_cast<v2i *>(at + 2 * ch) = v2i{pl[0][0] | (int)pl[1][0] << 16, pl[2][0] | (int)pl[3][0] << 16};
+          } else {
+            float v[4];
 #pragma unroll
-          for (int i = 0; i < NA; ++i)
-            *reinterpret_cast<v2i *>(at + i * N.planeb + 2 * ch) =
-                v2i{pl[0][i] | (int)pl[1][i] << 16, pl[2][i] | (int)pl[3][i] << 16};
+            for (int i = 0; i < 4; ++i) v[i] = acc[j][t][i];
+#pragma unroll
+            for (int i = 0; i < NA; ++i) {
+              const int lo = small_take(v[0], v[1], i + 1 < NA), hi = small_take(v[2], v[3], i + 1 < NA);
+              *reinterpret_cast<v2i *>(at + i * N.planeb + 2 * ch) = v2i{lo, hi};
+            }
+          }
         }
       }
       __syncthreads();
@@ -421,7 +516,9 @@ __global__ __launch_bounds__(64 * kSmallMaxWaves) void small_net_kernel(const Sm
         if (prm.mask_mode == C6_MASK_INPUT)
           occupied = small_load(prm.x, prm.x_dtype, (size_t)(b0 + b) * 3 * nn + s) != 0.0f ||
                      small_load(prm.x, prm.x_dtype, ((size_t)(b0 + b) * 3 + 1) * nn + s) != 0.0f;
-        prm.logits[(size_t)(b0 + b) * nn + s] = occupied ? prm.fill : p + pol_b;
+        float z = p + pol_b;
+        if constexpr (small_scaled<A>()) z = (float)((double)p * (1.0 / kSmallScale) + (double)pol_b);
+        prm.logits[(size_t)(b0 + b) * nn + s] = occupied ? prm.fill : z;
       }
     }
   }
@@ -431,7 +528,7 @@ __global__ __launch_bounds__(64 * kSmallMaxWaves) void small_net_kernel(const Sm
       float v = 0.0f;
       for (int s = lane; s < nn; s += 64) v += s_val[b * nn + s];
       v = wave_sum(v);
-      if (lane == 0) prm.value[b0 + b] = (float)tanh((double)v / nn + (double)val_b);   // (one rounding)
+      if (lane == 0) prm.value[b0 + b] = (float)tanh((double)v * (small_scaled<A>() ? 1.0 / kSmallScale : 1.0) / nn + (double)val_b);   // (one rounding)
     }
   }
 }
@@ -456,7 +553,8 @@ template <class A> __global__ void small_pack_kernel(const SmallPack prm) {
   unsigned char *packed = prm.packed + (size_t)g * prm.packed_stride;
   if (i < (long long)prm.frags * 64) {   // one thread per (group of planes, lane)
     const int lane = (int)(i & 63);
-    int f = (int)(i >> 6) * A::NW, l = 0;
+    // (the same in a whole wave: the layer's numbers then come through the scalar cache)
+    int f = __builtin_amdgcn_readfirstlane((int)(i >> 6)) * A::NW, l = 0;
     while (l + 1 < prm.layers && f >= prm.layer[l + 1].frag0) ++l;
     const SmallLayer &L = prm.layer[l];
     const int ct = (f - L.frag0) / A::NW, c = ct / L.tiles, t = ct - c * L.tiles;
@@ -467,7 +565,7 @@ template <class A> __global__ void small_pack_kernel(const SmallPack prm) {
       const int ci = 8 * cb + k;
       const bool in = e < L.blocks && co < L.cout && ci < L.cin;
       const float v = in ? w[((size_t)co * L.cin + ci) * L.k * L.k + tap] : 0.0f;
-      small_planes<SmallArith<A::NW, A::NW, A::F16>, true>(v, pl[k]);
+      small_weight_planes64<A>(small_scale<A>(v, l == 0), pl[k]);
     }
     for (int p = 0; p < A::NW; ++p) {
       v4i o;
@@ -479,14 +577,17 @@ template <class A> __global__ void small_pack_kernel(const SmallPack prm) {
   const int ti = (int)(i - (long long)prm.frags * 64);
   float *tail = reinterpret_cast<float *>(packed + prm.tail);
   constexpr int kHead = 16 * kSmallMaxTiles;
-  if (ti >= prm.bias_total + 2 * kHead + 4) return;
+  if (ti >= small_low(prm.bias_total)) return;
   float v = 0.0f;
   if (ti < prm.bias_total) {
     int l = 0;
     while (l + 1 < prm.layers && ti >= prm.layer[l + 1].bias0) ++l;
     const SmallLayer &L = prm.layer[l];
     const int c = ti - L.bias0;
-    if (c < L.cout && prm.conv_b[l] != nullptr) v = prm.conv_b[l][(size_t)g * L.cout + c];
+    double b = 0.0;
+    if (c < L.cout && prm.conv_b[l] != nullptr) b = small_scale<A>(prm.conv_b[l][(size_t)g * L.cout + c], true);
+    v = (float)b;
+    tail[small_low(prm.bias_total) + ti] = small_scaled<A>() ? small_rest(b, v) : 0.0f;
   } else {
     const int h = ti - prm.bias_total;
     const int c = h < kHead ? h : h - kHead;
@@ -516,18 +617,22 @@ static int small_arith(int prec) {
 static int small_weight_planes(int arith) { return arith == kSmallF32 ? 3 : 1; }
 static int small_act_planes(int arith) { return arith == kSmallF32 || arith == kSmallW16 ? 3 : 1; }
 
+// p / d as the high half of p * small_magic(d), for p * d < 2^32 (d = 1: p itself, see small_div)
+static unsigned small_magic(int d) { return d == 1 ? 0 : (unsigned)((0x100000000ull + d - 1) / d); }
+
 struct SmallPlan {
   SmallLayer layer[kSmallMaxLayers];
   int frags = 0, bias_total = 0, entries = 0, boardb = 0;
   size_t tail = 0, bytes = 0;
 };
 
-static int small_lds(const SmallPlan &pl, int nn, int nb, int *table_off, int *pix_off, int *val_off) {
+static int small_lds(const SmallPlan &pl, int nn, int nb, SmallParams *sp = nullptr) {
   const int t = (nb * pl.boardb + 15) & ~15;
   const int p = (t + 2 * pl.entries + 15) & ~15;
   const int v = p + 4 * nb * nn;
-  if (table_off) *table_off = t, *pix_off = p, *val_off = v;
-  return v + 4 * nb * nn;
+  const int w = (v + 4 * nb * nn + 15) & ~15, floats = (int)((pl.bytes - pl.tail) / 4);
+  if (sp) sp->table_off = t, sp->pix_off = p, sp->val_off = v, sp->tail_off = w, sp->tail_floats = floats;
+  return w + 4 * floats;
 }
 
 // The layout of a network, or false where one board does not fit: more than 48 channels (a wave
@@ -550,7 +655,9 @@ static bool small_plan(int n, int layers, const int *kernels, const int *channel
     L.frag0 = pl.frags;
     L.bias0 = pl.bias_total;
     L.pitch = n + L.r;
-    L.pitch_magic = (unsigned)((0x100000000ull + L.pitch - 1) / L.pitch);
+    L.pitch_magic = small_magic(L.pitch);
+    L.k_magic = small_magic(L.k);
+    L.cb_magic = small_magic(L.cb);
     L.positions = (n + 2 * L.r) * L.pitch + L.r;
     L.planeb = 16 * L.cb;
     // (an odd number of 16-byte units: sixteen consecutive squares then read sixteen bank groups)
@@ -565,8 +672,8 @@ static bool small_plan(int n, int layers, const int *kernels, const int *channel
     cin = L.cout;
   }
   pl.tail = (size_t)pl.frags * 1024;
-  pl.bytes = pl.tail + (size_t)(pl.bias_total + 2 * 16 * kSmallMaxTiles + 4) * 4;
-  return small_lds(pl, n * n, 1, nullptr, nullptr, nullptr) <= kSmallLds;
+  pl.bytes = pl.tail + (size_t)(small_low(pl.bias_total) + pl.bias_total) * 4;
+  return small_lds(pl, n * n, 1) <= kSmallLds;
 }
 
 size_t small_packed_bytes(int n, int layers, const int *kernels, const int *channels, int prec) {
@@ -608,7 +715,7 @@ int launch_small_pack(long long groups, int n, int layers, const int *kernels, c
   pp.frags = pl.frags / small_weight_planes(arith);
   pp.bias_total = pl.bias_total;
   pp.channels = channels[layers - 1];
-  const long long items = (long long)pp.frags * 64 + pl.bias_total + 2 * 16 * kSmallMaxTiles + 4;
+  const long long items = (long long)pp.frags * 64 + small_low(pl.bias_total);
   const dim3 grid((unsigned)((items + 255) / 256), (unsigned)groups);
   switch (arith) {
     case kSmallF32: hipLaunchKernelGGL((small_pack_kernel<SmallArith<3, 3, false>>), grid, dim3(256), 0, st, pp); break;
@@ -656,7 +763,7 @@ int launch_small(const void *x, int x_dtype, long long groups, long long per_gro
   // where that would leave CUs without a workgroup, one board at least
   long long nb = 4 * span / nn;
   if (nb > per_group) nb = per_group;
-  while (nb > 1 && (groups * ((per_group + nb - 1) / nb) < 256 || small_lds(pl, nn, (int)nb, nullptr, nullptr, nullptr) > kSmallLds / 2))
+  while (nb > 1 && (groups * ((per_group + nb - 1) / nb) < 256 || small_lds(pl, nn, (int)nb) > kSmallLds / 2))
     --nb;
   if (nb < 1) nb = 1;
   SmallParams sp;
@@ -669,6 +776,8 @@ int launch_small(const void *x, int x_dtype, long long groups, long long per_gro
   sp.tail = pl.tail;
   sp.n = n;
   sp.nn = nn;
+  sp.n_magic = small_magic(n);
+  sp.nn_magic = small_magic(nn);
   sp.layers = layers;
   sp.nb = (int)nb;
   sp.bias_total = pl.bias_total;
@@ -686,7 +795,7 @@ int launch_small(const void *x, int x_dtype, long long groups, long long per_gro
   sp.pol_b = pol_b;
   sp.val_w = val_w;
   sp.val_b = val_b;
-  const int lds = small_lds(pl, nn, (int)nb, &sp.table_off, &sp.pix_off, &sp.val_off);
+  const int lds = small_lds(pl, nn, (int)nb, &sp);
   const int waves = (int)((nb * nn + span - 1) / span);
   const long long grid = groups * sp.wgs_per_group;
   if (grid > 0x7fffffffLL) {

@@ -181,6 +181,24 @@ def test_parameters_are_read_on_every_call(cuda, precision):
             assert torch.equal(out, model(x)[0]), factor
 
 
+@pytest.mark.parametrize("board,kernels,channels,batch", [(5, [3, 3], [8, 17], 3), (9, [5, 3, 3], [16, 32, 48], 70), (19, [7, 1], [33, 8], 9)])
+@pytest.mark.parametrize("prec", [_lib.PREC_F32, _lib.PREC_BF16, _lib.PREC_BF16F6])
+def test_weights_packed_into_the_workspace_or_read_as_they_are(cuda, board, kernels, channels, batch, prec):
+    """The same bits; inputs that are exact in bf16 and inputs that are not, one of them in a batch of the other."""
+    st = {k: v.to(cuda) for k, v in R.init_state(9, "torch_default", kernels=kernels, channels=channels).items()}
+    x = _inputs(batch, board, 8)
+    x[:, 2] = 1.0
+    for inexact in (False, True):
+        if inexact:
+            x[batch // 2, 1] *= 0.3
+        with torch.inference_mode():
+            packed = run_forward_generic(x.to(cuda), st, kernels, channels, prec)
+            raw = run_forward_generic(x.to(cuda), st, kernels, channels, prec, static_workspace=True)
+            alone = run_forward_generic(x[:1].to(cuda), st, kernels, channels, prec)
+        assert torch.equal(packed[0], raw[0]) and torch.equal(packed[1], raw[1])
+        assert torch.equal(packed[0][:1], alone[0]) and torch.equal(packed[1][:1], alone[1])
+
+
 def test_board_size_set_after_construction(cuda):
     """The network is fully convolutional: the same module on boards of another size."""
     for kernels, channels, first, second in ((None, None, 19, 9), ([3, 3], [8, 16], 7, 13)):

@@ -2378,7 +2378,7 @@ static int second_mode(int cascade) { return cascade == C6_PREC_BF16C ? C6_PREC_
 // 549 / 553, 3,000 (153) 752 / 757, 1,000 (110) 335 / 337.
 
 // Boards of a batch that are shared between workgroups: all where they are few; behind whole rounds of one
-// workgroup per CU the rest (fp32: 257 boards 607 -> 373 us, 341 boards 607 -> 450 us, 777 boards 1,190 ->
+// workgroup per CU the rest (fp32: 257 boards 607 -> 373 us, 341 boards 607 -> 450 us, 384 boards 600 -> 531 us, 777 boards 1,190 ->
 // 975 us; bf16 + fp6 + low weights, 298 boards: 239 -> 191 us).  Not in the modes that put two workgroups on a
 // CU: 9 boards more than three rounds are half a round there.
 static long long team_boards(int prec, long long boards, int cus) {

@@ -1,7 +1,7 @@
 // Few boards: a TEAM of workgroups per board (included by c6_forward.hip).
 //
 // One workgroup per board leaves most of the chip idle when there are fewer boards than CUs, and one
-// board takes as long as 256.  Here 12, 6 or 3 workgroups share a board: each takes one, two or four
+// board takes as long as 256.  Here 12, 6, 3 or 2 workgroups share a board: each takes one, two, four or six
 // of the twelve tiles of 32 squares through all layers, its waves dividing tiles and output channels
 // between them.  A workgroup's own activations stay in its LDS; what a 3x3 layer reads beyond them,
 // twenty squares on either side, goes through memory: the owner stores its squares, waits until the
@@ -60,15 +60,15 @@ template <class P> struct TeamGeo {
   // value sums: SPLIT one per (cout tile, tile of squares), else nine per lane of each tile of squares
   static constexpr int VAL_OFF = HEAD_OFF + 3 * 384 * 4;
   static constexpr int BOARDB = (VAL_OFF + 12 * 9 * 64 * 4 + 255) & ~255;
-  // LDS: up to 11 rows of positions (128 squares lie in at most 8 board rows)
-  static constexpr int REGION = (11 * kPitch + 1) * RECB;
+  // LDS: up to 11 rows of positions (128 squares lie in at most 8 board rows), 13 for 192 squares (SPLIT; in 11)
+  static constexpr int REGION = ((SPLIT ? 13 : 11) * kPitch + 1) * RECB;
   static constexpr int BUF = REGION > G::COPIES_BYTES ? REGION : G::COPIES_BYTES;
   static constexpr int OCC_OFF = (BUF + 15) & ~15;
   static constexpr int LGT_OFF = OCC_OFF + 384;
   static constexpr int RED_OFF = LGT_OFF + 1456;
   static constexpr int RUNS_OFF = RED_OFF + 256 * 4;
   // a copy of the packed set's biases and head weights: no layer starts behind the latency of their loads
-  static constexpr int TAIL_OFF = (RUNS_OFF + (kCascadeMaxRuns + 4) * 4 + 15) & ~15;
+  static constexpr int TAIL_OFF = (RUNS_OFF + (P::LO6 ? (kCascadeMaxRuns + 4) * 4 : 0) + 15) & ~15;
   static constexpr int LDS_BYTES = TAIL_OFF + G::TAIL_FLOATS * 4;
   static_assert(RECB / 16 % 2 == 1 && LDS_BYTES <= 160 * 1024, "LDS map");
 };
@@ -79,9 +79,11 @@ template <class P> struct TeamGeo {
 // by two; with one tile of squares per wave it would be twice as many, 96 and 128 bytes a cycle where the L1
 // gives 64 (six workgroups, 22 to 42 boards, bf16 + fp6 62.6 -> 55 us).  (fp32 contracts a weight with three
 // parts: there the L1 keeps up, and all four waves have work in layers of two cout tiles.)
+// Three or six tiles of squares go to three waves, all cout tiles in each; the fourth watches the flags.
 template <class P, int TEAM> struct TeamShape {
-  static constexpr int PXT = 12 / TEAM, PT = PXT > 1 && !TeamGeo<P>::SPLIT ? 2 : 1;
-  static constexpr int PG = PXT / PT, CG = PG == 1 ? (PXT == 1 ? 3 : 4) : 4 / PG;   // groups of squares' tiles, of cout tiles
+  static constexpr int PXT = 12 / TEAM;
+  static constexpr int PT = PXT == 6 ? 2 : (PXT % 2 == 0 && !TeamGeo<P>::SPLIT ? 2 : 1), PG = PXT / PT;
+  static constexpr int CG = PG == 3 ? 1 : (PG == 1 ? (PXT == 1 ? 3 : 4) : 4 / PG);   // groups of squares' tiles, of cout tiles
   static constexpr int tiles(int nt) { return (nt + CG - 1) / CG; }   // cout tiles of a wave
 };
 
@@ -196,24 +198,36 @@ __device__ __forceinline__ void team_conv(const unsigned char *smem, const unsig
       for (int p = 0; p < PT; ++p)
 #pragma unroll
         for (int i = 0; i < NPL; ++i) a[(v + 2) % 3][p][i] = frag(rn, (v + 2) % U, p, i);
-#pragma unroll
-      for (int t = 0; t < TT; ++t) {
-        if constexpr (NPL == 3) {
-          constexpr int WP[6] = {0, 1, 2, 0, 1, 0}, AP[6] = {2, 1, 0, 1, 0, 0};
-#pragma unroll
-          for (int p = 0; p < PT; ++p)
-#pragma unroll
-            for (int m = 0; m < 6; ++m) mma<P>(ring[v % D][t][WP[m]], a[v % 3][p][AP[m]], m < 5 ? low[p][t] : acc[p][t]);
-        } else {
-#pragma unroll
-          for (int i = 0; i < W; ++i)
-#pragma unroll
-            for (int p = 0; p < PT; ++p) mma<P>(ring[v % D][t][i], a[v % 3][p][0], acc[p][t]);
-        }
+      auto refill = [&](int t) __attribute__((always_inline)) {
         const int kn = r * U + v + D;   // (behind the last k-steps: the last one again, unused)
         const int f = team_frag<P, L>(kn < KS ? kn : KS - 1, t0 + t < NT ? t0 + t : NT - 1);
 #pragma unroll
         for (int i = 0; i < W; ++i) ring[v % D][t][i] = wl[f + i];
+      };
+      if constexpr (NPL == 3) {
+        // (An accumulator's next MFMA is eight cycles late if it follows at once, so two tiles take turns: forty boards
+        // 102 -> 97 us.  With three the L1's 64 bytes a cycle bound the layer, and loads in a row per tile suit it better:
+        // 56 boards 120 us, in turns 123.)
+        constexpr int WP[6] = {0, 1, 2, 0, 1, 0}, AP[6] = {2, 1, 0, 1, 0, 0};
+        constexpr bool TURNS = TT == 2;
+#pragma unroll
+        for (int o = 0; o < (TURNS ? 6 : TT); ++o)
+#pragma unroll
+          for (int n = 0; n < (TURNS ? TT : 6); ++n) {
+            const int m = TURNS ? o : n, t = TURNS ? n : o;
+#pragma unroll
+            for (int p = 0; p < PT; ++p) mma<P>(ring[v % D][t][WP[m]], a[v % 3][p][AP[m]], m < 5 ? low[p][t] : acc[p][t]);
+            if (m == 5) refill(t);
+          }
+      } else {
+#pragma unroll
+        for (int t = 0; t < TT; ++t) {
+#pragma unroll
+          for (int i = 0; i < W; ++i)
+#pragma unroll
+            for (int p = 0; p < PT; ++p) mma<P>(ring[v % D][t][i], a[v % 3][p][0], acc[p][t]);
+          refill(t);
+        }
       }
       __builtin_amdgcn_sched_barrier(0);
     });
@@ -365,7 +379,7 @@ __device__ __forceinline__ void team_board(const TeamParams &prm, unsigned char 
   int unfinished = -1;   // word of the piece whose inner squares are still being stored
   // Are the inputs of stage l there for `role` (`own`: its own squares are in LDS)?  Bounded; the answer
   // is the same in every thread.  1: yes, 0: no, 2: no need, the stage itself has been done.
-  constexpr int kWatch = CG == 3 ? 3 : 0;   // the wave that watches the flags: one that has no weights to wait for
+  constexpr int kWatch = S::PG * CG == 3 ? 3 : 0;   // the wave that watches the flags: one that has no weights to wait for
   auto wait_inputs = [&](int l, int role, bool own) {
     if (wave == kWatch) {
       // (the words of the first layer's workgroups have been there since they started)
@@ -569,27 +583,35 @@ __device__ __forceinline__ void team_board(const TeamParams &prm, unsigned char 
       const float *pw = tail + kBiasTotal + 4 * h;
       const int tile = role * PXT + wpx;   // of the twelve
       if constexpr (T::SPLIT) {
-        static_assert(PT == 1, "one tile of squares per wave");
         if (active) {
 #pragma unroll
           for (int t = 0; t < TT; ++t) {
             if (t0 + t >= NT) continue;
-            float pol = 0.0f, val = 0.0f;
+            float pol[PT], val[PT];
+#pragma unroll
+            for (int i = 0; i < PT; ++i) pol[i] = val[i] = 0.0f;
 #pragma unroll
             for (int q = 0; q < 4; ++q)
 #pragma unroll
               for (int e = 0; e < 4; ++e) {
-                const float a = split_silu(acc[0][t][4 * q + e]);
-                pol = fmaf(a, pw[32 * (t0 + t) + 8 * q + e], pol);
-                val = fmaf(a, pw[kHeadC + 32 * (t0 + t) + 8 * q + e], val);
+                const float p1 = pw[32 * (t0 + t) + 8 * q + e], v1 = pw[kHeadC + 32 * (t0 + t) + 8 * q + e];
+#pragma unroll
+                for (int i = 0; i < PT; ++i) {
+                  const float a = split_silu(acc[i][t][4 * q + e]);
+                  pol[i] = fmaf(a, p1, pol[i]);
+                  val[i] = fmaf(a, v1, val[i]);
+                }
               }
-            const unsigned bits = __builtin_bit_cast(unsigned, pol);
-            const auto x = __builtin_amdgcn_permlane32_swap(bits, bits, false, false);
-            const unsigned x0 = x[0], x1 = x[1];
-            const float tot = __builtin_bit_cast(float, x0) + __builtin_bit_cast(float, x1);
-            const float vs = wave_sum(ok[0] ? val : 0.0f);
-            if (h == 0 && ok[0]) store4(tot, T::HEAD_OFF + ((t0 + t) * 384 + p[0]) * 4);
-            if (lane == 0) store4(vs, T::VAL_OFF + ((t0 + t) * 12 + tile) * 4);
+#pragma unroll
+            for (int i = 0; i < PT; ++i) {
+              const unsigned bits = __builtin_bit_cast(unsigned, pol[i]);
+              const auto x = __builtin_amdgcn_permlane32_swap(bits, bits, false, false);
+              const unsigned x0 = x[0], x1 = x[1];
+              const float tot = __builtin_bit_cast(float, x0) + __builtin_bit_cast(float, x1);
+              const float vs = wave_sum(ok[i] ? val[i] : 0.0f);
+              if (h == 0 && ok[i]) store4(tot, T::HEAD_OFF + ((t0 + t) * 384 + p[i]) * 4);
+              if (lane == 0) store4(vs, T::VAL_OFF + ((t0 + t) * 12 + tile + i) * 4);
+            }
           }
         }
       } else {
@@ -662,21 +684,22 @@ __device__ __forceinline__ void team_board(const TeamParams &prm, unsigned char 
   auto first_stage = [&](int role) __attribute__((always_inline)) -> bool {
     const Span sp = span_of(role);
     int *flag = reinterpret_cast<int *>(red) + 64;   // [0]: third plane varies, [1]: an input is not exact in bf16
-    const int px = PXT == 4 ? wave : (PXT == 2 ? wave & 1 : 0);   // (one cout tile: a wave per tile of squares)
-    const int p = sp.p0 + px * 32 + (lane & 31);
-    const int pc = p < kPix ? p : kPix - 1, r = pc / kBoard, c = pc - r * kBoard;
-    const bool active = wave < PXT;
+    constexpr int N1 = PXT > 4 ? 2 : 1;   // (one cout tile: a wave per tile of squares, or per two)
+    const int px = wave * N1 < PXT ? wave * N1 : 0;
+    const bool active = wave * N1 < PXT;
     region_role = -1;
-    f32x16 one[1][1];
-    f32x16 (&acc)[1] = one[0];
+    f32x16 acc[N1][1];
     if (active) {
       // (the table holds the squares as the one-workgroup kernels' lanes do: by tile of 32)
-      const WFrags tb = packed_frags<P>(packed, lane, G::PLANE2_FRAG_OFF + (role * PXT + px) * 4);
 #pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        const f32x4 t4 = __builtin_bit_cast(f32x4, tb[q]);
+      for (int n = 0; n < N1; ++n) {
+        const WFrags tb = packed_frags<P>(packed, lane, G::PLANE2_FRAG_OFF + (role * PXT + px + n) * 4);
 #pragma unroll
-        for (int e = 0; e < 4; ++e) acc[0][4 * q + e] = t4[e];
+        for (int q = 0; q < 4; ++q) {
+          const f32x4 t4 = __builtin_bit_cast(f32x4, tb[q]);
+#pragma unroll
+          for (int e = 0; e < 4; ++e) acc[n][0][4 * q + e] = t4[e];
+        }
       }
     }
     constexpr int TAIL_UNITS = (G::TAIL_FLOATS / 4 + THREADS - 1) / THREADS;
@@ -745,22 +768,33 @@ __device__ __forceinline__ void team_board(const TeamParams &prm, unsigned char 
       __syncthreads();
       parts = flag[1] != 0 ? 3 : 1;
     }
-    const int sh = c % G::E;
-    const int l1 = sh * G::COPY_BYTES + (r * 3 * kL1RowPitch + (c - sh)) * G::EB;
     const int rows = (plane2_varies ? G::STEPS1 : G::FAST1_STEPS) / 3;
-    const int row0 = l1 + (plane2_varies ? kL1RowsHalf : 1) * h * kL1RowPitch * G::EB;
+    int row0[N1];
+#pragma unroll
+    for (int n = 0; n < N1; ++n) {
+      const int p = sp.p0 + (px + n) * 32 + (lane & 31);
+      const int pc = p < kPix ? p : kPix - 1, r = pc / kBoard, c = pc - r * kBoard, sh = c % G::E;
+      row0[n] = sh * G::COPY_BYTES + (r * 3 * kL1RowPitch + (c - sh)) * G::EB + (plane2_varies ? kL1RowsHalf : 1) * h * kL1RowPitch * G::EB;
+    }
     const int rowb = (plane2_varies ? 1 : 3) * kL1RowPitch * G::EB;
     const WFrags wl = plane2_varies ? layer_weights<P, 0>(packed, lane) : packed_frags<P>(packed, lane, G::FAST1_OFF);
     if (active) {
       const f32x16 b0 = tail_tile(bias_offset(0));
 #pragma unroll
-      for (int i = 0; i < 16; ++i) acc[0][i] = plane2_varies ? b0[i] : fmaf(c2, acc[0][i], b0[i]);
-    }
-    f32x16 low, large;   // SPLIT: small products; the large ones, once all parts but the first follow
+      for (int n = 0; n < N1; ++n)
 #pragma unroll
-    for (int i = 0; i < 16; ++i) low[i] = large[i] = 0.0f;
+        for (int i = 0; i < 16; ++i) acc[n][0][i] = plane2_varies ? b0[i] : fmaf(c2, acc[n][0][i], b0[i]);
+    }
+    f32x16 low[N1], large[N1];   // SPLIT: small products; the large ones, once all parts but the first follow
+#pragma unroll
+    for (int n = 0; n < N1; ++n)
+#pragma unroll
+      for (int i = 0; i < 16; ++i) low[n][i] = large[n][i] = 0.0f;
     if constexpr (T::SPLIT) {
-      if (active) low = tail_tile(G::TAIL_BIAS_LOW + bias_offset(0));
+      if (active) {
+#pragma unroll
+        for (int n = 0; n < N1; ++n) low[n] = tail_tile(G::TAIL_BIAS_LOW + bias_offset(0));
+      }
     }
 #pragma unroll 1
     for (int part = 0; part < parts; ++part) {
@@ -795,12 +829,12 @@ __device__ __forceinline__ void team_board(const TeamParams &prm, unsigned char 
         // the matrix core waits for (all of a row's loads in front of it: bf16 54 cycles per MFMA, fp32 58).
         constexpr int DW = W == 3 ? 4 : 8;
         static_assert(DW % 2 == 0, "activations alternate");
-        v4i w[DW][3][W], a[2][3];
+        v4i w[DW][3][W], a[2][3][N1];
         auto weight = [&](int row, int i, int j) __attribute__((always_inline)) {
           return wl[((row < rows ? row : rows - 1) * 3 + i) * W + j];
         };
-        auto activation = [&](int row, int i) __attribute__((always_inline)) {
-          return *reinterpret_cast<const v4i *>(smem + row0 + (row < rows ? row : rows - 1) * rowb + i * 16);
+        auto activation = [&](int row, int i, int n) __attribute__((always_inline)) {
+          return *reinterpret_cast<const v4i *>(smem + row0[n] + (row < rows ? row : rows - 1) * rowb + i * 16);
         };
         auto one_row = [&](int row, auto sc) __attribute__((always_inline)) {
           constexpr int s8 = decltype(sc)::value;
@@ -808,16 +842,18 @@ __device__ __forceinline__ void team_board(const TeamParams &prm, unsigned char 
           for (int i = 0; i < 3; ++i) {
             static_for<0, W>([&](auto jc) __attribute__((always_inline)) {
               constexpr int j = decltype(jc)::value;
-              mma<P>(w[s8][i][j], a[s8 % 2][i], T::SPLIT && j > 0 ? low : acc[0]);
+#pragma unroll
+              for (int n = 0; n < N1; ++n) mma<P>(w[s8][i][j], a[s8 % 2][i][n], T::SPLIT && j > 0 ? low[n] : acc[n][0]);
               w[s8][i][j] = weight(row + DW, i, j);
             });
-            a[(s8 + 1) % 2][i] = activation(row + 1, i);
+#pragma unroll
+            for (int n = 0; n < N1; ++n) a[(s8 + 1) % 2][i][n] = activation(row + 1, i, n);
           }
 #pragma unroll
           for (int i = 0; i < 3 * W; ++i) {
-            __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);                    // one MFMA
-            __builtin_amdgcn_sched_group_barrier(0x020, 1, 0);                    // one weight
-            if (i % W == W - 1) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);   // one LDS read
+            __builtin_amdgcn_sched_group_barrier(0x008, N1, 0);                    // one MFMA per tile
+            __builtin_amdgcn_sched_group_barrier(0x020, 1, 0);                     // one weight
+            if (i % W == W - 1) __builtin_amdgcn_sched_group_barrier(0x100, N1, 0);   // one LDS read per tile
           }
           __builtin_amdgcn_sched_barrier(0);
         };
@@ -827,7 +863,9 @@ __device__ __forceinline__ void team_board(const TeamParams &prm, unsigned char 
           for (int i = 0; i < 3; ++i) {
 #pragma unroll
             for (int j = 0; j < W; ++j) w[s8][i][j] = weight(s8, i, j);
-            if (s8 == 0) a[0][i] = activation(0, i);
+            if (s8 == 0)
+#pragma unroll
+              for (int n = 0; n < N1; ++n) a[0][i][n] = activation(0, i, n);
           }
         int row = 0;
 #pragma unroll 1
@@ -837,22 +875,28 @@ __device__ __forceinline__ void team_board(const TeamParams &prm, unsigned char 
         });
         if constexpr (T::SPLIT) {
           if (parts > 1 && part == 0) {
-            large = acc[0];
-            acc[0] = low;
 #pragma unroll
-            for (int i = 0; i < 16; ++i) low[i] = 0.0f;
+            for (int n = 0; n < N1; ++n) {
+              large[n] = acc[n][0];
+              acc[n][0] = low[n];
+#pragma unroll
+              for (int i = 0; i < 16; ++i) low[n][i] = 0.0f;
+            }
           }
         }
       }
     }
     if constexpr (T::SPLIT) {
 #pragma unroll
-      for (int i = 0; i < 16; ++i) acc[0][i] = parts > 1 ? two_sums(large[i], low[i] + acc[0][i]) : two_sums(acc[0][i], low[i]);
+      for (int n = 0; n < N1; ++n)
+#pragma unroll
+        for (int i = 0; i < 16; ++i)
+          acc[n][0][i] = parts > 1 ? two_sums(large[n][i], low[n][i] + acc[n][0][i]) : two_sums(acc[n][0][i], low[n][i]);
     }
     C6_MARK(2);
     __syncthreads();   // the copies give way to the activations
     clear_region(sp);
-    write_out(IC<0>{}, IC<1>{}, role, sp, active, one, px, 0);
+    write_out(IC<0>{}, IC<N1>{}, role, sp, active, acc, px, 0);
     C6_MARK(3);
     return true;
   };
@@ -993,23 +1037,31 @@ __device__ __forceinline__ void team_board(const TeamParams &prm, unsigned char 
   __syncthreads();
 }
 
-// How many workgroups share a board when there are `boards` of them: as many as fit the chip at once, where
+// How many workgroups share a board (team_size, below) when there are `boards` of them: as many as fit the chip at once, where
 // that beats one workgroup (1: the one-workgroup kernels).  With fewer workgroups per board more waves read
-// the same weights, and the L1's 64 bytes a cycle bound the layers: measured, 20 / 40 / 80 boards against
-// one workgroup each, fp32 69 / 95 / 135 us against 225, bf16 + fp6 + low weights 52 / 67 / 92 against 90 (60
-// boards 83, so three workgroups take up to 73 of 256 CUs; behind a first pass, 53 listed boards, 85 us against
-// 110), bf16 + fp6 45 / 55 / 79 against 63, plain bf16 44 us (20 boards) against 46.
+// the same weights, and the L1's 64 bytes a cycle bound the layers; the 16-bit one-workgroup kernel hides its epilogues
+// behind its MFMAs, which a team does not.  Measured, us, teams of 12 / 6 / 3 / 2 against one workgroup each, boards:
+//   fp32  16: 66 / 82 / 110 / 178 / 223   40: 97 / 116 / 181 / 224   80: 132 / 185 / 224   128: 203 / 230
+//   bf16  16: 31 / 41 / 49 / 61 / 45      21: 36 / 41 / - / - / 46   40: 42 / 50 / 61 / 45   42: 48 (teams on two XCDs)
+//   bf16 + fp6  21: 44 / 51 / 64 / 81 / 63    42: 57 / 68 / 84 / 64    with low weights  21: 52 / 60 / 78 / 101 / 89
+//   42: 67 / 84 / 106 / 89    72: 89 / 110 / 89 (behind a first pass, 53 listed boards, 85 against 110)
+// Four workgroups per board are never the best of these by more than 4 %.
+//
+// The most boards that teams of a size take:
+template <class P> __host__ __device__ inline long long team_most(int wgs, int size) {
+  if (size == 6 && !TeamGeo<P>::SPLIT && !P::LO6) return wgs * 5 / 32;   // (where all teams have an XCD to themselves)
+  if (size == 3 && P::WLO == 1) return wgs * 2 / 7;
+  return wgs / size;
+}
+template <class P> constexpr int team_least() { return TeamGeo<P>::SPLIT ? 2 : (P::WLO ? 3 : 6); }
 template <class P> __host__ __device__ inline int team_size(long long boards, int wgs) {
-  if (boards * 12 <= wgs) return 12;
-  if ((TeamGeo<P>::SPLIT || P::LO6) && boards * 6 <= wgs) return 6;
-  if (TeamGeo<P>::SPLIT) return boards * 3 <= wgs ? 3 : 1;
-  return P::WLO && boards * 7 <= wgs * 2 ? 3 : 1;
+  const int sizes[4] = {12, 6, 3, 2};
+  for (int i = 0; i < 4; ++i)
+    if (sizes[i] >= team_least<P>() && boards <= team_most<P>(wgs, sizes[i])) return sizes[i];
+  return 1;
 }
-// ... and the most boards that are shared at all
-template <class P> inline long long team_most(int wgs) {
-  if (TeamGeo<P>::SPLIT) return wgs / 3;
-  return P::WLO ? wgs * 2 / 7 : wgs / (P::LO6 ? 6 : 12);
-}
+
+template <class P> inline long long team_most(int wgs) { return team_most<P>(wgs, team_least<P>()); }
 
 template <class P> __global__ __launch_bounds__(256) void team_forward_kernel(const TeamParams prm) {
   using T = TeamGeo<P>;
@@ -1070,11 +1122,12 @@ template <class P> __global__ __launch_bounds__(256) void team_forward_kernel(co
     b = (unsigned)prm.f.redo_list[(size_t)lo * prm.f.redo_per + (item - (unsigned)runs[lo])];
   }
   if (team == 12) team_board<P, 12>(prm, smem, b, slot, role);
-  if constexpr (TeamGeo<P>::SPLIT || P::LO6) {
-    if (team == 6) team_board<P, 6>(prm, smem, b, slot, role);
-  }
-  if constexpr (TeamGeo<P>::SPLIT || P::WLO) {
+  if (team == 6) team_board<P, 6>(prm, smem, b, slot, role);
+  if constexpr (team_least<P>() <= 3) {
     if (team == 3) team_board<P, 3>(prm, smem, b, slot, role);
+  }
+  if constexpr (team_least<P>() <= 2) {
+    if (team == 2) team_board<P, 2>(prm, smem, b, slot, role);
   }
 }
 

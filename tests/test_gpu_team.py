@@ -130,6 +130,25 @@ def test_cascade_with_few_listed_boards(cuda, prec):
                     assert int(stats["second_pass"]) == (0 if threshold == 0.0 else n)
 
 
+@pytest.mark.parametrize("prec,sizes", [(_lib.PREC_F32S, (86, 100, 127, 128, 129, 342, 384, 385)), (_lib.PREC_BF16, (22, 40, 41)),
+                                        (_lib.PREC_F16, (23, 39, 40, 41))])
+def test_edges_of_the_smallest_teams(cuda, prec, sizes):
+    model, (x, legal) = _model(cuda), _inputs(385)
+    xd, ld, u = x.to(cuda), legal.to(cuda), gen_uniform(385, 5).to(cuda)
+    packed = model.packed_weights(prec)
+    kw = dict(mask_mode=_lib.MASK_LEGAL, temperature=0.8, want_logprob=True)
+    with torch.inference_mode():
+        # (200 boards: one workgroup each)
+        want = [torch.cat(t) for t in zip(*[run_forward(xd[a:a + 200], packed, prec, 1, 200, legal=ld[a:a + 200], u=u[a:a + 200], **kw)
+                                            for a in (0, 185)])]
+        want = [torch.cat([t[:185], t[200:]]) for t in want]
+        for n in sizes:
+            for a in (0, 385 - n):
+                got = run_forward(xd[a:a + n], packed, prec, 1, n, legal=ld[a:a + n], u=u[a:a + n], **kw)
+                for p, q in zip(got, want):
+                    assert torch.equal(p, q[a:a + n]), (n, a)
+
+
 def test_boards_states_views_and_index(cuda):
     model, (x, _) = _model(cuda), gen_boards(300, 200, 5)
     boards = (x[:, 0] - x[:, 1]).to(torch.int8).to(cuda)

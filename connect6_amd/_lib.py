@@ -20,6 +20,7 @@ _LIBDIR = _PKG / "lib"
 _SO = _LIBDIR / "libconnect6_amd.so"
 _SOURCES = ("c6_forward.hip", "c6_tail.hip", "c6_generic.hip", "c6_small.hip", "c6_env.hip", "c6_api.hip")
 _MODES = ("PrecF32", "PrecF32S", "PrecBF16", "PrecF16", "PrecBF16F6", "PrecBF16F6W")   # of c6_forward.hip
+_SECOND_PASSES = ("PrecBF16F6", "PrecBF16F6W")   # modes of a cascade's second pass
 _RESOURCES = _LIBDIR / "resource_usage.txt"   # registers, scratch and LDS of every kernel, written by build()
 
 # arithmetic modes (include/connect6_amd.h)
@@ -90,6 +91,7 @@ def build(verbose: bool = False) -> Path:
     units = [(s, ["-DC6_SPLIT"] if s == "c6_forward.hip" else []) for s in _SOURCES]
     units = [("c6_forward.hip", [f"-DC6_INSTANCE={m}"] + team) for team in (["-DC6_TEAM"], []) for m in _MODES
              if not (team and m == "PrecF32")] + units
+    units = [("c6_forward.hip", [f"-DC6_INSTANCE={m}", "-DC6_CASCADE"]) for m in _SECOND_PASSES] + units
     with tempfile.TemporaryDirectory(dir=_LIBDIR) as tmp:
         objs = [str(Path(tmp) / f"{i}.o") for i in range(len(units))]
 

@@ -1919,7 +1919,7 @@ __global__ __launch_bounds__(256) void fused_forward_kernel(const FwdParams prm)
 
 #include "c6_split.h"
 #include "c6_duo.h"
-#if defined(C6_TEAM) || !defined(C6_INSTANCE)
+#if defined(C6_TEAM) || defined(C6_CASCADE) || !defined(C6_INSTANCE)
 #include "c6_team.h"
 #endif
 
@@ -2179,11 +2179,13 @@ template <class P> __global__ __launch_bounds__(256) void lo_scale_kernel(const 
 // ------------------------------------------------------------------------
 // The library is built with two object files per arithmetic mode (the compiler takes a minute and
 // more for each): C6_INSTANCE names the mode of this object file, C6_TEAM marks the one that holds its
-// team kernel, C6_SPLIT the one that holds the dispatch.  Without either, this file is all of them (what a traced copy is built from).
+// team kernel, C6_CASCADE the one that holds it as second pass of team_cascade_kernel, C6_SPLIT the one that holds the
+// dispatch.  Without either, this file is all of them (what a traced copy is built from).
 template <class P> int launch_pack(const PackParams &pp, hipStream_t st);
 template <class P> int launch_forward(const FwdParams &fp, hipStream_t st);
 
 template <class P> int launch_team(const TeamParams &tp, int grid, hipStream_t st);
+template <class P> int launch_team_cascade(const TeamCascadeParams &tp, int grid, hipStream_t st);
 
 #ifndef C6_SPLIT
 template <class P> int launch_pack(const PackParams &pp, hipStream_t st) {
@@ -2258,7 +2260,7 @@ template <class P> int launch_forward(const FwdParams &fp, hipStream_t st) {
   return C6_OK;
 }
 
-#if defined(C6_TEAM) || !defined(C6_INSTANCE)
+#if defined(C6_TEAM) || defined(C6_CASCADE) || !defined(C6_INSTANCE)
 template <class P> int launch_team(const TeamParams &tp, int grid, hipStream_t st) {
   using T = TeamGeo<P>;
   static thread_local int configured = -1;
@@ -2279,12 +2281,35 @@ template <class P> int launch_team(const TeamParams &tp, int grid, hipStream_t s
   }
   return C6_OK;
 }
+
+template <class P> int launch_team_cascade(const TeamCascadeParams &tp, int grid, hipStream_t st) {
+  constexpr int A = TeamGeo<PrecBF16>::LDS_BYTES, B = TeamGeo<P>::LDS_BYTES, LDS = A > B ? A : B;
+  static thread_local int configured = -1;
+  int dev = 0;
+  hipError_t e = hipGetDevice(&dev);
+  if (e == hipSuccess && configured != dev) {
+    e = hipFuncSetAttribute(reinterpret_cast<const void *>(&team_cascade_kernel<P>),
+                            hipFuncAttributeMaxDynamicSharedMemorySize, LDS);
+    if (e == hipSuccess) configured = dev;
+  }
+  if (e == hipSuccess) {
+    hipLaunchKernelGGL(team_cascade_kernel<P>, dim3((unsigned)grid), dim3(256), LDS, st, tp);
+    e = hipGetLastError();
+  }
+  if (e != hipSuccess) {
+    set_error("team_cascade launch failed: %s", hipGetErrorString(e));
+    return C6_ELAUNCH;
+  }
+  return C6_OK;
+}
 #endif
 
 #endif  // C6_SPLIT
 
 #ifdef C6_INSTANCE
-#ifdef C6_TEAM
+#if defined(C6_CASCADE)
+template int launch_team_cascade<C6_INSTANCE>(const TeamCascadeParams &, int, hipStream_t);
+#elif defined(C6_TEAM)
 template int launch_team<C6_INSTANCE>(const TeamParams &, int, hipStream_t);
 #else
 template int launch_pack<C6_INSTANCE>(const PackParams &, hipStream_t);
@@ -2372,7 +2397,7 @@ static int second_mode(int cascade) { return cascade == C6_PREC_BF16C ? C6_PREC_
 // The cascade's second pass hands what the listed boards leave beyond whole rounds of the CUs to teams, if it
 // is no more than they take (73 boards of 256 CUs with low weights, 42 without); their launch ends at once where
 // it is more.  How many are listed depends on the network (6 % of random ones' boards, a few of a peaked
-// policy's), not on the batch, so every cascade has that launch.  Measured without / with it, boards (listed)
+// policy's), not on the batch, so every cascade has that launch (21 boards and fewer: team_cascade_kernel).  Measured without / with it, boards (listed)
 // us: 512 (2) 200 / 161, 1,536 (13) 411 / 379, (67) 444 / 415, 2,048 (9) 520 / 485, 4,096 (4) 937 / 903,
 // (218) 958 / 967, 16,384 (19) 3,428 / 3,402; where it serves nothing it costs 3 to 6 us: 2,048 (99)
 // 549 / 553, 3,000 (153) 752 / 757, 1,000 (110) 335 / 337.
@@ -2389,6 +2414,9 @@ static long long team_boards(int prec, long long boards, int cus) {
   return m.rounds && rest <= m.most(cus) ? rest : 0;
 }
 
+// Boards of a cascade whose two passes are one launch: those that twelve workgroups share (team_cascade_kernel)
+static bool team_cascade_fits(long long boards, int cus) { return boards <= 64 && boards * 12 <= cus; }
+
 // Exchange memory of a call on `boards` boards of a mode, and how many boards it is for (0: one workgroup per
 // board serves them all).
 int team_workspace_bytes(int prec, long long boards, size_t *bytes, long long *shared) {
@@ -2398,7 +2426,11 @@ int team_workspace_bytes(int prec, long long boards, size_t *bytes, long long *s
   if (boards < 1) return C6_OK;
   const int rc = device_cus(cus);
   if (rc != C6_OK) return rc;
-  if (is_cascade(prec)) {
+  if (is_cascade(prec) && team_cascade_fits(boards, cus)) {
+    // both passes in one launch, each with exchange memory and flags of its own
+    *shared = 2 * boards;
+    *bytes = (team_mode(C6_PREC_BF16).board_bytes + team_mode(second_mode(prec)).board_bytes) * (size_t)boards;
+  } else if (is_cascade(prec)) {
     const TeamMode first = team_mode(C6_PREC_BF16), second = team_mode(second_mode(prec));
     const long long teams = second.most(cus), before = team_boards(C6_PREC_BF16, boards, cus);
     *shared = boards < teams ? boards : teams;
@@ -2458,6 +2490,14 @@ int dispatch_cascade(int prec, const FwdParams &fp, float threshold, void *works
   second.redo_mode = kRedoConsume;
   if (team == nullptr) {
     rc = launch_forward<PrecBF16>(first, st);
+  } else if (team_cascade_fits(fp.total_boards, cus)) {
+    TeamCascadeParams tp;
+    tp.first = *team;
+    tp.first.f = first;
+    tp.packed = second.packed;
+    tp.act = team->act + team_mode(C6_PREC_BF16).board_bytes * (size_t)fp.total_boards;
+    tp.flags = team->flags + (size_t)fp.total_boards * kTeamFlags;
+    return prec == C6_PREC_BF16C ? launch_team_cascade<PrecBF16F6W>(tp, cus, st) : launch_team_cascade<PrecBF16F6>(tp, cus, st);
   } else {
     TeamParams tp = *team;
     tp.f = first;

@@ -38,7 +38,8 @@ constexpr int kTeamStages = 9;   // eight layers, then the heads' write-out
 constexpr int kTeamAll = 128;    // flag words: see team_board
 constexpr int kSc1 = 16;         // cache policy: device scope
 constexpr int kTeamXcd = kTeamAll + kTeamStages * 12;
-static_assert(kTeamXcd + 12 <= kTeamFlags && kTeamStages * 12 <= kTeamAll, "flag words");
+constexpr int kTeamListed = kTeamXcd + 12, kTeamDone = kTeamListed + 1;   // see team_cascade_kernel
+static_assert(kTeamDone < kTeamFlags && kTeamStages * 12 <= kTeamAll, "flag words");
 
 // modes that have a team kernel
 template <class P> constexpr bool has_team() { return P::ID != C6_PREC_F32; }
@@ -985,8 +986,9 @@ __device__ __forceinline__ void team_board(const TeamParams &prm, unsigned char 
         const bool again = wave_margin_below(
             lane, f.redo_threshold, [&](int i) { return lgt[i]; }, [&](int i) { return (occ[i] & 2) == 0; });
         if (lane == 0) {
-          f.redo_counts[b] = again ? 1 : 0;
+          __hip_atomic_store(&f.redo_counts[b], again ? 1 : 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
           f.redo_list[b] = (int)b;
+          if (again) store_flag(kTeamListed);   // (in front of the stage's flag)
         }
       }
     }
@@ -1063,6 +1065,23 @@ template <class P> __host__ __device__ inline int team_size(long long boards, in
 
 template <class P> inline long long team_most(int wgs) { return team_most<P>(wgs, team_least<P>()); }
 
+// Which team this workgroup belongs to (`items` of them; a slot beyond: to none) and as which member.  A team
+// on one XCD (workgroup i runs on XCD i % 8), neighbouring boards on the same one, where that many teams fit: a weight
+// set then comes into one L2 and not into eight.  (27 listed boards of 128 weight sets: the cascade 183 -> 179 us; of 16
+// sets, 6 boards: 105 -> 96 us; eight fp32 boards of one set 66.5 -> 64.4 us.)
+struct TeamPlace {
+  unsigned slot;
+  int role;
+};
+__device__ __forceinline__ TeamPlace team_place(unsigned items, int team) {
+  if (gridDim.x % 8 == 0) {
+    const unsigned per = (items + 7) / 8, l = blockIdx.x / 8;
+    if (per * (unsigned)team <= gridDim.x / 8)
+      return {l / (unsigned)team < per ? blockIdx.x % 8 * per + l / (unsigned)team : items, (int)(l % (unsigned)team)};
+  }
+  return {blockIdx.x / (unsigned)team, (int)(blockIdx.x % (unsigned)team)};
+}
+
 template <class P> __global__ __launch_bounds__(256) void team_forward_kernel(const TeamParams prm) {
   using T = TeamGeo<P>;
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
@@ -1098,18 +1117,9 @@ template <class P> __global__ __launch_bounds__(256) void team_forward_kernel(co
   if (items == 0) return;
   const int team = team_size<P>(items, (int)gridDim.x);
   if (team == 1) return;
-  unsigned slot = blockIdx.x / (unsigned)team;
-  int role = (int)(blockIdx.x % (unsigned)team);
-  // A team on one XCD (workgroup i runs on XCD i % 8), neighbouring boards on the same one, where that many
-  // teams fit: a weight set then comes into one L2 and not into eight.  (27 listed boards of 128 weight sets:
-  // the cascade 183 -> 179 us; of 16 sets, 6 boards: 105 -> 96 us; eight fp32 boards of one set 66.5 -> 64.4 us.)
-  if (gridDim.x % 8 == 0) {
-    const unsigned per = (items + 7) / 8, l = blockIdx.x / 8;
-    if (per * (unsigned)team <= gridDim.x / 8) {
-      role = (int)(l % (unsigned)team);
-      slot = l / (unsigned)team < per ? blockIdx.x % 8 * per + l / (unsigned)team : items;
-    }
-  }
+  const TeamPlace at = team_place(items, team);
+  const unsigned slot = at.slot;
+  const int role = at.role;
   if (slot >= items) return;
   unsigned b = prm.first + slot;
   if (from_list) {
@@ -1129,6 +1139,63 @@ template <class P> __global__ __launch_bounds__(256) void team_forward_kernel(co
   if constexpr (team_least<P>() <= 2) {
     if (team == 2) team_board<P, 2>(prm, smem, b, slot, role);
   }
+}
+
+// The cascade over so few boards that twelve workgroups share each: both passes in one launch.  Where a board's last
+// stage is done, its team sees whether the board was listed and goes through it again in the second pass's mode, or ends:
+// one board that is not listed 41.4 -> 33.3 us with its mask (the second launch found nothing to do), of which waiting
+// for the verdict is 2.
+//   packed, act, flags: the second pass's
+struct TeamCascadeParams {
+  TeamParams first;
+  const unsigned char *packed;
+  unsigned char *act;
+  unsigned *flags;
+};
+template <class P2> __global__ __launch_bounds__(256) void team_cascade_kernel(const TeamCascadeParams prm) {
+  extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
+  const unsigned items = (unsigned)prm.first.f.total_boards;   // (at most 64)
+  const TeamPlace at = team_place(items, 12);
+  if (at.slot >= items) return;
+  team_board<PrecBF16, 12>(prm.first, smem, at.slot, at.slot, at.role);
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const unsigned tag = prm.first.tag;
+  auto word = [&](unsigned slot, int w) {
+    return __hip_atomic_load(&prm.first.flags[(size_t)slot * kTeamFlags + w], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  };
+  int *verdict = reinterpret_cast<int *>(smem);
+  if (wave == 0) {
+    // (bounded as every wait; a team without a member that left here finishes by itself)
+    int again = -1;
+    for (int k = 0; k < 16 * prm.first.polls && again < 0; ++k)
+      if (word(at.slot, 8 * 12) == tag) again = word(at.slot, kTeamListed) == tag ? 1 : 0;
+    if (lane == 0) *verdict = again;
+    if (at.role == 0) {
+      // The caller is told how many boards were listed.  Whoever finds all boards done, its own among them, adds them
+      // up: the last one does, and two would write the same.
+      if (lane == 0)
+        __hip_atomic_store(&prm.first.flags[(size_t)at.slot * kTeamFlags + kTeamDone], tag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+      const bool open = (unsigned)lane < items && word(lane, kTeamDone) != tag;
+      if (__builtin_amdgcn_ballot_w64(open) == 0) {
+        const bool listed = (unsigned)lane < items &&
+                            __hip_atomic_load(&prm.first.f.redo_counts[lane], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0;
+        const unsigned long long m = __builtin_amdgcn_ballot_w64(listed);
+        if (lane == 0) *prm.first.f.redo_count = __builtin_popcountll(m);
+      }
+    }
+  }
+  __syncthreads();
+  const int again = *verdict;
+  __syncthreads();
+  if (again != 1) return;
+  TeamParams second = prm.first;
+  second.f.packed = prm.packed;
+  second.f.redo_mode = kRedoNone;
+  second.act = prm.act;
+  second.flags = prm.flags;
+  second.tag = tag + 1;
+  team_board<P2, 12>(second, smem, at.slot, at.slot, at.role);
 }
 
 }  // namespace c6

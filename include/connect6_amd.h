@@ -189,7 +189,8 @@ int c6_forward_boards_cascade(const int8_t *boards, const int8_t *player,
  * better launch (or the mode has no such kernel): call c6_forward there.
  *   workspace  device, 16-byte aligned; contents need no preparation.  Per shared board 1.0 MB
  *              (C6_PREC_F32S), 0.5 MB (C6_PREC_BF16F6, _BF16F6W and the cascades), 0.35 MB (C6_PREC_BF16,
- *              _F16); of 256 CUs at most 128, 42 or 73, and 40 boards are shared
+ *              _F16); of 256 CUs at most 128, 42 or 73, and 40 boards are shared.  A cascade over at most 21
+ *              boards is one launch and takes both its passes' share
  *   (the cascade's workspace, where there is one, comes in front of these)
  *   flags      device words through which the workgroups of this launch tell one another what is
  *              done: no word may hold `tag` when the launch starts, and no other launch may use them

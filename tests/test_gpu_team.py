@@ -149,6 +149,43 @@ def test_edges_of_the_smallest_teams(cuda, prec, sizes):
                     assert torch.equal(p, q[a:a + n]), (n, a)
 
 
+@pytest.mark.parametrize("prec", [_lib.PREC_BF16C, _lib.PREC_BF16C6])
+def test_both_passes_in_one_launch(cuda, prec):
+    """At most 21 boards (of 256 CUs) go through c6_forward_cascade_team in one launch; also when nobody waits for long."""
+    model, (x, _) = _model(cuda), _inputs(21)
+    xd, lib = x.to(cuda), c6.load()
+    packed = model.packed_weights(prec)
+    flags = torch.zeros(2 * 21 * 256, dtype=torch.int32, device=cuda)
+    cw, tag = ctypes.c_size_t(), 1
+    with torch.inference_mode():
+        for threshold in (0.0, 0.02, 0.3, -1.0):
+            big = {}
+            want = run_forward(torch.cat([xd] * 4), packed, prec, 1, 84, threshold=threshold, stats=big)
+            counts = []
+            for b in (1, 2, 16, 17, 21):
+                for polls in (0, 1, 3):
+                    ws, fl = ctypes.c_size_t(), ctypes.c_size_t()
+                    assert lib.c6_team_bytes(prec, b, ctypes.byref(ws), ctypes.byref(fl)) == 0
+                    assert 0 < fl.value <= flags.numel() * 4
+                    assert lib.c6_cascade_workspace_bytes(b, ctypes.byref(cw)) == 0
+                    work = torch.full((ws.value,), 255, dtype=torch.uint8, device=cuda)
+                    cascade = torch.full((cw.value // 4,), -7, dtype=torch.int32, device=cuda)
+                    lg, vg = torch.empty(b, 361, device=cuda), torch.empty(b, device=cuda)
+                    rc = lib.c6_forward_cascade_team(xd.data_ptr(), 0, 1, b, packed.data_ptr(), packed.numel(), prec,
+                                                     lg.data_ptr(), 0, vg.data_ptr(), 0, None, 0.0, None, 1.0, None, None,
+                                                     threshold, cascade.data_ptr(), cw.value, work.data_ptr(), ws.value,
+                                                     flags.data_ptr(), flags.numel() * 4, tag, polls,
+                                                     _lib.stream_ptr(cuda))
+                    _lib.check(rc, "c6_forward_cascade_team")
+                    tag += 2
+                    assert torch.equal(lg, want[0][:b]) and torch.equal(vg, want[1][:b]), (threshold, b, polls)
+                    counts.append(int(cascade[0]))
+                assert counts[-1] == counts[-2] == counts[-3] and 0 <= counts[-1] <= b
+            assert int(big["second_pass"]) == 4 * counts[-1]
+            assert threshold != 0.0 or counts[-1] == 0
+            assert threshold != -1.0 or counts[-1] == 21
+
+
 def test_boards_states_views_and_index(cuda):
     model, (x, _) = _model(cuda), gen_boards(300, 200, 5)
     boards = (x[:, 0] - x[:, 1]).to(torch.int8).to(cuda)

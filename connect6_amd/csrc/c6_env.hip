@@ -81,15 +81,13 @@ __global__ __launch_bounds__(256) void env_step_kernel(const EnvParams p) {
 // stone of the turn.  Eight games per workgroup: their int8 boards are staged in LDS with
 // coalesced loads, then the 8 x 3 x cells output floats (a whole number of 16-byte units,
 // contiguous in memory) are written with 16-byte stores.
-// CELLS > 0 fixes the board size at compile time (divisions become multiplications).
+// (The 19 x 19 board has canonical_board_kernel.)
 constexpr int kCanonGames = 8;
-template <int CELLS>
 __global__ __launch_bounds__(256) void canonical_input_kernel(const int8_t *__restrict__ boards,
                                                               const int8_t *__restrict__ player,
                                                               const int8_t *__restrict__ stones_left,
-                                                              long long num, int cells_arg,
+                                                              long long num, int cells,
                                                               float *__restrict__ out) {
-  const int cells = CELLS > 0 ? CELLS : cells_arg;
   extern __shared__ __attribute__((aligned(16))) int8_t s_board[];  // kCanonGames * cells, + 8 so that word reads may run past the end
   __shared__ int s_me[kCanonGames];
   __shared__ float s_last[kCanonGames];
@@ -169,6 +167,60 @@ __global__ __launch_bounds__(256) void canonical_input_kernel(const int8_t *__re
   }
 }
 
+// The same on the 19 x 19 board: a thread writes QUADS times four consecutive floats, 256 apart, from the four bytes
+// they come from and, where they reach into the next plane or game, its first four.  No LDS and no barrier: as many
+// workgroups as fit the chip used to read all at once and then write all at once, each behind its loads' latency.
+// (1,024 / 4,096 / 16,384 / 65,536 games 6.9 / 8.7 / 15.3 / 68 us, so with two quads 3.2 / 6.2 / 14.0 / 76, with four
+// 3.7 / 6.7 / 13.8 / 62; a plain fill of the outputs 2.5 / 4.8 / 11.9 / 41.  Groups of games through LDS with the next
+// one's bytes ahead: 5.0 / 7.7 / 16.5 / 78.)
+template <int QUADS>
+__global__ __launch_bounds__(256) void canonical_board_kernel(const int8_t *__restrict__ boards,
+                                                              const int8_t *__restrict__ player,
+                                                              const int8_t *__restrict__ stones_left, unsigned num,
+                                                              float *__restrict__ out) {
+  constexpr unsigned GAME = 3 * kPix;
+  const unsigned total = num * GAME, quads = total / 4;   // (below 2^32, see launch_canonical_input)
+  const unsigned q0 = blockIdx.x * (256 * QUADS) + threadIdx.x;
+  int cell[QUADS], plane[QUADS], me[QUADS], next_me[QUADS], left[QUADS];
+  unsigned here[QUADS], next[QUADS];   // four squares of the plane the quad starts in, the first of the one behind it
+#pragma unroll
+  for (int k = 0; k < QUADS; ++k) {
+    const unsigned q = q0 + 256 * k < quads ? q0 + 256 * k : quads - 1;
+    const unsigned game = q * 4 / GAME;
+    const int rem = (int)(q * 4 - game * GAME);
+    plane[k] = rem >= 2 * kPix ? 2 : (rem >= kPix ? 1 : 0);
+    cell[k] = rem - plane[k] * kPix;
+    const unsigned behind = plane[k] == 2 && game + 1 < num ? game + 1 : game;
+    me[k] = player[game];
+    next_me[k] = player[behind];
+    left[k] = stones_left[game];
+    const int at = cell[k] + 3 < kPix ? cell[k] : kPix - 4;   // (not beyond the board)
+    __builtin_memcpy(&here[k], boards + (size_t)game * kPix + at, 4);
+    here[k] >>= 8 * (cell[k] - at);
+    next[k] = 0;
+    if (cell[k] + 3 >= kPix) __builtin_memcpy(&next[k], boards + (size_t)behind * kPix, 4);
+  }
+#pragma unroll
+  for (int k = 0; k < QUADS; ++k) {
+    const unsigned q = q0 + 256 * k;
+    if (q >= quads) break;
+    const float last = left[k] == 1 ? 1.0f : 0.0f;
+    const unsigned want = (plane[k] == 0 ? me[k] : -me[k]) & 0xff, want_next = (plane[k] == 0 ? -me[k] : next_me[k]) & 0xff;
+    f32x4 o;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) o[e] = plane[k] == 2 ? last : ((here[k] >> (8 * e) & 0xff) == want ? 1.0f : 0.0f);
+    if (cell[k] + 3 >= kPix) {
+      const int n = kPix - cell[k];   // squares left in the plane, 1 to 3
+#pragma unroll
+      for (int e = 1; e < 4; ++e)
+        if (e >= n) o[e] = plane[k] == 1 ? last : ((next[k] >> (8 * (e - n)) & 0xff) == want_next ? 1.0f : 0.0f);
+    }
+    reinterpret_cast<f32x4 *>(out)[q] = o;
+  }
+  // (up to three floats behind the last quad: the last game's third plane)
+  if (blockIdx.x == 0 && threadIdx.x < (total & 3u)) out[quads * 4 + threadIdx.x] = stones_left[num - 1] == 1 ? 1.0f : 0.0f;
+}
+
 int launch_env_step(const EnvParams &p, hipStream_t st) {
   if (p.num == 0) return C6_OK;
   const long long blocks = (p.num * kStepLanes + 255) / 256;
@@ -190,11 +242,14 @@ int launch_canonical_input(const int8_t *boards, const int8_t *player, const int
   if (num == 0) return C6_OK;
   const int cells = n * n;
   const long long blocks = (num + kCanonGames - 1) / kCanonGames;
-  if (n == kBoard) {
-    hipLaunchKernelGGL(canonical_input_kernel<kPix>, dim3((unsigned)blocks), dim3(256),
-                       (size_t)kCanonGames * cells + 8, st, boards, player, stones_left, num, cells, out);
+  if (n == kBoard && num <= 0xf0000000u / (3 * kPix) && (reinterpret_cast<uintptr_t>(out) & 15u) == 0) {
+    const unsigned quads = (unsigned)num * (3 * kPix) / 4;
+    if (num < 8192)
+      hipLaunchKernelGGL(canonical_board_kernel<2>, dim3((quads + 511) / 512), dim3(256), 0, st, boards, player, stones_left, (unsigned)num, out);
+    else
+      hipLaunchKernelGGL(canonical_board_kernel<4>, dim3((quads + 1023) / 1024), dim3(256), 0, st, boards, player, stones_left, (unsigned)num, out);
   } else {
-    hipLaunchKernelGGL(canonical_input_kernel<0>, dim3((unsigned)blocks), dim3(256),
+    hipLaunchKernelGGL(canonical_input_kernel, dim3((unsigned)blocks), dim3(256),
                        (size_t)kCanonGames * cells + 8, st, boards, player, stones_left, num, cells, out);
   }
   const hipError_t e = hipGetLastError();

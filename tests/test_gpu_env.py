@@ -127,6 +127,19 @@ def test_canonical_input_matches_oracle(cuda, num, board):
     assert torch.equal(c6.canonical_observation(boards.to(cuda), player.to(cuda), stones.to(cuda)).cpu(), want)
 
 
+@pytest.mark.parametrize("num", [2, 3, 5, 255, 8191, 8192, 8195])
+def test_canonical_input_at_the_edges_of_its_kernels(cuda, num):
+    """Last quads, games whose planes start inside a quad, states that are slices of larger tensors."""
+    gen = torch.Generator().manual_seed(num)
+    boards = torch.randint(-1, 2, (num + 1, 19, 19), generator=gen, dtype=torch.int8)
+    player = (torch.randint(0, 2, (num + 1,), generator=gen) * 2 - 1).to(torch.int8)
+    stones = torch.randint(1, 3, (num + 1,), generator=gen).to(torch.int8)
+    want = R.canonical_network_input(boards, player, stones)
+    b, p, s = boards.to(cuda), player.to(cuda), stones.to(cuda)
+    assert torch.equal(c6.canonical_network_input(b[1:], p[1:], s[1:]).cpu(), want[1:])
+    assert torch.equal(c6.canonical_network_input(b[:-1], p[:-1], s[:-1]).cpu(), want[:-1])
+
+
 def test_full_size_batch_is_periodic_in_the_small_one(cuda):
     # 262144 games driven by the first 1024 games' actions repeated: every block of 1024 must
     # reproduce the oracle-checked small batch bit for bit, at every step

@@ -79,6 +79,13 @@ at::Tensor fresh(at::IntArrayRef shape, at::ScalarType type, const at::Device &d
   return at::empty(shape, at::TensorOptions().dtype(type).device(dev));
 }
 
+// A tensor on a device, contiguous, of a type (or as it is: no trip through the dispatcher then).
+bool ready(const at::Tensor &t, const at::Device &dev) { return t.layout() == at::kStrided && t.device() == dev && t.is_contiguous(); }
+at::Tensor on(const at::Tensor &t, const at::Device &dev) { return ready(t, dev) ? t : t.to(dev).contiguous(); }
+at::Tensor on(const at::Tensor &t, const at::Device &dev, at::ScalarType type) {
+  return ready(t, dev) && t.scalar_type() == type ? t : t.to(dev, type).contiguous();
+}
+
 PyObject *wrap(const at::Tensor &t) {
   if (!t.defined()) Py_RETURN_NONE;
   return THPVariable_Wrap(t);
@@ -159,7 +166,7 @@ Team team_buffers(int prec, int64_t boards, const at::Device &dev, void *stream)
 
 // Uniform draws as the kernels read them: fp32 on the device, one per board.
 bool take_draws(const at::Tensor *u, int64_t total, const at::Device &dev, at::Tensor &out) {
-  out = u->to(dev, at::kFloat).contiguous();
+  out = on(*u, dev, at::kFloat);
   if (out.dim() == 1 && out.size(0) == total) return true;
   fail(PyExc_ValueError, "u must have shape (" + std::to_string(total) + ",), got " + shape_text(out));
   return false;
@@ -245,7 +252,7 @@ PyObject *forward(PyObject *, PyObject *const *a, Py_ssize_t n) {
                                         shape_text(*legal_in));
     if (legal_in->scalar_type() != at::kBool && legal_in->scalar_type() != at::kByte)
       return fail(PyExc_ValueError, "legal mask must be a bool or uint8 tensor");
-    legal = legal_in->to(dev).contiguous();
+    legal = on(*legal_in, dev);
   }
   const c10::DeviceGuard guard(dev);
   if (want_logits) logits = fresh({total, C6_ACTIONS}, type_of_code(logits_code), dev);
@@ -293,8 +300,8 @@ PyObject *forward_boards(PyObject *, PyObject *const *a, Py_ssize_t n) {
   const at::Device dev = boards_in.device();
   const int64_t states = boards_in.size(0);
   const at::Tensor boards = boards_in.contiguous();
-  const at::Tensor player = tensor(a[1]).to(dev).contiguous();
-  const at::Tensor left = tensor(a[2]).to(dev).contiguous();
+  const at::Tensor player = on(tensor(a[1]), dev);
+  const at::Tensor left = on(tensor(a[2]), dev);
   const at::Tensor *index_in = tensor_or_null(a[3]), *u_in = tensor_or_null(a[10]);
   const int view = (int)PyLong_AsLong(a[4]);
   const at::Tensor &packed = tensor(a[5]);
@@ -306,7 +313,7 @@ PyObject *forward_boards(PyObject *, PyObject *const *a, Py_ssize_t n) {
   void *stream = PyLong_AsVoidPtr(a[13]);
   if (PyErr_Occurred()) return nullptr;
   at::Tensor index, u, logits, actions, logprob, ws;
-  if (index_in != nullptr) index = index_in->to(dev).contiguous();
+  if (index_in != nullptr) index = on(*index_in, dev);
   const int64_t total = index.defined() ? index.numel() : states;
   if (u_in != nullptr && !take_draws(u_in, total, dev, u)) return nullptr;
   const c10::DeviceGuard guard(dev);
@@ -347,21 +354,35 @@ PyObject *forward_boards(PyObject *, PyObject *const *a, Py_ssize_t n) {
   END_HANDLE_TH_ERRORS
 }
 
+// Names as Python objects, made once: a look into a dictionary by a C string makes one each time.
+PyObject *interned(const char *name) { return PyUnicode_InternFromString(name); }
+PyObject *index_name(int i) {
+  static std::vector<PyObject *> &names = *new std::vector<PyObject *>;   // (under the interpreter's lock)
+  while ((int)names.size() <= i) names.push_back(interned(std::to_string(names.size()).c_str()));
+  return names[(size_t)i];
+}
+std::string path_text(std::initializer_list<PyObject *> path) {
+  std::string name;
+  for (PyObject *part : path) name += (name.empty() ? "" : ".") + std::string(PyUnicode_AsUTF8(part));
+  return name;
+}
+
 // A tensor of a module by the path of its name ("convs", "3", "weight"), as state_dict() finds it: null where
 // there is none (no Python error set).
-const at::Tensor *module_tensor(PyObject *module, std::initializer_list<const char *> path) {
-  static PyObject *dict_name = PyUnicode_InternFromString("__dict__");
+const at::Tensor *module_tensor(PyObject *module, std::initializer_list<PyObject *> path) {
+  static PyObject *dict_name = interned("__dict__"), *parameters_name = interned("_parameters"),
+                  *modules_name = interned("_modules"), *buffers_name = interned("_buffers");
   const at::Tensor *found = nullptr;
   PyObject *at = module;   // (borrowed: the module above holds it)
   for (size_t i = 0; i < path.size() && at != nullptr; ++i) {
     PyObject *dict = PyObject_GetAttr(at, dict_name);
     at = nullptr;
     if (dict == nullptr) break;
-    const char *name = path.begin()[i];
+    PyObject *name = path.begin()[i];
     const bool last = i + 1 == path.size();
-    for (const char *kind : {last ? "_parameters" : "_modules", "_buffers"}) {
-      PyObject *of = PyDict_GetItemString(dict, kind);
-      PyObject *v = of != nullptr && PyDict_Check(of) ? PyDict_GetItemString(of, name) : nullptr;
+    for (PyObject *kind : {last ? parameters_name : modules_name, buffers_name}) {
+      PyObject *of = PyDict_GetItem(dict, kind);
+      PyObject *v = of != nullptr && PyDict_Check(of) ? PyDict_GetItem(of, name) : nullptr;
       if (v == nullptr || v == Py_None) continue;
       if (!last) at = v;
       else if (THPVariable_Check(v)) found = &THPVariable_Unpack(v);
@@ -412,7 +433,7 @@ bool generic_call(GenericCall &c, PyObject *x, PyObject *arch_bytes, PyObject *p
                                  std::to_string(c.board * c.board) + "), got " + shape_text(*legal_in));
       return false;
     }
-    c.legal = legal_in->to(dev).contiguous();
+    c.legal = on(*legal_in, dev);
   }
   const c10::DeviceGuard guard(dev);
   c.logits = fresh({c.b, c.board * c.board}, at::kFloat, dev);
@@ -453,34 +474,37 @@ PyObject *forward_generic_module(PyObject *, PyObject *const *a, Py_ssize_t n) {
   if (!generic_call(c, a[1], a[3], a[4], Py_True, a[5], a[6], a[7], a[8])) return nullptr;
   const at::Device dev = c.x.device();
   const c10::DeviceGuard guard(dev);
+  static PyObject *convs = interned("convs"), *weight = interned("weight"), *bias_name = interned("bias"),
+                  *policy = interned("policy_output"), *value = interned("value_output");
   std::vector<at::Tensor> keep;   // (copies, where a parameter is not fp32, contiguous and on the device)
   bool ok = true;
-  const auto take = [&](std::initializer_list<const char *> path, int64_t count, bool required) -> const float * {
+  const auto take = [&](std::initializer_list<PyObject *> path, int64_t count, bool required) -> const float * {
     const at::Tensor *t = ok ? module_tensor(a[0], path) : nullptr;
-    std::string name;
-    for (const char *part : path) name += (name.empty() ? "" : ".") + std::string(part);
     if (t == nullptr) {
-      if (ok && required) ok = fail(PyExc_KeyError, "missing parameter " + name) != nullptr;
+      if (ok && required) ok = fail(PyExc_KeyError, "missing parameter " + path_text(path)) != nullptr;
       return nullptr;
     }
     if (t->numel() != count) {
-      ok = fail(PyExc_ValueError, name + " has " + std::to_string(t->numel()) + " elements, the network's layers need " +
-                                      std::to_string(count)) != nullptr;
+      ok = fail(PyExc_ValueError, path_text(path) + " has " + std::to_string(t->numel()) +
+                                      " elements, the network's layers need " + std::to_string(count)) != nullptr;
       return nullptr;
     }
+    // (as it is, where it is what the launch reads: the module holds it)
+    if (t->layout() == at::kStrided && t->scalar_type() == at::kFloat && t->device() == dev && t->is_contiguous() &&
+        !t->is_neg() && t->has_storage())
+      return ptr<float>(*t);
     keep.push_back(t->detach().to(dev, at::kFloat).contiguous());
     return ptr<float>(keep.back());
   };
   std::vector<const float *> w((size_t)c.layers), bias((size_t)c.layers);
   int64_t cin = 3;
   for (int l = 0; l < c.layers; ++l) {
-    const std::string at = std::to_string(l);
-    w[(size_t)l] = take({"convs", at.c_str(), "weight"}, cin * c.channels[l] * c.kernels[l] * c.kernels[l], true);
-    bias[(size_t)l] = take({"convs", at.c_str(), "bias"}, c.channels[l], false);
+    w[(size_t)l] = take({convs, index_name(l), weight}, cin * c.channels[l] * c.kernels[l] * c.kernels[l], true);
+    bias[(size_t)l] = take({convs, index_name(l), bias_name}, c.channels[l], false);
     cin = c.channels[l];
   }
-  const float *pol_w = take({"policy_output", "weight"}, cin, true), *pol_b = take({"policy_output", "bias"}, 1, false);
-  const float *val_w = take({"value_output", "weight"}, cin, false), *val_b = take({"value_output", "bias"}, 1, false);
+  const float *pol_w = take({policy, weight}, cin, true), *pol_b = take({policy, bias_name}, 1, false);
+  const float *val_w = take({value, weight}, cin, false), *val_b = take({value, bias_name}, 1, false);
   if (!ok) return nullptr;
   if (val_w == nullptr) return fail(PyExc_ValueError, "missing parameter value_output.weight: no value without it");
   const at::Tensor packed = fresh({bytes}, at::kByte, dev);
@@ -504,7 +528,7 @@ PyObject *mask_logits(PyObject *, PyObject *const *a, Py_ssize_t n) {
   if (code < 0)
     return fail(PyExc_ValueError, std::string("unsupported tensor dtype ") + c10::toString(src.scalar_type()) +
                                       "; expected float32, bfloat16 or float16");
-  const at::Tensor legal = legal_in.to(dev).contiguous();
+  const at::Tensor legal = on(legal_in, dev);
   // bit patterns of -(largest finite value): fp32, bf16, fp16
   const uint32_t fill = code == C6_DT_F32 ? 0xFF7FFFFFu : (code == C6_DT_BF16 ? 0xFF7Fu : 0xFBFFu);
   const c10::DeviceGuard guard(dev);
@@ -519,7 +543,7 @@ PyObject *mask_logits(PyObject *, PyObject *const *a, Py_ssize_t n) {
 PyObject *sample(PyObject *, PyObject *const *a, Py_ssize_t n) {
   if (n != 6) return fail(PyExc_TypeError, "sample takes 6 arguments");
   HANDLE_TH_ERRORS
-  const at::Tensor src = tensor(a[0]).to(at::kFloat).contiguous();
+  const at::Tensor src = on(tensor(a[0]), tensor(a[0]).device(), at::kFloat);
   const at::Tensor *legal_in = tensor_or_null(a[1]);
   const float temperature = (float)PyFloat_AsDouble(a[2]);
   const at::Device dev = src.device();
@@ -527,7 +551,7 @@ PyObject *sample(PyObject *, PyObject *const *a, Py_ssize_t n) {
   void *stream = PyLong_AsVoidPtr(a[5]);
   if (PyErr_Occurred()) return nullptr;
   at::Tensor legal, u, logprob;
-  if (legal_in != nullptr) legal = legal_in->to(dev).contiguous();
+  if (legal_in != nullptr) legal = on(*legal_in, dev);
   if (!take_draws(&tensor(a[3]), b, dev, u)) return nullptr;
   const c10::DeviceGuard guard(dev);
   const at::Tensor actions = fresh({b}, at::kLong, dev);
@@ -563,10 +587,19 @@ PyObject *env_step(PyObject *, PyObject *const *a, Py_ssize_t n) {
   END_HANDLE_TH_ERRORS
 }
 
-// canonical_input(boards, player, stones_left, stream) -> (rc, planes)
+// canonical_input(boards, player, stones_left, stream) -> (rc, planes); rc is kBadState where the state is not what
+// VectorConnect6 holds (the caller says what is wrong)
+constexpr int kBadState = -1000;
+bool state_ok(const at::Tensor &boards, const at::Tensor &player, const at::Tensor &left) {
+  if (!boards.is_cuda() || boards.dim() != 3 || boards.size(1) != boards.size(2)) return false;
+  for (const at::Tensor *t : {&boards, &player, &left})
+    if (t->scalar_type() != at::kChar || t->device() != boards.device()) return false;
+  return player.dim() == 1 && player.size(0) == boards.size(0) && left.dim() == 1 && left.size(0) == boards.size(0);
+}
 PyObject *canonical_input(PyObject *, PyObject *const *a, Py_ssize_t n) {
   if (n != 4) return fail(PyExc_TypeError, "canonical_input takes 4 arguments");
   HANDLE_TH_ERRORS
+  if (!state_ok(tensor(a[0]), tensor(a[1]), tensor(a[2]))) return answer<1>(kBadState, {at::Tensor()});
   const at::Tensor boards = tensor(a[0]).contiguous(), player = tensor(a[1]).contiguous(),
                    left = tensor(a[2]).contiguous();
   void *stream = PyLong_AsVoidPtr(a[3]);

@@ -47,9 +47,12 @@ def canonical_network_input(
 ) -> torch.Tensor:
     """connect6/vector_env.py:196-218: [N, 3, n, n] float32, planes = own stones, the other
     side's stones, "this decision is the last stone of the turn"."""
-    _require_state(boards, current_player, stones_left)
+    if not isinstance(boards, torch.Tensor) or not boards.is_cuda:
+        _require_state(boards, current_player, stones_left)
+    # (the native side looks at the state itself; what is wrong with it is told here)
     rc, out = _lib.host().canonical_input(boards, current_player, stones_left, _lib.stream_ptr(boards.device))
     if rc != 0:
+        _require_state(boards, current_player, stones_left)
         _lib.check(rc, "c6_canonical_input")
     return out
 

@@ -302,6 +302,13 @@ struct TeamParams {
   int polls;            // of a flag (about 0.7 us each) before a workgroup helps itself
 };
 constexpr int kTeamFlags = 256;   // words per board
+// ... both passes of a cascade in one launch
+struct TeamCascadeParams {
+  TeamParams first;
+  const unsigned char *packed;   // the second pass's
+  unsigned char *act;
+  unsigned *flags;
+};
 
 struct PackParams {
   const float *conv_w[8];     // each tensor stacked over the weight sets: [groups, ...]

@@ -1145,13 +1145,6 @@ template <class P> __global__ __launch_bounds__(256) void team_forward_kernel(co
 // stage is done, its team sees whether the board was listed and goes through it again in the second pass's mode, or ends:
 // one board that is not listed 41.4 -> 33.3 us with its mask (the second launch found nothing to do), of which waiting
 // for the verdict is 2.
-//   packed, act, flags: the second pass's
-struct TeamCascadeParams {
-  TeamParams first;
-  const unsigned char *packed;
-  unsigned char *act;
-  unsigned *flags;
-};
 template <class P2> __global__ __launch_bounds__(256) void team_cascade_kernel(const TeamCascadeParams prm) {
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
   const unsigned items = (unsigned)prm.first.f.total_boards;   // (at most 64)

@@ -156,10 +156,12 @@ template <class A, bool FIRST> struct RawWeights {   // FIRST: the first layer's
   const float *w;  // [cout, cin, k, k] of the weight set
   int cin, cout, kk, cb, cb_magic, blocks, lane;
   template <int CT> __device__ __forceinline__ void fetch(int c, v4i (&out)[CT][A::NW]) const {
-    const int e = 4 * c + (lane >> 4), tap = (e * cb_magic) >> 16, ci0 = 8 * (e - tap * cb);
+    int ln = lane;   // (what follows from it is formed here: registers)
+    asm volatile("" : "+v"(ln));
+    const int e = 4 * c + (ln >> 4), tap = (e * cb_magic) >> 16, ci0 = 8 * (e - tap * cb);
 #pragma unroll
     for (int t = 0; t < CT; ++t) {
-      const int co = 16 * t + (lane & 15);
+      const int co = 16 * t + (ln & 15);
       const bool row = e < blocks && co < cout;
       unsigned short pl[8][A::NW];
 #pragma unroll

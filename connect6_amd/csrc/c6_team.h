@@ -103,8 +103,8 @@ template <class P, int L> __device__ __forceinline__ int team_frag(int k, int t)
 
 // k-steps of weights that a wave keeps in flight: the loads take some 800 cycles and a k-step is
 // 32 cycles per MFMA
-template <class P, int TT> constexpr int team_ring() {
-  return Geo<P>::W == 3 ? 6 / TT : (Geo<P>::W == 1 ? 18 / TT : (TT == 1 ? 9 : (TT == 2 ? 6 : 3)));
+template <class P, int TT, int PT> constexpr int team_ring() {
+  return Geo<P>::W == 3 ? (PT > 1 ? 3 : 6) / TT : (Geo<P>::W == 1 ? 18 / TT : (TT == 1 ? 9 : (TT == 2 ? 6 : 3)));
 }
 
 // Low-order (fp6) pass of layer L for PT tiles of squares, conv3_lo_pass with TT cout tiles from t0 on.
@@ -158,12 +158,12 @@ __device__ __forceinline__ void team_lo_pass(const unsigned char *smem, const un
 //   low (fp32): what the bias leaves out, for the small products' sum (split_conv_tiles)
 template <class P, int L, int TT, int PT>
 __device__ __forceinline__ void team_conv(const unsigned char *smem, const unsigned char *packed, const WFrags &wl,
-                                          v4i (&ring)[team_ring<P, TT>()][TT][Geo<P>::W], int lane,
+                                          v4i (&ring)[team_ring<P, TT, PT>()][TT][Geo<P>::W], int lane,
                                           const int (&rec)[PT], int t0, f32x16 (&acc)[PT][TT],
                                           f32x16 (&low)[PT][TT]) {
   using T = TeamGeo<P>;
   constexpr int NT = kCoutArr[L] / 32, NTP = kCinArr[L] / 32;
-  constexpr int W = Geo<P>::W, NPL = T::NPL, D = team_ring<P, TT>();
+  constexpr int W = Geo<P>::W, NPL = T::NPL, D = team_ring<P, TT, PT>();
   constexpr int KC = kCinArr[L] / 16, KS = 9 * KC;
   constexpr int U = P::PIPE ? kPhaseSteps : 3 * KC;     // k-steps of one unrolled round
   constexpr bool LO = P::LO6 && ((P::LO_MASK >> L) & 1);
@@ -438,8 +438,10 @@ __device__ __forceinline__ void team_board(const TeamParams &prm, unsigned char 
   // `j` of each plane (then of the fp6 blocks), so that all its addresses are two sums and constants.
   auto unit_of = [&](auto cc, int &sq, int &j) __attribute__((always_inline)) {
     constexpr int J = decltype(cc)::value / 8;
-    sq = tid / J;
-    j = tid - sq * J;
+    int t = tid;   // (formed where it is used, not kept for all stages)
+    asm volatile("" : "+v"(t));
+    sq = t / J;
+    j = t - sq * J;
   };
   constexpr int PARTS = NPL + (P::LO6 ? 1 : 0);
   auto part_there = [](auto cc, int k, int j) __attribute__((always_inline)) { return k < NPL || j < decltype(cc)::value / 16; };
@@ -493,7 +495,7 @@ __device__ __forceinline__ void team_board(const TeamParams &prm, unsigned char 
 
   auto conv_stage = [&](auto lc, int role) __attribute__((always_inline)) -> bool {
     constexpr int L = decltype(lc)::value;
-    constexpr int NT = kCoutArr[L] / 32, TT = S::tiles(NT), D = team_ring<P, TT>();
+    constexpr int NT = kCoutArr[L] / 32, TT = S::tiles(NT), D = team_ring<P, TT, PT>();
     constexpr int C = kCinArr[L];
     // (opaque per stage: what follows from it is formed here and not, for all stages, in front of the
     // loop over them, in several hundred scalar registers that get spilled)
@@ -828,7 +830,7 @@ __device__ __forceinline__ void team_board(const TeamParams &prm, unsigned char 
         // Kernel rows (three fragments each), the row's activations asked for a row ahead and its weights DW rows, one
         // load behind each MFMA: a lone wave issues an instruction per five cycles, and what it issues between two rows
         // the matrix core waits for (all of a row's loads in front of it: bf16 54 cycles per MFMA, fp32 58).
-        constexpr int DW = W == 3 ? 4 : 8;
+        constexpr int DW = W == 3 ? (N1 > 1 ? 2 : 4) : 8;
         static_assert(DW % 2 == 0, "activations alternate");
         v4i w[DW][3][W], a[2][3][N1];
         auto weight = [&](int row, int i, int j) __attribute__((always_inline)) {

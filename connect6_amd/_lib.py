@@ -36,6 +36,7 @@ CASCADES = (PREC_BF16C, PREC_BF16C6)   # the modes that go through the cascade e
 # of those.
 CASCADE_THRESHOLD = 0.02
 DT_F32, DT_BF16, DT_F16 = 0, 1, 2
+DT_F32_AS_BF16, DT_F32_AS_F16 = 4, 5   # an fp32 input that counts as rounded to the 16-bit type
 MASK_NONE, MASK_INPUT, MASK_LEGAL = 0, 1, 2
 
 # every symbol include/connect6_amd.h declares
@@ -364,6 +365,13 @@ def cascade_workspace_bytes(boards: int) -> int:
     n = ctypes.c_size_t(0)
     check(load().c6_cascade_workspace_bytes(int(boards), ctypes.byref(n)), "c6_cascade_workspace_bytes")
     return int(n.value)
+
+
+def input_code(dtype) -> int:
+    """Input code of float32 planes that count as rounded to ``dtype`` (0: as they are)."""
+    import torch
+
+    return DT_F32_AS_BF16 if dtype == torch.bfloat16 else (DT_F32_AS_F16 if dtype == torch.float16 else 0)
 
 
 def torch_dtype_code(dtype) -> int:

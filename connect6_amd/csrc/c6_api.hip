@@ -92,6 +92,7 @@ static int device_ok(const char *who) {
 
 static bool aligned16(const void *p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
 static int elem_bytes(int dt) { return dt == C6_DT_F32 ? 4 : ((dt == C6_DT_BF16 || dt == C6_DT_F16) ? 2 : 0); }
+static bool valid_input(int dt) { return elem_bytes(dt) != 0 || dt == C6_DT_F32_AS_BF16 || dt == C6_DT_F32_AS_F16; }
 static bool valid_prec(int p) { return p >= C6_PREC_F32 && p <= C6_PREC_F32S; }
 
 // the cascade's workspace argument, checked; `who` names the entry point in the message
@@ -230,7 +231,7 @@ static int forward_planes(const char *who, const void *x, int x_dtype, int64_t g
               "take c6_forward_cascade, every other mode c6_forward)", who, prec);
     return C6_EINVAL;
   }
-  if (elem_bytes(x_dtype) == 0 || elem_bytes(logits_dtype) == 0) {
+  if (!valid_input(x_dtype) || elem_bytes(logits_dtype) == 0) {
     set_error("%s: unknown element type of the input (%d) or of the logits (%d)", who, x_dtype, logits_dtype);
     return C6_EINVAL;
   }
@@ -513,7 +514,7 @@ static int forward_generic(const char *who, const void *x, int x_dtype, int64_t 
                            const float *val_w, const float *val_b, int prec, void *workspace,
                            size_t workspace_bytes, float *logits, float *value, int mask_mode,
                            const uint8_t *legal, float fill, void *stream, bool pack = true) {
-  if (!valid_prec(prec) || elem_bytes(x_dtype) == 0 || groups < 1 || boards_per_group < 0 ||
+  if (!valid_prec(prec) || !valid_input(x_dtype) || groups < 1 || boards_per_group < 0 ||
       kernels == nullptr || (boards_per_group > 0 && groups > INT64_MAX / boards_per_group)) {
     set_error("%s: bad precision %d, input type %d, groups %lld, boards %lld or null kernels", who,
               prec, x_dtype, (long long)groups, (long long)boards_per_group);
@@ -683,7 +684,7 @@ int c6_forward_generic_packed(const void *x, int x_dtype, int64_t groups, int64_
   const char *who = "c6_forward_generic_packed";
   const int rc = check_generic_packed(who, groups, board, layers, kernels, channels, prec, packed, packed_stride);
   if (rc != C6_OK) return rc;
-  if (elem_bytes(x_dtype) == 0 || boards_per_group < 0 ||
+  if (!valid_input(x_dtype) || boards_per_group < 0 ||
       (boards_per_group > 0 && groups > 0x7fffffffLL / boards_per_group)) {
     set_error("%s: bad input type %d or %lld x %lld boards", who, x_dtype, (long long)groups,
               (long long)boards_per_group);

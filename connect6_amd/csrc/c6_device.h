@@ -13,6 +13,23 @@ template <class T> __device__ __forceinline__ void stream_store(T *p, const T &v
   __builtin_nontemporal_store(v, p);
 }
 
+// ---- input planes ----
+__device__ __forceinline__ bool input_is_f32(int dt) { return dt == C6_DT_F32 || dt >= C6_DT_F32_AS_BF16; }
+// An element as it lies in memory (a 16-bit one in the low half), and its value: apart, so that a kernel that asks for
+// its next board early does not wait for it to convert it.
+__device__ __forceinline__ float load_input_raw(const void *x, int dt, size_t i) {
+  if (input_is_f32(dt)) return reinterpret_cast<const float *>(x)[i];
+  return __builtin_bit_cast(float, (unsigned)reinterpret_cast<const unsigned short *>(x)[i]);
+}
+__device__ __forceinline__ float input_value(float raw, int dt) {
+  if (dt == C6_DT_F32 || dt == C6_DT_BOARD_I8) return raw;   // (board states: made as values)
+  if (dt == C6_DT_F32_AS_BF16) return (float)(__bf16)raw;
+  if (dt == C6_DT_F32_AS_F16) return (float)(_Float16)raw;
+  const unsigned b = __builtin_bit_cast(unsigned, raw);
+  return dt == C6_DT_BF16 ? __builtin_bit_cast(float, b << 16) : (float)__builtin_bit_cast(_Float16, (unsigned short)b);
+}
+__device__ __forceinline__ float load_input(const void *x, int dt, size_t i) { return input_value(load_input_raw(x, dt, i), dt); }
+
 // ---- fp32 operands as sums of three bf16 values ----
 // The bf16 value nearest to v; a finite v beyond the largest one rounds to that and not to an infinity.
 __device__ __forceinline__ unsigned short bf16_part(float v) {

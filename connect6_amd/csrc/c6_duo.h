@@ -210,7 +210,7 @@ __global__ __launch_bounds__(256, 2) void duo_forward_kernel(const FwdParams prm
           xin[r][2] = last;
         } else {
 #pragma unroll
-          for (int ch = 0; ch < 3; ++ch) xin[r][ch] = load_x(prm.x, prm.x_dtype, ((size_t)b * 3 + ch) * kPix + p);
+          for (int ch = 0; ch < 3; ++ch) xin[r][ch] = load_input_raw(prm.x, prm.x_dtype, ((size_t)b * 3 + ch) * kPix + p);
         }
         barred[r] = prm.mask_mode == C6_MASK_LEGAL ? (prm.legal[(size_t)b * kPix + p] == 0) : 0;
       }
@@ -244,6 +244,13 @@ __global__ __launch_bounds__(256, 2) void duo_forward_kernel(const FwdParams prm
       __builtin_amdgcn_sched_barrier(0);
     }
     // ---- stage the input: zero the shifted copies, then scatter the board ----
+    // (16-bit elements, and fp32 ones that count as rounded, become values here, when they have arrived)
+    if (prm.x_dtype != C6_DT_F32) {
+#pragma unroll
+      for (int r = 0; r < ROUNDS; ++r)
+#pragma unroll
+        for (int ch = 0; ch < 3; ++ch) xin[r][ch] = input_value(xin[r][ch], prm.x_dtype);
+    }
     if (tid == 0) {
       *flag = 0;
       red[9] = xin[0][2];   // the third plane's value at square 0

@@ -162,13 +162,6 @@ template <class P> __device__ __forceinline__ Scaled<P> act_scaled(Scaled<P> v) 
   else return v * act_scale<P>();
 }
 
-__device__ __forceinline__ float load_x(const void *x, int dt, size_t i) {
-  if (dt == C6_DT_F32) return reinterpret_cast<const float *>(x)[i];
-  const unsigned short b = reinterpret_cast<const unsigned short *>(x)[i];
-  if (dt == C6_DT_BF16) return __builtin_bit_cast(float, (unsigned)b << 16);
-  return (float)__builtin_bit_cast(_Float16, b);
-}
-
 // ------------------------------------------------------------------------
 // weight-fragment prefetch rings.  A ring holds the fragments of the next
 // kRing k-steps; the ring of layer L+1 is loaded before the epilogue of layer
@@ -1201,7 +1194,7 @@ __global__ __launch_bounds__(256) void fused_pipe_kernel(const FwdParams prm) {
       return;
     }
     constexpr int NE = 3 * kPix;
-    if (prm.x_dtype == C6_DT_F32) {
+    if (input_is_f32(prm.x_dtype)) {
       const float *xf = reinterpret_cast<const float *>(prm.x) + (size_t)b * NE;
       for (int i = wv; i < (NE + 63) / 64; i += NWAVES) {
         const int e = i * 64 + ln;
@@ -1236,10 +1229,7 @@ __global__ __launch_bounds__(256) void fused_pipe_kernel(const FwdParams prm) {
 #pragma unroll
       for (int ch = 0; ch < 3; ++ch) {
         const unsigned w = raw[ch * kPix + p];
-        const float as_bf16 = __builtin_bit_cast(float, w << 16);
-        const float as_f16 = (float)__builtin_bit_cast(_Float16, (unsigned short)w);
-        v[ch] = prm.x_dtype == C6_DT_F32 ? __builtin_bit_cast(float, w)
-                                          : (prm.x_dtype == C6_DT_BF16 ? as_bf16 : as_f16);
+        v[ch] = input_value(__builtin_bit_cast(float, w), prm.x_dtype);
       }
     }
     // bit 0: the square's logit is masked in the output; bit 1: the square counts as occupied
@@ -1252,6 +1242,11 @@ __global__ __launch_bounds__(256) void fused_pipe_kernel(const FwdParams prm) {
     const unsigned *raw = reinterpret_cast<const unsigned *>(smem + G::NEXT_IN_OFF);
     // (a 16-bit element arrives in the low half of its word; what the load leaves in the
     // upper half is not part of the value)
+    if (prm.x_dtype > C6_DT_BOARD_I8) {   // (as rounded)
+      const float a = input_value(__builtin_bit_cast(float, raw[2 * kPix + p]), prm.x_dtype);
+      const float b = input_value(__builtin_bit_cast(float, raw[2 * kPix]), prm.x_dtype);
+      return __builtin_bit_cast(unsigned, a) != __builtin_bit_cast(unsigned, b);
+    }
     const unsigned keep = prm.x_dtype == C6_DT_F32 ? 0xffffffffu : 0xffffu;
     return prm.x_dtype != C6_DT_BOARD_I8 && ((raw[2 * kPix + p] ^ raw[2 * kPix]) & keep) != 0;
   };
@@ -1737,7 +1732,7 @@ __global__ __launch_bounds__(256) void fused_forward_kernel(const FwdParams prm)
       if (p < kPix) {
 #pragma unroll
         for (int ch = 0; ch < 3; ++ch)
-          xin[r][ch] = load_x(prm.x, prm.x_dtype, ((size_t)b * 3 + ch) * kPix + p);
+          xin[r][ch] = load_input(prm.x, prm.x_dtype, ((size_t)b * 3 + ch) * kPix + p);
         occin[r] = prm.mask_mode == C6_MASK_LEGAL ? (prm.legal[(size_t)b * kPix + p] == 0) : 0;
       }
     }

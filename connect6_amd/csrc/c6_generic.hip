@@ -6,6 +6,7 @@
 #include <mutex>
 
 #include "c6_common.h"
+#include "c6_device.h"
 
 namespace c6 {
 
@@ -50,12 +51,7 @@ __device__ __forceinline__ float round_to(float v, int mode) {
   return v;
 }
 
-__device__ __forceinline__ float load_any(const void *x, int dt, size_t i) {
-  if (dt == C6_DT_F32) return reinterpret_cast<const float *>(x)[i];
-  const unsigned short b = reinterpret_cast<const unsigned short *>(x)[i];
-  if (dt == C6_DT_BF16) return __builtin_bit_cast(float, (unsigned)b << 16);
-  return (float)__builtin_bit_cast(_Float16, b);
-}
+__device__ __forceinline__ float load_any(const void *x, int dt, size_t i) { return load_input(x, dt, i); }
 
 // out[b,co,r,c] = act(bias[g,co] + sum_{ci,ky,kx} w[g,co,ci,ky,kx] * in[b,ci,r+ky-k/2,c+kx-k/2])
 // with g = b / per_group: the weight sets of a group of models lie one after the other

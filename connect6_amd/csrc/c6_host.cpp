@@ -221,10 +221,11 @@ PyObject *parameters(PyObject *, PyObject *module) {
 }
 
 // forward(x, packed, prec, groups, boards_per_group, want_logits, want_value, mask_mode, legal, fill, u,
-//         temperature, want_logprob, threshold, logits dtype code, stream)
+//         temperature, want_logprob, threshold, logits dtype code, stream[, input code])
+// input code: that of an fp32 input which counts as rounded to a 16-bit type (C6_DT_F32_AS_...), or 0
 //   -> (rc, logits, value, actions, logprob, cascade: boards evaluated twice as an int32[1])
 PyObject *forward(PyObject *, PyObject *const *a, Py_ssize_t n) {
-  if (n != 16) return fail(PyExc_TypeError, "forward takes 16 arguments");
+  if (n != 16 && n != 17) return fail(PyExc_TypeError, "forward takes 16 or 17 arguments");
   HANDLE_TH_ERRORS
   const at::Tensor x = tensor(a[0]).contiguous();
   const at::Tensor &packed = tensor(a[1]);
@@ -238,9 +239,10 @@ PyObject *forward(PyObject *, PyObject *const *a, Py_ssize_t n) {
   const float threshold = (float)PyFloat_AsDouble(a[13]);
   const int logits_code = (int)PyLong_AsLong(a[14]);
   void *stream = PyLong_AsVoidPtr(a[15]);
+  const int as_code = n > 16 ? (int)PyLong_AsLong(a[16]) : 0;
   if (PyErr_Occurred()) return nullptr;
   const at::Device dev = x.device();
-  const int x_code = dtype_code(x.scalar_type());
+  const int x_code = as_code != 0 && x.scalar_type() == at::kFloat ? as_code : dtype_code(x.scalar_type());
   if (x_code < 0)
     return fail(PyExc_ValueError, std::string("unsupported tensor dtype ") + c10::toString(x.scalar_type()) +
                                       "; expected float32, bfloat16 or float16");
@@ -447,16 +449,18 @@ int generic_launch(const GenericCall &c, const at::Tensor &packed, int64_t group
       static_cast<const uint8_t *>(c.legal.defined() ? c.legal.data_ptr() : nullptr), c.fill, c.stream);
 }
 
-// forward_generic(x, packed, groups, architecture, prec, want_value, mask_mode, legal, fill, stream)
+// forward_generic(x, packed, groups, architecture, prec, want_value, mask_mode, legal, fill, stream[, input code])
 //   -> (rc, logits, value).  architecture: bytes of the C ints kernels[layers], channels[layers]
 PyObject *forward_generic(PyObject *, PyObject *const *a, Py_ssize_t n) {
-  if (n != 10) return fail(PyExc_TypeError, "forward_generic takes 10 arguments");
+  if (n != 10 && n != 11) return fail(PyExc_TypeError, "forward_generic takes 10 or 11 arguments");
   HANDLE_TH_ERRORS
   const at::Tensor &packed = tensor(a[1]);
   const int64_t groups = PyLong_AsLongLong(a[2]);
+  const int as_code = n > 10 ? (int)PyLong_AsLong(a[10]) : 0;
   if (PyErr_Occurred()) return nullptr;
   GenericCall c;
   if (!generic_call(c, a[0], a[3], a[4], a[5], a[6], a[7], a[8], a[9])) return nullptr;
+  if (as_code != 0 && c.x.scalar_type() == at::kFloat) c.x_code = as_code;
   const c10::DeviceGuard guard(c.x.device());
   return answer<2>(generic_launch(c, packed, groups), {c.logits, c.value});
   END_HANDLE_TH_ERRORS

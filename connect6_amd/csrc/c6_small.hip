@@ -129,12 +129,7 @@ template <class A> __device__ __forceinline__ f32x4 small_mma(const v4i &w, cons
   }
 }
 
-__device__ __forceinline__ float small_load(const void *x, int dt, size_t i) {
-  if (dt == C6_DT_F32) return reinterpret_cast<const float *>(x)[i];
-  const unsigned short b = reinterpret_cast<const unsigned short *>(x)[i];
-  if (dt == C6_DT_BF16) return __builtin_bit_cast(float, (unsigned)b << 16);
-  return (float)__builtin_bit_cast(_Float16, b);
-}
+__device__ __forceinline__ float small_load(const void *x, int dt, size_t i) { return load_input(x, dt, i); }
 
 // Where a wave's weight fragments come from: the packed copy (fragment ((chunk * tiles + tile) *
 // planes + plane), see small_pack_kernel) ...

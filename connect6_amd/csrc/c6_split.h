@@ -357,7 +357,7 @@ __global__ __launch_bounds__(256) void split_forward_kernel(const FwdParams prm)
       const int p = tid + r * THREADS;
       if (p < kPix) {
 #pragma unroll
-        for (int ch = 0; ch < 3; ++ch) xin[r][ch] = load_x(prm.x, prm.x_dtype, ((size_t)b * 3 + ch) * kPix + p);
+        for (int ch = 0; ch < 3; ++ch) xin[r][ch] = load_input_raw(prm.x, prm.x_dtype, ((size_t)b * 3 + ch) * kPix + p);
         occin[r] = prm.mask_mode == C6_MASK_LEGAL ? (prm.legal[(size_t)b * kPix + p] == 0) : 0;
       }
     }
@@ -395,6 +395,13 @@ __global__ __launch_bounds__(256) void split_forward_kernel(const FwdParams prm)
       __builtin_amdgcn_sched_barrier(0);
     }
     // ---- stage the input: zero the shifted copies, then scatter the board ----
+    // (16-bit elements, and fp32 ones that count as rounded, become values here, when they have arrived)
+    if (prm.x_dtype != C6_DT_F32) {
+#pragma unroll
+      for (int r = 0; r < ROUNDS; ++r)
+#pragma unroll
+        for (int ch = 0; ch < 3; ++ch) xin[r][ch] = input_value(xin[r][ch], prm.x_dtype);
+    }
     if (tid < 2) flags[tid] = 0;
     if (tid == 0) red[42] = xin[0][2];   // the third plane's value at square 0
     {

@@ -726,7 +726,7 @@ __device__ __forceinline__ void team_board(const TeamParams &prm, unsigned char 
           xin[k][2] = f.stones_left[src] == 1 ? 1.0f : 0.0f;
         } else {
 #pragma unroll
-          for (int ch = 0; ch < 3; ++ch) xin[k][ch] = load_x(f.x, f.x_dtype, ((size_t)b * 3 + ch) * kPix + sq);
+          for (int ch = 0; ch < 3; ++ch) xin[k][ch] = load_input(f.x, f.x_dtype, ((size_t)b * 3 + ch) * kPix + sq);
         }
       }
     }
@@ -930,7 +930,7 @@ __device__ __forceinline__ void team_board(const TeamParams &prm, unsigned char 
         const int me = f.player[src];
         taken = stone == me || stone == -me;
       } else {
-        taken = load_x(f.x, f.x_dtype, (size_t)b * 3 * kPix + p) != 0.0f || load_x(f.x, f.x_dtype, ((size_t)b * 3 + 1) * kPix + p) != 0.0f;
+        taken = load_input(f.x, f.x_dtype, (size_t)b * 3 * kPix + p) != 0.0f || load_input(f.x, f.x_dtype, ((size_t)b * 3 + 1) * kPix + p) != 0.0f;
       }
       const bool masked = taken && f.mask_mode != C6_MASK_NONE;
       lgt[p] = z;

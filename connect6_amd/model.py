@@ -97,19 +97,20 @@ def run_forward(
     threshold: float | None = None,
     stats: dict | None = None,
     logits_dtype: torch.dtype = torch.float32,
+    input_dtype: torch.dtype | None = None,
 ):
     """Launch ``c6_forward`` (``c6_forward_cascade`` for the cascade mode, with ``threshold``
     and a workspace tensor of its own); returns (logits, value, actions, logprob), each None
     when not requested.  ``stats``, if given, receives ``second_pass`` for the cascade mode: a
     one-element int32 device tensor, the number of boards that were evaluated twice.
     ``logits_dtype`` other than float32 (the cascade mode's entry point only) makes the kernel
-    write the logits rounded to that type."""
+    write the logits rounded to that type.  ``input_dtype``: a float32 ``x`` counts as rounded to it."""
     if logits_dtype != torch.float32 and prec not in _lib.CASCADES:
         raise ValueError("only the cascade mode's entry point writes logits in another type than float32")
     rc, logits, value, actions, logprob, twice = _lib.host().forward(
         x, packed, prec, groups, boards_per_group, want_logits, want_value, mask_mode, legal, fill, u, temperature,
         want_logprob, _lib.CASCADE_THRESHOLD if threshold is None else threshold,
-        _lib.torch_dtype_code(logits_dtype), _lib.stream_ptr(x.device))
+        _lib.torch_dtype_code(logits_dtype), _lib.stream_ptr(x.device), _lib.input_code(input_dtype))
     if twice is not None and stats is not None:
         stats["second_pass"] = twice
     if rc != 0:
@@ -252,10 +253,12 @@ def pack_generic(state: dict[str, torch.Tensor], board: int, kernels, channels, 
 
 
 def run_packed_generic(x, packed, arch: bytes, prec: int, *, groups: int = 1, want_value: bool = True,
-                       mask_mode: int = _lib.MASK_NONE, legal=None, fill: float = _FILL_LOWEST):
-    """``c6_forward_generic_packed``: one launch.  ``arch``: see :func:`architecture_bytes`."""
+                       mask_mode: int = _lib.MASK_NONE, legal=None, fill: float = _FILL_LOWEST,
+                       input_dtype: torch.dtype | None = None):
+    """``c6_forward_generic_packed``: one launch.  ``arch``: see :func:`architecture_bytes`; ``input_dtype``: see
+    :func:`run_forward`."""
     rc, logits, value = _lib.host().forward_generic(x, packed, groups, arch, prec, want_value, mask_mode, legal, fill,
-                                                    _lib.stream_ptr(x.device))
+                                                    _lib.stream_ptr(x.device), _lib.input_code(input_dtype))
     if rc != 0:
         _lib.check(rc, "c6_forward_generic_packed")
     return logits, value

@@ -61,6 +61,10 @@ extern "C" {
 #define C6_DT_BF16 1
 #define C6_DT_F16 2
 #define C6_DT_BOARD_I8 3 /* int8 board states (+1 / -1 / 0), only through c6_forward_boards */
+/* input planes in fp32 that count as rounded to the 16-bit type (what a caller that holds its network in that
+ * type would convert them to first); x_dtype only */
+#define C6_DT_F32_AS_BF16 4
+#define C6_DT_F32_AS_F16 5
 
 /* masking of occupied squares in the policy logits */
 #define C6_MASK_NONE 0   /* logits as the network produced them (PolicyValueNet.forward)    */

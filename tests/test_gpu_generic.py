@@ -139,3 +139,30 @@ def test_generic_path_edge_cases(cuda):
             model.selfplay_step(torch.zeros(1, 3, 5, 5, device=cuda), torch.zeros(1, device=cuda))
     with pytest.raises(ValueError):
         model(torch.zeros(2, 3, 6, 6, device=cuda))
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("default,models,tables", [(True, 2, 3), (True, 2, 15), (True, 2, 70), (True, 3, 100), (False, 2, 9)])
+def test_history_rounds_fp32_planes_as_a_conversion_does(cuda, dtype, default, models, tables):
+    """The same bits as planes converted first, through every kernel an ensemble's batch goes to: inputs that
+    are not exact in the type, a constant and a varying third plane, planes that differ by less than its last bit."""
+    kernels, channels = (None, None) if default else ([5, 3], [16, 24])
+    board = 19 if default else 9
+    cps = []
+    for i in range(models):
+        net = c6.PolicyValueNet(board_size=board, kernels=kernels, channels=channels)
+        net.load_state_dict(R.init_state(40 + i, "torch_default", **({} if default else dict(kernels=kernels, channels=channels))))
+        cps.append(c6.HistoricalCheckpoint(path=Path(f"m{i}.pt"), update=i + 1, model_state=net.state_dict(),
+                                           model_config={"kernels": list(net.kernels), "channels": list(net.channels)},
+                                           game_config={"board_size": board, "win_length": 6}))
+    ens = c6.HistoricalPolicyEnsemble(cps, cuda, dtype=dtype)
+    g = torch.Generator().manual_seed(3)
+    x = (torch.rand(models, tables, 3, board, board, generator=g) > 0.7).float() * 0.3333
+    x[:, 0::3, 2] = 0.7001
+    x[:, 1::3, 2] = 0.7001 + 1e-6 * torch.rand(board, board, generator=g)
+    x[:, 0::2, 0, 0, 0] = 1e-42      # a zero in fp16, not in bf16
+    x[:, 0, 1, 2, 3] = 3.3e38        # an infinity in fp16
+    with torch.inference_mode():
+        a = ens.forward_grouped(x.to(cuda))
+        b = ens.forward_grouped(x.to(cuda).to(dtype))
+    assert a.dtype == dtype and torch.equal(a.isnan(), b.isnan()) and torch.equal(a.nan_to_num(), b.nan_to_num())

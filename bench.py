@@ -107,7 +107,7 @@ def main() -> int:
         # HIP events bracket the whole step: the bf16 kernel over all boards, then the kernel
         # that carries the low parts over the listed ones.  The first pass alone is timed with
         # threshold 0 (no board listed; the second kernel still starts and finds nothing).
-        kernel_name = "duo_forward_kernel<bf16> over all boards + fused_pipe_kernel<bf16f6w> over the listed boards"
+        kernel_name = "duo_forward_kernel<bf16> over all boards + second_pass_kernel<bf16f6w> over the listed boards"
         twice = int(model.cascade_stats["second_pass"].item())
         model.cascade_threshold = 0.0
         _, first = run_mode("bf16c", max(5, K // 2), 3)

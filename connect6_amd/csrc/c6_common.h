@@ -287,9 +287,6 @@ struct FwdParams {
   int *redo_list = nullptr;       // run r's list starts at entry r * redo_per
   int redo_runs = 0;              // workgroups (runs of boards) of the first pass
   int redo_per = 0;               // boards per run of the first pass
-  // second pass: where the listed boards leave up to redo_skip beyond a multiple of redo_round, that rest is
-  // another launch's
-  int redo_skip = -1, redo_round = 1;
 };
 
 // Few boards: several workgroups per board (c6_team.h)

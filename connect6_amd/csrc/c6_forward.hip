@@ -1122,10 +1122,52 @@ __device__ __forceinline__ void pipe_layer(
   (void)trace_on;
 }
 
-template <class P>
-__global__ __launch_bounds__(256) void fused_pipe_kernel(const FwdParams prm) {
+// ---- cascade, second pass (prm.redo_mode == kRedoConsume) ----
+// The boards to evaluate are the ones the first pass listed, run by run (run r: redo_counts[r] boards at
+// redo_list[r * redo_per ...]).  Every workgroup sums the counts up for itself -- `runs[r]` = boards listed by the
+// runs before r, `runs[redo_runs]` = all of them, which is what it returns -- and the listed boards, numbered in that
+// order, are dealt out like the boards of any batch.
+template <class P> __device__ __forceinline__ unsigned listed_runs(const FwdParams &prm, unsigned char *smem) {
   using G = Geo<P>;
-  extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
+  constexpr int THREADS = 256;
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  int *runs = reinterpret_cast<int *>(smem + G::RUNS_OFF);
+  int *part = reinterpret_cast<int *>(smem + G::RED_OFF);   // the four waves' sums
+  int before = 0;
+  for (int r0 = 0; r0 < prm.redo_runs; r0 += THREADS) {
+    const int r = r0 + tid;
+    const int c = r < prm.redo_runs ? prm.redo_counts[r] : 0;
+    const int incl = wave_inclusive_sum_i(c);
+    if (lane == 63) part[wave] = incl;
+    __syncthreads();
+    int lower = before;
+#pragma unroll
+    for (int w = 0; w < THREADS / 64; ++w) {
+      lower += w < wave ? part[w] : 0;
+      before += part[w];
+    }
+    if (r < prm.redo_runs) runs[r] = lower + incl - c;
+    __syncthreads();
+  }
+  if (tid == 0) runs[prm.redo_runs] = before;
+  __syncthreads();
+  return (unsigned)before;
+}
+// listed board i: the run r with runs[r] <= i < runs[r + 1] (a bisection; the same in every thread)
+template <class P> __device__ __forceinline__ unsigned listed_board(const FwdParams &prm, const unsigned char *smem, unsigned i) {
+  const int *runs = reinterpret_cast<const int *>(smem + Geo<P>::RUNS_OFF);
+  int lo = 0, hi = prm.redo_runs;
+  while (hi - lo > 1) {
+    const int mid = (lo + hi) >> 1;
+    if ((unsigned)runs[mid] <= i) lo = mid; else hi = mid;
+  }
+  return (unsigned)prm.redo_list[(size_t)lo * prm.redo_per + (i - (unsigned)runs[lo])];
+}
+
+// A workgroup's share of n_items boards: the batch's, or (LISTED) the first of those that a cascade's first pass listed.
+template <class P, bool LISTED>
+__device__ __forceinline__ void pipe_boards(const FwdParams &prm, unsigned char *smem, const unsigned n_items) {
+  using G = Geo<P>;
   constexpr int THREADS = 256, NWAVES = THREADS / 64;
   constexpr int ROUNDS = (kPix + THREADS - 1) / THREADS;  // pixels per thread when staging
 
@@ -1256,54 +1298,12 @@ __global__ __launch_bounds__(256) void fused_pipe_kernel(const FwdParams prm) {
   // workgroups of one XCD (workgroup i runs on XCD i % 8) cover one contiguous eighth of the
   // batch: with several weight sets an XCD's L2 then holds only the sets of its own boards, and
   // consecutive boards of a workgroup mostly reuse the set it has just streamed.
-  // Cascade, second pass (prm.redo_mode == kRedoConsume): the boards to evaluate are the ones the
-  // first pass listed, run by run (run r: redo_counts[r] boards at redo_list[r * redo_per ...]).
-  // Every workgroup sums the counts up for itself -- `runs[r]` = boards listed by the runs before
-  // r, `runs[redo_runs]` = all of them -- and the listed boards, numbered in that order, are dealt
-  // out like the boards of any batch.
-  // (compiled into the kernels that can be a cascade's passes only: the first pass is plain bf16,
-  // the second one of the modes that carry low parts)
-  constexpr bool kCanDetect = P::ID == C6_PREC_BF16, kCanConsume = P::LO6 != 0;
-  const bool from_list = kCanConsume && prm.redo_mode == kRedoConsume;
+  // (compiled into the kernel that can be a cascade's first pass only: plain bf16)
+  constexpr bool kCanDetect = P::ID == C6_PREC_BF16;
   const bool detect = kCanDetect && prm.redo_mode == kRedoDetect;
-  int *runs = reinterpret_cast<int *>(smem + G::RUNS_OFF);
-  unsigned n_items = (unsigned)prm.total_boards;
-  if (from_list) {
-    int *part = reinterpret_cast<int *>(red);   // the four waves' sums
-    int before = 0;
-    for (int r0 = 0; r0 < prm.redo_runs; r0 += THREADS) {
-      const int r = r0 + tid;
-      const int c = r < prm.redo_runs ? prm.redo_counts[r] : 0;
-      const int incl = wave_inclusive_sum_i(c);
-      if (lane == 63) part[wave] = incl;
-      __syncthreads();
-      int lower = before;
-#pragma unroll
-      for (int w = 0; w < NWAVES; ++w) {
-        lower += w < wave ? part[w] : 0;
-        before += part[w];
-      }
-      if (r < prm.redo_runs) runs[r] = lower + incl - c;
-      __syncthreads();
-    }
-    if (tid == 0) {
-      runs[prm.redo_runs] = before;
-      if (blockIdx.x == 0) *prm.redo_count = before;   // for the caller: boards evaluated twice
-    }
-    __syncthreads();
-    const int rest = before % prm.redo_round;
-    n_items = (unsigned)(rest <= prm.redo_skip ? before - rest : before);
-    if (n_items == 0) return;
-  }
-  // listed board i: the run r with runs[r] <= i < runs[r + 1] (a bisection; the same in every thread)
   auto board_of = [&](unsigned i) {
-    if (!from_list) return i;
-    int lo = 0, hi = prm.redo_runs;
-    while (hi - lo > 1) {
-      const int mid = (lo + hi) >> 1;
-      if ((unsigned)runs[mid] <= i) lo = mid; else hi = mid;
-    }
-    return (unsigned)prm.redo_list[(size_t)lo * prm.redo_per + (i - (unsigned)runs[lo])];
+    if constexpr (LISTED) return listed_board<P>(prm, smem, i);
+    else return i;
   };
   const unsigned per = (n_items + gridDim.x - 1) / gridDim.x;
   const unsigned xcds = (gridDim.x % 8 == 0) ? 8 : 1;
@@ -1657,6 +1657,11 @@ __global__ __launch_bounds__(256) void fused_pipe_kernel(const FwdParams prm) {
     b = bn;
   }
   if (detect && wave == 1 && lane == 0) prm.redo_counts[run] = listed;
+}
+template <class P>
+__global__ __launch_bounds__(256) void fused_pipe_kernel(const FwdParams prm) {
+  extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
+  pipe_boards<P, false>(prm, smem, (unsigned)prm.total_boards);
 }
 
 // ------------------------------------------------------------------------
@@ -2181,6 +2186,7 @@ template <class P> int launch_forward(const FwdParams &fp, hipStream_t st);
 
 template <class P> int launch_team(const TeamParams &tp, int grid, hipStream_t st);
 template <class P> int launch_team_cascade(const TeamCascadeParams &tp, int grid, hipStream_t st);
+template <class P> int launch_second_pass(const TeamParams &tp, int grid, hipStream_t st);
 
 #ifndef C6_SPLIT
 template <class P> int launch_pack(const PackParams &pp, hipStream_t st) {
@@ -2277,6 +2283,27 @@ template <class P> int launch_team(const TeamParams &tp, int grid, hipStream_t s
   return C6_OK;
 }
 
+template <class P> int launch_second_pass(const TeamParams &tp, int grid, hipStream_t st) {
+  constexpr int A = Geo<P>::LDS_BYTES, B = TeamGeo<P>::LDS_BYTES, LDS = A > B ? A : B;
+  static thread_local int configured = -1;
+  int dev = 0;
+  hipError_t e = hipGetDevice(&dev);
+  if (e == hipSuccess && configured != dev) {
+    e = hipFuncSetAttribute(reinterpret_cast<const void *>(&second_pass_kernel<P>),
+                            hipFuncAttributeMaxDynamicSharedMemorySize, LDS);
+    if (e == hipSuccess) configured = dev;
+  }
+  if (e == hipSuccess) {
+    hipLaunchKernelGGL(second_pass_kernel<P>, dim3((unsigned)grid), dim3(256), LDS, st, tp);
+    e = hipGetLastError();
+  }
+  if (e != hipSuccess) {
+    set_error("second_pass launch failed: %s", hipGetErrorString(e));
+    return C6_ELAUNCH;
+  }
+  return C6_OK;
+}
+
 template <class P> int launch_team_cascade(const TeamCascadeParams &tp, int grid, hipStream_t st) {
   constexpr int A = TeamGeo<PrecBF16>::LDS_BYTES, B = TeamGeo<P>::LDS_BYTES, LDS = A > B ? A : B;
   static thread_local int configured = -1;
@@ -2304,6 +2331,7 @@ template <class P> int launch_team_cascade(const TeamCascadeParams &tp, int grid
 #ifdef C6_INSTANCE
 #if defined(C6_CASCADE)
 template int launch_team_cascade<C6_INSTANCE>(const TeamCascadeParams &, int, hipStream_t);
+template int launch_second_pass<C6_INSTANCE>(const TeamParams &, int, hipStream_t);
 #elif defined(C6_TEAM)
 template int launch_team<C6_INSTANCE>(const TeamParams &, int, hipStream_t);
 #else
@@ -2390,12 +2418,10 @@ static TeamMode team_mode(int prec) {
 }
 static int second_mode(int cascade) { return cascade == C6_PREC_BF16C ? C6_PREC_BF16F6W : C6_PREC_BF16F6; }
 // The cascade's second pass hands what the listed boards leave beyond whole rounds of the CUs to teams, if it
-// is no more than they take (73 boards of 256 CUs with low weights, 42 without); their launch ends at once where
-// it is more.  How many are listed depends on the network (6 % of random ones' boards, a few of a peaked
-// policy's), not on the batch, so every cascade has that launch (21 boards and fewer: team_cascade_kernel).  Measured without / with it, boards (listed)
-// us: 512 (2) 200 / 161, 1,536 (13) 411 / 379, (67) 444 / 415, 2,048 (9) 520 / 485, 4,096 (4) 937 / 903,
-// (218) 958 / 967, 16,384 (19) 3,428 / 3,402; where it serves nothing it costs 3 to 6 us: 2,048 (99)
-// 549 / 553, 3,000 (153) 752 / 757, 1,000 (110) 335 / 337.
+// is no more than they take (73 boards of 256 CUs with low weights, 42 without; second_pass_kernel).  How many are
+// listed depends on the network (6 % of random ones' boards, a few of a peaked policy's), not on the batch.  Measured
+// without / with teams, boards (listed) us: 512 (2) 200 / 161, 1,536 (13) 411 / 379, (67) 444 / 415, 2,048 (9) 520 / 485,
+// 4,096 (4) 937 / 903, 16,384 (19) 3,428 / 3,402.
 
 // Boards of a batch that are shared between workgroups: all where they are few; behind whole rounds of one
 // workgroup per CU the rest (fp32: 257 boards 607 -> 373 us, 341 boards 607 -> 450 us, 384 boards 600 -> 531 us, 777 boards 1,190 ->
@@ -2458,8 +2484,7 @@ int dispatch_team(int prec, const TeamParams &tp, hipStream_t st) {
 // Cascade: every board through the plain bf16 kernel, whose workgroups list those of their boards
 // whose decision margin is below `threshold`; then the listed boards through the kernel that also
 // carries the low parts of activations and (C6_PREC_BF16C) weights, which overwrites their
-// outputs.  Two launches on the caller's stream (three where listed boards may share workgroups or
-// not, depending on their number: `team`), no host synchronisation, no atomic operation on the lists and nothing to clear:
+// outputs.  Two launches on the caller's stream, no host synchronisation, no atomic operation on the lists and nothing to clear:
 // the second kernel reads how many boards each workgroup of the first listed.
 int dispatch_cascade(int prec, const FwdParams &fp, float threshold, void *workspace, const TeamParams *team,
                      hipStream_t st) {
@@ -2480,36 +2505,25 @@ int dispatch_cascade(int prec, const FwdParams &fp, float threshold, void *works
   first.redo_list = ws + 4 + kCascadeMaxRuns;
   first.redo_runs = (int)runs;
   first.redo_per = (int)((fp.total_boards + runs - 1) / runs);
-  FwdParams second = first;
-  second.packed = fp.packed + kCascadeSecondOffset;
-  second.redo_mode = kRedoConsume;
-  if (team == nullptr) {
-    rc = launch_forward<PrecBF16>(first, st);
-  } else if (team_cascade_fits(fp.total_boards, cus)) {
-    TeamCascadeParams tp;
-    tp.first = *team;
-    tp.first.f = first;
-    tp.packed = second.packed;
-    tp.act = team->act + team_mode(C6_PREC_BF16).board_bytes * (size_t)fp.total_boards;
-    tp.flags = team->flags + (size_t)fp.total_boards * kTeamFlags;
-    return prec == C6_PREC_BF16C ? launch_team_cascade<PrecBF16F6W>(tp, cus, st) : launch_team_cascade<PrecBF16F6>(tp, cus, st);
-  } else {
-    TeamParams tp = *team;
-    tp.f = first;
-    rc = team_size<PrecBF16>(fp.total_boards, cus) > 1 ? dispatch_team(C6_PREC_BF16, tp, st)
-                                                       : launch_forward<PrecBF16>(first, st);
-    if (rc != C6_OK) return rc;
-    // teams for as many listed boards as they take, the ordinary launch for more
-    tp.f = second;
-    tp.tag = team->tag + 1;
-    const TeamMode teams = team_mode(second_mode(prec));
-    rc = teams.launch(tp, cus, st);
-    if (fp.total_boards <= teams.most(cus)) return rc;
-    second.redo_skip = (int)teams.most(cus);
-    second.redo_round = cus;
+  const unsigned char *packed2 = fp.packed + kCascadeSecondOffset;
+  TeamParams tp{};   // (no exchange memory: no board is shared)
+  if (team != nullptr) tp = *team;
+  tp.f = first;
+  if (team != nullptr && team_cascade_fits(fp.total_boards, cus)) {
+    TeamCascadeParams both;
+    both.first = tp;
+    both.packed = packed2;
+    both.act = team->act + team_mode(C6_PREC_BF16).board_bytes * (size_t)fp.total_boards;
+    both.flags = team->flags + (size_t)fp.total_boards * kTeamFlags;
+    return prec == C6_PREC_BF16C ? launch_team_cascade<PrecBF16F6W>(both, cus, st) : launch_team_cascade<PrecBF16F6>(both, cus, st);
   }
+  rc = team != nullptr && team_size<PrecBF16>(fp.total_boards, cus) > 1 ? dispatch_team(C6_PREC_BF16, tp, st)
+                                                                        : launch_forward<PrecBF16>(first, st);
   if (rc != C6_OK) return rc;
-  return prec == C6_PREC_BF16C ? launch_forward<PrecBF16F6W>(second, st) : launch_forward<PrecBF16F6>(second, st);
+  tp.f.packed = packed2;
+  tp.f.redo_mode = kRedoConsume;
+  tp.tag += 1;
+  return prec == C6_PREC_BF16C ? launch_second_pass<PrecBF16F6W>(tp, cus, st) : launch_second_pass<PrecBF16F6>(tp, cus, st);
 }
 
 size_t packed_bytes(int prec) {

@@ -67,9 +67,8 @@ template <class P> struct TeamGeo {
   static constexpr int OCC_OFF = (BUF + 15) & ~15;
   static constexpr int LGT_OFF = OCC_OFF + 384;
   static constexpr int RED_OFF = LGT_OFF + 1456;
-  static constexpr int RUNS_OFF = RED_OFF + 256 * 4;
   // a copy of the packed set's biases and head weights: no layer starts behind the latency of their loads
-  static constexpr int TAIL_OFF = (RUNS_OFF + (P::LO6 ? (kCascadeMaxRuns + 4) * 4 : 0) + 15) & ~15;
+  static constexpr int TAIL_OFF = (RED_OFF + 256 * 4 + 15) & ~15;
   static constexpr int LDS_BYTES = TAIL_OFF + G::TAIL_FLOATS * 4;
   static_assert(RECB / 16 % 2 == 1 && LDS_BYTES <= 160 * 1024, "LDS map");
 };
@@ -1084,63 +1083,26 @@ __device__ __forceinline__ TeamPlace team_place(unsigned items, int team) {
   return {blockIdx.x / (unsigned)team, (int)(blockIdx.x % (unsigned)team)};
 }
 
-template <class P> __global__ __launch_bounds__(256) void team_forward_kernel(const TeamParams prm) {
-  using T = TeamGeo<P>;
-  extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
-  unsigned items = (unsigned)prm.f.total_boards;
-  // cascade, second pass: the listed boards, as fused_pipe_kernel finds them
-  int *runs = reinterpret_cast<int *>(smem + T::RUNS_OFF);
-  const bool from_list = P::LO6 != 0 && prm.f.redo_mode == kRedoConsume;
-  if (from_list) {
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    int *part = reinterpret_cast<int *>(smem + T::RED_OFF);
-    int before = 0;
-    for (int r0 = 0; r0 < prm.f.redo_runs; r0 += 256) {
-      const int r = r0 + tid, c = r < prm.f.redo_runs ? prm.f.redo_counts[r] : 0;
-      const int incl = wave_inclusive_sum_i(c);
-      if (lane == 63) part[wave] = incl;
-      __syncthreads();
-      int lower = before;
-#pragma unroll
-      for (int w = 0; w < 4; ++w) {
-        lower += w < wave ? part[w] : 0;
-        before += part[w];
-      }
-      if (r < prm.f.redo_runs) runs[r] = lower + incl - c;
-      __syncthreads();
-    }
-    if (tid == 0 && blockIdx.x == 0) *prm.f.redo_count = before;
-    items = (unsigned)before;
+// A workgroup's share of board b, in a team of any size that the mode has.
+template <class P>
+__device__ __forceinline__ void team_share(const TeamParams &prm, unsigned char *smem, unsigned b, TeamPlace at, int team) {
+  if (team == 12) team_board<P, 12>(prm, smem, b, at.slot, at.role);
+  if (team == 6) team_board<P, 6>(prm, smem, b, at.slot, at.role);
+  if constexpr (team_least<P>() <= 3) {
+    if (team == 3) team_board<P, 3>(prm, smem, b, at.slot, at.role);
   }
-  // (listed boards beyond whole rounds of the CUs; the others, and a rest that is more than the teams take,
-  // are the launch's behind this one)
-  const unsigned from = from_list ? items - items % gridDim.x : 0;
-  items -= from;
-  if (items == 0) return;
+  if constexpr (team_least<P>() <= 2) {
+    if (team == 2) team_board<P, 2>(prm, smem, b, at.slot, at.role);
+  }
+}
+
+template <class P> __global__ __launch_bounds__(256) void team_forward_kernel(const TeamParams prm) {
+  extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
+  const unsigned items = (unsigned)prm.f.total_boards;
   const int team = team_size<P>(items, (int)gridDim.x);
   if (team == 1) return;
   const TeamPlace at = team_place(items, team);
-  const unsigned slot = at.slot;
-  const int role = at.role;
-  if (slot >= items) return;
-  unsigned b = prm.first + slot;
-  if (from_list) {
-    const unsigned item = from + slot;
-    int lo = 0, hi = prm.f.redo_runs;
-    while (hi - lo > 1) {
-      const int mid = (lo + hi) >> 1;
-      if ((unsigned)runs[mid] <= item) lo = mid; else hi = mid;
-    }
-    b = (unsigned)prm.f.redo_list[(size_t)lo * prm.f.redo_per + (item - (unsigned)runs[lo])];
-  }
-  if (team == 12) team_board<P, 12>(prm, smem, b, slot, role);
-  if (team == 6) team_board<P, 6>(prm, smem, b, slot, role);
-  if constexpr (team_least<P>() <= 3) {
-    if (team == 3) team_board<P, 3>(prm, smem, b, slot, role);
-  }
-  if constexpr (team_least<P>() <= 2) {
-    if (team == 2) team_board<P, 2>(prm, smem, b, slot, role);
-  }
+  if (at.slot < items) team_share<P>(prm, smem, prm.first + at.slot, at, team);
 }
 
 // The cascade over so few boards that twelve workgroups share each: both passes in one launch.  Where a board's last
@@ -1191,6 +1153,30 @@ template <class P2> __global__ __launch_bounds__(256) void team_cascade_kernel(c
   second.flags = prm.flags;
   second.tag = tag + 1;
   team_board<P2, 12>(second, smem, at.slot, at.slot, at.role);
+}
+
+// The cascade's second pass: what the listed boards leave beyond whole rounds of the workgroups goes to teams, if
+// it is no more than they take, and the others to one workgroup each.  One launch, since nobody knows before it runs how
+// many are listed; as a launch each, the one without a board took 4.8 us between the passes (512 boards of 128 sets
+// 186.6 -> 184.6 us, 4,096 of 8 sets 944.6 -> 937.2, 1,536 boards 447.9 -> 445.1; the kernel itself takes as long as
+// fused_pipe_kernel, 2,540 us on 3,300 listed boards).
+template <class P> __global__ __launch_bounds__(256) void second_pass_kernel(const TeamParams prm) {
+  extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
+  unsigned items = listed_runs<P>(prm.f, smem);
+  if (threadIdx.x == 0 && blockIdx.x == 0) *prm.f.redo_count = (int)items;   // for the caller: boards evaluated twice
+  const unsigned rest = items % gridDim.x;
+  const int team = rest != 0 && prm.act != nullptr ? team_size<P>(rest, (int)gridDim.x) : 1;
+  if (team > 1) {
+    items -= rest;
+    const TeamPlace at = team_place(rest, team);
+    if (at.slot < rest) {
+      const unsigned b = listed_board<P>(prm.f, smem, items + at.slot);
+      __syncthreads();   // (the runs are read; the team's tiles lie on them)
+      team_share<P>(prm, smem, b, at, team);
+      if (items != 0) listed_runs<P>(prm.f, smem);
+    }
+  }
+  if (items != 0) pipe_boards<P, true>(prm.f, smem, items);
 }
 
 }  // namespace c6

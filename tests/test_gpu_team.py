@@ -186,6 +186,24 @@ def test_both_passes_in_one_launch(cuda, prec):
             assert threshold != -1.0 or counts[-1] == 21
 
 
+@pytest.mark.parametrize("prec", [_lib.PREC_BF16C, _lib.PREC_BF16C6])
+@pytest.mark.parametrize("boards", [22, 42, 43, 73, 74, 255, 256, 257, 298, 299, 329, 330, 513])
+def test_second_pass_of_whole_rounds_and_a_rest(cuda, prec, boards):
+    """Every board listed: none, one or two whole rounds of one workgroup per board, and a rest at the edges of what
+    teams take, twice on the same stream; the bits and the count of the second pass's own mode."""
+    net = c6.PolicyValueNet().to(cuda).eval()
+    x = gen_boards(boards, 120, 3)[0].to(cuda)
+    alone = _lib.PREC_BF16F6W if prec == _lib.PREC_BF16C else _lib.PREC_BF16F6
+    with torch.inference_mode():
+        want = run_forward(torch.cat([x, x[:1].expand(600, -1, -1, -1)])[:512], net.packed_weights(alone), alone, 1, 512)
+        for _ in range(2):
+            stats = {}
+            got = run_forward(x, net.packed_weights(prec), prec, 1, boards, threshold=-1.0, stats=stats)
+            assert int(stats["second_pass"]) == boards
+            n = min(boards, 512)
+            assert torch.equal(got[0][:n], want[0][:n]) and torch.equal(got[1][:n], want[1][:n])
+
+
 def test_boards_states_views_and_index(cuda):
     model, (x, _) = _model(cuda), gen_boards(300, 200, 5)
     boards = (x[:, 0] - x[:, 1]).to(torch.int8).to(cuda)

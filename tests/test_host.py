@@ -56,6 +56,13 @@ def test_fused_kernels_stay_within_their_scratch_budget():
     assert split["ScratchSize"] <= 400
 
 
+def test_second_pass_kernels_use_no_scratch():
+    """The cascade's second pass holds the pipelined kernel's loop beside that of a shared board."""
+    usage = _lib.resource_usage()
+    second = [u for name, u in usage.items() if "second_pass_kernel" in name or "team_cascade_kernel" in name]
+    assert len(second) == 4 and all(u["ScratchSize"] == 0 for u in second)
+
+
 def test_history_dtype_follows_the_reference_policy():
     # connect6/train.py:133-145
     cpu, gpu = torch.device("cpu"), torch.device("cuda", 0)

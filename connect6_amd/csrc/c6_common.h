@@ -242,7 +242,7 @@ constexpr size_t cascade_packed_bytes(int prec) {
 // call.  The second pass sums the counts up (every workgroup for itself) and deals the listed boards
 // out evenly.  Layout, in int32: [0] boards listed in all (written by the second pass, for the
 // caller), [4, 4 + kCascadeMaxRuns) the counts per run, then the lists, `per` entries per run
-// (runs x per <= boards + runs).
+// (runs x per <= boards + kCascadeMaxRuns).
 constexpr int kCascadeMaxRuns = 1024;   // workgroups of the first pass: two per compute unit, at most
 constexpr size_t cascade_workspace_bytes(long long boards) {
   return (size_t)(16 + 4 * (long long)kCascadeMaxRuns + 4 * (boards + kCascadeMaxRuns) + 15) & ~(size_t)15;
@@ -296,6 +296,7 @@ struct TeamParams {
   unsigned *flags;      // kTeamFlags words per board
   unsigned tag;
   unsigned first = 0;   // the first of the f.total_boards boards
+  unsigned run = 0;     // cascade, first pass: the run that lists it (each board of a team is a run)
   int polls;            // of a flag (about 0.7 us each) before a workgroup helps itself
 };
 constexpr int kTeamFlags = 256;   // words per board

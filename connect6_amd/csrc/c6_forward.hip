@@ -2425,14 +2425,22 @@ static int second_mode(int cascade) { return cascade == C6_PREC_BF16C ? C6_PREC_
 
 // Boards of a batch that are shared between workgroups: all where they are few; behind whole rounds of one
 // workgroup per CU the rest (fp32: 257 boards 607 -> 373 us, 341 boards 607 -> 450 us, 384 boards 600 -> 531 us, 777 boards 1,190 ->
-// 975 us; bf16 + fp6 + low weights, 298 boards: 239 -> 191 us).  Not in the modes that put two workgroups on a
-// CU: 9 boards more than three rounds are half a round there.
+// 975 us; bf16 + fp6 + low weights, 298 boards: 239 -> 191 us).  In the modes that put two workgroups on a CU a rest is
+// a board more for some CUs; behind an odd number of rounds, where that is a fourth board beside three, a sixth beside
+// five ..., it takes longer than teams do, unless so few CUs have it that their clock makes up for it.  fp16, all as
+// one / rest in teams, us (the cascade, 768 + 9: 298 / 286, 1,280 + 9: 437 / 421, 2,816 + 2: 726 / 748, + 9: 762 / 748):
+//   768 + 1  202 / 194   + 9  208 / 195   + 24  208 / 205   + 40  208 / 205      512 + 9  141 / 144
+//   1,280 + 1  307 / 303   + 9  317 / 304   + 40  317 / 314                      1,024 + 9  249 / 252
+//   2,816 + 1  615 / 625   + 2  631 / 625   + 9  639 / 626   + 40  640 / 637
+//   4,864 + 2  1,057 / 1,061   + 9  1,070 / 1,061   + 40  1,072 / 1,074
 static long long team_boards(int prec, long long boards, int cus) {
   const TeamMode m = team_mode(prec);
   if (m.launch == nullptr) return 0;
   if (boards <= cus) return m.size(boards, cus) > 1 ? boards : 0;
   const long long rest = boards % cus;
-  return m.rounds && rest <= m.most(cus) ? rest : 0;
+  const long long rounds = boards / cus;
+  const bool shares = m.rounds || (rounds % 2 == 1 && rounds > 1 && rounds < 12 && 2 * rest > rounds);
+  return shares && rest <= m.most(cus) ? rest : 0;
 }
 
 // Boards of a cascade whose two passes are one launch: those that twelve workgroups share (team_cascade_kernel)
@@ -2478,6 +2486,7 @@ int dispatch_team(int prec, const TeamParams &tp, hipStream_t st) {
   }
   part.f.total_boards = shared;
   part.first = (unsigned)(all - shared);
+  if (tp.f.redo_mode == kRedoDetect) part.run = (unsigned)(tp.f.redo_runs - shared);
   return m.launch(part, cus, st);   // (workgroups without a board end at once)
 }
 
@@ -2491,7 +2500,9 @@ int dispatch_cascade(int prec, const FwdParams &fp, float threshold, void *works
   int cus = 0;
   int rc = device_cus(cus);
   if (rc != C6_OK) return rc;
-  const long long runs = forward_grid<PrecBF16>(fp.total_boards, cus);
+  // runs: the workgroups of the boards that have one each, then each board that teams share
+  const long long shared = team != nullptr ? team_boards(C6_PREC_BF16, fp.total_boards, cus) : 0;
+  const long long single = fp.total_boards - shared, grid = forward_grid<PrecBF16>(single, cus), runs = grid + shared;
   if (runs > kCascadeMaxRuns) {
     set_error("cascade: %lld workgroups exceed the %d the workspace layout provides for", runs, kCascadeMaxRuns);
     return C6_EINVAL;
@@ -2504,7 +2515,7 @@ int dispatch_cascade(int prec, const FwdParams &fp, float threshold, void *works
   first.redo_counts = ws + 4;
   first.redo_list = ws + 4 + kCascadeMaxRuns;
   first.redo_runs = (int)runs;
-  first.redo_per = (int)((fp.total_boards + runs - 1) / runs);
+  first.redo_per = single > 0 ? (int)((single + grid - 1) / grid) : 1;
   const unsigned char *packed2 = fp.packed + kCascadeSecondOffset;
   TeamParams tp{};   // (no exchange memory: no board is shared)
   if (team != nullptr) tp = *team;
@@ -2517,8 +2528,7 @@ int dispatch_cascade(int prec, const FwdParams &fp, float threshold, void *works
     both.flags = team->flags + (size_t)fp.total_boards * kTeamFlags;
     return prec == C6_PREC_BF16C ? launch_team_cascade<PrecBF16F6W>(both, cus, st) : launch_team_cascade<PrecBF16F6>(both, cus, st);
   }
-  rc = team != nullptr && team_size<PrecBF16>(fp.total_boards, cus) > 1 ? dispatch_team(C6_PREC_BF16, tp, st)
-                                                                        : launch_forward<PrecBF16>(first, st);
+  rc = shared > 0 ? dispatch_team(C6_PREC_BF16, tp, st) : launch_forward<PrecBF16>(first, st);
   if (rc != C6_OK) return rc;
   tp.f.packed = packed2;
   tp.f.redo_mode = kRedoConsume;

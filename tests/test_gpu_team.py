@@ -204,6 +204,36 @@ def test_second_pass_of_whole_rounds_and_a_rest(cuda, prec, boards):
             assert torch.equal(got[0][:n], want[0][:n]) and torch.equal(got[1][:n], want[1][:n])
 
 
+@pytest.mark.parametrize("prec", [_lib.PREC_BF16, _lib.PREC_F16, _lib.PREC_BF16C, _lib.PREC_BF16C6])
+def test_a_rest_behind_an_odd_number_of_rounds(cuda, prec):
+    """Two workgroups per CU, and teams for a few boards beyond 3, 5, ... 11 rounds: the bits and the listed boards of
+    batches that go to one kernel, at the edges of the rule."""
+    cus = torch.cuda.get_device_properties(cuda).multi_processor_count
+    most = cus * 5 // 32
+    total = 11 * cus + most + 1
+    x, legal = gen_boards(400, 200, 31)
+    pick = torch.arange(total) % 399
+    xd, ld, u = x[pick].to(cuda), legal[pick].to(cuda), gen_uniform(total, 5).to(cuda)
+    packed = _model(cuda).packed_weights(prec)
+    cascade = prec in _lib.CASCADES
+    with torch.inference_mode():
+        for threshold in (0.0, 0.02, -1.0) if cascade else (None,):
+            def call(a, b):
+                stats = {}
+                out = run_forward(xd[a:b], packed, prec, 1, b - a, mask_mode=_lib.MASK_LEGAL, legal=ld[a:b], u=u[a:b],
+                                  temperature=0.8, want_logprob=True, threshold=threshold, stats=stats)
+                return out, int(stats["second_pass"]) if cascade else 0
+            parts = [call(i, min(i + 100, total)) for i in range(0, total, 100)]
+            want = [torch.cat(t) for t in zip(*[p[0] for p in parts])]
+            for n in (2 * cus + 9, 3 * cus, 3 * cus + 1, 3 * cus + 2, 3 * cus + 9, 3 * cus + most, 3 * cus + most + 1,
+                      4 * cus + 9, 5 * cus + 21, 11 * cus + 5, 11 * cus + 6, total - 1, total):
+                got, listed = call(0, n)
+                for a, b in zip(got, want):
+                    assert torch.equal(a, b[:n]), (threshold, n)
+                tail = call(n // 100 * 100, n)[1] if n % 100 else 0
+                assert listed == sum(p[1] for p in parts[:n // 100]) + tail, (threshold, n)
+
+
 def test_boards_states_views_and_index(cuda):
     model, (x, _) = _model(cuda), gen_boards(300, 200, 5)
     boards = (x[:, 0] - x[:, 1]).to(torch.int8).to(cuda)

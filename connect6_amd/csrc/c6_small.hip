@@ -339,6 +339,7 @@ __global__ __launch_bounds__(64 * kSmallMaxWaves) void small_net_kernel(const Sm
     __syncthreads();
   }
   const bool one_plane = __builtin_amdgcn_readfirstlane(*s_inexact) == 0;
+  if (prm.layers == 1) __syncthreads();   // (no barrier of a layer's between this read and the heads' store to the word)
 
   int rc[PT];
   bool mine[PT];  // the lane's square exists (the others shadow the last one and store nothing)

@@ -199,6 +199,31 @@ def test_weights_packed_into_the_workspace_or_read_as_they_are(cuda, board, kern
         assert torch.equal(packed[0][:1], alone[0]) and torch.equal(packed[1][:1], alone[1])
 
 
+@pytest.mark.parametrize("board,kernels,channels,batch", [(1, [1], [1], 70), (9, [3], [48], 300), (19, [5], [17], 40)])
+def test_one_layer_with_inputs_that_are_not_exact_in_bf16(cuda, board, kernels, channels, batch):
+    """A network without a layer behind its first: with a value head, and packed without one (the heads then store
+    zeros where the inputs' exactness was noted).  Weights read as they are take every part of an input always."""
+    states = [R.init_state(40 + i, "torch_default", kernels=kernels, channels=channels) for i in range(2)]
+    x = torch.randn(2 * batch, 3, board, board, generator=torch.Generator().manual_seed(6))
+    xd, arch = x.to(cuda), architecture_bytes(kernels, channels)
+    model = c6.PolicyValueNet(board_size=board, kernels=kernels, channels=channels).to(cuda).eval()
+    stacked = {k: torch.stack([s[k] for s in states]).to(cuda) for k in states[0]}
+    policy_only = pack_generic(stacked, board, kernels, channels, _lib.PREC_F32, cuda, groups=2, want_value=False)
+    with torch.inference_mode():
+        sets, _ = run_packed_generic(xd, policy_only, arch, _lib.PREC_F32, groups=2, want_value=False)
+        for i, st in enumerate(states):
+            model.load_state_dict(st)
+            part = slice(i * batch, (i + 1) * batch)
+            raw = run_forward_generic(xd[part], {k: v.to(cuda) for k, v in st.items()}, kernels, channels, _lib.PREC_F32,
+                                      static_workspace=True)
+            lg, vg = model(xd[part])
+            assert torch.equal(lg, raw[0]) and torch.equal(vg, raw[1])
+            assert torch.equal(sets[part], raw[0])
+            lo, vo = R.forward(st, x[part])
+            # fp32 sums of at most 25 x 3 and 48 products; one part of the inputs alone would be off by 2^-9
+            assert rel_l2(lg, lo) <= 5e-6 and rel_l2(vg, vo) <= 5e-6
+
+
 def test_board_size_set_after_construction(cuda):
     """The network is fully convolutional: the same module on boards of another size."""
     for kernels, channels, first, second in ((None, None, 19, 9), ([3, 3], [8, 16], 7, 13)):

@@ -513,7 +513,7 @@ static int forward_generic(const char *who, const void *x, int x_dtype, int64_t 
                            const float *const *conv_b, const float *pol_w, const float *pol_b,
                            const float *val_w, const float *val_b, int prec, void *workspace,
                            size_t workspace_bytes, float *logits, float *value, int mask_mode,
-                           const uint8_t *legal, float fill, void *stream, bool pack = true) {
+                           const uint8_t *legal, float fill, void *stream) {
   if (!valid_prec(prec) || !valid_input(x_dtype) || groups < 1 || boards_per_group < 0 ||
       kernels == nullptr || (boards_per_group > 0 && groups > INT64_MAX / boards_per_group)) {
     set_error("%s: bad precision %d, input type %d, groups %lld, boards %lld or null kernels", who,
@@ -545,22 +545,13 @@ static int forward_generic(const char *who, const void *x, int x_dtype, int64_t 
     return C6_EINVAL;
   }
   C6_REQUIRE_DEVICE(who);
-  // A network that fits the one-launch kernel does not need the workspace for its activations: its weights are packed
-  // there, where they fit (9 x 9, kernels 5, 3, 3, 1,024 boards in fp32: 87 us with weights converted by every wave,
-  // 33 us so).
-  if (const size_t set = (small_packed_bytes(board, layers, kernels, channels, prec) + 15) & ~(size_t)15; set != 0) {
-    if (pack && groups <= 65535 && set <= workspace_bytes / (size_t)groups) {
-      const int rc2 = launch_small_pack(groups, board, layers, kernels, channels, conv_w, conv_b, pol_w, pol_b, val_w,
-                                        val_b, prec, workspace, set, static_cast<hipStream_t>(stream));
-      if (rc2 != C6_OK) return rc2;
-      return launch_small(x, x_dtype, groups, boards_per_group, board, layers, kernels, channels, workspace, set, nullptr,
-                          nullptr, nullptr, nullptr, nullptr, nullptr, prec, logits, value, mask_mode, legal, fill,
-                          static_cast<hipStream_t>(stream));
-    }
+  // A network that fits the one-launch kernel does not need the workspace, and leaves it alone: calls beside one another
+  // may share it.  (Nothing is packed into it, then: a caller who has room for that calls c6_generic_pack and
+  // c6_forward_generic_packed, 1,024 boards of 9 x 9, kernels 5, 3, 3, in fp32 87 -> 33 us.)
+  if (small_packed_bytes(board, layers, kernels, channels, prec) != 0)
     return launch_small(x, x_dtype, groups, boards_per_group, board, layers, kernels, channels, nullptr, 0, conv_w,
                         conv_b, pol_w, pol_b, val_w, val_b, prec, logits, value, mask_mode, legal, fill,
                         static_cast<hipStream_t>(stream));
-  }
   return launch_generic(x, x_dtype, batch, boards_per_group, board, layers, kernels, channels,
                         conv_w, conv_b, pol_w, pol_b, val_w, val_b, prec, workspace, logits, value,
                         mask_mode, legal, fill, static_cast<hipStream_t>(stream));
@@ -619,10 +610,9 @@ int c6_forward_generic_static(const void *x, int x_dtype, int64_t batch, int boa
   void *ws = nullptr;
   rc = static_scratch(&ws);
   if (rc != C6_OK) return rc;
-  // (no weights in the array: networks that need no workspace for their activations do not share it)
-  return forward_generic("c6_forward_generic", x, x_dtype, 1, batch, board, layers, kernels, channels, conv_w, conv_b,
-                         pol_w, pol_b, val_w, val_b, prec, ws, static_scratch_bytes(), logits, value, mask_mode, legal,
-                         fill, stream, false);
+  return c6_forward_generic(x, x_dtype, batch, board, layers, kernels, channels, conv_w, conv_b,
+                            pol_w, pol_b, val_w, val_b, prec, ws, static_scratch_bytes(), logits,
+                            value, mask_mode, legal, fill, stream);
 }
 
 int c6_generic_packed_bytes(int board, int layers, const int *kernels, const int *channels, int prec,

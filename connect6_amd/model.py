@@ -178,9 +178,7 @@ def run_forward_generic(
         nbytes = ctypes.c_size_t(0)
         _lib.check(lib.c6_generic_workspace_bytes(b, n, layers, cc, ctypes.byref(nbytes)),
                    "c6_generic_workspace_bytes")
-        # (room for the packed weights of a small network, which the call then packs there)
-        nbytes = max(int(nbytes.value), groups * _lib.generic_packed_bytes(n, kernels, channels, prec), 16)
-        workspace = torch.empty(nbytes, dtype=torch.uint8, device=dev)
+        workspace = torch.empty(max(int(nbytes.value), 16), dtype=torch.uint8, device=dev)
     if out is not None:
         logits, value = out
         if logits.shape != (b, n * n) or logits.dtype != torch.float32 or not logits.is_contiguous():

@@ -244,9 +244,10 @@ int c6_stream_capturing(void *stream);
  *   x        device [B,3,n,n] of element type x_dtype
  *   kernels, channels: HOST arrays of `layers` ints
  *   conv_w / conv_b:   HOST arrays of `layers` device fp32 pointers (PyTorch layouts)
- *   workspace: device, c6_generic_workspace_bytes(...) bytes, 16-byte aligned; where it also has room for
- *              c6_generic_packed_bytes(...) per weight set, a one-launch network's weights are packed there
- *              first, which is faster (1,024 boards of 9 x 9, kernels 5,3,3, fp32: 87 -> 32 us)
+ *   workspace: device, c6_generic_workspace_bytes(...) bytes, 16-byte aligned; neither read nor written for a
+ *              one-launch network, whose weights are read as they are (packed by c6_generic_pack in front of
+ *              every call and evaluated by c6_forward_generic_packed, 1,024 boards of 9 x 9, kernels 5,3,3,
+ *              take 33 us in fp32 instead of 87)
  *   logits fp32 [B,n*n] (may be NULL), value fp32 [B] (may be NULL; val_w may then be NULL) */
 int c6_generic_workspace_bytes(int64_t batch, int board, int layers, const int *channels,
                                size_t *bytes);

@@ -1,6 +1,8 @@
 """One-launch forward of small networks (c6_forward_generic_packed) against the oracle, at the sizes
 where its layout changes: boards of one square to 19 x 19, channels around multiples of 8 and 16,
 wide and 1x1 kernels, one to many boards per workgroup, several weight sets."""
+import ctypes
+
 import pytest
 import torch
 
@@ -183,20 +185,49 @@ def test_parameters_are_read_on_every_call(cuda, precision):
 
 @pytest.mark.parametrize("board,kernels,channels,batch", [(5, [3, 3], [8, 17], 3), (9, [5, 3, 3], [16, 32, 48], 70), (19, [7, 1], [33, 8], 9)])
 @pytest.mark.parametrize("prec", [_lib.PREC_F32, _lib.PREC_BF16, _lib.PREC_BF16F6])
-def test_weights_packed_into_the_workspace_or_read_as_they_are(cuda, board, kernels, channels, batch, prec):
+def test_weights_packed_for_the_call_or_read_as_they_are(cuda, board, kernels, channels, batch, prec):
     """The same bits; inputs that are exact in bf16 and inputs that are not, one of them in a batch of the other."""
     st = {k: v.to(cuda) for k, v in R.init_state(9, "torch_default", kernels=kernels, channels=channels).items()}
+    arch = architecture_bytes(kernels, channels)
     x = _inputs(batch, board, 8)
     x[:, 2] = 1.0
     for inexact in (False, True):
         if inexact:
             x[batch // 2, 1] *= 0.3
         with torch.inference_mode():
-            packed = run_forward_generic(x.to(cuda), st, kernels, channels, prec)
+            weights = pack_generic(st, board, kernels, channels, prec, cuda)
+            packed = run_packed_generic(x.to(cuda), weights, arch, prec)
             raw = run_forward_generic(x.to(cuda), st, kernels, channels, prec, static_workspace=True)
-            alone = run_forward_generic(x[:1].to(cuda), st, kernels, channels, prec)
+            alone = run_packed_generic(x[:1].to(cuda), weights, arch, prec)
         assert torch.equal(packed[0], raw[0]) and torch.equal(packed[1], raw[1])
         assert torch.equal(packed[0][:1], alone[0]) and torch.equal(packed[1][:1], alone[1])
+
+
+@pytest.mark.parametrize("groups", [1, 3])
+@pytest.mark.parametrize("prec", [_lib.PREC_F32, _lib.PREC_BF16])
+def test_the_workspace_of_a_one_launch_network_is_left_alone(cuda, groups, prec):
+    """Calls on several streams may share it, however large it is."""
+    board, kernels, channels, batch = 9, [5, 3, 3], [16, 32, 32], 20
+    states = [R.init_state(50 + i, "torch_default", kernels=kernels, channels=channels) for i in range(groups)]
+    st = {k: torch.stack([s[k] for s in states]).to(cuda) for k in states[0]}
+    x = _inputs(groups * batch, board, 4).to(cuda)
+    ints, ptrs, lib = ctypes.c_int * 3, ctypes.c_void_p * 3, _lib.load()
+    ks, cs = ints(*kernels), ints(*channels)
+    need = ctypes.c_size_t(0)
+    _lib.check(lib.c6_generic_workspace_bytes(groups * batch, board, 3, cs, ctypes.byref(need)), "c6_generic_workspace_bytes")
+    size = need.value + groups * _lib.generic_packed_bytes(board, kernels, channels, prec)
+    workspace = torch.full((size,), 0xA5, dtype=torch.uint8, device=cuda)
+    logits, value = torch.empty(groups * batch, board * board, device=cuda), torch.empty(groups * batch, device=cuda)
+    rc = lib.c6_forward_generic_grouped(
+        x.data_ptr(), _lib.DT_F32, groups, batch, board, 3, ks, cs, ptrs(*[st[f"convs.{i}.weight"].data_ptr() for i in range(3)]),
+        ptrs(*[st[f"convs.{i}.bias"].data_ptr() for i in range(3)]), *[st[f"{h}_output.{k}"].data_ptr() for h in ("policy", "value")
+                                                                      for k in ("weight", "bias")],
+        prec, workspace.data_ptr(), size, logits.data_ptr(), value.data_ptr(), _lib.MASK_NONE, None, 0.0, _lib.stream_ptr(cuda))
+    _lib.check(rc, "c6_forward_generic_grouped")
+    assert bool((workspace == 0xA5).all())
+    packed = pack_generic(st, board, kernels, channels, prec, cuda, groups=groups)
+    want = run_packed_generic(x, packed, architecture_bytes(kernels, channels), prec, groups=groups)
+    assert torch.equal(logits, want[0]) and torch.equal(value, want[1])
 
 
 @pytest.mark.parametrize("board,kernels,channels,batch", [(1, [1], [1], 70), (9, [3], [48], 300), (19, [5], [17], 40)])

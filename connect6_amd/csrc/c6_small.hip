@@ -51,7 +51,7 @@ struct SmallParams {
   int n, nn, layers, nb;       // nb: boards per workgroup
   unsigned n_magic, nn_magic;
   int table_off, pix_off, val_off, tail_off;  // LDS: offset tables, squares, value sums, the packed tail
-  int tail_floats;
+  int tail_floats;             // of the copy in LDS (0: none)
   int bias_total;
   float *logits, *value;
   int mask_mode;
@@ -273,10 +273,11 @@ __device__ __forceinline__ float small_silu2(float u) {
 // kernels 7,3,3,3,3 and 32 channels 64 -> 53 us).  The MFMAs are 8 us of it at 2.4 GHz, all but the contractions 8 us
 // (launch, staging, epilogues); the rest is the two waves per SIMD meeting at two barriers per layer and the reads of
 // weights and activations, some 2 and 3 us.
-template <class A, int PT, bool RAW>
-__global__ __launch_bounds__(64 * kSmallMaxWaves) void small_net_kernel(const SmallParams prm) {
+enum : int { kTailInLds, kTailFar, kTailNone };   // (the last: weights read as they are)
+template <class A, int PT, int TAIL>
+__device__ __forceinline__ void small_net(const SmallParams &prm, unsigned char *smem) {
+  constexpr bool RAW = TAIL == kTailNone;
   constexpr int NA = A::NA;
-  extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
   const int tid = threadIdx.x, threads = blockDim.x;
   const int lane = tid & 63, wave = tid >> 6, q = lane >> 4;
   const int n = prm.n, nn = prm.nn;
@@ -290,7 +291,11 @@ __global__ __launch_bounds__(64 * kSmallMaxWaves) void small_net_kernel(const Sm
   const int boards = (int)(prm.per_group - first < prm.nb ? prm.per_group - first : prm.nb);
   const long long b0 = g * prm.per_group + first;
   const unsigned char *weights = prm.packed + (size_t)g * prm.packed_stride;
-  const float *tail = reinterpret_cast<const float *>(smem + prm.tail_off);   // (a copy: no layer starts behind its loads)
+  // Four words of the packed tail, from `at` on (+ 4 words per lane group): of a copy in LDS, so that no layer starts
+  // behind their loads, or (small_full_kernel) from where they lie.
+  auto tail4 = [&](int at, int group) __attribute__((always_inline)) {
+    return *reinterpret_cast<const f32x4 *>((TAIL == kTailInLds ? smem + prm.tail_off : weights + prm.tail) + 4 * at + 16 * group);
+  };
   const int npx = boards * nn;
 
   // a thread's square (there are as many threads as squares) and its input, asked for before anything else
@@ -301,7 +306,7 @@ __global__ __launch_bounds__(64 * kSmallMaxWaves) void small_net_kernel(const Sm
   for (int ch = 0; ch < 3; ++ch)
     xin[ch] = has ? small_load(prm.x, prm.x_dtype, ((size_t)(b0 + my_b) * 3 + ch) * nn + my_s) : 0.0f;
   if (has) s_pix[tid] = my_b << 16 | my_r << 8 | my_c;
-  if constexpr (!RAW)
+  if constexpr (TAIL == kTailInLds)
     for (int i = tid; i < prm.tail_floats / 4; i += threads)
       reinterpret_cast<v4i *>(smem + prm.tail_off)[i] = reinterpret_cast<const v4i *>(weights + prm.tail)[i];
   // every layer's table of offsets (16-byte units)
@@ -369,7 +374,7 @@ __global__ __launch_bounds__(64 * kSmallMaxWaves) void small_net_kernel(const Sm
         for (int t = 0; t < CT; ++t) {
           f32x4 b = {0.0f, 0.0f, 0.0f, 0.0f};
           if constexpr (!RAW) {  // (the tail holds zeros up to the next multiple of sixteen channels)
-            b = *reinterpret_cast<const f32x4 *>(tail + L.bias0 + 16 * t + 4 * q);
+            b = tail4(L.bias0 + 16 * t, q);
           } else if (prm.conv_b[l] != nullptr) {
 #pragma unroll
             for (int i = 0; i < 4; ++i)
@@ -396,7 +401,7 @@ __global__ __launch_bounds__(64 * kSmallMaxWaves) void small_net_kernel(const Sm
         for (int t = 0; t < CT; ++t) {
           f32x4 bl = {0.0f, 0.0f, 0.0f, 0.0f};   // what rounding the scaled biases left out, with the small products
           if constexpr (small_scaled<A>() && !RAW) {
-            bl = *reinterpret_cast<const f32x4 *>(tail + small_low(prm.bias_total) + L.bias0 + 16 * t + 4 * q);
+            bl = tail4(small_low(prm.bias_total) + L.bias0 + 16 * t, q);
           } else if constexpr (small_scaled<A>()) {
             if (prm.conv_b[l] != nullptr)
 #pragma unroll
@@ -418,7 +423,7 @@ __global__ __launch_bounds__(64 * kSmallMaxWaves) void small_net_kernel(const Sm
       }
       if (last) {
         if (busy) {
-          const float *pw = tail + prm.bias_total + 4 * q, *vw = pw + 16 * kSmallMaxTiles;
+          const int pw = prm.bias_total, vw = pw + 16 * kSmallMaxTiles;
 #pragma unroll
           for (int t = 0; t < CT; ++t) {
             f32x4 p4 = {0.0f, 0.0f, 0.0f, 0.0f}, v4 = p4;
@@ -431,8 +436,8 @@ __global__ __launch_bounds__(64 * kSmallMaxWaves) void small_net_kernel(const Sm
                 if (prm.val_w != nullptr) v4[i] = prm.val_w[(size_t)g * L.cout + ch];
               }
             } else {
-              p4 = *reinterpret_cast<const f32x4 *>(pw + 16 * t);
-              v4 = *reinterpret_cast<const f32x4 *>(vw + 16 * t);
+              p4 = tail4(pw + 16 * t, q);
+              v4 = tail4(vw + 16 * t, q);
             }
 #pragma unroll
             for (int j = 0; j < PT; ++j)
@@ -494,7 +499,7 @@ __global__ __launch_bounds__(64 * kSmallMaxWaves) void small_net_kernel(const Sm
     if (prm.pol_b != nullptr) pol_b = prm.pol_b[g];
     if (prm.val_b != nullptr) val_b = prm.val_b[g];
   } else {
-    const float *heads = tail + prm.bias_total + 2 * 16 * kSmallMaxTiles;
+    const f32x4 heads = tail4(prm.bias_total + 2 * 16 * kSmallMaxTiles, 0);
     pol_b = heads[0];
     val_b = heads[1];
   }
@@ -529,6 +534,17 @@ __global__ __launch_bounds__(64 * kSmallMaxWaves) void small_net_kernel(const Sm
       if (lane == 0) prm.value[b0 + b] = (float)tanh((double)v * (small_scaled<A>() ? 1.0 / kSmallScale : 1.0) / nn + (double)val_b);   // (one rounding)
     }
   }
+}
+
+template <class A, int PT, bool RAW> __global__ __launch_bounds__(64 * kSmallMaxWaves) void small_net_kernel(const SmallParams prm) {
+  extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
+  small_net<A, PT, RAW ? kTailNone : kTailInLds>(prm, smem);
+}
+// Networks whose activations leave no room for the tail's copy (19 x 19, ten layers of kernels 9 and 40 channels): a
+// kernel of their own, since a branch at each read of the tail cost the others 1 % (9 x 9, 1,024 boards).
+template <class A> __global__ __launch_bounds__(64 * kSmallMaxWaves) void small_full_kernel(const SmallParams prm) {
+  extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
+  small_net<A, 3, kTailFar>(prm, smem);
 }
 
 // ---- weights ---------------------------------------------------------------------------------
@@ -624,11 +640,12 @@ struct SmallPlan {
   size_t tail = 0, bytes = 0;
 };
 
-static int small_lds(const SmallPlan &pl, int nn, int nb, SmallParams *sp = nullptr) {
+// copy: with the packed tail behind the rest
+static int small_lds(const SmallPlan &pl, int nn, int nb, bool copy, SmallParams *sp = nullptr) {
   const int t = (nb * pl.boardb + 15) & ~15;
   const int p = (t + 2 * pl.entries + 15) & ~15;
   const int v = p + 4 * nb * nn;
-  const int w = (v + 4 * nb * nn + 15) & ~15, floats = (int)((pl.bytes - pl.tail) / 4);
+  const int w = (v + 4 * nb * nn + 15) & ~15, floats = copy ? (int)((pl.bytes - pl.tail) / 4) : 0;
   if (sp) sp->table_off = t, sp->pix_off = p, sp->val_off = v, sp->tail_off = w, sp->tail_floats = floats;
   return w + 4 * floats;
 }
@@ -671,7 +688,7 @@ static bool small_plan(int n, int layers, const int *kernels, const int *channel
   }
   pl.tail = (size_t)pl.frags * 1024;
   pl.bytes = pl.tail + (size_t)(small_low(pl.bias_total) + pl.bias_total) * 4;
-  return small_lds(pl, n * n, 1) <= kSmallLds;
+  return small_lds(pl, n * n, 1, false) <= kSmallLds;
 }
 
 size_t small_packed_bytes(int n, int layers, const int *kernels, const int *channels, int prec) {
@@ -723,20 +740,19 @@ int launch_small_pack(long long groups, int n, int layers, const int *kernels, c
   return small_done("small_pack_kernel");
 }
 
-template <class A, int PT, bool RAW = false> static int small_launch(const SmallParams &sp, unsigned grid, int waves, int lds, hipStream_t st) {
+template <auto KERNEL> static int small_launch(const SmallParams &sp, unsigned grid, int waves, int lds, hipStream_t st) {
   static thread_local int configured = -1;
   int dev = 0;
   hipError_t e = hipGetDevice(&dev);
   if (e == hipSuccess && configured != dev) {
-    e = hipFuncSetAttribute(reinterpret_cast<const void *>(&small_net_kernel<A, PT, RAW>),
-                            hipFuncAttributeMaxDynamicSharedMemorySize, kSmallLds);
+    e = hipFuncSetAttribute(reinterpret_cast<const void *>(KERNEL), hipFuncAttributeMaxDynamicSharedMemorySize, kSmallLds);
     if (e == hipSuccess) configured = dev;
   }
   if (e != hipSuccess) {
     set_error("small_net_kernel setup failed: %s", hipGetErrorString(e));
     return C6_ELAUNCH;
   }
-  hipLaunchKernelGGL((small_net_kernel<A, PT, RAW>), dim3(grid), dim3(64 * waves), lds, st, sp);
+  hipLaunchKernelGGL(KERNEL, dim3(grid), dim3(64 * waves), lds, st, sp);
   return small_done("small_net_kernel");
 }
 
@@ -754,14 +770,16 @@ int launch_small(const void *x, int x_dtype, long long groups, long long per_gro
   // Three tiles of 16 squares per wave read a weight fragment once for three MFMAs (18 in fp32), so
   // that the matrix cores and not the reads from L2 bound the wave; that takes enough squares to
   // give every SIMD of the chip a wave.  Below that one tile per wave: latency counts.
-  // (Weights straight from the tensors are converted by every wave: always three tiles.)
-  const bool wide = groups * per_group * nn >= 48LL * 1024 || nn > 16 * kSmallMaxWaves || packed == nullptr;
+  // (Weights straight from the tensors are converted by every wave: always three tiles.  So where there is no room for
+  // the tail's copy: one kernel for those is enough.)
+  const bool copy = packed != nullptr && small_lds(pl, nn, 1, true) <= kSmallLds;
+  const bool wide = groups * per_group * nn >= 48LL * 1024 || nn > 16 * kSmallMaxWaves || !copy;
   const int span = wide ? 48 : 16;
   // boards per workgroup: four waves' worth of squares (two workgroups and more share a CU), fewer
   // where that would leave CUs without a workgroup, one board at least
   long long nb = 4 * span / nn;
   if (nb > per_group) nb = per_group;
-  while (nb > 1 && (groups * ((per_group + nb - 1) / nb) < 256 || small_lds(pl, nn, (int)nb) > kSmallLds / 2))
+  while (nb > 1 && (groups * ((per_group + nb - 1) / nb) < 256 || small_lds(pl, nn, (int)nb, copy) > kSmallLds / 2))
     --nb;
   if (nb < 1) nb = 1;
   SmallParams sp;
@@ -793,7 +811,7 @@ int launch_small(const void *x, int x_dtype, long long groups, long long per_gro
   sp.pol_b = pol_b;
   sp.val_w = val_w;
   sp.val_b = val_b;
-  const int lds = small_lds(pl, nn, (int)nb, &sp);
+  const int lds = small_lds(pl, nn, (int)nb, copy, &sp);
   const int waves = (int)((nb * nn + span - 1) / span);
   const long long grid = groups * sp.wgs_per_group;
   if (grid > 0x7fffffffLL) {
@@ -801,9 +819,10 @@ int launch_small(const void *x, int x_dtype, long long groups, long long per_gro
     return C6_EINVAL;
   }
 #define C6_SMALL(A)                                                           \
-  if (packed == nullptr) return small_launch<A, 3, true>(sp, (unsigned)grid, waves, lds, st); \
-  return wide ? small_launch<A, 3>(sp, (unsigned)grid, waves, lds, st)        \
-              : small_launch<A, 1>(sp, (unsigned)grid, waves, lds, st)
+  if (packed == nullptr) return small_launch<small_net_kernel<A, 3, true>>(sp, (unsigned)grid, waves, lds, st); \
+  if (!copy) return small_launch<small_full_kernel<A>>(sp, (unsigned)grid, waves, lds, st);                      \
+  return wide ? small_launch<small_net_kernel<A, 3, false>>(sp, (unsigned)grid, waves, lds, st)                 \
+              : small_launch<small_net_kernel<A, 1, false>>(sp, (unsigned)grid, waves, lds, st)
   using F32 = SmallArith<3, 3, false>;
   using W16 = SmallArith<3, 1, false>;
   using B16 = SmallArith<1, 1, false>;

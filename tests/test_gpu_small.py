@@ -255,6 +255,26 @@ def test_one_layer_with_inputs_that_are_not_exact_in_bf16(cuda, board, kernels, 
             assert rel_l2(lg, lo) <= 5e-6 and rel_l2(vg, vo) <= 5e-6
 
 
+@pytest.mark.parametrize("board,kernels,channels,batch", [
+    (18, [7] * 8, [48] * 8, 3), (16, [9] * 15, [48] * 15, 2), (11, [17, 17], [48, 48], 1), (19, [11] * 16, [32] * 16, 300)])
+def test_networks_that_fill_the_lds(cuda, board, kernels, channels, batch):
+    """No room beside the activations for a copy of the biases and head weights: one launch all the same."""
+    states = [R.init_state(60 + i, "torch_default", kernels=kernels, channels=channels) for i in range(2)]
+    stacked = {k: torch.stack([s[k] for s in states]).to(cuda) for k in states[0]}
+    x, arch = _inputs(2 * batch, board, 7).to(cuda), architecture_bytes(kernels, channels)
+    for prec in (_lib.PREC_F32, _lib.PREC_BF16F6):
+        packed = pack_generic(stacked, board, kernels, channels, prec, cuda, groups=2)
+        lg, vg = run_packed_generic(x, packed, arch, prec, groups=2)
+        for i, st in enumerate(states):
+            part = slice(i * batch, (i + 1) * batch)
+            raw = run_forward_generic(x[part], {k: v.to(cuda) for k, v in st.items()}, kernels, channels, prec)
+            assert torch.equal(lg[part], raw[0]) and torch.equal(vg[part], raw[1])
+            if prec == _lib.PREC_F32 and batch <= 3:
+                l64, v64 = R.forward({k: v.double() for k, v in st.items()}, x[part].double().cpu())
+                # sixteen layers at most, each a sum of at most 17 x 17 x 48 products rounded to fp32 (2^-24)
+                assert rel_l2(lg[part], l64) <= 1e-5 and rel_l2(vg[part], v64) <= 1e-5
+
+
 def test_board_size_set_after_construction(cuda):
     """The network is fully convolutional: the same module on boards of another size."""
     for kernels, channels, first, second in ((None, None, 19, 9), ([3, 3], [8, 16], 7, 13)):

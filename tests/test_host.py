@@ -113,6 +113,37 @@ def test_packed_sizes_follow_the_layout():
         _lib.packed_bytes(9)
 
 
+def test_small_networks_with_a_packed_form():
+    """One board's padded activations (three bf16 planes in fp32, one in bf16), two bytes per group of eight contracted
+    values, a square's place and value sum: 160 KiB.  Nothing else counts (a copy of the biases and head weights is
+    made where it fits)."""
+    def fits(board, kernels, channels, planes):
+        cin, largest, entries = 3, 0, 0
+        for k, cout in zip(kernels, channels):
+            blocks, radius = -(-cin // 8), k // 2
+            positions = (board + 2 * radius) * (board + radius) + radius
+            record = 16 * planes * blocks + (0 if planes * blocks % 2 else 16)
+            largest, entries = max(largest, positions * record), entries + (k * k * blocks + 3) // 4 * 4
+            cin = cout
+        tables = -(-largest // 16) * 16 + 2 * entries
+        return entries <= 8192 and -(-tables // 16) * 16 + 8 * board * board <= 160 * 1024
+
+    seen = 0
+    for board in (1, 5, 9, 11, 12, 15, 16, 17, 18, 19):
+        for k in (1, 3, 7, 9, 11, 13, 15, 17):
+            for c in (8, 32, 40, 48):
+                for layers in (1, 2, 4, 6, 8, 12, 14, 16):
+                    for prec, planes in ((_lib.PREC_F32, 3), (_lib.PREC_BF16F6, 3), (_lib.PREC_BF16, 1)):
+                        want = fits(board, [k] * layers, [c] * layers, planes)
+                        seen += want
+                        assert (_lib.generic_packed_bytes(board, [k] * layers, [c] * layers, prec) > 0) == want, (board, k, c, layers)
+    assert seen > 1000
+    # full of activations
+    for board, k, c, layers in ((18, 7, 48, 8), (18, 7, 48, 12), (16, 9, 48, 15), (19, 9, 40, 14), (19, 11, 32, 16), (11, 17, 48, 2)):
+        assert _lib.generic_packed_bytes(board, [k] * layers, [c] * layers, _lib.PREC_F32) > 0
+    assert _lib.generic_packed_bytes(18, [7] * 13, [48] * 13, _lib.PREC_F32) == 0
+
+
 def test_entry_points_reject_bad_arguments_before_touching_the_device():
     lib = _lib.load()
     assert lib.c6_forward(None, 0, 1, 4, None, 0, 1, None, None, 0, None, 0.0, None, 1.0, None, None, None) == -1

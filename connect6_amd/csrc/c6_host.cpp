@@ -115,7 +115,17 @@ struct Team {
   uint32_t tag = 0;
 };
 
-// The flag words are kept per stream, with the last tag written into them: calls on one stream follow
+// The tag of a call behind one that took `last` and last + 1, or 1 where the flag words have to be cleared for it: a word
+// that says which XCD a workgroup is on holds a tag's low 28 bits, and one in a slot that few calls use may be as old as
+// the words.  A cascade's second pass takes the next tag, so a call counts two.
+constexpr uint32_t kTagsEnd = 1u << 28;
+constexpr uint32_t next_tag(uint32_t last) { return last == 0 || last > kTagsEnd - 4 ? 1 : last + 2; }
+PyObject *team_tag(PyObject *, PyObject *last) {
+  const unsigned long v = PyLong_AsUnsignedLong(last);
+  return PyErr_Occurred() ? nullptr : PyLong_FromUnsignedLong(next_tag((uint32_t)v));
+}
+
+// The flag words are kept per stream, with the last call's tag: calls on one stream follow
 // one another, so a tag counted up per call is one that no word holds.  Sixteen streams at most; the
 // one that has waited longest gives its words back.  (Only under the interpreter's lock.)  Inside a
 // graph capture the words are the graph's own, cleared in the graph: a replay has the same tag.
@@ -153,14 +163,12 @@ Team team_buffers(int prec, int64_t boards, const at::Device &dev, void *stream)
     kept.push_back(Kept{dev.index(), stream, {}, 0, 0});
     k = &kept.back();
   }
-  if (!k->flags.defined() || (size_t)k->flags.nbytes() < flag_bytes || k->tag >= UINT32_MAX - 4) {
-    k->flags = zeros((int64_t)(flag_bytes / 4));
-    k->tag = 0;
-  }
+  if (!k->flags.defined() || (size_t)k->flags.nbytes() < flag_bytes) k->tag = 0;
+  t.tag = next_tag(k->tag);
+  if (t.tag == 1) k->flags = zeros((int64_t)(flag_bytes / 4));
+  k->tag = t.tag;
   k->used = ++clock;
   t.flags = k->flags;
-  t.tag = k->tag + 1;
-  k->tag += 2;   // (a cascade's second pass takes the next one)
   return t;
 }
 
@@ -634,6 +642,7 @@ PyMethodDef methods[] = {C6_FAST(bind),        C6_FAST(forward),        C6_FAST(
                          C6_FAST(mask_logits), C6_FAST(sample),         C6_FAST(env_step),
                          C6_FAST(canonical_input), C6_FAST(forward_generic), C6_FAST(forward_generic_module),
                          {"parameters", parameters, METH_O, nullptr},
+                         {"team_tag", team_tag, METH_O, nullptr},
                          {nullptr, nullptr, 0, nullptr}};
 PyModuleDef module_def = {PyModuleDef_HEAD_INIT, "_c6_host", nullptr, -1, methods, nullptr, nullptr, nullptr, nullptr};
 

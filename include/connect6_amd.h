@@ -200,8 +200,9 @@ int c6_forward_boards_cascade(const int8_t *boards, const int8_t *player,
  *              done: no word may hold `tag` when the launch starts, and no other launch may use them
  *              at the same time.  (Words zeroed once and a tag counted up from 1 by every launch on
  *              a stream; in a captured graph, words cleared inside the graph.)
- *   tag        not 0; a cascade also uses tag + 1 (tags of a buffer should differ in their low 28 bits, as
- *              those of 2^28 calls in turn do: which XCD a workgroup is on is told with those)
+ *   tag        not 0; a cascade also uses tag + 1.  Which XCD a workgroup is on is told with a tag's low 28
+ *              bits, so those are not used twice either between two clearings of the words: after 2^27 calls
+ *              that count two each, clear them and begin at 1 again
  *   polls      how often a workgroup looks at a flag before it computes the piece itself; 0: 64
  * No synchronisation with the host.  Every wait is bounded: a workgroup that has
  * waited too long computes what it waits for. */

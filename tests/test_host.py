@@ -425,6 +425,19 @@ def test_native_host_side_refuses_what_is_no_tensor():
             call()
 
 
+def test_tags_of_a_streams_flag_words():
+    """A call's two tags, in turn; a word that names an XCD holds 28 bits of one, so they begin anew (at 1, on cleared
+    words) before those come round."""
+    step, end = _lib.host().team_tag, 1 << 28
+    assert [step(v) for v in (0, 1, 3, 5)] == [1, 3, 5, 7]
+    last, seen = end - 21, []
+    while last != 1:
+        seen += [last, last + 1]
+        last = step(last)
+    assert seen == list(range(end - 21, end - 1))
+    assert step(end + 1) == 1 and step(2**32 - 2) == 1
+
+
 def test_native_host_side_checks_a_modules_parameters():
     from connect6_amd.model import architecture_bytes
 

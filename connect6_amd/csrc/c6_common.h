@@ -241,9 +241,14 @@ constexpr size_t cascade_packed_bytes(int prec) {
 // writes their number when its run is done: no atomic operation, and nothing to clear before a
 // call.  The second pass sums the counts up (every workgroup for itself) and deals the listed boards
 // out evenly.  Layout, in int32: [0] boards listed in all (written by the second pass, for the
-// caller), [4, 4 + kCascadeMaxRuns) the counts per run, then the lists, `per` entries per run
-// (runs x per <= boards + kCascadeMaxRuns).
+// caller), [4, 4 + kCascadeMaxRuns) the counts per run, then the lists: `per` entries for each of the `grid` runs
+// that a workgroup evaluates (per = its share of their boards, rounded up: less than `grid` entries more than
+// those), and behind them one for each board that a team shares, a run by itself.  So the entries are fewer than the
+// boards and kCascadeMaxRuns together, whatever the rules share out.
 constexpr int kCascadeMaxRuns = 1024;   // workgroups of the first pass: two per compute unit, at most
+constexpr long long redo_entry(long long run, long long grid, long long per) {   // where a run's list starts
+  return run < grid ? run * per : grid * per + (run - grid);
+}
 constexpr size_t cascade_workspace_bytes(long long boards) {
   return (size_t)(16 + 4 * (long long)kCascadeMaxRuns + 4 * (boards + kCascadeMaxRuns) + 15) & ~(size_t)15;
 }
@@ -284,9 +289,10 @@ struct FwdParams {
   float redo_threshold = 0.0f;    // first pass: < 0 = every board goes on the list
   int *redo_count = nullptr;      // boards listed in all (device memory; the second pass writes it)
   int *redo_counts = nullptr;     // boards listed by run r of the first pass
-  int *redo_list = nullptr;       // run r's list starts at entry r * redo_per
-  int redo_runs = 0;              // workgroups (runs of boards) of the first pass
-  int redo_per = 0;               // boards per run of the first pass
+  int *redo_list = nullptr;       // run r's list starts at entry redo_entry(r, redo_grid, redo_per)
+  int redo_runs = 0;              // runs of boards of the first pass
+  int redo_grid = 0;              // ... those of a workgroup each, in front of those of a board each
+  int redo_per = 0;               // boards per workgroup's run of the first pass
 };
 
 // Few boards: several workgroups per board (c6_team.h)
@@ -296,7 +302,6 @@ struct TeamParams {
   unsigned *flags;      // kTeamFlags words per board
   unsigned tag;
   unsigned first = 0;   // the first of the f.total_boards boards
-  unsigned run = 0;     // cascade, first pass: the run that lists it (each board of a team is a run)
   int polls;            // of a flag (about 0.7 us each) before a workgroup helps itself
 };
 constexpr int kTeamFlags = 256;   // words per board

@@ -1123,8 +1123,8 @@ __device__ __forceinline__ void pipe_layer(
 }
 
 // ---- cascade, second pass (prm.redo_mode == kRedoConsume) ----
-// The boards to evaluate are the ones the first pass listed, run by run (run r: redo_counts[r] boards at
-// redo_list[r * redo_per ...]).  Every workgroup sums the counts up for itself -- `runs[r]` = boards listed by the
+// The boards to evaluate are the ones the first pass listed, run by run (run r: redo_counts[r] boards, its list from
+// redo_entry(r) on).  Every workgroup sums the counts up for itself -- `runs[r]` = boards listed by the
 // runs before r, `runs[redo_runs]` = all of them, which is what it returns -- and the listed boards, numbered in that
 // order, are dealt out like the boards of any batch.
 template <class P> __device__ __forceinline__ unsigned listed_runs(const FwdParams &prm, unsigned char *smem) {
@@ -1161,7 +1161,7 @@ template <class P> __device__ __forceinline__ unsigned listed_board(const FwdPar
     const int mid = (lo + hi) >> 1;
     if ((unsigned)runs[mid] <= i) lo = mid; else hi = mid;
   }
-  return (unsigned)prm.redo_list[(size_t)lo * prm.redo_per + (i - (unsigned)runs[lo])];
+  return (unsigned)prm.redo_list[redo_entry(lo, prm.redo_grid, prm.redo_per) + (i - (unsigned)runs[lo])];
 }
 
 // A workgroup's share of n_items boards: the batch's, or (LISTED) the first of those that a cascade's first pass listed.
@@ -2486,7 +2486,6 @@ int dispatch_team(int prec, const TeamParams &tp, hipStream_t st) {
   }
   part.f.total_boards = shared;
   part.first = (unsigned)(all - shared);
-  if (tp.f.redo_mode == kRedoDetect) part.run = (unsigned)(tp.f.redo_runs - shared);
   return m.launch(part, cus, st);   // (workgroups without a board end at once)
 }
 
@@ -2515,6 +2514,7 @@ int dispatch_cascade(int prec, const FwdParams &fp, float threshold, void *works
   first.redo_counts = ws + 4;
   first.redo_list = ws + 4 + kCascadeMaxRuns;
   first.redo_runs = (int)runs;
+  first.redo_grid = (int)grid;
   first.redo_per = single > 0 ? (int)((single + grid - 1) / grid) : 1;
   const unsigned char *packed2 = fp.packed + kCascadeSecondOffset;
   TeamParams tp{};   // (no exchange memory: no board is shared)

@@ -987,8 +987,8 @@ __device__ __forceinline__ void team_board(const TeamParams &prm, unsigned char 
         const bool again = wave_margin_below(
             lane, f.redo_threshold, [&](int i) { return lgt[i]; }, [&](int i) { return (occ[i] & 2) == 0; });
         if (lane == 0) {
-          __hip_atomic_store(&f.redo_counts[prm.run + slot], again ? 1 : 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-          f.redo_list[(size_t)(prm.run + slot) * f.redo_per] = (int)b;
+          __hip_atomic_store(&f.redo_counts[(unsigned)f.redo_grid + slot], again ? 1 : 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+          f.redo_list[redo_entry(f.redo_grid + (long long)slot, f.redo_grid, f.redo_per)] = (int)b;
           if (again) store_flag(kTeamListed);   // (in front of the stage's flag)
         }
       }

@@ -144,6 +144,40 @@ def test_small_networks_with_a_packed_form():
     assert _lib.generic_packed_bytes(18, [7] * 13, [48] * 13, _lib.PREC_F32) == 0
 
 
+def test_cascade_lists_stay_within_the_workspace(tmp_path):
+    """Runs of a workgroup's share of the boards, then runs of one board that a team shares, as many as the counts have
+    room for: the last entry lies within cascade_workspace_bytes(boards), and no two lists overlap."""
+    import os
+    import subprocess
+
+    source = tmp_path / "lists.cpp"
+    source.write_text("""#include "c6_common.h"
+using namespace c6;
+constexpr bool fits(long long single, long long grid, long long shared) {
+  const long long per = single > 0 ? (single + grid - 1) / grid : 1, runs = grid + shared;
+  for (long long r : {0LL, grid - 1, grid, runs - 1})
+    if (r >= 0 && r < runs && redo_entry(r + 1, grid, per) - redo_entry(r, grid, per) != (r < grid ? per : 1)) return false;
+  const size_t end = 4 * (4 + kCascadeMaxRuns + redo_entry(runs, grid, per));
+  return end <= cascade_workspace_bytes(single + shared);
+}
+constexpr bool all() {
+  for (long long grid : {0, 1, 7, 64, 256, 511, 512, 984, 1024})
+    for (long long rounds : {1, 2, 3, 6, 12, 100, 1000})
+      for (long long more : {-1, 0, 1})
+        for (long long shared : {0LL, 1LL, 40LL, 128LL, kCascadeMaxRuns - grid}) {
+          const long long single = grid * rounds + more;
+          if (grid == 0 ? !fits(0, 0, shared) : (single >= grid && grid + shared <= kCascadeMaxRuns && !fits(single, grid, shared)))
+            return false;
+        }
+  return true;
+}
+static_assert(all(), "lists");
+""")
+    proc = subprocess.run([os.environ.get("HIPCC", "/opt/rocm/bin/hipcc"), "-x", "hip", "--cuda-host-only", "-nogpulib", "-std=c++17", "-fsyntax-only",
+                           f"-I{ROOT / 'connect6_amd' / 'csrc'}", str(source)], capture_output=True, text=True)
+    assert proc.returncode == 0, proc.stderr
+
+
 def test_entry_points_reject_bad_arguments_before_touching_the_device():
     lib = _lib.load()
     assert lib.c6_forward(None, 0, 1, 4, None, 0, 1, None, None, 0, None, 0.0, None, 1.0, None, None, None) == -1

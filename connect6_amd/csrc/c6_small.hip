@@ -27,6 +27,8 @@ constexpr int kSmallMaxWaves = 8;
 constexpr int kSmallTableEntries = 8192;
 constexpr int kSmallLds = 160 * 1024;
 
+constexpr int kPlanes = 3;             // of an input board
+
 struct SmallLayer {
   int k, r;              // kernel size and its padding k / 2
   int cin, cb;           // input channels and their blocks of eight
@@ -158,9 +160,9 @@ template <class A, bool FIRST> struct RawWeights {   // FIRST: the first layer's
     for (int t = 0; t < CT; ++t) {
       const int co = 16 * t + (ln & 15);
       const bool row = e < blocks && co < cout;
-      unsigned short pl[8][A::NW];
+      unsigned short pl[8][A::NW] = {};
 #pragma unroll
-      for (int i = 0; i < 8; ++i) {
+      for (int i = 0; i < (FIRST ? kPlanes : 8); ++i) {   // (the first layer's other channels are padding)
         const bool in = row && ci0 + i < cin;
         const float v = w[in ? (size_t)(co * cin + ci0 + i) * kk + tap : 0];
         if constexpr (small_scaled<A>() && FIRST) small_weight_planes64<A>(small_scale<A>(in ? v : 0.0f, true), pl[i]);

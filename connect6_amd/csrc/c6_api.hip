@@ -547,7 +547,7 @@ static int forward_generic(const char *who, const void *x, int x_dtype, int64_t 
   C6_REQUIRE_DEVICE(who);
   // A network that fits the one-launch kernel does not need the workspace, and leaves it alone: calls beside one another
   // may share it.  (Nothing is packed into it, then: a caller who has room for that calls c6_generic_pack and
-  // c6_forward_generic_packed, 1,024 boards of 9 x 9, kernels 5, 3, 3, in fp32 87 -> 33 us.)
+  // c6_forward_generic_packed, 1,024 boards of 9 x 9, kernels 5, 3, 3, in fp32 82 -> 28 us.)
   if (small_packed_bytes(board, layers, kernels, channels, prec) != 0)
     return launch_small(x, x_dtype, groups, boards_per_group, board, layers, kernels, channels, nullptr, 0, conv_w,
                         conv_b, pol_w, pol_b, val_w, val_b, prec, logits, value, mask_mode, legal, fill,

@@ -2427,12 +2427,19 @@ static int second_mode(int cascade) { return cascade == C6_PREC_BF16C ? C6_PREC_
 // workgroup per CU the rest (fp32: 257 boards 607 -> 373 us, 341 boards 607 -> 450 us, 384 boards 600 -> 531 us, 777 boards 1,190 ->
 // 975 us; bf16 + fp6 + low weights, 298 boards: 239 -> 191 us).  In the modes that put two workgroups on a CU a rest is
 // a board more for some CUs; behind an odd number of rounds, where that is a fourth board beside three, a sixth beside
-// five ..., it takes longer than teams do, unless so few CUs have it that their clock makes up for it.  fp16, all as
-// one / rest in teams, us (the cascade, 768 + 9: 298 / 286, 1,280 + 9: 437 / 421, 2,816 + 2: 726 / 748, + 9: 762 / 748):
-//   768 + 1  202 / 194   + 9  208 / 195   + 24  208 / 205   + 40  208 / 205      512 + 9  141 / 144
-//   1,280 + 1  307 / 303   + 9  317 / 304   + 40  317 / 314                      1,024 + 9  249 / 252
-//   2,816 + 1  615 / 625   + 2  631 / 625   + 9  639 / 626   + 40  640 / 637
-//   4,864 + 2  1,057 / 1,061   + 9  1,070 / 1,061   + 40  1,072 / 1,074
+// five ..., it takes longer than teams do, unless so few CUs have it that their clock makes up for it.  One line for fp16,
+// bf16 and the cascade's first pass: more than half as many boards as rounds.  It leaves out a few sizes where teams would
+// gain 1 to 4 % (fp16, 768 + 1 boards 202 / 194, 1,280 + 1 307 / 303, 2,816 + 2 631 / 625) for those where they lose
+// (2,816 + 1 615 / 625, the cascade at 2,816 + 2 726 / 748); rounds end at eleven: 4,864 + 2 1,057 / 1,061, + 9 1,070 /
+// 1,061, + 40 1,072 / 1,074; even ones fill a CU's second place: 512 + 9 141 / 144, 1,024 + 9 249 / 252.  What the line takes in,
+// all as one / rest in teams, us (medians of two runs a side, which differ by 0.5 %, the cascade's above 2,304 boards by 1 %;
+// the cascade's first with the second pass as two launches, 3 us):
+//           fp16 + 9     + 40         bf16 + 9     + 40         cascade + 9   + 40
+//   768     208 / 195    209 / 206    198 / 185    199 / 195    276 / 264     291 / 290
+//   1,280   316 / 303    315 / 311    299 / 286    299 / 296    425 / 412     426 / 421
+//   1,792   423 / 409    423 / 419    402 / 388    402 / 398    528 / 517     530 / 527
+//   2,304   530 / 516    530 / 527    502 / 490    503 / 500    632 / 627     636 / 639
+//   2,816   638 / 627    639 / 639    604 / 594    605 / 605    736 / 730     738 / 741
 static long long team_boards(int prec, long long boards, int cus) {
   const TeamMode m = team_mode(prec);
   if (m.launch == nullptr) return 0;

@@ -269,7 +269,7 @@ __device__ __forceinline__ float small_silu2(float u) {
 // their padding columns), so that a (tap, block of eight channels) is a constant offset, looked up
 // in a table by the lane group that contracts it.
 //
-// Measured on 1024 boards of the 9x9 network above, fp32: 23 us (914 us layer by layer; 26 with a SiLU that puts the
+// Measured on 1024 boards of the 9x9 network above, fp32, calls in a row: 23 us (914 us layer by layer; 26 with a SiLU that puts the
 // factor log2(e) in by itself, planes split value by value, a chunk's offset read in front of its operands, and the
 // input loaded board by board behind the tables; 4096 boards of four such networks 96 -> 83 us, twenty 19x19 boards of
 // kernels 7,3,3,3,3 and 32 channels 64 -> 53 us).  The MFMAs are 8 us of it at 2.4 GHz, all but the contractions 8 us

@@ -19,8 +19,8 @@
 // then on they stay in that XCD's L2, where the loads find them.  Measured between neighbours of a team on one XCD,
 // store, wait for the acknowledgement, flag, load: 4 KB a side 2.2 us with the stores going through to memory, 1.1 us
 // with stores that stay in L2; 12 KB 3.9 and 1.9 us; 0.3 KB 1.5 and 0.7 us.  (Each word with its tag beside it, no
-// flag and no wait, 1.0, 2.0 and 0.5 us: not worth twice the words and memory of its own.)  One board 38 -> 33 us in
-// bf16, 66 -> 60 us in fp32, 53 fp32 boards 123 -> 117 us, with what else changed there: weights asked for in front
+// flag and no wait, 1.0, 2.0 and 0.5 us: not worth twice the words and memory of its own.)  One board's forward 35.8 ->
+// 30.1 us in bf16, 65.5 -> 58.9 us in fp32, 53 fp32 boards 121 -> 115 us, with what else changed there: weights asked for in front
 // of the wait, addresses of exchanged squares formed once, biases and head weights from LDS.
 //
 // Nothing waits for a workgroup that may not be running: a wait is bounded, and a workgroup whose

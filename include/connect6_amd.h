@@ -248,7 +248,7 @@ int c6_stream_capturing(void *stream);
  *   workspace: device, c6_generic_workspace_bytes(...) bytes, 16-byte aligned; neither read nor written for a
  *              one-launch network, whose weights are read as they are (packed by c6_generic_pack in front of
  *              every call and evaluated by c6_forward_generic_packed, 1,024 boards of 9 x 9, kernels 5,3,3,
- *              take 33 us in fp32 instead of 87)
+ *              take 28 us in fp32 instead of 82)
  *   logits fp32 [B,n*n] (may be NULL), value fp32 [B] (may be NULL; val_w may then be NULL) */
 int c6_generic_workspace_bytes(int64_t batch, int board, int layers, const int *channels,
                                size_t *bytes);

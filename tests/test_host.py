@@ -63,6 +63,11 @@ def test_second_pass_kernels_use_no_scratch():
     assert len(second) == 4 and all(u["ScratchSize"] == 0 for u in second)
 
 
+def test_kernels_of_networks_that_fill_the_lds_use_no_scratch():
+    full = [u for name, u in _lib.resource_usage().items() if "small_full_kernel" in name]
+    assert len(full) == 4 and all(u["ScratchSize"] == 0 for u in full)
+
+
 def test_history_dtype_follows_the_reference_policy():
     # connect6/train.py:133-145
     cpu, gpu = torch.device("cpu"), torch.device("cuda", 0)

@@ -302,6 +302,7 @@ struct TeamParams {
   unsigned *flags;      // kTeamFlags words per board
   unsigned tag;
   unsigned first = 0;   // the first of the f.total_boards boards
+  unsigned rest = 0;    // duo_rest_kernel: boards behind the f.total_boards that one workgroup each serves
   int polls;            // of a flag (about 0.7 us each) before a workgroup helps itself
 };
 constexpr int kTeamFlags = 256;   // words per board

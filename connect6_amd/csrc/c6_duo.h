@@ -38,7 +38,7 @@ struct DuoGeo {
 // modes that have this kernel
 template <class P> constexpr bool has_duo() { return P::ID == C6_PREC_BF16 || P::ID == C6_PREC_F16; }
 
-// Workgroups of a forward over `boards` boards.  More boards than CUs: two workgroups per CU, where the mode
+// Workgroups of a forward over `boards` boards, all with one workgroup each.  More boards than CUs: two workgroups per CU, where the mode
 // has the kernel for it (257 boards take 86 us so, 112 in two rounds of one).  With a CU per board nothing
 // shares the matrix cores, and fused_pipe_kernel's 102 k cycles per board beat this kernel's 111 k.
 template <class P> inline long long forward_grid(long long boards, int cus) {
@@ -52,14 +52,15 @@ template <class P> inline long long forward_grid(long long boards, int cus) {
 // while the others arrive.
 struct DuoRun {
   unsigned run, first, count;
+  bool second;   // of the two that share a CU
 };
-__device__ __forceinline__ DuoRun duo_run(unsigned boards) {
-  const unsigned xcds = (gridDim.x % 8 == 0) ? 8 : 1, local = gridDim.x / xcds;
+__device__ __forceinline__ DuoRun duo_run(unsigned boards, unsigned grid) {
+  const unsigned xcds = (grid % 8 == 0) ? 8 : 1, local = grid / xcds;
   const unsigned x = blockIdx.x % xcds, l = blockIdx.x / xcds;
   const unsigned n0 = boards / xcds, n1 = boards % xcds;
   const unsigned part = x * n0 + (x < n1 ? x : n1), n = n0 + (x < n1 ? 1 : 0);
   const unsigned c0 = n / local, c1 = n % local;
-  return {x * local + l, part + l * c0 + (l < c1 ? l : c1), c0 + (l < c1 ? 1 : 0)};
+  return {x * local + l, part + l * c0 + (l < c1 ? l : c1), c0 + (l < c1 ? 1 : 0), 2 * l >= local};
 }
 
 // Depths, in k-steps: weights in flight (they come from L2 in some 800 cycles; a k-step is 96 cycles per
@@ -157,11 +158,11 @@ __device__ __forceinline__ void duo_layer(unsigned char *smem, const unsigned ch
   __syncthreads();
 }
 
-template <class P>
-__global__ __launch_bounds__(256, 2) void duo_forward_kernel(const FwdParams prm) {
+// This workgroup's run of the boards, dealt out to the first `grid` workgroups of the launch
+template <class P, bool REST = false>
+__device__ __forceinline__ void duo_boards(const FwdParams &prm, unsigned char *smem, unsigned grid) {
   using G = Geo<P>;
   using S = DuoGeo;
-  extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
   constexpr int THREADS = 256, ROUNDS = (kPix + THREADS - 1) / THREADS;
   constexpr bool kCanDetect = P::ID == C6_PREC_BF16;
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), h = lane >> 5;
@@ -217,13 +218,15 @@ __global__ __launch_bounds__(256, 2) void duo_forward_kernel(const FwdParams prm
     }
   };
 
-  const DuoRun mine = duo_run((unsigned)prm.total_boards);
+  const DuoRun mine = duo_run((unsigned)prm.total_boards, grid);
   const bool detect = kCanDetect && prm.redo_mode == kRedoDetect;
   int listed = 0;   // cascade: boards of this run listed so far (wave 1 counts)
   if (mine.count > 0) fetch_board(mine.first);
   for (unsigned b = mine.first; b < mine.first + mine.count; ++b) {
     int tidv = tid;
     asm volatile("" : "+v"(tidv));
+    // (duo_rest_kernel: its place is wanted)
+    if (REST && mine.second && b + 1 == mine.first + mine.count) __builtin_amdgcn_s_setprio(2);
     const unsigned char *packed = packed_of(b);
     const float *tail = reinterpret_cast<const float *>(packed + G::TAIL_OFF);
     __syncthreads();  // previous board fully written out; LDS is free
@@ -452,6 +455,11 @@ __global__ __launch_bounds__(256, 2) void duo_forward_kernel(const FwdParams prm
     }
   }
   if (detect && wave == 1 && lane == 0) prm.redo_counts[mine.run] = listed;
+}
+
+template <class P> __global__ __launch_bounds__(256, 2) void duo_forward_kernel(const FwdParams prm) {
+  extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
+  duo_boards<P>(prm, smem, gridDim.x);
 }
 
 }  // namespace c6

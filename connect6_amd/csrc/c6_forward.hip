@@ -2185,6 +2185,7 @@ template <class P> int launch_pack(const PackParams &pp, hipStream_t st);
 template <class P> int launch_forward(const FwdParams &fp, hipStream_t st);
 
 template <class P> int launch_team(const TeamParams &tp, int grid, hipStream_t st);
+template <class P> int launch_rest(const TeamParams &tp, int cus, hipStream_t st);
 template <class P> int launch_team_cascade(const TeamCascadeParams &tp, int grid, hipStream_t st);
 template <class P> int launch_second_pass(const TeamParams &tp, int grid, hipStream_t st);
 
@@ -2283,6 +2284,32 @@ template <class P> int launch_team(const TeamParams &tp, int grid, hipStream_t s
   return C6_OK;
 }
 
+// whole rounds and a rest of a mode that has duo_rest_kernel
+template <class P> int launch_rest(const TeamParams &tp, int cus, hipStream_t st) {
+  if constexpr (has_duo<P>()) {
+    constexpr int A = DuoGeo::LDS_BYTES, B = TeamGeo<P>::LDS_BYTES, LDS = A > B ? A : B;
+    static_assert(2 * LDS <= 160 * 1024, "two workgroups per CU");
+    static thread_local int configured = -1;
+    int dev = 0;
+    hipError_t e = hipGetDevice(&dev);
+    if (e == hipSuccess && configured != dev) {
+      e = hipFuncSetAttribute(reinterpret_cast<const void *>(&duo_rest_kernel<P>),
+                              hipFuncAttributeMaxDynamicSharedMemorySize, LDS);
+      if (e == hipSuccess) configured = dev;
+    }
+    if (e == hipSuccess) {
+      hipLaunchKernelGGL(duo_rest_kernel<P>, dim3(3 * (unsigned)cus), dim3(256), LDS, st, tp);
+      e = hipGetLastError();
+    }
+    if (e == hipSuccess) return C6_OK;
+    set_error("duo_rest launch failed: %s", hipGetErrorString(e));
+    return C6_ELAUNCH;
+  } else {
+    set_error("this mode has no workgroups that share a CU");
+    return C6_EINVAL;
+  }
+}
+
 template <class P> int launch_second_pass(const TeamParams &tp, int grid, hipStream_t st) {
   constexpr int A = Geo<P>::LDS_BYTES, B = TeamGeo<P>::LDS_BYTES, LDS = A > B ? A : B;
   static thread_local int configured = -1;
@@ -2334,6 +2361,7 @@ template int launch_team_cascade<C6_INSTANCE>(const TeamCascadeParams &, int, hi
 template int launch_second_pass<C6_INSTANCE>(const TeamParams &, int, hipStream_t);
 #elif defined(C6_TEAM)
 template int launch_team<C6_INSTANCE>(const TeamParams &, int, hipStream_t);
+template int launch_rest<C6_INSTANCE>(const TeamParams &, int, hipStream_t);
 #else
 template int launch_pack<C6_INSTANCE>(const PackParams &, hipStream_t);
 template int launch_forward<C6_INSTANCE>(const FwdParams &, hipStream_t);
@@ -2400,11 +2428,12 @@ struct TeamMode {
   int (*size)(long long boards, int wgs);      // workgroups per board
   long long (*most)(int wgs);                  // boards that are shared at all
   int (*launch)(const TeamParams &, int grid, hipStream_t);
-  bool rounds;                                 // many boards run in rounds of one workgroup per CU
+  int (*launch_rest)(const TeamParams &, int cus, hipStream_t);   // modes that put two workgroups on a CU
+  int (*rest)(long long boards, int cus);      // ... workgroups per board of a rest beside them
 };
 template <class P> static TeamMode team_mode_of() {
   return {TeamGeo<P>::BOARDB, &team_size<P>, &team_most<P>, &launch_team<P>,
-          !has_duo<P>()};
+          has_duo<P>() ? &launch_rest<P> : nullptr, &rest_team<P>};
 }
 static TeamMode team_mode(int prec) {
   switch (prec) {
@@ -2414,7 +2443,7 @@ static TeamMode team_mode(int prec) {
     case C6_PREC_BF16F6: return team_mode_of<PrecBF16F6>();
     case C6_PREC_BF16F6W: return team_mode_of<PrecBF16F6W>();
   }
-  return {0, nullptr, nullptr, nullptr, false};
+  return {0, nullptr, nullptr, nullptr, nullptr, nullptr};
 }
 static int second_mode(int cascade) { return cascade == C6_PREC_BF16C ? C6_PREC_BF16F6W : C6_PREC_BF16F6; }
 // The cascade's second pass hands what the listed boards leave beyond whole rounds of the CUs to teams, if it
@@ -2425,29 +2454,32 @@ static int second_mode(int cascade) { return cascade == C6_PREC_BF16C ? C6_PREC_
 
 // Boards of a batch that are shared between workgroups: all where they are few; behind whole rounds of one
 // workgroup per CU the rest (fp32: 257 boards 607 -> 373 us, 341 boards 607 -> 450 us, 384 boards 600 -> 531 us, 777 boards 1,190 ->
-// 975 us; bf16 + fp6 + low weights, 298 boards: 239 -> 191 us).  In the modes that put two workgroups on a CU a rest is
-// a board more for some CUs; behind an odd number of rounds, where that is a fourth board beside three, a sixth beside
-// five ..., it takes longer than teams do, unless so few CUs have it that their clock makes up for it.  One line for fp16,
-// bf16 and the cascade's first pass: more than half as many boards as rounds.  It leaves out a few sizes where teams would
-// gain 1 to 4 % (fp16, 768 + 1 boards 202 / 194, 1,280 + 1 307 / 303, 2,816 + 2 631 / 625) for those where they lose
-// (2,816 + 1 615 / 625, the cascade at 2,816 + 2 726 / 748); rounds end at eleven: 4,864 + 2 1,057 / 1,061, + 9 1,070 /
-// 1,061, + 40 1,072 / 1,074; even ones fill a CU's second place: 512 + 9 141 / 144, 1,024 + 9 249 / 252.  What the line takes in,
-// all as one / rest in teams, us (medians of two runs a side, which differ by 0.5 %, the cascade's above 2,304 boards by 1 %;
-// the cascade's first with the second pass as two launches, 3 us):
-//           fp16 + 9     + 40         bf16 + 9     + 40         cascade + 9   + 40
-//   768     208 / 195    209 / 206    198 / 185    199 / 195    276 / 264     291 / 290
-//   1,280   316 / 303    315 / 311    299 / 286    299 / 296    425 / 412     426 / 421
-//   1,792   423 / 409    423 / 419    402 / 388    402 / 398    528 / 517     530 / 527
-//   2,304   530 / 516    530 / 527    502 / 490    503 / 500    632 / 627     636 / 639
-//   2,816   638 / 627    639 / 639    604 / 594    605 / 605    736 / 730     738 / 741
+// 975 us; bf16 + fp6 + low weights, 298 boards: 239 -> 191 us).  In the modes that put two workgroups on a CU a rest of up
+// to five sixteenths of the CUs goes to teams that run beside the last boards of the others (duo_rest_kernel).  Without
+// that each is a board more for its CU, the last one alone there, 35 to 45 us; with teams in a launch behind the others 30 to 35.
+// Measured, us, without / with; the cascade's with its second pass:
+//     boards       fp16          bf16          cascade           boards       fp16          bf16          cascade
+//     256 + 1      93 / 72       90 / 67       148 / 125         1,024 + 9    257 / 231     243 / 220     339 / 311
+//         + 9      92 / 70       89 / 67       155 / 135             + 40     258 / 241     245 / 228     369 / 354
+//         + 40     93 / 77       90 / 73       158 / 145             + 80     260 / 254     247 / 240     370 / 367
+//         + 80     95 / 90       92 / 86       161 / 158         1,280 + 1    311 / 279     296 / 264     411 / 388
+//     512 + 9      143 / 122     137 / 115     228 / 207             + 40     324 / 302     306 / 287     433 / 412
+//         + 40     145 / 133     138 / 127     228 / 221             + 80     325 / 318     310 / 302     435 / 429
+//         + 80     146 / 150     139 / 144     230 / 236         1,536 + 9    368 / 340     350 / 324     472 / 448
+//     768 + 9      202 / 181     193 / 172     288 / 260             + 80     372 / 365     353 / 346     480 / 473
+//         + 40     212 / 190     202 / 180     297 / 272         4,096 + 9    923 / 900     872 / 852     1,011 / 986
+//         + 80     214 / 203     204 / 192     299 / 284         4,864 + 9    1,106 / 1,063 1,045 / 1,005 1,245 / 1,205
+// (256, 768, 1,280 + 9 "without" is a launch of teams behind the others from 768 on.)  So at two rounds teams of three are
+// not worth it, and neither are teams of two anywhere but at an odd few rounds (256 + 104 94 / 94 and 768 + 128 209 / 204, but 256
+// + 128 95 / 100 and 1,280 + 128 315 / 327).
 static long long team_boards(int prec, long long boards, int cus) {
   const TeamMode m = team_mode(prec);
   if (m.launch == nullptr) return 0;
   if (boards <= cus) return m.size(boards, cus) > 1 ? boards : 0;
   const long long rest = boards % cus;
-  const long long rounds = boards / cus;
-  const bool shares = m.rounds || (rounds % 2 == 1 && rounds > 1 && rounds < 12 && 2 * rest > rounds);
-  return shares && rest <= m.most(cus) ? rest : 0;
+  if (m.launch_rest == nullptr) return rest <= m.most(cus) ? rest : 0;
+  const int size = m.rest(rest, cus);
+  return size > 3 || (size > 1 && boards / cus != 2) ? rest : 0;
 }
 
 // Boards of a cascade whose two passes are one launch: those that twelve workgroups share (team_cascade_kernel)
@@ -2486,6 +2518,12 @@ int dispatch_team(int prec, const TeamParams &tp, hipStream_t st) {
   const TeamMode m = team_mode(prec);
   const long long all = tp.f.total_boards, shared = team_boards(prec, all, cus);
   TeamParams part = tp;
+  if (shared < all && m.launch_rest != nullptr) {
+    part.f.total_boards = all - shared;
+    part.rest = (unsigned)shared;
+    part.polls = tp.polls < (1 << 20) ? 4 * tp.polls : tp.polls;   // (a team's workgroups start as others end, within some microseconds)
+    return m.launch_rest(part, cus, st);
+  }
   if (shared < all) {
     part.f.total_boards = all - shared;
     const int rc2 = dispatch_forward(prec, part.f, st);
@@ -2508,7 +2546,8 @@ int dispatch_cascade(int prec, const FwdParams &fp, float threshold, void *works
   if (rc != C6_OK) return rc;
   // runs: the workgroups of the boards that have one each, then each board that teams share
   const long long shared = team != nullptr ? team_boards(C6_PREC_BF16, fp.total_boards, cus) : 0;
-  const long long single = fp.total_boards - shared, grid = forward_grid<PrecBF16>(single, cus), runs = grid + shared;
+  const long long single = fp.total_boards - shared;
+  const long long grid = shared > 0 && single > 0 ? 2 * (long long)cus : forward_grid<PrecBF16>(single, cus), runs = grid + shared;
   if (runs > kCascadeMaxRuns) {
     set_error("cascade: %lld workgroups exceed the %d the workspace layout provides for", runs, kCascadeMaxRuns);
     return C6_EINVAL;

@@ -63,7 +63,10 @@ template <class P> struct TeamGeo {
   static constexpr int BOARDB = (VAL_OFF + 12 * 9 * 64 * 4 + 255) & ~255;
   // LDS: up to 11 rows of positions (128 squares lie in at most 8 board rows), 13 for 192 squares (SPLIT; in 11)
   static constexpr int REGION = ((SPLIT ? 13 : 11) * kPitch + 1) * RECB;
-  static constexpr int BUF = REGION > G::COPIES_BYTES ? REGION : G::COPIES_BYTES;
+  // The first layer's shifted copies hold the halo rows that a workgroup's squares see: three per kernel row of up to
+  // twelve rows of squares, and the zero row (an odd number: a copy is then an odd number of 16-byte units long).
+  static constexpr int COPY_ROWS = 105, COPY_BYTES = COPY_ROWS * kL1RowPitch * G::EB, COPIES_BYTES = G::E * COPY_BYTES;
+  static constexpr int BUF = REGION > COPIES_BYTES ? REGION : COPIES_BYTES;
   static constexpr int OCC_OFF = (BUF + 15) & ~15;
   static constexpr int LGT_OFF = OCC_OFF + 384;
   static constexpr int RED_OFF = LGT_OFF + 1456;
@@ -729,7 +732,8 @@ __device__ __forceinline__ void team_board(const TeamParams &prm, unsigned char 
         }
       }
     }
-    // halo rows that the squares' 23 kernel rows reach (and the zero row behind the last)
+    // halo rows that the squares' 23 kernel rows reach (and the zero row behind the last): those from ha on are staged
+    static_assert(((PXT * 32 + kBoard - 2) / kBoard + kK1) * 3 + 1 <= T::COPY_ROWS, "rows of the copies");
     const int ha = sp.p0 / kBoard * 3, hb = (sp.p1 / kBoard + kK1) * 3 + 1;
     {
       const v4i z = {0, 0, 0, 0};
@@ -737,7 +741,7 @@ __device__ __forceinline__ void team_board(const TeamParams &prm, unsigned char 
 #pragma unroll
       for (int s = 0; s < G::E; ++s)
         for (int i = tid; i < per; i += THREADS)
-          *reinterpret_cast<v4i *>(smem + s * G::COPY_BYTES + ha * kL1RowPitch * G::EB + i * 16) = z;
+          *reinterpret_cast<v4i *>(smem + s * T::COPY_BYTES + i * 16) = z;
     }
 #pragma unroll
     for (int i = 0; i < TAIL_UNITS; ++i)
@@ -776,7 +780,7 @@ __device__ __forceinline__ void team_board(const TeamParams &prm, unsigned char 
     for (int n = 0; n < N1; ++n) {
       const int p = sp.p0 + (px + n) * 32 + (lane & 31);
       const int pc = p < kPix ? p : kPix - 1, r = pc / kBoard, c = pc - r * kBoard, sh = c % G::E;
-      row0[n] = sh * G::COPY_BYTES + (r * 3 * kL1RowPitch + (c - sh)) * G::EB + (plane2_varies ? kL1RowsHalf : 1) * h * kL1RowPitch * G::EB;
+      row0[n] = sh * T::COPY_BYTES + ((r * 3 - ha) * kL1RowPitch + (c - sh)) * G::EB + (plane2_varies ? kL1RowsHalf : 1) * h * kL1RowPitch * G::EB;
     }
     const int rowb = (plane2_varies ? 1 : 3) * kL1RowPitch * G::EB;
     const WFrags wl = plane2_varies ? layer_weights<P, 0>(packed, lane) : packed_frags<P>(packed, lane, G::FAST1_OFF);
@@ -820,7 +824,7 @@ __device__ __forceinline__ void team_board(const TeamParams &prm, unsigned char 
           if (hrow < ha || hrow >= hb) continue;
 #pragma unroll
           for (int q = 0; q < G::E; ++q)
-            *reinterpret_cast<unsigned short *>(smem + q * G::COPY_BYTES + (hrow * kL1RowPitch + (col + kK1 / 2 - q)) * G::EB) = v16;
+            *reinterpret_cast<unsigned short *>(smem + q * T::COPY_BYTES + ((hrow - ha) * kL1RowPitch + (col + kK1 / 2 - q)) * G::EB) = v16;
         }
       }
       __syncthreads();
@@ -1074,14 +1078,15 @@ struct TeamPlace {
   unsigned slot;
   int role;
 };
-__device__ __forceinline__ TeamPlace team_place(unsigned items, int team) {
-  if (gridDim.x % 8 == 0) {
-    const unsigned per = (items + 7) / 8, l = blockIdx.x / 8;
-    if (per * (unsigned)team <= gridDim.x / 8)
-      return {l / (unsigned)team < per ? blockIdx.x % 8 * per + l / (unsigned)team : items, (int)(l % (unsigned)team)};
+__device__ __forceinline__ TeamPlace team_place(unsigned items, int team, unsigned wg, unsigned wgs) {   // (wg of wgs)
+  if (wgs % 8 == 0) {
+    const unsigned per = (items + 7) / 8, l = wg / 8;
+    if (per * (unsigned)team <= wgs / 8)
+      return {l / (unsigned)team < per ? wg % 8 * per + l / (unsigned)team : items, (int)(l % (unsigned)team)};
   }
-  return {blockIdx.x / (unsigned)team, (int)(blockIdx.x % (unsigned)team)};
+  return {wg / (unsigned)team, (int)(wg % (unsigned)team)};
 }
+__device__ __forceinline__ TeamPlace team_place(unsigned items, int team) { return team_place(items, team, blockIdx.x, gridDim.x); }
 
 // A workgroup's share of board b, in a team of any size that the mode has.
 template <class P>
@@ -1103,6 +1108,41 @@ template <class P> __global__ __launch_bounds__(256) void team_forward_kernel(co
   if (team == 1) return;
   const TeamPlace at = team_place(items, team);
   if (at.slot < items) team_share<P>(prm, smem, prm.first + at.slot, at, team);
+}
+
+// The plain 16-bit modes with a few boards beyond whole rounds of one board per CU: teams for them in one launch with the
+// two workgroups per CU that serve the others (c6_duo.h).  They start where the first of those end, so the second of the two
+// on each CU goes first with its last board (s_setprio): its place is free some 25 us before the other, which had as
+// little of the matrix cores as that takes, ends, with an odd number of rounds a board before it; the team's waves, a chain that
+// leaves the matrix cores idle most of the time, go in front of the other's.  What it gives stands at team_boards: 777 boards
+// in fp16 202 -> 181 us (teams in front without the second workgroup's priority 189; without either, 188 and 71 -> 74 at
+// 257 boards).  What bounds it: 512 + 9 boards take 15 us more than 512, of which the other workgroups, alone on their CUs
+// in the end, are most.
+// Registers: the teams' contractions want more than the 256 that two workgroups per CU leave; what is in scratch (under 128
+// bytes a lane) is theirs.
+// The workgroups per board of a rest (1: none are shared), as many as half of the places hold, and a team on one XCD.
+template <class P> __host__ __device__ inline int rest_team(long long boards, int cus) {
+  if (!has_duo<P>()) return 1;
+  if (boards * 12 <= cus) return 12;
+  if (boards <= cus * 5 / 32) return 6;
+  return boards <= cus * 5 / 16 ? 3 : 1;
+}
+template <class P> __global__ __launch_bounds__(256, 2) void duo_rest_kernel(const TeamParams prm) {
+  extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
+  const unsigned cus = gridDim.x / 3, grid = 2 * cus;
+  if (blockIdx.x < grid) {
+    duo_boards<P, true>(prm.f, smem, grid);
+    return;
+  }
+  const unsigned wg = blockIdx.x - grid;
+  const int team = rest_team<P>(prm.rest, (int)cus);
+  const TeamPlace at = team_place(prm.rest, team, wg, cus);
+  if (at.slot >= prm.rest) return;
+  const unsigned b = (unsigned)prm.f.total_boards + at.slot;
+  __builtin_amdgcn_s_setprio(3);
+  if (team == 12) team_board<P, 12>(prm, smem, b, at.slot, at.role);
+  if (team == 6) team_board<P, 6>(prm, smem, b, at.slot, at.role);
+  if (team == 3) team_board<P, 3>(prm, smem, b, at.slot, at.role);
 }
 
 // The cascade over so few boards that twelve workgroups share each: both passes in one launch.  Where a board's last

@@ -193,7 +193,7 @@ int c6_forward_boards_cascade(const int8_t *boards, const int8_t *player,
  * better launch (or the mode has no such kernel): call c6_forward there.
  *   workspace  device, 16-byte aligned; contents need no preparation.  Per shared board 1.0 MB
  *              (C6_PREC_F32S), 0.5 MB (C6_PREC_BF16F6, _BF16F6W and the cascades), 0.35 MB (C6_PREC_BF16,
- *              _F16); of 256 CUs at most 128, 42 or 73, and 40 boards are shared.  A cascade over at most 21
+ *              _F16); of 256 CUs at most 128, 42 or 73, and 80 boards are shared.  A cascade over at most 21
  *              boards is one launch and takes both its passes' share
  *   (the cascade's workspace, where there is one, comes in front of these)
  *   flags      device words through which the workgroups of this launch tell one another what is
@@ -203,7 +203,8 @@ int c6_forward_boards_cascade(const int8_t *boards, const int8_t *player,
  *   tag        not 0; a cascade also uses tag + 1.  Which XCD a workgroup is on is told with a tag's low 28
  *              bits, so those are not used twice either between two clearings of the words: after 2^27 calls
  *              that count two each, clear them and begin at 1 again
- *   polls      how often a workgroup looks at a flag before it computes the piece itself; 0: 64
+ *   polls      how often a workgroup looks at a flag before it computes the piece itself; 0: 64 (four times as often
+ *              where the teams start beside other workgroups: C6_PREC_BF16, _F16 and the cascades, more boards than CUs)
  * No synchronisation with the host.  Every wait is bounded: a workgroup that has
  * waited too long computes what it waits for. */
 int c6_team_bytes(int prec, int64_t boards, size_t *workspace_bytes, size_t *flag_bytes);

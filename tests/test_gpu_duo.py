@@ -1,6 +1,8 @@
 """Two workgroups per CU (more boards than CUs, plain 16-bit modes) against one workgroup per board:
 the same bits at batch sizes around whole rounds, for every input form, mask and output type, and
 the cascade's lists."""
+import ctypes
+
 import pytest
 import torch
 
@@ -87,7 +89,43 @@ def test_weight_sets_and_board_state(cuda, prec):
             _same(part(slice(0, 613)), _pieces(part, 613))
 
 
-@pytest.mark.parametrize("boards", [257, 513, 1400, 4096])
+@pytest.mark.parametrize("rounds", [1, 2, 3, 4])
+@pytest.mark.parametrize("prec", [_lib.PREC_BF16, _lib.PREC_F16])
+def test_rest_in_teams_beside_whole_rounds(cuda, prec, rounds):
+    """A few boards beyond whole rounds go to teams in the same launch: sizes on either side of a change of the
+    team's size and of the most that are shared, also when no workgroup waits for another for long."""
+    cus = torch.cuda.get_device_properties(cuda).multi_processor_count
+    most = rounds * cus + cus * 5 // 16 + 1
+    model, (x, legal) = _model(cuda), _inputs(most)
+    x, legal, u = x.to(cuda), legal.to(cuda), gen_uniform(most, 5).to(cuda)
+    packed = model.packed_weights(prec)
+
+    def call(s):
+        return run_forward(x[s], packed, prec, 1, x[s].shape[0], mask_mode=_lib.MASK_LEGAL, legal=legal[s], u=u[s],
+                           temperature=0.8, want_logprob=True)
+
+    with torch.inference_mode():
+        want = _pieces(call, most)
+        for rest in (1, 2, cus // 12, cus // 12 + 1, cus * 5 // 32, cus * 5 // 32 + 1, cus * 5 // 16, cus * 5 // 16 + 1):
+            n = rounds * cus + rest
+            _same(call(slice(0, n)), [w[:n] for w in want])
+        # through the C ABI, each workgroup looking at a flag four times only
+        lib, n = c6.load(), rounds * cus + cus * 5 // 32
+        ws, fl = ctypes.c_size_t(), ctypes.c_size_t()
+        assert lib.c6_team_bytes(prec, n, ctypes.byref(ws), ctypes.byref(fl)) == 0 and ws.value > 0
+        work = torch.full((ws.value,), 255, dtype=torch.uint8, device=cuda)
+        flags = torch.zeros(fl.value // 4, dtype=torch.int32, device=cuda)
+        raw = run_forward(x, packed, prec, 1, most)
+        for tag in (1, 2):
+            logits, value = torch.empty(n, 361, device=cuda), torch.empty(n, device=cuda)
+            rc = lib.c6_forward_team(x.data_ptr(), 0, 1, n, packed.data_ptr(), packed.numel(), prec, logits.data_ptr(),
+                                     value.data_ptr(), 0, None, 0.0, None, 1.0, None, None, work.data_ptr(), ws.value,
+                                     flags.data_ptr(), flags.numel() * 4, tag, 1, _lib.stream_ptr(x.device))
+            _lib.check(rc, "c6_forward_team")
+            _same((logits, value), (raw[0][:n], raw[1][:n]))
+
+
+@pytest.mark.parametrize("boards", [257, 336, 513, 1400, 1576, 4096])
 def test_cascade_lists_the_same_boards(cuda, boards):
     model = c6.PolicyValueNet().to(cuda).eval()
     model.load_state_dict(R.init_state(5, "reference"))

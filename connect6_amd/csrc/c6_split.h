@@ -23,13 +23,15 @@
 // they are: 0.7e-9; medians over 256 networks with PyTorch's initialisation).
 //
 // What bounds it: the matrix cores, 383 k cycles per board with the 1,890 MFMAs of the 3x3 layers
-// six times and the first layer's 207 three times (0/1 inputs are exact in one bf16 value), of 548 k that a
-// board takes; then the epilogues, 98 cycles per output of a lane (one wave per SIMD issues an instruction
-// per 5 cycles or so), and in the layers of 96 outputs the second reading of the weights (split_conv).  The
-// activations of up to 64 channels lie in LDS as their three planes, split once when a layer writes
+// six times and the first layer's 207 three times (0/1 inputs are exact in one bf16 value); then the epilogues,
+// some 25 instructions per output of a lane (two of them at a quarter of the rate) that one wave per SIMD issues in
+// the open.  They go step by step over eight outputs, because a lone wave waits wherever an instruction needs the
+// one before it.  The activations of up to 64 channels lie in LDS as their three planes, split once when a layer writes
 // them; 96 channels only fit as fp32 (421 positions x 384 bytes are the CU's whole LDS), and the two
 // layers that read them split them in registers, 44 instructions for eight values, a few behind each
-// MFMA.  2,048 boards take 2.33 ms (4.35 with fp32 instructions; 2.11 with one sum).
+// MFMA.  2,048 boards take 2.29 ms (2.42 on the same box while the layers of 96 outputs ran in two passes over
+// the pixel tiles and read their weights twice, and epilogues output by output; 4.35 with
+// fp32 instructions).
 //
 // An infinity is its own first part; what is left of it is a NaN in the sum of the small products, and the
 // large ones alone, which are then infinite or NaN as in fp32 arithmetic, are the result (two_sums; 0.4 % of
@@ -94,6 +96,16 @@ __device__ __forceinline__ int split_take(float &a, float &b) {
   split_drop(a, b, w);
   return w;
 }
+// split_drop of four pairs, step by step
+__device__ __forceinline__ void split_drop4(float (&v)[8], const int (&w)[4]) {
+#pragma clang fp contract(off)
+  float r[8];
+#pragma unroll
+  for (int e = 0; e < 8; ++e) r[e] = __builtin_bit_cast(float, e % 2 ? w[e / 2] & (int)0xffff0000 : w[e / 2] << 16);
+  __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+  for (int e = 0; e < 8; ++e) v[e] -= r[e];
+}
 
 // Weight ring of a 3x3 layer: two k-steps of all cout tiles and planes.  A k-step of NT cout tiles and N
 // pixel tiles is 6 NT N MFMAs, 192 NT N cycles, and a slot is refilled behind its last use.
@@ -109,16 +121,28 @@ template <int NT> __device__ __forceinline__ void split_preload(v4i (&ring)[kSpl
       for (int i = 0; i < 3; ++i) ring[d][t][i] = wl[(d * NT + t) * 3 + i];
 }
 
-// The contraction of 3x3 layer L for N pixel tiles from J0 on.  K runs over taps, then 16 channels at a
-// time; each k-step is 6 N MFMAs per cout tile: six products of each pixel tile.  The five small ones have
+// A product whose sum is in vector registers: the compiler puts every sum of the instruction in accumulation
+// registers, and there are 256 of those.  (s_nop: an operand may just have been written by the vector unit.)
+__device__ __forceinline__ void mma_vector(const v4i &a, const v4i &b, f32x16 &c) {
+  asm volatile("s_nop 1\n\tv_mfma_f32_32x32x16_bf16 %0, %1, %2, %0" : "+v"(c) : "v"(a), "v"(b));
+}
+// ... and the wait in front of the first other use of such a sum (the instruction's sixteen passes and what the
+// compiler leaves behind them for the sums that it knows of)
+__device__ __forceinline__ void mma_vector_wait(f32x16 &a, f32x16 &b) {
+  asm volatile("s_nop 15\n\ts_nop 7" : "+v"(a), "+v"(b));
+}
+
+// The contraction of 3x3 layer L.  K runs over taps, then 16 channels at a
+// time; each k-step is 18 MFMAs per cout tile: six products of each pixel tile.  The five small ones have
 // a sum of their own, low, and the large one adds to acc.  Behind each MFMA at most one LDS read of the
 // next k-step's activations, one weight load, and (96 input channels) a few instructions of their split.
-//   ring: the first k-steps on entry; at the end the first ones again (AGAIN) or those behind the layer's last
-template <int L, int J0, int N, bool AGAIN>
-__device__ __forceinline__ void split_conv_tiles(const unsigned char *smem, const WFrags &wl, const float *bias,
-                                                 SplitWeights<L> &ring, const int (&ci)[3], int h,
-                                                 f32x16 (&acc)[kCoutArr[L] / 32][3], f32x16 (&low)[kCoutArr[L] / 32][N]) {
-  constexpr int CIN = kCinArr[L], NT = kCoutArr[L] / 32, KC = CIN / 16, D = kSplitRing<NT>;
+//   ring: the first k-steps on entry, those behind the layer's last at the end
+// The sums of three cout tiles are 288 registers: those of the last pixel tile's last cout tile are vector registers.
+template <int L>
+__device__ __forceinline__ void split_conv(const unsigned char *smem, const WFrags &wl, const float *bias,
+                                           SplitWeights<L> &ring, const int (&ci)[3], int h,
+                                           f32x16 (&acc)[kCoutArr[L] / 32][3], f32x16 (&low)[kCoutArr[L] / 32][3]) {
+  constexpr int CIN = kCinArr[L], NT = kCoutArr[L] / 32, KC = CIN / 16, D = kSplitRing<NT>, N = 3;
   constexpr bool WIDE = CIN == 96;   // activations arrive as fp32
   static_assert(KC % 2 == 0 && KC % D == 0, "double buffers must line up across taps");
   int pb[N], xo[N];
@@ -126,7 +150,7 @@ __device__ __forceinline__ void split_conv_tiles(const unsigned char *smem, cons
     const int ky = tap / 3, kx = tap - 3 * ky;
 #pragma unroll
     for (int j = 0; j < N; ++j) {
-      const int pos = ci[J0 + j] + (ky - 1) * kPitch + (kx - 1);
+      const int pos = ci[j] + (ky - 1) * kPitch + (kx - 1);
       pb[j] = pos * SplitGeo::PIXB;
       xo[j] = (WIDE ? h << 5 : h << 4) ^ split_swz(pos);
     }
@@ -177,7 +201,7 @@ __device__ __forceinline__ void split_conv_tiles(const unsigned char *smem, cons
     load_bias_tiles(bl, bias + Geo<PrecF32S>::TAIL_BIAS_LOW + 32 * t, h);
 #pragma unroll
     for (int j = 0; j < N; ++j) {
-      acc[t][J0 + j] = b[0];
+      acc[t][j] = b[0];
       low[t][j] = bl[0];
     }
   }
@@ -185,7 +209,6 @@ __device__ __forceinline__ void split_conv_tiles(const unsigned char *smem, cons
 #pragma unroll 1
   for (int tap = 0; tap < 9; ++tap) {
     const WFrags wn = wl + (tap * KC + D) * NT * 3;
-    const WFrags wrap = wl + (AGAIN && tap == 8 ? (D - KC) * NT * 3 : (tap * KC + D) * NT * 3);
     static_for<0, KC>([&](auto uc) __attribute__((always_inline)) {
       constexpr int u = decltype(uc)::value, par = u & 1;
       // (after the last tap this wraps to the first: harmless extra reads)
@@ -193,7 +216,9 @@ __device__ __forceinline__ void split_conv_tiles(const unsigned char *smem, cons
       static_for<0, NT * 6 * N>([&](auto gc) __attribute__((always_inline)) {
         constexpr int g = decltype(gc)::value, t = g / (6 * N), m = (g % (6 * N)) / N, j = g % N;
         constexpr int WP[6] = {0, 1, 2, 0, 1, 0}, AP[6] = {2, 1, 0, 1, 0, 0};
-        mma<PrecBF16>(ring[u % D][t][WP[m]], bq[par][j][AP[m]], m < 5 ? low[t][j] : acc[t][J0 + j]);
+        f32x16 &sum = m < 5 ? low[t][j] : acc[t][j];
+        if constexpr (t == 2 && j == 2) mma_vector(ring[u % D][t][WP[m]], bq[par][j][AP[m]], sum);
+        else mma<PrecBF16>(ring[u % D][t][WP[m]], bq[par][j][AP[m]], sum);
         if constexpr (WIDE) {
           // raw[par] was split during the k-step before: free for the k-step after next
           if constexpr (g >= 1 && g < 1 + 2 * N) read((u + 2) % KC, par, (g - 1) / 2, (g - 1) % 2);
@@ -204,73 +229,108 @@ __device__ __forceinline__ void split_conv_tiles(const unsigned char *smem, cons
         // a plane's fragment after its last use in the tile: 2 after product 2, 1 after 4, 0 after 5
         constexpr int done = j == N - 1 ? (m == 2 ? 2 : (m == 4 ? 1 : (m == 5 ? 0 : -1))) : -1;
         if constexpr (done >= 0) {
-          if constexpr (u + D >= KC) ring[u % D][t][done] = wrap[(u * NT + t) * 3 + done];
-          else ring[u % D][t][done] = wn[(u * NT + t) * 3 + done];
+          ring[u % D][t][done] = wn[(u * NT + t) * 3 + done];
         }
         __builtin_amdgcn_sched_barrier(0);
       });
     });
   }
-}
-// All pixel tiles.  With three cout tiles the third pixel tile goes first and the other two after it: the
-// sums of all three, 288 registers, are more than the 256 the instruction's accumulators live in (2,048 boards
-// 2.33 ms; cout tiles apart, where 96 input channels are split twice, 2.53; two sums per k-step, added up by
-// the vector unit, 3.23).  The first two are left in two sums each.
-template <int NT> using SplitLow = f32x16[NT][NT < 3 ? 3 : 2];
-template <int L>
-__device__ __forceinline__ void split_conv(const unsigned char *smem, const WFrags &wl, const float *bias,
-                                           SplitWeights<L> &ring, const int (&ci)[3], int h,
-                                           f32x16 (&acc)[kCoutArr[L] / 32][3], SplitLow<kCoutArr[L] / 32> &low) {
-  if constexpr (kCoutArr[L] == 96) {
-    f32x16 one[3][1];
-    split_conv_tiles<L, 2, 1, true>(smem, wl, bias, ring, ci, h, acc, one);
+  if constexpr (NT == 3) {
+    mma_vector_wait(acc[2][2], low[2][2]);
 #pragma unroll
-    for (int t = 0; t < 3; ++t) {
-#pragma unroll
-      for (int e = 0; e < 16; ++e) acc[t][2][e] = two_sums(acc[t][2][e], one[t][0][e]);
-      asm volatile("" : "+v"(acc[t][2]));   // (kept out of the accumulators' registers, which the others fill)
-      __builtin_amdgcn_sched_barrier(0);
-    }
-    split_conv_tiles<L, 0, 2, false>(smem, wl, bias, ring, ci, h, acc, low);
-#pragma unroll
-    for (int t = 0; t < 3; ++t) asm volatile("" : "+v"(acc[t][2]));
-  } else {
-    split_conv_tiles<L, 0, 3, false>(smem, wl, bias, ring, ci, h, acc, low);
+    for (int k = 0; k < 8; ++k) asm volatile("" : "+a"(acc[k / 3][k % 3]), "+a"(low[k / 3][k % 3]));
   }
 }
+// The sums of one tile, taken out of the accumulation registers here and not with all the others at once
 template <int NT>
-__device__ __forceinline__ float split_total(const f32x16 (&acc)[NT][3], const SplitLow<NT> &low, int t, int j, int e) {
-  return NT < 3 || j < 2 ? two_sums(acc[t][j][e], low[t][j][e]) : acc[t][j][e];
+__device__ __forceinline__ f32x16 split_total(const f32x16 (&acc)[NT][3], const f32x16 (&low)[NT][3], int t, int j) {
+  f32x16 large = acc[t][j], small = low[t][j], sum;
+  __builtin_amdgcn_sched_barrier(0);
+  if (t == 2 && j == 2) asm volatile("" : "+v"(large), "+v"(small));
+  else asm volatile("" : "+a"(large), "+a"(small));
+#pragma unroll
+  for (int e = 0; e < 16; ++e) sum[e] = large[e] + small[e];
+  __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+  for (int e = 0; e < 16; e += 8) {
+    bool number[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) number[i] = sum[e + i] == sum[e + i];
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int i = 0; i < 8; ++i) sum[e + i] = number[i] ? sum[e + i] : large[e + i];
+    __builtin_amdgcn_sched_barrier(0);
+  }
+  return sum;
+}
+// SiLU of eight sums from e0 on, step by step: a lone wave waits for each result that its next instruction needs
+__device__ __forceinline__ void split_silu8(const f32x16 &sum, int e0, float (&v)[8]) {
+#pragma clang fp contract(off)
+  float d[8], r[8], q[8];
+#pragma unroll
+  for (int e = 0; e < 8; ++e) d[e] = __builtin_amdgcn_exp2f(sum[e0 + e]);
+  __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+  for (int e = 0; e < 8; ++e) d[e] = 1.0f + d[e];
+  __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+  for (int e = 0; e < 8; ++e) r[e] = __builtin_amdgcn_rcpf(d[e]);
+  __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+  for (int e = 0; e < 8; ++e) q[e] = sum[e0 + e] * r[e];
+  __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+  for (int e = 0; e < 8; ++e) d[e] = fmaf(-d[e], q[e], sum[e0 + e]);
+  __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+  for (int e = 0; e < 8; ++e) d[e] = fminf(d[e], 0x1p100f);
+  __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+  for (int e = 0; e < 8; ++e) v[e] = fmaf(d[e], r[e], q[e]);
+  __builtin_amdgcn_sched_barrier(0);
 }
 
 // SiLU and store of one layer's outputs in the form the next one reads.
 template <int NT, bool PLANES>
 __device__ __forceinline__ void split_store(unsigned char *smem, const int (&ci)[3], int h, const f32x16 (&acc)[NT][3],
-                                            const SplitLow<NT> &low) {
+                                            const f32x16 (&low)[NT][3]) {
 #pragma unroll
   for (int j = 0; j < 3; ++j) {
     int pos = ci[j];
     asm volatile("" : "+v"(pos));  // (addresses formed here, not kept for the whole kernel)
     const int at = pos * SplitGeo::PIXB, sw = split_swz(pos);
 #pragma unroll
-    for (int t = 0; t < NT; ++t)
+    for (int t = 0; t < NT; ++t) {
+      const f32x16 sum = split_total<NT>(acc, low, t, j);
 #pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        float v[4];
-#pragma unroll
-        for (int e = 0; e < 4; ++e) v[e] = split_silu(split_total<NT>(acc, low, t, j, 4 * q + e));
+      for (int q = 0; q < 4; q += 2) {
+        float v[8];
+        split_silu8(sum, 4 * q, v);
         if constexpr (PLANES) {
-          unsigned char *p = smem + at + ((64 * t + 16 * q) ^ sw) + 8 * h;
+          int w[3][4];
 #pragma unroll
           for (int i = 0; i < 3; ++i) {
-            const int a = i < 2 ? split_take(v[0], v[1]) : pack2<PrecBF16>(v[0], v[1]);
-            const int b = i < 2 ? split_take(v[2], v[3]) : pack2<PrecBF16>(v[2], v[3]);
-            *reinterpret_cast<v2i *>(p + i * SplitGeo::PLANEB) = v2i{a, b};
+#pragma unroll
+            for (int e = 0; e < 4; ++e) w[i][e] = pack2<PrecBF16>(v[2 * e], v[2 * e + 1]);
+            __builtin_amdgcn_sched_barrier(0);
+            if (i < 2) {
+              split_drop4(v, w[i]);
+              __builtin_amdgcn_sched_barrier(0);
+            }
+          }
+#pragma unroll
+          for (int e = 0; e < 2; ++e) {
+            unsigned char *p = smem + at + ((64 * t + 16 * (q + e)) ^ sw) + 8 * h;
+#pragma unroll
+            for (int i = 0; i < 3; ++i) *reinterpret_cast<v2i *>(p + i * SplitGeo::PLANEB) = v2i{w[i][2 * e], w[i][2 * e + 1]};
           }
         } else {
-          *reinterpret_cast<f32x4 *>(smem + at + 128 * t + ((32 * q + 16 * h) ^ sw)) = f32x4{v[0], v[1], v[2], v[3]};
+#pragma unroll
+          for (int e = 0; e < 2; ++e)
+            *reinterpret_cast<f32x4 *>(smem + at + 128 * t + ((32 * (q + e) + 16 * h) ^ sw)) = f32x4{v[4 * e], v[4 * e + 1], v[4 * e + 2], v[4 * e + 3]};
         }
       }
+    }
   }
 }
 
@@ -280,8 +340,7 @@ __device__ __forceinline__ void split_layer(unsigned char *smem, const unsigned 
                                             SplitWeights<L> &ring, SplitWeights<L + 1> &next, const int (&ci)[3], int h,
                                             int lane) {
   constexpr int NT = kCoutArr[L] / 32;
-  f32x16 acc[NT][3];
-  SplitLow<NT> low;
+  f32x16 acc[NT][3], low[NT][3];
   split_conv<L>(smem, layer_weights<PrecF32S, L>(packed, lane), tail + bias_offset(L), ring, ci, h, acc, low);
   // (with equal widths the over-read has left the next layer's first k-steps in the ring)
   if constexpr (kCoutArr[L + 1] != kCoutArr[L]) split_preload(next, layer_weights<PrecF32S, L + 1>(packed, lane));
@@ -552,8 +611,7 @@ __global__ __launch_bounds__(256) void split_forward_kernel(const FwdParams prm)
 
     // ---- layer 8 + both 1x1 heads straight from the fp32 accumulators ----
     {
-      f32x16 acc[3][3];
-      SplitLow<3> low8;
+      f32x16 acc[3][3], low8[3][3];
       split_conv<7>(smem, layer_weights<P, 7>(packed, lane), tail + bias_offset(7), r678, ci, h, acc, low8);
       const float *valw = tail + kBiasTotal + kHeadC;
       const float *pwl = tail + kBiasTotal + 4 * h;  // per-lane base: channel 32t + 8q + 4h + e
@@ -571,18 +629,25 @@ __global__ __launch_bounds__(256) void split_forward_kernel(const FwdParams prm)
 #pragma unroll
       for (int t = 0; t < 3; ++t) {
         float pol[3] = {0.0f, 0.0f, 0.0f}, val[3] = {0.0f, 0.0f, 0.0f};
+        f32x4 pw[4], vw[4];
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
-          const f32x4 pw = *(GlobalF32x4)(pwg + 32 * t + 8 * q);
-          const f32x4 vw = *(GlobalF32x4)(pwg + kHeadC + 32 * t + 8 * q);
+          pw[q] = *(GlobalF32x4)(pwg + 32 * t + 8 * q);
+          vw[q] = *(GlobalF32x4)(pwg + kHeadC + 32 * t + 8 * q);
+        }
 #pragma unroll
-          for (int j = 0; j < 3; ++j)
+        for (int j = 0; j < 3; ++j) {
+          const f32x16 sum = split_total<3>(acc, low8, t, j);
 #pragma unroll
-            for (int e = 0; e < 4; ++e) {
-              const float a = split_silu(split_total<3>(acc, low8, t, j, 4 * q + e));
-              pol[j] = fmaf(a, pw[e], pol[j]);
-              val[j] = fmaf(a, vw[e], val[j]);
+          for (int q = 0; q < 4; q += 2) {
+            float v[8];
+            split_silu8(sum, 4 * q, v);
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+              pol[j] = fmaf(v[e], pw[q + e / 4][e % 4], pol[j]);
+              val[j] = fmaf(v[e], vw[q + e / 4][e % 4], val[j]);
             }
+          }
         }
 #pragma unroll
         for (int j = 0; j < 3; ++j) {

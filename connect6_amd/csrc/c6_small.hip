@@ -253,7 +253,7 @@ __device__ __forceinline__ float small_silu(float u) {
   return u * (t < 126.0f ? fmaf(r, fmaf(-d, r, 1.0f), r) : 0.0f);
 }
 // u / (1 + 2^(2 u)), of activations that carry the factor: the quotient by the approximate reciprocal, then by what it
-// leaves (0.48 ulp rms; see split_silu in c6_split.h)
+// leaves (0.48 ulp rms; see split_silu8 in c6_split.h)
 __device__ __forceinline__ float small_silu2(float u) {
 #pragma clang fp contract(off)
   const float d = 1.0f + __builtin_amdgcn_exp2f(u + u);

@@ -64,17 +64,6 @@ struct SplitGeo {
 // 16-byte granule XOR of a position: sixteen consecutive positions read sixteen bank groups
 __device__ __forceinline__ int split_swz(int pos) { return ((pos >> 1) & 7) << 4; }
 
-// u / (1 + 2^u): the quotient by the approximate reciprocal, then by what it leaves (0.48 ulp rms; by a refined
-// reciprocal 0.58).  Where the denominator is infinite, or u is, what it leaves is a NaN, which min() drops: 0 and
-// u itself are the results.
-__device__ __forceinline__ float split_silu(float u) {
-#pragma clang fp contract(off)   // (the product is rounded before its parts are taken)
-  const float d = 1.0f + __builtin_amdgcn_exp2f(u);
-  const float r = __builtin_amdgcn_rcpf(d);
-  const float q = u * r;
-  return fmaf(fminf(fmaf(-d, q, u), 0x1p100f), r, q);
-}
-
 // The heads: sums over the channels, which carry -log2(e), and over all squares.  (In 64 bits, once per square
 // and once per board: one rounding each.)
 __device__ __forceinline__ float split_logit(float sum, float bias) {
@@ -89,12 +78,6 @@ __device__ __forceinline__ void split_drop(float &a, float &b, int w) {
 #pragma clang fp contract(off)
   a -= __builtin_bit_cast(float, w << 16);
   b -= __builtin_bit_cast(float, w & (int)0xffff0000);
-}
-// The next bf16 plane of a pair of values, which keep what it leaves out.
-__device__ __forceinline__ int split_take(float &a, float &b) {
-  const int w = pack2<PrecBF16>(a, b);
-  split_drop(a, b, w);
-  return w;
 }
 // split_drop of four pairs, step by step
 __device__ __forceinline__ void split_drop4(float (&v)[8], const int (&w)[4]) {
@@ -263,7 +246,10 @@ __device__ __forceinline__ f32x16 split_total(const f32x16 (&acc)[NT][3], const 
   }
   return sum;
 }
-// SiLU of eight sums from e0 on, step by step: a lone wave waits for each result that its next instruction needs
+// SiLU of eight sums from e0 on, step by step (a lone wave waits for each result that its next instruction needs):
+// u / (1 + 2^u): the quotient by the approximate reciprocal, then by what it leaves (0.48 ulp rms; by a refined
+// reciprocal 0.58).  Where the denominator is infinite, or u is, what it leaves is a NaN, which min() drops: 0 and
+// u itself are the results.
 __device__ __forceinline__ void split_silu8(const f32x16 &sum, int e0, float (&v)[8]) {
 #pragma clang fp contract(off)
   float d[8], r[8], q[8];
@@ -290,6 +276,20 @@ __device__ __forceinline__ void split_silu8(const f32x16 &sum, int e0, float (&v
   __builtin_amdgcn_sched_barrier(0);
 }
 
+// The three planes of eight values, step by step
+__device__ __forceinline__ void split_planes8(float (&v)[8], int (&w)[3][4]) {
+#pragma unroll
+  for (int i = 0; i < 3; ++i) {
+#pragma unroll
+    for (int e = 0; e < 4; ++e) w[i][e] = pack2<PrecBF16>(v[2 * e], v[2 * e + 1]);
+    __builtin_amdgcn_sched_barrier(0);
+    if (i < 2) {
+      split_drop4(v, w[i]);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  }
+}
+
 // SiLU and store of one layer's outputs in the form the next one reads.
 template <int NT, bool PLANES>
 __device__ __forceinline__ void split_store(unsigned char *smem, const int (&ci)[3], int h, const f32x16 (&acc)[NT][3],
@@ -308,16 +308,7 @@ __device__ __forceinline__ void split_store(unsigned char *smem, const int (&ci)
         split_silu8(sum, 4 * q, v);
         if constexpr (PLANES) {
           int w[3][4];
-#pragma unroll
-          for (int i = 0; i < 3; ++i) {
-#pragma unroll
-            for (int e = 0; e < 4; ++e) w[i][e] = pack2<PrecBF16>(v[2 * e], v[2 * e + 1]);
-            __builtin_amdgcn_sched_barrier(0);
-            if (i < 2) {
-              split_drop4(v, w[i]);
-              __builtin_amdgcn_sched_barrier(0);
-            }
-          }
+          split_planes8(v, w);
 #pragma unroll
           for (int e = 0; e < 2; ++e) {
             unsigned char *p = smem + at + ((64 * t + 16 * (q + e)) ^ sw) + 8 * h;

@@ -252,6 +252,33 @@ __device__ __forceinline__ void team_conv(const unsigned char *smem, const unsig
   }
 }
 
+// SiLU of one accumulator tile, step by step: a lone wave waits for each result that its next instruction needs.
+template <class P> __device__ __forceinline__ void silu_tile(const f32x16 &acc, float (&v)[16]) {
+  if constexpr (TeamGeo<P>::SPLIT) {
+    float half[8];
+#pragma unroll
+    for (int e0 = 0; e0 < 16; e0 += 8) {
+      split_silu8(acc, e0, half);
+#pragma unroll
+      for (int e = 0; e < 8; ++e) v[e0 + e] = half[e];
+    }
+  } else {
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int e = 0; e < 16; ++e) v[e] = __builtin_amdgcn_exp2f(acc[e]);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int e = 0; e < 16; ++e) v[e] = 1.0f + v[e];
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int e = 0; e < 16; ++e) v[e] = __builtin_amdgcn_rcpf(v[e]);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int e = 0; e < 16; ++e) v[e] = acc[e] * v[e];
+    __builtin_amdgcn_sched_barrier(0);
+  }
+}
+
 // SiLU of one accumulator tile into the record at `rec` (cout tile t): planes, and the fp6 block.
 // UNDER: the one-workgroup kernel takes this tile's low-order parts behind MFMAs (see epi_atom).
 template <class P, bool LO, bool UNDER>
@@ -260,28 +287,27 @@ __device__ __forceinline__ void team_store(unsigned char *smem, int rec, int h, 
   unsigned char *at = smem + rec + 64 * t + 8 * h;
   if constexpr (T::SPLIT) {
 #pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      float v[4];
+    for (int q = 0; q < 4; q += 2) {
+      float v[8];
+      int w[3][4];
+      split_silu8(acc, 4 * q, v);
+      split_planes8(v, w);
 #pragma unroll
-      for (int e = 0; e < 4; ++e) v[e] = split_silu(acc[4 * q + e]);
+      for (int i = 0; i < 3; ++i)
 #pragma unroll
-      for (int i = 0; i < 3; ++i) {
-        const int a = i < 2 ? split_take(v[0], v[1]) : pack2<PrecBF16>(v[0], v[1]);
-        const int b = i < 2 ? split_take(v[2], v[3]) : pack2<PrecBF16>(v[2], v[3]);
-        *reinterpret_cast<v2i *>(at + i * 192 + 16 * q) = v2i{a, b};
-      }
+        for (int e = 0; e < 2; ++e) *reinterpret_cast<v2i *>(at + i * 192 + 16 * (q + e)) = v2i{w[i][2 * e], w[i][2 * e + 1]};
     }
   } else {
     const DropConsts k = drop_consts<P>();
-    float lo[16], m = 0.0f;
+    float v[16], lo[16], m = 0.0f;
+    silu_tile<P>(acc, v);
 #pragma unroll
     for (int q = 0; q < 4; ++q) {
       int hi[2];
 #pragma unroll
       for (int p = 0; p < 2; ++p) {
         const int i = 4 * q + 2 * p;
-        const float v0 = acc[i] * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(acc[i]));
-        const float v1 = acc[i + 1] * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(acc[i + 1]));
+        const float v0 = v[i], v1 = v[i + 1];
         hi[p] = pack2<P>(v0, v1);
         if constexpr (LO) {
           if constexpr (UNDER) {
@@ -595,6 +621,9 @@ __device__ __forceinline__ void team_board(const TeamParams &prm, unsigned char 
             float pol[PT], val[PT];
 #pragma unroll
             for (int i = 0; i < PT; ++i) pol[i] = val[i] = 0.0f;
+            float a[PT][16];
+#pragma unroll
+            for (int i = 0; i < PT; ++i) silu_tile<P>(acc[i][t], a[i]);
 #pragma unroll
             for (int q = 0; q < 4; ++q)
 #pragma unroll
@@ -602,9 +631,8 @@ __device__ __forceinline__ void team_board(const TeamParams &prm, unsigned char 
                 const float p1 = pw[32 * (t0 + t) + 8 * q + e], v1 = pw[kHeadC + 32 * (t0 + t) + 8 * q + e];
 #pragma unroll
                 for (int i = 0; i < PT; ++i) {
-                  const float a = split_silu(acc[i][t][4 * q + e]);
-                  pol[i] = fmaf(a, p1, pol[i]);
-                  val[i] = fmaf(a, v1, val[i]);
+                  pol[i] = fmaf(a[i][4 * q + e], p1, pol[i]);
+                  val[i] = fmaf(a[i][4 * q + e], v1, val[i]);
                 }
               }
 #pragma unroll
@@ -630,7 +658,13 @@ __device__ __forceinline__ void team_board(const TeamParams &prm, unsigned char 
             if (t0 + t >= NT) continue;
             float val0[PT];
 #pragma unroll
-            for (int i = 0; i < PT; ++i) val0[i] = 0.0f;
+            for (int i = 0; i < PT; ++i) {
+              val0[i] = 0.0f;
+              float a[16];
+              silu_tile<P>(acc[i][t], a);
+#pragma unroll
+              for (int e = 0; e < 16; ++e) acc[i][t][e] = a[e];
+            }
 #pragma unroll
             for (int q = 0; q < 4; ++q) {
               pw4[t][q] = *reinterpret_cast<const f32x4 *>(pw + 32 * (t0 + t) + 8 * q);
@@ -640,8 +674,7 @@ __device__ __forceinline__ void team_board(const TeamParams &prm, unsigned char 
                 float vs = 0.0f;
 #pragma unroll
                 for (int e = 0; e < 4; ++e) {
-                  const float a = silu<P>(acc[i][t][4 * q + e]);
-                  acc[i][t][4 * q + e] = a;
+                  const float a = acc[i][t][4 * q + e];
                   val0[i] = fmaf(a, vw4[e], val0[i]);
                   vs = fmaf(a, vw4[e], vs);
                 }

@@ -245,7 +245,7 @@ constexpr size_t cascade_packed_bytes(int prec) {
 // that a workgroup evaluates (per = its share of their boards, rounded up: less than `grid` entries more than
 // those), and behind them one for each board that a team shares, a run by itself.  So the entries are fewer than the
 // boards and kCascadeMaxRuns together, whatever the rules share out.
-constexpr int kCascadeMaxRuns = 1024;   // workgroups of the first pass: two per compute unit, at most
+constexpr int kCascadeMaxRuns = 1024;   // runs of the first pass: two per compute unit and a board that teams share each, at most
 constexpr long long redo_entry(long long run, long long grid, long long per) {   // where a run's list starts
   return run < grid ? run * per : grid * per + (run - grid);
 }

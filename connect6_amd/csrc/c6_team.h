@@ -252,7 +252,9 @@ __device__ __forceinline__ void team_conv(const unsigned char *smem, const unsig
   }
 }
 
-// SiLU of one accumulator tile, step by step: a lone wave waits for each result that its next instruction needs.
+// SiLU of one accumulator tile, step by step: a lone wave waits for each result that its next instruction needs.  Against
+// output by output, in a forward: one board in fp32 61.3 -> 60.3 us, in bf16 33.8 -> 33.4; 53 boards in fp32, whose waves
+// wait for weights rather, 117.7 -> 116.8 on one box and nothing on another.
 template <class P> __device__ __forceinline__ void silu_tile(const f32x16 &acc, float (&v)[16]) {
   if constexpr (TeamGeo<P>::SPLIT) {
     float half[8];

@@ -2521,7 +2521,6 @@ int dispatch_team(int prec, const TeamParams &tp, hipStream_t st) {
   if (shared < all && m.launch_rest != nullptr) {
     part.f.total_boards = all - shared;
     part.rest = (unsigned)shared;
-    part.polls = tp.polls < (1 << 20) ? 4 * tp.polls : tp.polls;   // (a team's workgroups start as others end, within some microseconds)
     return m.launch_rest(part, cus, st);
   }
   if (shared < all) {

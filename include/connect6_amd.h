@@ -203,8 +203,7 @@ int c6_forward_boards_cascade(const int8_t *boards, const int8_t *player,
  *   tag        not 0; a cascade also uses tag + 1.  Which XCD a workgroup is on is told with a tag's low 28
  *              bits, so those are not used twice either between two clearings of the words: after 2^27 calls
  *              that count two each, clear them and begin at 1 again
- *   polls      how often a workgroup looks at a flag before it computes the piece itself; 0: 64 (four times as often
- *              where the teams start beside other workgroups: C6_PREC_BF16, _F16 and the cascades, more boards than CUs)
+ *   polls      how often a workgroup looks at a flag before it computes the piece itself; 0: 64
  * No synchronisation with the host.  Every wait is bounded: a workgroup that has
  * waited too long computes what it waits for. */
 int c6_team_bytes(int prec, int64_t boards, size_t *workspace_bytes, size_t *flag_bytes);

@@ -71,6 +71,15 @@ def test_kernels_of_networks_that_fill_the_lds_use_no_scratch():
     assert len(full) == 4 and all(u["ScratchSize"] == 0 for u in full)
 
 
+def test_every_launch_waits_as_long_as_its_caller_says():
+    """A wait for a flag is bounded by the caller's polls, whatever the route: the entry point sets them, no rule behind it
+    makes them more."""
+    sources = sorted((ROOT / "connect6_amd" / "csrc").glob("*.h*"))
+    written = [(f.name, line.strip()) for f in sources for line in f.read_text().splitlines()
+               if re.search(r"\bpolls\s*[-+*/|&^]?=(?!=)", line)]
+    assert written == [("c6_api.hip", "tp.polls = t.polls > 0 ? t.polls : kTeamPolls;")]
+
+
 def test_history_dtype_follows_the_reference_policy():
     # connect6/train.py:133-145
     cpu, gpu = torch.device("cpu"), torch.device("cuda", 0)

@@ -2470,16 +2470,27 @@ static int second_mode(int cascade) { return cascade == C6_PREC_BF16C ? C6_PREC_
 //         + 40     212 / 190     202 / 180     297 / 272         4,096 + 9    923 / 900     872 / 852     1,011 / 986
 //         + 80     214 / 203     204 / 192     299 / 284         4,864 + 9    1,106 / 1,063 1,045 / 1,005 1,245 / 1,205
 // (256, 768, 1,280 + 9 "without" is a launch of teams behind the others from 768 on.)  So at two rounds teams of three are
-// not worth it, and neither are teams of two anywhere but at an odd few rounds (256 + 104 94 / 94 and 768 + 128 209 / 204, but 256
-// + 128 95 / 100 and 1,280 + 128 315 / 327).
+// not worth it (one point, 512 + 80), and neither are teams of two anywhere but at an odd few rounds (256 + 104 94 / 94 and 768 + 128
+// 209 / 204, but 256 + 128 95 / 100 and 1,280 + 128 315 / 327).  Behind many rounds the clock has time to give back what the rest
+// costs, and what teams gain gets small; one board behind sixteen rounds, two behind 32 and three behind 48 are in the end
+// slower in teams and stay with the others.  Without / with in turn, us (medians of sixteen; they repeat to 0.3 %):
+//     rounds   fp16 + 1       + 3          + 40         + 80         bf16 + 1       + 3          + 40         + 80
+//     8        473 / 465      487 / 463    489 / 473    492 / 484    444 / 439      459 / 437    464 / 451    471 / 467
+//     13       750 / 736                   786 / 754    786 / 765    712 / 695                   744 / 711    745 / 721
+//     16       913 / 913      941 / 921    960 / 942    962 / 952    869 / 865      883 / 874    897 / 884    899 / 901
+//     20       1,141 / 1,140  1,171 / 1,163             1,188 / 1,176  1,082 / 1,093  1,091 / 1,087             1,115 / 1,114
+//     32       1,882 / 1,874  1,880 / 1,874  1,901 / 1,878  1,919 / 1,901  1,735 / 1,750  1,741 / 1,742  1,762 / 1,755  1,762 / 1,764
+//     48       2,831 / 2,824  2,838 / 2,831  2,846 / 2,828  2,857 / 2,841  2,611 / 2,617  2,612 / 2,626  2,629 / 2,637  2,634 / 2,638
+//     63       3,733 / 3,716  3,735 / 3,727  3,745 / 3,688  3,749 / 3,699  3,430 / 3,440  3,430 / 3,444  3,466 / 3,448  3,476 / 3,462
 static long long team_boards(int prec, long long boards, int cus) {
   const TeamMode m = team_mode(prec);
   if (m.launch == nullptr) return 0;
   if (boards <= cus) return m.size(boards, cus) > 1 ? boards : 0;
   const long long rest = boards % cus;
   if (m.launch_rest == nullptr) return rest <= m.most(cus) ? rest : 0;
+  const long long rounds = boards / cus;
   const int size = m.rest(rest, cus);
-  return size > 3 || (size > 1 && boards / cus != 2) ? rest : 0;
+  return (size > 3 || (size > 1 && rounds != 2)) && 16 * rest > rounds ? rest : 0;
 }
 
 // Boards of a cascade whose two passes are one launch: those that twelve workgroups share (team_cascade_kernel)

@@ -109,7 +109,7 @@ def test_rest_in_teams_beside_whole_rounds(cuda, prec, rounds):
         for rest in (1, 2, cus // 12, cus // 12 + 1, cus * 5 // 32, cus * 5 // 32 + 1, cus * 5 // 16, cus * 5 // 16 + 1):
             n = rounds * cus + rest
             _same(call(slice(0, n)), [w[:n] for w in want])
-        # through the C ABI, each workgroup looking at a flag four times only
+        # through the C ABI, each workgroup looking at a flag once only
         lib, n = c6.load(), rounds * cus + cus * 5 // 32
         ws, fl = ctypes.c_size_t(), ctypes.c_size_t()
         assert lib.c6_team_bytes(prec, n, ctypes.byref(ws), ctypes.byref(fl)) == 0 and ws.value > 0
@@ -125,7 +125,28 @@ def test_rest_in_teams_beside_whole_rounds(cuda, prec, rounds):
             _same((logits, value), (raw[0][:n], raw[1][:n]))
 
 
-@pytest.mark.parametrize("boards", [257, 336, 513, 1400, 1576, 4096])
+@pytest.mark.parametrize("prec", [_lib.PREC_BF16, _lib.PREC_F16])
+def test_one_board_behind_many_rounds_is_not_shared(cuda, prec):
+    """Teams gain nothing there: they take a rest of more than one board for every sixteen rounds, here at the edges of that
+    rule.  (Exchange memory is what tells which way a batch goes.)  The same bits on either side."""
+    cus = torch.cuda.get_device_properties(cuda).multi_processor_count
+    model, lib = _model(cuda), c6.load()
+    packed = model.packed_weights(prec)
+    ws, fl = ctypes.c_size_t(), ctypes.c_size_t()
+    for rounds, rest, shared in ((15, 1, True), (16, 1, False), (16, 2, True), (31, 2, True), (32, 2, False), (32, 3, True),
+                                 (63, 3, False), (63, 4, True), (63, 80, True)):
+        assert lib.c6_team_bytes(prec, rounds * cus + rest, ctypes.byref(ws), ctypes.byref(fl)) == 0
+        assert (ws.value > 0) == shared and (fl.value > 0) == shared, (rounds, rest)
+    x = _inputs(399)[0].to(cuda)
+    with torch.inference_mode():
+        part = run_forward(x[:100], packed, prec, 1, 100)
+        for n in (15 * cus + 1, 16 * cus + 1, 16 * cus + 2):
+            pick = torch.arange(n, device=cuda) % 100
+            got = run_forward(x[pick], packed, prec, 1, n)
+            assert torch.equal(got[0], part[0][pick]) and torch.equal(got[1], part[1][pick]), n
+
+
+@pytest.mark.parametrize("boards", [257, 336, 513, 1400, 1576, 4096, 4097, 4098])
 def test_cascade_lists_the_same_boards(cuda, boards):
     model = c6.PolicyValueNet().to(cuda).eval()
     model.load_state_dict(R.init_state(5, "reference"))

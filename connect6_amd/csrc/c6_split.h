@@ -106,6 +106,9 @@ template <int NT> __device__ __forceinline__ void split_preload(v4i (&ring)[kSpl
 
 // A product whose sum is in vector registers: the compiler puts every sum of the instruction in accumulation
 // registers, and there are 256 of those.  (s_nop: an operand may just have been written by the vector unit.)
+// Nothing else may touch such a sum in front of mma_vector_wait: the compiler does not know that it is still being written.
+// It has no reason to, since the sums of a layer are written in front of its loop and read behind the wait;
+// tests/test_registers.py reads off the built kernel that it did not.
 __device__ __forceinline__ void mma_vector(const v4i &a, const v4i &b, f32x16 &c) {
   asm volatile("s_nop 1\n\tv_mfma_f32_32x32x16_bf16 %0, %1, %2, %0" : "+v"(c) : "v"(a), "v"(b));
 }

@@ -125,6 +125,64 @@ def test_rest_in_teams_beside_whole_rounds(cuda, prec, rounds):
             _same((logits, value), (raw[0][:n], raw[1][:n]))
 
 
+@pytest.mark.parametrize("rounds,rest", [(1, 9), (2, 30), (3, 60)])   # twelve, six and three workgroups per board
+@pytest.mark.parametrize("precision", ["bf16", "fp16"])
+def test_board_state_of_a_rest(cuda, precision, rounds, rest):
+    """int8 states, rows picked (some outside: they are clamped), every board symmetry, where a rest goes to teams."""
+    n = rounds * torch.cuda.get_device_properties(cuda).multi_processor_count + rest
+    model = _model(cuda, 20)
+    model.precision = precision
+    g = torch.Generator().manual_seed(3)
+    boards = torch.randint(-1, 2, (700, 19, 19), generator=g, dtype=torch.int8).to(cuda)
+    player = (torch.randint(0, 2, (700,), generator=g, dtype=torch.int8) * 2 - 1).to(cuda)
+    left = torch.randint(1, 3, (700,), generator=g, dtype=torch.int8).to(cuda)
+    index, u = torch.randint(-5, 710, (n,), generator=g).to(cuda), gen_uniform(n, 6).to(cuda)
+    with torch.inference_mode():
+        for view in range(8):
+            part = lambda s: model.forward_boards(boards, player, left, index=index[s], view=view)
+            _same(part(slice(0, n)), _pieces(part, n))
+            part = lambda s: model.selfplay_step_boards(boards, player, left, u[s], 0.7, index=index[s], view=view)
+            _same(part(slice(0, n)), _pieces(part, n))
+
+
+@pytest.mark.parametrize("rounds,rest", [(1, 9), (2, 30), (3, 60)])
+@pytest.mark.parametrize("precision", ["bf16", "fp16", "bf16c"])
+def test_graphs_and_streams_of_a_rest(cuda, precision, rounds, rest):
+    """A rest in teams: a graph replayed behind eager work, and calls on three streams at once."""
+    n = rounds * torch.cuda.get_device_properties(cuda).multi_processor_count + rest
+    model = _model(cuda)
+    model.precision = precision
+    x = _inputs(n)[0]
+    xs = [torch.roll(x, 100 * i, 0).to(cuda) for i in range(3)]
+    with torch.inference_mode():
+        want = [_pieces(lambda s: model(v[s]), n) for v in xs]
+        static = xs[0].clone()
+        side = torch.cuda.Stream()
+        side.wait_stream(torch.cuda.current_stream())
+        with torch.cuda.stream(side):
+            model(static)
+        torch.cuda.current_stream().wait_stream(side)
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph):
+            out = model(static)
+        for i in (0, 1, 2, 1, 0):
+            static.copy_(xs[i])
+            graph.replay()
+            model(xs[2])                       # eager work in between
+            torch.cuda.synchronize()
+            _same(out, want[i])
+        streams = [torch.cuda.Stream() for _ in range(3)]
+        torch.cuda.synchronize()
+        got = []
+        for _ in range(4):
+            for i, s in enumerate(streams):
+                with torch.cuda.stream(s):
+                    got.append((i, model(xs[i])))
+        torch.cuda.synchronize()
+        for i, answer in got:
+            _same(answer, want[i])
+
+
 @pytest.mark.parametrize("prec", [_lib.PREC_BF16, _lib.PREC_F16])
 def test_one_board_behind_many_rounds_is_not_shared(cuda, prec):
     """Teams gain nothing there: they take a rest of more than one board for every sixteen rounds, here at the edges of that

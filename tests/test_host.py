@@ -45,9 +45,10 @@ def test_fused_kernels_stay_within_their_scratch_budget():
     # two workgroups per CU: half the registers, half the LDS
     duo = [u for name, u in usage.items() if "duo_forward_kernel" in name]
     assert len(duo) == 2 and all(u["Occupancy"] == 2 and u["ScratchSize"] <= 16 for u in duo)
-    # ... and teams beside them: the teams' code may use some scratch
+    # ... and teams beside them: in scratch is what teams of three keep, and a few addresses of the others, touched at a
+    # board's head and end
     rest = [u for name, u in usage.items() if "duo_rest_kernel" in name]
-    assert len(rest) == 2 and all(u["Occupancy"] == 2 and u["ScratchSize"] <= 128 for u in rest)
+    assert len(rest) == 2 and all(u["Occupancy"] == 2 and u["ScratchSize"] <= 88 for u in rest)
     # a board shared by several workgroups, and small networks: nothing in scratch (scalar registers spill
     # into vector ones)
     team = [u for name, u in usage.items() if "team_forward_kernel" in name]

@@ -26,11 +26,11 @@
 // six times and the first layer's 207 three times (0/1 inputs are exact in one bf16 value); then the epilogues,
 // some 25 instructions per output of a lane (two of them at a quarter of the rate) that one wave per SIMD issues in
 // the open.  They go step by step over eight outputs, because a lone wave waits wherever an instruction needs the
-// one before it.  The activations of up to 64 channels lie in LDS as their three planes, split once when a layer writes
+// one before it (a per cent: 256 boards 281.8 -> 278.6 us, 2,048 boards 2,200 -> 2,184; scratch 200 -> 84 bytes a lane).  The activations of up to 64 channels lie in LDS as their three planes, split once when a layer writes
 // them; 96 channels only fit as fp32 (421 positions x 384 bytes are the CU's whole LDS), and the two
 // layers that read them split them in registers, 44 instructions for eight values, a few behind each
-// MFMA.  2,048 boards take 2.29 ms (2.42 on the same box while the layers of 96 outputs ran in two passes over
-// the pixel tiles and read their weights twice, and epilogues output by output; 4.35 with
+// MFMA.  2,048 boards take 2.18 ms (2.31 on the same box while the layers of 96 outputs ran in two passes over
+// the pixel tiles and read their weights twice, 2.20 in one pass with epilogues output by output; on another 4.35 with
 // fp32 instructions).
 //
 // An infinity is its own first part; what is left of it is a NaN in the sum of the small products, and the
@@ -227,7 +227,8 @@ __device__ __forceinline__ void split_conv(const unsigned char *smem, const WFra
     for (int k = 0; k < 8; ++k) asm volatile("" : "+a"(acc[k / 3][k % 3]), "+a"(low[k / 3][k % 3]));
   }
 }
-// The sums of one tile, taken out of the accumulation registers here and not with all the others at once
+// The sums of one tile, taken out of the accumulation registers here and not with all the others at once (which is 1,020 bytes of
+// scratch a lane, and 3.49 ms for 2,048 boards in place of 2.20)
 template <int NT>
 __device__ __forceinline__ f32x16 split_total(const f32x16 (&acc)[NT][3], const f32x16 (&low)[NT][3], int t, int j) {
   f32x16 large = acc[t][j], small = low[t][j], sum;

@@ -80,8 +80,10 @@ template <class P> struct TeamGeo {
 // tiles of squares each, whose four waves take PT of them and form CG groups of cout tiles.  A wave takes two
 // tiles of squares where there are two: with six workgroups each weight is then read by one wave, with three
 // by two; with one tile of squares per wave it would be twice as many, 96 and 128 bytes a cycle where the L1
-// gives 64 (six workgroups, 22 to 42 boards, bf16 + fp6 62.6 -> 55 us).  (fp32 contracts a weight with three
-// parts: there the L1 keeps up, and all four waves have work in layers of two cout tiles.)
+// gives 64 (six workgroups, 22 to 42 boards, bf16 + fp6 62.6 -> 55 us).  (fp32 contracts a weight with three parts, so
+// that a tile of squares per wave asks for just those 64, and all four waves have work in layers of two cout tiles.  Counted
+// over 53 boards, three workgroups each: of the 263 k cycles of a workgroup 150 k are reads from the L1, 64 bytes each, 128 k
+// MFMAs, so the L1 bounds the contractions by a sixth.)
 // Three or six tiles of squares go to three waves, all cout tiles in each; the fourth watches the flags.
 template <class P, int TEAM> struct TeamShape {
   static constexpr int PXT = 12 / TEAM;
@@ -157,7 +159,7 @@ __device__ __forceinline__ void team_lo_pass(const unsigned char *smem, const un
 // The contraction of 3x3 layer L for PT tiles of 32 squares and TT cout tiles from t0 on (tiles beyond
 // the layer's last repeat it; their results are not used).
 //   rec: LDS addresses of the lane's squares' records;  acc: the bias on entry
-//   low (fp32): what the bias leaves out, for the small products' sum (split_conv_tiles)
+//   low (fp32): what the bias leaves out, for the small products' sum (split_conv)
 template <class P, int L, int TT, int PT>
 __device__ __forceinline__ void team_conv(const unsigned char *smem, const unsigned char *packed, const WFrags &wl,
                                           v4i (&ring)[team_ring<P, TT, PT>()][TT][Geo<P>::W], int lane,
@@ -253,8 +255,9 @@ __device__ __forceinline__ void team_conv(const unsigned char *smem, const unsig
 }
 
 // SiLU of one accumulator tile, step by step: a lone wave waits for each result that its next instruction needs.  Against
-// output by output, in a forward: one board in fp32 61.3 -> 60.3 us, in bf16 33.8 -> 33.4; 53 boards in fp32, whose waves
-// wait for weights rather, 117.7 -> 116.8 on one box and nothing on another.
+// output by output it is worth a per cent, one way or the other: 22 to 40 boards in bf16 and fp16 40.0 -> 39.6 us, 40 boards that
+// a cascade lists 117.2 -> 116.2, 86 to 128 fp32 boards 217.2 -> 215.5; but 1 to 16 boards in bf16 30.2 -> 30.6; one and 53 fp32
+// boards, and the teams beside whole rounds, the same.
 template <class P> __device__ __forceinline__ void silu_tile(const f32x16 &acc, float (&v)[16]) {
   if constexpr (TeamGeo<P>::SPLIT) {
     float half[8];
@@ -413,7 +416,9 @@ __device__ __forceinline__ void team_board(const TeamParams &prm, unsigned char 
   constexpr int kWatch = S::PG * CG == 3 ? 3 : 0;   // the wave that watches the flags: one that has no weights to wait for
   auto wait_inputs = [&](int l, int role, bool own) {
     if (wave == kWatch) {
-      // (the words of the first layer's workgroups have been there since they started)
+      // (Looked at once.  A word that is missing is that of a workgroup that has not come as far as the first layer: then this one
+      // stores through to memory to the end, which is correct and slower.  It does not happen where a team lies on one XCD, also
+      // not in duo_rest_kernel, whose workgroups start as others end: counted over 257 to 1,616 boards, every one saw all.)
       unsigned about = xcd;
       if (l == 1 && lane < TEAM) about = __hip_atomic_load(&flags[kTeamXcd + lane], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) ^ xcd_tag;
       if (l == 1 && __builtin_amdgcn_ballot_w64(about != xcd) == 0) local = true;
@@ -1153,9 +1158,12 @@ template <class P> __global__ __launch_bounds__(256) void team_forward_kernel(co
 // in fp16 202 -> 181 us (teams in front without the second workgroup's priority 189; without either, 188 and 71 -> 74 at
 // 257 boards).  What bounds it: 512 + 9 boards take 15 us more than 512, of which the other workgroups, alone on their CUs
 // in the end, are most.
-// Registers: the teams' contractions want more than the 256 that two workgroups per CU leave; what is in scratch (under 128
-// bytes a lane) is theirs.
-// The workgroups per board of a rest (1: none are shared), as many as half of the places hold, and a team on one XCD.
+// Registers: the teams' contractions want more than the 256 that two workgroups per CU leave.  In scratch (80 bytes a lane) is
+// what teams of three keep, and with it some addresses of the boards that have a workgroup each: a dozen accesses at the
+// head and the end of a board, none between its MFMAs.
+// The workgroups per board of a rest (1: none are shared), as many as half of the places hold.  A team lies on one XCD but for
+// 17 to 21 boards (of 256 CUs): three teams of twelve do not fit the 32 places that an XCD has, so they are dealt out over all
+// XCDs and exchange through memory, as they do without other boards.
 template <class P> __host__ __device__ inline int rest_team(long long boards, int cus) {
   if (!has_duo<P>()) return 1;
   if (boards * 12 <= cus) return 12;

@@ -206,11 +206,11 @@ def test_second_pass_of_whole_rounds_and_a_rest(cuda, prec, boards):
 
 @pytest.mark.parametrize("prec", [_lib.PREC_BF16, _lib.PREC_F16, _lib.PREC_BF16C, _lib.PREC_BF16C6])
 def test_a_rest_behind_an_odd_number_of_rounds(cuda, prec):
-    """Two workgroups per CU, and teams for a few boards beyond 3, 5, ... 11 rounds: the bits and the listed boards of
-    batches that go to one kernel, at the edges of the rule."""
+    """Two workgroups per CU, and teams for a rest beside them: the bits and the listed boards of batches that have no team, at
+    the edges of the rule (teams of twelve, six and three; at two rounds of the first two only)."""
     cus = torch.cuda.get_device_properties(cuda).multi_processor_count
-    most = cus * 5 // 32
-    total = 11 * cus + most + 1
+    most, three = cus * 5 // 32, cus * 5 // 16
+    total = 11 * cus + three + 1
     x, legal = gen_boards(400, 200, 31)
     pick = torch.arange(total) % 399
     xd, ld, u = x[pick].to(cuda), legal[pick].to(cuda), gen_uniform(total, 5).to(cuda)
@@ -225,8 +225,9 @@ def test_a_rest_behind_an_odd_number_of_rounds(cuda, prec):
                 return out, int(stats["second_pass"]) if cascade else 0
             parts = [call(i, min(i + 100, total)) for i in range(0, total, 100)]
             want = [torch.cat(t) for t in zip(*[p[0] for p in parts])]
-            for n in (2 * cus + 9, 3 * cus, 3 * cus + 1, 3 * cus + 2, 3 * cus + 9, 3 * cus + most, 3 * cus + most + 1,
-                      4 * cus + 9, 5 * cus + 21, 11 * cus + 5, 11 * cus + 6, total - 1, total):
+            for n in (2 * cus + 9, 2 * cus + most, 2 * cus + most + 1, 3 * cus, 3 * cus + 1, 3 * cus + 2, 3 * cus + 9,
+                      3 * cus + most, 3 * cus + most + 1, 3 * cus + three, 3 * cus + three + 1, 4 * cus + 9, 5 * cus + 21,
+                      11 * cus + 5, 11 * cus + 6, total - 1, total):
                 got, listed = call(0, n)
                 for a, b in zip(got, want):
                     assert torch.equal(a, b[:n]), (threshold, n)

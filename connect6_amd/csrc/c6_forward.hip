@@ -2472,16 +2472,16 @@ static int second_mode(int cascade) { return cascade == C6_PREC_BF16C ? C6_PREC_
 // (256, 768, 1,280 + 9 "without" is a launch of teams behind the others from 768 on.)  So at two rounds teams of three are
 // not worth it (one point, 512 + 80), and neither are teams of two anywhere but at an odd few rounds (256 + 104 94 / 94 and 768 + 128
 // 209 / 204, but 256 + 128 95 / 100 and 1,280 + 128 315 / 327).  Behind many rounds the clock has time to give back what the rest
-// costs, and what teams gain gets small; one board behind sixteen rounds, two behind 32 and three behind 48 are in the end
-// slower in teams and stay with the others.  Without / with in turn, us (medians of sixteen; they repeat to 0.3 %):
-//     rounds   fp16 + 1       + 3          + 40         + 80         bf16 + 1       + 3          + 40         + 80
-//     8        473 / 465      487 / 463    489 / 473    492 / 484    444 / 439      459 / 437    464 / 451    471 / 467
-//     13       750 / 736                   786 / 754    786 / 765    712 / 695                   744 / 711    745 / 721
-//     16       913 / 913      941 / 921    960 / 942    962 / 952    869 / 865      883 / 874    897 / 884    899 / 901
-//     20       1,141 / 1,140  1,171 / 1,163             1,188 / 1,176  1,082 / 1,093  1,091 / 1,087             1,115 / 1,114
-//     32       1,882 / 1,874  1,880 / 1,874  1,901 / 1,878  1,919 / 1,901  1,735 / 1,750  1,741 / 1,742  1,762 / 1,755  1,762 / 1,764
-//     48       2,831 / 2,824  2,838 / 2,831  2,846 / 2,828  2,857 / 2,841  2,611 / 2,617  2,612 / 2,626  2,629 / 2,637  2,634 / 2,638
-//     63       3,733 / 3,716  3,735 / 3,727  3,745 / 3,688  3,749 / 3,699  3,430 / 3,440  3,430 / 3,444  3,466 / 3,448  3,476 / 3,462
+// costs, and what teams gain gets small: from some twenty rounds on one board, from 28 on two and three are no faster in teams in
+// fp16 and up to 1 % slower in bf16.  The line leaves them with the others: one board behind sixteen rounds, two behind 32, three
+// behind 48.  Without / with in turn, us (medians of sixteen; the ratios repeat to half a per cent, to one at a single board):
+//     rounds  fp16 + 1       + 3            + 40           + 80           bf16 + 1       + 3            + 40           + 80
+//     8       473 / 465      487 / 463      489 / 473      492 / 484      444 / 439      459 / 437      464 / 451      471 / 467
+//     16      913 / 913      941 / 921      960 / 942      962 / 952      869 / 865      883 / 874      897 / 884      899 / 901
+//     20      1,141 / 1,140  1,171 / 1,163  -              1,188 / 1,176  1,082 / 1,093  1,091 / 1,087  -              1,115 / 1,114
+//     32      1,882 / 1,874  1,880 / 1,874  1,901 / 1,878  1,919 / 1,901  1,735 / 1,750  1,741 / 1,742  1,762 / 1,755  1,762 / 1,764
+//     48      2,831 / 2,824  2,838 / 2,831  2,846 / 2,828  2,857 / 2,841  2,611 / 2,617  2,612 / 2,626  2,629 / 2,637  2,634 / 2,638
+//     63      3,733 / 3,716  3,735 / 3,727  3,745 / 3,688  3,749 / 3,699  3,430 / 3,440  3,430 / 3,444  3,466 / 3,448  3,476 / 3,462
 static long long team_boards(int prec, long long boards, int cus) {
   const TeamMode m = team_mode(prec);
   if (m.launch == nullptr) return 0;

@@ -100,7 +100,7 @@ def main() -> int:
     wall, kern = run_mode(args.precision, K, W)
     value = B / wall
     achieved = B * CONV_FLOP_PER_BOARD / kern / 1e12
-    kernel_name = {"fp32": "split_forward_kernel<fp32>", "bf16": "duo_forward_kernel<bf16>",
+    kernel_name = {"fp32": "half_forward_kernel<fp32>", "bf16": "duo_forward_kernel<bf16>",
                    "fp16": "duo_forward_kernel<fp16>"}.get(args.precision, f"fused_pipe_kernel<{args.precision}>")
     cascade = None
     if args.precision == "bf16c":

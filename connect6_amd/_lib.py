@@ -342,7 +342,7 @@ def check(rc: int, what: str) -> None:
 
 def kernel_prec(prec: int) -> int:
     """The mode whose kernel and packed weights serve ``prec`` in the default architecture: fp32
-    operands go through the bf16 matrix cores as three exact parts each."""
+    operands go through the fp16 matrix cores as two parts each."""
     return PREC_F32S if prec == PREC_F32 else prec
 
 

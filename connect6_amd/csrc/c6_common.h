@@ -112,8 +112,8 @@ struct PrecBF16F6W {
   static constexpr int LO_MASK = 0xfe;
 };
 
-// fp32 on the bf16 matrix cores: every weight is the exact sum of three bf16 values (8 mantissa bits
-// each), packed as three fragments that follow one another; so is every activation.  c6_split.h.
+// fp32 on the fp16 matrix cores: every weight is two fp16 values, and what they leave of it, packed as three fragments that
+// follow one another; an activation is two.  c6_half.h; boards beyond fp16's range: c6_split.h, on the same weights.
 struct PrecF32S {
   static constexpr int WLO = 2;
   static constexpr int PIPE = 0;      // weights packed tap-major
@@ -142,6 +142,11 @@ __host__ __device__ constexpr int lo6_channel(int block, int slot) {
   const int i = (s >> 1) + 8 * (s & 1);
   return 32 * block + 8 * (i >> 2) + 4 * hh + (i & 3);
 }
+
+// Factors of weights and activations there, of the second parts, the largest number that counts as within the range, and how
+// small a layer's largest may be.  kHalfMark: a weight that is beyond it (an fp16 NaN).
+constexpr float kHalfW = 16.0f, kHalfA = 16.0f, kHalfLow = 2048.0f, kHalfMost = 32768.0f, kHalfLeast = 0x1p-14f;
+constexpr int kHalfMark = 0x7fff;
 
 template <class P> struct Geo {
   static constexpr int EB = P::EB;

@@ -1918,6 +1918,7 @@ __global__ __launch_bounds__(256) void fused_forward_kernel(const FwdParams prm)
 }  // namespace c6
 
 #include "c6_split.h"
+#include "c6_half.h"
 #include "c6_duo.h"
 #if defined(C6_TEAM) || defined(C6_CASCADE) || !defined(C6_INSTANCE)
 #include "c6_team.h"
@@ -1948,14 +1949,16 @@ template <class P> __device__ __forceinline__ float weight_part(Scaled<P> v, int
   if constexpr (P::EB == 4) {
     return v;
   } else {
-    static_assert(P::WLO == 0 || P::ID != C6_PREC_F16, "the low part is defined for bf16 storage");
-    if constexpr (P::WLO == 2) {
-      for (int i = 0; i < part; ++i) v = bf16_rest(v, bf16_part((float)v));
-      return __builtin_bit_cast(float, (unsigned)bf16_part((float)v) << 16);
-    }
+    static_assert(P::WLO < 2 && (P::WLO == 0 || P::ID != C6_PREC_F16), "the low part is defined for bf16 storage");
     for (int i = 0; i < part; ++i) v -= __builtin_bit_cast(float, (unsigned)bits16<P>((float)v) << 16);
     return (float)v;
   }
+}
+
+// One weight's `part` as element e of a lane's 16 bytes
+template <class P> __device__ __forceinline__ void put_weight(unsigned char *dst, int e, Scaled<P> v, int part) {
+  if constexpr (P::WLO == 2) reinterpret_cast<unsigned short *>(dst)[e] = half_parts(v).part[part];
+  else put_elem<P>(dst, e, weight_part<P>(v, part));
 }
 
 // The parameters of weight set `g` of a (possibly stacked) PackParams.
@@ -1981,7 +1984,7 @@ struct GroupView {
 // one thread per (fragment, lane): writes the 16 bytes that lane will load
 // (blockIdx.y = weight set: the parameter tensors are stacked [sets, ...], the packed sets lie
 // packed_stride bytes apart)
-template <class P> __global__ void pack_kernel(const PackParams all) {
+template <class P> __global__ __launch_bounds__(256) void pack_kernel(const PackParams all) {
   using G = Geo<P>;
   const GroupView prm(all, blockIdx.y);
   const long long gid = (long long)blockIdx.x * blockDim.x + threadIdx.x;
@@ -2025,7 +2028,7 @@ template <class P> __global__ void pack_kernel(const PackParams all) {
         const float *w = prm.conv_w(0);
         for (int e = 0; e < G::E; ++e) {
           const int kx = jj * G::E + e;
-          put_elem<P>(dst, e, weight_part<P>(act_scaled<P>(kx < kK1 ? w[((m * 3 + h) * kK1 + ky) * kK1 + kx] : 0.0f), part));
+          put_weight<P>(dst, e, act_scaled<P>(kx < kK1 ? w[((m * 3 + h) * kK1 + ky) * kK1 + kx] : 0.0f), part);
         }
         return;
       }
@@ -2088,8 +2091,29 @@ template <class P> __global__ void pack_kernel(const PackParams all) {
         const int kx = jj * G::E + e;
         Scaled<P> v = 0;
         if (row < kK1 * 3 && kx < kK1) v = act_scaled<P>(w[((co * 3 + ch) * kK1 + ky) * kK1 + kx]);
-        put_elem<P>(dst, e, weight_part<P>(v, part));
+        put_weight<P>(dst, e, v, part);
       }
+    } else if constexpr (P::WLO == 2) {
+      // (tap-major; the first tap's thread takes all nine: what their parts leave is balanced over them)
+      const int kc_per_tap = cin / G::KSTEP;
+      if (part != 0 || s >= kc_per_tap) return;
+      v4i o[9][3];
+#pragma unroll
+      for (int e = 0; e < G::E; ++e) {
+        HalfParts taps[9];
+        half_taps(w + (size_t)(co * cin + s * G::KSTEP + h * G::E + e) * 9, taps);
+#pragma unroll
+        for (int k = 0; k < 9; ++k)
+#pragma unroll
+          for (int i = 0; i < 3; ++i) {
+            const int bits = taps[k].part[i];
+            o[k][i][e / 2] = e % 2 ? o[k][i][e / 2] | bits << 16 : bits;
+          }
+      }
+#pragma unroll
+      for (int k = 0; k < 9; ++k)
+#pragma unroll
+        for (int i = 0; i < 3; ++i) *reinterpret_cast<v4i *>(dst + (size_t)(k * kc_per_tap * nt * G::W + i) * 1024) = o[k][i];
     } else {
       // k-step s -> (tap, 16 or 8 input channels): tap-major, or for the pipelined kernel
       // phase-major (a phase = all nine taps of 32 input channels)
@@ -2109,7 +2133,7 @@ template <class P> __global__ void pack_kernel(const PackParams all) {
       const int cot = 32 * tile + m;
       for (int e = 0; e < G::E; ++e) {
         const int c = cbase + h * G::E + e;
-        put_elem<P>(dst, e, weight_part<P>(w[(cot * cin + c) * 9 + tap], part));
+        put_weight<P>(dst, e, w[(cot * cin + c) * 9 + tap], part);
       }
     }
     return;
@@ -2184,6 +2208,7 @@ template <class P> __global__ __launch_bounds__(256) void lo_scale_kernel(const 
 template <class P> int launch_pack(const PackParams &pp, hipStream_t st);
 template <class P> int launch_forward(const FwdParams &fp, hipStream_t st);
 
+template <class P> int launch_left(const FwdParams &fp, int cus, hipStream_t st);
 template <class P> int launch_team(const TeamParams &tp, int grid, hipStream_t st);
 template <class P> int launch_rest(const TeamParams &tp, int cus, hipStream_t st);
 template <class P> int launch_team_cascade(const TeamCascadeParams &tp, int grid, hipStream_t st);
@@ -2216,7 +2241,7 @@ template <class P> int launch_forward(const FwdParams &fp, hipStream_t st) {
   static thread_local int cus = 0;
   const void *kernel;
   if constexpr (P::ID == C6_PREC_F32S) {
-    kernel = reinterpret_cast<const void *>(&split_forward_kernel<P>);
+    kernel = reinterpret_cast<const void *>(&half_forward_kernel<P>);
   } else if constexpr (P::PIPE) {
     kernel = reinterpret_cast<const void *>(&fused_pipe_kernel<P>);
   } else {
@@ -2243,7 +2268,7 @@ template <class P> int launch_forward(const FwdParams &fp, hipStream_t st) {
   }
   const long long grid = forward_grid<P>(fp.total_boards, cus > 0 ? cus : 256);
   if constexpr (P::ID == C6_PREC_F32S) {
-    hipLaunchKernelGGL(split_forward_kernel<P>, dim3((unsigned)grid), dim3(256), LDS, st, fp);
+    hipLaunchKernelGGL(half_forward_kernel<P>, dim3((unsigned)grid), dim3(256), LDS, st, fp);
   } else if constexpr (P::PIPE) {
     bool duo = false;
     if constexpr (has_duo<P>()) {
@@ -2258,6 +2283,30 @@ template <class P> int launch_forward(const FwdParams &fp, hipStream_t st) {
   if (e != hipSuccess) {
     set_error("fused_forward launch failed: %s", hipGetErrorString(e));
     return C6_ELAUNCH;
+  }
+  return C6_OK;
+}
+
+// fp32: the boards that the kernels above left to split_forward_kernel
+template <class P> int launch_left(const FwdParams &fp, int cus, hipStream_t st) {
+  if constexpr (P::ID == C6_PREC_F32S) {
+    static thread_local int configured = -1;
+    int dev = 0;
+    hipError_t e = hipGetDevice(&dev);
+    if (e == hipSuccess && configured != dev) {
+      e = hipFuncSetAttribute(reinterpret_cast<const void *>(&split_forward_kernel<P>),
+                              hipFuncAttributeMaxDynamicSharedMemorySize, SplitGeo::LDS_BYTES);
+      if (e == hipSuccess) configured = dev;
+    }
+    if (e == hipSuccess) {
+      const long long grid = fp.total_boards < cus ? fp.total_boards : cus;
+      hipLaunchKernelGGL(split_forward_kernel<P>, dim3((unsigned)grid), dim3(256), SplitGeo::LDS_BYTES, st, fp);
+      e = hipGetLastError();
+    }
+    if (e != hipSuccess) {
+      set_error("split_forward launch failed: %s", hipGetErrorString(e));
+      return C6_ELAUNCH;
+    }
   }
   return C6_OK;
 }
@@ -2365,6 +2414,7 @@ template int launch_rest<C6_INSTANCE>(const TeamParams &, int, hipStream_t);
 #else
 template int launch_pack<C6_INSTANCE>(const PackParams &, hipStream_t);
 template int launch_forward<C6_INSTANCE>(const FwdParams &, hipStream_t);
+template int launch_left<C6_INSTANCE>(const FwdParams &, int, hipStream_t);
 #endif
 #else
 
@@ -2388,7 +2438,9 @@ int dispatch_pack(int prec, const PackParams &pp, hipStream_t st) {
   return C6_EINVAL;
 }
 
-int dispatch_forward(int prec, const FwdParams &fp, hipStream_t st) {
+static int device_cus(int &cus);
+// one workgroup per board (fp32: but for the boards that are left to split_forward_kernel)
+static int dispatch_boards(int prec, const FwdParams &fp, hipStream_t st) {
   switch (prec) {
     case C6_PREC_F32: return launch_forward<PrecF32>(fp, st);
     case C6_PREC_F32S: return launch_forward<PrecF32S>(fp, st);
@@ -2399,6 +2451,18 @@ int dispatch_forward(int prec, const FwdParams &fp, hipStream_t st) {
   }
   set_error("unknown precision mode %d", prec);
   return C6_EINVAL;
+}
+
+// ... and those: behind all other launches over these boards
+static int dispatch_left(int prec, const FwdParams &fp, hipStream_t st) {
+  if (prec != C6_PREC_F32S) return C6_OK;
+  int cus = 0;
+  const int rc = device_cus(cus);
+  return rc != C6_OK ? rc : launch_left<PrecF32S>(fp, cus, st);
+}
+int dispatch_forward(int prec, const FwdParams &fp, hipStream_t st) {
+  const int rc = dispatch_boards(prec, fp, st);
+  return rc != C6_OK ? rc : dispatch_left(prec, fp, st);
 }
 
 // compute units of the current device (the grid of the persistent kernels)
@@ -2536,12 +2600,13 @@ int dispatch_team(int prec, const TeamParams &tp, hipStream_t st) {
   }
   if (shared < all) {
     part.f.total_boards = all - shared;
-    const int rc2 = dispatch_forward(prec, part.f, st);
+    const int rc2 = dispatch_boards(prec, part.f, st);
     if (rc2 != C6_OK) return rc2;
   }
   part.f.total_boards = shared;
   part.first = (unsigned)(all - shared);
-  return m.launch(part, cus, st);   // (workgroups without a board end at once)
+  const int rc3 = m.launch(part, cus, st);   // (workgroups without a board end at once)
+  return rc3 != C6_OK ? rc3 : dispatch_left(prec, tp.f, st);
 }
 
 // Cascade: every board through the plain bf16 kernel, whose workgroups list those of their boards

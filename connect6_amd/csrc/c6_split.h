@@ -1,41 +1,35 @@
-// fp32 forward on the bf16 matrix cores (included by c6_forward.hip, whose weight rings, first-layer
-// loops and board mapping it shares).
+// fp32 forward of any board on the bf16 matrix cores (included by c6_forward.hip): the boards whose numbers do not fit
+// the two fp16 parts of c6_half.h, which serves all others.
 //
 // Every fp32 operand is the exact sum of three bf16 values: hi = bf16(v), mid = bf16(v - hi),
 // lo = v - hi - mid (8 mantissa bits each, both differences exact).  A product is then nine products
 // of bf16 values, each exact in fp32; the six down to 2^-17 of the largest are accumulated in fp32,
-// the other three are below 2^-25 of it, less than the rounding of one fp32 addition.  Against the
-// fp32 instructions (157 TFLOP/s) six bf16 ones at sixteen times the rate take 3/8 of the time.
+// the other three are below 2^-25 of it, less than the rounding of one fp32 addition.
 //
 // Two sums per output: the products of the two hi in one, the five small products in the other, added
 // up at the end.  The matrix instruction drops what lies some eight bits below the last of its sum, towards
 // minus infinity: with the small products in the large sum (324 instructions for the 864 products of the
 // last layer) that is a bias of 0.77, in units of 2^-24 of the sum's own size, the same in every square,
 // which the value head's mean over 361 squares keeps; apart, 0.02, and the scatter is 2.9 in place
-// of 7.5 (fp32 instructions: 0.03 and 8.9).  Over 64 networks with the reference's initialisation (PyTorch's)
-// the value's error against a 64-bit forward is 2.0e-10 (1.5e-9) rms, with fp32 instructions 3.9e-10
-// (2.0e-9), its mean per network 5e-11 (3.4e-10) against 2.3e-10 (5.1e-10), and the logits' relative error
-// 4.6e-7 (8e-8) against 1.4e-6 (2.0e-7).
+// of 7.5 (fp32 instructions: 0.03 and 8.9).
 //
 // The biases, scaled by -log2(e), are not fp32 numbers any more: the large sum starts with them as fp32, the
-// small one with what that leaves.  Rounded, they are an error of the same sign in every square: the mean
-// of a network's logit errors is then 2.4e-9 of the logits, so 1.1e-9 (fp32 instructions, on parameters as
-// they are: 0.7e-9; medians over 256 networks with PyTorch's initialisation).
+// small one with what that leaves.
+//
+// The packed weights are c6_half.h's three fp16 parts; split_decode makes three bf16 ones of them, in registers, in front of
+// their MFMAs.
 //
 // What bounds it: the matrix cores, 383 k cycles per board with the 1,890 MFMAs of the 3x3 layers
-// six times and the first layer's 207 three times (0/1 inputs are exact in one bf16 value); then the epilogues,
-// some 25 instructions per output of a lane (two of them at a quarter of the rate) that one wave per SIMD issues in
-// the open.  They go step by step over eight outputs, because a lone wave waits wherever an instruction needs the
-// one before it (a per cent: 256 boards 281.8 -> 278.6 us, 2,048 boards 2,200 -> 2,184; scratch 200 -> 84 bytes a lane).  The activations of up to 64 channels lie in LDS as their three planes, split once when a layer writes
+// six times and the first layer's 207 three times (0/1 inputs are exact in one bf16 value); then the weights' decoding and the
+// epilogues, some 25 instructions per output of a lane that one wave per SIMD issues in the open, step by step over eight
+// outputs.  The activations of up to 64 channels lie in LDS as their three planes, split once when a layer writes
 // them; 96 channels only fit as fp32 (421 positions x 384 bytes are the CU's whole LDS), and the two
 // layers that read them split them in registers, 44 instructions for eight values, a few behind each
-// MFMA.  2,048 boards take 2.18 ms (2.31 on the same box while the layers of 96 outputs ran in two passes over
-// the pixel tiles and read their weights twice, 2.20 in one pass with epilogues output by output; on another 4.35 with
-// fp32 instructions).
+// MFMA.
 //
 // An infinity is its own first part; what is left of it is a NaN in the sum of the small products, and the
-// large ones alone, which are then infinite or NaN as in fp32 arithmetic, are the result (two_sums; 0.4 % of
-// the time).  Parameters and inputs have three parts up to the end of fp32;
+// large ones alone, which are then infinite or NaN as in fp32 arithmetic, are the result (two_sums).  Parameters and inputs
+// have three parts up to the end of fp32;
 // a sum or an activation has them up to 2.3e38 (3.39e38, the largest bf16 value, with its factor of 1.44) and
 // counts as infinite beyond.
 //
@@ -44,10 +38,6 @@
 #pragma once
 
 namespace c6 {
-
-template <> __device__ __forceinline__ void mma<PrecF32S>(const v4i &a, const v4i &b, f32x16 &c) {
-  mma<PrecBF16>(a, b, c);
-}
 
 struct SplitGeo {
   using G = Geo<PrecF32S>;                     // weight stream and first-layer geometry
@@ -69,8 +59,8 @@ __device__ __forceinline__ int split_swz(int pos) { return ((pos >> 1) & 7) << 4
 __device__ __forceinline__ float split_logit(float sum, float bias) {
   return (float)((double)sum * (1.0 / kActScale64) + (double)bias);
 }
-__device__ __forceinline__ float split_value(float sum, float bias) {
-  return (float)tanh((double)sum * (1.0 / kActScale64 / kPix) + (double)bias);
+__device__ __forceinline__ float split_value(double sum, float bias) {
+  return (float)tanh(sum * (1.0 / kActScale64 / kPix) + (double)bias);
 }
 
 // What rounding a pair of values to the bf16 pair `w` leaves out.
@@ -95,13 +85,70 @@ __device__ __forceinline__ void split_drop4(float (&v)[8], const int (&w)[4]) {
 template <int NT> constexpr int kSplitRing = NT == 3 ? 1 : 2;
 template <int L> using SplitWeights = v4i[kSplitRing<kCoutArr[L] / 32>][kCoutArr[L] / 32][3];
 
-template <int NT> __device__ __forceinline__ void split_preload(v4i (&ring)[kSplitRing<NT>][NT][3], const WFrags &wl) {
+template <int L> __device__ __forceinline__ void split_preload(SplitWeights<L> &ring, const WFrags &wl) {
+  constexpr int NT = kCoutArr[L] / 32;
 #pragma unroll
   for (int d = 0; d < kSplitRing<NT>; ++d)
 #pragma unroll
     for (int t = 0; t < NT; ++t)
 #pragma unroll
       for (int i = 0; i < 3; ++i) ring[d][t][i] = wl[(d * NT + t) * 3 + i];
+}
+
+// Weights of one fragment, from the packed set's parts (half_parts) to three bf16 ones.  A weight beyond fp16 is marked and
+// lies there as it is.
+// FIRST: of the first layer.
+template <bool FIRST> __device__ __forceinline__ void split_decode(v4i (&w)[3]) {
+  constexpr float kRest = FIRST ? 1.0f : 1.0f / kHalfLow;
+#pragma unroll
+  for (int d = 0; d < 4; ++d) {
+    float v[2];
+    const int w0 = w[0][d], w1 = w[1][d], w2 = w[2][d];
+    const f16x2 hi = __builtin_bit_cast(f16x2, w0), lo = __builtin_bit_cast(f16x2, w1), rest = __builtin_bit_cast(f16x2, w2);
+#pragma unroll
+    for (int e = 0; e < 2; ++e) {
+      v[e] = fmaf(fmaf((float)rest[e], kRest, (float)lo[e]), 1.0f / (kHalfW * kHalfLow), (float)hi[e] * (1.0f / kHalfW));
+      const unsigned raw = e ? ((unsigned)w1 >> 16) | ((unsigned)w2 & 0xffff0000u) : ((unsigned)w1 & 0xffffu) | ((unsigned)w2 << 16);
+      v[e] = ((w0 >> (16 * e)) & 0x7fff) == kHalfMark ? __builtin_bit_cast(float, raw) : v[e];
+    }
+#pragma unroll
+    for (int i = 0; i < 3; ++i) {
+      const unsigned short a = bf16_part(v[0]), b = bf16_part(v[1]);
+      v[0] = bf16_rest(v[0], a);
+      v[1] = bf16_rest(v[1], b);
+      w[i][d] = (int)((unsigned)a | (unsigned)b << 16);
+    }
+  }
+}
+
+// First layer: ROWS rows of K, three fragments of 8 columns each, rowb bytes apart in LDS; large products to acc, small ones
+// to low.  at[j]: where the lane's square of pixel tile j begins.
+template <int ROWS>
+__device__ __forceinline__ void split_first(const unsigned char *smem, const WFrags &wl, const int (&at)[3], int rowb,
+                                            f32x16 (&acc)[1][3], f32x16 (&low)[1][3]) {
+  v4i next[3][3];
+#pragma unroll
+  for (int i = 0; i < 9; ++i) next[i / 3][i % 3] = wl[i];
+#pragma unroll 1
+  for (int row = 0; row < ROWS; ++row) {
+#pragma unroll
+    for (int i = 0; i < 3; ++i) {
+      v4i w[3];
+#pragma unroll
+      for (int p = 0; p < 3; ++p) {
+        w[p] = next[i][p];
+        next[i][p] = wl[((row + 1) * 3 + i) * 3 + p];   // (behind the last row: what follows, unused)
+      }
+      split_decode<true>(w);
+#pragma unroll
+      for (int j = 0; j < 3; ++j) {
+        const v4i x = *reinterpret_cast<const v4i *>(smem + at[j] + row * rowb + i * 16);
+        mma<PrecBF16>(w[0], x, acc[0][j]);
+        mma<PrecBF16>(w[1], x, low[0][j]);
+        mma<PrecBF16>(w[2], x, low[0][j]);
+      }
+    }
+  }
 }
 
 // A product whose sum is in vector registers: the compiler puts every sum of the instruction in accumulation
@@ -203,6 +250,7 @@ __device__ __forceinline__ void split_conv(const unsigned char *smem, const WFra
         constexpr int g = decltype(gc)::value, t = g / (6 * N), m = (g % (6 * N)) / N, j = g % N;
         constexpr int WP[6] = {0, 1, 2, 0, 1, 0}, AP[6] = {2, 1, 0, 1, 0, 0};
         f32x16 &sum = m < 5 ? low[t][j] : acc[t][j];
+        if constexpr (g % (6 * N) == 0) split_decode<false>(ring[u % D][t]);
         if constexpr (t == 2 && j == 2) mma_vector(ring[u % D][t][WP[m]], bq[par][j][AP[m]], sum);
         else mma<PrecBF16>(ring[u % D][t][WP[m]], bq[par][j][AP[m]], sum);
         if constexpr (WIDE) {
@@ -331,37 +379,139 @@ __device__ __forceinline__ void split_store(unsigned char *smem, const int (&ci)
 
 // one 3x3 layer that is not the last
 template <int L>
-__device__ __forceinline__ void split_layer(unsigned char *smem, const unsigned char *packed, const float *tail,
-                                            SplitWeights<L> &ring, SplitWeights<L + 1> &next, const int (&ci)[3], int h,
-                                            int lane) {
+__device__ __forceinline__ void split_layer(unsigned char *smem, const unsigned char *packed, const float *tail, const int (&ci)[3],
+                                            int h, int lane) {
   constexpr int NT = kCoutArr[L] / 32;
+  const WFrags wl = layer_weights<PrecF32S, L>(packed, lane);
+  SplitWeights<L> ring;
+  split_preload<L>(ring, wl);
   f32x16 acc[NT][3], low[NT][3];
-  split_conv<L>(smem, layer_weights<PrecF32S, L>(packed, lane), tail + bias_offset(L), ring, ci, h, acc, low);
-  // (with equal widths the over-read has left the next layer's first k-steps in the ring)
-  if constexpr (kCoutArr[L + 1] != kCoutArr[L]) split_preload(next, layer_weights<PrecF32S, L + 1>(packed, lane));
+  split_conv<L>(smem, wl, tail + bias_offset(L), ring, ci, h, acc, low);
   __syncthreads();  // every wave has finished reading the layer's input
   split_store<NT, kCinArr[L + 1] != 96>(smem, ci, h, acc, low);
   __syncthreads();
 }
 
-// the value head's sum over (cout tile, tile of 32 squares)
-__device__ __forceinline__ float split_value_sum(const float *part) {
-  float s = 0.0f;
-  for (int i = 0; i < 36; ++i) s += part[i];
+// the value head's sum over (cout tile, tile of 32 squares).  (In 64 bits: 36 additions in fp32 were most of the value's error,
+// 2.5e-10 rms of values of 6e-4 with the reference's initialisation.)
+__device__ __forceinline__ double split_value_sum(const float *part) {
+  double s = 0.0;
+  for (int i = 0; i < 36; ++i) s += (double)part[i];
   return s;
 }
 
-// One workgroup (4 waves) per board, persistent over a contiguous run of boards, as
-// fused_forward_kernel.
-template <class P>
-__global__ __launch_bounds__(256) void split_forward_kernel(const FwdParams prm) {
+// ---- what c6_half.h shares ----
+// An input value, and whether a square counts as occupied (what the mask of the caller's choice says of it)
+__device__ __forceinline__ float board_input(const FwdParams &prm, long long b, int p, int ch) {
+  if (prm.x_dtype != C6_DT_BOARD_I8) return load_input(prm.x, prm.x_dtype, ((size_t)b * 3 + ch) * kPix + p);
+  long long src = prm.index ? prm.index[b] : b;
+  src = src < 0 ? 0 : (src >= prm.num_states ? prm.num_states - 1 : src);
+  if (ch == 2) return prm.stones_left[src] == 1 ? 1.0f : 0.0f;
+  const int stone = reinterpret_cast<const int8_t *>(prm.x)[(size_t)src * kPix + (prm.view ? d4_from_view(p, prm.view) : p)];
+  const int me = prm.player[src];
+  return stone == (ch == 0 ? me : -me) ? 1.0f : 0.0f;
+}
+__device__ __forceinline__ unsigned char board_taken(const FwdParams &prm, long long b, int p, float own, float other) {
+  if (prm.mask_mode == C6_MASK_LEGAL) return prm.legal[(size_t)b * kPix + p] == 0;
+  return prm.mask_mode == C6_MASK_INPUT && (own != 0.0f || other != 0.0f);
+}
+
+// Both heads over a wave's squares.  Partial sums per cout tile and tile of 32 squares, added up in a fixed order: what
+// the kernel that shares a board between workgroups can reproduce.
+struct SplitHeads {
+  int lane, wave, h;
+  float *red;
+  GlobalF32 pwg;   // the lane's channels of the policy weights: channel 32t + 8q + 4h + e
+  int pix[3];
+  bool valid[3];
+  float tot[3];
+  __device__ __forceinline__ SplitHeads(const float *tail, int tid, int lane_, int wave_, int h_, float *red_)
+      : lane(lane_), wave(wave_), h(h_), red(red_) {
+    const float *pwl = tail + kBiasTotal + 4 * h;
+    asm volatile("" : "+v"(pwl));
+    pwg = (GlobalF32)pwl;
+    int th = tid;
+    asm volatile("" : "+v"(th));
+#pragma unroll
+    for (int j = 0; j < 3; ++j) {
+      const int p = (th >> 6) * kPixPerWave + j * 32 + (th & 31);
+      valid[j] = p < kPix;
+      pix[j] = valid[j] ? p : kPix - 1;
+      tot[j] = 0.0f;
+    }
+  }
+  // cout tile t; values(j, e0, v): eight of the activations of the lane's square of pixel tile j, from register e0 on
+  template <class V> __device__ __forceinline__ void tile(int t, V values) {
+    float pol[3] = {0.0f, 0.0f, 0.0f}, val[3] = {0.0f, 0.0f, 0.0f};
+    f32x4 pw[4], vw[4];
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      pw[q] = *(GlobalF32x4)(pwg + 32 * t + 8 * q);
+      vw[q] = *(GlobalF32x4)(pwg + kHeadC + 32 * t + 8 * q);
+    }
+#pragma unroll
+    for (int j = 0; j < 3; ++j)
+#pragma unroll
+      for (int q = 0; q < 4; q += 2) {
+        float v[8];
+        values(j, 4 * q, v);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+          pol[j] = fmaf(v[e], pw[q + e / 4][e % 4], pol[j]);
+          val[j] = fmaf(v[e], vw[q + e / 4][e % 4], val[j]);
+        }
+      }
+#pragma unroll
+    for (int j = 0; j < 3; ++j) {
+      const unsigned bits = __builtin_bit_cast(unsigned, pol[j]);
+      const auto r = __builtin_amdgcn_permlane32_swap(bits, bits, false, false);  // the other lane half's channels
+      const unsigned r0 = r[0], r1 = r[1];
+      const float both = __builtin_bit_cast(float, r0) + __builtin_bit_cast(float, r1);
+      tot[j] = t == 0 ? both : tot[j] + both;
+      const float vs = wave_sum(valid[j] ? val[j] : 0.0f);
+      if (lane == 0) red[t * 12 + 3 * wave + j] = vs;
+    }
+  }
+  __device__ __forceinline__ void logits(float *lgt, float bias) const {
+#pragma unroll
+    for (int j = 0; j < 3; ++j)
+      if (h == 0 && valid[j]) lgt[pix[j]] = split_logit(tot[j], bias);
+  }
+};
+
+// ---- write out: value, masked logits, optional sampled action ----
+__device__ __forceinline__ void split_write(const FwdParams &prm, long long b, int tid, int lane, int wave, const unsigned char *occ,
+                                            const float *lgt, const float *red, float value_bias) {
+  if (tid == 0 && prm.value != nullptr) prm.value[b] = split_value(split_value_sum(red), value_bias);
+  if (prm.logits != nullptr) {
+    for (int p = tid; p < kPix; p += 256) static_cast<float *>(prm.logits)[(size_t)b * kPix + p] = occ[p] ? prm.fill : lgt[p];
+  }
+  if (prm.actions != nullptr && wave == 0) {
+    float it = prm.inv_temperature;
+    asm volatile("" : "+s"(it));
+    int a;
+    float lp;
+    int lane_here = lane;
+    asm volatile("" : "+v"(lane_here));
+    wave_sample(
+        lane_here, prm.u[b], it, [&](int i) { return lgt[i]; }, [&](int i) { return occ[i] == 0; }, a, lp);
+    if (lane == 0) {
+      prm.actions[b] = a;
+      if (prm.logprob != nullptr) prm.logprob[b] = lp;
+    }
+  }
+}
+
+// Board b, by one workgroup of four waves: logits, value and draw, whatever its numbers.
+__device__ __forceinline__ void split_board(const FwdParams &prm, unsigned char *smem, long long b) {
+  using P = PrecF32S;
   using G = Geo<P>;
   using S = SplitGeo;
-  extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
   constexpr int THREADS = 256, ROUNDS = (kPix + THREADS - 1) / THREADS;
-  const int tid = threadIdx.x;
+  int tid = threadIdx.x;
+  asm volatile("" : "+v"(tid));   // (nothing of this is formed, or kept, in front of it)
   const int lane = tid & 63;
-  const int wave = tid >> 6;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int h = lane >> 5;
   auto tile_pixel = [](int t, int j, bool &ok) __attribute__((always_inline)) {
     const int p = (t >> 6) * kPixPerWave + j * 32 + (t & 31);
@@ -379,309 +529,147 @@ __global__ __launch_bounds__(256) void split_forward_kernel(const FwdParams prm)
   float *lgt = reinterpret_cast<float *>(smem + S::LGT_OFF);
   float *red = reinterpret_cast<float *>(smem + S::RED_OFF);
   int *flags = reinterpret_cast<int *>(red) + 40;   // [0]: third plane varies, [1]: an input is not exact in bf16
+  const unsigned char *packed = prm.packed + (size_t)((unsigned)b / (unsigned)prm.boards_per_group) * prm.packed_stride;
+  const float *tail = reinterpret_cast<const float *>(packed + G::TAIL_OFF);
 
-  const unsigned per_group = (unsigned)prm.boards_per_group;
-  auto packed_of = [&](long long b) { return prm.packed + (size_t)((unsigned)b / per_group) * prm.packed_stride; };
-  float xin[ROUNDS][3];
-  unsigned char occin[ROUNDS];
-  auto fetch_board = [&](long long b) {
-    int tid = threadIdx.x;
-    asm volatile("" : "+v"(tid));
-    if (prm.x_dtype == C6_DT_BOARD_I8) {
-      long long src = prm.index ? prm.index[b] : b;
-      src = src < 0 ? 0 : (src >= prm.num_states ? prm.num_states - 1 : src);
-      const int8_t *board = reinterpret_cast<const int8_t *>(prm.x) + (size_t)src * kPix;
-      const int me = prm.player[src];
-      const float last = prm.stones_left[src] == 1 ? 1.0f : 0.0f;
+  float left[ROUNDS][3];   // the input; then what the parts staged so far leave of it
 #pragma unroll
-      for (int r = 0; r < ROUNDS; ++r) {
-        const int p = tid + r * THREADS;
-        if (p < kPix) {
-          const int stone = board[prm.view ? d4_from_view(p, prm.view) : p];
-          xin[r][0] = stone == me ? 1.0f : 0.0f;
-          xin[r][1] = stone == -me ? 1.0f : 0.0f;
-          xin[r][2] = last;
-          occin[r] = 0;
-        }
+  for (int r = 0; r < ROUNDS; ++r) {
+    const int p = tid + r * THREADS;
+    if (p < kPix)
+#pragma unroll
+      for (int ch = 0; ch < 3; ++ch) left[r][ch] = board_input(prm, b, p, ch);
+  }
+  __syncthreads();  // LDS is free
+  if (tid < 2) flags[tid] = 0;
+  if (tid == 0) red[42] = left[0][2];   // the third plane's value at square 0
+  for (int i = tid * 16; i < G::COPIES_BYTES; i += THREADS * 16) *reinterpret_cast<v4i *>(smem + i) = v4i{0, 0, 0, 0};
+  __syncthreads();
+  const float c2 = red[42];
+  bool varies = false;
+#pragma unroll
+  for (int r = 0; r < ROUNDS; ++r)
+    if (tid + r * THREADS < kPix) varies |= __builtin_bit_cast(int, left[r][2]) != __builtin_bit_cast(int, c2);
+  if (varies) flags[0] = 1;
+  __syncthreads();
+  const bool plane2_varies = flags[0] != 0;
+  const int planes_staged = plane2_varies ? 3 : 2;
+  // An input that is exact in bf16 (stones, flags) is one part; any other goes through the first
+  // layer's loop three times, once for each of its bf16 values.
+  bool inexact = false;
+#pragma unroll
+  for (int r = 0; r < ROUNDS; ++r)
+    if (tid + r * THREADS < kPix)
+#pragma unroll
+      for (int ch = 0; ch < 3; ++ch) inexact |= (__builtin_bit_cast(int, left[r][ch]) & 0xffff) != 0 && ch < planes_staged;
+  if (inexact) flags[1] = 1;
+  __syncthreads();
+  const int parts = flags[1] != 0 ? 3 : 1;
+  f32x16 a0[1][3], low[1][3], first[1][3];   // large products, small ones; the large ones, once all parts but the first follow
+  {
+    const WFrags tb = packed_frags<P>(packed, lane, G::PLANE2_FRAG_OFF + wave * 12);
+    f32x16 b0[1], bl[1];
+    load_bias_tiles(b0, tail + bias_offset(0), h);
+    load_bias_tiles(bl, tail + G::TAIL_BIAS_LOW + bias_offset(0), h);
+#pragma unroll
+    for (int j = 0; j < 3; ++j) {
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const f32x4 t4 = __builtin_bit_cast(f32x4, tb[j * 4 + q]);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) a0[0][j][4 * q + e] = plane2_varies ? b0[0][4 * q + e] : fmaf(c2, t4[e], b0[0][4 * q + e]);
       }
-      return;
+      low[0][j] = bl[0];
+#pragma unroll
+      for (int i = 0; i < 16; ++i) first[0][j][i] = 0.0f;
     }
+  }
+  int l1base[3];
+#pragma unroll
+  for (int j = 0; j < 3; ++j) {
+    bool ok;
+    const int pc = tile_pixel(tid, j, ok), r = pc / kBoard, c = pc - r * kBoard, s = c % G::E;
+    l1base[j] = s * G::COPY_BYTES + ((r * 3 + (plane2_varies ? kL1RowsHalf : 1) * h) * kL1RowPitch + (c - s)) * G::EB;
+  }
+#pragma unroll 1
+  for (int part = 0; part < parts; ++part) {
+    if (part > 0) __syncthreads();  // everybody has read the part before
 #pragma unroll
     for (int r = 0; r < ROUNDS; ++r) {
       const int p = tid + r * THREADS;
       if (p < kPix) {
+        const int row = p / kBoard, c = p - row * kBoard;
+        if (part == 0) occ[p] = board_taken(prm, b, p, left[r][0], left[r][1]);
 #pragma unroll
-        for (int ch = 0; ch < 3; ++ch) xin[r][ch] = load_input_raw(prm.x, prm.x_dtype, ((size_t)b * 3 + ch) * kPix + p);
-        occin[r] = prm.mask_mode == C6_MASK_LEGAL ? (prm.legal[(size_t)b * kPix + p] == 0) : 0;
+        for (int ch = 0; ch < 3; ++ch) {
+          if (ch >= planes_staged) break;
+          const unsigned short v16 = bf16_part(left[r][ch]);
+          left[r][ch] = bf16_rest(left[r][ch], v16);
+          const int hrow = (row + kK1 / 2) * 3 + ch;
+#pragma unroll
+          for (int s = 0; s < G::E; ++s)
+            *reinterpret_cast<unsigned short *>(smem + s * G::COPY_BYTES + (hrow * kL1RowPitch + (c + kK1 / 2 - s)) * G::EB) = v16;
+        }
       }
     }
-  };
-
-  // (board runs dealt out by XCD, as in fused_pipe_kernel)
-  const long long per = (prm.total_boards + gridDim.x - 1) / gridDim.x;
-  const unsigned xcds = (gridDim.x % 8 == 0) ? 8 : 1;
-  const long long run = (long long)(blockIdx.x % xcds) * (gridDim.x / xcds) + blockIdx.x / xcds;
-  long long b = run * per;
-  const long long b_end = b + per < prm.total_boards ? b + per : prm.total_boards;
-  if (b >= b_end) return;
-  v4i r1[L1Pipe<P>::D][1];
-  fetch_board(b);
-
-  for (; b < b_end; ++b) {
-    int tidv = tid;
-    asm volatile("" : "+v"(tidv));
-    const unsigned char *packed = packed_of(b);
-    const float *tail = reinterpret_cast<const float *>(packed + G::TAIL_OFF);
-    __syncthreads();  // previous board fully written out; LDS is free
-    preload_ring<L1Pipe<P>::D, 1>(r1, packed_frags<P>(packed, lane, G::FAST1_OFF));
-    // the third plane's share of the first layer, should the plane be constant (see fused_pipe_kernel)
-    f32x16 a0[1][3];
-    {
-      const WFrags tb = packed_frags<P>(packed, lane, G::PLANE2_FRAG_OFF + __builtin_amdgcn_readfirstlane(wave) * 12);
-#pragma unroll
-      for (int j = 0; j < 3; ++j)
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {
-          const f32x4 t4 = __builtin_bit_cast(f32x4, tb[j * 4 + q]);
-#pragma unroll
-          for (int e = 0; e < 4; ++e) a0[0][j][4 * q + e] = t4[e];
-        }
-      __builtin_amdgcn_sched_barrier(0);
-    }
-    // ---- stage the input: zero the shifted copies, then scatter the board ----
-    // (16-bit elements, and fp32 ones that count as rounded, become values here, when they have arrived)
-    if (prm.x_dtype != C6_DT_F32) {
-#pragma unroll
-      for (int r = 0; r < ROUNDS; ++r)
-#pragma unroll
-        for (int ch = 0; ch < 3; ++ch) xin[r][ch] = input_value(xin[r][ch], prm.x_dtype);
-    }
-    if (tid < 2) flags[tid] = 0;
-    if (tid == 0) red[42] = xin[0][2];   // the third plane's value at square 0
-    {
-      const v4i z = {0, 0, 0, 0};
-      for (int i = tidv * 16; i < G::COPIES_BYTES; i += THREADS * 16) *reinterpret_cast<v4i *>(smem + i) = z;
-    }
     __syncthreads();
-    const float c2 = red[42];
-    {
-      bool varies = false, inexact = false;
-#pragma unroll
-      for (int r = 0; r < ROUNDS; ++r)
-        if (tidv + r * THREADS < kPix) {
-          varies |= __builtin_bit_cast(int, xin[r][2]) != __builtin_bit_cast(int, c2);
-#pragma unroll
-          for (int ch = 0; ch < 3; ++ch)
-            inexact |= (__builtin_bit_cast(int, xin[r][ch]) & 0xffff) != 0 && (ch < 2 || varies);
-        }
-      if (varies) flags[0] = 1;
-      if (inexact) flags[1] = 1;
-    }
-    __syncthreads();
-    const bool plane2_varies = flags[0] != 0;
-    const int planes_staged = plane2_varies ? 3 : 2;
-    // An input that is exact in bf16 (stones, flags) is one part; any other goes through the first
-    // layer's loop three times, once for each of its bf16 values.
-    // (a third plane that varies on another thread's squares may be inexact here: look again)
-    bool again = false;
-    if (plane2_varies) {
-#pragma unroll
-      for (int r = 0; r < ROUNDS; ++r)
-        if (tidv + r * THREADS < kPix) again |= (__builtin_bit_cast(int, xin[r][2]) & 0xffff) != 0;
-      if (again) flags[1] = 1;
-      __syncthreads();
-    }
-    const int parts = flags[1] != 0 ? 3 : 1;
-    int l1base[3];
-#pragma unroll
-    for (int j = 0; j < 3; ++j) {
-      bool ok;
-      const int pc = tile_pixel(tidv, j, ok), r = pc / kBoard, c = pc - r * kBoard, s = c % G::E;
-      l1base[j] = s * G::COPY_BYTES + ((r * 3 + kL1RowsHalf * ((tidv >> 5) & 1)) * kL1RowPitch + (c - s)) * G::EB;
-    }
-    {
-      f32x16 b0[1];
-      load_bias_tiles(b0, tail + bias_offset(0), h);
-#pragma unroll
-      for (int j = 0; j < 3; ++j)
-#pragma unroll
-        for (int i = 0; i < 16; ++i) a0[0][j][i] = plane2_varies ? b0[0][i] : fmaf(c2, a0[0][j][i], b0[0][i]);
-    }
-    float left[ROUNDS][3];   // what the parts staged so far leave of the input
-#pragma unroll
-    for (int r = 0; r < ROUNDS; ++r)
-#pragma unroll
-      for (int ch = 0; ch < 3; ++ch) left[r][ch] = xin[r][ch];
-    SplitWeights<1> r2;
-    f32x16 low[1][3], first[1][3];   // small products; the large ones, once all parts but the first follow
-    {
-      f32x16 bl[1];
-      load_bias_tiles(bl, tail + G::TAIL_BIAS_LOW + bias_offset(0), h);
+    if (plane2_varies) split_first<kL1RowsHalf>(smem, layer_weights<P, 0>(packed, lane), l1base, kL1RowPitch * G::EB, a0, low);
+    else split_first<kK1>(smem, packed_frags<P>(packed, lane, G::FAST1_OFF), l1base, 3 * kL1RowPitch * G::EB, a0, low);
+    if (parts > 1 && part == 0) {
 #pragma unroll
       for (int j = 0; j < 3; ++j) {
-        low[0][j] = bl[0];
+        first[0][j] = a0[0][j];
+        a0[0][j] = low[0][j];
 #pragma unroll
-        for (int i = 0; i < 16; ++i) first[0][j][i] = 0.0f;
-      }
-    }
-#pragma unroll 1
-    for (int part = 0; part < parts; ++part) {
-      if (part > 0) __syncthreads();  // everybody has read the part before
-#pragma unroll
-      for (int r = 0; r < ROUNDS; ++r) {
-        const int p = tidv + r * THREADS;
-        if (p < kPix) {
-          const int row = p / kBoard, c = p - row * kBoard;
-          if (part == 0) {
-            unsigned char o = occin[r];
-            if (prm.mask_mode == C6_MASK_INPUT) o = (left[r][0] != 0.0f) || (left[r][1] != 0.0f);
-            occ[p] = o;
-          }
-#pragma unroll
-          for (int ch = 0; ch < 3; ++ch) {
-            if (ch >= planes_staged) break;
-            const unsigned short v16 = bf16_part(left[r][ch]);
-            left[r][ch] = bf16_rest(left[r][ch], v16);
-            const int hrow = (row + kK1 / 2) * 3 + ch;
-#pragma unroll
-            for (int s = 0; s < G::E; ++s) {
-              const int a = s * G::COPY_BYTES + (hrow * kL1RowPitch + (c + kK1 / 2 - s)) * G::EB;
-              *reinterpret_cast<unsigned short *>(smem + a) = v16;
-            }
-          }
-        }
-      }
-      __syncthreads();
-      if (!plane2_varies) {
-        int l1fast[3];
-#pragma unroll
-        for (int j = 0; j < 3; ++j) l1fast[j] = l1base[j] - (kL1RowsHalf - 1) * h * kL1RowPitch * G::EB;
-        const WFrags wf = packed_frags<P>(packed, lane, G::FAST1_OFF);
-        if (part > 0) preload_ring<L1Pipe<P>::D, 1>(r1, wf);
-        conv1_fast_pass<P>(smem, wf, r1, l1fast, a0, low);
-      } else {
-        preload_ring<L1Pipe<P>::D, 1>(r1, layer_weights<P, 0>(packed, lane));
-        conv1_pass<P>(smem, layer_weights<P, 0>(packed, lane), r1, l1base, a0, low);
-      }
-      if (parts > 1 && part == 0) {
-#pragma unroll
-        for (int j = 0; j < 3; ++j) {
-          first[0][j] = a0[0][j];
-          a0[0][j] = low[0][j];
-#pragma unroll
-          for (int i = 0; i < 16; ++i) low[0][j][i] = 0.0f;
-        }
-      }
-    }
-    if (parts > 1) {
-#pragma unroll
-      for (int j = 0; j < 3; ++j)
-#pragma unroll
-        for (int i = 0; i < 16; ++i) {
-          low[0][j][i] += a0[0][j][i];
-          a0[0][j][i] = first[0][j][i];
-        }
-    }
-    const long long bn = b + 1;
-    if (bn < b_end) fetch_board(bn);  // lands while this board is computed
-    split_preload(r2, layer_weights<P, 1>(packed, lane));
-    __syncthreads();
-    // the copies overlapped the activation tile: restore its zero padding
-    for (int i = tidv; i < 60 * (S::PIXB / 16); i += THREADS) {
-      const int k = i / (S::PIXB / 16), w16 = i - k * (S::PIXB / 16);
-      const int pos = k < 20 ? k : (k < 41 ? 400 + (k - 20) : (k - 40) * kPitch);
-      *reinterpret_cast<v4i *>(smem + pos * S::PIXB + w16 * 16) = v4i{0, 0, 0, 0};
-    }
-    split_store<1, true>(smem, ci, h, a0, low);
-    __syncthreads();
-
-    SplitWeights<2> r345;
-    SplitWeights<5> r678;
-    split_layer<1>(smem, packed, tail, r2, r345, ci, h, lane);
-    split_layer<2>(smem, packed, tail, r345, r345, ci, h, lane);
-    split_layer<3>(smem, packed, tail, r345, r345, ci, h, lane);
-    split_layer<4>(smem, packed, tail, r345, r678, ci, h, lane);
-    split_layer<5>(smem, packed, tail, r678, r678, ci, h, lane);
-    split_layer<6>(smem, packed, tail, r678, r678, ci, h, lane);
-
-    // ---- layer 8 + both 1x1 heads straight from the fp32 accumulators ----
-    {
-      f32x16 acc[3][3], low8[3][3];
-      split_conv<7>(smem, layer_weights<P, 7>(packed, lane), tail + bias_offset(7), r678, ci, h, acc, low8);
-      const float *valw = tail + kBiasTotal + kHeadC;
-      const float *pwl = tail + kBiasTotal + 4 * h;  // per-lane base: channel 32t + 8q + 4h + e
-      asm volatile("" : "+v"(pwl));
-      const GlobalF32 pwg = (GlobalF32)pwl;
-      int pix[3];
-      bool valid[3];
-      int th = tidv;
-      asm volatile("" : "+v"(th));
-#pragma unroll
-      for (int j = 0; j < 3; ++j) pix[j] = tile_pixel(th, j, valid[j]);
-      // Partial sums per cout tile and tile of 32 squares, added up in a fixed order: what
-      // the kernel that shares a board between workgroups can reproduce.
-      float tot[3];
-#pragma unroll
-      for (int t = 0; t < 3; ++t) {
-        float pol[3] = {0.0f, 0.0f, 0.0f}, val[3] = {0.0f, 0.0f, 0.0f};
-        f32x4 pw[4], vw[4];
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {
-          pw[q] = *(GlobalF32x4)(pwg + 32 * t + 8 * q);
-          vw[q] = *(GlobalF32x4)(pwg + kHeadC + 32 * t + 8 * q);
-        }
-#pragma unroll
-        for (int j = 0; j < 3; ++j) {
-          const f32x16 sum = split_total<3>(acc, low8, t, j);
-#pragma unroll
-          for (int q = 0; q < 4; q += 2) {
-            float v[8];
-            split_silu8(sum, 4 * q, v);
-#pragma unroll
-            for (int e = 0; e < 8; ++e) {
-              pol[j] = fmaf(v[e], pw[q + e / 4][e % 4], pol[j]);
-              val[j] = fmaf(v[e], vw[q + e / 4][e % 4], val[j]);
-            }
-          }
-        }
-#pragma unroll
-        for (int j = 0; j < 3; ++j) {
-          const unsigned bits = __builtin_bit_cast(unsigned, pol[j]);
-          const auto r = __builtin_amdgcn_permlane32_swap(bits, bits, false, false);  // the other lane half's channels
-          const unsigned r0 = r[0], r1 = r[1];
-          const float both = __builtin_bit_cast(float, r0) + __builtin_bit_cast(float, r1);
-          tot[j] = t == 0 ? both : tot[j] + both;
-          const float vs = wave_sum(valid[j] ? val[j] : 0.0f);
-          if (lane == 0) red[t * 12 + 3 * wave + j] = vs;
-        }
-      }
-      const float polb = valw[kHeadC], valb = valw[kHeadC + 1];
-#pragma unroll
-      for (int j = 0; j < 3; ++j)
-        if (h == 0 && valid[j]) lgt[pix[j]] = split_logit(tot[j], polb);
-      __syncthreads();
-      if (tid == 0 && prm.value != nullptr) prm.value[b] = split_value(split_value_sum(red), valb);
-    }
-    // ---- write out: masked logits, optional sampled action ----
-    if (prm.logits != nullptr) {
-      for (int p = tidv; p < kPix; p += THREADS)
-        static_cast<float *>(prm.logits)[(size_t)b * kPix + p] = occ[p] ? prm.fill : lgt[p];
-    }
-    if (prm.actions != nullptr && wave == 0) {
-      float it = prm.inv_temperature;
-      asm volatile("" : "+s"(it));
-      int a;
-      float lp;
-      int lane_here = lane;
-      asm volatile("" : "+v"(lane_here));
-      wave_sample(
-          lane_here, prm.u[b], it, [&](int i) { return lgt[i]; }, [&](int i) { return occ[i] == 0; }, a, lp);
-      if (lane == 0) {
-        prm.actions[b] = a;
-        if (prm.logprob != nullptr) prm.logprob[b] = lp;
+        for (int i = 0; i < 16; ++i) low[0][j][i] = 0.0f;
       }
     }
   }
+  if (parts > 1) {
+#pragma unroll
+    for (int j = 0; j < 3; ++j)
+#pragma unroll
+      for (int i = 0; i < 16; ++i) {
+        low[0][j][i] += a0[0][j][i];
+        a0[0][j][i] = first[0][j][i];
+      }
+  }
+  __syncthreads();
+  // the copies overlapped the activation tile: restore its zero padding
+  for (int i = tid; i < 60 * (S::PIXB / 16); i += THREADS) {
+    const int k = i / (S::PIXB / 16), w16 = i - k * (S::PIXB / 16);
+    const int pos = k < 20 ? k : (k < 41 ? 400 + (k - 20) : (k - 40) * kPitch);
+    *reinterpret_cast<v4i *>(smem + pos * S::PIXB + w16 * 16) = v4i{0, 0, 0, 0};
+  }
+  split_store<1, true>(smem, ci, h, a0, low);
+  __syncthreads();
+
+  split_layer<1>(smem, packed, tail, ci, h, lane);
+  split_layer<2>(smem, packed, tail, ci, h, lane);
+  split_layer<3>(smem, packed, tail, ci, h, lane);
+  split_layer<4>(smem, packed, tail, ci, h, lane);
+  split_layer<5>(smem, packed, tail, ci, h, lane);
+  split_layer<6>(smem, packed, tail, ci, h, lane);
+
+  // ---- layer 8 + both 1x1 heads straight from the fp32 accumulators ----
+  const float *valw = tail + kBiasTotal + kHeadC;
+  SplitHeads heads(tail, tid, lane, wave, h, red);
+  const WFrags wl = layer_weights<P, 7>(packed, lane);
+  SplitWeights<7> ring;
+  split_preload<7>(ring, wl);
+  f32x16 acc[3][3], low8[3][3];
+  split_conv<7>(smem, wl, tail + bias_offset(7), ring, ci, h, acc, low8);
+#pragma unroll
+  for (int t = 0; t < 3; ++t) {
+    f32x16 sum;
+    heads.tile(t, [&](int j, int e0, float (&v)[8]) __attribute__((always_inline)) {
+      if (e0 == 0) sum = split_total<3>(acc, low8, t, j);
+      split_silu8(sum, e0, v);
+    });
+  }
+  heads.logits(lgt, valw[kHeadC]);
+  __syncthreads();
+  split_write(prm, b, tid, lane, wave, occ, lgt, red, valw[kHeadC + 1]);
 }
 
 }  // namespace c6

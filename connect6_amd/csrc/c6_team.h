@@ -11,8 +11,8 @@
 //
 // What it takes (cycles of a 2.4 GHz clock; twelve workgroups, one board): staging the input 7 k, the first layer
 // 3 k (fp32 9 k), then per layer 1.2 k until the neighbours' flags are seen, 0.5 k until their squares are in LDS,
-// the MFMAs (bf16 0.5-2.1 k, fp32 4-12.5 k: one accumulator's chain, 40 cycles each) and 1.3 k until the outputs are
-// stored and acknowledged, at the end 6 k for the heads' sums: 66 k in bf16, 136 k in fp32.
+// the MFMAs (bf16 0.5-2.1 k, fp32 2-6 k: three per product) and 1.3 k until the outputs are
+// stored and acknowledged, at the end 6 k for the heads' sums: 66 k in bf16.
 //
 // The exchange: loads of activations and flags carry the device-scope cache policy (sc1).  So do stores until a
 // workgroup has seen that all of its team run on its own XCD (each leaves its XCD's number beside the flags): from
@@ -47,7 +47,8 @@ template <class P> constexpr bool has_team() { return P::ID != C6_PREC_F32; }
 template <class P> struct TeamGeo {
   using G = Geo<P>;
   static constexpr bool SPLIT = P::ID == C6_PREC_F32S;
-  static constexpr int NPL = SPLIT ? 3 : 1;                   // planes of an activation
+  static constexpr int NPL = SPLIT ? 2 : 1;                   // planes of an activation
+  static constexpr int WPL = SPLIT ? 2 : G::W;                // ... and of a 3x3 layer's weight that are contracted
   static constexpr int LO_OFF = NPL * 192;                    // fp6 blocks of a record (LO6)
   static constexpr int RECB = NPL * 192 + (P::LO6 ? 96 : 0) + 16;   // an odd number of 16-byte units
   // a square of c channels in memory: 16-byte units of its planes, then of its fp6 blocks
@@ -60,7 +61,8 @@ template <class P> struct TeamGeo {
   static constexpr int HEAD_OFF = act_off(7);                 // policy sums: SPLIT [3][384], else [384]
   // value sums: SPLIT one per (cout tile, tile of squares), else nine per lane of each tile of squares
   static constexpr int VAL_OFF = HEAD_OFF + 3 * 384 * 4;
-  static constexpr int BOARDB = (VAL_OFF + 12 * 9 * 64 * 4 + 255) & ~255;
+  static constexpr int NOTE_OFF = VAL_OFF + 12 * 9 * 64 * 4;   // SPLIT: a word per (layer, member, wave), half_note
+  static constexpr int BOARDB = (NOTE_OFF + (SPLIT ? 8 * 12 * 4 * 4 : 0) + 255) & ~255;
   // LDS: up to 11 rows of positions (128 squares lie in at most 8 board rows), 13 for 192 squares (SPLIT; in 11)
   static constexpr int REGION = ((SPLIT ? 13 : 11) * kPitch + 1) * RECB;
   // The first layer's shifted copies hold the halo rows that a workgroup's squares see: three per kernel row of up to
@@ -80,10 +82,9 @@ template <class P> struct TeamGeo {
 // tiles of squares each, whose four waves take PT of them and form CG groups of cout tiles.  A wave takes two
 // tiles of squares where there are two: with six workgroups each weight is then read by one wave, with three
 // by two; with one tile of squares per wave it would be twice as many, 96 and 128 bytes a cycle where the L1
-// gives 64 (six workgroups, 22 to 42 boards, bf16 + fp6 62.6 -> 55 us).  (fp32 contracts a weight with three parts, so
-// that a tile of squares per wave asks for just those 64, and all four waves have work in layers of two cout tiles.  Counted
-// over 53 boards, three workgroups each: of the 263 k cycles of a workgroup 150 k are reads from the L1, 64 bytes each, 128 k
-// MFMAs, so the L1 bounds the contractions by a sixth.)
+// gives 64 (six workgroups, 22 to 42 boards, bf16 + fp6 62.6 -> 55 us).  (fp32 takes one
+// tile of squares per wave: all four waves then have work in layers of two cout tiles.  Three workgroups per board ask for 85 bytes
+// a cycle in layers of three, where the L1 bounds the contractions.)
 // Three or six tiles of squares go to three waves, all cout tiles in each; the fourth watches the flags.
 template <class P, int TEAM> struct TeamShape {
   static constexpr int PXT = 12 / TEAM;
@@ -108,7 +109,14 @@ template <class P, int L> __device__ __forceinline__ int team_frag(int k, int t)
 // k-steps of weights that a wave keeps in flight: the loads take some 800 cycles and a k-step is
 // 32 cycles per MFMA
 template <class P, int TT, int PT> constexpr int team_ring() {
-  return Geo<P>::W == 3 ? (PT > 1 ? 3 : 6) / TT : (Geo<P>::W == 1 ? 18 / TT : (TT == 1 ? 9 : (TT == 2 ? 6 : 3)));
+  if (TeamGeo<P>::SPLIT) return PT > 1 ? 2 : (TT == 1 ? 9 : (TT == 2 ? 6 : 3));
+  return Geo<P>::W == 1 ? 18 / TT : (TT == 1 ? 9 : (TT == 2 ? 6 : 3));
+}
+// ... and those of one unrolled round: a phase in the pipelined modes; fp32: a kernel row, or all three of them where a k-step is
+// so short that nine are in flight
+template <class P, int L, int TT, int PT> constexpr int team_round() {
+  if (P::PIPE) return kPhaseSteps;
+  return (TT == 1 && PT == 1 ? 9 : 3) * kCinArr[L] / 16;
 }
 
 // Low-order (fp6) pass of layer L for PT tiles of squares, conv3_lo_pass with TT cout tiles from t0 on.
@@ -159,37 +167,41 @@ __device__ __forceinline__ void team_lo_pass(const unsigned char *smem, const un
 // The contraction of 3x3 layer L for PT tiles of 32 squares and TT cout tiles from t0 on (tiles beyond
 // the layer's last repeat it; their results are not used).
 //   rec: LDS addresses of the lane's squares' records;  acc: the bias on entry
-//   low (fp32): what the bias leaves out, for the small products' sum (split_conv)
+//   fp32 (as half_conv): the sums start at zero; acc: the rows' sums of the largest products, low: the others
 template <class P, int L, int TT, int PT>
 __device__ __forceinline__ void team_conv(const unsigned char *smem, const unsigned char *packed, const WFrags &wl,
-                                          v4i (&ring)[team_ring<P, TT, PT>()][TT][Geo<P>::W], int lane,
+                                          v4i (&ring)[team_ring<P, TT, PT>()][TT][TeamGeo<P>::WPL], int lane,
                                           const int (&rec)[PT], int t0, f32x16 (&acc)[PT][TT],
                                           f32x16 (&low)[PT][TT]) {
   using T = TeamGeo<P>;
   constexpr int NT = kCoutArr[L] / 32, NTP = kCinArr[L] / 32;
-  constexpr int W = Geo<P>::W, NPL = T::NPL, D = team_ring<P, TT, PT>();
+  constexpr int W = T::WPL, NPL = T::NPL, D = team_ring<P, TT, PT>();
   constexpr int KC = kCinArr[L] / 16, KS = 9 * KC;
-  constexpr int U = P::PIPE ? kPhaseSteps : 3 * KC;     // k-steps of one unrolled round
+  constexpr int U = team_round<P, L, TT, PT>();
   constexpr bool LO = P::LO6 && ((P::LO_MASK >> L) & 1);
   static_assert(KS % U == 0 && U % D == 0, "ring");
   int corner[PT];
 #pragma unroll
   for (int p = 0; p < PT; ++p) corner[p] = rec[p] - (kPitch + 1) * T::RECB + 16 * (lane >> 5);
   // k-step v of round r: (tap, 16 channels).  Pipelined modes: a round is a phase, all taps of 32
-  // channels; fp32: a round is a kernel row.
+  // channels; fp32: a round is a kernel row, or all three.
   auto frag = [&](int r, int v, int p, int pl) __attribute__((always_inline)) {
     const int tap = v / 2;
-    const int off = P::PIPE ? ((tap / 3) * kPitch + tap % 3) * T::RECB + (v % 2) * 32 : (v / KC) * T::RECB + (v % KC) * 32;
+    const int off = P::PIPE ? ((tap / 3) * kPitch + tap % 3) * T::RECB + (v % 2) * 32
+                            : ((v / KC / 3) * kPitch + v / KC % 3) * T::RECB + (v % KC) * 32;
     const int base = P::PIPE ? r * 64 : r * kPitch * T::RECB;
     return *reinterpret_cast<const v4i *>(smem + corner[p] + base + off + pl * 192);
   };
-  v4i a[3][PT][NPL];
+  // activations two k-steps ahead; one where that is eighteen MFMAs (and registers are short)
+  constexpr int AHEAD = T::SPLIT && PT > 1 ? 1 : 2;
+  v4i a[AHEAD + 1][PT][NPL];
 #pragma unroll
-  for (int v = 0; v < 2; ++v)
+  for (int v = 0; v < AHEAD; ++v)
 #pragma unroll
     for (int p = 0; p < PT; ++p)
 #pragma unroll
       for (int i = 0; i < NPL; ++i) a[v][p][i] = frag(0, v, p, i);
+  [[maybe_unused]] f32x16 sum[PT][TT];   // fp32: the largest products of a kernel row
   auto round = [&](int r) __attribute__((always_inline)) {
     // (the low-order pass comes in front of the last phase, as in pipe_layer)
     if constexpr (LO) {
@@ -197,40 +209,54 @@ __device__ __forceinline__ void team_conv(const unsigned char *smem, const unsig
     }
     static_for<0, U>([&](auto vc) __attribute__((always_inline)) {
       constexpr int v = decltype(vc)::value;
-      // activations two k-steps ahead (behind the last one: the last round again, unused)
-      const int rn = v + 2 < U ? r : (r + 1 < KS / U ? r + 1 : r);
+      // (behind the last k-step: the last round again, unused)
+      const int rn = v + AHEAD < U ? r : (r + 1 < KS / U ? r + 1 : r);
 #pragma unroll
       for (int p = 0; p < PT; ++p)
 #pragma unroll
-        for (int i = 0; i < NPL; ++i) a[(v + 2) % 3][p][i] = frag(rn, (v + 2) % U, p, i);
+        for (int i = 0; i < NPL; ++i) a[(v + AHEAD) % (AHEAD + 1)][p][i] = frag(rn, (v + AHEAD) % U, p, i);
       auto refill = [&](int t) __attribute__((always_inline)) {
         const int kn = r * U + v + D;   // (behind the last k-steps: the last one again, unused)
         const int f = team_frag<P, L>(kn < KS ? kn : KS - 1, t0 + t < NT ? t0 + t : NT - 1);
 #pragma unroll
         for (int i = 0; i < W; ++i) ring[v % D][t][i] = wl[f + i];
       };
-      if constexpr (NPL == 3) {
-        // (An accumulator's next MFMA is eight cycles late if it follows at once, so two tiles take turns: forty boards
-        // 102 -> 97 us.  With three the L1's 64 bytes a cycle bound the layer, and loads in a row per tile suit it better:
-        // 56 boards 120 us, in turns 123.)
-        constexpr int WP[6] = {0, 1, 2, 0, 1, 0}, AP[6] = {2, 1, 0, 1, 0, 0};
+      if constexpr (T::SPLIT) {
+        // lo hi, hi hi, hi lo (weight, activation).  (An accumulator's next MFMA is eight cycles late if it follows at once: the
+        // two sums take turns, and so do two tiles.  With three the L1's 64 bytes a cycle bound the layer, and loads in a row per
+        // tile suit it better.)
+        constexpr int WP[3] = {1, 0, 0}, AP[3] = {0, 0, 1};
         constexpr bool TURNS = TT == 2;
+        if constexpr (v % (3 * KC) == 0) {
 #pragma unroll
-        for (int o = 0; o < (TURNS ? 6 : TT); ++o)
+          for (int p = 0; p < PT; ++p)
 #pragma unroll
-          for (int n = 0; n < (TURNS ? TT : 6); ++n) {
+            for (int t = 0; t < TT; ++t) sum[p][t] = f32x16{};
+        }
+#pragma unroll
+        for (int o = 0; o < (TURNS ? 3 : TT); ++o)
+#pragma unroll
+          for (int n = 0; n < (TURNS ? TT : 3); ++n) {
             const int m = TURNS ? o : n, t = TURNS ? n : o;
 #pragma unroll
-            for (int p = 0; p < PT; ++p) mma<P>(ring[v % D][t][WP[m]], a[v % 3][p][AP[m]], m < 5 ? low[p][t] : acc[p][t]);
-            if (m == 5) refill(t);
+            for (int p = 0; p < PT; ++p) mma<P>(ring[v % D][t][WP[m]], a[v % (AHEAD + 1)][p][AP[m]], m == 1 ? sum[p][t] : low[p][t]);
+            if (m == 2) refill(t);
           }
+        if constexpr ((v + 1) % (3 * KC) == 0) {
+#pragma unroll
+          for (int p = 0; p < PT; ++p)
+#pragma unroll
+            for (int t = 0; t < TT; ++t)
+#pragma unroll
+              for (int e = 0; e < 16; ++e) acc[p][t][e] = fmaf(sum[p][t][e], kHalfUnit, acc[p][t][e]);
+        }
       } else {
 #pragma unroll
         for (int t = 0; t < TT; ++t) {
 #pragma unroll
           for (int i = 0; i < W; ++i)
 #pragma unroll
-            for (int p = 0; p < PT; ++p) mma<P>(ring[v % D][t][i], a[v % 3][p][0], acc[p][t]);
+            for (int p = 0; p < PT; ++p) mma<P>(ring[v % D][t][i], a[v % (AHEAD + 1)][p][0], acc[p][t]);
           refill(t);
         }
       }
@@ -244,63 +270,49 @@ __device__ __forceinline__ void team_conv(const unsigned char *smem, const unsig
 #pragma unroll 1
     for (int r = 0; r < KS / U; ++r) round(r);
   }
-  if constexpr (NPL == 3) {
+  if constexpr (T::SPLIT) {   // (or its products are put off until the sum is used, and their operands kept for that)
 #pragma unroll
     for (int p = 0; p < PT; ++p)
 #pragma unroll
-      for (int t = 0; t < TT; ++t)
-#pragma unroll
-        for (int e = 0; e < 16; ++e) acc[p][t][e] = two_sums(acc[p][t][e], low[p][t][e]);
+      for (int t = 0; t < TT; ++t) asm volatile("" : "+a"(low[p][t]));
   }
 }
 
 // SiLU of one accumulator tile, step by step: a lone wave waits for each result that its next instruction needs.  Against
 // output by output it is worth a per cent, one way or the other: 22 to 40 boards in bf16 and fp16 40.0 -> 39.6 us, 40 boards that
-// a cascade lists 117.2 -> 116.2, 86 to 128 fp32 boards 217.2 -> 215.5; but 1 to 16 boards in bf16 30.2 -> 30.6; one and 53 fp32
-// boards, and the teams beside whole rounds, the same.
+// a cascade lists 117.2 -> 116.2, but 1 to 16 boards in bf16 30.2 -> 30.6; the
+// teams beside whole rounds the same.  (fp32: half_silu8.)
 template <class P> __device__ __forceinline__ void silu_tile(const f32x16 &acc, float (&v)[16]) {
-  if constexpr (TeamGeo<P>::SPLIT) {
-    float half[8];
+  __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-    for (int e0 = 0; e0 < 16; e0 += 8) {
-      split_silu8(acc, e0, half);
+  for (int e = 0; e < 16; ++e) v[e] = __builtin_amdgcn_exp2f(acc[e]);
+  __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-      for (int e = 0; e < 8; ++e) v[e0 + e] = half[e];
-    }
-  } else {
-    __builtin_amdgcn_sched_barrier(0);
+  for (int e = 0; e < 16; ++e) v[e] = 1.0f + v[e];
+  __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-    for (int e = 0; e < 16; ++e) v[e] = __builtin_amdgcn_exp2f(acc[e]);
-    __builtin_amdgcn_sched_barrier(0);
+  for (int e = 0; e < 16; ++e) v[e] = __builtin_amdgcn_rcpf(v[e]);
+  __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-    for (int e = 0; e < 16; ++e) v[e] = 1.0f + v[e];
-    __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-    for (int e = 0; e < 16; ++e) v[e] = __builtin_amdgcn_rcpf(v[e]);
-    __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-    for (int e = 0; e < 16; ++e) v[e] = acc[e] * v[e];
-    __builtin_amdgcn_sched_barrier(0);
-  }
+  for (int e = 0; e < 16; ++e) v[e] = acc[e] * v[e];
+  __builtin_amdgcn_sched_barrier(0);
 }
 
 // SiLU of one accumulator tile into the record at `rec` (cout tile t): planes, and the fp6 block.
-// UNDER: the one-workgroup kernel takes this tile's low-order parts behind MFMAs (see epi_atom).
+// UNDER: the one-workgroup kernel takes this tile's low-order parts behind MFMAs (see epi_atom).  most (fp32): the largest so far.
 template <class P, bool LO, bool UNDER>
-__device__ __forceinline__ void team_store(unsigned char *smem, int rec, int h, int t, const f32x16 &acc) {
+__device__ __forceinline__ void team_store(unsigned char *smem, int rec, int h, int t, const f32x16 &acc, float &most) {
   using T = TeamGeo<P>;
   unsigned char *at = smem + rec + 64 * t + 8 * h;
   if constexpr (T::SPLIT) {
+    const HalfTile v = half_tile([&](int e0, float (&u)[8]) __attribute__((always_inline)) {
 #pragma unroll
-    for (int q = 0; q < 4; q += 2) {
-      float v[8];
-      int w[3][4];
-      split_silu8(acc, 4 * q, v);
-      split_planes8(v, w);
+      for (int i = 0; i < 8; ++i) u[i] = acc[e0 + i];
+    }, most);
 #pragma unroll
-      for (int i = 0; i < 3; ++i)
-#pragma unroll
-        for (int e = 0; e < 2; ++e) *reinterpret_cast<v2i *>(at + i * 192 + 16 * (q + e)) = v2i{w[i][2 * e], w[i][2 * e + 1]};
+    for (int q = 0; q < 4; ++q) {
+      *reinterpret_cast<v2i *>(at + 16 * q) = v2i{v.hi[2 * q], v.hi[2 * q + 1]};
+      *reinterpret_cast<v2i *>(at + 192 + 16 * q) = v2i{v.lo[2 * q], v.lo[2 * q + 1]};
     }
   } else {
     const DropConsts k = drop_consts<P>();
@@ -359,8 +371,9 @@ __device__ __forceinline__ void team_board(const TeamParams &prm, unsigned char 
   using G = Geo<P>;
   using T = TeamGeo<P>;
   using S = TeamShape<P, TEAM>;
-  constexpr int NPL = T::NPL, W = G::W, THREADS = 256, PXT = S::PXT, PT = S::PT, CG = S::CG;
-  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), h = lane >> 5;
+  constexpr int NPL = T::NPL, W = G::W, WPL = T::WPL, THREADS = 256, PXT = S::PXT, PT = S::PT, CG = S::CG;
+  std::conditional_t<T::SPLIT, int, const int> tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), h = lane >> 5;
   const FwdParams &f = prm.f;
   unsigned char *occ = smem + T::OCC_OFF;
   float *lgt = reinterpret_cast<float *>(smem + T::LGT_OFF);
@@ -400,6 +413,12 @@ __device__ __forceinline__ void team_board(const TeamParams &prm, unsigned char 
     else __hip_atomic_store(&flags[word], prm.tag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   };
   [[maybe_unused]] const bool trace_on = true;
+  // fp32: what this wave stored of layer l of role's squares (nothing: 0), for the last stage
+  bool bad_input = false;
+  auto store_note = [&](int l, int role, float most, bool bad) __attribute__((always_inline)) {
+    const unsigned note = half_note(l, most) | (bad ? 1u : 0u);
+    if (lane == 0) store4(__builtin_bit_cast(float, note), T::NOTE_OFF + ((l * 12 + role) * 4 + wave) * 4);
+  };
 
   // the wave's first tile of squares within the workgroup's, and its group of cout tiles
   const int wpx = wave % S::PG * PT, cg = wave / S::PG;
@@ -492,6 +511,7 @@ __device__ __forceinline__ void team_board(const TeamParams &prm, unsigned char 
     constexpr int L = decltype(lc)::value, N = decltype(nc)::value, C = kCoutArr[L], NT = C / 32;
     constexpr int TT = S::tiles(NT);
     constexpr bool LO = P::LO6 && ((P::LO_MASK >> (L + 1)) & 1);
+    float most = 0.0f;
     if (active) {
 #pragma unroll
       for (int i = 0; i < N; ++i) {
@@ -499,9 +519,10 @@ __device__ __forceinline__ void team_board(const TeamParams &prm, unsigned char 
         const int rec = record(pc, sp.base);
 #pragma unroll
         for (int t = 0; t < TT; ++t)
-          if (t0 + t < NT) team_store<P, LO, (L >= 2)>(smem, rec, h, t0 + t, acc[i][t]);
+          if (t0 + t < NT) team_store<P, LO, (L >= 2)>(smem, rec, h, t0 + t, acc[i][t], most);
       }
     }
+    if constexpr (T::SPLIT) store_note(L, role, most, L == 0 && bad_input);
     __syncthreads();
     int sq, j;
     unit_of(IC<C>{}, sq, j);
@@ -541,7 +562,7 @@ __device__ __forceinline__ void team_board(const TeamParams &prm, unsigned char 
     const WFrags wl = layer_weights<P, L>(packed, lane);
     C6_MARK(6 * L);
     const bool own = region_role == role && region_layer == L - 1;
-    v4i ring[D][TT][W];
+    v4i ring[D][TT][WPL];
     f32x16 acc[PT][TT], low[PT][TT];
     auto first_weights = [&]() __attribute__((always_inline)) {
 #pragma unroll
@@ -549,7 +570,7 @@ __device__ __forceinline__ void team_board(const TeamParams &prm, unsigned char 
 #pragma unroll
         for (int t = 0; t < TT; ++t)
 #pragma unroll
-          for (int i = 0; i < W; ++i) ring[d][t][i] = wl[team_frag<P, L>(d, t0 + t < NT ? t0 + t : NT - 1) + i];
+          for (int i = 0; i < WPL; ++i) ring[d][t][i] = wl[team_frag<P, L>(d, t0 + t < NT ? t0 + t : NT - 1) + i];
       __builtin_amdgcn_sched_barrier(0);
     };
     // (on their way while the neighbours are waited for; the wave that does the waiting asks for its own behind that)
@@ -595,8 +616,8 @@ __device__ __forceinline__ void team_board(const TeamParams &prm, unsigned char 
         const int word = bias_offset(L) + 32 * (t0 + t < NT ? t0 + t : NT - 1);
 #pragma unroll
         for (int i = 0; i < PT; ++i) {
-          acc[i][t] = tail_tile(word);
-          if constexpr (T::SPLIT) low[i][t] = tail_tile(G::TAIL_BIAS_LOW + word);
+          if constexpr (T::SPLIT) acc[i][t] = low[i][t] = f32x16{};
+          else acc[i][t] = tail_tile(word);
         }
       }
     }
@@ -612,6 +633,20 @@ __device__ __forceinline__ void team_board(const TeamParams &prm, unsigned char 
       rec[i] = record(ok[i] ? p[i] : kPix - 1, sp.base);
     }
     if (active) team_conv<P, L, TT, PT>(smem, packed, wl, ring, lane, rec, t0, acc, low);
+    if constexpr (T::SPLIT) {
+      if (active) {   // (as half_total8)
+#pragma unroll
+        for (int t = 0; t < TT; ++t) {
+          const int word = bias_offset(L) + 32 * (t0 + t < NT ? t0 + t : NT - 1);
+          const f32x16 bias = tail_tile(word) * kHalfA, rest = tail_tile(G::TAIL_BIAS_LOW + word) * kHalfA;
+#pragma unroll
+          for (int i = 0; i < PT; ++i)
+#pragma unroll
+            for (int e = 0; e < 16; ++e)
+              acc[i][t][e] = fmaf(low[i][t][e], kHalfUnit / kHalfLow, rest[e]) + (acc[i][t][e] + bias[e]);
+        }
+      }
+    }
     C6_MARK(6 * L + 3);
     if constexpr (L < 7) {
       __syncthreads();   // everybody has read this layer's input
@@ -621,6 +656,7 @@ __device__ __forceinline__ void team_board(const TeamParams &prm, unsigned char 
       const float *pw = tail + kBiasTotal + 4 * h;
       const int tile = role * PXT + wpx;   // of the twelve
       if constexpr (T::SPLIT) {
+        float most = 0.0f;
         if (active) {
 #pragma unroll
           for (int t = 0; t < TT; ++t) {
@@ -630,7 +666,16 @@ __device__ __forceinline__ void team_board(const TeamParams &prm, unsigned char 
             for (int i = 0; i < PT; ++i) pol[i] = val[i] = 0.0f;
             float a[PT][16];
 #pragma unroll
-            for (int i = 0; i < PT; ++i) silu_tile<P>(acc[i][t], a[i]);
+            for (int i = 0; i < PT; ++i)
+#pragma unroll
+              for (int e0 = 0; e0 < 16; e0 += 8) {
+                float u[8], v[8];
+#pragma unroll
+                for (int e = 0; e < 8; ++e) u[e] = acc[i][t][e0 + e];
+                half_last8(u, v, most);
+#pragma unroll
+                for (int e = 0; e < 8; ++e) a[i][e0 + e] = v[e];
+              }
 #pragma unroll
             for (int q = 0; q < 4; ++q)
 #pragma unroll
@@ -654,6 +699,7 @@ __device__ __forceinline__ void team_board(const TeamParams &prm, unsigned char 
             }
           }
         }
+        store_note(L, role, most, false);
       } else {
         // The one-workgroup kernel runs one chain of multiply-adds over the channels of a lane's
         // square, cout tile after cout tile: the groups of cout tiles take turns and hand it on.
@@ -728,7 +774,7 @@ __device__ __forceinline__ void team_board(const TeamParams &prm, unsigned char 
   // first layer: every workgroup stages the part of the board that its squares see
   auto first_stage = [&](int role) __attribute__((always_inline)) -> bool {
     const Span sp = span_of(role);
-    int *flag = reinterpret_cast<int *>(red) + 64;   // [0]: third plane varies, [1]: an input is not exact in bf16
+    int *flag = reinterpret_cast<int *>(red) + 64;   // [0]: third plane varies, fp32: [1]: an input is not exact, [3] beyond the range, [4] not small
     constexpr int N1 = PXT > 4 ? 2 : 1;   // (one cout tile: a wave per tile of squares, or per two)
     const int px = wave * N1 < PXT ? wave * N1 : 0;
     const bool active = wave * N1 < PXT;
@@ -786,7 +832,7 @@ __device__ __forceinline__ void team_board(const TeamParams &prm, unsigned char 
 #pragma unroll
     for (int i = 0; i < TAIL_UNITS; ++i)
       if (tid + i * THREADS < G::TAIL_FLOATS / 4) reinterpret_cast<v4i *>(smem + T::TAIL_OFF)[tid + i * THREADS] = tl[i];
-    if (tid < 2) flag[tid] = 0;
+    if (tid < 5 && tid != 2) flag[tid] = 0;
     if (tid == 0) red[66] = xin[0][2];
     __syncthreads();
     const float c2 = red[66];
@@ -803,16 +849,23 @@ __device__ __forceinline__ void team_board(const TeamParams &prm, unsigned char 
     const bool plane2_varies = flag[0] != 0;
     int parts = 1;
     if constexpr (T::SPLIT) {
-      bool inexact = false;
+      bool inexact = false, beyond = false, ordinary = false;   // (as half_forward_kernel)
 #pragma unroll
       for (int k = 0; k < 2; ++k)
         if (tid + k * THREADS < kPix)
 #pragma unroll
-          for (int ch = 0; ch < 3; ++ch)
-            inexact |= (ch < 2 || plane2_varies) && (__builtin_bit_cast(int, xin[k][ch]) & 0xffff) != 0;
+          for (int ch = 0; ch < 3; ++ch) {
+            if (ch == 2 && !plane2_varies) continue;
+            inexact |= xin[k][ch] - half_value(half_bits(xin[k][ch])) != 0.0f;
+            beyond |= !half_fits(xin[k][ch]);
+            ordinary |= __builtin_fabsf(xin[k][ch]) >= kHalfLeast;
+          }
       if (inexact) flag[1] = 1;
+      if (beyond) flag[3] = 1;
+      if (ordinary) flag[4] = 1;
       __syncthreads();
-      parts = flag[1] != 0 ? 3 : 1;
+      parts = flag[1] != 0 ? 2 : 1;
+      bad_input = parts > 1 && (flag[3] != 0 || flag[4] == 0);
     }
     const int rows = (plane2_varies ? G::STEPS1 : G::FAST1_STEPS) / 3;
     int row0[N1];
@@ -829,17 +882,13 @@ __device__ __forceinline__ void team_board(const TeamParams &prm, unsigned char 
 #pragma unroll
       for (int n = 0; n < N1; ++n)
 #pragma unroll
-        for (int i = 0; i < 16; ++i) acc[n][0][i] = plane2_varies ? b0[i] : fmaf(c2, acc[n][0][i], b0[i]);
+        for (int i = 0; i < 16; ++i) acc[n][0][i] = (T::SPLIT ? kHalfA : 1.0f) * (plane2_varies ? b0[i] : fmaf(c2, acc[n][0][i], b0[i]));
     }
-    f32x16 low[N1], large[N1];   // SPLIT: small products; the large ones, once all parts but the first follow
-#pragma unroll
-    for (int n = 0; n < N1; ++n)
-#pragma unroll
-      for (int i = 0; i < 16; ++i) low[n][i] = large[n][i] = 0.0f;
+    f32x16 low[N1], large[N1];   // SPLIT: small products; the large ones, once a second part follows
     if constexpr (T::SPLIT) {
       if (active) {
 #pragma unroll
-        for (int n = 0; n < N1; ++n) low[n] = tail_tile(G::TAIL_BIAS_LOW + bias_offset(0));
+        for (int n = 0; n < N1; ++n) low[n] = tail_tile(G::TAIL_BIAS_LOW + bias_offset(0)) * (kHalfA * kHalfLow);
       }
     }
 #pragma unroll 1
@@ -856,8 +905,8 @@ __device__ __forceinline__ void team_board(const TeamParams &prm, unsigned char 
           if (sq >= kPix) continue;
           unsigned short v16;
           if constexpr (T::SPLIT) {
-            v16 = bf16_part(xin[k][ch]);
-            xin[k][ch] = bf16_rest(xin[k][ch], v16);
+            v16 = half_bits(xin[k][ch]);
+            xin[k][ch] = (xin[k][ch] - half_value(v16)) * kHalfLow;
           } else {
             v16 = bits16<P>(xin[k][ch]);
           }
@@ -920,14 +969,19 @@ __device__ __forceinline__ void team_board(const TeamParams &prm, unsigned char 
           if (row + decltype(sc)::value < rows) one_row(row + decltype(sc)::value, sc);
         });
         if constexpr (T::SPLIT) {
-          if (parts > 1 && part == 0) {
+          if (parts > 1) {   // (the second part's products with the weights' first are small ones, the others are dropped)
 #pragma unroll
-            for (int n = 0; n < N1; ++n) {
-              large[n] = acc[n][0];
-              acc[n][0] = low[n];
+            for (int n = 0; n < N1; ++n)
 #pragma unroll
-              for (int i = 0; i < 16; ++i) low[n][i] = 0.0f;
-            }
+              for (int i = 0; i < 16; ++i) {
+                if (part == 0) {
+                  large[n][i] = acc[n][0][i];
+                  acc[n][0][i] = low[n][i];
+                } else {
+                  low[n][i] = acc[n][0][i];
+                  acc[n][0][i] = large[n][i];
+                }
+              }
           }
         }
       }
@@ -936,8 +990,7 @@ __device__ __forceinline__ void team_board(const TeamParams &prm, unsigned char 
 #pragma unroll
       for (int n = 0; n < N1; ++n)
 #pragma unroll
-        for (int i = 0; i < 16; ++i)
-          acc[n][0][i] = parts > 1 ? two_sums(large[n][i], low[n][i] + acc[n][0][i]) : two_sums(acc[n][0][i], low[n][i]);
+        for (int i = 0; i < 16; ++i) acc[n][0][i] = fmaf(low[n][i], 1.0f / kHalfLow, acc[n][0][i]);
     }
     C6_MARK(2);
     __syncthreads();   // the copies give way to the activations
@@ -949,9 +1002,21 @@ __device__ __forceinline__ void team_board(const TeamParams &prm, unsigned char 
 
   // the heads' sums into logits, value, draw and (cascade) the list of close boards: one workgroup
   auto last_stage = [&](int role) __attribute__((always_inline)) -> bool {
+    [[maybe_unused]] unsigned *check = reinterpret_cast<unsigned *>(red) + 128;
+    if constexpr (T::SPLIT) {
+      if (tid == 0) *check = 0;
+    }
     const int got = wait_inputs(8, role, true);
     if (got != 1) return got == 2;
     region_role = -1;
+    if constexpr (T::SPLIT) {
+      unsigned note = 0;
+      for (int i = tid; i < 8 * TEAM * 4; i += THREADS) {
+        const int l = i / (TEAM * 4), j = i - l * (TEAM * 4);
+        note |= (unsigned)__builtin_amdgcn_raw_buffer_load_b32(mem, T::NOTE_OFF + (l * 48 + j) * 4, 0, kSc1);
+      }
+      if (note != 0) atomicOr(check, note);
+    }
     const float *valw = tail + kBiasTotal + kHeadC;
     const float polb = valw[kHeadC], valb = valw[kHeadC + 1];
     auto partial = [&](int at) __attribute__((always_inline)) {
@@ -1026,6 +1091,14 @@ __device__ __forceinline__ void team_board(const TeamParams &prm, unsigned char 
         if (f.logprob != nullptr) f.logprob[b] = lp;
       }
     }
+    if constexpr (T::SPLIT) {   // (behind the stores of the outputs that it goes into)
+      const bool failed = half_failed(__builtin_amdgcn_readfirstlane(*check));
+      if (failed) {
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        __syncthreads();
+        if (tid == 0) half_leave(f, b);
+      }
+    }
     if constexpr (P::ID == C6_PREC_BF16) {
       if (f.redo_mode == kRedoDetect && wave == 1) {   // (a run of one board: see fused_pipe_kernel)
         const bool again = wave_margin_below(
@@ -1067,6 +1140,10 @@ __device__ __forceinline__ void team_board(const TeamParams &prm, unsigned char 
       __syncthreads();
     }
     bool ok = false;
+    if constexpr (T::SPLIT) {   // (opaque: what follows from them is formed in each stage, and not kept for all of them)
+      asm volatile("" : "+v"(tid));
+      lane = tid & 63;
+    }
     switch (stage) {
       case 0: ok = first_stage(role); break;
       case 1: ok = conv_stage(IC<1>{}, role); break;

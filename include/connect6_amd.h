@@ -47,14 +47,16 @@ extern "C" {
                             weights to bf16 dropped (a second bf16 weight fragment per fragment,
                             twice the bf16 matrix work): within 3e-4 relative L2 of fp32 */
 
-#define C6_PREC_F32S 7   /* fp32 operands, each the exact sum of three bf16 values: six bf16 MFMAs per
-                            product, fp32 accumulate.  fp32 results, no further from a 64-bit
-                            forward than those of C6_PREC_F32 (the products left out are below
-                            2^-25), at half the time; its packed weights take three halves of that
-                            mode's.  Infinities and NaN as in fp32, except that a sum or an
+#define C6_PREC_F32S 7   /* fp32 operands, each as two fp16 values of 11 mantissa bits: three fp16 MFMAs
+                            per product, fp32 accumulate.  fp32 results, less than half as far from a
+                            64-bit forward as those of C6_PREC_F32, at a third of the time; its packed
+                            weights take three halves of that mode's.  A board that has numbers beyond
+                            what fp16 holds so (weights up to 2048 and from 2e-10 on, activations up to
+                            1400 and not all below 5e-6) is computed with three bf16 values per operand and six MFMAs
+                            per product.  Infinities and NaN as in fp32, except that a sum or an
                             activation beyond 2.3e38 (fp32: 3.4e38) counts as infinite.  In an
                             architecture that c6_generic_packed_bytes is not 0 for, C6_PREC_F32
-                            too is computed so, with sums and activations up to 3.38e38 */
+                            too is computed with three bf16 values, with sums and activations up to 3.38e38 */
 
 /* element types of caller tensors */
 #define C6_DT_F32 0
@@ -191,7 +193,7 @@ int c6_forward_boards_cascade(const int8_t *boards, const int8_t *player,
  * most of the chip idle, all the time or in their last round; the same results, bit for bit.
  * c6_team_bytes gives the sizes of the two buffers, or 0 and 0 where one workgroup per board is the
  * better launch (or the mode has no such kernel): call c6_forward there.
- *   workspace  device, 16-byte aligned; contents need no preparation.  Per shared board 1.0 MB
+ *   workspace  device, 16-byte aligned; contents need no preparation.  Per shared board 0.7 MB
  *              (C6_PREC_F32S), 0.5 MB (C6_PREC_BF16F6, _BF16F6W and the cascades), 0.35 MB (C6_PREC_BF16,
  *              _F16); of 256 CUs at most 128, 42 or 73, and 80 boards are shared.  A cascade over at most 21
  *              boards is one launch and takes both its passes' share

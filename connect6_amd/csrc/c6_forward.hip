@@ -2149,7 +2149,7 @@ template <class P> __global__ __launch_bounds__(256) void pack_kernel(const Pack
   if (ti >= G::TAIL_BIAS_LOW && ti < G::TAIL_FLOATS) {
     const Scaled<P> b = conv_bias(ti - G::TAIL_BIAS_LOW);
     const float low = (float)(b - (float)b);
-    tail[ti] = low == low ? low : 0.0f;   // (an infinite bias leaves nothing)
+    tail[ti] = low == low ? low / kTailLow : 0.0f;   // (an infinite bias leaves nothing)
   }
   if (ti < G::TAIL_SW) {  // the sw[] words behind it are written by lo_scale_kernel
     constexpr float head_scale = P::WLO == 2 ? 1.0f : act_scale<P>();

@@ -29,10 +29,12 @@
 // that has an infinity or a NaN anywhere, is seen at its end: every layer keeps the largest of what it stored (half_note), and a
 // weight beyond the range is packed as a NaN (with itself in the other two parts).  Such a board goes through c6_split.h.
 //
-// What bounds it: the matrix cores, 200 k cycles per board (the 1,890 MFMAs of the 3x3 layers and the first layer's 207 three
-// times each) of some 310 k; the epilogues, 22 instructions per output of a lane, go in the open.  2,048 boards 2,117 -> 1,382 us (six
-// products with the same structure; both sides on one box), 256 boards 271 -> 184, and in teams (c6_team.h) one board 58 -> 49, 53
-// boards 117 -> 98, 128 boards 215 -> 142, of which the launch that looks for boards left over is 4.
+// What bounds it: the matrix cores, 195 k cycles per board (the 1,890 MFMAs of the 3x3 layers and the first layer's 207 three
+// times each) of 330 k at 1.9 GHz; what goes in the open is the epilogue of each layer's last cout tile (5 k), the sums at the ends of kernel rows
+// and the first operands of each pass (3 to 5 k), and staging (7 k).  2,048 boards, both sides in turn: 2,117 -> 1,382 us from six
+// products to three with the same structure, and 2,260 -> 1,436 on another box with all epilogues but the last tile's behind MFMAs and
+// three instructions fewer in each (in cycles 350 k -> 330 k; the clock gives back half of it).  In teams (c6_team.h) one board 58 ->
+// 49 us, 53 boards 117 -> 98, 128 boards 215 -> 142, of which the launch that looks for boards left over is 4.
 #pragma once
 
 namespace c6 {
@@ -104,8 +106,8 @@ struct HalfGeo {
   static constexpr int CHECK = 44;   // words of RED: [0] half_note's, [1] an input is out of range, [2] one is not small
 };
 
-// What a sum over a 3x3 layer's products has to be multiplied by to be the pre-activation times kHalfA
-constexpr float kHalfUnit = 1.0f / kHalfW;
+// What a sum over a 3x3 layer's products has to be multiplied by to be the pre-activation
+constexpr float kHalfUnit = 1.0f / (kHalfW * kHalfA);
 
 // ---- range ----
 // What a wave's lanes stored of layer l (m: the largest magnitude of a lane's, NaN if there was one), in one word
@@ -122,106 +124,130 @@ __device__ __forceinline__ unsigned half_note(int l, float m) {
 __device__ __forceinline__ bool half_failed(unsigned w) { return (w & 1u) != 0 || ((w >> 16) & ~(w >> 8) & 0x7fu) != 0; }
 
 // ---- activations ----
-// SiLU of eight sums (times kHalfA), step by step (a lone wave waits for each result that its next instruction needs):
-// u / (1 + 2^u) by the approximate reciprocal r of the denominator: quotient q, and what it leaves, e (the result is
-// q + e r).  Where the denominator is infinite, what it leaves is a NaN, which min() drops, and q is 0.
-// LAST: without the factor (the heads' sums end where fp32 does).
-template <bool LAST> __device__ __forceinline__ void half_silu8(float (&u)[8], float (&q)[8], float (&e)[8], float (&r)[8]) {
-#pragma clang fp contract(off)
-  float d[8];
-#pragma unroll
-  for (int i = 0; i < 8; ++i) {
-    d[i] = u[i] * (1.0f / kHalfA);
-    if constexpr (LAST) u[i] = d[i];
-  }
-  __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-  for (int i = 0; i < 8; ++i) d[i] = __builtin_amdgcn_exp2f(d[i]);
-  __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-  for (int i = 0; i < 8; ++i) d[i] = 1.0f + d[i];
-  __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-  for (int i = 0; i < 8; ++i) r[i] = __builtin_amdgcn_rcpf(d[i]);
-  __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-  for (int i = 0; i < 8; ++i) q[i] = u[i] * r[i];
-  __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-  for (int i = 0; i < 8; ++i) e[i] = fmaf(-d[i], q[i], u[i]);
-  __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-  for (int i = 0; i < 8; ++i) e[i] = fminf(e[i], 0x1p100f);
-  __builtin_amdgcn_sched_barrier(0);
-}
 __device__ __forceinline__ float half_larger(float m, float a, float b) {   // (a NaN stays one)
   return __builtin_elementwise_maximum(m, __builtin_elementwise_maximum(__builtin_fabsf(a), __builtin_fabsf(b)));
 }
-// Both parts of the activations of eight sums; m: the largest so far
-__device__ __forceinline__ void half_store8(float (&u)[8], int (&hi)[4], int (&lo)[4], float &m) {
+// The epilogue of one tile, a lane's sixteen pre-activations u, as a list of single instructions: SiLU, eight outputs at a time and
+// step by step (a lone wave waits for each result that its next instruction needs): u / (1 + 2^u) by the approximate reciprocal r of
+// the denominator, quotient q, and what it leaves, e (the result is q + e r).  Where the denominator is infinite, what it
+// leaves is a NaN, which min() drops, and q is 0.  Of q + e r come both parts, times kHalfA (by the denominator); in the last layer (LAST)
+// the activations themselves, into the heads' sums.  m: the largest magnitude.
+struct HalfTemps {
+  float d[8], r[8], q[8], e[8];
+};
+typedef int v16i __attribute__((ext_vector_type(16)));   // both parts of sixteen channels: hi in pairs, then lo
+struct HalfHeads {
+  float pol, val;
+  f32x16 pw, vw;   // the tile's head weights, as a lane's registers hold its channels
+};
+template <bool LAST> struct HalfEpi {
+  static constexpr int GROUP = LAST ? 76 : 84;
+  template <int I, class Out>
+  __device__ __forceinline__ static void atom(const f32x16 &u, HalfTemps &t, Out &out, float &m, float minus) {
 #pragma clang fp contract(off)
-  float q[8], e[8], r[8], minus = -1.0f;
-  asm volatile("" : "+s"(minus));   // (q - hi as one instruction that takes hi as it is)
-  half_silu8<false>(u, q, e, r);
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    hi[i] = pack2<PrecF16>(q[2 * i], q[2 * i + 1]);
-    m = half_larger(m, q[2 * i], q[2 * i + 1]);
+    constexpr int k = I % GROUP, x0 = I / GROUP * 8, i = k % 8, p = k % 4;
+    if constexpr (k < 8) t.d[i] = __builtin_amdgcn_exp2f(u[x0 + i]);
+    else if constexpr (k < 16) t.d[i] = LAST ? 1.0f + t.d[i] : fmaf(t.d[i], 1.0f / kHalfA, 1.0f / kHalfA);
+    else if constexpr (k < 24) t.r[i] = __builtin_amdgcn_rcpf(t.d[i]);
+    else if constexpr (k < 32) t.q[i] = u[x0 + i] * t.r[i];
+    else if constexpr (k < 40) t.e[i] = fmaf(-t.d[i], t.q[i], u[x0 + i]);
+    else if constexpr (k < 48) t.e[i] = fminf(t.e[i], 0x1p100f);
+    else if constexpr (LAST) {
+      if constexpr (k < 56) t.q[i] = fmaf(t.e[i], t.r[i], t.q[i]);
+      else if constexpr (k < 60) m = half_larger(m, t.q[2 * p], t.q[2 * p + 1]);
+      else if constexpr (k < 68) out.pol = fmaf(t.q[k - 60], out.pw[x0 + k - 60], out.pol);
+      else out.val = fmaf(t.q[k - 68], out.vw[x0 + k - 68], out.val);
+    } else {
+      if constexpr (k < 52) out[x0 / 2 + p] = pack2<PrecF16>(t.q[2 * p], t.q[2 * p + 1]);
+      else if constexpr (k < 56) m = half_larger(m, t.q[2 * p], t.q[2 * p + 1]);
+      else if constexpr (k < 64) {
+        const int hi = out[x0 / 2 + i / 2];
+        t.q[i] = fmaf((float)__builtin_bit_cast(f16x2, hi)[i % 2], minus, t.q[i]);
+      } else if constexpr (k < 72) t.q[i] = fmaf(t.e[i], t.r[i], t.q[i]);
+      else if constexpr (k < 80) t.q[i] *= kHalfLow;
+      else out[8 + x0 / 2 + p] = pack2<PrecF16>(t.q[2 * p], t.q[2 * p + 1]);
+    }
   }
-  __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-  for (int i = 0; i < 8; ++i) q[i] = fmaf((float)__builtin_bit_cast(f16x2, hi[i / 2])[i % 2], minus, q[i]);
-  __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-  for (int i = 0; i < 8; ++i) q[i] = fmaf(e[i], r[i], q[i]);
-  __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-  for (int i = 0; i < 8; ++i) q[i] *= kHalfLow;
-  __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-  for (int i = 0; i < 4; ++i) lo[i] = pack2<PrecF16>(q[2 * i], q[2 * i + 1]);
-  __builtin_amdgcn_sched_barrier(0);
+  // all at once
+  template <class Out> __device__ __forceinline__ static void run(const f32x16 &u, Out &out, float &m) {
+    float minus = -1.0f;
+    asm volatile("" : "+s"(minus));   // (q - hi as one instruction that takes hi as it is)
+    HalfTemps t;
+    static_for<0, 2 * GROUP>([&](auto ic) __attribute__((always_inline)) {
+      constexpr int i = decltype(ic)::value;
+      atom<i>(u, t, out, m, minus);
+      if constexpr (i % 4 == 3) __builtin_amdgcn_sched_barrier(0);
+    });
+  }
+};
+__device__ __forceinline__ v16i half_activations(const f32x16 &u, float &m) {
+  v16i out;
+  HalfEpi<false>::run(u, out, m);
+  return out;
 }
-// ... of the last layer: the activations themselves, for the heads
-__device__ __forceinline__ void half_last8(float (&u)[8], float (&v)[8], float &m) {
-#pragma clang fp contract(off)
-  float q[8], e[8], r[8];
-  half_silu8<true>(u, q, e, r);
+__device__ __forceinline__ void half_put(unsigned char *smem, int pos, int h, int t, const v16i &v) {
+  const int base = pos * HalfGeo::PIXB + 8 * h, sw = split_swz(pos);
 #pragma unroll
-  for (int i = 0; i < 8; ++i) v[i] = fmaf(e[i], r[i], q[i]);
-#pragma unroll
-  for (int i = 0; i < 4; ++i) m = half_larger(m, v[2 * i], v[2 * i + 1]);
-  __builtin_amdgcn_sched_barrier(0);
+  for (int q = 0; q < 4; ++q) {
+    *reinterpret_cast<v2i *>(smem + base + ((64 * t + 16 * q) ^ sw)) = v2i{v[2 * q], v[2 * q + 1]};
+    *reinterpret_cast<v2i *>(smem + base + ((HalfGeo::PLANEB + 64 * t + 16 * q) ^ sw)) = v2i{v[8 + 2 * q], v[8 + 2 * q + 1]};
+  }
 }
 
 // ---- the 3x3 layers ----
-// Weight ring: k-steps of TN cout tiles and two planes in flight.  The loads take some 800 cycles, a k-step 288 TN.
-template <int L, int TN> constexpr int half_ring() {
-  constexpr int U = 3 * kCinArr[L] / 16;   // k-steps of a kernel row: 6, 12, 18
-  return TN == 2 ? 2 : (U % 3 == 0 ? 3 : 2);
+// words of the tail as a lane's registers hold a cout tile's channels
+__device__ __forceinline__ f32x16 half_tail(const float *words, int h) {
+  f32x16 v[1];
+  load_bias_tiles(v, words, h);
+  return v[0];
 }
-template <int L, int TN> using HalfWeights = v4i[half_ring<L, TN>()][TN][2];
-
-template <int L, int T0, int TN> __device__ __forceinline__ void half_preload(HalfWeights<L, TN> &ring, const WFrags &wl) {
+// What a pass over TN cout tiles of layer L, from T0 on, starts with, asked for in front of the epilogue before it: the weights of
+// its first k-steps (two planes; the loads take some 800 cycles, a k-step 288 TN) and its biases.
+template <int TN> constexpr int kHalfRing = TN == 2 ? 2 : 3;
+template <int TN> struct HalfStart {
+  v4i ring[kHalfRing<TN>][TN][2];
+  f32x16 bias[TN], low[TN];
+};
+template <int L, int T0, int TN> __device__ __forceinline__ HalfStart<TN> half_start(const unsigned char *packed, const float *tail, int lane) {
   constexpr int NT = kCoutArr[L] / 32;
+  const WFrags wl = layer_weights<PrecF32S, L>(packed, lane);
+  HalfStart<TN> v;
 #pragma unroll
-  for (int d = 0; d < half_ring<L, TN>(); ++d)
+  for (int t = 0; t < TN; ++t) {
+    v.bias[t] = half_tail(tail + bias_offset(L) + 32 * (T0 + t), lane >> 5);
+    v.low[t] = half_tail(tail + Geo<PrecF32S>::TAIL_BIAS_LOW + bias_offset(L) + 32 * (T0 + t), lane >> 5);
+  }
+#pragma unroll
+  for (int d = 0; d < kHalfRing<TN>; ++d)
 #pragma unroll
     for (int t = 0; t < TN; ++t)
 #pragma unroll
-      for (int i = 0; i < 2; ++i) ring[d][t][i] = wl[(d * NT + T0 + t) * 3 + i];
+      for (int i = 0; i < 2; ++i) v.ring[d][t][i] = wl[(d * NT + T0 + t) * 3 + i];
   __builtin_amdgcn_sched_barrier(0);
+  return v;
 }
+
+// Pixel tiles whose pre-activations wait for their epilogue while a pass over K runs: UN of them per kernel row, the first in the queue,
+// a few instructions behind each MFMA, and then to its end as both parts.
+template <int UN> struct HalfQueue {
+  f32x16 q[3 * UN];
+};
+struct HalfIdle {};
 
 // The contraction of 3x3 layer L, TN of its cout tiles from T0 on.  K runs over kernel rows, the three taps of a row, then 16
 // channels at a time; each k-step is nine MFMAs per cout tile: three products of each of three pixel tiles.  The sum of a row's hi hi
-// products goes to held at its end, the others' sum, low, runs through.
-//   ring: the first k-steps on entry
-template <int L, int T0, int TN>
-__device__ __forceinline__ void half_conv(const unsigned char *smem, const WFrags &wl, HalfWeights<L, TN> &ring, const int (&ci)[3],
-                                          int h, f32x16 (&held)[TN][3], f32x16 (&low)[TN][3]) {
-  constexpr int NT = kCoutArr[L] / 32, KC = kCinArr[L] / 16, U = 3 * KC, D = half_ring<L, TN>();
+// products goes to held at its end, the others' sum, low, runs through (from what the bias leaves out); at the end held is the
+// pre-activation.
+template <int L, int T0, int TN, class Queue>
+__device__ __forceinline__ void half_conv(const unsigned char *smem, const unsigned char *packed, HalfStart<TN> &start, const int (&ci)[3],
+                                          int lane, f32x16 (&held)[TN][3], Queue &queue, float &m) {
+  constexpr int NT = kCoutArr[L] / 32, KC = kCinArr[L] / 16, U = 3 * KC, D = kHalfRing<TN>, SLOTS = U * TN * 9;
   static_assert(U % D == 0 && U % 2 == 0, "double buffers must line up across rows");
+  constexpr int UN = std::is_same_v<Queue, HalfIdle> ? 0 : sizeof(Queue) / sizeof(f32x16) / 3;
+  const int h = lane >> 5;
+  const WFrags wl = layer_weights<PrecF32S, L>(packed, lane);
+  float minus = -1.0f;
+  asm volatile("" : "+s"(minus));   // (q - hi as one instruction that takes hi as it is)
   int at[3][4];   // the lane's squares at a tap: where units 32 k (k = 0 ... 3) of a 128-byte block are
   auto set_tap = [&](int ky, int kx) __attribute__((always_inline)) {
 #pragma unroll
@@ -237,13 +263,14 @@ __device__ __forceinline__ void half_conv(const unsigned char *smem, const WFrag
     const int o = i * HalfGeo::PLANEB + c * 32;
     a[par][j][i] = *reinterpret_cast<const v4i *>(smem + at[j][o / 32 % 4] + o / 128 * 128);
   };
-  f32x16 sum[TN][3];
+  f32x16 sum[TN][3], low[TN][3];
 #pragma unroll
   for (int t = 0; t < TN; ++t)
 #pragma unroll
-    for (int j = 0; j < 3; ++j)
-#pragma unroll
-      for (int e = 0; e < 16; ++e) held[t][j][e] = low[t][j][e] = 0.0f;
+    for (int j = 0; j < 3; ++j) {
+      held[t][j] = start.bias[t];
+      low[t][j] = start.low[t];
+    }
   set_tap(0, 0);
 #pragma unroll
   for (int j = 0; j < 3; ++j)
@@ -252,22 +279,32 @@ __device__ __forceinline__ void half_conv(const unsigned char *smem, const WFrag
 #pragma unroll 1
   for (int ky = 0; ky < 3; ++ky) {
     const WFrags wn = wl + ((ky * U + D) * NT + T0) * 3;
+    HalfTemps temps;
+    v16i done[UN > 0 ? UN : 1];
     static_for<0, U>([&](auto uc) __attribute__((always_inline)) {
       constexpr int u = decltype(uc)::value, par = u & 1, un = u + 1;
       // (behind the last tap this wraps to the first: harmless extra reads)
       if constexpr (un % KC == 0) set_tap(un < U ? ky : (ky == 2 ? 0 : ky + 1), un < U ? un / KC : 0);
       static_for<0, TN * 9>([&](auto gc) __attribute__((always_inline)) {
-        constexpr int g = decltype(gc)::value, t = g / 9, m = g % 9 / 3, j = g % 3;
+        constexpr int g = decltype(gc)::value, t = g / 9, mm = g % 9 / 3, j = g % 3;
         // lo hi, hi lo, hi hi (weight, activation)
-        if constexpr (m == 0) mma<PrecF16>(ring[u % D][t][1], a[par][j][0], low[t][j]);
-        if constexpr (m == 1) mma<PrecF16>(ring[u % D][t][0], a[par][j][1], low[t][j]);
-        if constexpr (m == 2) {
+        if constexpr (mm == 0) mma<PrecF16>(start.ring[u % D][t][1], a[par][j][0], low[t][j]);
+        if constexpr (mm == 1) mma<PrecF16>(start.ring[u % D][t][0], a[par][j][1], low[t][j]);
+        if constexpr (mm == 2) {
           if constexpr (u == 0) sum[t][j] = f32x16{};
-          mma<PrecF16>(ring[u % D][t][0], a[par][j][0], sum[t][j]);
+          mma<PrecF16>(start.ring[u % D][t][0], a[par][j][0], sum[t][j]);
         }
         if constexpr (g < 6) read(un % KC, par ^ 1, g / 2, g % 2);
-        if constexpr (j == 2 && m == 0) ring[u % D][t][1] = wn[(u * NT + t) * 3 + 1];
-        if constexpr (j == 2 && m == 2) ring[u % D][t][0] = wn[(u * NT + t) * 3];
+        if constexpr (j == 2 && mm == 0) start.ring[u % D][t][1] = wn[(u * NT + t) * 3 + 1];
+        if constexpr (j == 2 && mm == 2) start.ring[u % D][t][0] = wn[(u * NT + t) * 3];
+        if constexpr (UN > 0) {
+          using Epi = HalfEpi<false>;
+          constexpr int slot = u * TN * 9 + g, N = UN * 2 * Epi::GROUP;
+          static_for<slot * N / SLOTS, (slot + 1) * N / SLOTS>([&](auto ac) __attribute__((always_inline)) {
+            constexpr int i = decltype(ac)::value, unit = i / (2 * Epi::GROUP);
+            Epi::atom<i % (2 * Epi::GROUP)>(queue.q[unit], temps, done[unit], m, minus);
+          });
+        }
         __builtin_amdgcn_sched_barrier(0);
       });
     });
@@ -281,11 +318,64 @@ __device__ __forceinline__ void half_conv(const unsigned char *smem, const WFrag
         for (int e = 0; e < 16; ++e) held[t][j][e] = fmaf(sum[t][j][e], kHalfUnit, held[t][j][e]);
         __builtin_amdgcn_sched_barrier(0);
       }
+    if constexpr (UN > 0) {
+#pragma unroll
+      for (int i = 0; i < 2 * UN; ++i) queue.q[i] = queue.q[i + UN];
+#pragma unroll
+      for (int i = 0; i < UN; ++i) queue.q[2 * UN + i] = __builtin_bit_cast(f32x16, done[i]);
+    }
   }
 #pragma unroll
   for (int t = 0; t < TN; ++t)
 #pragma unroll
-    for (int j = 0; j < 3; ++j) asm volatile("" : "+a"(low[t][j]));
+    for (int j = 0; j < 3; ++j) {
+      asm volatile("" : "+a"(low[t][j]));
+#pragma unroll
+      for (int e = 0; e < 16; ++e) held[t][j][e] = fmaf(low[t][j][e], kHalfUnit / kHalfLow, held[t][j][e]);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+}
+
+// one 3x3 layer that is not the last.  Its cout tiles go in two passes over K, all but the last (two at most: the sums of three would
+// fill the registers) and the last: behind the second pass's MFMAs go the first one's epilogues, whose activations wait
+// in registers until every wave has read the layer's input.
+//   start: of the layer's first pass on entry, of the next layer's on return
+template <int L, int TN, int TNN>
+__device__ __forceinline__ void half_layer(unsigned char *smem, const unsigned char *packed, const float *tail, const int (&ci)[3],
+                                           int lane, HalfStart<TN> &start, HalfStart<TNN> &next, unsigned &note) {
+  constexpr int NT = kCoutArr[L] / 32;
+  static_assert(TN == (NT == 3 ? 2 : 1), "passes");
+  const int h = lane >> 5;
+  float m = 0.0f;
+  f32x16 held[1][3];
+  HalfQueue<TN> queue;
+  HalfIdle idle;
+  if constexpr (NT == 1) {
+    half_conv<L, 0, 1>(smem, packed, start, ci, lane, held, idle, m);
+  } else {
+    f32x16 first[TN][3];
+    half_conv<L, 0, TN>(smem, packed, start, ci, lane, first, idle, m);
+    HalfStart<1> second = half_start<L, TN, 1>(packed, tail, lane);
+#pragma unroll
+    for (int t = 0; t < TN; ++t)
+#pragma unroll
+      for (int j = 0; j < 3; ++j) queue.q[j * TN + t] = first[t][j];
+    half_conv<L, TN, 1>(smem, packed, second, ci, lane, held, queue, m);
+  }
+  next = half_start<L + 1, 0, TNN>(packed, tail, lane);
+  __syncthreads();   // every wave has finished reading the layer's input
+#pragma unroll
+  for (int j = 0; j < 3; ++j) {
+    int pos = ci[j];
+    asm volatile("" : "+v"(pos));  // (addresses formed here, not kept for the whole kernel)
+    if constexpr (NT > 1) {
+#pragma unroll
+      for (int t = 0; t < TN; ++t) half_put(smem, pos, h, t, __builtin_bit_cast(v16i, queue.q[j * TN + t]));
+    }
+    half_put(smem, pos, h, NT - 1, half_activations(held[0][j], m));
+  }
+  note |= half_note(L, m);
+  __syncthreads();
 }
 
 // First layer, what the inputs' first parts leave: ROWS rows of K, three fragments of 8 columns each, rowb bytes apart in LDS.
@@ -299,132 +389,6 @@ __device__ __forceinline__ void half_second(const unsigned char *smem, const WFr
 #pragma unroll
       for (int j = 0; j < 3; ++j) mma<PrecF16>(w, *reinterpret_cast<const v4i *>(smem + at[j] + row * rowb + i * 16), low[0][j]);
     }
-}
-
-// the bias of a cout tile as a lane's registers hold its channels, times kHalfA, and what its rounding to fp32 left
-struct HalfBias {
-  f32x16 high, low;
-};
-template <int L> __device__ __forceinline__ HalfBias half_bias(const float *tail, int t, int h) {
-  f32x16 b[1], l[1];
-  load_bias_tiles(b, tail + bias_offset(L) + 32 * t, h);
-  load_bias_tiles(l, tail + Geo<PrecF32S>::TAIL_BIAS_LOW + bias_offset(L) + 32 * t, h);
-  return {b[0] * kHalfA, l[0] * kHalfA};
-}
-// eight outputs' pre-activations (times kHalfA) from register e0 on
-__device__ __forceinline__ void half_total8(const f32x16 &held, const f32x16 &small, const HalfBias &b, int e0, float (&u)[8]) {
-  f32x16 low = small;
-  __builtin_amdgcn_sched_barrier(0);
-  asm volatile("" : "+a"(low));
-#pragma unroll
-  for (int i = 0; i < 8; ++i) u[i] = fmaf(low[e0 + i], kHalfUnit / kHalfLow, b.low[e0 + i]);
-  __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-  for (int i = 0; i < 8; ++i) u[i] += held[e0 + i] + b.high[e0 + i];
-  __builtin_amdgcn_sched_barrier(0);
-}
-
-// one tile's activations, both parts of sixteen channels of the lane's square
-struct HalfTile {
-  int hi[8], lo[8];
-};
-typedef int v16i __attribute__((ext_vector_type(16)));
-__device__ __forceinline__ void half_put(unsigned char *smem, int pos, int h, int t, const HalfTile &v) {
-  const int base = pos * HalfGeo::PIXB + 8 * h, sw = split_swz(pos);
-#pragma unroll
-  for (int q = 0; q < 4; ++q) {
-    *reinterpret_cast<v2i *>(smem + base + ((64 * t + 16 * q) ^ sw)) = v2i{v.hi[2 * q], v.hi[2 * q + 1]};
-    *reinterpret_cast<v2i *>(smem + base + ((HalfGeo::PLANEB + 64 * t + 16 * q) ^ sw)) = v2i{v.lo[2 * q], v.lo[2 * q + 1]};
-  }
-}
-template <class U> __device__ __forceinline__ HalfTile half_tile(U sums, float &m) {   // sums(e0, u): eight pre-activations
-  HalfTile v;
-#pragma unroll
-  for (int e0 = 0; e0 < 16; e0 += 8) {
-    float u[8];
-    int hi[4], lo[4];
-    sums(e0, u);
-    half_store8(u, hi, lo, m);
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      v.hi[e0 / 2 + i] = hi[i];
-      v.lo[e0 / 2 + i] = lo[i];
-    }
-  }
-  return v;
-}
-
-// one 3x3 layer that is not the last.  Three cout tiles go in two passes over K, two and one (the sums of three would fill the
-// registers): the first pass's activations wait in registers until every wave has read its last input.
-template <int L>
-__device__ __forceinline__ void half_layer(unsigned char *smem, const unsigned char *packed, const float *tail, const int (&ci)[3],
-                                           int h, int lane, unsigned &note) {
-  constexpr int NT = kCoutArr[L] / 32, TN = NT < 2 ? NT : 2;
-  const WFrags wl = layer_weights<PrecF32S, L>(packed, lane);
-  float m = 0.0f;
-  HalfTile wait[TN][3];
-  {
-    HalfWeights<L, TN> ring;
-    half_preload<L, 0, TN>(ring, wl);
-    f32x16 held[TN][3], low[TN][3];
-    half_conv<L, 0, TN>(smem, wl, ring, ci, h, held, low);
-    if constexpr (NT < 3) __syncthreads();   // every wave has finished reading the layer's input
-#pragma unroll
-    for (int t = 0; t < TN; ++t) {
-      const HalfBias b = half_bias<L>(tail, t, h);
-#pragma unroll
-      for (int j = 0; j < 3; ++j) {
-        wait[t][j] = half_tile([&](int e0, float (&u)[8]) __attribute__((always_inline)) { half_total8(held[t][j], low[t][j], b, e0, u); }, m);
-        if constexpr (NT < 3) {
-          int pos = ci[j];
-          asm volatile("" : "+v"(pos));  // (addresses formed here, not kept for the whole kernel)
-          half_put(smem, pos, h, t, wait[t][j]);
-        }
-      }
-    }
-  }
-  if constexpr (NT == 3) {
-    // (in accumulation registers, of which this pass leaves some; the vector ones are short)
-    v16i kept[2][3];
-#pragma unroll
-    for (int t = 0; t < 2; ++t)
-#pragma unroll
-      for (int j = 0; j < 3; ++j) {
-#pragma unroll
-        for (int i = 0; i < 8; ++i) {
-          kept[t][j][i] = wait[t][j].hi[i];
-          kept[t][j][8 + i] = wait[t][j].lo[i];
-        }
-        asm volatile("" : "+a"(kept[t][j]));
-      }
-    HalfWeights<L, 1> ring;
-    half_preload<L, 2, 1>(ring, wl);
-    f32x16 held[1][3], low[1][3];
-    half_conv<L, 2, 1>(smem, wl, ring, ci, h, held, low);
-    __syncthreads();
-    const HalfBias b = half_bias<L>(tail, 2, h);
-#pragma unroll
-    for (int j = 0; j < 3; ++j) {
-      int pos = ci[j];
-      asm volatile("" : "+v"(pos));
-#pragma unroll
-      for (int t = 0; t < 2; ++t) {
-        v16i v = kept[t][j];
-        asm volatile("" : "+a"(v));
-        HalfTile w;
-#pragma unroll
-        for (int i = 0; i < 8; ++i) {
-          w.hi[i] = v[i];
-          w.lo[i] = v[8 + i];
-        }
-        half_put(smem, pos, h, t, w);
-        __builtin_amdgcn_sched_barrier(0);
-      }
-      half_put(smem, pos, h, 2, half_tile([&](int e0, float (&u)[8]) __attribute__((always_inline)) { half_total8(held[0][j], low[0][j], b, e0, u); }, m));
-    }
-  }
-  note |= half_note(L, m);
-  __syncthreads();
 }
 
 // A board that this kernel leaves to split_forward_kernel, which follows it on the stream: a word among its outputs that
@@ -593,11 +557,10 @@ __global__ __launch_bounds__(256) void half_forward_kernel(const FwdParams prm) 
       for (int j = 0; j < 3; ++j)
 #pragma unroll
         for (int i = 0; i < 16; ++i) {
-          a0[0][j][i] = kHalfA * (plane2_varies ? b0[0][i] : fmaf(c2, a0[0][j][i], b0[0][i]));
-          low[0][j][i] = kHalfA * kHalfLow * bl[0][i];
+          a0[0][j][i] = kHalfW * (plane2_varies ? b0[0][i] : fmaf(c2, a0[0][j][i], b0[0][i]));
+          low[0][j][i] = bl[0][i] * (1.0f / kHalfA);   // (the inputs carry no factor)
         }
     }
-    static_assert(kHalfA == kHalfW, "the first layer's sums carry the weights' factor alone, and are the others' units");
     // An input that is exact in fp16 (stones, flags) is one part; what is left of any other is staged behind it, for the
     // products with the weights' first parts, which are small ones.
     auto stage = [&](bool first) __attribute__((always_inline)) {
@@ -669,57 +632,63 @@ __global__ __launch_bounds__(256) void half_forward_kernel(const FwdParams prm) 
       const int pos = k < 20 ? k : (k < 41 ? 400 + (k - 20) : (k - 40) * kPitch);
       *reinterpret_cast<v4i *>(smem + pos * S::PIXB + w16 * 16) = v4i{0, 0, 0, 0};
     }
+    HalfStart<1> one = half_start<1, 0, 1>(packed, tail, lane);
+    HalfStart<2> two;
     {
       float m = 0.0f;
 #pragma unroll
       for (int j = 0; j < 3; ++j) {
         int pos = ci[j];
         asm volatile("" : "+v"(pos));
-        half_put(smem, pos, h, 0, half_tile([&](int e0, float (&u)[8]) __attribute__((always_inline)) {
-          f32x16 small = low[0][j], large = a0[0][j];
-          __builtin_amdgcn_sched_barrier(0);
-          asm volatile("" : "+a"(small), "+a"(large));
+        f32x16 small = low[0][j], large = a0[0][j], u;
+        __builtin_amdgcn_sched_barrier(0);
+        asm volatile("" : "+a"(small), "+a"(large));
 #pragma unroll
-          for (int i = 0; i < 8; ++i) u[i] = fmaf(small[e0 + i], 1.0f / kHalfLow, large[e0 + i]);
-          __builtin_amdgcn_sched_barrier(0);
-        }, m));
+        for (int i = 0; i < 16; ++i) u[i] = fmaf(small[i], 1.0f / (kHalfW * kHalfLow), large[i] * (1.0f / kHalfW));
+        half_put(smem, pos, h, 0, half_activations(u, m));
       }
       note |= half_note(0, m);
     }
     __syncthreads();
 
-    half_layer<1>(smem, packed, tail, ci, h, lane, note);
-    half_layer<2>(smem, packed, tail, ci, h, lane, note);
-    half_layer<3>(smem, packed, tail, ci, h, lane, note);
-    half_layer<4>(smem, packed, tail, ci, h, lane, note);
-    half_layer<5>(smem, packed, tail, ci, h, lane, note);
-    half_layer<6>(smem, packed, tail, ci, h, lane, note);
+    half_layer<1>(smem, packed, tail, ci, lane, one, one, note);
+    half_layer<2>(smem, packed, tail, ci, lane, one, one, note);
+    half_layer<3>(smem, packed, tail, ci, lane, one, one, note);
+    half_layer<4>(smem, packed, tail, ci, lane, one, two, note);
+    half_layer<5>(smem, packed, tail, ci, lane, two, two, note);
+    half_layer<6>(smem, packed, tail, ci, lane, two, two, note);
 
-    // ---- layer 8 + both 1x1 heads straight from the fp32 accumulators ----
+    // ---- layer 8 + both 1x1 heads ----
     const float *valw = tail + kBiasTotal + kHeadC;
     {
       float m = 0.0f;
+      HalfIdle idle;
       SplitHeads heads(tail, tidv, lane, wave, h, red);
-      const WFrags wl = layer_weights<P, 7>(packed, lane);
-      auto pass = [&](auto t0c, auto tnc) __attribute__((always_inline)) {
-        constexpr int T0 = decltype(t0c)::value, TN = decltype(tnc)::value;
-        HalfWeights<7, TN> ring;
-        half_preload<7, T0, TN>(ring, wl);
-        f32x16 held[TN][3], low8[TN][3];
-        half_conv<7, T0, TN>(smem, wl, ring, ci, h, held, low8);
+      auto head = [&](int t, const f32x16 (&u)[3]) __attribute__((always_inline)) {
+        HalfHeads out;
+        out.pw = half_tail(tail + kBiasTotal + 32 * t, h);
+        out.vw = half_tail(tail + kBiasTotal + kHeadC + 32 * t, h);
+        float pol[3], val[3];
 #pragma unroll
-        for (int t = 0; t < TN; ++t) {
-          const HalfBias bias = half_bias<7>(tail, T0 + t, h);
-          heads.tile(T0 + t, [&](int j, int e0, float (&v)[8]) __attribute__((always_inline)) {
-            float u[8];
-            half_total8(held[t][j], low8[t][j], bias, e0, u);
-            half_last8(u, v, m);
-          });
+        for (int j = 0; j < 3; ++j) {
+          out.pol = out.val = 0.0f;
+          HalfEpi<true>::run(u[j], out, m);
+          pol[j] = out.pol;
+          val[j] = out.val;
         }
+        heads.reduce(t, pol, val);
       };
-      pass(IC<0>{}, IC<2>{});
+      {
+        f32x16 u[2][3];
+        half_conv<7, 0, 2>(smem, packed, two, ci, lane, u, idle, m);
+        one = half_start<7, 2, 1>(packed, tail, lane);
+        head(0, u[0]);
+        head(1, u[1]);
+      }
       if (b + 1 < b_end) fetch_board(b + 1);  // lands while this board is finished
-      pass(IC<2>{}, IC<1>{});
+      f32x16 u[1][3];
+      half_conv<7, 2, 1>(smem, packed, one, ci, lane, u, idle, m);
+      head(2, u[0]);
       note |= half_note(7, m);
       if (lane == 0) atomicOr(check, note);
       heads.logits(lgt, valw[kHeadC]);

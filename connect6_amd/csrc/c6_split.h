@@ -39,6 +39,9 @@
 
 namespace c6 {
 
+// What the packed low words of the biases have to be multiplied by (they are c6_half.h's, in the units of its small sums)
+constexpr float kTailLow = 1.0f / (kHalfW * kHalfA * kHalfLow);
+
 struct SplitGeo {
   using G = Geo<PrecF32S>;                     // weight stream and first-layer geometry
   static constexpr int PIXB = 384;             // 3 planes x 64 channels x 2 bytes, or 96 x 4
@@ -235,7 +238,7 @@ __device__ __forceinline__ void split_conv(const unsigned char *smem, const WFra
 #pragma unroll
     for (int j = 0; j < N; ++j) {
       acc[t][j] = b[0];
-      low[t][j] = bl[0];
+      low[t][j] = bl[0] * kTailLow;
     }
   }
   constexpr int AHEAD = WIDE ? 2 : 1;
@@ -461,6 +464,10 @@ struct SplitHeads {
           val[j] = fmaf(v[e], vw[q + e / 4][e % 4], val[j]);
         }
       }
+    reduce(t, pol, val);
+  }
+  // ... from a lane's sums over the tile's channels
+  __device__ __forceinline__ void reduce(int t, const float (&pol)[3], const float (&val)[3]) {
 #pragma unroll
     for (int j = 0; j < 3; ++j) {
       const unsigned bits = __builtin_bit_cast(unsigned, pol[j]);
@@ -579,7 +586,7 @@ __device__ __forceinline__ void split_board(const FwdParams &prm, unsigned char 
 #pragma unroll
         for (int e = 0; e < 4; ++e) a0[0][j][4 * q + e] = plane2_varies ? b0[0][4 * q + e] : fmaf(c2, t4[e], b0[0][4 * q + e]);
       }
-      low[0][j] = bl[0];
+      low[0][j] = bl[0] * kTailLow;
 #pragma unroll
       for (int i = 0; i < 16; ++i) first[0][j][i] = 0.0f;
     }

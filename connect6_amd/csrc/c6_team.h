@@ -167,7 +167,7 @@ __device__ __forceinline__ void team_lo_pass(const unsigned char *smem, const un
 // The contraction of 3x3 layer L for PT tiles of 32 squares and TT cout tiles from t0 on (tiles beyond
 // the layer's last repeat it; their results are not used).
 //   rec: LDS addresses of the lane's squares' records;  acc: the bias on entry
-//   fp32 (as half_conv): the sums start at zero; acc: the rows' sums of the largest products, low: the others
+//   fp32 (as half_layer): low: what the bias leaves out, for the small products' sum
 template <class P, int L, int TT, int PT>
 __device__ __forceinline__ void team_conv(const unsigned char *smem, const unsigned char *packed, const WFrags &wl,
                                           v4i (&ring)[team_ring<P, TT, PT>()][TT][TeamGeo<P>::WPL], int lane,
@@ -274,14 +274,18 @@ __device__ __forceinline__ void team_conv(const unsigned char *smem, const unsig
 #pragma unroll
     for (int p = 0; p < PT; ++p)
 #pragma unroll
-      for (int t = 0; t < TT; ++t) asm volatile("" : "+a"(low[p][t]));
+      for (int t = 0; t < TT; ++t) {
+        asm volatile("" : "+a"(low[p][t]));
+#pragma unroll
+        for (int e = 0; e < 16; ++e) acc[p][t][e] = fmaf(low[p][t][e], kHalfUnit / kHalfLow, acc[p][t][e]);
+      }
   }
 }
 
 // SiLU of one accumulator tile, step by step: a lone wave waits for each result that its next instruction needs.  Against
 // output by output it is worth a per cent, one way or the other: 22 to 40 boards in bf16 and fp16 40.0 -> 39.6 us, 40 boards that
 // a cascade lists 117.2 -> 116.2, but 1 to 16 boards in bf16 30.2 -> 30.6; the
-// teams beside whole rounds the same.  (fp32: half_silu8.)
+// teams beside whole rounds the same.  (fp32: HalfEpi.)
 template <class P> __device__ __forceinline__ void silu_tile(const f32x16 &acc, float (&v)[16]) {
   __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
@@ -305,14 +309,11 @@ __device__ __forceinline__ void team_store(unsigned char *smem, int rec, int h, 
   using T = TeamGeo<P>;
   unsigned char *at = smem + rec + 64 * t + 8 * h;
   if constexpr (T::SPLIT) {
-    const HalfTile v = half_tile([&](int e0, float (&u)[8]) __attribute__((always_inline)) {
-#pragma unroll
-      for (int i = 0; i < 8; ++i) u[i] = acc[e0 + i];
-    }, most);
+    const v16i v = half_activations(acc, most);
 #pragma unroll
     for (int q = 0; q < 4; ++q) {
-      *reinterpret_cast<v2i *>(at + 16 * q) = v2i{v.hi[2 * q], v.hi[2 * q + 1]};
-      *reinterpret_cast<v2i *>(at + 192 + 16 * q) = v2i{v.lo[2 * q], v.lo[2 * q + 1]};
+      *reinterpret_cast<v2i *>(at + 16 * q) = v2i{v[2 * q], v[2 * q + 1]};
+      *reinterpret_cast<v2i *>(at + 192 + 16 * q) = v2i{v[8 + 2 * q], v[8 + 2 * q + 1]};
     }
   } else {
     const DropConsts k = drop_consts<P>();
@@ -616,8 +617,8 @@ __device__ __forceinline__ void team_board(const TeamParams &prm, unsigned char 
         const int word = bias_offset(L) + 32 * (t0 + t < NT ? t0 + t : NT - 1);
 #pragma unroll
         for (int i = 0; i < PT; ++i) {
-          if constexpr (T::SPLIT) acc[i][t] = low[i][t] = f32x16{};
-          else acc[i][t] = tail_tile(word);
+          acc[i][t] = tail_tile(word);
+          if constexpr (T::SPLIT) low[i][t] = tail_tile(G::TAIL_BIAS_LOW + word);
         }
       }
     }
@@ -633,20 +634,6 @@ __device__ __forceinline__ void team_board(const TeamParams &prm, unsigned char 
       rec[i] = record(ok[i] ? p[i] : kPix - 1, sp.base);
     }
     if (active) team_conv<P, L, TT, PT>(smem, packed, wl, ring, lane, rec, t0, acc, low);
-    if constexpr (T::SPLIT) {
-      if (active) {   // (as half_total8)
-#pragma unroll
-        for (int t = 0; t < TT; ++t) {
-          const int word = bias_offset(L) + 32 * (t0 + t < NT ? t0 + t : NT - 1);
-          const f32x16 bias = tail_tile(word) * kHalfA, rest = tail_tile(G::TAIL_BIAS_LOW + word) * kHalfA;
-#pragma unroll
-          for (int i = 0; i < PT; ++i)
-#pragma unroll
-            for (int e = 0; e < 16; ++e)
-              acc[i][t][e] = fmaf(low[i][t][e], kHalfUnit / kHalfLow, rest[e]) + (acc[i][t][e] + bias[e]);
-        }
-      }
-    }
     C6_MARK(6 * L + 3);
     if constexpr (L < 7) {
       __syncthreads();   // everybody has read this layer's input
@@ -664,29 +651,16 @@ __device__ __forceinline__ void team_board(const TeamParams &prm, unsigned char 
             float pol[PT], val[PT];
 #pragma unroll
             for (int i = 0; i < PT; ++i) pol[i] = val[i] = 0.0f;
-            float a[PT][16];
+            HalfHeads out;
+            out.pw = tail_tile(kBiasTotal + 32 * (t0 + t));
+            out.vw = tail_tile(kBiasTotal + kHeadC + 32 * (t0 + t));
 #pragma unroll
-            for (int i = 0; i < PT; ++i)
-#pragma unroll
-              for (int e0 = 0; e0 < 16; e0 += 8) {
-                float u[8], v[8];
-#pragma unroll
-                for (int e = 0; e < 8; ++e) u[e] = acc[i][t][e0 + e];
-                half_last8(u, v, most);
-#pragma unroll
-                for (int e = 0; e < 8; ++e) a[i][e0 + e] = v[e];
-              }
-#pragma unroll
-            for (int q = 0; q < 4; ++q)
-#pragma unroll
-              for (int e = 0; e < 4; ++e) {
-                const float p1 = pw[32 * (t0 + t) + 8 * q + e], v1 = pw[kHeadC + 32 * (t0 + t) + 8 * q + e];
-#pragma unroll
-                for (int i = 0; i < PT; ++i) {
-                  pol[i] = fmaf(a[i][4 * q + e], p1, pol[i]);
-                  val[i] = fmaf(a[i][4 * q + e], v1, val[i]);
-                }
-              }
+            for (int i = 0; i < PT; ++i) {
+              out.pol = out.val = 0.0f;
+              HalfEpi<true>::run(acc[i][t], out, most);
+              pol[i] = out.pol;
+              val[i] = out.val;
+            }
 #pragma unroll
             for (int i = 0; i < PT; ++i) {
               const unsigned bits = __builtin_bit_cast(unsigned, pol[i]);
@@ -882,13 +856,13 @@ __device__ __forceinline__ void team_board(const TeamParams &prm, unsigned char 
 #pragma unroll
       for (int n = 0; n < N1; ++n)
 #pragma unroll
-        for (int i = 0; i < 16; ++i) acc[n][0][i] = (T::SPLIT ? kHalfA : 1.0f) * (plane2_varies ? b0[i] : fmaf(c2, acc[n][0][i], b0[i]));
+        for (int i = 0; i < 16; ++i) acc[n][0][i] = (T::SPLIT ? kHalfW : 1.0f) * (plane2_varies ? b0[i] : fmaf(c2, acc[n][0][i], b0[i]));
     }
     f32x16 low[N1], large[N1];   // SPLIT: small products; the large ones, once a second part follows
     if constexpr (T::SPLIT) {
       if (active) {
 #pragma unroll
-        for (int n = 0; n < N1; ++n) low[n] = tail_tile(G::TAIL_BIAS_LOW + bias_offset(0)) * (kHalfA * kHalfLow);
+        for (int n = 0; n < N1; ++n) low[n] = tail_tile(G::TAIL_BIAS_LOW + bias_offset(0)) * (1.0f / kHalfA);
       }
     }
 #pragma unroll 1
@@ -990,7 +964,7 @@ __device__ __forceinline__ void team_board(const TeamParams &prm, unsigned char 
 #pragma unroll
       for (int n = 0; n < N1; ++n)
 #pragma unroll
-        for (int i = 0; i < 16; ++i) acc[n][0][i] = fmaf(low[n][i], 1.0f / kHalfLow, acc[n][0][i]);
+        for (int i = 0; i < 16; ++i) acc[n][0][i] = fmaf(low[n][i], 1.0f / (kHalfW * kHalfLow), acc[n][0][i] * (1.0f / kHalfW));
     }
     C6_MARK(2);
     __syncthreads();   // the copies give way to the activations

@@ -10,9 +10,9 @@
 // order, so the results are the same bit for bit.
 //
 // What it takes (cycles of a 2.4 GHz clock; twelve workgroups, one board): staging the input 7 k, the first layer
-// 3 k (fp32 9 k), then per layer 1.2 k until the neighbours' flags are seen, 0.5 k until their squares are in LDS,
-// the MFMAs (bf16 0.5-2.1 k, fp32 2-6 k: three per product) and 1.3 k until the outputs are
-// stored and acknowledged, at the end 6 k for the heads' sums: 66 k in bf16.
+// 3 k (fp32 11 k), then per layer 1.2 k (fp32 1.8 k) until the neighbours' flags are seen, 0.5 k (fp32 1 k) until their squares are in LDS,
+// the MFMAs (bf16 0.5-2.1 k, fp32 2.8-6.9 k: three per product) and 1.3 k (fp32 2.6-2.9 k: two parts and the range) until the outputs are
+// stored and acknowledged, at the end 6 k (fp32 13 k) for the heads' sums: 66 k in bf16, 112 k in fp32.
 //
 // The exchange: loads of activations and flags carry the device-scope cache policy (sc1).  So do stores until a
 // workgroup has seen that all of its team run on its own XCD (each leaves its XCD's number beside the flags): from
@@ -20,7 +20,7 @@
 // store, wait for the acknowledgement, flag, load: 4 KB a side 2.2 us with the stores going through to memory, 1.1 us
 // with stores that stay in L2; 12 KB 3.9 and 1.9 us; 0.3 KB 1.5 and 0.7 us.  (Each word with its tag beside it, no
 // flag and no wait, 1.0, 2.0 and 0.5 us: not worth twice the words and memory of its own.)  One board's forward 35.8 ->
-// 30.1 us in bf16, 65.5 -> 58.9 us in fp32, 53 fp32 boards 121 -> 115 us, with what else changed there: weights asked for in front
+// 30.1 us in bf16, with what else changed there: weights asked for in front
 // of the wait, addresses of exchanged squares formed once, biases and head weights from LDS.
 //
 // Nothing waits for a workgroup that may not be running: a wait is bounded, and a workgroup whose
@@ -82,16 +82,25 @@ template <class P> struct TeamGeo {
 // tiles of squares each, whose four waves take PT of them and form CG groups of cout tiles.  A wave takes two
 // tiles of squares where there are two: with six workgroups each weight is then read by one wave, with three
 // by two; with one tile of squares per wave it would be twice as many, 96 and 128 bytes a cycle where the L1
-// gives 64 (six workgroups, 22 to 42 boards, bf16 + fp6 62.6 -> 55 us).  (fp32 takes one
-// tile of squares per wave: all four waves then have work in layers of two cout tiles.  Three workgroups per board ask for 85 bytes
-// a cycle in layers of three, where the L1 bounds the contractions.)
-// Three or six tiles of squares go to three waves, all cout tiles in each; the fourth watches the flags.
+// gives 64 (six workgroups, 22 to 42 boards, bf16 + fp6 62.6 -> 55 us).
+// Three tiles of squares go to three waves, all cout tiles in each; the fourth watches the flags.
+// fp32, four or six tiles of squares (RAGGED): a wave takes half of them (PR).  Of two cout tiles it takes one; of three, one for all its
+// squares and the middle one for half of them, which balances the waves (nine tiles' MFMAs in each per k-step of four tiles of squares, fifteen of six:
+// the fourth group takes one of them a second time, to the same bytes) and has 64 bytes of weights a cycle or less asked for.  One cout
+// tile: the tiles of squares are dealt out to the waves.  (All cout tiles of one tile of squares per wave were 85 bytes a cycle, and two of
+// squares in three waves left one idle: 53 boards 96 -> 88 us, 85 boards 104 -> 95 us, 100 boards 132 -> 121 us, 128 boards 140 -> 130 us.)
 template <class P, int TEAM> struct TeamShape {
   static constexpr int PXT = 12 / TEAM;
-  static constexpr int PT = PXT == 6 ? 2 : (PXT % 2 == 0 && !TeamGeo<P>::SPLIT ? 2 : 1), PG = PXT / PT;
+  static constexpr bool RAGGED = TeamGeo<P>::SPLIT && PXT >= 4;
+  static constexpr int PR = RAGGED ? PXT / 2 : 0;
+  static constexpr int PT = RAGGED ? PR : (PXT % 2 == 0 && !TeamGeo<P>::SPLIT ? 2 : 1), PG = PXT / PT;
   static constexpr int CG = PG == 3 ? 1 : (PG == 1 ? (PXT == 1 ? 3 : 4) : 4 / PG);   // groups of squares' tiles, of cout tiles
-  static constexpr int tiles(int nt) { return (nt + CG - 1) / CG; }   // cout tiles of a wave
+  static constexpr int tiles(int nt) { return RAGGED ? (nt == 3 ? 2 : 1) : (nt + CG - 1) / CG; }   // cout tiles of a wave
+  // ... and of its pairs of a tile of squares and a cout tile, tiles of squares: all cout tiles of each, or (RAGGED) one: team_used()
+  static constexpr int squares(int nt) { return !RAGGED ? PT : (nt == 3 ? PR + (PR + 1) / 2 : (nt == 2 ? PR : (PXT + 3) / 4)); }
 };
+// does a wave have cout tile t of tile of squares p? (PR: of a ragged shape)
+template <int PR> constexpr bool team_used(int p, int t) { return PR == 0 || t == (p < PR ? 0 : 1); }
 
 // fragment (k-step k, cout tile t) of 3x3 layer L in the weight stream of mode P: first of its planes
 template <class P, int L> __device__ __forceinline__ int team_frag(int k, int t) {
@@ -109,14 +118,15 @@ template <class P, int L> __device__ __forceinline__ int team_frag(int k, int t)
 // k-steps of weights that a wave keeps in flight: the loads take some 800 cycles and a k-step is
 // 32 cycles per MFMA
 template <class P, int TT, int PT> constexpr int team_ring() {
-  if (TeamGeo<P>::SPLIT) return PT > 1 ? 2 : (TT == 1 ? 9 : (TT == 2 ? 6 : 3));
+  // (fp32: three MFMAs per tile, PT of them in a ragged shape)
+  if (TeamGeo<P>::SPLIT) return PT * TT == 1 ? 9 : (PT >= 5 ? 2 : (PT >= 3 ? 3 : 6));
   return Geo<P>::W == 1 ? 18 / TT : (TT == 1 ? 9 : (TT == 2 ? 6 : 3));
 }
 // ... and those of one unrolled round: a phase in the pipelined modes; fp32: a kernel row, or all three of them where a k-step is
 // so short that nine are in flight
 template <class P, int L, int TT, int PT> constexpr int team_round() {
   if (P::PIPE) return kPhaseSteps;
-  return (TT == 1 && PT == 1 ? 9 : 3) * kCinArr[L] / 16;
+  return (PT * TT == 1 ? 9 : 3) * kCinArr[L] / 16;
 }
 
 // Low-order (fp6) pass of layer L for PT tiles of squares, conv3_lo_pass with TT cout tiles from t0 on.
@@ -164,14 +174,14 @@ __device__ __forceinline__ void team_lo_pass(const unsigned char *smem, const un
   });
 }
 
-// The contraction of 3x3 layer L for PT tiles of 32 squares and TT cout tiles from t0 on (tiles beyond
-// the layer's last repeat it; their results are not used).
+// The contraction of 3x3 layer L for PT tiles of 32 squares and TT cout tiles, tile(t) of the layer's (beyond
+// its last they repeat it; their results are not used).
 //   rec: LDS addresses of the lane's squares' records;  acc: the bias on entry
 //   fp32 (as half_layer): low: what the bias leaves out, for the small products' sum
-template <class P, int L, int TT, int PT>
+template <class P, int L, int TT, int PT, int PR, class Tile>
 __device__ __forceinline__ void team_conv(const unsigned char *smem, const unsigned char *packed, const WFrags &wl,
                                           v4i (&ring)[team_ring<P, TT, PT>()][TT][TeamGeo<P>::WPL], int lane,
-                                          const int (&rec)[PT], int t0, f32x16 (&acc)[PT][TT],
+                                          const int (&rec)[PT], Tile tile, f32x16 (&acc)[PT][TT],
                                           f32x16 (&low)[PT][TT]) {
   using T = TeamGeo<P>;
   constexpr int NT = kCoutArr[L] / 32, NTP = kCinArr[L] / 32;
@@ -192,8 +202,8 @@ __device__ __forceinline__ void team_conv(const unsigned char *smem, const unsig
     const int base = P::PIPE ? r * 64 : r * kPitch * T::RECB;
     return *reinterpret_cast<const v4i *>(smem + corner[p] + base + off + pl * 192);
   };
-  // activations two k-steps ahead; one where that is eighteen MFMAs (and registers are short)
-  constexpr int AHEAD = T::SPLIT && PT > 1 ? 1 : 2;
+  // activations two k-steps ahead; one where that is nine MFMAs or more
+  constexpr int AHEAD = T::SPLIT && PT > 2 ? 1 : 2;
   v4i a[AHEAD + 1][PT][NPL];
 #pragma unroll
   for (int v = 0; v < AHEAD; ++v)
@@ -205,7 +215,7 @@ __device__ __forceinline__ void team_conv(const unsigned char *smem, const unsig
   auto round = [&](int r) __attribute__((always_inline)) {
     // (the low-order pass comes in front of the last phase, as in pipe_layer)
     if constexpr (LO) {
-      if (r == NTP - 1) team_lo_pass<P, L, TT, PT>(smem, packed, lane, rec, t0, acc);
+      if (r == NTP - 1) team_lo_pass<P, L, TT, PT>(smem, packed, lane, rec, tile(0), acc);
     }
     static_for<0, U>([&](auto vc) __attribute__((always_inline)) {
       constexpr int v = decltype(vc)::value;
@@ -217,7 +227,7 @@ __device__ __forceinline__ void team_conv(const unsigned char *smem, const unsig
         for (int i = 0; i < NPL; ++i) a[(v + AHEAD) % (AHEAD + 1)][p][i] = frag(rn, (v + AHEAD) % U, p, i);
       auto refill = [&](int t) __attribute__((always_inline)) {
         const int kn = r * U + v + D;   // (behind the last k-steps: the last one again, unused)
-        const int f = team_frag<P, L>(kn < KS ? kn : KS - 1, t0 + t < NT ? t0 + t : NT - 1);
+        const int f = team_frag<P, L>(kn < KS ? kn : KS - 1, tile(t) < NT ? tile(t) : NT - 1);
 #pragma unroll
         for (int i = 0; i < W; ++i) ring[v % D][t][i] = wl[f + i];
       };
@@ -239,16 +249,19 @@ __device__ __forceinline__ void team_conv(const unsigned char *smem, const unsig
           for (int n = 0; n < (TURNS ? TT : 3); ++n) {
             const int m = TURNS ? o : n, t = TURNS ? n : o;
 #pragma unroll
-            for (int p = 0; p < PT; ++p) mma<P>(ring[v % D][t][WP[m]], a[v % (AHEAD + 1)][p][AP[m]], m == 1 ? sum[p][t] : low[p][t]);
+            for (int p = 0; p < PT; ++p)
+              if (team_used<PR>(p, t)) mma<P>(ring[v % D][t][WP[m]], a[v % (AHEAD + 1)][p][AP[m]], m == 1 ? sum[p][t] : low[p][t]);
             if (m == 2) refill(t);
           }
         if constexpr ((v + 1) % (3 * KC) == 0) {
 #pragma unroll
           for (int p = 0; p < PT; ++p)
 #pragma unroll
-            for (int t = 0; t < TT; ++t)
+            for (int t = 0; t < TT; ++t) {
+              if (!team_used<PR>(p, t)) continue;
 #pragma unroll
               for (int e = 0; e < 16; ++e) acc[p][t][e] = fmaf(sum[p][t][e], kHalfUnit, acc[p][t][e]);
+            }
         }
       } else {
 #pragma unroll
@@ -275,6 +288,7 @@ __device__ __forceinline__ void team_conv(const unsigned char *smem, const unsig
     for (int p = 0; p < PT; ++p)
 #pragma unroll
       for (int t = 0; t < TT; ++t) {
+        if (!team_used<PR>(p, t)) continue;
         asm volatile("" : "+a"(low[p][t]));
 #pragma unroll
         for (int e = 0; e < 16; ++e) acc[p][t][e] = fmaf(low[p][t][e], kHalfUnit / kHalfLow, acc[p][t][e]);
@@ -372,7 +386,7 @@ __device__ __forceinline__ void team_board(const TeamParams &prm, unsigned char 
   using G = Geo<P>;
   using T = TeamGeo<P>;
   using S = TeamShape<P, TEAM>;
-  constexpr int NPL = T::NPL, W = G::W, WPL = T::WPL, THREADS = 256, PXT = S::PXT, PT = S::PT, CG = S::CG;
+  constexpr int NPL = T::NPL, W = G::W, WPL = T::WPL, THREADS = 256, PXT = S::PXT, CG = S::CG;
   std::conditional_t<T::SPLIT, int, const int> tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), h = lane >> 5;
   const FwdParams &f = prm.f;
@@ -422,7 +436,7 @@ __device__ __forceinline__ void team_board(const TeamParams &prm, unsigned char 
   };
 
   // the wave's first tile of squares within the workgroup's, and its group of cout tiles
-  const int wpx = wave % S::PG * PT, cg = wave / S::PG;
+  const int wpx = wave % S::PG * S::PT, cg = wave / S::PG;
 
   // word l * 12 + role: the squares of stage l that the neighbours read are there; kTeamAll further on:
   // all of them
@@ -507,8 +521,8 @@ __device__ __forceinline__ void team_board(const TeamParams &prm, unsigned char 
   auto part_lds = [](int k, int j) __attribute__((always_inline)) { return (k < NPL ? k * 192 : T::LO_OFF) + j * 16; };
 
   // Outputs of layer L (own squares): into the records, and to memory what the neighbours read.
-  // acc: N tiles of squares from the workgroup's tile px on
-  auto write_out = [&](auto lc, auto nc, int role, const Span &sp, bool active, const auto &acc, int px, int t0) __attribute__((always_inline)) {
+  // acc: N tiles of squares, px(i) of the workgroup's, and a wave's cout tiles, tile(t) of the layer's
+  auto write_out = [&](auto lc, auto nc, int role, const Span &sp, bool active, const auto &acc, auto px, auto tile) __attribute__((always_inline)) {
     constexpr int L = decltype(lc)::value, N = decltype(nc)::value, C = kCoutArr[L], NT = C / 32;
     constexpr int TT = S::tiles(NT);
     constexpr bool LO = P::LO6 && ((P::LO_MASK >> (L + 1)) & 1);
@@ -516,11 +530,15 @@ __device__ __forceinline__ void team_board(const TeamParams &prm, unsigned char 
     if (active) {
 #pragma unroll
       for (int i = 0; i < N; ++i) {
-        const int p = sp.p0 + (px + i) * 32 + (lane & 31), pc = p < kPix ? p : kPix - 1;
+        const int p = sp.p0 + px(i) * 32 + (lane & 31), pc = p < kPix ? p : kPix - 1;
         const int rec = record(pc, sp.base);
 #pragma unroll
-        for (int t = 0; t < TT; ++t)
-          if (t0 + t < NT) team_store<P, LO, (L >= 2)>(smem, rec, h, t0 + t, acc[i][t], most);
+        for (int t = 0; t < TT; ++t) {
+          if constexpr (S::RAGGED && L > 0) {
+            if (!team_used<S::PR>(i, t)) continue;
+          }
+          if (tile(t) < NT) team_store<P, LO, (L >= 2)>(smem, rec, h, tile(t), acc[i][t], most);
+        }
       }
     }
     if constexpr (T::SPLIT) store_note(L, role, most, L == 0 && bad_input);
@@ -552,13 +570,24 @@ __device__ __forceinline__ void team_board(const TeamParams &prm, unsigned char 
 
   auto conv_stage = [&](auto lc, int role) __attribute__((always_inline)) -> bool {
     constexpr int L = decltype(lc)::value;
-    constexpr int NT = kCoutArr[L] / 32, TT = S::tiles(NT), D = team_ring<P, TT, PT>();
+    constexpr int NT = kCoutArr[L] / 32, TT = S::tiles(NT), PT = S::squares(NT), D = team_ring<P, TT, PT>();
     constexpr int C = kCinArr[L];
     // (opaque per stage: what follows from it is formed here and not, for all stages, in front of the
     // loop over them, in several hundred scalar registers that get spilled)
-    int t0 = cg * TT;
+    int t0 = S::RAGGED ? cg : cg * TT;
     asm volatile("" : "+s"(t0));
-    const bool active = cg < CG && t0 < NT;
+    const bool active = S::RAGGED ? NT > 1 || wave * PT < PXT : cg < CG && t0 < NT;
+    // the wave's cout tiles (one beyond the layer's last repeats it, and is not used) and tiles of squares
+    auto tile = [&](int t) __attribute__((always_inline)) {
+      if constexpr (S::RAGGED) return NT == 3 ? (t == 0 ? 2 * t0 : 1) : (NT == 2 ? t0 : 0);
+      else return t0 + t;
+    };
+    auto tile_or_last = [&](int t) __attribute__((always_inline)) { return tile(t) < NT ? tile(t) : NT - 1; };
+    auto px = [&](int i) __attribute__((always_inline)) {
+      if constexpr (!S::RAGGED) return wpx + i;
+      else if constexpr (NT == 1) return wave * PT + i;
+      else return wpx + (i < S::PR ? i : (t0 == 0 ? i - S::PR : 2 * S::PR - 1 - i));
+    };
     const Span sp = span_of(role);
     const WFrags wl = layer_weights<P, L>(packed, lane);
     C6_MARK(6 * L);
@@ -571,7 +600,7 @@ __device__ __forceinline__ void team_board(const TeamParams &prm, unsigned char 
 #pragma unroll
         for (int t = 0; t < TT; ++t)
 #pragma unroll
-          for (int i = 0; i < WPL; ++i) ring[d][t][i] = wl[team_frag<P, L>(d, t0 + t < NT ? t0 + t : NT - 1) + i];
+          for (int i = 0; i < WPL; ++i) ring[d][t][i] = wl[team_frag<P, L>(d, tile_or_last(t)) + i];
       __builtin_amdgcn_sched_barrier(0);
     };
     // (on their way while the neighbours are waited for; the wave that does the waiting asks for its own behind that)
@@ -614,9 +643,10 @@ __device__ __forceinline__ void team_board(const TeamParams &prm, unsigned char 
     if (active) {
 #pragma unroll
       for (int t = 0; t < TT; ++t) {
-        const int word = bias_offset(L) + 32 * (t0 + t < NT ? t0 + t : NT - 1);
+        const int word = bias_offset(L) + 32 * tile_or_last(t);
 #pragma unroll
         for (int i = 0; i < PT; ++i) {
+          if (!team_used<S::PR>(i, t)) continue;
           acc[i][t] = tail_tile(word);
           if constexpr (T::SPLIT) low[i][t] = tail_tile(G::TAIL_BIAS_LOW + word);
         }
@@ -629,52 +659,45 @@ __device__ __forceinline__ void team_board(const TeamParams &prm, unsigned char 
     bool ok[PT];
 #pragma unroll
     for (int i = 0; i < PT; ++i) {
-      p[i] = sp.p0 + (wpx + i) * 32 + (lane & 31);
+      p[i] = sp.p0 + px(i) * 32 + (lane & 31);
       ok[i] = p[i] < kPix;
       rec[i] = record(ok[i] ? p[i] : kPix - 1, sp.base);
     }
-    if (active) team_conv<P, L, TT, PT>(smem, packed, wl, ring, lane, rec, t0, acc, low);
+    if (active) team_conv<P, L, TT, PT, S::PR>(smem, packed, wl, ring, lane, rec, tile, acc, low);
     C6_MARK(6 * L + 3);
     if constexpr (L < 7) {
       __syncthreads();   // everybody has read this layer's input
-      write_out(lc, IC<PT>{}, role, sp, active, acc, wpx, t0);
+      write_out(lc, IC<PT>{}, role, sp, active, acc, px, tile);
     } else {
       // heads: this wave's share of the policy (per square) and of the value
       const float *pw = tail + kBiasTotal + 4 * h;
-      const int tile = role * PXT + wpx;   // of the twelve
       if constexpr (T::SPLIT) {
         float most = 0.0f;
         if (active) {
 #pragma unroll
           for (int t = 0; t < TT; ++t) {
-            if (t0 + t >= NT) continue;
-            float pol[PT], val[PT];
-#pragma unroll
-            for (int i = 0; i < PT; ++i) pol[i] = val[i] = 0.0f;
+            if (tile(t) >= NT) continue;
             HalfHeads out;
-            out.pw = tail_tile(kBiasTotal + 32 * (t0 + t));
-            out.vw = tail_tile(kBiasTotal + kHeadC + 32 * (t0 + t));
+            out.pw = tail_tile(kBiasTotal + 32 * tile(t));
+            out.vw = tail_tile(kBiasTotal + kHeadC + 32 * tile(t));
 #pragma unroll
             for (int i = 0; i < PT; ++i) {
+              if (!team_used<S::PR>(i, t)) continue;
               out.pol = out.val = 0.0f;
               HalfEpi<true>::run(acc[i][t], out, most);
-              pol[i] = out.pol;
-              val[i] = out.val;
-            }
-#pragma unroll
-            for (int i = 0; i < PT; ++i) {
-              const unsigned bits = __builtin_bit_cast(unsigned, pol[i]);
+              const unsigned bits = __builtin_bit_cast(unsigned, out.pol);
               const auto x = __builtin_amdgcn_permlane32_swap(bits, bits, false, false);
               const unsigned x0 = x[0], x1 = x[1];
               const float tot = __builtin_bit_cast(float, x0) + __builtin_bit_cast(float, x1);
-              const float vs = wave_sum(ok[i] ? val[i] : 0.0f);
-              if (h == 0 && ok[i]) store4(tot, T::HEAD_OFF + ((t0 + t) * 384 + p[i]) * 4);
-              if (lane == 0) store4(vs, T::VAL_OFF + ((t0 + t) * 12 + tile + i) * 4);
+              const float vs = wave_sum(ok[i] ? out.val : 0.0f);
+              if (h == 0 && ok[i]) store4(tot, T::HEAD_OFF + (tile(t) * 384 + p[i]) * 4);
+              if (lane == 0) store4(vs, T::VAL_OFF + (tile(t) * 12 + role * PXT + px(i)) * 4);
             }
           }
         }
         store_note(L, role, most, false);
       } else {
+        const int first = role * PXT + wpx;   // of the twelve tiles of squares
         // The one-workgroup kernel runs one chain of multiply-adds over the channels of a lane's
         // square, cout tile after cout tile: the groups of cout tiles take turns and hand it on.
         float *chain = reinterpret_cast<float *>(smem + T::OCC_OFF);   // (not in use before the last stage)
@@ -706,12 +729,12 @@ __device__ __forceinline__ void team_board(const TeamParams &prm, unsigned char 
                   vs = fmaf(a, vw4[e], vs);
                 }
                 // (tile 0: one chain over its sixteen channels; the others: one sum per four)
-                if (t0 + t > 0) store4(vs, T::VAL_OFF + (((tile + i) * 9 + 1 + 4 * (t0 + t - 1) + q) * 64 + lane) * 4);
+                if (t0 + t > 0) store4(vs, T::VAL_OFF + (((first + i) * 9 + 1 + 4 * (t0 + t - 1) + q) * 64 + lane) * 4);
               }
             }
 #pragma unroll
             for (int i = 0; i < PT; ++i)
-              if (t0 + t == 0) store4(val0[i], T::VAL_OFF + ((tile + i) * 9 * 64 + lane) * 4);
+              if (t0 + t == 0) store4(val0[i], T::VAL_OFF + ((first + i) * 9 * 64 + lane) * 4);
           }
         }
 #pragma unroll
@@ -969,7 +992,7 @@ __device__ __forceinline__ void team_board(const TeamParams &prm, unsigned char 
     C6_MARK(2);
     __syncthreads();   // the copies give way to the activations
     clear_region(sp);
-    write_out(IC<0>{}, IC<N1>{}, role, sp, active, acc, px, 0);
+    write_out(IC<0>{}, IC<N1>{}, role, sp, active, acc, [&](int i) { return px + i; }, [](int t) { return t; });
     C6_MARK(3);
     return true;
   };
@@ -983,6 +1006,11 @@ __device__ __forceinline__ void team_board(const TeamParams &prm, unsigned char 
     const int got = wait_inputs(8, role, true);
     if (got != 1) return got == 2;
     region_role = -1;
+    const float *valw = tail + kBiasTotal + kHeadC;
+    const float polb = valw[kHeadC], valb = valw[kHeadC + 1];
+    auto partial = [&](int at) __attribute__((always_inline)) {
+      return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(mem, at, 0, kSc1));
+    };
     if constexpr (T::SPLIT) {
       unsigned note = 0;
       for (int i = tid; i < 8 * TEAM * 4; i += THREADS) {
@@ -991,11 +1019,6 @@ __device__ __forceinline__ void team_board(const TeamParams &prm, unsigned char 
       }
       if (note != 0) atomicOr(check, note);
     }
-    const float *valw = tail + kBiasTotal + kHeadC;
-    const float polb = valw[kHeadC], valb = valw[kHeadC + 1];
-    auto partial = [&](int at) __attribute__((always_inline)) {
-      return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(mem, at, 0, kSc1));
-    };
     const bool state = f.x_dtype == C6_DT_BOARD_I8;
     long long src = state && f.index ? f.index[b] : (long long)b;
     if (state) src = src < 0 ? 0 : (src >= f.num_states ? f.num_states - 1 : src);
@@ -1139,7 +1162,7 @@ __device__ __forceinline__ void team_board(const TeamParams &prm, unsigned char 
 // that beats one workgroup (1: the one-workgroup kernels).  With fewer workgroups per board more waves read
 // the same weights, and the L1's 64 bytes a cycle bound the layers; the 16-bit one-workgroup kernel hides its epilogues
 // behind its MFMAs, which a team does not.  Measured, us, teams of 12 / 6 / 3 / 2 against one workgroup each, boards:
-//   fp32  16: 66 / 82 / 110 / 178 / 223   40: 97 / 116 / 181 / 224   80: 132 / 185 / 224   128: 203 / 230
+//   fp32  16: 52 / 68 / 83 / 108 / 192   40: 74 / 87 / 112 / 192 (without 12)   80: 103 / 119 / 192   128: 146 / 192
 //   bf16  16: 31 / 41 / 49 / 61 / 45      21: 36 / 41 / - / - / 46   40: 42 / 50 / 61 / 45   42: 48 (teams on two XCDs)
 //   bf16 + fp6  21: 44 / 51 / 64 / 81 / 63    42: 57 / 68 / 84 / 64    with low weights  21: 52 / 60 / 78 / 101 / 89
 //   42: 67 / 84 / 106 / 89    72: 89 / 110 / 89 (behind a first pass, 53 listed boards, 85 against 110)

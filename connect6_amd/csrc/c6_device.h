@@ -73,6 +73,27 @@ __device__ __forceinline__ float wave_sum(float v) {
     return __builtin_bit_cast(int, __builtin_bit_cast(float, a) + __builtin_bit_cast(float, b));
   }));
 }
+// The same of 64-bit numbers: their two halves move as words.
+__device__ __forceinline__ double wave_sum_f64(double v) {
+  auto step = [](double x, auto move) {
+    const unsigned long long b = __builtin_bit_cast(unsigned long long, x);
+    const unsigned lo = move((unsigned)b), hi = move((unsigned)(b >> 32));
+    return x + __builtin_bit_cast(double, (unsigned long long)hi << 32 | lo);
+  };
+  v = step(v, [](unsigned w) { return (unsigned)__builtin_amdgcn_update_dpp((int)w, (int)w, 0xB1, 0xF, 0xF, false); });
+  v = step(v, [](unsigned w) { return (unsigned)__builtin_amdgcn_update_dpp((int)w, (int)w, 0x4E, 0xF, 0xF, false); });
+  v = step(v, [](unsigned w) { return (unsigned)__builtin_amdgcn_update_dpp((int)w, (int)w, 0x141, 0xF, 0xF, false); });
+  v = step(v, [](unsigned w) { return (unsigned)__builtin_amdgcn_update_dpp((int)w, (int)w, 0x140, 0xF, 0xF, false); });
+  // (lane 0's row; the other rows' sums from their first lanes)
+  const unsigned long long b = __builtin_bit_cast(unsigned long long, v);
+  double rows[4];
+#pragma unroll
+  for (int r = 0; r < 4; ++r) {
+    const unsigned lo = __builtin_amdgcn_readlane((unsigned)b, 16 * r), hi = __builtin_amdgcn_readlane((unsigned)(b >> 32), 16 * r);
+    rows[r] = __builtin_bit_cast(double, (unsigned long long)hi << 32 | lo);
+  }
+  return (rows[0] + rows[1]) + (rows[2] + rows[3]);
+}
 __device__ __forceinline__ float wave_max(float v) {
   return __builtin_bit_cast(float, wave_allreduce_bits(__builtin_bit_cast(int, v), [](int a, int b) {
     return __builtin_bit_cast(int, fmaxf(__builtin_bit_cast(float, a), __builtin_bit_cast(float, b)));

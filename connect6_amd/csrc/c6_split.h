@@ -395,12 +395,10 @@ __device__ __forceinline__ void split_layer(unsigned char *smem, const unsigned 
   __syncthreads();
 }
 
-// the value head's sum over (cout tile, tile of 32 squares).  (In 64 bits: 36 additions in fp32 were most of the value's error,
-// 2.5e-10 rms of values of 6e-4 with the reference's initialisation.)
-__device__ __forceinline__ double split_value_sum(const float *part) {
-  double s = 0.0;
-  for (int i = 0; i < 36; ++i) s += (double)part[i];
-  return s;
+// the value head's sum over (cout tile, tile of 32 squares), part(i) of a whole wave's lanes i < 36.  (In 64 bits: 36 additions in
+// fp32 were most of the value's error, 2.5e-10 rms of values of 6e-4 with the reference's initialisation.)
+template <class Part> __device__ __forceinline__ double split_value_sum(int lane, Part part) {
+  return wave_sum_f64(lane < 36 ? (double)part(lane) : 0.0);
 }
 
 // ---- what c6_half.h shares ----
@@ -489,7 +487,10 @@ struct SplitHeads {
 // ---- write out: value, masked logits, optional sampled action ----
 __device__ __forceinline__ void split_write(const FwdParams &prm, long long b, int tid, int lane, int wave, const unsigned char *occ,
                                             const float *lgt, const float *red, float value_bias) {
-  if (tid == 0 && prm.value != nullptr) prm.value[b] = split_value(split_value_sum(red), value_bias);
+  if (prm.value != nullptr && wave == 3) {   // (beside the draw)
+    const double sum = split_value_sum(lane, [&](int i) { return red[i]; });
+    if (lane == 0) prm.value[b] = split_value(sum, value_bias);
+  }
   if (prm.logits != nullptr) {
     for (int p = tid; p < kPix; p += 256) static_cast<float *>(prm.logits)[(size_t)b * kPix + p] = occ[p] ? prm.fill : lgt[p];
   }

@@ -12,7 +12,7 @@
 // What it takes (cycles of a 2.4 GHz clock; twelve workgroups, one board): staging the input 7 k, the first layer
 // 3 k (fp32 11 k), then per layer 1.2 k (fp32 1.8 k) until the neighbours' flags are seen, 0.5 k (fp32 1 k) until their squares are in LDS,
 // the MFMAs (bf16 0.5-2.1 k, fp32 2.8-6.9 k: three per product) and 1.3 k (fp32 2.6-2.9 k: two parts and the range) until the outputs are
-// stored and acknowledged, at the end 6 k (fp32 13 k) for the heads' sums: 66 k in bf16, 112 k in fp32.
+// stored and acknowledged, at the end 6 k (fp32 11 k) for the heads' sums: 66 k in bf16, 110 k in fp32.
 //
 // The exchange: loads of activations and flags carry the device-scope cache policy (sc1).  So do stores until a
 // workgroup has seen that all of its team run on its own XCD (each leaves its XCD's number beside the flags): from
@@ -428,11 +428,14 @@ __device__ __forceinline__ void team_board(const TeamParams &prm, unsigned char 
     else __hip_atomic_store(&flags[word], prm.tag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   };
   [[maybe_unused]] const bool trace_on = true;
-  // fp32: what this wave stored of layer l of role's squares (nothing: 0), for the last stage
+  // fp32: what this wave knows of the numbers in role's squares up to layer l (half_note); a word per layer, so that whoever
+  // goes on with another's squares finds it
   bool bad_input = false;
+  [[maybe_unused]] unsigned trail = 0;
+  auto note_at = [&](int l, int role) { return T::NOTE_OFF + ((l * 12 + role) * 4 + wave) * 4; };
   auto store_note = [&](int l, int role, float most, bool bad) __attribute__((always_inline)) {
-    const unsigned note = half_note(l, most) | (bad ? 1u : 0u);
-    if (lane == 0) store4(__builtin_bit_cast(float, note), T::NOTE_OFF + ((l * 12 + role) * 4 + wave) * 4);
+    trail = (l > 0 ? trail : 0) | half_note(l, most) | (bad ? 1u : 0u);
+    if (lane == 0) store4(__builtin_bit_cast(float, trail), note_at(l, role));
   };
 
   // the wave's first tile of squares within the workgroup's, and its group of cout tiles
@@ -640,6 +643,9 @@ __device__ __forceinline__ void team_board(const TeamParams &prm, unsigned char 
         to_region(q, v);
       }
     region_role = -1;   // (until the outputs are in place)
+    if constexpr (T::SPLIT) {
+      if (!own) trail = (unsigned)__builtin_amdgcn_raw_buffer_load_b32(mem, note_at(L - 1, role), 0, kSc1);
+    }
     if (active) {
 #pragma unroll
       for (int t = 0; t < TT; ++t) {
@@ -1011,22 +1017,29 @@ __device__ __forceinline__ void team_board(const TeamParams &prm, unsigned char 
     auto partial = [&](int at) __attribute__((always_inline)) {
       return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(mem, at, 0, kSc1));
     };
+    // fp32: everything that is read here is asked for at once, and the value's sum runs beside the logits; a board's squares are
+    // known to be in range from the last layer's words alone (store_note).  (Words of all layers, then logits, then the value's
+    // 36 sums one after the other in one lane: 21 boards 59.1 -> 56.8 us, 42 boards 79 -> 77 us, one board 48.7 -> 47.8 us.)
+    [[maybe_unused]] float head[2][3], val = 0.0f;
+    [[maybe_unused]] unsigned note = 0;
     if constexpr (T::SPLIT) {
-      unsigned note = 0;
-      for (int i = tid; i < 8 * TEAM * 4; i += THREADS) {
-        const int l = i / (TEAM * 4), j = i - l * (TEAM * 4);
-        note |= (unsigned)__builtin_amdgcn_raw_buffer_load_b32(mem, T::NOTE_OFF + (l * 48 + j) * 4, 0, kSc1);
-      }
+#pragma unroll
+      for (int k = 0; k < 2; ++k)
+#pragma unroll
+        for (int t = 0; t < 3; ++t) head[k][t] = partial(T::HEAD_OFF + (t * 384 + (tid + k * THREADS) % 384) * 4);   // (beyond 360: unused)
+      if (wave == 3) val = lane < 36 ? partial(T::VAL_OFF + lane * 4) : 0.0f;
+      else if (tid < TEAM * 4) note = __builtin_bit_cast(unsigned, partial(T::NOTE_OFF + (7 * 48 + tid) * 4));
+      __builtin_amdgcn_sched_barrier(0);
       if (note != 0) atomicOr(check, note);
+      if (wave == 3 && f.value != nullptr) {   // (the sum needs its lanes together)
+        const double sum = split_value_sum(lane, [&](int) { return val; });
+        if (lane == 0) f.value[b] = split_value(sum, valb);
+      }
     }
     const bool state = f.x_dtype == C6_DT_BOARD_I8;
     long long src = state && f.index ? f.index[b] : (long long)b;
     if (state) src = src < 0 ? 0 : (src >= f.num_states ? f.num_states - 1 : src);
-    for (int p = tid; p < kPix; p += THREADS) {
-      float z = partial(T::HEAD_OFF + p * 4);
-      if constexpr (T::SPLIT) z = (z + partial(T::HEAD_OFF + (384 + p) * 4)) + partial(T::HEAD_OFF + (768 + p) * 4);
-      if constexpr (T::SPLIT) z = split_logit(z, polb);
-      else z += polb;
+    auto put = [&](int p, float z) __attribute__((always_inline)) {
       bool taken;
       if (f.mask_mode == C6_MASK_LEGAL) {
         taken = f.legal[(size_t)b * kPix + p] == 0;
@@ -1047,10 +1060,15 @@ __device__ __forceinline__ void team_board(const TeamParams &prm, unsigned char 
         else if (f.logits_dtype == C6_DT_BF16) static_cast<unsigned short *>(f.logits)[at] = __builtin_bit_cast(unsigned short, (__bf16)v);
         else static_cast<unsigned short *>(f.logits)[at] = __builtin_bit_cast(unsigned short, (_Float16)v);
       }
-    }
+    };
     if constexpr (T::SPLIT) {
-      if (tid < 36) red[tid] = partial(T::VAL_OFF + tid * 4);
+#pragma unroll
+      for (int k = 0; k < 2; ++k)
+        if (tid + k * THREADS < kPix) put(tid + k * THREADS, split_logit((head[k][0] + head[k][1]) + head[k][2], polb));
     } else {
+      for (int p = tid; p < kPix; p += THREADS) put(p, partial(T::HEAD_OFF + p * 4) + polb);
+    }
+    if constexpr (!T::SPLIT) {
       // as lane `lane` of wave `wave` of the one-workgroup kernel adds its three squares' sums up
       float part[3][9], vsum = 0.0f;
       bool valid[3];
@@ -1068,10 +1086,8 @@ __device__ __forceinline__ void team_board(const TeamParams &prm, unsigned char 
       if (lane == 0) red[wave] = vsum;
     }
     __syncthreads();
-    if (tid == 192 && f.value != nullptr) {   // (beside the draw and the margin)
-      if constexpr (T::SPLIT) {
-        f.value[b] = split_value(split_value_sum(red), valb);
-      } else {
+    if constexpr (!T::SPLIT) {
+      if (tid == 192 && f.value != nullptr) {   // (beside the draw and the margin)
         float s = 0.0f;
 #pragma unroll
         for (int w = 0; w < 4; ++w) s += red[w];
@@ -1107,7 +1123,7 @@ __device__ __forceinline__ void team_board(const TeamParams &prm, unsigned char 
         }
       }
     }
-    raise_flag(8, role);
+    if constexpr (!T::SPLIT) raise_flag(8, role);   // (fp32: nobody waits for it)
     C6_MARK(49);
     return true;
   };

@@ -2313,17 +2313,17 @@ template <class P> int launch_left(const FwdParams &fp, int cus, hipStream_t st)
 
 #if defined(C6_TEAM) || defined(C6_CASCADE) || !defined(C6_INSTANCE)
 template <class P> int launch_team(const TeamParams &tp, int grid, hipStream_t st) {
-  using T = TeamGeo<P>;
+  constexpr int A = TeamGeo<P>::LDS_BYTES, B = TeamGeo<P>::SPLIT ? SplitGeo::LDS_BYTES : 0, LDS = A > B ? A : B;
   static thread_local int configured = -1;
   int dev = 0;
   hipError_t e = hipGetDevice(&dev);
   if (e == hipSuccess && configured != dev) {
     e = hipFuncSetAttribute(reinterpret_cast<const void *>(&team_forward_kernel<P>),
-                            hipFuncAttributeMaxDynamicSharedMemorySize, T::LDS_BYTES);
+                            hipFuncAttributeMaxDynamicSharedMemorySize, LDS);
     if (e == hipSuccess) configured = dev;
   }
   if (e == hipSuccess) {
-    hipLaunchKernelGGL(team_forward_kernel<P>, dim3((unsigned)grid), dim3(256), T::LDS_BYTES, st, tp);
+    hipLaunchKernelGGL(team_forward_kernel<P>, dim3((unsigned)grid), dim3(256), LDS, st, tp);
     e = hipGetLastError();
   }
   if (e != hipSuccess) {
@@ -2600,13 +2600,12 @@ int dispatch_team(int prec, const TeamParams &tp, hipStream_t st) {
   }
   if (shared < all) {
     part.f.total_boards = all - shared;
-    const int rc2 = dispatch_boards(prec, part.f, st);
+    const int rc2 = dispatch_forward(prec, part.f, st);
     if (rc2 != C6_OK) return rc2;
   }
   part.f.total_boards = shared;
   part.first = (unsigned)(all - shared);
-  const int rc3 = m.launch(part, cus, st);   // (workgroups without a board end at once)
-  return rc3 != C6_OK ? rc3 : dispatch_left(prec, tp.f, st);
+  return m.launch(part, cus, st);   // (workgroups without a board end at once)
 }
 
 // Cascade: every board through the plain bf16 kernel, whose workgroups list those of their boards

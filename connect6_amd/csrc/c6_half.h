@@ -405,7 +405,8 @@ __device__ __forceinline__ bool half_left(const FwdParams &prm, long long b) {
   return prm.actions != nullptr && prm.actions[b] == -1;
 }
 
-// The boards that half_forward_kernel left, one workgroup each; there are hardly ever any, and then this takes 4 us.
+// The boards that half_forward_kernel left, one workgroup each; there are hardly ever any, and then this takes 4 us, of which the
+// launch is most.  (Teams do without: team_forward_kernel.)
 template <class P> __global__ __launch_bounds__(256) void split_forward_kernel(const FwdParams prm) {
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
   // boards dealt out one by one; every wave looks at the same 64, so that all agree
@@ -414,7 +415,7 @@ template <class P> __global__ __launch_bounds__(256) void split_forward_kernel(c
     const long long mine = first + (threadIdx.x & 63) * grid;
     unsigned long long left = __builtin_amdgcn_ballot_w64(mine < prm.total_boards && half_left(prm, mine));
     if (left != 0) __syncthreads();   // (all have looked before an output is written)
-    for (; left != 0; left &= left - 1) split_board(prm, smem, first + __builtin_ctzll(left) * grid);
+    for (; left != 0; left &= left - 1) split_board<false>(prm, smem, first + __builtin_ctzll(left) * grid);
   }
 }
 

@@ -85,17 +85,18 @@ __device__ __forceinline__ void split_drop4(float (&v)[8], const int (&w)[4]) {
 
 // Weight ring of a 3x3 layer: two k-steps of all cout tiles and planes.  A k-step of NT cout tiles and N
 // pixel tiles is 6 NT N MFMAs, 192 NT N cycles, and a slot is refilled behind its last use.
-template <int NT> constexpr int kSplitRing = NT == 3 ? 1 : 2;
-template <int L> using SplitWeights = v4i[kSplitRing<kCoutArr[L] / 32>][kCoutArr[L] / 32][3];
+// (TN of its cout tiles, from T0 on.)
+template <int TN> constexpr int kSplitRing = TN == 3 ? 1 : 2;
+template <int TN> using SplitWeights = v4i[kSplitRing<TN>][TN][3];
 
-template <int L> __device__ __forceinline__ void split_preload(SplitWeights<L> &ring, const WFrags &wl) {
+template <int L, int T0, int TN> __device__ __forceinline__ void split_preload(SplitWeights<TN> &ring, const WFrags &wl) {
   constexpr int NT = kCoutArr[L] / 32;
 #pragma unroll
-  for (int d = 0; d < kSplitRing<NT>; ++d)
+  for (int d = 0; d < kSplitRing<TN>; ++d)
 #pragma unroll
-    for (int t = 0; t < NT; ++t)
+    for (int t = 0; t < TN; ++t)
 #pragma unroll
-      for (int i = 0; i < 3; ++i) ring[d][t][i] = wl[(d * NT + t) * 3 + i];
+      for (int i = 0; i < 3; ++i) ring[d][t][i] = wl[(d * NT + T0 + t) * 3 + i];
 }
 
 // Weights of one fragment, from the packed set's parts (half_parts) to three bf16 ones.  A weight beyond fp16 is marked and
@@ -174,11 +175,12 @@ __device__ __forceinline__ void mma_vector_wait(f32x16 &a, f32x16 &b) {
 // next k-step's activations, one weight load, and (96 input channels) a few instructions of their split.
 //   ring: the first k-steps on entry, those behind the layer's last at the end
 // The sums of three cout tiles are 288 registers: those of the last pixel tile's last cout tile are vector registers.
-template <int L>
+// TN of the layer's cout tiles, from T0 on.
+template <int L, int T0, int TN>
 __device__ __forceinline__ void split_conv(const unsigned char *smem, const WFrags &wl, const float *bias,
-                                           SplitWeights<L> &ring, const int (&ci)[3], int h,
-                                           f32x16 (&acc)[kCoutArr[L] / 32][3], f32x16 (&low)[kCoutArr[L] / 32][3]) {
-  constexpr int CIN = kCinArr[L], NT = kCoutArr[L] / 32, KC = CIN / 16, D = kSplitRing<NT>, N = 3;
+                                           SplitWeights<TN> &ring, const int (&ci)[3], int h,
+                                           f32x16 (&acc)[TN][3], f32x16 (&low)[TN][3]) {
+  constexpr int CIN = kCinArr[L], NT = kCoutArr[L] / 32, KC = CIN / 16, D = kSplitRing<TN>, N = 3;
   constexpr bool WIDE = CIN == 96;   // activations arrive as fp32
   static_assert(KC % 2 == 0 && KC % D == 0, "double buffers must line up across taps");
   int pb[N], xo[N];
@@ -231,10 +233,10 @@ __device__ __forceinline__ void split_conv(const unsigned char *smem, const WFra
     static_for<0, 16 * N>([&](auto ac) __attribute__((always_inline)) { split_some(0, ac); });
   }
 #pragma unroll
-  for (int t = 0; t < NT; ++t) {
+  for (int t = 0; t < TN; ++t) {
     f32x16 b[1], bl[1];
-    load_bias_tiles(b, bias + 32 * t, h);
-    load_bias_tiles(bl, bias + Geo<PrecF32S>::TAIL_BIAS_LOW + 32 * t, h);
+    load_bias_tiles(b, bias + 32 * (T0 + t), h);
+    load_bias_tiles(bl, bias + Geo<PrecF32S>::TAIL_BIAS_LOW + 32 * (T0 + t), h);
 #pragma unroll
     for (int j = 0; j < N; ++j) {
       acc[t][j] = b[0];
@@ -244,12 +246,12 @@ __device__ __forceinline__ void split_conv(const unsigned char *smem, const WFra
   constexpr int AHEAD = WIDE ? 2 : 1;
 #pragma unroll 1
   for (int tap = 0; tap < 9; ++tap) {
-    const WFrags wn = wl + (tap * KC + D) * NT * 3;
+    const WFrags wn = wl + ((tap * KC + D) * NT + T0) * 3;
     static_for<0, KC>([&](auto uc) __attribute__((always_inline)) {
       constexpr int u = decltype(uc)::value, par = u & 1;
       // (after the last tap this wraps to the first: harmless extra reads)
       if constexpr (u + AHEAD == KC) set_tap(tap == 8 ? 0 : tap + 1);
-      static_for<0, NT * 6 * N>([&](auto gc) __attribute__((always_inline)) {
+      static_for<0, TN * 6 * N>([&](auto gc) __attribute__((always_inline)) {
         constexpr int g = decltype(gc)::value, t = g / (6 * N), m = (g % (6 * N)) / N, j = g % N;
         constexpr int WP[6] = {0, 1, 2, 0, 1, 0}, AP[6] = {2, 1, 0, 1, 0, 0};
         f32x16 &sum = m < 5 ? low[t][j] : acc[t][j];
@@ -259,7 +261,10 @@ __device__ __forceinline__ void split_conv(const unsigned char *smem, const WFra
         if constexpr (WIDE) {
           // raw[par] was split during the k-step before: free for the k-step after next
           if constexpr (g >= 1 && g < 1 + 2 * N) read((u + 2) % KC, par, (g - 1) / 2, (g - 1) % 2);
-          if constexpr (g < 16 * N) split_some(par ^ 1, gc);
+          constexpr int PER = TN == 1 ? 3 : 1;   // (few MFMAs per k-step: more instructions behind each)
+          static_for<PER * g, PER * g + PER>([&](auto ac) __attribute__((always_inline)) {
+            if constexpr (decltype(ac)::value < 16 * N) split_some(par ^ 1, ac);
+          });
         } else {
           if constexpr (g < 3 * N) read((u + 1) % KC, par ^ 1, g / 3, g % 3);
         }
@@ -272,7 +277,7 @@ __device__ __forceinline__ void split_conv(const unsigned char *smem, const WFra
       });
     });
   }
-  if constexpr (NT == 3) {
+  if constexpr (TN == 3) {
     mma_vector_wait(acc[2][2], low[2][2]);
 #pragma unroll
     for (int k = 0; k < 8; ++k) asm volatile("" : "+a"(acc[k / 3][k % 3]), "+a"(low[k / 3][k % 3]));
@@ -345,53 +350,82 @@ __device__ __forceinline__ void split_planes8(float (&v)[8], int (&w)[3][4]) {
   }
 }
 
-// SiLU and store of one layer's outputs in the form the next one reads.
-template <int NT, bool PLANES>
-__device__ __forceinline__ void split_store(unsigned char *smem, const int (&ci)[3], int h, const f32x16 (&acc)[NT][3],
-                                            const f32x16 (&low)[NT][3]) {
+// SiLU and store of one tile of outputs, in the form the next layer reads.
+template <bool PLANES>
+__device__ __forceinline__ void split_put(unsigned char *smem, int at, int sw, int h, int t, const f32x16 &sum) {
+#pragma unroll
+  for (int q = 0; q < 4; q += 2) {
+    float v[8];
+    split_silu8(sum, 4 * q, v);
+    if constexpr (PLANES) {
+      int w[3][4];
+      split_planes8(v, w);
+#pragma unroll
+      for (int e = 0; e < 2; ++e) {
+        unsigned char *p = smem + at + ((64 * t + 16 * (q + e)) ^ sw) + 8 * h;
+#pragma unroll
+        for (int i = 0; i < 3; ++i) *reinterpret_cast<v2i *>(p + i * SplitGeo::PLANEB) = v2i{w[i][2 * e], w[i][2 * e + 1]};
+      }
+    } else {
+#pragma unroll
+      for (int e = 0; e < 2; ++e)
+        *reinterpret_cast<f32x4 *>(smem + at + 128 * t + ((32 * (q + e) + 16 * h) ^ sw)) = f32x4{v[4 * e], v[4 * e + 1], v[4 * e + 2], v[4 * e + 3]};
+    }
+  }
+}
+// ... of a layer; sum(t, j): its outputs' sums
+template <int NT, bool PLANES, class Sum>
+__device__ __forceinline__ void split_store(unsigned char *smem, const int (&ci)[3], int h, Sum sum) {
 #pragma unroll
   for (int j = 0; j < 3; ++j) {
     int pos = ci[j];
     asm volatile("" : "+v"(pos));  // (addresses formed here, not kept for the whole kernel)
     const int at = pos * SplitGeo::PIXB, sw = split_swz(pos);
 #pragma unroll
-    for (int t = 0; t < NT; ++t) {
-      const f32x16 sum = split_total<NT>(acc, low, t, j);
-#pragma unroll
-      for (int q = 0; q < 4; q += 2) {
-        float v[8];
-        split_silu8(sum, 4 * q, v);
-        if constexpr (PLANES) {
-          int w[3][4];
-          split_planes8(v, w);
-#pragma unroll
-          for (int e = 0; e < 2; ++e) {
-            unsigned char *p = smem + at + ((64 * t + 16 * (q + e)) ^ sw) + 8 * h;
-#pragma unroll
-            for (int i = 0; i < 3; ++i) *reinterpret_cast<v2i *>(p + i * SplitGeo::PLANEB) = v2i{w[i][2 * e], w[i][2 * e + 1]};
-          }
-        } else {
-#pragma unroll
-          for (int e = 0; e < 2; ++e)
-            *reinterpret_cast<f32x4 *>(smem + at + 128 * t + ((32 * (q + e) + 16 * h) ^ sw)) = f32x4{v[4 * e], v[4 * e + 1], v[4 * e + 2], v[4 * e + 3]};
-        }
-      }
-    }
+    for (int t = 0; t < NT; ++t) split_put<PLANES>(smem, at, sw, h, t, sum(t, j));
   }
 }
 
-// one 3x3 layer that is not the last
+// The sums of a layer's cout tiles one tile after the other (SLIM: in team_forward_kernel, which has no scratch to pay for on every
+// launch): the activations are read once per tile, and fewer registers are in use.  The same arithmetic for every output.
 template <int L>
+__device__ __forceinline__ void split_slim(const unsigned char *smem, const unsigned char *packed, const float *tail,
+                                           const int (&ci)[3], int h, int lane, f32x16 (&sum)[kCoutArr[L] / 32][3]) {
+  const WFrags wl = layer_weights<PrecF32S, L>(packed, lane);
+  static_for<0, kCoutArr[L] / 32>([&](auto tc) __attribute__((always_inline)) {
+    constexpr int t = decltype(tc)::value;
+    SplitWeights<1> ring;
+    f32x16 acc[1][3], low[1][3];
+    split_preload<L, t, 1>(ring, wl);
+    split_conv<L, t, 1>(smem, wl, tail + bias_offset(L), ring, ci, h, acc, low);
+#pragma unroll
+    for (int j = 0; j < 3; ++j)
+#pragma unroll
+      for (int e = 0; e < 16; ++e) sum[t][j][e] = two_sums(acc[0][j][e], low[0][j][e]);
+    __builtin_amdgcn_sched_barrier(0);
+  });
+}
+
+// one 3x3 layer that is not the last
+template <int L, bool SLIM>
 __device__ __forceinline__ void split_layer(unsigned char *smem, const unsigned char *packed, const float *tail, const int (&ci)[3],
                                             int h, int lane) {
   constexpr int NT = kCoutArr[L] / 32;
-  const WFrags wl = layer_weights<PrecF32S, L>(packed, lane);
-  SplitWeights<L> ring;
-  split_preload<L>(ring, wl);
-  f32x16 acc[NT][3], low[NT][3];
-  split_conv<L>(smem, wl, tail + bias_offset(L), ring, ci, h, acc, low);
-  __syncthreads();  // every wave has finished reading the layer's input
-  split_store<NT, kCinArr[L + 1] != 96>(smem, ci, h, acc, low);
+  constexpr bool PLANES = kCinArr[L + 1] != 96;
+  if constexpr (SLIM) {
+    f32x16 sum[NT][3];
+    split_slim<L>(smem, packed, tail, ci, h, lane, sum);
+    __syncthreads();  // every wave has finished reading the layer's input
+    split_store<NT, PLANES>(smem, ci, h, [&](int t, int j) __attribute__((always_inline)) { return sum[t][j]; });
+  } else {
+    const WFrags wl = layer_weights<PrecF32S, L>(packed, lane);
+    SplitWeights<NT> ring;
+    split_preload<L, 0, NT>(ring, wl);
+    f32x16 acc[NT][3], low[NT][3];
+    split_conv<L, 0, NT>(smem, wl, tail + bias_offset(L), ring, ci, h, acc, low);
+    __syncthreads();
+    split_store<NT, PLANES>(smem, ci, h, [&](int t, int j) __attribute__((always_inline)) { return split_total<NT>(acc, low, t, j); });
+  }
   __syncthreads();
 }
 
@@ -511,6 +545,7 @@ __device__ __forceinline__ void split_write(const FwdParams &prm, long long b, i
 }
 
 // Board b, by one workgroup of four waves: logits, value and draw, whatever its numbers.
+template <bool SLIM>
 __device__ __forceinline__ void split_board(const FwdParams &prm, unsigned char *smem, long long b) {
   using P = PrecF32S;
   using G = Geo<P>;
@@ -649,31 +684,39 @@ __device__ __forceinline__ void split_board(const FwdParams &prm, unsigned char 
     const int pos = k < 20 ? k : (k < 41 ? 400 + (k - 20) : (k - 40) * kPitch);
     *reinterpret_cast<v4i *>(smem + pos * S::PIXB + w16 * 16) = v4i{0, 0, 0, 0};
   }
-  split_store<1, true>(smem, ci, h, a0, low);
+  split_store<1, true>(smem, ci, h, [&](int, int j) __attribute__((always_inline)) { return split_total<1>(a0, low, 0, j); });
   __syncthreads();
 
-  split_layer<1>(smem, packed, tail, ci, h, lane);
-  split_layer<2>(smem, packed, tail, ci, h, lane);
-  split_layer<3>(smem, packed, tail, ci, h, lane);
-  split_layer<4>(smem, packed, tail, ci, h, lane);
-  split_layer<5>(smem, packed, tail, ci, h, lane);
-  split_layer<6>(smem, packed, tail, ci, h, lane);
+  split_layer<1, SLIM>(smem, packed, tail, ci, h, lane);
+  split_layer<2, SLIM>(smem, packed, tail, ci, h, lane);
+  split_layer<3, SLIM>(smem, packed, tail, ci, h, lane);
+  split_layer<4, SLIM>(smem, packed, tail, ci, h, lane);
+  split_layer<5, SLIM>(smem, packed, tail, ci, h, lane);
+  split_layer<6, SLIM>(smem, packed, tail, ci, h, lane);
 
   // ---- layer 8 + both 1x1 heads straight from the fp32 accumulators ----
   const float *valw = tail + kBiasTotal + kHeadC;
   SplitHeads heads(tail, tid, lane, wave, h, red);
-  const WFrags wl = layer_weights<P, 7>(packed, lane);
-  SplitWeights<7> ring;
-  split_preload<7>(ring, wl);
-  f32x16 acc[3][3], low8[3][3];
-  split_conv<7>(smem, wl, tail + bias_offset(7), ring, ci, h, acc, low8);
+  if constexpr (SLIM) {
+    f32x16 sum[3][3];
+    split_slim<7>(smem, packed, tail, ci, h, lane, sum);
 #pragma unroll
-  for (int t = 0; t < 3; ++t) {
-    f32x16 sum;
-    heads.tile(t, [&](int j, int e0, float (&v)[8]) __attribute__((always_inline)) {
-      if (e0 == 0) sum = split_total<3>(acc, low8, t, j);
-      split_silu8(sum, e0, v);
-    });
+    for (int t = 0; t < 3; ++t)
+      heads.tile(t, [&](int j, int e0, float (&v)[8]) __attribute__((always_inline)) { split_silu8(sum[t][j], e0, v); });
+  } else {
+    const WFrags wl = layer_weights<P, 7>(packed, lane);
+    SplitWeights<3> ring;
+    split_preload<7, 0, 3>(ring, wl);
+    f32x16 acc[3][3], low8[3][3];
+    split_conv<7, 0, 3>(smem, wl, tail + bias_offset(7), ring, ci, h, acc, low8);
+#pragma unroll
+    for (int t = 0; t < 3; ++t) {
+      f32x16 sum;
+      heads.tile(t, [&](int j, int e0, float (&v)[8]) __attribute__((always_inline)) {
+        if (e0 == 0) sum = split_total<3>(acc, low8, t, j);
+        split_silu8(sum, e0, v);
+      });
+    }
   }
   heads.logits(lgt, valw[kHeadC]);
   __syncthreads();

@@ -381,7 +381,7 @@ __device__ __forceinline__ void team_store(unsigned char *smem, int rec, int h, 
 // Board `b` by the team that this workgroup (its member my_role) belongs to; `slot`: the team's share of
 // the exchange memory and of the flags.
 template <class P, int TEAM>
-__device__ __forceinline__ void team_board(const TeamParams &prm, unsigned char *smem, unsigned b, unsigned slot,
+__device__ __forceinline__ bool team_board(const TeamParams &prm, unsigned char *smem, unsigned b, unsigned slot,
                                            int my_role) {
   using G = Geo<P>;
   using T = TeamGeo<P>;
@@ -430,7 +430,7 @@ __device__ __forceinline__ void team_board(const TeamParams &prm, unsigned char 
   [[maybe_unused]] const bool trace_on = true;
   // fp32: what this wave knows of the numbers in role's squares up to layer l (half_note); a word per layer, so that whoever
   // goes on with another's squares finds it
-  bool bad_input = false;
+  bool bad_input = false, again = false;   // again: what team_board returns
   [[maybe_unused]] unsigned trail = 0;
   auto note_at = [&](int l, int role) { return T::NOTE_OFF + ((l * 12 + role) * 4 + wave) * 4; };
   auto store_note = [&](int l, int role, float most, bool bad) __attribute__((always_inline)) {
@@ -1104,14 +1104,7 @@ __device__ __forceinline__ void team_board(const TeamParams &prm, unsigned char 
         if (f.logprob != nullptr) f.logprob[b] = lp;
       }
     }
-    if constexpr (T::SPLIT) {   // (behind the stores of the outputs that it goes into)
-      const bool failed = half_failed(__builtin_amdgcn_readfirstlane(*check));
-      if (failed) {
-        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-        __syncthreads();
-        if (tid == 0) half_leave(f, b);
-      }
-    }
+    if constexpr (T::SPLIT) again = half_failed(__builtin_amdgcn_readfirstlane(*check));
     if constexpr (P::ID == C6_PREC_BF16) {
       if (f.redo_mode == kRedoDetect && wave == 1) {   // (a run of one board: see fused_pipe_kernel)
         const bool again = wave_margin_below(
@@ -1172,6 +1165,7 @@ __device__ __forceinline__ void team_board(const TeamParams &prm, unsigned char 
     help = !ok;
   }
   __syncthreads();
+  return again;
 }
 
 // How many workgroups share a board (team_size, below) when there are `boards` of them: as many as fit the chip at once, where
@@ -1218,17 +1212,19 @@ __device__ __forceinline__ TeamPlace team_place(unsigned items, int team, unsign
 }
 __device__ __forceinline__ TeamPlace team_place(unsigned items, int team) { return team_place(items, team, blockIdx.x, gridDim.x); }
 
-// A workgroup's share of board b, in a team of any size that the mode has.
+// A workgroup's share of board b, in a team of any size that the mode has.  (fp32) true: a number on the way was beyond what the
+// parts hold, and the board is this workgroup's to do again.
 template <class P>
-__device__ __forceinline__ void team_share(const TeamParams &prm, unsigned char *smem, unsigned b, TeamPlace at, int team) {
-  if (team == 12) team_board<P, 12>(prm, smem, b, at.slot, at.role);
-  if (team == 6) team_board<P, 6>(prm, smem, b, at.slot, at.role);
+__device__ __forceinline__ bool team_share(const TeamParams &prm, unsigned char *smem, unsigned b, TeamPlace at, int team) {
+  if (team == 12) return team_board<P, 12>(prm, smem, b, at.slot, at.role);
+  if (team == 6) return team_board<P, 6>(prm, smem, b, at.slot, at.role);
   if constexpr (team_least<P>() <= 3) {
-    if (team == 3) team_board<P, 3>(prm, smem, b, at.slot, at.role);
+    if (team == 3) return team_board<P, 3>(prm, smem, b, at.slot, at.role);
   }
   if constexpr (team_least<P>() <= 2) {
-    if (team == 2) team_board<P, 2>(prm, smem, b, at.slot, at.role);
+    if (team == 2) return team_board<P, 2>(prm, smem, b, at.slot, at.role);
   }
+  return false;
 }
 
 template <class P> __global__ __launch_bounds__(256) void team_forward_kernel(const TeamParams prm) {
@@ -1237,7 +1233,17 @@ template <class P> __global__ __launch_bounds__(256) void team_forward_kernel(co
   const int team = team_size<P>(items, (int)gridDim.x);
   if (team == 1) return;
   const TeamPlace at = team_place(items, team);
-  if (at.slot < items) team_share<P>(prm, smem, prm.first + at.slot, at, team);
+  // fp32: the workgroup that ends a board does it again, alone, where it has to.  (In a launch behind this one, as for
+  // boards with a workgroup each: one board 47.7 -> 45.8 us, 21 boards 56.3 -> 53.7 us, 53 boards 84.9 -> 83.3 us, 128 boards
+  // 126.7 -> 124.3 us.)
+  const bool again = at.slot < items && team_share<P>(prm, smem, prm.first + at.slot, at, team);
+  if constexpr (TeamGeo<P>::SPLIT) {   // (behind the other stores of the outputs)
+    if (again) {
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+      __syncthreads();
+      split_board<true>(prm.f, smem, prm.first + at.slot);
+    }
+  }
 }
 
 // The plain 16-bit modes with a few boards beyond whole rounds of one board per CU: teams for them in one launch with the

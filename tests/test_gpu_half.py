@@ -138,3 +138,15 @@ def test_draws_alone_of_boards_that_take_either_way(cuda, boards):
                             0.0, u.data_ptr(), 1.0, actions.data_ptr(), logprob.data_ptr(), _lib.stream_ptr(cuda))
         _lib.check(rc, "c6_forward")
         assert torch.equal(actions, want[2]) and torch.equal(logprob, want[3])
+
+
+def test_a_rest_behind_whole_rounds_takes_either_way(cuda):
+    """The boards with a workgroup each and the rest in teams, half of either beyond the line, in one call."""
+    st, x = _case("planes", 40000.0)
+    packed = _model(cuda, st).packed_weights(PREC)
+    cus = torch.cuda.get_device_properties(cuda).multi_processor_count
+    rows = torch.arange(cus + 41) % 40
+    with torch.inference_mode():
+        want = run_forward(x.to(cuda), packed, PREC, 1, 40)
+        got = run_forward(x[rows].to(cuda), packed, PREC, 1, len(rows))
+    assert torch.equal(got[0], want[0][rows]) and torch.equal(got[1], want[1][rows])

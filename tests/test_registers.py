@@ -98,3 +98,33 @@ def test_a_sum_that_moves_is_seen(split, planted, where):
     while split[at - 1][1] == "s_nop 1":   # (the pair of a wait state and its instruction stays one)
         at += 1
     assert text in _moved(split[:at] + [(split[at][0] - 1, text, None)] + split[at:])
+
+
+# Where two ways meet, a copy of a constant or of a register in front of the instruction that brings the other lanes back is one
+# that they do not get.  (The compiler has put such copies there in fp32 kernels whose registers were all in use.)
+def _copies_for_some_lanes(lines):
+    at = {address: i for i, (address, _, _) in enumerate(lines)}
+    found = []
+    for i in sorted({at[to] for _, text, to in lines if text.startswith("s_cbranch_execz") and to in at}):
+        copies = []
+        for _, text, _ in lines[i:]:
+            if text.startswith("s_or_b64 exec, exec"):
+                found += copies
+            if "exec" in text or text.startswith(("s_branch", "s_cbranch", "s_endpgm", "s_setpc")):
+                break
+            if re.match(r"v_mov_b32|v_mov_b64|v_accvgpr|scratch_load|buffer_load_dword\S* .* off, s\[0:3\]", text):
+                copies.append(text)
+    return found
+
+
+@pytest.mark.parametrize("kernel", ["19team_forward_kernelINS_8PrecF32SEEEvNS_10TeamParamsE",
+                                    "19half_forward_kernelINS_8PrecF32SEEEvNS_9FwdParamsE",
+                                    "20split_forward_kernelINS_8PrecF32SEEEvNS_9FwdParamsE"])
+def test_no_copy_is_made_for_some_lanes_only(kernel, tmp_path):
+    lines = _listing(tmp_path, "_ZN2c6" + kernel)
+    assert _copies_for_some_lanes(lines) == []
+    joins = [i for i, (address, text, _) in enumerate(lines) if text.startswith("s_or_b64 exec, exec") and
+             any(to == address and other.startswith("s_cbranch_execz") for _, other, to in lines)]
+    address, text, to = lines[joins[0]]
+    planted = [(address, "v_mov_b32_e32 v1, 0x100", None), (address + 1, text, to)]
+    assert _copies_for_some_lanes(lines[:joins[0]] + planted + lines[joins[0] + 1:]) == [planted[0][1]]

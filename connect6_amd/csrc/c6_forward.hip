@@ -2298,8 +2298,8 @@ template <class P> int launch_left(const FwdParams &fp, int cus, hipStream_t st)
                               hipFuncAttributeMaxDynamicSharedMemorySize, SplitGeo::LDS_BYTES);
       if (e == hipSuccess) configured = dev;
     }
-    if (e == hipSuccess) {
-      const long long grid = fp.total_boards < cus ? fp.total_boards : cus;
+    const long long grid = forward_grid<P>(fp.total_boards, cus);   // (as that of half_forward_kernel)
+    if (e == hipSuccess && !half_redone((fp.total_boards + grid - 1) / grid)) {
       hipLaunchKernelGGL(split_forward_kernel<P>, dim3((unsigned)grid), dim3(256), SplitGeo::LDS_BYTES, st, fp);
       e = hipGetLastError();
     }
@@ -2517,8 +2517,8 @@ static int second_mode(int cascade) { return cascade == C6_PREC_BF16C ? C6_PREC_
 // 4,096 (4) 937 / 903, 16,384 (19) 3,428 / 3,402.
 
 // Boards of a batch that are shared between workgroups: all where they are few; behind whole rounds of one
-// workgroup per CU the rest (fp32: 257 boards 389 -> 244 us, 341 boards 389 -> 305 us, 384 boards 389 -> 350 us, 777 boards 748 ->
-// 614 us; bf16 + fp6 + low weights, 298 boards: 239 -> 191 us).  In the modes that put two workgroups on a CU a rest of up
+// workgroup per CU the rest (fp32: 257 boards 231 us, 341 boards 281 us, 384 boards 318 us where two whole rounds take 366 us; 777 boards
+// 589 us, four rounds 720 us; bf16 + fp6 + low weights, 298 boards: 239 -> 191 us).  In the modes that put two workgroups on a CU a rest of up
 // to five sixteenths of the CUs goes to teams that run beside the last boards of the others (duo_rest_kernel).  Without
 // that each is a board more for its CU, the last one alone there, 35 to 45 us; with teams in a launch behind the others 30 to 35.
 // Measured, us, without / with; the cascade's with its second pass:

@@ -34,7 +34,7 @@
 // and the first operands of each pass (3 to 5 k), and staging (7 k).  2,048 boards, both sides in turn: 2,117 -> 1,382 us from six
 // products to three with the same structure, and 2,260 -> 1,436 on another box with all epilogues but the last tile's behind MFMAs and
 // three instructions fewer in each (in cycles 350 k -> 330 k; the clock gives back half of it).  In teams (c6_team.h) one board 58 ->
-// 49 us, 53 boards 117 -> 98, 128 boards 215 -> 142, of which the launch that looks for boards left over is 4.
+// 49 us, 53 boards 117 -> 98, 128 boards 215 -> 142, of which the launch that looked for boards left over was 4.
 #pragma once
 
 namespace c6 {
@@ -405,8 +405,15 @@ __device__ __forceinline__ bool half_left(const FwdParams &prm, long long b) {
   return prm.actions != nullptr && prm.actions[b] == -1;
 }
 
-// The boards that half_forward_kernel left, one workgroup each; there are hardly ever any, and then this takes 4 us, of which the
-// launch is most.  (Teams do without: team_forward_kernel.)
+// Whether a workgroup of half_forward_kernel does a board that it cannot hold again itself: where that is its only one.  A launch of
+// split_forward_kernel, which looks for such boards and hardly ever finds one, takes 4 us: 129 boards 150.5 -> 147 us, 256
+// boards 190.2 -> 187.1 us, 384 boards (128 of them in teams) 322 -> 318.5 us.  (With every board beyond the range 256 take 793 -> 832 us, since the
+// form that needs no scratch is the slower one.)  Behind more boards each the launch stays: up to eight done again where
+// they ended gain as much, 512 boards 366.7 -> 363.6 us, 2,048 boards 1,427 -> 1,423 us, but a weight set beyond the range, whose boards
+// lie side by side, would go through few workgroups one after the other.
+__host__ __device__ inline bool half_redone(long long per_workgroup) { return per_workgroup == 1; }
+
+// The boards that half_forward_kernel left, one workgroup each.  (Teams do without: team_forward_kernel.)
 template <class P> __global__ __launch_bounds__(256) void split_forward_kernel(const FwdParams prm) {
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
   // boards dealt out one by one; every wave looks at the same 64, so that all agree
@@ -492,6 +499,7 @@ __global__ __launch_bounds__(256) void half_forward_kernel(const FwdParams prm) 
   const long long b_end = b + per < prm.total_boards ? b + per : prm.total_boards;
   if (b >= b_end) return;
   v4i r1[L1Pipe<P>::D][1];
+  bool again = false;
   fetch_board(b);
 
   for (; b < b_end; ++b) {
@@ -696,11 +704,13 @@ __global__ __launch_bounds__(256) void half_forward_kernel(const FwdParams prm) 
     }
     __syncthreads();
     if (half_failed(__builtin_amdgcn_readfirstlane(*check))) {
-      if (tid == 0) half_leave(prm, b);
+      again = half_redone(per);
+      if (!again && tid == 0) half_leave(prm, b);
     } else {
       split_write(prm, b, tidv, lane, wave, occ, lgt, red, valw[kHeadC + 1]);
     }
   }
+  if (again) split_board<true>(prm, smem, run);   // (its only board)
 }
 
 }  // namespace c6

@@ -1172,7 +1172,7 @@ __device__ __forceinline__ bool team_board(const TeamParams &prm, unsigned char 
 // that beats one workgroup (1: the one-workgroup kernels).  With fewer workgroups per board more waves read
 // the same weights, and the L1's 64 bytes a cycle bound the layers; the 16-bit one-workgroup kernel hides its epilogues
 // behind its MFMAs, which a team does not.  Measured, us, teams of 12 / 6 / 3 / 2 against one workgroup each, boards:
-//   fp32  16: 52 / 68 / 83 / 108 / 192   40: 74 / 87 / 112 / 192 (without 12)   80: 103 / 119 / 192   128: 146 / 192
+//   fp32  16: 47 / 62 / 77 / 102   40: 71 / 81 / 108 (without 12)   80: 94 / 113   128: 131   one workgroup each, 129: 147
 //   bf16  16: 31 / 41 / 49 / 61 / 45      21: 36 / 41 / - / - / 46   40: 42 / 50 / 61 / 45   42: 48 (teams on two XCDs)
 //   bf16 + fp6  21: 44 / 51 / 64 / 81 / 63    42: 57 / 68 / 84 / 64    with low weights  21: 52 / 60 / 78 / 101 / 89
 //   42: 67 / 84 / 106 / 89    72: 89 / 110 / 89 (behind a first pass, 53 listed boards, 85 against 110)

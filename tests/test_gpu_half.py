@@ -150,3 +150,27 @@ def test_a_rest_behind_whole_rounds_takes_either_way(cuda):
         want = run_forward(x.to(cuda), packed, PREC, 1, 40)
         got = run_forward(x[rows].to(cuda), packed, PREC, 1, len(rows))
     assert torch.equal(got[0], want[0][rows]) and torch.equal(got[1], want[1][rows])
+
+
+@pytest.mark.parametrize("per", [1, 2, 3])
+@pytest.mark.parametrize("outputs", ["all", "value", "actions"])
+def test_boards_with_a_workgroup_each_take_either_way(cuda, per, outputs):
+    """One board for each workgroup, which does it again itself, and more, which leave it to the next launch; the last workgroups
+    have fewer or none."""
+    st, x = _case("planes", 40000.0)
+    packed = _model(cuda, st).packed_weights(PREC)
+    cus = torch.cuda.get_device_properties(cuda).multi_processor_count
+    for boards in (per * cus, per * cus - 3):
+        rows = torch.arange(boards) % 40
+        u = gen_uniform(40, 5)
+        with torch.inference_mode():
+            want = run_forward(x.to(cuda), packed, PREC, 1, 40, mask_mode=_lib.MASK_INPUT, u=u.to(cuda))
+            if outputs == "actions":
+                got = run_forward(x[rows].to(cuda), packed, PREC, 1, boards, mask_mode=_lib.MASK_INPUT, u=u[rows].to(cuda),
+                                  want_logits=False, want_value=False)
+                assert torch.equal(got[2], want[2][rows])
+                continue
+            got = run_forward(x[rows].to(cuda), packed, PREC, 1, boards, mask_mode=_lib.MASK_INPUT, want_logits=outputs == "all")
+        assert torch.equal(got[1], want[1][rows])
+        if outputs == "all":
+            assert torch.equal(got[0], want[0][rows])

@@ -113,7 +113,7 @@ struct PrecBF16F6W {
 };
 
 // fp32 on the fp16 matrix cores: every weight is two fp16 values, and what they leave of it, packed as three fragments that
-// follow one another; an activation is two.  c6_half.h; boards beyond fp16's range: c6_split.h, on the same weights.
+// follow one another; an activation is two.  c6_half.h.
 struct PrecF32S {
   static constexpr int WLO = 2;
   static constexpr int PIPE = 0;      // weights packed tap-major
@@ -122,6 +122,21 @@ struct PrecF32S {
   static constexpr int LO6 = 0;
   static constexpr int LO_MASK = 0;
 };
+
+// ... and for the boards beyond fp16's range: every operand the exact sum of three bf16 values.  c6_split.h.  No mode of its own:
+// its packed weights lie behind those of PrecF32S (kSplitOffset).
+struct PrecF32X {
+  static constexpr int WLO = 2;
+  static constexpr int PIPE = 0;
+  static constexpr int ID = -1;
+  static constexpr int EB = 2;
+  static constexpr int LO6 = 0;
+  static constexpr int LO_MASK = 0;
+};
+// how many 16-bit values an fp32 operand is (0: operands are not fp32, or are contracted as such)
+template <class P> inline constexpr int kParts = 0;
+template <> inline constexpr int kParts<PrecF32S> = 2;
+template <> inline constexpr int kParts<PrecF32X> = 3;
 
 // bf16 + fp6 mode: what rounding an activation to bf16 drops (|lo| <= 2^-9 |a|) is contracted
 // with an e2m3 copy of the weights in a second pass of v_mfma_scale_f32_32x32x64_f8f6f4 (K = 64
@@ -226,11 +241,14 @@ template <class P> struct Geo {
   static constexpr size_t TAIL_OFF = (size_t)TOTAL_FRAGS * 1024;  // fp32 tail: biases, heads
   // tail words: bias[544] polw[96] valw[96] polb valb pad pad, then 8 ints sw[layer]
   static constexpr int TAIL_SW = kBiasTotal + 2 * kHeadC + 4;
-  // fp32 by three parts: then what rounding the scaled biases to fp32 left out
+  // fp32 by parts: then what rounding the scaled biases to fp32 left out (by two: in the units of the small products' sum)
   static constexpr int TAIL_BIAS_LOW = TAIL_SW + 8;
   static constexpr int TAIL_FLOATS = TAIL_BIAS_LOW + (P::WLO == 2 ? kBiasTotal : 0);
   static constexpr size_t PACKED_BYTES = TAIL_OFF + (size_t)TAIL_FLOATS * 4;
 };
+
+// fp32: one packed set = that of two fp16 parts, then (256-byte aligned) that of three bf16 parts.
+constexpr size_t kSplitOffset = (Geo<PrecF32S>::PACKED_BYTES + 255) & ~(size_t)255;
 
 // Cascade modes: one packed set = the plain bf16 set, then (256-byte aligned) the set of the same
 // parameters for the second pass: bf16 + fp6 + the weights' low part (C6_PREC_BF16C), or, for

@@ -155,10 +155,10 @@ template <class P> __host__ __device__ constexpr float act_scale() { return P::E
 // What is scaled while the weights are packed: fp32 by three parts takes the factor to 53 bits, so that a
 // weight is rounded once, when its three parts are taken, and a bias and a sum of weights once, to fp32.
 // (Its head weights are not divided by it: the sums over them are, in the kernel.)
-template <class P> using Scaled = std::conditional_t<P::WLO == 2, double, float>;
+template <class P> using Scaled = std::conditional_t<kParts<P> != 0, double, float>;
 constexpr double kActScale64 = -1.4426950408889634074;
 template <class P> __device__ __forceinline__ Scaled<P> act_scaled(Scaled<P> v) {
-  if constexpr (P::WLO == 2) return v * kActScale64;
+  if constexpr (kParts<P> != 0) return v * kActScale64;
   else return v * act_scale<P>();
 }
 
@@ -1949,7 +1949,11 @@ template <class P> __device__ __forceinline__ float weight_part(Scaled<P> v, int
   if constexpr (P::EB == 4) {
     return v;
   } else {
-    static_assert(P::WLO < 2 && (P::WLO == 0 || P::ID != C6_PREC_F16), "the low part is defined for bf16 storage");
+    static_assert(P::WLO == 0 || P::ID != C6_PREC_F16, "the low part is defined for bf16 storage");
+    if constexpr (kParts<P> == 3) {
+      for (int i = 0; i < part; ++i) v = bf16_rest(v, bf16_part((float)v));
+      return __builtin_bit_cast(float, (unsigned)bf16_part((float)v) << 16);
+    }
     for (int i = 0; i < part; ++i) v -= __builtin_bit_cast(float, (unsigned)bits16<P>((float)v) << 16);
     return (float)v;
   }
@@ -1957,7 +1961,7 @@ template <class P> __device__ __forceinline__ float weight_part(Scaled<P> v, int
 
 // One weight's `part` as element e of a lane's 16 bytes
 template <class P> __device__ __forceinline__ void put_weight(unsigned char *dst, int e, Scaled<P> v, int part) {
-  if constexpr (P::WLO == 2) reinterpret_cast<unsigned short *>(dst)[e] = half_parts(v).part[part];
+  if constexpr (kParts<P> == 2) reinterpret_cast<unsigned short *>(dst)[e] = half_parts(v).part[part];
   else put_elem<P>(dst, e, weight_part<P>(v, part));
 }
 
@@ -1967,8 +1971,8 @@ struct GroupView {
   int g;
   unsigned char *packed;
   const float *pol_w, *pol_b, *val_w, *val_b;
-  __device__ GroupView(const PackParams &pp, int group)
-      : p(pp), g(group), packed(pp.packed + (size_t)group * pp.packed_stride),
+  __device__ GroupView(const PackParams &pp, int group, size_t offset = 0)
+      : p(pp), g(group), packed(pp.packed + (size_t)group * pp.packed_stride + offset),
         pol_w(pp.pol_w + (size_t)group * kHeadC), pol_b(pp.pol_b ? pp.pol_b + group : nullptr),
         val_w(pp.val_w ? pp.val_w + (size_t)group * kHeadC : nullptr),
         val_b(pp.val_b ? pp.val_b + group : nullptr) {}
@@ -1982,12 +1986,8 @@ struct GroupView {
 };
 
 // one thread per (fragment, lane): writes the 16 bytes that lane will load
-// (blockIdx.y = weight set: the parameter tensors are stacked [sets, ...], the packed sets lie
-// packed_stride bytes apart)
-template <class P> __global__ __launch_bounds__(256) void pack_kernel(const PackParams all) {
+template <class P> __device__ __forceinline__ void pack_thread(const GroupView &prm, long long gid) {
   using G = Geo<P>;
-  const GroupView prm(all, blockIdx.y);
-  const long long gid = (long long)blockIdx.x * blockDim.x + threadIdx.x;
   const long long nfl = (long long)G::TOTAL_FRAGS * 64;
   if (gid < nfl) {
     const int frag = (int)(gid >> 6), lane = (int)(gid & 63);
@@ -2093,7 +2093,7 @@ template <class P> __global__ __launch_bounds__(256) void pack_kernel(const Pack
         if (row < kK1 * 3 && kx < kK1) v = act_scaled<P>(w[((co * 3 + ch) * kK1 + ky) * kK1 + kx]);
         put_weight<P>(dst, e, v, part);
       }
-    } else if constexpr (P::WLO == 2) {
+    } else if constexpr (kParts<P> == 2) {
       // (tap-major; the first tap's thread takes all nine: what their parts leave is balanced over them)
       const int kc_per_tap = cin / G::KSTEP;
       if (part != 0 || s >= kc_per_tap) return;
@@ -2149,10 +2149,11 @@ template <class P> __global__ __launch_bounds__(256) void pack_kernel(const Pack
   if (ti >= G::TAIL_BIAS_LOW && ti < G::TAIL_FLOATS) {
     const Scaled<P> b = conv_bias(ti - G::TAIL_BIAS_LOW);
     const float low = (float)(b - (float)b);
-    tail[ti] = low == low ? low / kTailLow : 0.0f;   // (an infinite bias leaves nothing)
+    constexpr float unit = kParts<P> == 2 ? 1.0f / (kHalfW * kHalfA * kHalfLow) : 1.0f;
+    tail[ti] = low == low ? low / unit : 0.0f;   // (an infinite bias leaves nothing)
   }
   if (ti < G::TAIL_SW) {  // the sw[] words behind it are written by lo_scale_kernel
-    constexpr float head_scale = P::WLO == 2 ? 1.0f : act_scale<P>();
+    constexpr float head_scale = kParts<P> != 0 ? 1.0f : act_scale<P>();
     float v = 0.0f;
     if (ti < kBiasTotal) {
       v = (float)conv_bias(ti);
@@ -2167,6 +2168,25 @@ template <class P> __global__ __launch_bounds__(256) void pack_kernel(const Pack
     }
     tail[ti] = v;
   }
+}
+
+constexpr int kPackThreads = 256;
+template <class P> constexpr int pack_blocks() {
+  return (int)(((long long)Geo<P>::TOTAL_FRAGS * 64 + Geo<P>::TAIL_FLOATS + kPackThreads - 1) / kPackThreads);
+}
+// (blockIdx.y = weight set: the parameter tensors are stacked [sets, ...], the packed sets lie
+// packed_stride bytes apart.  fp32: both of its sets in one launch, since what a thread with a square's sum of the third plane's
+// weights takes, most of the time, is then waited for once: 252 -> 135 us.)
+template <class P> __global__ __launch_bounds__(kPackThreads) void pack_kernel(const PackParams all) {
+  const long long at = threadIdx.x;
+  if constexpr (kParts<P> == 2) {
+    const int block = (int)blockIdx.x - pack_blocks<P>();
+    if (block >= 0) {
+      pack_thread<PrecF32X>(GroupView(all, blockIdx.y, kSplitOffset), block * (long long)kPackThreads + at);
+      return;
+    }
+  }
+  pack_thread<P>(GroupView(all, blockIdx.y), blockIdx.x * (long long)kPackThreads + at);
 }
 
 // sw[l] = largest power of two that keeps 2^sw * max|w_l| inside the range of the low-order
@@ -2216,13 +2236,10 @@ template <class P> int launch_second_pass(const TeamParams &tp, int grid, hipStr
 
 #ifndef C6_SPLIT
 template <class P> int launch_pack(const PackParams &pp, hipStream_t st) {
-  using G = Geo<P>;
-  const long long total = (long long)G::TOTAL_FRAGS * 64 + G::TAIL_FLOATS;
-  const int threads = 256;
-  const int blocks = (int)((total + threads - 1) / threads);
+  const int blocks = pack_blocks<P>() + (kParts<P> == 2 ? pack_blocks<PrecF32X>() : 0);
   const unsigned sets = (unsigned)pp.groups;
   if constexpr (P::LO6) hipLaunchKernelGGL(lo_scale_kernel<P>, dim3(8, sets), dim3(256), 0, st, pp);
-  hipLaunchKernelGGL(pack_kernel<P>, dim3(blocks, sets), dim3(threads), 0, st, pp);
+  hipLaunchKernelGGL(pack_kernel<P>, dim3(blocks, sets), dim3(kPackThreads), 0, st, pp);
   const hipError_t e = hipGetLastError();
   if (e != hipSuccess) {
     set_error("pack_kernel launch failed: %s", hipGetErrorString(e));
@@ -2660,7 +2677,7 @@ size_t packed_bytes(int prec) {
   if (is_cascade(prec)) return cascade_packed_bytes(prec);
   switch (prec) {
     case C6_PREC_F32: return Geo<PrecF32>::PACKED_BYTES;
-    case C6_PREC_F32S: return Geo<PrecF32S>::PACKED_BYTES;
+    case C6_PREC_F32S: return kSplitOffset + Geo<PrecF32X>::PACKED_BYTES;
     case C6_PREC_BF16: return Geo<PrecBF16>::PACKED_BYTES;
     case C6_PREC_F16: return Geo<PrecF16>::PACKED_BYTES;
     case C6_PREC_BF16F6: return Geo<PrecBF16F6>::PACKED_BYTES;

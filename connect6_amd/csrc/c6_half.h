@@ -27,7 +27,7 @@
 // 2^4, activations 2^4 (and -log2(e), as in c6_split.h).  So two parts hold what they should while weights are below 2048 (and
 // no less than 2e-13, first layer 2e-10, but for zeros), activations below 1400 and the largest activation of each layer's above 5e-6.  A board for which that does not hold, or
 // that has an infinity or a NaN anywhere, is seen at its end: every layer keeps the largest of what it stored (half_note), and a
-// weight beyond the range is packed as a NaN (with itself in the other two parts).  Such a board goes through c6_split.h.
+// weight beyond the range is packed as a NaN.  Such a board goes through c6_split.h, which has packed weights of its own.
 //
 // What bounds it: the matrix cores, 195 k cycles per board (the 1,890 MFMAs of the 3x3 layers and the first layer's 207 three
 // times each) of 330 k at 1.9 GHz; what goes in the open is the epilogue of each layer's last cout tile (5 k), the sums at the ends of kernel rows
@@ -40,7 +40,7 @@
 namespace c6 {
 
 // Parts of a weight that carries kHalfW: two as above, and what they leave of it, in units of the second (first layer) or times
-// 2^11 once more (the others, where it is for split_decode alone).  A weight beyond the range, or so small that the parts would hold
+// 2^11 once more (the others, where nothing reads it).  A weight beyond the range, or so small that the parts would hold
 // few of its bits, is a NaN, with itself (the fp32 number `raw`) in the other two.
 struct HalfParts {
   unsigned short part[3];

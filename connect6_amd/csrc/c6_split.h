@@ -16,11 +16,8 @@
 // The biases, scaled by -log2(e), are not fp32 numbers any more: the large sum starts with them as fp32, the
 // small one with what that leaves.
 //
-// The packed weights are c6_half.h's three fp16 parts; split_decode makes three bf16 ones of them, in registers, in front of
-// their MFMAs.
-//
 // What bounds it: the matrix cores, 383 k cycles per board with the 1,890 MFMAs of the 3x3 layers
-// six times and the first layer's 207 three times (0/1 inputs are exact in one bf16 value); then the weights' decoding and the
+// six times and the first layer's 207 three times (0/1 inputs are exact in one bf16 value); then the
 // epilogues, some 25 instructions per output of a lane that one wave per SIMD issues in the open, step by step over eight
 // outputs.  The activations of up to 64 channels lie in LDS as their three planes, split once when a layer writes
 // them; 96 channels only fit as fp32 (421 positions x 384 bytes are the CU's whole LDS), and the two
@@ -39,11 +36,10 @@
 
 namespace c6 {
 
-// What the packed low words of the biases have to be multiplied by (they are c6_half.h's, in the units of its small sums)
-constexpr float kTailLow = 1.0f / (kHalfW * kHalfA * kHalfLow);
+template <> __device__ __forceinline__ void mma<PrecF32X>(const v4i &a, const v4i &b, f32x16 &c) { mma<PrecBF16>(a, b, c); }
 
 struct SplitGeo {
-  using G = Geo<PrecF32S>;                     // weight stream and first-layer geometry
+  using G = Geo<PrecF32X>;                     // weight stream and first-layer geometry
   static constexpr int PIXB = 384;             // 3 planes x 64 channels x 2 bytes, or 96 x 4
   static constexpr int PLANEB = 128;
   static constexpr int ACT_BYTES = kPos * PIXB;
@@ -99,32 +95,6 @@ template <int L, int T0, int TN> __device__ __forceinline__ void split_preload(S
       for (int i = 0; i < 3; ++i) ring[d][t][i] = wl[(d * NT + T0 + t) * 3 + i];
 }
 
-// Weights of one fragment, from the packed set's parts (half_parts) to three bf16 ones.  A weight beyond fp16 is marked and
-// lies there as it is.
-// FIRST: of the first layer.
-template <bool FIRST> __device__ __forceinline__ void split_decode(v4i (&w)[3]) {
-  constexpr float kRest = FIRST ? 1.0f : 1.0f / kHalfLow;
-#pragma unroll
-  for (int d = 0; d < 4; ++d) {
-    float v[2];
-    const int w0 = w[0][d], w1 = w[1][d], w2 = w[2][d];
-    const f16x2 hi = __builtin_bit_cast(f16x2, w0), lo = __builtin_bit_cast(f16x2, w1), rest = __builtin_bit_cast(f16x2, w2);
-#pragma unroll
-    for (int e = 0; e < 2; ++e) {
-      v[e] = fmaf(fmaf((float)rest[e], kRest, (float)lo[e]), 1.0f / (kHalfW * kHalfLow), (float)hi[e] * (1.0f / kHalfW));
-      const unsigned raw = e ? ((unsigned)w1 >> 16) | ((unsigned)w2 & 0xffff0000u) : ((unsigned)w1 & 0xffffu) | ((unsigned)w2 << 16);
-      v[e] = ((w0 >> (16 * e)) & 0x7fff) == kHalfMark ? __builtin_bit_cast(float, raw) : v[e];
-    }
-#pragma unroll
-    for (int i = 0; i < 3; ++i) {
-      const unsigned short a = bf16_part(v[0]), b = bf16_part(v[1]);
-      v[0] = bf16_rest(v[0], a);
-      v[1] = bf16_rest(v[1], b);
-      w[i][d] = (int)((unsigned)a | (unsigned)b << 16);
-    }
-  }
-}
-
 // First layer: ROWS rows of K, three fragments of 8 columns each, rowb bytes apart in LDS; large products to acc, small ones
 // to low.  at[j]: where the lane's square of pixel tile j begins.
 template <int ROWS>
@@ -143,7 +113,6 @@ __device__ __forceinline__ void split_first(const unsigned char *smem, const WFr
         w[p] = next[i][p];
         next[i][p] = wl[((row + 1) * 3 + i) * 3 + p];   // (behind the last row: what follows, unused)
       }
-      split_decode<true>(w);
 #pragma unroll
       for (int j = 0; j < 3; ++j) {
         const v4i x = *reinterpret_cast<const v4i *>(smem + at[j] + row * rowb + i * 16);
@@ -236,11 +205,11 @@ __device__ __forceinline__ void split_conv(const unsigned char *smem, const WFra
   for (int t = 0; t < TN; ++t) {
     f32x16 b[1], bl[1];
     load_bias_tiles(b, bias + 32 * (T0 + t), h);
-    load_bias_tiles(bl, bias + Geo<PrecF32S>::TAIL_BIAS_LOW + 32 * (T0 + t), h);
+    load_bias_tiles(bl, bias + Geo<PrecF32X>::TAIL_BIAS_LOW + 32 * (T0 + t), h);
 #pragma unroll
     for (int j = 0; j < N; ++j) {
       acc[t][j] = b[0];
-      low[t][j] = bl[0] * kTailLow;
+      low[t][j] = bl[0];
     }
   }
   constexpr int AHEAD = WIDE ? 2 : 1;
@@ -255,7 +224,6 @@ __device__ __forceinline__ void split_conv(const unsigned char *smem, const WFra
         constexpr int g = decltype(gc)::value, t = g / (6 * N), m = (g % (6 * N)) / N, j = g % N;
         constexpr int WP[6] = {0, 1, 2, 0, 1, 0}, AP[6] = {2, 1, 0, 1, 0, 0};
         f32x16 &sum = m < 5 ? low[t][j] : acc[t][j];
-        if constexpr (g % (6 * N) == 0) split_decode<false>(ring[u % D][t]);
         if constexpr (t == 2 && j == 2) mma_vector(ring[u % D][t][WP[m]], bq[par][j][AP[m]], sum);
         else mma<PrecBF16>(ring[u % D][t][WP[m]], bq[par][j][AP[m]], sum);
         if constexpr (WIDE) {
@@ -391,7 +359,7 @@ __device__ __forceinline__ void split_store(unsigned char *smem, const int (&ci)
 template <int L>
 __device__ __forceinline__ void split_slim(const unsigned char *smem, const unsigned char *packed, const float *tail,
                                            const int (&ci)[3], int h, int lane, f32x16 (&sum)[kCoutArr[L] / 32][3]) {
-  const WFrags wl = layer_weights<PrecF32S, L>(packed, lane);
+  const WFrags wl = layer_weights<PrecF32X, L>(packed, lane);
   static_for<0, kCoutArr[L] / 32>([&](auto tc) __attribute__((always_inline)) {
     constexpr int t = decltype(tc)::value;
     SplitWeights<1> ring;
@@ -418,7 +386,7 @@ __device__ __forceinline__ void split_layer(unsigned char *smem, const unsigned 
     __syncthreads();  // every wave has finished reading the layer's input
     split_store<NT, PLANES>(smem, ci, h, [&](int t, int j) __attribute__((always_inline)) { return sum[t][j]; });
   } else {
-    const WFrags wl = layer_weights<PrecF32S, L>(packed, lane);
+    const WFrags wl = layer_weights<PrecF32X, L>(packed, lane);
     SplitWeights<NT> ring;
     split_preload<L, 0, NT>(ring, wl);
     f32x16 acc[NT][3], low[NT][3];
@@ -547,7 +515,7 @@ __device__ __forceinline__ void split_write(const FwdParams &prm, long long b, i
 // Board b, by one workgroup of four waves: logits, value and draw, whatever its numbers.
 template <bool SLIM>
 __device__ __forceinline__ void split_board(const FwdParams &prm, unsigned char *smem, long long b) {
-  using P = PrecF32S;
+  using P = PrecF32X;
   using G = Geo<P>;
   using S = SplitGeo;
   constexpr int THREADS = 256, ROUNDS = (kPix + THREADS - 1) / THREADS;
@@ -572,7 +540,7 @@ __device__ __forceinline__ void split_board(const FwdParams &prm, unsigned char 
   float *lgt = reinterpret_cast<float *>(smem + S::LGT_OFF);
   float *red = reinterpret_cast<float *>(smem + S::RED_OFF);
   int *flags = reinterpret_cast<int *>(red) + 40;   // [0]: third plane varies, [1]: an input is not exact in bf16
-  const unsigned char *packed = prm.packed + (size_t)((unsigned)b / (unsigned)prm.boards_per_group) * prm.packed_stride;
+  const unsigned char *packed = prm.packed + (size_t)((unsigned)b / (unsigned)prm.boards_per_group) * prm.packed_stride + kSplitOffset;
   const float *tail = reinterpret_cast<const float *>(packed + G::TAIL_OFF);
 
   float left[ROUNDS][3];   // the input; then what the parts staged so far leave of it
@@ -622,7 +590,7 @@ __device__ __forceinline__ void split_board(const FwdParams &prm, unsigned char 
 #pragma unroll
         for (int e = 0; e < 4; ++e) a0[0][j][4 * q + e] = plane2_varies ? b0[0][4 * q + e] : fmaf(c2, t4[e], b0[0][4 * q + e]);
       }
-      low[0][j] = bl[0] * kTailLow;
+      low[0][j] = bl[0];
 #pragma unroll
       for (int i = 0; i < 16; ++i) first[0][j][i] = 0.0f;
     }

@@ -50,7 +50,7 @@ extern "C" {
 #define C6_PREC_F32S 7   /* fp32 operands, each as two fp16 values of 11 mantissa bits: three fp16 MFMAs
                             per product, fp32 accumulate.  fp32 results, less than half as far from a
                             64-bit forward as those of C6_PREC_F32, at a third of the time; its packed
-                            weights take three halves of that mode's.  A board that has numbers beyond
+                            weights (of both ways below) take three times that mode's.  A board that has numbers beyond
                             what fp16 holds so (weights up to 2048 and from 2e-10 on, activations up to
                             1400 and not all below 5e-6) is computed with three bf16 values per operand and six MFMAs
                             per product.  Infinities and NaN as in fp32, except that a sum or an

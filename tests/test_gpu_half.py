@@ -174,3 +174,29 @@ def test_boards_with_a_workgroup_each_take_either_way(cuda, per, outputs):
         assert torch.equal(got[1], want[1][rows])
         if outputs == "all":
             assert torch.equal(got[0], want[0][rows])
+
+
+def _against_float64(cuda, st, x, boards=(None,)):
+    """Errors of logits and values against a float64 forward: the fp32 instructions', and this for each number of boards."""
+    model = _model(cuda, st)
+    l64, v64 = R.forward({k: v.double() for k, v in st.items()}, x.double())
+    xd = x.to(cuda)
+
+    def errors(prec, n):
+        rows = torch.arange(n) % len(x)
+        with torch.inference_mode():
+            lg, vg, _, _ = run_forward(xd[rows], model.packed_weights(prec), prec, 1, n)
+        return rel_l2(lg.double().cpu(), l64[rows]), float((vg.double().cpu() - v64[rows]).abs().max())
+
+    return errors(_lib.PREC_F32, len(x)), [errors(PREC, n or len(x)) for n in boards]
+
+
+@pytest.mark.parametrize("factors", [{0: 1e-5, 1: 1e3, 2: 1e2}, {0: 1e-6, 1: 1e3, 2: 1e3}, {0: 1e-7, 1: 1e3, 2: 1e4}])
+def test_small_weights_of_the_first_layer(cuda, factors):
+    """Whichever way these boards go, their weights are those of the caller to 24 bits."""
+    st, x = R.init_state(5, "reference"), gen_boards(6, 200, 3)[0]
+    for layer, factor in factors.items():
+        st[f"convs.{layer}.weight"] *= factor
+    was, now = _against_float64(cuda, st, x, (6, 60, 200, 600))
+    for n in now:
+        assert n[0] <= 2 * was[0] + 3e-8 and n[1] <= 2 * was[1] + 1e-7, (was, now)

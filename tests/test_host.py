@@ -107,8 +107,10 @@ def test_packed_sizes_follow_the_layout():
     assert _lib.packed_bytes(_lib.PREC_BF16) == (frags(8) + fast1) * 1024 + tail
     assert _lib.packed_bytes(_lib.PREC_F16) == (frags(8) + fast1) * 1024 + tail
     assert _lib.packed_bytes(_lib.PREC_F32) == frags(4) * 1024 + tail
-    # fp32 by three parts: every fragment three times, and the low parts of the biases behind the tail
-    assert _lib.packed_bytes(_lib.PREC_F32S) == (3 * (frags(8) - 24 + 23 * 3) + 24 + 8 + 4 * 3 * 4) * 1024 + tail + 544 * 4
+    # fp32 by parts: every fragment three times, and the low parts of the biases behind the tail; as fp16 parts, then (256-byte
+    # aligned) as bf16 parts
+    parts = (3 * (frags(8) - 24 + 23 * 3) + 24 + 8 + 4 * 3 * 4) * 1024 + tail + 544 * 4
+    assert _lib.packed_bytes(_lib.PREC_F32S) == (parts + 255) // 256 * 256 + parts
     # bf16 + fp6: plus the e2m3 copy of the 3x3 layers (64-wide chunks, two fragments per chunk and
     # cout tile: 16 bytes per lane, then 8 bytes per lane packed densely) and its over-read padding
     lo = 0

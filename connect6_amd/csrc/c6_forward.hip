@@ -1922,6 +1922,7 @@ __global__ __launch_bounds__(256) void fused_forward_kernel(const FwdParams prm)
 #include "c6_duo.h"
 #if defined(C6_TEAM) || defined(C6_CASCADE) || !defined(C6_INSTANCE)
 #include "c6_team.h"
+#include "c6_half_team.h"
 #endif
 
 namespace c6 {

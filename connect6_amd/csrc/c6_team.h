@@ -12,7 +12,7 @@
 // What it takes (cycles of a 2.4 GHz clock; twelve workgroups, one board): staging the input 7 k, the first layer
 // 3 k (fp32 11 k), then per layer 1.2 k (fp32 1.8 k) until the neighbours' flags are seen, 0.5 k (fp32 1 k) until their squares are in LDS,
 // the MFMAs (bf16 0.5-2.1 k, fp32 2.8-6.9 k: three per product) and 1.3 k (fp32 2.6-2.9 k: two parts and the range) until the outputs are
-// stored and acknowledged, at the end 6 k (fp32 11 k) for the heads' sums: 66 k in bf16, 110 k in fp32.
+// stored and acknowledged, at the end 6 k (fp32 11 k) for the heads' sums: 66 k in bf16, 110 k in fp32 (c6_half_team.h).
 //
 // The exchange: loads of activations and flags carry the device-scope cache policy (sc1).  So do stores until a
 // workgroup has seen that all of its team run on its own XCD (each leaves its XCD's number beside the flags): from
@@ -46,9 +46,8 @@ template <class P> constexpr bool has_team() { return P::ID != C6_PREC_F32; }
 
 template <class P> struct TeamGeo {
   using G = Geo<P>;
-  static constexpr bool SPLIT = P::ID == C6_PREC_F32S;
-  static constexpr int NPL = SPLIT ? 2 : 1;                   // planes of an activation
-  static constexpr int WPL = SPLIT ? 2 : G::W;                // ... and of a 3x3 layer's weight that are contracted
+  static constexpr bool SPLIT = kParts<P> != 0;               // fp32 (two parts: c6_half_team.h)
+  static constexpr int NPL = SPLIT ? kParts<P> : 1;           // planes of an activation
   static constexpr int LO_OFF = NPL * 192;                    // fp6 blocks of a record (LO6)
   static constexpr int RECB = NPL * 192 + (P::LO6 ? 96 : 0) + 16;   // an odd number of 16-byte units
   // a square of c channels in memory: 16-byte units of its planes, then of its fp6 blocks
@@ -61,8 +60,8 @@ template <class P> struct TeamGeo {
   static constexpr int HEAD_OFF = act_off(7);                 // policy sums: SPLIT [3][384], else [384]
   // value sums: SPLIT one per (cout tile, tile of squares), else nine per lane of each tile of squares
   static constexpr int VAL_OFF = HEAD_OFF + 3 * 384 * 4;
-  static constexpr int NOTE_OFF = VAL_OFF + 12 * 9 * 64 * 4;   // SPLIT: a word per (layer, member, wave), half_note
-  static constexpr int BOARDB = (NOTE_OFF + (SPLIT ? 8 * 12 * 4 * 4 : 0) + 255) & ~255;
+  static constexpr int NOTE_OFF = VAL_OFF + 12 * 9 * 64 * 4;   // two parts: a word per (layer, member, wave), half_note
+  static constexpr int BOARDB = (NOTE_OFF + (kParts<P> == 2 ? 8 * 12 * 4 * 4 : 0) + 255) & ~255;
   // LDS: up to 11 rows of positions (128 squares lie in at most 8 board rows), 13 for 192 squares (SPLIT; in 11)
   static constexpr int REGION = ((SPLIT ? 13 : 11) * kPitch + 1) * RECB;
   // The first layer's shifted copies hold the halo rows that a workgroup's squares see: three per kernel row of up to
@@ -82,25 +81,17 @@ template <class P> struct TeamGeo {
 // tiles of squares each, whose four waves take PT of them and form CG groups of cout tiles.  A wave takes two
 // tiles of squares where there are two: with six workgroups each weight is then read by one wave, with three
 // by two; with one tile of squares per wave it would be twice as many, 96 and 128 bytes a cycle where the L1
-// gives 64 (six workgroups, 22 to 42 boards, bf16 + fp6 62.6 -> 55 us).
-// Three tiles of squares go to three waves, all cout tiles in each; the fourth watches the flags.
-// fp32, four or six tiles of squares (RAGGED): a wave takes half of them (PR).  Of two cout tiles it takes one; of three, one for all its
-// squares and the middle one for half of them, which balances the waves (nine tiles' MFMAs in each per k-step of four tiles of squares, fifteen of six:
-// the fourth group takes one of them a second time, to the same bytes) and has 64 bytes of weights a cycle or less asked for.  One cout
-// tile: the tiles of squares are dealt out to the waves.  (All cout tiles of one tile of squares per wave were 85 bytes a cycle, and two of
-// squares in three waves left one idle: 53 boards 96 -> 88 us, 85 boards 104 -> 95 us, 100 boards 132 -> 121 us, 128 boards 140 -> 130 us.)
+// gives 64 (six workgroups, 22 to 42 boards, bf16 + fp6 62.6 -> 55 us).  (fp32 contracts a weight with three parts, so
+// that a tile of squares per wave asks for just those 64, and all four waves have work in layers of two cout tiles.  Counted
+// over 53 boards, three workgroups each: of the 263 k cycles of a workgroup 150 k are reads from the L1, 64 bytes each, 128 k
+// MFMAs, so the L1 bounds the contractions by a sixth.)
+// Three or six tiles of squares go to three waves, all cout tiles in each; the fourth watches the flags.
 template <class P, int TEAM> struct TeamShape {
   static constexpr int PXT = 12 / TEAM;
-  static constexpr bool RAGGED = TeamGeo<P>::SPLIT && PXT >= 4;
-  static constexpr int PR = RAGGED ? PXT / 2 : 0;
-  static constexpr int PT = RAGGED ? PR : (PXT % 2 == 0 && !TeamGeo<P>::SPLIT ? 2 : 1), PG = PXT / PT;
+  static constexpr int PT = PXT == 6 ? 2 : (PXT % 2 == 0 && !TeamGeo<P>::SPLIT ? 2 : 1), PG = PXT / PT;
   static constexpr int CG = PG == 3 ? 1 : (PG == 1 ? (PXT == 1 ? 3 : 4) : 4 / PG);   // groups of squares' tiles, of cout tiles
-  static constexpr int tiles(int nt) { return RAGGED ? (nt == 3 ? 2 : 1) : (nt + CG - 1) / CG; }   // cout tiles of a wave
-  // ... and of its pairs of a tile of squares and a cout tile, tiles of squares: all cout tiles of each, or (RAGGED) one: team_used()
-  static constexpr int squares(int nt) { return !RAGGED ? PT : (nt == 3 ? PR + (PR + 1) / 2 : (nt == 2 ? PR : (PXT + 3) / 4)); }
+  static constexpr int tiles(int nt) { return (nt + CG - 1) / CG; }   // cout tiles of a wave
 };
-// does a wave have cout tile t of tile of squares p? (PR: of a ragged shape)
-template <int PR> constexpr bool team_used(int p, int t) { return PR == 0 || t == (p < PR ? 0 : 1); }
 
 // fragment (k-step k, cout tile t) of 3x3 layer L in the weight stream of mode P: first of its planes
 template <class P, int L> __device__ __forceinline__ int team_frag(int k, int t) {
@@ -118,15 +109,7 @@ template <class P, int L> __device__ __forceinline__ int team_frag(int k, int t)
 // k-steps of weights that a wave keeps in flight: the loads take some 800 cycles and a k-step is
 // 32 cycles per MFMA
 template <class P, int TT, int PT> constexpr int team_ring() {
-  // (fp32: three MFMAs per tile, PT of them in a ragged shape)
-  if (TeamGeo<P>::SPLIT) return PT * TT == 1 ? 9 : (PT >= 5 ? 2 : (PT >= 3 ? 3 : 6));
-  return Geo<P>::W == 1 ? 18 / TT : (TT == 1 ? 9 : (TT == 2 ? 6 : 3));
-}
-// ... and those of one unrolled round: a phase in the pipelined modes; fp32: a kernel row, or all three of them where a k-step is
-// so short that nine are in flight
-template <class P, int L, int TT, int PT> constexpr int team_round() {
-  if (P::PIPE) return kPhaseSteps;
-  return (PT * TT == 1 ? 9 : 3) * kCinArr[L] / 16;
+  return Geo<P>::W == 3 ? (PT > 1 ? 3 : 6) / TT : (Geo<P>::W == 1 ? 18 / TT : (TT == 1 ? 9 : (TT == 2 ? 6 : 3)));
 }
 
 // Low-order (fp6) pass of layer L for PT tiles of squares, conv3_lo_pass with TT cout tiles from t0 on.
@@ -174,102 +157,81 @@ __device__ __forceinline__ void team_lo_pass(const unsigned char *smem, const un
   });
 }
 
-// The contraction of 3x3 layer L for PT tiles of 32 squares and TT cout tiles, tile(t) of the layer's (beyond
-// its last they repeat it; their results are not used).
+// The contraction of 3x3 layer L for PT tiles of 32 squares and TT cout tiles from t0 on (tiles beyond
+// the layer's last repeat it; their results are not used).
 //   rec: LDS addresses of the lane's squares' records;  acc: the bias on entry
-//   fp32 (as half_layer): low: what the bias leaves out, for the small products' sum
-template <class P, int L, int TT, int PT, int PR, class Tile>
+//   low (fp32): what the bias leaves out, for the small products' sum (split_conv)
+template <class P, int L, int TT, int PT>
 __device__ __forceinline__ void team_conv(const unsigned char *smem, const unsigned char *packed, const WFrags &wl,
-                                          v4i (&ring)[team_ring<P, TT, PT>()][TT][TeamGeo<P>::WPL], int lane,
-                                          const int (&rec)[PT], Tile tile, f32x16 (&acc)[PT][TT],
+                                          v4i (&ring)[team_ring<P, TT, PT>()][TT][Geo<P>::W], int lane,
+                                          const int (&rec)[PT], int t0, f32x16 (&acc)[PT][TT],
                                           f32x16 (&low)[PT][TT]) {
   using T = TeamGeo<P>;
   constexpr int NT = kCoutArr[L] / 32, NTP = kCinArr[L] / 32;
-  constexpr int W = T::WPL, NPL = T::NPL, D = team_ring<P, TT, PT>();
+  constexpr int W = Geo<P>::W, NPL = T::NPL, D = team_ring<P, TT, PT>();
   constexpr int KC = kCinArr[L] / 16, KS = 9 * KC;
-  constexpr int U = team_round<P, L, TT, PT>();
+  constexpr int U = P::PIPE ? kPhaseSteps : 3 * KC;     // k-steps of one unrolled round
   constexpr bool LO = P::LO6 && ((P::LO_MASK >> L) & 1);
   static_assert(KS % U == 0 && U % D == 0, "ring");
   int corner[PT];
 #pragma unroll
   for (int p = 0; p < PT; ++p) corner[p] = rec[p] - (kPitch + 1) * T::RECB + 16 * (lane >> 5);
   // k-step v of round r: (tap, 16 channels).  Pipelined modes: a round is a phase, all taps of 32
-  // channels; fp32: a round is a kernel row, or all three.
+  // channels; fp32: a round is a kernel row.
   auto frag = [&](int r, int v, int p, int pl) __attribute__((always_inline)) {
     const int tap = v / 2;
-    const int off = P::PIPE ? ((tap / 3) * kPitch + tap % 3) * T::RECB + (v % 2) * 32
-                            : ((v / KC / 3) * kPitch + v / KC % 3) * T::RECB + (v % KC) * 32;
+    const int off = P::PIPE ? ((tap / 3) * kPitch + tap % 3) * T::RECB + (v % 2) * 32 : (v / KC) * T::RECB + (v % KC) * 32;
     const int base = P::PIPE ? r * 64 : r * kPitch * T::RECB;
     return *reinterpret_cast<const v4i *>(smem + corner[p] + base + off + pl * 192);
   };
-  // activations two k-steps ahead; one where that is nine MFMAs or more
-  constexpr int AHEAD = T::SPLIT && PT > 2 ? 1 : 2;
-  v4i a[AHEAD + 1][PT][NPL];
+  v4i a[3][PT][NPL];
 #pragma unroll
-  for (int v = 0; v < AHEAD; ++v)
+  for (int v = 0; v < 2; ++v)
 #pragma unroll
     for (int p = 0; p < PT; ++p)
 #pragma unroll
       for (int i = 0; i < NPL; ++i) a[v][p][i] = frag(0, v, p, i);
-  [[maybe_unused]] f32x16 sum[PT][TT];   // fp32: the largest products of a kernel row
   auto round = [&](int r) __attribute__((always_inline)) {
     // (the low-order pass comes in front of the last phase, as in pipe_layer)
     if constexpr (LO) {
-      if (r == NTP - 1) team_lo_pass<P, L, TT, PT>(smem, packed, lane, rec, tile(0), acc);
+      if (r == NTP - 1) team_lo_pass<P, L, TT, PT>(smem, packed, lane, rec, t0, acc);
     }
     static_for<0, U>([&](auto vc) __attribute__((always_inline)) {
       constexpr int v = decltype(vc)::value;
-      // (behind the last k-step: the last round again, unused)
-      const int rn = v + AHEAD < U ? r : (r + 1 < KS / U ? r + 1 : r);
+      // activations two k-steps ahead (behind the last one: the last round again, unused)
+      const int rn = v + 2 < U ? r : (r + 1 < KS / U ? r + 1 : r);
 #pragma unroll
       for (int p = 0; p < PT; ++p)
 #pragma unroll
-        for (int i = 0; i < NPL; ++i) a[(v + AHEAD) % (AHEAD + 1)][p][i] = frag(rn, (v + AHEAD) % U, p, i);
+        for (int i = 0; i < NPL; ++i) a[(v + 2) % 3][p][i] = frag(rn, (v + 2) % U, p, i);
       auto refill = [&](int t) __attribute__((always_inline)) {
         const int kn = r * U + v + D;   // (behind the last k-steps: the last one again, unused)
-        const int f = team_frag<P, L>(kn < KS ? kn : KS - 1, tile(t) < NT ? tile(t) : NT - 1);
+        const int f = team_frag<P, L>(kn < KS ? kn : KS - 1, t0 + t < NT ? t0 + t : NT - 1);
 #pragma unroll
         for (int i = 0; i < W; ++i) ring[v % D][t][i] = wl[f + i];
       };
-      if constexpr (T::SPLIT) {
-        // lo hi, hi hi, hi lo (weight, activation).  (An accumulator's next MFMA is eight cycles late if it follows at once: the
-        // two sums take turns, and so do two tiles.  With three the L1's 64 bytes a cycle bound the layer, and loads in a row per
-        // tile suit it better.)
-        constexpr int WP[3] = {1, 0, 0}, AP[3] = {0, 0, 1};
+      if constexpr (NPL == 3) {
+        // (An accumulator's next MFMA is eight cycles late if it follows at once, so two tiles take turns: forty boards
+        // 102 -> 97 us.  With three the L1's 64 bytes a cycle bound the layer, and loads in a row per tile suit it better:
+        // 56 boards 120 us, in turns 123.)
+        constexpr int WP[6] = {0, 1, 2, 0, 1, 0}, AP[6] = {2, 1, 0, 1, 0, 0};
         constexpr bool TURNS = TT == 2;
-        if constexpr (v % (3 * KC) == 0) {
 #pragma unroll
-          for (int p = 0; p < PT; ++p)
+        for (int o = 0; o < (TURNS ? 6 : TT); ++o)
 #pragma unroll
-            for (int t = 0; t < TT; ++t) sum[p][t] = f32x16{};
-        }
-#pragma unroll
-        for (int o = 0; o < (TURNS ? 3 : TT); ++o)
-#pragma unroll
-          for (int n = 0; n < (TURNS ? TT : 3); ++n) {
+          for (int n = 0; n < (TURNS ? TT : 6); ++n) {
             const int m = TURNS ? o : n, t = TURNS ? n : o;
 #pragma unroll
-            for (int p = 0; p < PT; ++p)
-              if (team_used<PR>(p, t)) mma<P>(ring[v % D][t][WP[m]], a[v % (AHEAD + 1)][p][AP[m]], m == 1 ? sum[p][t] : low[p][t]);
-            if (m == 2) refill(t);
+            for (int p = 0; p < PT; ++p) mma<P>(ring[v % D][t][WP[m]], a[v % 3][p][AP[m]], m < 5 ? low[p][t] : acc[p][t]);
+            if (m == 5) refill(t);
           }
-        if constexpr ((v + 1) % (3 * KC) == 0) {
-#pragma unroll
-          for (int p = 0; p < PT; ++p)
-#pragma unroll
-            for (int t = 0; t < TT; ++t) {
-              if (!team_used<PR>(p, t)) continue;
-#pragma unroll
-              for (int e = 0; e < 16; ++e) acc[p][t][e] = fmaf(sum[p][t][e], kHalfUnit, acc[p][t][e]);
-            }
-        }
       } else {
 #pragma unroll
         for (int t = 0; t < TT; ++t) {
 #pragma unroll
           for (int i = 0; i < W; ++i)
 #pragma unroll
-            for (int p = 0; p < PT; ++p) mma<P>(ring[v % D][t][i], a[v % (AHEAD + 1)][p][0], acc[p][t]);
+            for (int p = 0; p < PT; ++p) mma<P>(ring[v % D][t][i], a[v % 3][p][0], acc[p][t]);
           refill(t);
         }
       }
@@ -283,51 +245,63 @@ __device__ __forceinline__ void team_conv(const unsigned char *smem, const unsig
 #pragma unroll 1
     for (int r = 0; r < KS / U; ++r) round(r);
   }
-  if constexpr (T::SPLIT) {   // (or its products are put off until the sum is used, and their operands kept for that)
+  if constexpr (NPL == 3) {
 #pragma unroll
     for (int p = 0; p < PT; ++p)
 #pragma unroll
-      for (int t = 0; t < TT; ++t) {
-        if (!team_used<PR>(p, t)) continue;
-        asm volatile("" : "+a"(low[p][t]));
+      for (int t = 0; t < TT; ++t)
 #pragma unroll
-        for (int e = 0; e < 16; ++e) acc[p][t][e] = fmaf(low[p][t][e], kHalfUnit / kHalfLow, acc[p][t][e]);
-      }
+        for (int e = 0; e < 16; ++e) acc[p][t][e] = two_sums(acc[p][t][e], low[p][t][e]);
   }
 }
 
 // SiLU of one accumulator tile, step by step: a lone wave waits for each result that its next instruction needs.  Against
 // output by output it is worth a per cent, one way or the other: 22 to 40 boards in bf16 and fp16 40.0 -> 39.6 us, 40 boards that
-// a cascade lists 117.2 -> 116.2, but 1 to 16 boards in bf16 30.2 -> 30.6; the
-// teams beside whole rounds the same.  (fp32: HalfEpi.)
+// a cascade lists 117.2 -> 116.2, 86 to 128 fp32 boards 217.2 -> 215.5; but 1 to 16 boards in bf16 30.2 -> 30.6; one and 53 fp32
+// boards, and the teams beside whole rounds, the same.
 template <class P> __device__ __forceinline__ void silu_tile(const f32x16 &acc, float (&v)[16]) {
-  __builtin_amdgcn_sched_barrier(0);
+  if constexpr (TeamGeo<P>::SPLIT) {
+    float half[8];
 #pragma unroll
-  for (int e = 0; e < 16; ++e) v[e] = __builtin_amdgcn_exp2f(acc[e]);
-  __builtin_amdgcn_sched_barrier(0);
+    for (int e0 = 0; e0 < 16; e0 += 8) {
+      split_silu8(acc, e0, half);
 #pragma unroll
-  for (int e = 0; e < 16; ++e) v[e] = 1.0f + v[e];
-  __builtin_amdgcn_sched_barrier(0);
+      for (int e = 0; e < 8; ++e) v[e0 + e] = half[e];
+    }
+  } else {
+    __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-  for (int e = 0; e < 16; ++e) v[e] = __builtin_amdgcn_rcpf(v[e]);
-  __builtin_amdgcn_sched_barrier(0);
+    for (int e = 0; e < 16; ++e) v[e] = __builtin_amdgcn_exp2f(acc[e]);
+    __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-  for (int e = 0; e < 16; ++e) v[e] = acc[e] * v[e];
-  __builtin_amdgcn_sched_barrier(0);
+    for (int e = 0; e < 16; ++e) v[e] = 1.0f + v[e];
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int e = 0; e < 16; ++e) v[e] = __builtin_amdgcn_rcpf(v[e]);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int e = 0; e < 16; ++e) v[e] = acc[e] * v[e];
+    __builtin_amdgcn_sched_barrier(0);
+  }
 }
 
 // SiLU of one accumulator tile into the record at `rec` (cout tile t): planes, and the fp6 block.
-// UNDER: the one-workgroup kernel takes this tile's low-order parts behind MFMAs (see epi_atom).  most (fp32): the largest so far.
+// UNDER: the one-workgroup kernel takes this tile's low-order parts behind MFMAs (see epi_atom).
 template <class P, bool LO, bool UNDER>
-__device__ __forceinline__ void team_store(unsigned char *smem, int rec, int h, int t, const f32x16 &acc, float &most) {
+__device__ __forceinline__ void team_store(unsigned char *smem, int rec, int h, int t, const f32x16 &acc) {
   using T = TeamGeo<P>;
   unsigned char *at = smem + rec + 64 * t + 8 * h;
   if constexpr (T::SPLIT) {
-    const v16i v = half_activations(acc, most);
 #pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      *reinterpret_cast<v2i *>(at + 16 * q) = v2i{v[2 * q], v[2 * q + 1]};
-      *reinterpret_cast<v2i *>(at + 192 + 16 * q) = v2i{v[8 + 2 * q], v[8 + 2 * q + 1]};
+    for (int q = 0; q < 4; q += 2) {
+      float v[8];
+      int w[3][4];
+      split_silu8(acc, 4 * q, v);
+      split_planes8(v, w);
+#pragma unroll
+      for (int i = 0; i < 3; ++i)
+#pragma unroll
+        for (int e = 0; e < 2; ++e) *reinterpret_cast<v2i *>(at + i * 192 + 16 * (q + e)) = v2i{w[i][2 * e], w[i][2 * e + 1]};
     }
   } else {
     const DropConsts k = drop_consts<P>();
@@ -381,14 +355,13 @@ __device__ __forceinline__ void team_store(unsigned char *smem, int rec, int h, 
 // Board `b` by the team that this workgroup (its member my_role) belongs to; `slot`: the team's share of
 // the exchange memory and of the flags.
 template <class P, int TEAM>
-__device__ __forceinline__ bool team_board(const TeamParams &prm, unsigned char *smem, unsigned b, unsigned slot,
+__device__ __forceinline__ void team_board(const TeamParams &prm, unsigned char *smem, unsigned b, unsigned slot,
                                            int my_role) {
   using G = Geo<P>;
   using T = TeamGeo<P>;
   using S = TeamShape<P, TEAM>;
-  constexpr int NPL = T::NPL, W = G::W, WPL = T::WPL, THREADS = 256, PXT = S::PXT, CG = S::CG;
-  std::conditional_t<T::SPLIT, int, const int> tid = threadIdx.x, lane = tid & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), h = lane >> 5;
+  constexpr int NPL = T::NPL, W = G::W, THREADS = 256, PXT = S::PXT, PT = S::PT, CG = S::CG;
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), h = lane >> 5;
   const FwdParams &f = prm.f;
   unsigned char *occ = smem + T::OCC_OFF;
   float *lgt = reinterpret_cast<float *>(smem + T::LGT_OFF);
@@ -428,18 +401,9 @@ __device__ __forceinline__ bool team_board(const TeamParams &prm, unsigned char 
     else __hip_atomic_store(&flags[word], prm.tag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   };
   [[maybe_unused]] const bool trace_on = true;
-  // fp32: what this wave knows of the numbers in role's squares up to layer l (half_note); a word per layer, so that whoever
-  // goes on with another's squares finds it
-  bool bad_input = false, again = false;   // again: what team_board returns
-  [[maybe_unused]] unsigned trail = 0;
-  auto note_at = [&](int l, int role) { return T::NOTE_OFF + ((l * 12 + role) * 4 + wave) * 4; };
-  auto store_note = [&](int l, int role, float most, bool bad) __attribute__((always_inline)) {
-    trail = (l > 0 ? trail : 0) | half_note(l, most) | (bad ? 1u : 0u);
-    if (lane == 0) store4(__builtin_bit_cast(float, trail), note_at(l, role));
-  };
 
   // the wave's first tile of squares within the workgroup's, and its group of cout tiles
-  const int wpx = wave % S::PG * S::PT, cg = wave / S::PG;
+  const int wpx = wave % S::PG * PT, cg = wave / S::PG;
 
   // word l * 12 + role: the squares of stage l that the neighbours read are there; kTeamAll further on:
   // all of them
@@ -524,27 +488,21 @@ __device__ __forceinline__ bool team_board(const TeamParams &prm, unsigned char 
   auto part_lds = [](int k, int j) __attribute__((always_inline)) { return (k < NPL ? k * 192 : T::LO_OFF) + j * 16; };
 
   // Outputs of layer L (own squares): into the records, and to memory what the neighbours read.
-  // acc: N tiles of squares, px(i) of the workgroup's, and a wave's cout tiles, tile(t) of the layer's
-  auto write_out = [&](auto lc, auto nc, int role, const Span &sp, bool active, const auto &acc, auto px, auto tile) __attribute__((always_inline)) {
+  // acc: N tiles of squares from the workgroup's tile px on
+  auto write_out = [&](auto lc, auto nc, int role, const Span &sp, bool active, const auto &acc, int px, int t0) __attribute__((always_inline)) {
     constexpr int L = decltype(lc)::value, N = decltype(nc)::value, C = kCoutArr[L], NT = C / 32;
     constexpr int TT = S::tiles(NT);
     constexpr bool LO = P::LO6 && ((P::LO_MASK >> (L + 1)) & 1);
-    float most = 0.0f;
     if (active) {
 #pragma unroll
       for (int i = 0; i < N; ++i) {
-        const int p = sp.p0 + px(i) * 32 + (lane & 31), pc = p < kPix ? p : kPix - 1;
+        const int p = sp.p0 + (px + i) * 32 + (lane & 31), pc = p < kPix ? p : kPix - 1;
         const int rec = record(pc, sp.base);
 #pragma unroll
-        for (int t = 0; t < TT; ++t) {
-          if constexpr (S::RAGGED && L > 0) {
-            if (!team_used<S::PR>(i, t)) continue;
-          }
-          if (tile(t) < NT) team_store<P, LO, (L >= 2)>(smem, rec, h, tile(t), acc[i][t], most);
-        }
+        for (int t = 0; t < TT; ++t)
+          if (t0 + t < NT) team_store<P, LO, (L >= 2)>(smem, rec, h, t0 + t, acc[i][t]);
       }
     }
-    if constexpr (T::SPLIT) store_note(L, role, most, L == 0 && bad_input);
     __syncthreads();
     int sq, j;
     unit_of(IC<C>{}, sq, j);
@@ -573,29 +531,18 @@ __device__ __forceinline__ bool team_board(const TeamParams &prm, unsigned char 
 
   auto conv_stage = [&](auto lc, int role) __attribute__((always_inline)) -> bool {
     constexpr int L = decltype(lc)::value;
-    constexpr int NT = kCoutArr[L] / 32, TT = S::tiles(NT), PT = S::squares(NT), D = team_ring<P, TT, PT>();
+    constexpr int NT = kCoutArr[L] / 32, TT = S::tiles(NT), D = team_ring<P, TT, PT>();
     constexpr int C = kCinArr[L];
     // (opaque per stage: what follows from it is formed here and not, for all stages, in front of the
     // loop over them, in several hundred scalar registers that get spilled)
-    int t0 = S::RAGGED ? cg : cg * TT;
+    int t0 = cg * TT;
     asm volatile("" : "+s"(t0));
-    const bool active = S::RAGGED ? NT > 1 || wave * PT < PXT : cg < CG && t0 < NT;
-    // the wave's cout tiles (one beyond the layer's last repeats it, and is not used) and tiles of squares
-    auto tile = [&](int t) __attribute__((always_inline)) {
-      if constexpr (S::RAGGED) return NT == 3 ? (t == 0 ? 2 * t0 : 1) : (NT == 2 ? t0 : 0);
-      else return t0 + t;
-    };
-    auto tile_or_last = [&](int t) __attribute__((always_inline)) { return tile(t) < NT ? tile(t) : NT - 1; };
-    auto px = [&](int i) __attribute__((always_inline)) {
-      if constexpr (!S::RAGGED) return wpx + i;
-      else if constexpr (NT == 1) return wave * PT + i;
-      else return wpx + (i < S::PR ? i : (t0 == 0 ? i - S::PR : 2 * S::PR - 1 - i));
-    };
+    const bool active = cg < CG && t0 < NT;
     const Span sp = span_of(role);
     const WFrags wl = layer_weights<P, L>(packed, lane);
     C6_MARK(6 * L);
     const bool own = region_role == role && region_layer == L - 1;
-    v4i ring[D][TT][WPL];
+    v4i ring[D][TT][W];
     f32x16 acc[PT][TT], low[PT][TT];
     auto first_weights = [&]() __attribute__((always_inline)) {
 #pragma unroll
@@ -603,7 +550,7 @@ __device__ __forceinline__ bool team_board(const TeamParams &prm, unsigned char 
 #pragma unroll
         for (int t = 0; t < TT; ++t)
 #pragma unroll
-          for (int i = 0; i < WPL; ++i) ring[d][t][i] = wl[team_frag<P, L>(d, tile_or_last(t)) + i];
+          for (int i = 0; i < W; ++i) ring[d][t][i] = wl[team_frag<P, L>(d, t0 + t < NT ? t0 + t : NT - 1) + i];
       __builtin_amdgcn_sched_barrier(0);
     };
     // (on their way while the neighbours are waited for; the wave that does the waiting asks for its own behind that)
@@ -643,16 +590,12 @@ __device__ __forceinline__ bool team_board(const TeamParams &prm, unsigned char 
         to_region(q, v);
       }
     region_role = -1;   // (until the outputs are in place)
-    if constexpr (T::SPLIT) {
-      if (!own) trail = (unsigned)__builtin_amdgcn_raw_buffer_load_b32(mem, note_at(L - 1, role), 0, kSc1);
-    }
     if (active) {
 #pragma unroll
       for (int t = 0; t < TT; ++t) {
-        const int word = bias_offset(L) + 32 * tile_or_last(t);
+        const int word = bias_offset(L) + 32 * (t0 + t < NT ? t0 + t : NT - 1);
 #pragma unroll
         for (int i = 0; i < PT; ++i) {
-          if (!team_used<S::PR>(i, t)) continue;
           acc[i][t] = tail_tile(word);
           if constexpr (T::SPLIT) low[i][t] = tail_tile(G::TAIL_BIAS_LOW + word);
         }
@@ -665,45 +608,54 @@ __device__ __forceinline__ bool team_board(const TeamParams &prm, unsigned char 
     bool ok[PT];
 #pragma unroll
     for (int i = 0; i < PT; ++i) {
-      p[i] = sp.p0 + px(i) * 32 + (lane & 31);
+      p[i] = sp.p0 + (wpx + i) * 32 + (lane & 31);
       ok[i] = p[i] < kPix;
       rec[i] = record(ok[i] ? p[i] : kPix - 1, sp.base);
     }
-    if (active) team_conv<P, L, TT, PT, S::PR>(smem, packed, wl, ring, lane, rec, tile, acc, low);
+    if (active) team_conv<P, L, TT, PT>(smem, packed, wl, ring, lane, rec, t0, acc, low);
     C6_MARK(6 * L + 3);
     if constexpr (L < 7) {
       __syncthreads();   // everybody has read this layer's input
-      write_out(lc, IC<PT>{}, role, sp, active, acc, px, tile);
+      write_out(lc, IC<PT>{}, role, sp, active, acc, wpx, t0);
     } else {
       // heads: this wave's share of the policy (per square) and of the value
       const float *pw = tail + kBiasTotal + 4 * h;
+      const int tile = role * PXT + wpx;   // of the twelve
       if constexpr (T::SPLIT) {
-        float most = 0.0f;
         if (active) {
 #pragma unroll
           for (int t = 0; t < TT; ++t) {
-            if (tile(t) >= NT) continue;
-            HalfHeads out;
-            out.pw = tail_tile(kBiasTotal + 32 * tile(t));
-            out.vw = tail_tile(kBiasTotal + kHeadC + 32 * tile(t));
+            if (t0 + t >= NT) continue;
+            float pol[PT], val[PT];
+#pragma unroll
+            for (int i = 0; i < PT; ++i) pol[i] = val[i] = 0.0f;
+            float a[PT][16];
+#pragma unroll
+            for (int i = 0; i < PT; ++i) silu_tile<P>(acc[i][t], a[i]);
+#pragma unroll
+            for (int q = 0; q < 4; ++q)
+#pragma unroll
+              for (int e = 0; e < 4; ++e) {
+                const float p1 = pw[32 * (t0 + t) + 8 * q + e], v1 = pw[kHeadC + 32 * (t0 + t) + 8 * q + e];
+#pragma unroll
+                for (int i = 0; i < PT; ++i) {
+                  pol[i] = fmaf(a[i][4 * q + e], p1, pol[i]);
+                  val[i] = fmaf(a[i][4 * q + e], v1, val[i]);
+                }
+              }
 #pragma unroll
             for (int i = 0; i < PT; ++i) {
-              if (!team_used<S::PR>(i, t)) continue;
-              out.pol = out.val = 0.0f;
-              HalfEpi<true>::run(acc[i][t], out, most);
-              const unsigned bits = __builtin_bit_cast(unsigned, out.pol);
+              const unsigned bits = __builtin_bit_cast(unsigned, pol[i]);
               const auto x = __builtin_amdgcn_permlane32_swap(bits, bits, false, false);
               const unsigned x0 = x[0], x1 = x[1];
               const float tot = __builtin_bit_cast(float, x0) + __builtin_bit_cast(float, x1);
-              const float vs = wave_sum(ok[i] ? out.val : 0.0f);
-              if (h == 0 && ok[i]) store4(tot, T::HEAD_OFF + (tile(t) * 384 + p[i]) * 4);
-              if (lane == 0) store4(vs, T::VAL_OFF + (tile(t) * 12 + role * PXT + px(i)) * 4);
+              const float vs = wave_sum(ok[i] ? val[i] : 0.0f);
+              if (h == 0 && ok[i]) store4(tot, T::HEAD_OFF + ((t0 + t) * 384 + p[i]) * 4);
+              if (lane == 0) store4(vs, T::VAL_OFF + ((t0 + t) * 12 + tile + i) * 4);
             }
           }
         }
-        store_note(L, role, most, false);
       } else {
-        const int first = role * PXT + wpx;   // of the twelve tiles of squares
         // The one-workgroup kernel runs one chain of multiply-adds over the channels of a lane's
         // square, cout tile after cout tile: the groups of cout tiles take turns and hand it on.
         float *chain = reinterpret_cast<float *>(smem + T::OCC_OFF);   // (not in use before the last stage)
@@ -735,12 +687,12 @@ __device__ __forceinline__ bool team_board(const TeamParams &prm, unsigned char 
                   vs = fmaf(a, vw4[e], vs);
                 }
                 // (tile 0: one chain over its sixteen channels; the others: one sum per four)
-                if (t0 + t > 0) store4(vs, T::VAL_OFF + (((first + i) * 9 + 1 + 4 * (t0 + t - 1) + q) * 64 + lane) * 4);
+                if (t0 + t > 0) store4(vs, T::VAL_OFF + (((tile + i) * 9 + 1 + 4 * (t0 + t - 1) + q) * 64 + lane) * 4);
               }
             }
 #pragma unroll
             for (int i = 0; i < PT; ++i)
-              if (t0 + t == 0) store4(val0[i], T::VAL_OFF + ((first + i) * 9 * 64 + lane) * 4);
+              if (t0 + t == 0) store4(val0[i], T::VAL_OFF + ((tile + i) * 9 * 64 + lane) * 4);
           }
         }
 #pragma unroll
@@ -777,7 +729,7 @@ __device__ __forceinline__ bool team_board(const TeamParams &prm, unsigned char 
   // first layer: every workgroup stages the part of the board that its squares see
   auto first_stage = [&](int role) __attribute__((always_inline)) -> bool {
     const Span sp = span_of(role);
-    int *flag = reinterpret_cast<int *>(red) + 64;   // [0]: third plane varies, fp32: [1]: an input is not exact, [3] beyond the range, [4] not small
+    int *flag = reinterpret_cast<int *>(red) + 64;   // [0]: third plane varies, [1]: an input is not exact in bf16
     constexpr int N1 = PXT > 4 ? 2 : 1;   // (one cout tile: a wave per tile of squares, or per two)
     const int px = wave * N1 < PXT ? wave * N1 : 0;
     const bool active = wave * N1 < PXT;
@@ -835,7 +787,7 @@ __device__ __forceinline__ bool team_board(const TeamParams &prm, unsigned char 
 #pragma unroll
     for (int i = 0; i < TAIL_UNITS; ++i)
       if (tid + i * THREADS < G::TAIL_FLOATS / 4) reinterpret_cast<v4i *>(smem + T::TAIL_OFF)[tid + i * THREADS] = tl[i];
-    if (tid < 5 && tid != 2) flag[tid] = 0;
+    if (tid < 2) flag[tid] = 0;
     if (tid == 0) red[66] = xin[0][2];
     __syncthreads();
     const float c2 = red[66];
@@ -852,23 +804,16 @@ __device__ __forceinline__ bool team_board(const TeamParams &prm, unsigned char 
     const bool plane2_varies = flag[0] != 0;
     int parts = 1;
     if constexpr (T::SPLIT) {
-      bool inexact = false, beyond = false, ordinary = false;   // (as half_forward_kernel)
+      bool inexact = false;
 #pragma unroll
       for (int k = 0; k < 2; ++k)
         if (tid + k * THREADS < kPix)
 #pragma unroll
-          for (int ch = 0; ch < 3; ++ch) {
-            if (ch == 2 && !plane2_varies) continue;
-            inexact |= xin[k][ch] - half_value(half_bits(xin[k][ch])) != 0.0f;
-            beyond |= !half_fits(xin[k][ch]);
-            ordinary |= __builtin_fabsf(xin[k][ch]) >= kHalfLeast;
-          }
+          for (int ch = 0; ch < 3; ++ch)
+            inexact |= (ch < 2 || plane2_varies) && (__builtin_bit_cast(int, xin[k][ch]) & 0xffff) != 0;
       if (inexact) flag[1] = 1;
-      if (beyond) flag[3] = 1;
-      if (ordinary) flag[4] = 1;
       __syncthreads();
-      parts = flag[1] != 0 ? 2 : 1;
-      bad_input = parts > 1 && (flag[3] != 0 || flag[4] == 0);
+      parts = flag[1] != 0 ? 3 : 1;
     }
     const int rows = (plane2_varies ? G::STEPS1 : G::FAST1_STEPS) / 3;
     int row0[N1];
@@ -885,13 +830,17 @@ __device__ __forceinline__ bool team_board(const TeamParams &prm, unsigned char 
 #pragma unroll
       for (int n = 0; n < N1; ++n)
 #pragma unroll
-        for (int i = 0; i < 16; ++i) acc[n][0][i] = (T::SPLIT ? kHalfW : 1.0f) * (plane2_varies ? b0[i] : fmaf(c2, acc[n][0][i], b0[i]));
+        for (int i = 0; i < 16; ++i) acc[n][0][i] = plane2_varies ? b0[i] : fmaf(c2, acc[n][0][i], b0[i]);
     }
-    f32x16 low[N1], large[N1];   // SPLIT: small products; the large ones, once a second part follows
+    f32x16 low[N1], large[N1];   // SPLIT: small products; the large ones, once all parts but the first follow
+#pragma unroll
+    for (int n = 0; n < N1; ++n)
+#pragma unroll
+      for (int i = 0; i < 16; ++i) low[n][i] = large[n][i] = 0.0f;
     if constexpr (T::SPLIT) {
       if (active) {
 #pragma unroll
-        for (int n = 0; n < N1; ++n) low[n] = tail_tile(G::TAIL_BIAS_LOW + bias_offset(0)) * (1.0f / kHalfA);
+        for (int n = 0; n < N1; ++n) low[n] = tail_tile(G::TAIL_BIAS_LOW + bias_offset(0));
       }
     }
 #pragma unroll 1
@@ -908,8 +857,8 @@ __device__ __forceinline__ bool team_board(const TeamParams &prm, unsigned char 
           if (sq >= kPix) continue;
           unsigned short v16;
           if constexpr (T::SPLIT) {
-            v16 = half_bits(xin[k][ch]);
-            xin[k][ch] = (xin[k][ch] - half_value(v16)) * kHalfLow;
+            v16 = bf16_part(xin[k][ch]);
+            xin[k][ch] = bf16_rest(xin[k][ch], v16);
           } else {
             v16 = bits16<P>(xin[k][ch]);
           }
@@ -972,19 +921,14 @@ __device__ __forceinline__ bool team_board(const TeamParams &prm, unsigned char 
           if (row + decltype(sc)::value < rows) one_row(row + decltype(sc)::value, sc);
         });
         if constexpr (T::SPLIT) {
-          if (parts > 1) {   // (the second part's products with the weights' first are small ones, the others are dropped)
+          if (parts > 1 && part == 0) {
 #pragma unroll
-            for (int n = 0; n < N1; ++n)
+            for (int n = 0; n < N1; ++n) {
+              large[n] = acc[n][0];
+              acc[n][0] = low[n];
 #pragma unroll
-              for (int i = 0; i < 16; ++i) {
-                if (part == 0) {
-                  large[n][i] = acc[n][0][i];
-                  acc[n][0][i] = low[n][i];
-                } else {
-                  low[n][i] = acc[n][0][i];
-                  acc[n][0][i] = large[n][i];
-                }
-              }
+              for (int i = 0; i < 16; ++i) low[n][i] = 0.0f;
+            }
           }
         }
       }
@@ -993,22 +937,19 @@ __device__ __forceinline__ bool team_board(const TeamParams &prm, unsigned char 
 #pragma unroll
       for (int n = 0; n < N1; ++n)
 #pragma unroll
-        for (int i = 0; i < 16; ++i) acc[n][0][i] = fmaf(low[n][i], 1.0f / (kHalfW * kHalfLow), acc[n][0][i] * (1.0f / kHalfW));
+        for (int i = 0; i < 16; ++i)
+          acc[n][0][i] = parts > 1 ? two_sums(large[n][i], low[n][i] + acc[n][0][i]) : two_sums(acc[n][0][i], low[n][i]);
     }
     C6_MARK(2);
     __syncthreads();   // the copies give way to the activations
     clear_region(sp);
-    write_out(IC<0>{}, IC<N1>{}, role, sp, active, acc, [&](int i) { return px + i; }, [](int t) { return t; });
+    write_out(IC<0>{}, IC<N1>{}, role, sp, active, acc, px, 0);
     C6_MARK(3);
     return true;
   };
 
   // the heads' sums into logits, value, draw and (cascade) the list of close boards: one workgroup
   auto last_stage = [&](int role) __attribute__((always_inline)) -> bool {
-    [[maybe_unused]] unsigned *check = reinterpret_cast<unsigned *>(red) + 128;
-    if constexpr (T::SPLIT) {
-      if (tid == 0) *check = 0;
-    }
     const int got = wait_inputs(8, role, true);
     if (got != 1) return got == 2;
     region_role = -1;
@@ -1017,29 +958,14 @@ __device__ __forceinline__ bool team_board(const TeamParams &prm, unsigned char 
     auto partial = [&](int at) __attribute__((always_inline)) {
       return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(mem, at, 0, kSc1));
     };
-    // fp32: everything that is read here is asked for at once, and the value's sum runs beside the logits; a board's squares are
-    // known to be in range from the last layer's words alone (store_note).  (Words of all layers, then logits, then the value's
-    // 36 sums one after the other in one lane: 21 boards 59.1 -> 56.8 us, 42 boards 79 -> 77 us, one board 48.7 -> 47.8 us.)
-    [[maybe_unused]] float head[2][3], val = 0.0f;
-    [[maybe_unused]] unsigned note = 0;
-    if constexpr (T::SPLIT) {
-#pragma unroll
-      for (int k = 0; k < 2; ++k)
-#pragma unroll
-        for (int t = 0; t < 3; ++t) head[k][t] = partial(T::HEAD_OFF + (t * 384 + (tid + k * THREADS) % 384) * 4);   // (beyond 360: unused)
-      if (wave == 3) val = lane < 36 ? partial(T::VAL_OFF + lane * 4) : 0.0f;
-      else if (tid < TEAM * 4) note = __builtin_bit_cast(unsigned, partial(T::NOTE_OFF + (7 * 48 + tid) * 4));
-      __builtin_amdgcn_sched_barrier(0);
-      if (note != 0) atomicOr(check, note);
-      if (wave == 3 && f.value != nullptr) {   // (the sum needs its lanes together)
-        const double sum = split_value_sum(lane, [&](int) { return val; });
-        if (lane == 0) f.value[b] = split_value(sum, valb);
-      }
-    }
     const bool state = f.x_dtype == C6_DT_BOARD_I8;
     long long src = state && f.index ? f.index[b] : (long long)b;
     if (state) src = src < 0 ? 0 : (src >= f.num_states ? f.num_states - 1 : src);
-    auto put = [&](int p, float z) __attribute__((always_inline)) {
+    for (int p = tid; p < kPix; p += THREADS) {
+      float z = partial(T::HEAD_OFF + p * 4);
+      if constexpr (T::SPLIT) z = (z + partial(T::HEAD_OFF + (384 + p) * 4)) + partial(T::HEAD_OFF + (768 + p) * 4);
+      if constexpr (T::SPLIT) z = split_logit(z, polb);
+      else z += polb;
       bool taken;
       if (f.mask_mode == C6_MASK_LEGAL) {
         taken = f.legal[(size_t)b * kPix + p] == 0;
@@ -1060,15 +986,10 @@ __device__ __forceinline__ bool team_board(const TeamParams &prm, unsigned char 
         else if (f.logits_dtype == C6_DT_BF16) static_cast<unsigned short *>(f.logits)[at] = __builtin_bit_cast(unsigned short, (__bf16)v);
         else static_cast<unsigned short *>(f.logits)[at] = __builtin_bit_cast(unsigned short, (_Float16)v);
       }
-    };
-    if constexpr (T::SPLIT) {
-#pragma unroll
-      for (int k = 0; k < 2; ++k)
-        if (tid + k * THREADS < kPix) put(tid + k * THREADS, split_logit((head[k][0] + head[k][1]) + head[k][2], polb));
-    } else {
-      for (int p = tid; p < kPix; p += THREADS) put(p, partial(T::HEAD_OFF + p * 4) + polb);
     }
-    if constexpr (!T::SPLIT) {
+    if constexpr (T::SPLIT) {
+      if (tid < 36) red[tid] = partial(T::VAL_OFF + tid * 4);
+    } else {
       // as lane `lane` of wave `wave` of the one-workgroup kernel adds its three squares' sums up
       float part[3][9], vsum = 0.0f;
       bool valid[3];
@@ -1086,7 +1007,12 @@ __device__ __forceinline__ bool team_board(const TeamParams &prm, unsigned char 
       if (lane == 0) red[wave] = vsum;
     }
     __syncthreads();
-    if constexpr (!T::SPLIT) {
+    if constexpr (T::SPLIT) {
+      if (wave == 3 && f.value != nullptr) {   // (beside the draw)
+        const double sum = split_value_sum(lane, [&](int i) { return red[i]; });
+        if (lane == 0) f.value[b] = split_value(sum, valb);
+      }
+    } else {
       if (tid == 192 && f.value != nullptr) {   // (beside the draw and the margin)
         float s = 0.0f;
 #pragma unroll
@@ -1104,7 +1030,6 @@ __device__ __forceinline__ bool team_board(const TeamParams &prm, unsigned char 
         if (f.logprob != nullptr) f.logprob[b] = lp;
       }
     }
-    if constexpr (T::SPLIT) again = half_failed(__builtin_amdgcn_readfirstlane(*check));
     if constexpr (P::ID == C6_PREC_BF16) {
       if (f.redo_mode == kRedoDetect && wave == 1) {   // (a run of one board: see fused_pipe_kernel)
         const bool again = wave_margin_below(
@@ -1116,7 +1041,7 @@ __device__ __forceinline__ bool team_board(const TeamParams &prm, unsigned char 
         }
       }
     }
-    if constexpr (!T::SPLIT) raise_flag(8, role);   // (fp32: nobody waits for it)
+    raise_flag(8, role);
     C6_MARK(49);
     return true;
   };
@@ -1146,10 +1071,6 @@ __device__ __forceinline__ bool team_board(const TeamParams &prm, unsigned char 
       __syncthreads();
     }
     bool ok = false;
-    if constexpr (T::SPLIT) {   // (opaque: what follows from them is formed in each stage, and not kept for all of them)
-      asm volatile("" : "+v"(tid));
-      lane = tid & 63;
-    }
     switch (stage) {
       case 0: ok = first_stage(role); break;
       case 1: ok = conv_stage(IC<1>{}, role); break;
@@ -1165,7 +1086,6 @@ __device__ __forceinline__ bool team_board(const TeamParams &prm, unsigned char 
     help = !ok;
   }
   __syncthreads();
-  return again;
 }
 
 // How many workgroups share a board (team_size, below) when there are `boards` of them: as many as fit the chip at once, where
@@ -1181,7 +1101,7 @@ __device__ __forceinline__ bool team_board(const TeamParams &prm, unsigned char 
 // The most boards that teams of a size take:
 template <class P> __host__ __device__ inline long long team_most(int wgs, int size) {
   if (size == 6 && !TeamGeo<P>::SPLIT && !P::LO6) return wgs * 5 / 32;   // (where all teams have an XCD to themselves)
-  if (size == 3 && P::WLO == 1) return wgs * 2 / 7;
+  if (size == 3 && P::LO6 && P::WLO == 1) return wgs * 2 / 7;
   return wgs / size;
 }
 template <class P> constexpr int team_least() { return TeamGeo<P>::SPLIT ? 2 : (P::WLO ? 3 : 6); }
@@ -1212,37 +1132,32 @@ __device__ __forceinline__ TeamPlace team_place(unsigned items, int team, unsign
 }
 __device__ __forceinline__ TeamPlace team_place(unsigned items, int team) { return team_place(items, team, blockIdx.x, gridDim.x); }
 
-// A workgroup's share of board b, in a team of any size that the mode has.  (fp32) true: a number on the way was beyond what the
-// parts hold, and the board is this workgroup's to do again.
+// A workgroup's share of board b, in a team of any size that the mode has.
 template <class P>
-__device__ __forceinline__ bool team_share(const TeamParams &prm, unsigned char *smem, unsigned b, TeamPlace at, int team) {
-  if (team == 12) return team_board<P, 12>(prm, smem, b, at.slot, at.role);
-  if (team == 6) return team_board<P, 6>(prm, smem, b, at.slot, at.role);
+__device__ __forceinline__ void team_share(const TeamParams &prm, unsigned char *smem, unsigned b, TeamPlace at, int team) {
+  if (team == 12) team_board<P, 12>(prm, smem, b, at.slot, at.role);
+  if (team == 6) team_board<P, 6>(prm, smem, b, at.slot, at.role);
   if constexpr (team_least<P>() <= 3) {
-    if (team == 3) return team_board<P, 3>(prm, smem, b, at.slot, at.role);
+    if (team == 3) team_board<P, 3>(prm, smem, b, at.slot, at.role);
   }
   if constexpr (team_least<P>() <= 2) {
-    if (team == 2) return team_board<P, 2>(prm, smem, b, at.slot, at.role);
+    if (team == 2) team_board<P, 2>(prm, smem, b, at.slot, at.role);
   }
-  return false;
 }
 
+template <class P> __device__ __forceinline__ void half_team(const TeamParams &prm, unsigned char *smem);   // c6_half_team.h
 template <class P> __global__ __launch_bounds__(256) void team_forward_kernel(const TeamParams prm) {
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
+  if constexpr (kParts<P> == 2) {
+    half_team<P>(prm, smem);
+    return;
+  }
   const unsigned items = (unsigned)prm.f.total_boards;
   const int team = team_size<P>(items, (int)gridDim.x);
   if (team == 1) return;
   const TeamPlace at = team_place(items, team);
-  // fp32: the workgroup that ends a board does it again, alone, where it has to.  (In a launch behind this one, as for
-  // boards with a workgroup each: one board 47.7 -> 45.8 us, 21 boards 56.3 -> 53.7 us, 53 boards 84.9 -> 83.3 us, 128 boards
-  // 126.7 -> 124.3 us.)
-  const bool again = at.slot < items && team_share<P>(prm, smem, prm.first + at.slot, at, team);
-  if constexpr (TeamGeo<P>::SPLIT) {   // (behind the other stores of the outputs)
-    if (again) {
-      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-      __syncthreads();
-      split_board<true>(prm.f, smem, prm.first + at.slot);
-    }
+  if constexpr (kParts<P> != 2) {
+    if (at.slot < items) team_share<P>(prm, smem, prm.first + at.slot, at, team);
   }
 }
 

@@ -2331,7 +2331,7 @@ template <class P> int launch_left(const FwdParams &fp, int cus, hipStream_t st)
 
 #if defined(C6_TEAM) || defined(C6_CASCADE) || !defined(C6_INSTANCE)
 template <class P> int launch_team(const TeamParams &tp, int grid, hipStream_t st) {
-  constexpr int A = TeamGeo<P>::LDS_BYTES, B = TeamGeo<P>::SPLIT ? SplitGeo::LDS_BYTES : 0, LDS = A > B ? A : B;
+  constexpr int A = TeamGeo<P>::LDS_BYTES, B = kParts<P> == 2 ? TeamGeo<PrecF32X>::LDS_BYTES : 0, LDS = A > B ? A : B;
   static thread_local int configured = -1;
   int dev = 0;
   hipError_t e = hipGetDevice(&dev);
@@ -2514,7 +2514,7 @@ struct TeamMode {
   int (*rest)(long long boards, int cus);      // ... workgroups per board of a rest beside them
 };
 template <class P> static TeamMode team_mode_of() {
-  return {TeamGeo<P>::BOARDB, &team_size<P>, &team_most<P>, &launch_team<P>,
+  return {team_board_bytes<P>(), &team_size<P>, &team_most<P>, &launch_team<P>,
           has_duo<P>() ? &launch_rest<P> : nullptr, &rest_team<P>};
 }
 static TeamMode team_mode(int prec) {

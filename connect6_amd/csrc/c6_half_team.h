@@ -135,11 +135,12 @@ __device__ __forceinline__ void half_team_store(unsigned char *smem, int rec, in
   }
 }
 
-// Board `b` by the team that this workgroup (its member my_role) belongs to, as team_board.  true: a number on the way was beyond what
-// two parts hold, and the board is this workgroup's to do again.
+// Board `b` by the team that this workgroup (its member my_role) belongs to, as team_board; next: the slot's flags of the second way, cleared
+// here.  true, in the workgroup that ends the board (for the others it stands in word kTeamListed): a number on the way was beyond what two
+// parts hold, and the board is to be done again.
 template <int TEAM>
 __device__ __forceinline__ bool half_team_board(const TeamParams &prm, unsigned char *smem, unsigned b, unsigned slot,
-                                                int my_role) {
+                                                int my_role, unsigned *next) {
   using P = PrecF32S;
   using G = Geo<P>;
   using T = TeamGeo<P>;
@@ -531,6 +532,9 @@ __device__ __forceinline__ bool half_team_board(const TeamParams &prm, unsigned 
     if (varies) flag[0] = 1;
     // (the tag and the XCD in one word, at a place that holds nothing else; behind the input's loads, so that
     // nothing waits for its acknowledgement)
+    if (tid < 2 * kTeamStages + 1)   // (role's words; acknowledged in front of this stage's flag)
+      __hip_atomic_store(&next[tid < kTeamStages ? tid * 12 + role : (tid < 2 * kTeamStages ? kTeamAll + (tid - kTeamStages) * 12 : kTeamXcd) + role], 0u,
+                         __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     if (tid == 0 && role == my_role)
       __hip_atomic_store(&flags[kTeamXcd + role], xcd_tag ^ xcd, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     __syncthreads();
@@ -676,8 +680,6 @@ __device__ __forceinline__ bool half_team_board(const TeamParams &prm, unsigned 
 
   // the heads' sums into logits, value and draw: one workgroup
   auto last_stage = [&](int role) __attribute__((always_inline)) -> bool {
-    unsigned *check = reinterpret_cast<unsigned *>(red) + 128;
-    if (tid == 0) *check = 0;
     const int got = wait_inputs(8, role, true);
     if (got != 1) return got == 2;
     region_role = -1;
@@ -689,16 +691,25 @@ __device__ __forceinline__ bool half_team_board(const TeamParams &prm, unsigned 
     // Everything that is read here is asked for at once, and the value's sum runs beside the logits; a board's squares are
     // known to be in range from the last layer's words alone (store_note).  (Words of all layers, then logits, then the value's
     // 36 sums one after the other in one lane: 21 boards 59.1 -> 56.8 us, 42 boards 79 -> 77 us, one board 48.7 -> 47.8 us.)
+    static_assert(TEAM * 4 <= 64, "a wave reads the words");
     float head[2][3], val = 0.0f;
-    unsigned note = 0;
+    int note = 0;
 #pragma unroll
     for (int k = 0; k < 2; ++k)
 #pragma unroll
       for (int t = 0; t < 3; ++t) head[k][t] = partial(T::HEAD_OFF + (t * 384 + (tid + k * THREADS) % 384) * 4);   // (beyond 360: unused)
     if (wave == 3) val = lane < 36 ? partial(T::VAL_OFF + lane * 4) : 0.0f;
-    else if (tid < TEAM * 4) note = __builtin_bit_cast(unsigned, partial(T::NOTE_OFF + (7 * 48 + tid) * 4));
+    else if (wave == 0 && lane < TEAM * 4) note = __builtin_bit_cast(int, partial(T::NOTE_OFF + (7 * 48 + lane) * 4));
     __builtin_amdgcn_sched_barrier(0);
-    if (note != 0) atomicOr(check, note);
+    if (wave == 0) {   // the verdict, as early as it is known
+      again = half_failed((unsigned)wave_allreduce_bits(note, [](int a, int b) { return a | b; }));
+      if (again && lane == 0) store_flag(kTeamListed);
+      if (again) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+      if (lane == 0) {
+        store_flag(8 * 12 + role);
+        *word = again ? 1 : 0;
+      }
+    }
     if (wave == 3 && f.value != nullptr) {   // (the sum needs its lanes together)
       const double sum = split_value_sum(lane, [&](int) { return val; });
       if (lane == 0) f.value[b] = split_value(sum, valb);
@@ -727,6 +738,7 @@ __device__ __forceinline__ bool half_team_board(const TeamParams &prm, unsigned 
       if (f.logits != nullptr) static_cast<float *>(f.logits)[(size_t)b * kPix + sq] = masked ? f.fill : z;
     }
     __syncthreads();
+    again = __builtin_amdgcn_readfirstlane(*word) != 0;
     if (f.actions != nullptr && wave == 0) {
       int a;
       float lp;
@@ -737,7 +749,6 @@ __device__ __forceinline__ bool half_team_board(const TeamParams &prm, unsigned 
         if (f.logprob != nullptr) f.logprob[b] = lp;
       }
     }
-    again = half_failed(__builtin_amdgcn_readfirstlane(*check));   // (no flag: nobody waits for one)
     C6_MARK(49);
     return true;
   };
@@ -789,27 +800,44 @@ __device__ __forceinline__ bool half_team_board(const TeamParams &prm, unsigned 
 }
 
 // A workgroup's share of board b, in a team of any size.
-__device__ __forceinline__ bool half_team_share(const TeamParams &prm, unsigned char *smem, unsigned b, TeamPlace at, int team) {
-  if (team == 12) return half_team_board<12>(prm, smem, b, at.slot, at.role);
-  if (team == 6) return half_team_board<6>(prm, smem, b, at.slot, at.role);
-  if (team == 3) return half_team_board<3>(prm, smem, b, at.slot, at.role);
-  if (team == 2) return half_team_board<2>(prm, smem, b, at.slot, at.role);
+__device__ __forceinline__ bool half_team_share(const TeamParams &prm, unsigned char *smem, unsigned b, TeamPlace at, int team, unsigned *next) {
+  if (team == 12) return half_team_board<12>(prm, smem, b, at.slot, at.role, next);
+  if (team == 6) return half_team_board<6>(prm, smem, b, at.slot, at.role, next);
+  if (team == 3) return half_team_board<3>(prm, smem, b, at.slot, at.role, next);
+  if (team == 2) return half_team_board<2>(prm, smem, b, at.slot, at.role, next);
   return false;
 }
 
-template <class P> __device__ __forceinline__ void half_team(const TeamParams &prm, unsigned char *smem) {
-  const unsigned items = (unsigned)prm.f.total_boards;
-  const int team = team_size<P>(items, (int)gridDim.x);
-  if (team == 1) return;
-  const TeamPlace at = team_place(items, team);
-  // The workgroup that ends a board does it again, alone, where it has to.  (In a launch behind this one, as for
-  // boards with a workgroup each: one board 47.7 -> 45.8 us, 21 boards 56.3 -> 53.7 us, 53 boards 84.9 -> 83.3 us, 128 boards
-  // 126.7 -> 124.3 us.)
-  if (at.slot < items && half_team_share(prm, smem, prm.first + at.slot, at, team)) {
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // (behind the other stores of the outputs)
+// A board that two parts do not hold is done again by its team with three: one board 111 us, 53 boards 200, 128 boards 330 (by the workgroup
+// that ends it, alone, 314, 347 and 380).  The members wait for the last stage's verdict, which is given as soon as that stage's loads have
+// arrived, so that they end with the workgroup that gives it: boards in range take what they took (given behind the outputs one board 45.2 ->
+// 45.7 us, 85 boards 98.5 -> 99.6 us).  The second way has exchange memory and flags of its own, behind the first one's: a member that comes late may
+// still be at its part of the first.
+template <class P> __device__ __forceinline__ void half_team(const TeamParams &prm, unsigned char *smem, unsigned items, TeamPlace at, int team) {
+  TeamParams exact = prm;
+  exact.f.packed += kSplitOffset;
+  exact.act += (size_t)items * TeamGeo<P>::BOARDB;
+  exact.flags = reinterpret_cast<unsigned *>(exact.act + (size_t)items * TeamGeo<PrecF32X>::BOARDB);
+  const unsigned b = prm.first + at.slot;
+  bool again = half_team_share(prm, smem, b, at, team, exact.flags + (size_t)at.slot * kTeamFlags);
+  if (at.role != 0) {
+    const unsigned *flags = prm.flags + (size_t)at.slot * kTeamFlags;
+    auto is_set = [&](int w) { return __hip_atomic_load(&flags[w], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == prm.tag; };
+    int *verdict = reinterpret_cast<int *>(smem);
+    if (threadIdx.x < 64) {
+      // (bounded as every wait; a team without a member that left here finishes by itself)
+      int found = -1;
+      for (int k = 0; k < prm.polls && found < 0; ++k)
+        if (is_set(8 * 12)) found = is_set(kTeamListed) ? 1 : 0;
+      if (threadIdx.x == 0) *verdict = found;
+    }
     __syncthreads();
-    split_board<true>(prm.f, smem, prm.first + at.slot);
+    again = __builtin_amdgcn_readfirstlane(*verdict) == 1;
   }
+  if (!again) return;
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // (behind the other stores of the outputs)
+  __syncthreads();
+  team_share<PrecF32X>(exact, smem, b, at, team);
 }
 
 }  // namespace c6

@@ -1112,6 +1112,11 @@ template <class P> __host__ __device__ inline int team_size(long long boards, in
   return 1;
 }
 
+// exchange memory per board (fp32: of both ways through it, and the second one's flags)
+template <class P> constexpr size_t team_board_bytes() {
+  if constexpr (kParts<P> == 2) return TeamGeo<P>::BOARDB + TeamGeo<PrecF32X>::BOARDB + kTeamFlags * 4;
+  else return TeamGeo<P>::BOARDB;
+}
 template <class P> inline long long team_most(int wgs) { return team_most<P>(wgs, team_least<P>()); }
 
 // Which team this workgroup belongs to (`items` of them; a slot beyond: to none) and as which member.  A team
@@ -1145,20 +1150,17 @@ __device__ __forceinline__ void team_share(const TeamParams &prm, unsigned char 
   }
 }
 
-template <class P> __device__ __forceinline__ void half_team(const TeamParams &prm, unsigned char *smem);   // c6_half_team.h
+// fp32: c6_half_team.h
+template <class P> __device__ __forceinline__ void half_team(const TeamParams &prm, unsigned char *smem, unsigned items, TeamPlace at, int team);
 template <class P> __global__ __launch_bounds__(256) void team_forward_kernel(const TeamParams prm) {
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
-  if constexpr (kParts<P> == 2) {
-    half_team<P>(prm, smem);
-    return;
-  }
   const unsigned items = (unsigned)prm.f.total_boards;
   const int team = team_size<P>(items, (int)gridDim.x);
   if (team == 1) return;
   const TeamPlace at = team_place(items, team);
-  if constexpr (kParts<P> != 2) {
-    if (at.slot < items) team_share<P>(prm, smem, prm.first + at.slot, at, team);
-  }
+  if (at.slot >= items) return;
+  if constexpr (kParts<P> == 2) half_team<P>(prm, smem, items, at, team);
+  else team_share<P>(prm, smem, prm.first + at.slot, at, team);
 }
 
 // The plain 16-bit modes with a few boards beyond whole rounds of one board per CU: teams for them in one launch with the

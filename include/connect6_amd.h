@@ -193,7 +193,7 @@ int c6_forward_boards_cascade(const int8_t *boards, const int8_t *player,
  * most of the chip idle, all the time or in their last round; the same results, bit for bit.
  * c6_team_bytes gives the sizes of the two buffers, or 0 and 0 where one workgroup per board is the
  * better launch (or the mode has no such kernel): call c6_forward there.
- *   workspace  device, 16-byte aligned; contents need no preparation.  Per shared board 0.7 MB
+ *   workspace  device, 16-byte aligned; contents need no preparation.  Per shared board 1.7 MB
  *              (C6_PREC_F32S), 0.5 MB (C6_PREC_BF16F6, _BF16F6W and the cascades), 0.35 MB (C6_PREC_BF16,
  *              _F16); of 256 CUs at most 128, 42 or 73, and 80 boards are shared.  A cascade over at most 21
  *              boards is one launch and takes both its passes' share

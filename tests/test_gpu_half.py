@@ -8,6 +8,7 @@ from connect6_amd import _lib
 from connect6_amd.model import run_forward
 from connect6_amd.synthetic import gen_boards, gen_uniform
 from oracle import torch_ref as R
+from tests.test_gpu_team import _team
 from tests.util import rel_l2
 
 pytestmark = pytest.mark.gpu
@@ -200,3 +201,42 @@ def test_small_weights_of_the_first_layer(cuda, factors):
     was, now = _against_float64(cuda, st, x, (6, 60, 200, 600))
     for n in now:
         assert n[0] <= 2 * was[0] + 3e-8 and n[1] <= 2 * was[1] + 1e-7, (was, now)
+
+
+@pytest.mark.parametrize("boards", [1, 7, 30, 60, 100])
+def test_a_team_without_all_its_members_does_a_board_again(cuda, boards):
+    """Boards of either kind in teams whose waits run out at once, so that members leave before the verdict or come late, and in
+    ordinary ones."""
+    st, x = _case("planes", 40000.0)
+    packed = _model(cuda, st).packed_weights(PREC)
+    xd = x[(torch.arange(boards) + 1) % 40].to(cuda)
+    flags = torch.zeros(boards * 256, dtype=torch.int32, device=cuda)
+    with torch.inference_mode():
+        want = run_forward(torch.cat([xd] * (300 // boards + 1)), packed, PREC, 1, boards * (300 // boards + 1))
+        for tag, polls in ((1, 1), (2, 2), (3, 5), (4, 0), (5, 1)):
+            lg, vg = _team(PREC, xd, packed, tag, flags, polls)
+            assert torch.equal(lg, want[0][:boards]) and torch.equal(vg, want[1][:boards]), polls
+
+
+@pytest.mark.parametrize("boards", [20, 300])
+def test_graphs_of_boards_that_take_either_way(cuda, boards):
+    st, x = _case("planes", 40000.0)
+    model = _model(cuda, st)
+    xs = [x[(torch.arange(boards) + i) % 40].to(cuda) for i in range(3)]
+    with torch.inference_mode():
+        want = [model(v) for v in xs]
+        static = xs[0].clone()
+        side = torch.cuda.Stream()
+        side.wait_stream(torch.cuda.current_stream())
+        with torch.cuda.stream(side):
+            model(static)
+        torch.cuda.current_stream().wait_stream(side)
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph):
+            out = model(static)
+        for i in (0, 1, 2, 1, 0):
+            static.copy_(xs[i])
+            graph.replay()
+            model(xs[2])                       # eager work in between
+            torch.cuda.synchronize()
+            assert torch.equal(out[0], want[i][0]) and torch.equal(out[1], want[i][1]), i

@@ -158,10 +158,9 @@ __host__ __device__ constexpr int lo6_channel(int block, int slot) {
   return 32 * block + 8 * (i >> 2) + 4 * hh + (i & 3);
 }
 
-// Factors of weights and activations there, of the second parts, the largest number that counts as within the range, and how
-// small a layer's largest may be.  kHalfMark: a weight that is beyond it (an fp16 NaN).
-constexpr float kHalfW = 16.0f, kHalfA = 16.0f, kHalfLow = 2048.0f, kHalfMost = 32768.0f, kHalfLeast = 0x1p-14f;
-constexpr int kHalfMark = 0x7fff;
+// Factors of activations there and of the second parts, the largest number that counts as within the range, and how small a layer's
+// largest may be.
+constexpr float kHalfA = 16.0f, kHalfLow = 2048.0f, kHalfMost = 32768.0f, kHalfLeast = 0x1p-7f;
 
 template <class P> struct Geo {
   static constexpr int EB = P::EB;
@@ -239,7 +238,8 @@ template <class P> struct Geo {
   static constexpr int FAST1_FRAGS = EB == 2 ? FAST1_STREAM + 8 + PLANE2_FRAGS : 0;
   static constexpr int TOTAL_FRAGS = HI_FRAGS + LO_FRAGS + FAST1_FRAGS;
   static constexpr size_t TAIL_OFF = (size_t)TOTAL_FRAGS * 1024;  // fp32 tail: biases, heads
-  // tail words: bias[544] polw[96] valw[96] polb valb pad pad, then 8 ints sw[layer]
+  // tail words: bias[544] polw[96] valw[96] polb valb pad pad, then 8 ints sw[layer]; fp32 by two parts: 8 floats, what a layer's
+  // sums have to be multiplied by (half_scale_kernel), or 0 where two parts do not hold its weights
   static constexpr int TAIL_SW = kBiasTotal + 2 * kHeadC + 4;
   // fp32 by parts: then what rounding the scaled biases to fp32 left out (by two: in the units of the small products' sum)
   static constexpr int TAIL_BIAS_LOW = TAIL_SW + 8;

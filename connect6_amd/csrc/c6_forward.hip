@@ -1960,9 +1960,9 @@ template <class P> __device__ __forceinline__ float weight_part(Scaled<P> v, int
   }
 }
 
-// One weight's `part` as element e of a lane's 16 bytes
-template <class P> __device__ __forceinline__ void put_weight(unsigned char *dst, int e, Scaled<P> v, int part) {
-  if constexpr (kParts<P> == 2) reinterpret_cast<unsigned short *>(dst)[e] = half_parts(v).part[part];
+// One weight's `part` as element e of a lane's 16 bytes (factor: of layer 0, fp32 by two parts)
+template <class P> __device__ __forceinline__ void put_weight(unsigned char *dst, int e, Scaled<P> v, int part, [[maybe_unused]] float factor) {
+  if constexpr (kParts<P> == 2) reinterpret_cast<unsigned short *>(dst)[e] = half_parts(v * factor).part[part];
   else put_elem<P>(dst, e, weight_part<P>(v, part));
 }
 
@@ -1990,6 +1990,13 @@ struct GroupView {
 template <class P> __device__ __forceinline__ void pack_thread(const GroupView &prm, long long gid) {
   using G = Geo<P>;
   const long long nfl = (long long)G::TOTAL_FRAGS * 64;
+  // the factor of a layer's weights, fp32 by two parts (where they do not hold the weights, what is packed is not used)
+  [[maybe_unused]] auto half_unit = [&](int l) { return reinterpret_cast<const float *>(prm.packed + G::TAIL_OFF)[G::TAIL_SW + l]; };
+  auto half_factor = [&](int l) -> float {
+    if constexpr (kParts<P> != 2) return 1.0f;
+    const float unit = half_unit(l);
+    return unit == 0.0f ? 0.0f : half_inverse(unit) * (l > 0 ? 1.0f / kHalfA : 1.0f);
+  };
   if (gid < nfl) {
     const int frag = (int)(gid >> 6), lane = (int)(gid & 63);
     const int m = lane & 31, h = lane >> 5;
@@ -2029,7 +2036,7 @@ template <class P> __device__ __forceinline__ void pack_thread(const GroupView &
         const float *w = prm.conv_w(0);
         for (int e = 0; e < G::E; ++e) {
           const int kx = jj * G::E + e;
-          put_weight<P>(dst, e, act_scaled<P>(kx < kK1 ? w[((m * 3 + h) * kK1 + ky) * kK1 + kx] : 0.0f), part);
+          put_weight<P>(dst, e, act_scaled<P>(kx < kK1 ? w[((m * 3 + h) * kK1 + ky) * kK1 + kx] : 0.0f), part, half_factor(0));
         }
         return;
       }
@@ -2092,17 +2099,18 @@ template <class P> __device__ __forceinline__ void pack_thread(const GroupView &
         const int kx = jj * G::E + e;
         Scaled<P> v = 0;
         if (row < kK1 * 3 && kx < kK1) v = act_scaled<P>(w[((co * 3 + ch) * kK1 + ky) * kK1 + kx]);
-        put_weight<P>(dst, e, v, part);
+        put_weight<P>(dst, e, v, part, half_factor(0));
       }
     } else if constexpr (kParts<P> == 2) {
       // (tap-major; the first tap's thread takes all nine: what their parts leave is balanced over them)
       const int kc_per_tap = cin / G::KSTEP;
       if (part != 0 || s >= kc_per_tap) return;
+      const float factor = half_factor(l);
       v4i o[9][3];
 #pragma unroll
       for (int e = 0; e < G::E; ++e) {
         HalfParts taps[9];
-        half_taps(w + (size_t)(co * cin + s * G::KSTEP + h * G::E + e) * 9, taps);
+        half_taps(w + (size_t)(co * cin + s * G::KSTEP + h * G::E + e) * 9, factor, taps);
 #pragma unroll
         for (int k = 0; k < 9; ++k)
 #pragma unroll
@@ -2134,7 +2142,7 @@ template <class P> __device__ __forceinline__ void pack_thread(const GroupView &
       const int cot = 32 * tile + m;
       for (int e = 0; e < G::E; ++e) {
         const int c = cbase + h * G::E + e;
-        put_weight<P>(dst, e, w[(cot * cin + c) * 9 + tap], part);
+        put_weight<P>(dst, e, w[(cot * cin + c) * 9 + tap], part, 1.0f);
       }
     }
     return;
@@ -2150,10 +2158,15 @@ template <class P> __device__ __forceinline__ void pack_thread(const GroupView &
   if (ti >= G::TAIL_BIAS_LOW && ti < G::TAIL_FLOATS) {
     const Scaled<P> b = conv_bias(ti - G::TAIL_BIAS_LOW);
     const float low = (float)(b - (float)b);
-    constexpr float unit = kParts<P> == 2 ? 1.0f / (kHalfW * kHalfA * kHalfLow) : 1.0f;
-    tail[ti] = low == low ? low / unit : 0.0f;   // (an infinite bias leaves nothing)
+    float unit = 1.0f;   // (of the small products' sum)
+    if constexpr (kParts<P> == 2) {
+      int l = 0;
+      while (ti - G::TAIL_BIAS_LOW >= bias_offset(l + 1)) ++l;
+      unit = half_unit(l) * (1.0f / kHalfLow);
+    }
+    tail[ti] = low == low && unit != 0.0f ? low / unit : 0.0f;   // (an infinite bias leaves nothing)
   }
-  if (ti < G::TAIL_SW) {  // the sw[] words behind it are written by lo_scale_kernel
+  if (ti < G::TAIL_SW) {  // the sw[] words behind it are written by lo_scale_kernel or half_scale_kernel
     constexpr float head_scale = kParts<P> != 0 ? 1.0f : act_scale<P>();
     float v = 0.0f;
     if (ti < kBiasTotal) {
@@ -2219,6 +2232,79 @@ template <class P> __global__ __launch_bounds__(256) void lo_scale_kernel(const 
   }
 }
 
+// fp32 by two parts: the layers' units, a block per layer.  The factor is the power of two that takes the layer's largest weight
+// to [2^14, 2^15), where two parts resolve 2^-50 of that weight.  0, and the set goes through c6_split.h, where a layer has
+//  * an infinity or a NaN, or a largest weight outside 2^-46 ... 2^74 (a unit and a bias's low word are then fp32 numbers),
+//  * an output all of whose weights are small beside the layer's (below 2^-10, but for zeros): two parts could drop them, or
+//  * an input that one of its outputs takes little of (below 2^-6 of the largest weight of that output).  half_failed sees that
+//    the largest input is not small; only so is it known that the sum is not one over small inputs alone, whose last bits two
+//    parts drop.  (Of 2.4e5 kernels of six networks with either initialisation the smallest such share is 0.11, the smallest output's
+//    largest weight 0.5 of its layer's.)
+template <class P> __global__ __launch_bounds__(1024) void half_scale_kernel(const PackParams all) {
+  using G = Geo<P>;
+  const GroupView prm(all, blockIdx.y);
+  constexpr int STRIDE = 97;
+  __shared__ float most[96 * STRIDE], row_most[96];
+  __shared__ int loose;
+  const int l = blockIdx.x, tid = threadIdx.x, cin = kCinArr[l], cout = kCoutArr[l];
+  const float *w = prm.conv_w(l);
+  if (tid == 0) loose = 0;
+  auto larger = [](float m, float v) { return __builtin_elementwise_maximum(m, __builtin_fabsf(v)); };   // (a NaN stays one)
+  if (l == 0) {   // a wave per kernel
+    for (int k = tid >> 6; k < cout * 3; k += 16) {
+      float m = 0.0f;
+      for (int i = tid & 63; i < kK1 * kK1; i += 64) m = larger(m, w[k * kK1 * kK1 + i]);
+      for (int d = 32; d > 0; d >>= 1) m = larger(m, __shfl_xor(m, d));
+      if ((tid & 63) == 0) most[k / 3 * STRIDE + k % 3] = m * 1.5f;   // (the weights there carry -log2(e), 1.44)
+    }
+  } else {
+    constexpr int AT_ONCE = 3;
+    for (int k = tid; k < cout * cin; k += AT_ONCE * 1024) {
+      float v[AT_ONCE][9];
+#pragma unroll
+      for (int j = 0; j < AT_ONCE; ++j)
+#pragma unroll
+        for (int i = 0; i < 9; ++i) v[j][i] = k + j * 1024 < cout * cin ? w[(k + j * 1024) * 9 + i] : 0.0f;
+#pragma unroll
+      for (int j = 0; j < AT_ONCE; ++j) {
+        const int n = k + j * 1024;
+        if (n >= cout * cin) break;
+        float m = 0.0f;
+#pragma unroll
+        for (int i = 0; i < 9; ++i) m = larger(m, v[j][i]);
+        most[n / cin * STRIDE + n % cin] = m;
+      }
+    }
+  }
+  __syncthreads();
+  bool uneven = false;
+  if (tid < cout) {
+    float m = 0.0f, least = INFINITY;
+#pragma unroll 8
+    for (int c = 0; c < cin; ++c) {
+      m = larger(m, most[tid * STRIDE + c]);
+      least = fminf(least, most[tid * STRIDE + c]);
+    }
+    row_most[tid] = m;
+    uneven = !(least >= m * 0x1p-6f);
+  }
+  __syncthreads();
+  float largest = 0.0f;
+#pragma unroll 8
+  for (int c = 0; c < cout; ++c) largest = larger(largest, row_most[c]);
+  if (tid < cout) uneven |= row_most[tid] != 0.0f && !(row_most[tid] >= largest * 0x1p-10f);
+  if (uneven) loose = 1;
+  __syncthreads();
+  if (tid == 0) {
+    float unit = 1.0f;   // (all weights zero)
+    if (largest != 0.0f) {
+      const bool within = largest >= 0x1p-46f && largest <= 0x1p74f && loose == 0;
+      unit = within ? __builtin_bit_cast(float, (__builtin_bit_cast(int, largest) & 0x7f800000) - (14 << 23)) : 0.0f;
+    }
+    reinterpret_cast<float *>(prm.packed + G::TAIL_OFF)[G::TAIL_SW + l] = l > 0 ? unit * (1.0f / kHalfA) : unit;
+  }
+}
+
 // ------------------------------------------------------------------------
 // host side
 // ------------------------------------------------------------------------
@@ -2240,6 +2326,7 @@ template <class P> int launch_pack(const PackParams &pp, hipStream_t st) {
   const int blocks = pack_blocks<P>() + (kParts<P> == 2 ? pack_blocks<PrecF32X>() : 0);
   const unsigned sets = (unsigned)pp.groups;
   if constexpr (P::LO6) hipLaunchKernelGGL(lo_scale_kernel<P>, dim3(8, sets), dim3(256), 0, st, pp);
+  if constexpr (kParts<P> == 2) hipLaunchKernelGGL(half_scale_kernel<P>, dim3(8, sets), dim3(1024), 0, st, pp);
   hipLaunchKernelGGL(pack_kernel<P>, dim3(blocks, sets), dim3(kPackThreads), 0, st, pp);
   const hipError_t e = hipGetLastError();
   if (e != hipSuccess) {

@@ -23,11 +23,17 @@
 // (three products with one sum per layer and every lo rounded to nearest are off by 5.6e-7 and, from the last layer on in 64
 // bits, 2.2e-7 with the reference's initialisation; half of what the values gained is their sum over the board in 64 bits.)
 //
-// fp16 ends at 65504 and is exact to 2^-24 of itself in two parts down to 2^-14; all numbers carry factors for that: weights
-// 2^4, activations 2^4 (and -log2(e), as in c6_split.h).  So two parts hold what they should while weights are below 2048 (and
-// no less than 2e-13, first layer 2e-10, but for zeros), activations below 1400 and the largest activation of each layer's above 5e-6.  A board for which that does not hold, or
-// that has an infinity or a NaN anywhere, is seen at its end: every layer keeps the largest of what it stored (half_note), and a
-// weight beyond the range is packed as a NaN.  Such a board goes through c6_split.h, which has packed weights of its own.
+// fp16 ends at 65504, and two parts hold a number to 2^-24 of itself down to 2^-14, below that to 2^-36 (the unit of the second
+// part's subnormals).  All numbers carry factors for that.  A layer's weights: the power of two that takes the largest of them to
+// [2^14, 2^15) (half_scale_kernel), so that they are held to 2^-50 of the largest.  Activations: 2^4 (and -log2(e), as in
+// c6_split.h), so that they are held to 2^-24 of themselves or 6e-13.
+// What is not held so goes through c6_split.h, which has packed weights of its own:
+//  * a set of weights with an infinity, a NaN, or a layer whose weights are too unequal (half_scale_kernel has the rule): known when
+//    the set is packed, so that none of its boards starts here;
+//  * a board with activations beyond 1400 or none beyond 3.4e-4 in a layer that has any (but for the last), with an infinity or a
+//    NaN, seen at its end: every layer keeps the largest of what it stored (half_note).
+// What an output's sum loses to small inputs is then at most 2^-20 of it, and that if its weights for all others are 64 times the
+// one for the input that is not small.
 //
 // What bounds it: the matrix cores, 195 k cycles per board (the 1,890 MFMAs of the 3x3 layers and the first layer's 207 three
 // times each) of 330 k at 1.9 GHz; what goes in the open is the epilogue of each layer's last cout tile (5 k), the sums at the ends of kernel rows
@@ -39,22 +45,22 @@
 
 namespace c6 {
 
-// Parts of a weight that carries kHalfW: two as above, and what they leave of it, in units of the second (first layer) or times
-// 2^11 once more (the others, where nothing reads it).  A weight beyond the range, or so small that the parts would hold
-// few of its bits, is a NaN, with itself (the fp32 number `raw`) in the other two.
+// Parts of a weight that carries its layer's factor: two as above, and what they leave of it, in units of the second (first layer) or
+// times 2^11 once more (the others, where nothing reads it).
 struct HalfParts {
   unsigned short part[3];
 };
+// What layer l's sums have to be multiplied by to be pre-activations (a scalar load, behind its use in no register of a lane's)
+__device__ __forceinline__ float half_unit(const float *tail, int l) {
+  typedef const __attribute__((address_space(4))) float scalar;
+  return *reinterpret_cast<scalar *>(reinterpret_cast<uintptr_t>(tail + Geo<PrecF32S>::TAIL_SW + l));
+}
+// A power of two's reciprocal
+__device__ __forceinline__ float half_inverse(float p) { return __builtin_bit_cast(float, 0x7f000000 - __builtin_bit_cast(int, p)); }
 __device__ __forceinline__ unsigned short half_bits(float v) { return __builtin_bit_cast(unsigned short, (_Float16)v); }
 __device__ __forceinline__ float half_value(unsigned short b) { return (float)__builtin_bit_cast(_Float16, b); }
-__device__ __forceinline__ HalfParts half_marked(float raw) {
-  const unsigned b = __builtin_bit_cast(unsigned, raw);
-  return {{(unsigned short)kHalfMark, (unsigned short)b, (unsigned short)(b >> 16)}};
-}
 __device__ __forceinline__ bool half_fits(float v) { return __builtin_fabsf(v) <= kHalfMost; }   // (no NaN does)
-__device__ __forceinline__ HalfParts half_parts(double w) {
-  const double v = w * kHalfW;
-  if (!half_fits((float)v) || (w != 0.0 && __builtin_fabs(w) < 0x1p-32)) return half_marked((float)w);
+__device__ __forceinline__ HalfParts half_parts(double v) {
   const unsigned short hi = half_bits((float)v);
   const double rest = (v - half_value(hi)) * kHalfLow;
   const unsigned short lo = half_bits((float)rest);
@@ -62,16 +68,12 @@ __device__ __forceinline__ HalfParts half_parts(double w) {
 }
 // The nine taps of one channel of a 3x3 layer.  Where lo lies half-way between two fp16 numbers it takes the one that makes the
 // sum of what the taps leave smaller; then the smallest lo, whose steps are the finest, takes that sum in.
-__device__ __forceinline__ void half_taps(const float *w, HalfParts (&out)[9]) {
+__device__ __forceinline__ void half_taps(const float *w, float factor, HalfParts (&out)[9]) {
   float rest[9], sum = 0.0f, least = __builtin_inff();
   int fine = -1;
 #pragma unroll
   for (int k = 0; k < 9; ++k) {
-    const float v = w[k] * kHalfW;
-    if (!half_fits(v) || (w[k] != 0.0f && __builtin_fabsf(w[k]) < 0x1p-42f)) {
-      out[k] = half_marked(w[k]);
-      continue;
-    }
+    const float v = w[k] * factor;
     const unsigned short hi = half_bits(v);
     rest[k] = (v - half_value(hi)) * kHalfLow;
     unsigned short lo = half_bits(rest[k]);
@@ -91,7 +93,6 @@ __device__ __forceinline__ void half_taps(const float *w, HalfParts (&out)[9]) {
   }
 #pragma unroll
   for (int k = 0; k < 9; ++k) {
-    if (out[k].part[0] == kHalfMark) continue;
     if (k == fine) out[k].part[1] = half_bits(half_value(out[k].part[1]) + sum);
     out[k].part[2] = half_bits((rest[k] - half_value(out[k].part[1])) * kHalfLow);
   }
@@ -105,9 +106,6 @@ struct HalfGeo {
   static constexpr int PIXB = SplitGeo::PIXB, PLANEB = 192;
   static constexpr int CHECK = 44;   // words of RED: [0] half_note's, [1] an input is out of range, [2] one is not small
 };
-
-// What a sum over a 3x3 layer's products has to be multiplied by to be the pre-activation
-constexpr float kHalfUnit = 1.0f / (kHalfW * kHalfA);
 
 // ---- range ----
 // What a wave's lanes stored of layer l (m: the largest magnitude of a lane's, NaN if there was one), in one word
@@ -239,13 +237,14 @@ struct HalfIdle {};
 // products goes to held at its end, the others' sum, low, runs through (from what the bias leaves out); at the end held is the
 // pre-activation.
 template <int L, int T0, int TN, class Queue>
-__device__ __forceinline__ void half_conv(const unsigned char *smem, const unsigned char *packed, HalfStart<TN> &start, const int (&ci)[3],
+__device__ __forceinline__ void half_conv(const unsigned char *smem, const unsigned char *packed, const float *tail, HalfStart<TN> &start, const int (&ci)[3],
                                           int lane, f32x16 (&held)[TN][3], Queue &queue, float &m) {
   constexpr int NT = kCoutArr[L] / 32, KC = kCinArr[L] / 16, U = 3 * KC, D = kHalfRing<TN>, SLOTS = U * TN * 9;
   static_assert(U % D == 0 && U % 2 == 0, "double buffers must line up across rows");
   constexpr int UN = std::is_same_v<Queue, HalfIdle> ? 0 : sizeof(Queue) / sizeof(f32x16) / 3;
   const int h = lane >> 5;
   const WFrags wl = layer_weights<PrecF32S, L>(packed, lane);
+  const float unit = half_unit(tail, L);
   float minus = -1.0f;
   asm volatile("" : "+s"(minus));   // (q - hi as one instruction that takes hi as it is)
   int at[3][4];   // the lane's squares at a tap: where units 32 k (k = 0 ... 3) of a 128-byte block are
@@ -315,7 +314,7 @@ __device__ __forceinline__ void half_conv(const unsigned char *smem, const unsig
         // (out of the accumulation registers here, and not all tiles' at once)
         asm volatile("" : "+a"(sum[t][j]));
 #pragma unroll
-        for (int e = 0; e < 16; ++e) held[t][j][e] = fmaf(sum[t][j][e], kHalfUnit, held[t][j][e]);
+        for (int e = 0; e < 16; ++e) held[t][j][e] = fmaf(sum[t][j][e], unit, held[t][j][e]);
         __builtin_amdgcn_sched_barrier(0);
       }
     if constexpr (UN > 0) {
@@ -331,7 +330,7 @@ __device__ __forceinline__ void half_conv(const unsigned char *smem, const unsig
     for (int j = 0; j < 3; ++j) {
       asm volatile("" : "+a"(low[t][j]));
 #pragma unroll
-      for (int e = 0; e < 16; ++e) held[t][j][e] = fmaf(low[t][j][e], kHalfUnit / kHalfLow, held[t][j][e]);
+      for (int e = 0; e < 16; ++e) held[t][j][e] = fmaf(low[t][j][e], unit * (1.0f / kHalfLow), held[t][j][e]);
       __builtin_amdgcn_sched_barrier(0);
     }
 }
@@ -351,16 +350,16 @@ __device__ __forceinline__ void half_layer(unsigned char *smem, const unsigned c
   HalfQueue<TN> queue;
   HalfIdle idle;
   if constexpr (NT == 1) {
-    half_conv<L, 0, 1>(smem, packed, start, ci, lane, held, idle, m);
+    half_conv<L, 0, 1>(smem, packed, tail, start, ci, lane, held, idle, m);
   } else {
     f32x16 first[TN][3];
-    half_conv<L, 0, TN>(smem, packed, start, ci, lane, first, idle, m);
+    half_conv<L, 0, TN>(smem, packed, tail, start, ci, lane, first, idle, m);
     HalfStart<1> second = half_start<L, TN, 1>(packed, tail, lane);
 #pragma unroll
     for (int t = 0; t < TN; ++t)
 #pragma unroll
       for (int j = 0; j < 3; ++j) queue.q[j * TN + t] = first[t][j];
-    half_conv<L, TN, 1>(smem, packed, second, ci, lane, held, queue, m);
+    half_conv<L, TN, 1>(smem, packed, tail, second, ci, lane, held, queue, m);
   }
   next = half_start<L + 1, 0, TNN>(packed, tail, lane);
   __syncthreads();   // every wave has finished reading the layer's input
@@ -500,16 +499,34 @@ __global__ __launch_bounds__(256) void half_forward_kernel(const FwdParams prm) 
   if (b >= b_end) return;
   v4i r1[L1Pipe<P>::D][1];
   bool again = false;
-  fetch_board(b);
+  // A set of weights that two parts do not hold: none of its boards starts here, but where a run has boards of other sets too.
+  // (256 boards of such a set 490 -> 325 us, 2,048 boards 3,660 -> 2,260 us.)
+  auto unheld = [&](const unsigned char *packed) __attribute__((always_inline)) {
+    bool none = false;
+#pragma unroll
+    for (int l = 0; l < 8; ++l) none |= half_unit(reinterpret_cast<const float *>(packed + G::TAIL_OFF), l) == 0.0f;
+    return none;
+  };
+  {
+    bool all = true;
+    for (long long i = b; all && i < b_end; i = ((unsigned)i / per_group + 1ll) * per_group) all = unheld(packed_of(i));
+    if (all) {
+      again = half_redone(per);
+      for (long long i = b + tid; !again && i < b_end; i += THREADS) half_leave(prm, i);
+      b = b_end;
+    }
+  }
+  if (b < b_end) fetch_board(b);
 
   for (; b < b_end; ++b) {
     int tidv = tid;
     asm volatile("" : "+v"(tidv));
     const unsigned char *packed = packed_of(b);
     const float *tail = reinterpret_cast<const float *>(packed + G::TAIL_OFF);
-    unsigned note = 0;
+    unsigned note = unheld(packed) ? 1 : 0;
     __syncthreads();  // previous board fully written out; LDS is free
     preload_ring<L1Pipe<P>::D, 1>(r1, packed_frags<P>(packed, lane, G::FAST1_OFF));
+    const float unit0 = half_unit(tail, 0);
     // the third plane's share of the first layer, should the plane be constant (see fused_pipe_kernel)
     f32x16 a0[1][3];
     {
@@ -562,12 +579,13 @@ __global__ __launch_bounds__(256) void half_forward_kernel(const FwdParams prm) 
       f32x16 b0[1], bl[1];
       load_bias_tiles(b0, tail + bias_offset(0), h);
       load_bias_tiles(bl, tail + G::TAIL_BIAS_LOW + bias_offset(0), h);
+      const float factor = half_inverse(unit0);
 #pragma unroll
       for (int j = 0; j < 3; ++j)
 #pragma unroll
         for (int i = 0; i < 16; ++i) {
-          a0[0][j][i] = kHalfW * (plane2_varies ? b0[0][i] : fmaf(c2, a0[0][j][i], b0[0][i]));
-          low[0][j][i] = bl[0][i] * (1.0f / kHalfA);   // (the inputs carry no factor)
+          a0[0][j][i] = factor * (plane2_varies ? b0[0][i] : fmaf(c2, a0[0][j][i], b0[0][i]));
+          low[0][j][i] = bl[0][i];
         }
     }
     // An input that is exact in fp16 (stones, flags) is one part; what is left of any other is staged behind it, for the
@@ -653,7 +671,7 @@ __global__ __launch_bounds__(256) void half_forward_kernel(const FwdParams prm) 
         __builtin_amdgcn_sched_barrier(0);
         asm volatile("" : "+a"(small), "+a"(large));
 #pragma unroll
-        for (int i = 0; i < 16; ++i) u[i] = fmaf(small[i], 1.0f / (kHalfW * kHalfLow), large[i] * (1.0f / kHalfW));
+        for (int i = 0; i < 16; ++i) u[i] = fmaf(small[i], unit0 * (1.0f / kHalfLow), large[i] * unit0);
         half_put(smem, pos, h, 0, half_activations(u, m));
       }
       note |= half_note(0, m);
@@ -689,14 +707,14 @@ __global__ __launch_bounds__(256) void half_forward_kernel(const FwdParams prm) 
       };
       {
         f32x16 u[2][3];
-        half_conv<7, 0, 2>(smem, packed, two, ci, lane, u, idle, m);
+        half_conv<7, 0, 2>(smem, packed, tail, two, ci, lane, u, idle, m);
         one = half_start<7, 2, 1>(packed, tail, lane);
         head(0, u[0]);
         head(1, u[1]);
       }
       if (b + 1 < b_end) fetch_board(b + 1);  // lands while this board is finished
       f32x16 u[1][3];
-      half_conv<7, 2, 1>(smem, packed, one, ci, lane, u, idle, m);
+      half_conv<7, 2, 1>(smem, packed, tail, one, ci, lane, u, idle, m);
       head(2, u[0]);
       note |= half_note(7, m);
       if (lane == 0) atomicOr(check, note);

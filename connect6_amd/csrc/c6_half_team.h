@@ -33,11 +33,11 @@ template <int L, int TT, int PT> constexpr int half_team_round() { return (PT * 
 
 // The contraction of 3x3 layer L for PT tiles of 32 squares and TT cout tiles, tile(t) of the layer's (beyond
 // its last they repeat it; their results are not used), as half_conv.
-//   rec: LDS addresses of the lane's squares' records;  acc: the bias on entry, low: what it leaves out
+//   rec: LDS addresses of the lane's squares' records;  unit: the layer's;  acc: the bias on entry, low: what it leaves out
 template <int L, int TT, int PT, int PR, class Tile>
 __device__ __forceinline__ void half_team_conv(const unsigned char *smem, const unsigned char *packed, const WFrags &wl,
                                                v4i (&ring)[half_team_ring<TT, PT>()][TT][2], int lane,
-                                               const int (&rec)[PT], Tile tile, f32x16 (&acc)[PT][TT],
+                                               const int (&rec)[PT], Tile tile, float unit, f32x16 (&acc)[PT][TT],
                                                f32x16 (&low)[PT][TT]) {
   using T = TeamGeo<PrecF32S>;
   constexpr int NT = kCoutArr[L] / 32, W = Geo<PrecF32S>::W, NPL = T::NPL, D = half_team_ring<TT, PT>();
@@ -106,7 +106,7 @@ __device__ __forceinline__ void half_team_conv(const unsigned char *smem, const 
           for (int t = 0; t < TT; ++t) {
             if (!team_used<PR>(p, t)) continue;
 #pragma unroll
-            for (int e = 0; e < 16; ++e) acc[p][t][e] = fmaf(sum[p][t][e], kHalfUnit, acc[p][t][e]);
+            for (int e = 0; e < 16; ++e) acc[p][t][e] = fmaf(sum[p][t][e], unit, acc[p][t][e]);
           }
       }
       __builtin_amdgcn_sched_barrier(0);
@@ -120,7 +120,7 @@ __device__ __forceinline__ void half_team_conv(const unsigned char *smem, const 
       if (!team_used<PR>(p, t)) continue;
       asm volatile("" : "+a"(low[p][t]));
 #pragma unroll
-      for (int e = 0; e < 16; ++e) acc[p][t][e] = fmaf(low[p][t][e], kHalfUnit / kHalfLow, acc[p][t][e]);
+      for (int e = 0; e < 16; ++e) acc[p][t][e] = fmaf(low[p][t][e], unit * (1.0f / kHalfLow), acc[p][t][e]);
     }
 }
 
@@ -136,10 +136,12 @@ __device__ __forceinline__ void half_team_store(unsigned char *smem, int rec, in
 }
 
 // Board `b` by the team that this workgroup (its member my_role) belongs to, as team_board; next: the slot's flags of the second way, cleared
-// here.  true, in the workgroup that ends the board (for the others it stands in word kTeamListed): a number on the way was beyond what two
-// parts hold, and the board is to be done again.
+// here.  kHalfAgain, in the workgroup that ends the board (for the others it stands in word kTeamListed): a number on the way was beyond
+// what two parts hold, and the board is to be done again.  kHalfUnheld, in every member and before any has raised a flag: two parts do not
+// hold the weights.
+enum HalfHow { kHalfDone, kHalfAgain, kHalfUnheld };
 template <int TEAM>
-__device__ __forceinline__ bool half_team_board(const TeamParams &prm, unsigned char *smem, unsigned b, unsigned slot,
+__device__ __forceinline__ HalfHow half_team_board(const TeamParams &prm, unsigned char *smem, unsigned b, unsigned slot,
                                                 int my_role, unsigned *next) {
   using P = PrecF32S;
   using G = Geo<P>;
@@ -189,7 +191,8 @@ __device__ __forceinline__ bool half_team_board(const TeamParams &prm, unsigned 
   [[maybe_unused]] const bool trace_on = true;
   // what this wave knows of the numbers in role's squares up to layer l (half_note); a word per layer, so that whoever
   // goes on with another's squares finds it
-  bool bad_input = false, again = false;   // again: what is returned
+  bool bad_input = false;
+  HalfHow how = kHalfDone;
   unsigned trail = 0;
   auto note_at = [&](int l, int role) { return T::NOTE_OFF + ((l * 12 + role) * 4 + wave) * 4; };
   auto store_note = [&](int l, int role, float most, bool bad) __attribute__((always_inline)) {
@@ -350,6 +353,7 @@ __device__ __forceinline__ bool half_team_board(const TeamParams &prm, unsigned 
     };
     const Span sp = span_of(role);
     const WFrags wl = layer_weights<P, L>(packed, lane);
+    const float unit = __builtin_bit_cast(float, __builtin_amdgcn_readfirstlane(__builtin_bit_cast(int, tail[G::TAIL_SW + L])));
     C6_MARK(6 * L);
     const bool own = region_role == role && region_layer == L - 1;
     v4i ring[D][TT][2];
@@ -423,7 +427,7 @@ __device__ __forceinline__ bool half_team_board(const TeamParams &prm, unsigned 
       ok[i] = p[i] < kPix;
       rec[i] = record(ok[i] ? p[i] : kPix - 1, sp.base);
     }
-    if (active) half_team_conv<L, TT, PT, S::PR>(smem, packed, wl, ring, lane, rec, tile, acc, low);
+    if (active) half_team_conv<L, TT, PT, S::PR>(smem, packed, wl, ring, lane, rec, tile, unit, acc, low);
     C6_MARK(6 * L + 3);
     if constexpr (L < 7) {
       __syncthreads();   // everybody has read this layer's input
@@ -538,6 +542,14 @@ __device__ __forceinline__ bool half_team_board(const TeamParams &prm, unsigned 
     if (tid == 0 && role == my_role)
       __hip_atomic_store(&flags[kTeamXcd + role], xcd_tag ^ xcd, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     __syncthreads();
+    // (the same in every member)
+    float held = 1.0f;
+#pragma unroll
+    for (int l = 0; l < 8; ++l) held = tail[G::TAIL_SW + l] == 0.0f ? 0.0f : held;
+    if (__builtin_amdgcn_ballot_w64(held == 0.0f) != 0) {
+      how = kHalfUnheld;
+      return true;
+    }
     const bool plane2_varies = flag[0] != 0;
     bool inexact = false, beyond = false, ordinary = false;   // (as half_forward_kernel)
 #pragma unroll
@@ -566,17 +578,18 @@ __device__ __forceinline__ bool half_team_board(const TeamParams &prm, unsigned 
     }
     const int rowb = (plane2_varies ? 1 : 3) * kL1RowPitch * G::EB;
     const WFrags wl = plane2_varies ? layer_weights<P, 0>(packed, lane) : packed_frags<P>(packed, lane, G::FAST1_OFF);
+    const float unit = tail[G::TAIL_SW], factor = half_inverse(unit);
     if (active) {
       const f32x16 b0 = tail_tile(bias_offset(0));
 #pragma unroll
       for (int n = 0; n < N1; ++n)
 #pragma unroll
-        for (int i = 0; i < 16; ++i) acc[n][0][i] = kHalfW * (plane2_varies ? b0[i] : fmaf(c2, acc[n][0][i], b0[i]));
+        for (int i = 0; i < 16; ++i) acc[n][0][i] = factor * (plane2_varies ? b0[i] : fmaf(c2, acc[n][0][i], b0[i]));
     }
     f32x16 low[N1], large[N1];   // small products; the large ones, once a second part follows
     if (active) {
 #pragma unroll
-      for (int n = 0; n < N1; ++n) low[n] = tail_tile(G::TAIL_BIAS_LOW + bias_offset(0)) * (1.0f / kHalfA);
+      for (int n = 0; n < N1; ++n) low[n] = tail_tile(G::TAIL_BIAS_LOW + bias_offset(0));
     }
 #pragma unroll 1
     for (int part = 0; part < parts; ++part) {
@@ -669,7 +682,7 @@ __device__ __forceinline__ bool half_team_board(const TeamParams &prm, unsigned 
 #pragma unroll
     for (int n = 0; n < N1; ++n)
 #pragma unroll
-      for (int i = 0; i < 16; ++i) acc[n][0][i] = fmaf(low[n][i], 1.0f / (kHalfW * kHalfLow), acc[n][0][i] * (1.0f / kHalfW));
+      for (int i = 0; i < 16; ++i) acc[n][0][i] = fmaf(low[n][i], unit * (1.0f / kHalfLow), acc[n][0][i] * unit);
     C6_MARK(2);
     __syncthreads();   // the copies give way to the activations
     clear_region(sp);
@@ -702,7 +715,7 @@ __device__ __forceinline__ bool half_team_board(const TeamParams &prm, unsigned 
     else if (wave == 0 && lane < TEAM * 4) note = __builtin_bit_cast(int, partial(T::NOTE_OFF + (7 * 48 + lane) * 4));
     __builtin_amdgcn_sched_barrier(0);
     if (wave == 0) {   // the verdict, as early as it is known
-      again = half_failed((unsigned)wave_allreduce_bits(note, [](int a, int b) { return a | b; }));
+      const bool again = half_failed((unsigned)wave_allreduce_bits(note, [](int a, int b) { return a | b; }));
       if (again && lane == 0) store_flag(kTeamListed);
       if (again) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
       if (lane == 0) {
@@ -738,7 +751,7 @@ __device__ __forceinline__ bool half_team_board(const TeamParams &prm, unsigned 
       if (f.logits != nullptr) static_cast<float *>(f.logits)[(size_t)b * kPix + sq] = masked ? f.fill : z;
     }
     __syncthreads();
-    again = __builtin_amdgcn_readfirstlane(*word) != 0;
+    if (__builtin_amdgcn_readfirstlane(*word) != 0) how = kHalfAgain;
     if (f.actions != nullptr && wave == 0) {
       int a;
       float lp;
@@ -792,20 +805,21 @@ __device__ __forceinline__ bool half_team_board(const TeamParams &prm, unsigned 
       case 7: ok = conv_stage(IC<7>{}, role); break;
       default: ok = last_stage(role); break;
     }
+    if (how == kHalfUnheld) break;
     if (ok && stage == l && role == my_role) ++l;
     help = !ok;
   }
   __syncthreads();
-  return again;
+  return how;
 }
 
 // A workgroup's share of board b, in a team of any size.
-__device__ __forceinline__ bool half_team_share(const TeamParams &prm, unsigned char *smem, unsigned b, TeamPlace at, int team, unsigned *next) {
+__device__ __forceinline__ HalfHow half_team_share(const TeamParams &prm, unsigned char *smem, unsigned b, TeamPlace at, int team, unsigned *next) {
   if (team == 12) return half_team_board<12>(prm, smem, b, at.slot, at.role, next);
   if (team == 6) return half_team_board<6>(prm, smem, b, at.slot, at.role, next);
   if (team == 3) return half_team_board<3>(prm, smem, b, at.slot, at.role, next);
   if (team == 2) return half_team_board<2>(prm, smem, b, at.slot, at.role, next);
-  return false;
+  return kHalfDone;
 }
 
 // A board that two parts do not hold is done again by its team with three: one board 111 us, 53 boards 200, 128 boards 330 (by the workgroup
@@ -819,8 +833,11 @@ template <class P> __device__ __forceinline__ void half_team(const TeamParams &p
   exact.act += (size_t)items * TeamGeo<P>::BOARDB;
   exact.flags = reinterpret_cast<unsigned *>(exact.act + (size_t)items * TeamGeo<PrecF32X>::BOARDB);
   const unsigned b = prm.first + at.slot;
-  bool again = half_team_share(prm, smem, b, at, team, exact.flags + (size_t)at.slot * kTeamFlags);
-  if (at.role != 0) {
+  const HalfHow how = half_team_share(prm, smem, b, at, team, exact.flags + (size_t)at.slot * kTeamFlags);
+  bool again = how != kHalfDone;
+  if (how == kHalfUnheld) {
+    exact.flags = prm.flags;   // (nobody has raised one of them; the others' words may not be clear yet)
+  } else if (at.role != 0) {
     const unsigned *flags = prm.flags + (size_t)at.slot * kTeamFlags;
     auto is_set = [&](int w) { return __hip_atomic_load(&flags[w], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == prm.tag; };
     int *verdict = reinterpret_cast<int *>(smem);

@@ -32,55 +32,122 @@ def _parts(packed, layer):
     return w.reshape(3, cout, cin, 9)
 
 
+def _units(packed):
+    """What each layer's sums are multiplied by (0: the set goes through three parts)."""
+    one = (packed.numel() - 208) // 2          # (the set of three parts lies behind it, 256-byte aligned)
+    return packed.cpu()[one - 4 * (8 + 544):one - 4 * 544].view(torch.float32).double()
+
+
+def _factors(packed):
+    return 1.0 / _units(packed) / torch.tensor([1.0] + [16.0] * 7).double()
+
+
+@pytest.mark.parametrize("size", [1.0, 1e-7, 1e-12, 1e5])
 @pytest.mark.parametrize("layer", [1, 3, 5, 7])
-def test_parts_of_weights(cuda, layer):
-    """16 w = hi + (lo + rest / 2048) / 2048, in fp16 each: exactly where hi is a normal number, but for the tap that takes in what the
-    others of its channel leave; and hi and lo leave nothing of the sum over a channel's taps."""
+def test_parts_of_weights(cuda, layer, size):
+    """hi + lo / 2048, which is what a 3x3 layer reads, is its weights times a power of two to three units of lo's last bit, and what they
+    leave adds up to nothing over a channel's taps; whatever the size of the layer's weights."""
     st = R.init_state(3, "reference")
     w = st[f"convs.{layer}.weight"]
-    w[0, 0] = torch.tensor([[1e-3, -1e-4, 1e-6], [0.0, 2000.0, -2047.9], [1e-9, -1e-12, 3e-13]])
-    w[1, 1, 0] = torch.tensor([2049.0, -3e38, float("nan")])
-    w[1, 1, 1] = torch.tensor([2e-13, -1e-30, 0.0])
-    bits = _parts(_model(cuda, st).packed_weights(PREC), layer)
-    want = w.flatten(2).double()
-    marked = torch.zeros_like(want, dtype=torch.bool)
-    marked[1, 1, :5] = True
-    assert bool(((bits[0] == 0x7fff) == marked).all())
-    raw = (bits[1][marked].int() & 0xffff) | (bits[2][marked].int() << 16)
-    assert torch.equal(raw, w.flatten(2)[marked].view(torch.int32))
-    hi, lo, rest = bits.view(torch.float16).double().masked_fill(marked, 0.0).unbind(0)
-    rest = rest / 2048.0
-    off = ((hi + (lo + rest) / 2048.0) / 16.0 - want).abs().masked_fill(marked, 0.0)
-    largest = want.masked_fill(marked, 0.0).abs().amax(2, keepdim=True)
-    # that tap's third part is the others' rest with the sign changed, up to three units of lo's last bit (2^-21 of the largest), to
-    # half a unit of its own
-    assert bool((off <= 3 * largest * 2.0 ** -33 + 2.0 ** -51).all())
-    inexact = (off != 0) & (want.abs() >= 2.0 ** -18)
-    assert int(inexact.sum(2).max()) <= 1
-    step = lo.abs().amax(2, keepdim=True) * 2.0 ** -10 + 2.0 ** -24   # one unit of the largest lo's last bit
-    plain = ~marked.any(2)
-    assert bool((rest.abs() <= 3 * step)[plain].all())
-    assert float((rest.sum(2, keepdim=True).abs() / step)[plain].mean()) <= 0.02
+    w[0, 0] = torch.tensor([[1e-3, -1e-4, 1e-6], [0.0, 0.1, -0.05], [1e-9, -1e-12, 3e-13]])
+    w *= size
+    packed = _model(cuda, st).packed_weights(PREC)
+    factor = _factors(packed)[layer]
+    want = w.flatten(2).double() * factor
+    assert 2.0 ** 14 <= float(want.abs().max()) < 2.0 ** 15 and float(factor.log2()) % 1 == 0
+    hi, lo, _ = _parts(packed, layer).view(torch.float16).double().unbind(0)
+    left = want - hi - lo / 2048.0
+    # half a unit of lo each, a whole one where it is rounded the other way for the sum, and the sum of nine such in one of them
+    step = (lo.abs().amax(2, keepdim=True) * 2.0 ** -10 + 2.0 ** -24) / 2048.0   # one unit of the largest lo's last bit
+    assert bool((left.abs() <= 3 * step).all())
+    assert float((left.sum(2, keepdim=True).abs() / step).mean()) <= 0.02
+    # ... and over an output's weights: half a unit of 2^-22 of a weight, at random
+    assert bool((left.flatten(1).norm(dim=1) <= 2.0 ** -23 * want.flatten(1).norm(dim=1)).all())
+
+
+@pytest.mark.parametrize("size", [1.0, 1e-7, 1e-12, 1e5])
+def test_parts_of_the_first_layer(cuda, size):
+    """... of which all three are read: to 2^-33 of a weight, or half of the third's smallest number."""
+    st = R.init_state(3, "reference")
+    st["convs.0.weight"] *= size
+    packed = _model(cuda, st).packed_weights(PREC)
+    factor = _factors(packed)[0]
+    w = st["convs.0.weight"].double() * -1.4426950408889634 * factor                # [32, 3, 23, 23]
+    assert 2.0 ** 14 / 1.5 <= float(w.abs().max()) < 2.0 ** 15
+    rows = torch.zeros(32, 70, 24, dtype=torch.float64)                             # 35 K rows per lane half, (ky, plane)
+    rows[:, :69, :23] = w.permute(0, 2, 1, 3).reshape(32, 69, 23)
+    # fragment (row, 8 columns), part, lane (half, output), 8 columns
+    got = packed.cpu()[:105 * 3 * 1024].view(torch.float16).double().view(35, 3, 3, 2, 32, 8).permute(2, 4, 3, 0, 1, 5).reshape(3, 32, 70, 24)
+    off = (got[0] + (got[1] + got[2]) / 2048.0 - rows).abs()
+    assert bool((off <= rows.abs() * 2.0 ** -33 + 2.0 ** -36).all())
+
+
+def _scale_kernel(st, layer, share):
+    """One input of one output: its largest weight to `share` of that output's."""
+    w = st[f"convs.{layer}.weight"]
+    w[5, 9] *= share * w[5].abs().max() / w[5, 9].abs().max()
+
+
+def _scale_output(st, layer, share):
+    w = st[f"convs.{layer}.weight"]
+    factor = share * w.abs().max() / w[5].abs().max()
+    w[5] *= factor
+    st[f"convs.{layer}.bias"][5] *= factor
+
+
+def _set(st, layer, index, value):
+    st[f"convs.{layer}.weight"][index] = value
+
+
+@pytest.mark.parametrize("layer", [0, 1, 4, 7])
+@pytest.mark.parametrize("change,held", [
+    (lambda st, l: None, True),
+    (lambda st, l: _set(st, l, slice(None), 0.0), True),                            # a layer, an output of zeros
+    (lambda st, l: _set(st, l, 3, 0.0), True),
+    (lambda st, l: _set(st, l, (3, 1, 1, 1), 1e-38), True),                         # one weight that nothing depends on
+    (lambda st, l: st[f"convs.{l}.weight"].mul_(1e-13), True),
+    (lambda st, l: st[f"convs.{l}.weight"].mul_(1e20), True),
+    (lambda st, l: st[f"convs.{l}.weight"].mul_(1e-15), False),
+    (lambda st, l: st[f"convs.{l}.weight"].mul_(1e25), False),
+    (lambda st, l: _scale_output(st, l, 2.0 ** -9.9), True),
+    (lambda st, l: _scale_output(st, l, 2.0 ** -10.1), False),
+    (lambda st, l: st[f"convs.{l}.weight"][5, 1].mul_(2.0 ** -6.1 * st[f"convs.{l}.weight"][5].abs().max() / st[f"convs.{l}.weight"][5, 1].abs().max()), False),
+    (lambda st, l: st[f"convs.{l}.weight"][5, 1].mul_(2.0 ** -5.9 * st[f"convs.{l}.weight"][5].abs().max() / st[f"convs.{l}.weight"][5, 1].abs().max()), True),
+    (lambda st, l: _set(st, l, (3, 1), 0.0), False),
+    (lambda st, l: _set(st, l, (3, 1, 1, 1), float("inf")), False),
+    (lambda st, l: _set(st, l, (3, 1, 1, 1), float("nan")), False),
+    (lambda st, l: _set(st, l, (3, 1, 1, 1), 1e5), False),
+])
+def test_which_weights_two_parts_hold(cuda, layer, change, held):
+    st = R.init_state(3, "reference")
+    change(st, layer)
+    units = _units(_model(cuda, st).packed_weights(PREC))
+    assert ((units != 0) == torch.tensor([held or l != layer for l in range(8)])).all()
 
 
 # (name, what it does to the parameters or the planes): on this side of the line, beyond it
 _LINES = [
-    ("weights", 2047.0, 2049.0), ("activations", 1350.0, 1500.0), ("activations", 1e5, 1e30),
-    ("small layer", 2e-5, 1e-6), ("planes", 32768.0, 32800.0), ("small planes", 2e-4, 1e-5), ("zero", 0.0, 0.0),
+    ("weights", 2047.0, 2e5), ("an input", 2.0 ** -5.9, 2.0 ** -6.1), ("an output", 2.0 ** -9.9, 2.0 ** -10.1),
+    ("activations", 1350.0, 1500.0), ("activations", 1e5, 1e30),
+    ("small layer", 2e-2, 5e-3), ("planes", 32768.0, 32800.0), ("small planes", 0.2, 0.05), ("zero", 0.0, 0.0),
 ]
 
 
 def _case(name, size):
     st, x = R.init_state(7, "torch_default"), gen_boards(40, 200, 3)[0]
-    if name == "weights":            # ... with an input of the same channel that is zero but for a bias
+    if name == "an input":
+        _scale_kernel(st, 4, size)
+    elif name == "an output":
+        _scale_output(st, 4, size)
+    elif name == "weights":          # one of them, with an input of the same channel that is zero but for a bias
         st["convs.4.weight"][5, 9] = 0.0
         st["convs.4.weight"][5, 9, 1, 1] = size
         st["convs.3.bias"][9] = 1e-3
         st["convs.3.weight"][9] *= 1e-3
-    elif name == "activations":      # one channel, of which the next layer takes little
+    elif name == "activations":      # one channel, of which the next layer takes little (less than two parts hold beside the others, the second line)
         st["convs.4.bias"][11] = size
         st["convs.4.weight"][11] = 0.0
-        st["convs.5.weight"][:, 11] *= 1.0 / size
+        st["convs.5.weight"][:, 11] *= 1.0 / 8 if size < 1e4 else 1.0 / size
     elif name == "small layer":      # a layer of small numbers, blown up again behind it
         st["convs.4.weight"] *= size
         st["convs.4.bias"] *= size
@@ -201,6 +268,51 @@ def test_small_weights_of_the_first_layer(cuda, factors):
     was, now = _against_float64(cuda, st, x, (6, 60, 200, 600))
     for n in now:
         assert n[0] <= 2 * was[0] + 3e-8 and n[1] <= 2 * was[1] + 1e-7, (was, now)
+
+
+def _channels(st, layer, channels, factor):
+    """Outputs of a layer times factor, and what the next takes of them divided by it."""
+    st[f"convs.{layer}.weight"][channels] *= factor
+    st[f"convs.{layer}.bias"][channels] *= factor
+    st[f"convs.{layer + 1}.weight"][:, channels] /= factor
+
+
+@pytest.mark.parametrize("factors", [
+    {3: 300, 4: 1e-6, 5: 1e3}, {3: 300, 4: 1e-7, 5: 1e3}, {3: 300, 4: 5e-8, 5: 3e3}, {3: 1e3, 4: 1.6e-8, 5: 3e3}, {3: 1e3, 4: 5e-9, 5: 3e3},
+    {1: 1e-4, 6: 1e4}, {2: 1e3, 3: 1e-9, 4: 1e4, 5: 1e2},
+    (3, slice(5, 6), 1e-5), (3, slice(5, 6), 1e-8), (3, slice(0, 32), 1e-3), (3, slice(0, 32), 1e-6), (3, slice(0, 63), 1e-6), (5, slice(0, 95), 1e-8),
+    (3, slice(0, 32), 2.0 ** -5), (3, slice(0, 63), 2.0 ** -3),
+])
+def test_small_weights_behind_large_activations(cuda, factors):
+    """Layers of small weights between others, and outputs of a layer that are small where the next layer's weights for them are large:
+    as near to float64 as the fp32 instructions."""
+    st, x = R.init_state(5, "reference"), gen_boards(6, 200, 3)[0]
+    if isinstance(factors, tuple):
+        _channels(st, *factors)
+    else:
+        for layer, factor in factors.items():
+            st[f"convs.{layer}.weight"] *= factor
+    was, now = _against_float64(cuda, st, x, (6, 60, 200, 600))
+    for n in now:
+        assert n[0] <= 2 * was[0] + 3e-8 and n[1] <= 2 * was[1] + 1e-7, (was, now)
+
+
+@pytest.mark.parametrize("per", [1, 5, 150, 300, 700])
+def test_sets_that_go_either_way_in_one_call(cuda, per):
+    """Weight sets of which every other is beyond two parts: teams, one board and several for each workgroup, runs of boards of both."""
+    states = [R.init_state(20 + i, "reference") for i in range(4)]
+    for st in states[1::2]:
+        _scale_output(st, 4, 2.0 ** -12)
+    packed = [_model(cuda, st).packed_weights(PREC) for st in states]
+    assert [bool((_units(p) != 0).all()) for p in packed] == [True, False, True, False]
+    x = gen_boards(4 * 30, 200, 9)[0][torch.arange(4 * per) % 120].to(cuda)
+    u = gen_uniform(4 * per, 5).to(cuda)
+    with torch.inference_mode():
+        got = run_forward(x, torch.stack(packed), PREC, 4, per, mask_mode=_lib.MASK_INPUT, u=u, want_logprob=True)
+        for i in range(4):
+            rows = slice(i * per, (i + 1) * per)
+            want = run_forward(x[rows], packed[i], PREC, 1, per, mask_mode=_lib.MASK_INPUT, u=u[rows], want_logprob=True)
+            assert all(torch.equal(g[rows].flatten(), w.flatten()) for g, w in zip(got, want)), i
 
 
 @pytest.mark.parametrize("boards", [1, 7, 30, 60, 100])

@@ -406,8 +406,7 @@ __device__ __forceinline__ bool half_left(const FwdParams &prm, long long b) {
 
 // Whether a workgroup of half_forward_kernel does a board that it cannot hold again itself: where that is its only one.  A launch of
 // split_forward_kernel, which looks for such boards and hardly ever finds one, takes 4 us: 129 boards 150.5 -> 147 us, 256
-// boards 190.2 -> 187.1 us, 384 boards (128 of them in teams) 322 -> 318.5 us.  (With every board beyond the range 256 take 793 -> 832 us, since the
-// form that needs no scratch is the slower one.)  Behind more boards each the launch stays: up to eight done again where
+// boards 190.2 -> 187.1 us, 384 boards (128 of them in teams) 322 -> 318.5 us.  Behind more boards each the launch stays: up to eight done again where
 // they ended gain as much, 512 boards 366.7 -> 363.6 us, 2,048 boards 1,427 -> 1,423 us, but a weight set beyond the range, whose boards
 // lie side by side, would go through few workgroups one after the other.
 __host__ __device__ inline bool half_redone(long long per_workgroup) { return per_workgroup == 1; }
@@ -421,7 +420,7 @@ template <class P> __global__ __launch_bounds__(256) void split_forward_kernel(c
     const long long mine = first + (threadIdx.x & 63) * grid;
     unsigned long long left = __builtin_amdgcn_ballot_w64(mine < prm.total_boards && half_left(prm, mine));
     if (left != 0) __syncthreads();   // (all have looked before an output is written)
-    for (; left != 0; left &= left - 1) split_board<false>(prm, smem, first + __builtin_ctzll(left) * grid);
+    for (; left != 0; left &= left - 1) split_board(prm, smem, first + __builtin_ctzll(left) * grid);
   }
 }
 
@@ -500,7 +499,7 @@ __global__ __launch_bounds__(256) void half_forward_kernel(const FwdParams prm) 
   v4i r1[L1Pipe<P>::D][1];
   bool again = false;
   // A set of weights that two parts do not hold: none of its boards starts here, but where a run has boards of other sets too.
-  // (256 boards of such a set 490 -> 325 us, 2,048 boards 3,660 -> 2,260 us.)
+  // (256 boards of such a set 445 -> 283 us, 2,048 boards 3,660 -> 2,260 us.)
   auto unheld = [&](const unsigned char *packed) __attribute__((always_inline)) {
     bool none = false;
 #pragma unroll
@@ -728,7 +727,7 @@ __global__ __launch_bounds__(256) void half_forward_kernel(const FwdParams prm) 
       split_write(prm, b, tidv, lane, wave, occ, lgt, red, valw[kHeadC + 1]);
     }
   }
-  if (again) split_board<true>(prm, smem, run);   // (its only board)
+  if (again) split_board(prm, smem, run);   // (its only board)
 }
 
 }  // namespace c6

@@ -354,46 +354,19 @@ __device__ __forceinline__ void split_store(unsigned char *smem, const int (&ci)
   }
 }
 
-// The sums of a layer's cout tiles one tile after the other (SLIM: in team_forward_kernel, which has no scratch to pay for on every
-// launch): the activations are read once per tile, and fewer registers are in use.  The same arithmetic for every output.
-template <int L>
-__device__ __forceinline__ void split_slim(const unsigned char *smem, const unsigned char *packed, const float *tail,
-                                           const int (&ci)[3], int h, int lane, f32x16 (&sum)[kCoutArr[L] / 32][3]) {
-  const WFrags wl = layer_weights<PrecF32X, L>(packed, lane);
-  static_for<0, kCoutArr[L] / 32>([&](auto tc) __attribute__((always_inline)) {
-    constexpr int t = decltype(tc)::value;
-    SplitWeights<1> ring;
-    f32x16 acc[1][3], low[1][3];
-    split_preload<L, t, 1>(ring, wl);
-    split_conv<L, t, 1>(smem, wl, tail + bias_offset(L), ring, ci, h, acc, low);
-#pragma unroll
-    for (int j = 0; j < 3; ++j)
-#pragma unroll
-      for (int e = 0; e < 16; ++e) sum[t][j][e] = two_sums(acc[0][j][e], low[0][j][e]);
-    __builtin_amdgcn_sched_barrier(0);
-  });
-}
-
 // one 3x3 layer that is not the last
-template <int L, bool SLIM>
+template <int L>
 __device__ __forceinline__ void split_layer(unsigned char *smem, const unsigned char *packed, const float *tail, const int (&ci)[3],
                                             int h, int lane) {
   constexpr int NT = kCoutArr[L] / 32;
   constexpr bool PLANES = kCinArr[L + 1] != 96;
-  if constexpr (SLIM) {
-    f32x16 sum[NT][3];
-    split_slim<L>(smem, packed, tail, ci, h, lane, sum);
-    __syncthreads();  // every wave has finished reading the layer's input
-    split_store<NT, PLANES>(smem, ci, h, [&](int t, int j) __attribute__((always_inline)) { return sum[t][j]; });
-  } else {
-    const WFrags wl = layer_weights<PrecF32X, L>(packed, lane);
-    SplitWeights<NT> ring;
-    split_preload<L, 0, NT>(ring, wl);
-    f32x16 acc[NT][3], low[NT][3];
-    split_conv<L, 0, NT>(smem, wl, tail + bias_offset(L), ring, ci, h, acc, low);
-    __syncthreads();
-    split_store<NT, PLANES>(smem, ci, h, [&](int t, int j) __attribute__((always_inline)) { return split_total<NT>(acc, low, t, j); });
-  }
+  const WFrags wl = layer_weights<PrecF32X, L>(packed, lane);
+  SplitWeights<NT> ring;
+  split_preload<L, 0, NT>(ring, wl);
+  f32x16 acc[NT][3], low[NT][3];
+  split_conv<L, 0, NT>(smem, wl, tail + bias_offset(L), ring, ci, h, acc, low);
+  __syncthreads();  // every wave has finished reading the layer's input
+  split_store<NT, PLANES>(smem, ci, h, [&](int t, int j) __attribute__((always_inline)) { return split_total<NT>(acc, low, t, j); });
   __syncthreads();
 }
 
@@ -513,7 +486,6 @@ __device__ __forceinline__ void split_write(const FwdParams &prm, long long b, i
 }
 
 // Board b, by one workgroup of four waves: logits, value and draw, whatever its numbers.
-template <bool SLIM>
 __device__ __forceinline__ void split_board(const FwdParams &prm, unsigned char *smem, long long b) {
   using P = PrecF32X;
   using G = Geo<P>;
@@ -655,36 +627,28 @@ __device__ __forceinline__ void split_board(const FwdParams &prm, unsigned char 
   split_store<1, true>(smem, ci, h, [&](int, int j) __attribute__((always_inline)) { return split_total<1>(a0, low, 0, j); });
   __syncthreads();
 
-  split_layer<1, SLIM>(smem, packed, tail, ci, h, lane);
-  split_layer<2, SLIM>(smem, packed, tail, ci, h, lane);
-  split_layer<3, SLIM>(smem, packed, tail, ci, h, lane);
-  split_layer<4, SLIM>(smem, packed, tail, ci, h, lane);
-  split_layer<5, SLIM>(smem, packed, tail, ci, h, lane);
-  split_layer<6, SLIM>(smem, packed, tail, ci, h, lane);
+  split_layer<1>(smem, packed, tail, ci, h, lane);
+  split_layer<2>(smem, packed, tail, ci, h, lane);
+  split_layer<3>(smem, packed, tail, ci, h, lane);
+  split_layer<4>(smem, packed, tail, ci, h, lane);
+  split_layer<5>(smem, packed, tail, ci, h, lane);
+  split_layer<6>(smem, packed, tail, ci, h, lane);
 
   // ---- layer 8 + both 1x1 heads straight from the fp32 accumulators ----
   const float *valw = tail + kBiasTotal + kHeadC;
   SplitHeads heads(tail, tid, lane, wave, h, red);
-  if constexpr (SLIM) {
-    f32x16 sum[3][3];
-    split_slim<7>(smem, packed, tail, ci, h, lane, sum);
+  const WFrags wl = layer_weights<P, 7>(packed, lane);
+  SplitWeights<3> ring;
+  split_preload<7, 0, 3>(ring, wl);
+  f32x16 acc[3][3], low8[3][3];
+  split_conv<7, 0, 3>(smem, wl, tail + bias_offset(7), ring, ci, h, acc, low8);
 #pragma unroll
-    for (int t = 0; t < 3; ++t)
-      heads.tile(t, [&](int j, int e0, float (&v)[8]) __attribute__((always_inline)) { split_silu8(sum[t][j], e0, v); });
-  } else {
-    const WFrags wl = layer_weights<P, 7>(packed, lane);
-    SplitWeights<3> ring;
-    split_preload<7, 0, 3>(ring, wl);
-    f32x16 acc[3][3], low8[3][3];
-    split_conv<7, 0, 3>(smem, wl, tail + bias_offset(7), ring, ci, h, acc, low8);
-#pragma unroll
-    for (int t = 0; t < 3; ++t) {
-      f32x16 sum;
-      heads.tile(t, [&](int j, int e0, float (&v)[8]) __attribute__((always_inline)) {
-        if (e0 == 0) sum = split_total<3>(acc, low8, t, j);
-        split_silu8(sum, e0, v);
-      });
-    }
+  for (int t = 0; t < 3; ++t) {
+    f32x16 sum;
+    heads.tile(t, [&](int j, int e0, float (&v)[8]) __attribute__((always_inline)) {
+      if (e0 == 0) sum = split_total<3>(acc, low8, t, j);
+      split_silu8(sum, e0, v);
+    });
   }
   heads.logits(lgt, valw[kHeadC]);
   __syncthreads();

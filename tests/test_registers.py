@@ -11,7 +11,7 @@ import pytest
 from connect6_amd import _lib
 
 OBJDUMP = Path("/opt/rocm/llvm/bin/llvm-objdump")
-SPLIT = "_ZN2c620split_forward_kernelINS_8PrecF32SEEEvNS_9FwdParamsE"
+SPLIT = ["_ZN2c620split_forward_kernelINS_8PrecF32SEEEvNS_9FwdParamsE", "_ZN2c619half_forward_kernelINS_8PrecF32SEEEvNS_9FwdParamsE"]
 
 
 def _listing(tmp_path, symbol):
@@ -71,9 +71,9 @@ def _moved(lines):
     return wrong
 
 
-@pytest.fixture(scope="module")
-def split(tmp_path_factory):
-    return _listing(tmp_path_factory.mktemp("split"), SPLIT)
+@pytest.fixture(scope="module", params=SPLIT)
+def split(tmp_path_factory, request):
+    return _listing(tmp_path_factory.mktemp("split"), request.param)
 
 
 def test_sums_of_hand_written_instructions_stay_in_their_registers(split):

@@ -1966,6 +1966,12 @@ template <class P> __device__ __forceinline__ void put_weight(unsigned char *dst
   else put_elem<P>(dst, e, weight_part<P>(v, part));
 }
 
+// A lane's 16 bytes.  (Its weights are all there first: a load behind a store to what may be the same place waits for its turn.)
+template <class P> __device__ __forceinline__ void put_weights(unsigned char *dst, const Scaled<P> (&v)[Geo<P>::E], int part, float factor) {
+#pragma unroll
+  for (int e = 0; e < Geo<P>::E; ++e) put_weight<P>(dst, e, v[e], part, factor);
+}
+
 // The parameters of weight set `g` of a (possibly stacked) PackParams.
 struct GroupView {
   const PackParams &p;
@@ -2012,20 +2018,28 @@ template <class P> __device__ __forceinline__ void pack_thread(const GroupView &
         int p = wv * kPixPerWave + j * 32 + m;
         p = p < kPix ? p : kPix - 1;
         const int r = p / kBoard, c = p % kBoard;
-        f32x4 t4;
-        for (int e = 0; e < 4; ++e) {
-          const float *w = prm.conv_w(0) + (size_t)((8 * q + 4 * h + e) * 3 + 2) * kK1 * kK1;
-          Scaled<P> sum = 0;
-          for (int ky = 0; ky < kK1; ++ky) {
-            const int rr = r + ky - kK1 / 2;
-            if (rr < 0 || rr >= kBoard) continue;
-            for (int kx = 0; kx < kK1; ++kx) {
-              const int cc = c + kx - kK1 / 2;
-              if (cc >= 0 && cc < kBoard) sum += w[ky * kK1 + kx];
-            }
+        // (kernel rows and columns that fall inside, in order; twenty weights are asked for together.  One by one they were what
+        // packing took: bf16 115 -> 46 us.)
+        const float *w = prm.conv_w(0) + (size_t)((8 * q + 4 * h) * 3 + 2) * kK1 * kK1;
+        Scaled<P> sum[4] = {};
+        const int kx0 = kK1 / 2 - c, ky0 = kK1 / 2 - r;
+        for (int ky = ky0 > 0 ? ky0 : 0; ky < kK1 && ky < ky0 + kBoard; ++ky) {
+          const int first = kx0 > 0 ? kx0 : 0, last = kx0 + kBoard < kK1 ? kx0 + kBoard : kK1;
+          for (int kx = first; kx < last; kx += 5) {
+            float v[5][4];
+#pragma unroll
+            for (int i = 0; i < 5; ++i)
+#pragma unroll
+              for (int e = 0; e < 4; ++e) v[i][e] = kx + i < last ? w[(e * 3 * kK1 + ky) * kK1 + kx + i] : 0.0f;
+#pragma unroll
+            for (int i = 0; i < 5; ++i)
+#pragma unroll
+              for (int e = 0; e < 4; ++e) sum[e] += v[i][e];
           }
-          t4[e] = (float)act_scaled<P>(sum);
         }
+        f32x4 t4;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) t4[e] = (float)act_scaled<P>(sum[e]);
         *reinterpret_cast<f32x4 *>(dst) = t4;
         return;
       }
@@ -2033,11 +2047,14 @@ template <class P> __device__ __forceinline__ void pack_thread(const GroupView &
         // k-step (ky, 8 columns); lane half = input plane
         const int part = (frag - G::FAST1_OFF) % G::W;
         const int fi = (frag - G::FAST1_OFF) / G::W, ky = fi / G::CPR, jj = fi % G::CPR;
-        const float *w = prm.conv_w(0);
+        const float *w = prm.conv_w(0), factor = half_factor(0);
+        Scaled<P> v[G::E];
+#pragma unroll
         for (int e = 0; e < G::E; ++e) {
           const int kx = jj * G::E + e;
-          put_weight<P>(dst, e, act_scaled<P>(kx < kK1 ? w[((m * 3 + h) * kK1 + ky) * kK1 + kx] : 0.0f), part, half_factor(0));
+          v[e] = act_scaled<P>(kx < kK1 ? w[((m * 3 + h) * kK1 + ky) * kK1 + kx] : 0.0f);
         }
+        put_weights<P>(dst, v, part, factor);
         return;
       }
       if constexpr (P::LO6) {
@@ -2095,34 +2112,27 @@ template <class P> __device__ __forceinline__ void pack_thread(const GroupView &
       const int row = s / G::CPR + kL1RowsHalf * h;  // (ky, plane) row, 69 real + 1 pad
       const int jj = s % G::CPR;
       const int ky = row / 3, ch = row - ky * 3;
+      const float factor = half_factor(0);
+      Scaled<P> v[G::E];
+#pragma unroll
       for (int e = 0; e < G::E; ++e) {
         const int kx = jj * G::E + e;
-        Scaled<P> v = 0;
-        if (row < kK1 * 3 && kx < kK1) v = act_scaled<P>(w[((co * 3 + ch) * kK1 + ky) * kK1 + kx]);
-        put_weight<P>(dst, e, v, part, half_factor(0));
+        v[e] = 0;
+        if (row < kK1 * 3 && kx < kK1) v[e] = act_scaled<P>(w[((co * 3 + ch) * kK1 + ky) * kK1 + kx]);
       }
+      put_weights<P>(dst, v, part, factor);
     } else if constexpr (kParts<P> == 2) {
-      // (tap-major; the first tap's thread takes all nine: what their parts leave is balanced over them)
-      const int kc_per_tap = cin / G::KSTEP;
-      if (part != 0 || s >= kc_per_tap) return;
-      const float factor = half_factor(l);
-      v4i o[9][3];
-#pragma unroll
-      for (int e = 0; e < G::E; ++e) {
-        HalfParts taps[9];
-        half_taps(w + (size_t)(co * cin + s * G::KSTEP + h * G::E + e) * 9, factor, taps);
-#pragma unroll
-        for (int k = 0; k < 9; ++k)
-#pragma unroll
-          for (int i = 0; i < 3; ++i) {
-            const int bits = taps[k].part[i];
-            o[k][i][e / 2] = e % 2 ? o[k][i][e / 2] | bits << 16 : bits;
-          }
-      }
+      // (tap-major; what the nine taps' parts leave is balanced over them: a thread of tap e takes all taps of channel e)
+      const int kc_per_tap = cin / G::KSTEP, e = s / kc_per_tap, c = s - e * kc_per_tap;
+      static_assert(G::E == 8, "eight channels, nine taps");
+      if (part != 0 || e >= G::E) return;
+      HalfParts taps[9];
+      half_taps(w + (size_t)(co * cin + c * G::KSTEP + h * G::E + e) * 9, half_factor(l), taps);
 #pragma unroll
       for (int k = 0; k < 9; ++k)
 #pragma unroll
-        for (int i = 0; i < 3; ++i) *reinterpret_cast<v4i *>(dst + (size_t)(k * kc_per_tap * nt * G::W + i) * 1024) = o[k][i];
+        for (int i = 0; i < 3; ++i)
+          reinterpret_cast<unsigned short *>(dst + ((k - e) * kc_per_tap * nt * G::W + i) * 1024)[e] = taps[k].part[i];
     } else {
       // k-step s -> (tap, 16 or 8 input channels): tap-major, or for the pipelined kernel
       // phase-major (a phase = all nine taps of 32 input channels)
@@ -2140,10 +2150,10 @@ template <class P> __device__ __forceinline__ void pack_thread(const GroupView &
         cbase = (s - tap * kc_per_tap) * G::KSTEP;
       }
       const int cot = 32 * tile + m;
-      for (int e = 0; e < G::E; ++e) {
-        const int c = cbase + h * G::E + e;
-        put_weight<P>(dst, e, w[(cot * cin + c) * 9 + tap], part, 1.0f);
-      }
+      Scaled<P> v[G::E];
+#pragma unroll
+      for (int e = 0; e < G::E; ++e) v[e] = w[(cot * cin + cbase + h * G::E + e) * 9 + tap];
+      put_weights<P>(dst, v, part, 1.0f);
     }
     return;
   }
@@ -2189,18 +2199,18 @@ template <class P> constexpr int pack_blocks() {
   return (int)(((long long)Geo<P>::TOTAL_FRAGS * 64 + Geo<P>::TAIL_FLOATS + kPackThreads - 1) / kPackThreads);
 }
 // (blockIdx.y = weight set: the parameter tensors are stacked [sets, ...], the packed sets lie
-// packed_stride bytes apart.  fp32: both of its sets in one launch, since what a thread with a square's sum of the third plane's
-// weights takes, most of the time, is then waited for once: 252 -> 135 us.)
+// packed_stride bytes apart.  fp32: both of its sets in one launch, 108 us; 15 more for half_scale_kernel.)
 template <class P> __global__ __launch_bounds__(kPackThreads) void pack_kernel(const PackParams all) {
   const long long at = threadIdx.x;
+  const int turn = (int)(gridDim.x - 1 - blockIdx.x);   // (the threads that take longest are the last: they start first)
   if constexpr (kParts<P> == 2) {
-    const int block = (int)blockIdx.x - pack_blocks<P>();
+    const int block = turn - pack_blocks<P>();
     if (block >= 0) {
       pack_thread<PrecF32X>(GroupView(all, blockIdx.y, kSplitOffset), block * (long long)kPackThreads + at);
       return;
     }
   }
-  pack_thread<P>(GroupView(all, blockIdx.y), blockIdx.x * (long long)kPackThreads + at);
+  pack_thread<P>(GroupView(all, blockIdx.y), turn * (long long)kPackThreads + at);
 }
 
 // sw[l] = largest power of two that keeps 2^sw * max|w_l| inside the range of the low-order

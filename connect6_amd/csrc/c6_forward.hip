@@ -1966,20 +1966,14 @@ template <class P> __device__ __forceinline__ void put_weight(unsigned char *dst
   else put_elem<P>(dst, e, weight_part<P>(v, part));
 }
 
-// A lane's 16 bytes.  (Its weights are all there first: a load behind a store to what may be the same place waits for its turn.)
-template <class P> __device__ __forceinline__ void put_weights(unsigned char *dst, const Scaled<P> (&v)[Geo<P>::E], int part, float factor) {
-#pragma unroll
-  for (int e = 0; e < Geo<P>::E; ++e) put_weight<P>(dst, e, v[e], part, factor);
-}
-
 // The parameters of weight set `g` of a (possibly stacked) PackParams.
 struct GroupView {
   const PackParams &p;
   int g;
   unsigned char *packed;
   const float *pol_w, *pol_b, *val_w, *val_b;
-  __device__ GroupView(const PackParams &pp, int group, size_t offset = 0)
-      : p(pp), g(group), packed(pp.packed + (size_t)group * pp.packed_stride + offset),
+  __device__ GroupView(const PackParams &pp, int group)
+      : p(pp), g(group), packed(pp.packed + (size_t)group * pp.packed_stride),
         pol_w(pp.pol_w + (size_t)group * kHeadC), pol_b(pp.pol_b ? pp.pol_b + group : nullptr),
         val_w(pp.val_w ? pp.val_w + (size_t)group * kHeadC : nullptr),
         val_b(pp.val_b ? pp.val_b + group : nullptr) {}
@@ -1993,8 +1987,14 @@ struct GroupView {
 };
 
 // one thread per (fragment, lane): writes the 16 bytes that lane will load
-template <class P> __device__ __forceinline__ void pack_thread(const GroupView &prm, long long gid) {
+// (blockIdx.y = weight set: the parameter tensors are stacked [sets, ...], the packed sets lie
+// packed_stride bytes apart)
+template <class P> __global__ __launch_bounds__(256) void pack_kernel(const PackParams all) {
   using G = Geo<P>;
+  const GroupView prm(all, blockIdx.y);
+  // (fp32: from the end, where the threads are that take longest)
+  const unsigned block = kParts<P> != 0 ? gridDim.x - 1 - blockIdx.x : blockIdx.x;
+  const long long gid = (long long)block * blockDim.x + threadIdx.x;
   const long long nfl = (long long)G::TOTAL_FRAGS * 64;
   // the factor of a layer's weights, fp32 by two parts (where they do not hold the weights, what is packed is not used)
   [[maybe_unused]] auto half_unit = [&](int l) { return reinterpret_cast<const float *>(prm.packed + G::TAIL_OFF)[G::TAIL_SW + l]; };
@@ -2018,28 +2018,45 @@ template <class P> __device__ __forceinline__ void pack_thread(const GroupView &
         int p = wv * kPixPerWave + j * 32 + m;
         p = p < kPix ? p : kPix - 1;
         const int r = p / kBoard, c = p % kBoard;
-        // (kernel rows and columns that fall inside, in order; twenty weights are asked for together.  One by one they were what
-        // packing took: bf16 115 -> 46 us.)
-        const float *w = prm.conv_w(0) + (size_t)((8 * q + 4 * h) * 3 + 2) * kK1 * kK1;
-        Scaled<P> sum[4] = {};
-        const int kx0 = kK1 / 2 - c, ky0 = kK1 / 2 - r;
-        for (int ky = ky0 > 0 ? ky0 : 0; ky < kK1 && ky < ky0 + kBoard; ++ky) {
-          const int first = kx0 > 0 ? kx0 : 0, last = kx0 + kBoard < kK1 ? kx0 + kBoard : kK1;
-          for (int kx = first; kx < last; kx += 5) {
-            float v[5][4];
+        f32x4 t4;
+        if constexpr (kParts<P> != 0) {
+          // (the four channels' side by side, twenty weights asked for together: one by one they are most of what packing takes, 115 us of 123
+          // where this takes 53.  The 16-bit modes' kernels stay what they are: compiled to other code, some of their weights
+          // are rounded differently.)
+          const float *w = prm.conv_w(0) + (size_t)((8 * q + 4 * h) * 3 + 2) * kK1 * kK1;
+          Scaled<P> sum[4] = {};
+          const int kx0 = kK1 / 2 - c, ky0 = kK1 / 2 - r;
+          for (int ky = ky0 > 0 ? ky0 : 0; ky < kK1 && ky < ky0 + kBoard; ++ky) {
+            const int first = kx0 > 0 ? kx0 : 0, last = kx0 + kBoard < kK1 ? kx0 + kBoard : kK1;
+            for (int kx = first; kx < last; kx += 5) {
+              float v[5][4];
 #pragma unroll
-            for (int i = 0; i < 5; ++i)
+              for (int i = 0; i < 5; ++i)
 #pragma unroll
-              for (int e = 0; e < 4; ++e) v[i][e] = kx + i < last ? w[(e * 3 * kK1 + ky) * kK1 + kx + i] : 0.0f;
+                for (int e = 0; e < 4; ++e) v[i][e] = w[(e * 3 * kK1 + ky) * kK1 + (kx + i < last ? kx + i : last - 1)];
 #pragma unroll
-            for (int i = 0; i < 5; ++i)
+              for (int i = 0; i < 5; ++i)
 #pragma unroll
-              for (int e = 0; e < 4; ++e) sum[e] += v[i][e];
+                for (int e = 0; e < 4; ++e) sum[e] += kx + i < last ? v[i][e] : 0.0f;
+            }
+          }
+#pragma unroll
+          for (int e = 0; e < 4; ++e) t4[e] = (float)act_scaled<P>(sum[e]);
+        } else {
+          for (int e = 0; e < 4; ++e) {
+            const float *w = prm.conv_w(0) + (size_t)((8 * q + 4 * h + e) * 3 + 2) * kK1 * kK1;
+            Scaled<P> sum = 0;
+            for (int ky = 0; ky < kK1; ++ky) {
+              const int rr = r + ky - kK1 / 2;
+              if (rr < 0 || rr >= kBoard) continue;
+              for (int kx = 0; kx < kK1; ++kx) {
+                const int cc = c + kx - kK1 / 2;
+                if (cc >= 0 && cc < kBoard) sum += w[ky * kK1 + kx];
+              }
+            }
+            t4[e] = (float)act_scaled<P>(sum);
           }
         }
-        f32x4 t4;
-#pragma unroll
-        for (int e = 0; e < 4; ++e) t4[e] = (float)act_scaled<P>(sum[e]);
         *reinterpret_cast<f32x4 *>(dst) = t4;
         return;
       }
@@ -2048,13 +2065,10 @@ template <class P> __device__ __forceinline__ void pack_thread(const GroupView &
         const int part = (frag - G::FAST1_OFF) % G::W;
         const int fi = (frag - G::FAST1_OFF) / G::W, ky = fi / G::CPR, jj = fi % G::CPR;
         const float *w = prm.conv_w(0), factor = half_factor(0);
-        Scaled<P> v[G::E];
-#pragma unroll
         for (int e = 0; e < G::E; ++e) {
           const int kx = jj * G::E + e;
-          v[e] = act_scaled<P>(kx < kK1 ? w[((m * 3 + h) * kK1 + ky) * kK1 + kx] : 0.0f);
+          put_weight<P>(dst, e, act_scaled<P>(kx < kK1 ? w[((m * 3 + h) * kK1 + ky) * kK1 + kx] : 0.0f), part, factor);
         }
-        put_weights<P>(dst, v, part, factor);
         return;
       }
       if constexpr (P::LO6) {
@@ -2113,14 +2127,12 @@ template <class P> __device__ __forceinline__ void pack_thread(const GroupView &
       const int jj = s % G::CPR;
       const int ky = row / 3, ch = row - ky * 3;
       const float factor = half_factor(0);
-      Scaled<P> v[G::E];
-#pragma unroll
       for (int e = 0; e < G::E; ++e) {
         const int kx = jj * G::E + e;
-        v[e] = 0;
-        if (row < kK1 * 3 && kx < kK1) v[e] = act_scaled<P>(w[((co * 3 + ch) * kK1 + ky) * kK1 + kx]);
+        Scaled<P> v = 0;
+        if (row < kK1 * 3 && kx < kK1) v = act_scaled<P>(w[((co * 3 + ch) * kK1 + ky) * kK1 + kx]);
+        put_weight<P>(dst, e, v, part, factor);
       }
-      put_weights<P>(dst, v, part, factor);
     } else if constexpr (kParts<P> == 2) {
       // (tap-major; what the nine taps' parts leave is balanced over them: a thread of tap e takes all taps of channel e)
       const int kc_per_tap = cin / G::KSTEP, e = s / kc_per_tap, c = s - e * kc_per_tap;
@@ -2150,10 +2162,10 @@ template <class P> __device__ __forceinline__ void pack_thread(const GroupView &
         cbase = (s - tap * kc_per_tap) * G::KSTEP;
       }
       const int cot = 32 * tile + m;
-      Scaled<P> v[G::E];
-#pragma unroll
-      for (int e = 0; e < G::E; ++e) v[e] = w[(cot * cin + cbase + h * G::E + e) * 9 + tap];
-      put_weights<P>(dst, v, part, 1.0f);
+      for (int e = 0; e < G::E; ++e) {
+        const int c = cbase + h * G::E + e;
+        put_weight<P>(dst, e, w[(cot * cin + c) * 9 + tap], part, 1.0f);
+      }
     }
     return;
   }
@@ -2192,25 +2204,6 @@ template <class P> __device__ __forceinline__ void pack_thread(const GroupView &
     }
     tail[ti] = v;
   }
-}
-
-constexpr int kPackThreads = 256;
-template <class P> constexpr int pack_blocks() {
-  return (int)(((long long)Geo<P>::TOTAL_FRAGS * 64 + Geo<P>::TAIL_FLOATS + kPackThreads - 1) / kPackThreads);
-}
-// (blockIdx.y = weight set: the parameter tensors are stacked [sets, ...], the packed sets lie
-// packed_stride bytes apart.  fp32: both of its sets in one launch, 108 us; 15 more for half_scale_kernel.)
-template <class P> __global__ __launch_bounds__(kPackThreads) void pack_kernel(const PackParams all) {
-  const long long at = threadIdx.x;
-  const int turn = (int)(gridDim.x - 1 - blockIdx.x);   // (the threads that take longest are the last: they start first)
-  if constexpr (kParts<P> == 2) {
-    const int block = turn - pack_blocks<P>();
-    if (block >= 0) {
-      pack_thread<PrecF32X>(GroupView(all, blockIdx.y, kSplitOffset), block * (long long)kPackThreads + at);
-      return;
-    }
-  }
-  pack_thread<P>(GroupView(all, blockIdx.y), turn * (long long)kPackThreads + at);
 }
 
 // sw[l] = largest power of two that keeps 2^sw * max|w_l| inside the range of the low-order
@@ -2333,11 +2326,20 @@ template <class P> int launch_second_pass(const TeamParams &tp, int grid, hipStr
 
 #ifndef C6_SPLIT
 template <class P> int launch_pack(const PackParams &pp, hipStream_t st) {
-  const int blocks = pack_blocks<P>() + (kParts<P> == 2 ? pack_blocks<PrecF32X>() : 0);
+  using G = Geo<P>;
+  const long long total = (long long)G::TOTAL_FRAGS * 64 + G::TAIL_FLOATS;
+  const int threads = 256;
+  const int blocks = (int)((total + threads - 1) / threads);
   const unsigned sets = (unsigned)pp.groups;
   if constexpr (P::LO6) hipLaunchKernelGGL(lo_scale_kernel<P>, dim3(8, sets), dim3(256), 0, st, pp);
   if constexpr (kParts<P> == 2) hipLaunchKernelGGL(half_scale_kernel<P>, dim3(8, sets), dim3(1024), 0, st, pp);
-  hipLaunchKernelGGL(pack_kernel<P>, dim3(blocks, sets), dim3(kPackThreads), 0, st, pp);
+  hipLaunchKernelGGL(pack_kernel<P>, dim3(blocks, sets), dim3(threads), 0, st, pp);
+  if constexpr (kParts<P> == 2) {   // (a set of the same size for the other way)
+    static_assert(Geo<PrecF32X>::TOTAL_FRAGS == G::TOTAL_FRAGS && Geo<PrecF32X>::TAIL_FLOATS == G::TAIL_FLOATS, "one grid");
+    PackParams exact = pp;
+    exact.packed += kSplitOffset;
+    hipLaunchKernelGGL(pack_kernel<PrecF32X>, dim3(blocks, sets), dim3(threads), 0, st, exact);
+  }
   const hipError_t e = hipGetLastError();
   if (e != hipSuccess) {
     set_error("pack_kernel launch failed: %s", hipGetErrorString(e));

@@ -152,8 +152,8 @@ template <class P> __device__ __forceinline__ float silu(float v) {
   }
 }
 template <class P> __host__ __device__ constexpr float act_scale() { return P::EB == 4 ? 1.0f : kActScale; }
-// What is scaled while the weights are packed: fp32 by three parts takes the factor to 53 bits, so that a
-// weight is rounded once, when its three parts are taken, and a bias and a sum of weights once, to fp32.
+// What is scaled while the weights are packed: fp32 by 16-bit parts takes the factor to 53 bits, so that a
+// weight is rounded once, when its parts are taken, and a bias and a sum of weights once, to fp32.
 // (Its head weights are not divided by it: the sums over them are, in the kernel.)
 template <class P> using Scaled = std::conditional_t<kParts<P> != 0, double, float>;
 constexpr double kActScale64 = -1.4426950408889634074;
@@ -2241,7 +2241,7 @@ template <class P> __global__ __launch_bounds__(256) void lo_scale_kernel(const 
 //  * an output all of whose weights are small beside the layer's (below 2^-10, but for zeros): two parts could drop them, or
 //  * an input that one of its outputs takes little of (below 2^-6 of the largest weight of that output).  half_failed sees that
 //    the largest input is not small; only so is it known that the sum is not one over small inputs alone, whose last bits two
-//    parts drop.  (Of 2.4e5 kernels of six networks with either initialisation the smallest such share is 0.11, the smallest output's
+//    parts drop.  (Of 2.1e5 kernels, three networks of either initialisation, the smallest such share is 0.11, the smallest output's
 //    largest weight 0.5 of its layer's.)
 template <class P> __global__ __launch_bounds__(1024) void half_scale_kernel(const PackParams all) {
   using G = Geo<P>;

@@ -18,7 +18,7 @@
 // Relative error of logits / of values against a 64-bit forward (24 networks x 12 boards, rms) with the reference's
 // initialisation and PyTorch's, and the mean of a network's logit errors:
 //     six products                            4.6e-7 / 1.6e-7   6.9e-8 / 3.7e-8   0.8e-8, 0.5e-8
-//     three, as they are here                 4.0e-7 / 0.7e-7   3.5e-8 / 2.5e-8   1.3e-8, 0.2e-8
+//     three, as they are here                 4.0e-7 / 0.8e-7   3.6e-8 / 2.5e-8   1.3e-8, 0.1e-8
 //     fp32 instructions                       1.4e-6 / 3.7e-7   1.8e-7 / 3.6e-8   7.3e-8, 0.3e-8
 // (three products with one sum per layer and every lo rounded to nearest are off by 5.6e-7 and, from the last layer on in 64
 // bits, 2.2e-7 with the reference's initialisation; half of what the values gained is their sum over the board in 64 bits.)
@@ -39,8 +39,8 @@
 // times each) of 330 k at 1.9 GHz; what goes in the open is the epilogue of each layer's last cout tile (5 k), the sums at the ends of kernel rows
 // and the first operands of each pass (3 to 5 k), and staging (7 k).  2,048 boards, both sides in turn: 2,117 -> 1,382 us from six
 // products to three with the same structure, and 2,260 -> 1,436 on another box with all epilogues but the last tile's behind MFMAs and
-// three instructions fewer in each (in cycles 350 k -> 330 k; the clock gives back half of it).  In teams (c6_team.h) one board 58 ->
-// 49 us, 53 boards 117 -> 98, 128 boards 215 -> 142, of which the launch that looked for boards left over was 4.
+// three instructions fewer in each (in cycles 350 k -> 330 k; the clock gives back half of it).  In teams (c6_half_team.h) one board 57 ->
+// 45 us, 53 boards 114 -> 82, 128 boards 217 -> 134.
 #pragma once
 
 namespace c6 {

@@ -822,8 +822,8 @@ __device__ __forceinline__ HalfHow half_team_share(const TeamParams &prm, unsign
   return kHalfDone;
 }
 
-// A board that two parts do not hold is done again by its team with three: one board 111 us, 53 boards 200, 128 boards 330 (by the workgroup
-// that ends it, alone, 314, 347 and 380).  The members wait for the last stage's verdict, which is given as soon as that stage's loads have
+// A board that two parts do not hold is done again by its team with three: one board 110 us, 53 boards 196, 128 boards 356 (by the workgroup
+// that ends it, alone, 314, 347 and 380); a set of weights that they do not hold, at once: 62, 120, 224.  The members wait for the last stage's verdict, which is given as soon as that stage's loads have
 // arrived, so that they end with the workgroup that gives it: boards in range take what they took (given behind the outputs one board 45.2 ->
 // 45.7 us, 85 boards 98.5 -> 99.6 us).  The second way has exchange memory and flags of its own, behind the first one's: a member that comes late may
 // still be at its part of the first.

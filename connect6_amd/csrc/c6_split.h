@@ -1,5 +1,5 @@
-// fp32 forward of any board on the bf16 matrix cores (included by c6_forward.hip): the boards whose numbers do not fit
-// the two fp16 parts of c6_half.h, which serves all others.
+// fp32 forward of any board on the bf16 matrix cores (included by c6_forward.hip): the boards and sets of weights whose numbers
+// do not fit the two fp16 parts of c6_half.h, which serves all others.
 //
 // Every fp32 operand is the exact sum of three bf16 values: hi = bf16(v), mid = bf16(v - hi),
 // lo = v - hi - mid (8 mantissa bits each, both differences exact).  A product is then nine products

@@ -54,7 +54,7 @@ def test_fused_kernels_stay_within_their_scratch_budget():
     team = [u for name, u in usage.items() if "team_forward_kernel" in name]
     small = [u for name, u in usage.items() if "small_net_kernel" in name]
     assert len(team) == 5 and len(small) == 12 and all(u["ScratchSize"] == 0 for u in team + small)
-    # fp32 by three parts: two sums of every tile fill the accumulators and 32 vector registers (test_registers.py); what
+    # fp32 by three bf16 parts: two sums of every tile fill the accumulators and 32 vector registers (test_registers.py); what
     # is in scratch is touched between the K-loops, not in them
     (split,) = [u for name, u in usage.items() if "split_forward_kernel" in name]
     assert split["ScratchSize"] <= 96

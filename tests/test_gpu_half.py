@@ -316,10 +316,11 @@ def test_sets_that_go_either_way_in_one_call(cuda, per):
 
 
 @pytest.mark.parametrize("boards", [1, 7, 30, 60, 100])
-def test_a_team_without_all_its_members_does_a_board_again(cuda, boards):
-    """Boards of either kind in teams whose waits run out at once, so that members leave before the verdict or come late, and in
-    ordinary ones."""
-    st, x = _case("planes", 40000.0)
+@pytest.mark.parametrize("case", [("planes", 40000.0), ("an output", 2.0 ** -12)])
+def test_a_team_without_all_its_members_does_a_board_again(cuda, boards, case):
+    """Boards of either kind, and those of a set that two parts do not hold, in teams whose waits run out at once, so that members leave
+    before the verdict or come late, and in ordinary ones."""
+    st, x = _case(*case)
     packed = _model(cuda, st).packed_weights(PREC)
     xd = x[(torch.arange(boards) + 1) % 40].to(cuda)
     flags = torch.zeros(boards * 256, dtype=torch.int32, device=cuda)
@@ -330,9 +331,10 @@ def test_a_team_without_all_its_members_does_a_board_again(cuda, boards):
             assert torch.equal(lg, want[0][:boards]) and torch.equal(vg, want[1][:boards]), polls
 
 
-@pytest.mark.parametrize("boards", [20, 300])
-def test_graphs_of_boards_that_take_either_way(cuda, boards):
-    st, x = _case("planes", 40000.0)
+@pytest.mark.parametrize("boards", [20, 300, 600])
+@pytest.mark.parametrize("case", [("planes", 40000.0), ("an output", 2.0 ** -12)])
+def test_graphs_of_boards_that_take_either_way(cuda, boards, case):
+    st, x = _case(*case)
     model = _model(cuda, st)
     xs = [x[(torch.arange(boards) + i) % 40].to(cuda) for i in range(3)]
     with torch.inference_mode():

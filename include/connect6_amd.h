@@ -48,15 +48,16 @@ extern "C" {
                             twice the bf16 matrix work): within 3e-4 relative L2 of fp32 */
 
 #define C6_PREC_F32S 7   /* fp32 operands, each as two fp16 values of 11 mantissa bits: three fp16 MFMAs
-                            per product, fp32 accumulate.  fp32 results (with random weights less than half
-                            as far from a 64-bit forward as those of C6_PREC_F32) at a third of the time; its packed
+                            per product, fp32 accumulate.  fp32 results (with random weights logits less than
+                            half as far from a 64-bit forward as those of C6_PREC_F32) at a third of the time; its packed
                             weights (of both ways below) take three times that mode's.  What fp16 does not hold
                             so is computed with three bf16 values per operand and six MFMAs per product: a set of
                             weights with a layer that has an output whose weights are all below 1/1024 of the layer's
                             largest, or an output whose weights for one input are all below 1/64 of its largest (but
                             for layers and outputs of zeros), or weights that are all below 2e-14 or one beyond 1e22; a
                             board with an activation beyond 1400, or a layer of activations that are all below
-                            3.4e-4 and not all zero.  Infinities and NaN as in fp32, except that a sum or an
+                            3.4e-4 and not all zero, or with planes that are not exact in fp16 and beyond 32768 or
+                            all below 1/128.  Infinities and NaN as in fp32, except that a sum or an
                             activation beyond 2.3e38 (fp32: 3.4e38) counts as infinite.  In an
                             architecture that c6_generic_packed_bytes is not 0 for, C6_PREC_F32
                             too is computed with three bf16 values, with sums and activations up to 3.38e38 */
